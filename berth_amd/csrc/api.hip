@@ -161,6 +161,7 @@ Knobs read_knobs()
     k.gemm_wg_per_cu = env_int("BERTH_GEMM_WG_PER_CU", 0);
     k.gemm_balanced = env_int("BERTH_GEMM_BALANCED", 1);
     k.gemm_rows256 = env_int("BERTH_GEMM_ROWS256", 1);
+    k.gemm_rows_units = env_int("BERTH_GEMM_ROWS_UNITS", -1);
     k.counter_stride = clamp(env_int("BERTH_COUNTER_STRIDE", 32), 1, 32);
     k.moe_big_min = env_int("BERTH_MOE_BIG_MIN", 33);
     k.moe_route_slab = env_int("BERTH_MOE_ROUTE_SLAB", 1);
@@ -567,6 +568,15 @@ extern "C" int berth_prefill_had_r_128(const void* input, void* output, const vo
 extern "C" const char* berth_prefill_last_error(void) { return g_prefill_err.c_str(); }
 extern "C" const char* berth_prefill_last_launch(void) { return g_prefill_launch.c_str(); }
 
+// gate and up of an MLP for 1..8 rows: on the few-row MFMA kernel where that serves them (the up
+// projection's rotated copy of the input waits in act_had, as above 8 rows), else in one VALU launch
+static std::string launch_pair_few_rows(const PairArgs& pair, void* act_had)
+{
+    if (pair.size_n >= pair.size_k && gemv_rows_on_matrix_units(2, pair.size_m, pair.size_k, pair.size_n))
+        return launch_gemm_pair(pair, act_had);
+    return launch_gemv_pair(pair);
+}
+
 extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* gate_out, void* up_out, void* a_had,
                               void* act_had, void* y, int size_m, int hidden, int intermediate, int k_bits,
                               int codebook, void* stream)
@@ -589,7 +599,7 @@ extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* g
         if (size_m <= 8) {
             PairArgs pair{x, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh}, {lins[0].svh, lins[1].svh},
                           {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits, codebook, st};
-            std::string desc = launch_gemv_pair(pair);
+            std::string desc = launch_pair_few_rows(pair, act_had);
             down.a = gate_out;
             down.a_up = up_out;
             g_exl3_launch = desc + " ; " + launch_gemv(down);
@@ -612,7 +622,10 @@ extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* g
             desc = launch_gemm(gate);
             desc += " ; " + launch_gemm(up);
         }
-        desc += " ; " + launch_silu_mul(gate_out, up_out, up_out, (int64_t)size_m * intermediate, 0.0f, st);
+        // the gated activation and its rotation in one launch; up_out ends up holding the activation
+        down.a = gate_out;
+        down.a_up = up_out;
+        down.act_out = up_out;
         g_exl3_launch = desc + " ; " + launch_gemm(down);
         return 0;
     } catch (const std::exception& err) {
@@ -675,7 +688,7 @@ extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* r
                 PairArgs pair{h_norm, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh},
                               {lins[0].svh, lins[1].svh}, {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits,
                               codebook, st};
-                desc += " ; " + launch_gemv_pair(pair);
+                desc += " ; " + launch_pair_few_rows(pair, act_had);
             }
             down.a = gate_out;
             down.a_up = up_out;

@@ -2,6 +2,8 @@
 #include "exl3_decode.cuh"
 #include "hadamard.cuh"
 #include "launch.h"
+#include "rows_operand.cuh"
+#include "silu.cuh"
 
 namespace berth {
 
@@ -52,33 +54,53 @@ __global__ __launch_bounds__(256) void had_r_128_kernel(const T* __restrict__ in
     }
 }
 
-// The rotated inputs of a bundle in one launch: blockIdx.y is the slab, whose sign scales come
-// from a device list of pointers or from the pointers passed by value.
-struct SuhTable {
+// The rotated inputs of a launch of the MFMA kernels: Hh(in * suh) per row and 128 columns, for
+// one or more slabs (blockIdx.y), whose sign scales come from a device list of pointers or by
+// value.  SILU: the input is silu(in) * up with the fp16 steps of silu_mul_kernel, formed here
+// instead of in a launch of its own (act_out, when given, still receives it: it may be `up`, whose
+// elements a lane has read before it writes them); 6 bytes an element (8 with act_out) against 10
+// of the two launches.  `operand`, when given, receives a second copy of the result in the operand
+// order of the few-row kernel.
+struct RotateTable {
     const _Float16* suh[kBundleMaxSlices];
     _Float16* out[kBundleMaxSlices];        // null: slab s goes to out + s * out_stride
 };
-__global__ __launch_bounds__(256) void had_r_128_slabs_kernel(const _Float16* __restrict__ in, size_t in_stride,
-                                                              _Float16* __restrict__ out, size_t out_stride,
-                                                              const uint64_t* __restrict__ suh_list, SuhTable tab,
-                                                              long blocks, int col_blocks)
+struct RotateParams {
+    const _Float16* in;
+    const _Float16* up;
+    _Float16* act_out;
+    _Float16* out;
+    _Float16* operand;
+    const uint64_t* suh_list;
+    size_t in_stride, out_stride, operand_stride;
+    long blocks;
+    int col_blocks, mt;
+    RotateTable tab;
+};
+template <bool SILU>
+__device__ __forceinline__ void rotate_rows(const RotateParams& p)
 {
     const int slab = blockIdx.y;
-    const _Float16* scale = suh_list ? (const _Float16*)suh_list[slab] : tab.suh[slab];
-    in += (size_t)slab * in_stride;
-    out = (!suh_list && tab.out[slab]) ? tab.out[slab] : out + (size_t)slab * out_stride;
+    const _Float16* scale = p.suh_list ? (const _Float16*)p.suh_list[slab] : p.tab.suh[slab];
+    const _Float16* in = p.in + (size_t)slab * p.in_stride;
+    _Float16* out = (!p.suh_list && p.tab.out[slab]) ? p.tab.out[slab] : p.out + (size_t)slab * p.out_stride;
     const int lane = threadIdx.x & 63;
     const int l16 = lane & 15;
     const long waves = (long)gridDim.x * 4;
-    const long groups = (blocks + 3) / 4;
+    const long groups = (p.blocks + 3) / 4;
     for (long g = (long)blockIdx.x * 4 + (threadIdx.x >> 6); g < groups; g += waves) {
         const long blk = g * 4 + (lane >> 4);
-        const bool live = blk < blocks;
-        const long b = live ? blk : blocks - 1;             // lanes past the end redo the last block and store nothing
-        const int cb = (int)(b % col_blocks);
+        const bool live = blk < p.blocks;
+        const unsigned b = (unsigned)(live ? blk : p.blocks - 1);   // lanes past the end redo the last block and store nothing
+        const unsigned row = b / (unsigned)p.col_blocks, cb = b - row * (unsigned)p.col_blocks;
         const size_t at = (size_t)b * 128 + 8 * l16;
-        const half8_t x = *(const half8_t*)(in + at);
+        half8_t x = *(const half8_t*)(in + at);
         const half8_t s8 = *(const half8_t*)(scale + cb * 128 + 8 * l16);
+        if (SILU) {
+            const half8_t u = *(const half8_t*)(p.up + at);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = silu_mul_h(x[i], u[i]);
+        }
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = (float)x[i] * (float)s8[i];
@@ -86,31 +108,49 @@ __global__ __launch_bounds__(256) void had_r_128_slabs_kernel(const _Float16* __
         half8_t o;
 #pragma unroll
         for (int i = 0; i < 8; ++i) o[i] = (_Float16)(v[i] * kRsqrt128);
-        if (live) *(half8_t*)(out + at) = o;
-    }
-}
-
-std::string launch_had_r_128_slabs(const void* in, size_t in_stride, void* out, size_t out_stride, const void* suh_list,
-                                   const void* const* suh_host, int slabs, int rows, int cols, hipStream_t stream,
-                                   void* const* out_host)
-{
-    if (slabs < 1 || slabs > 65535) throw std::runtime_error("had_r_128 slabs: between 1 and 65535 slabs");
-    SuhTable tab{};
-    if (!suh_list) {
-        if (slabs > kBundleMaxSlices) throw std::runtime_error("had_r_128 slabs: too many slabs for the by-value table");
-        for (int i = 0; i < slabs; ++i) {
-            tab.suh[i] = (const _Float16*)suh_host[i];
-            tab.out[i] = out_host ? (_Float16*)out_host[i] : nullptr;
+        if (live) {
+            if (SILU && p.act_out) *(half8_t*)(p.act_out + at) = x;
+            *(half8_t*)(out + at) = o;
+            if (p.operand)
+                *(half8_t*)(p.operand + (size_t)slab * p.operand_stride +
+                            rows_operand_offset((int)row, (int)cb * 128 + 8 * l16, p.mt)) = o;
         }
     }
-    const int col_blocks = cols / 128;
-    const long blocks = (long)rows * col_blocks;
-    const long wgs = (blocks + 15) / 16;
-    const dim3 grid((unsigned)(wgs < 4096 ? wgs : 4096), (unsigned)slabs);
-    hipLaunchKernelGGL(had_r_128_slabs_kernel, grid, dim3(256), 0, stream, (const _Float16*)in, in_stride, (_Float16*)out,
-                       out_stride, (const uint64_t*)suh_list, tab, blocks, col_blocks);
+}
+__global__ __launch_bounds__(256) void had_r_128_slabs_kernel(RotateParams p) { rotate_rows<false>(p); }
+__global__ __launch_bounds__(256) void silu_mul_had_r_128_kernel(RotateParams p) { rotate_rows<true>(p); }
+
+std::string launch_rotate(const RotateArgs& a)
+{
+    if (a.slabs < 1 || a.slabs > 65535) throw std::runtime_error("had_r_128 slabs: between 1 and 65535 slabs");
+    RotateParams p{};
+    p.in = (const _Float16*)a.in;
+    p.up = (const _Float16*)a.up;
+    p.act_out = (_Float16*)a.act_out;
+    p.out = (_Float16*)a.out;
+    p.operand = (_Float16*)a.operand;
+    p.suh_list = (const uint64_t*)a.suh_list;
+    p.in_stride = a.in_stride;
+    p.out_stride = a.out_stride;
+    p.mt = a.mt;
+    p.operand_stride = rows_operand_elements(a.cols, a.mt);
+    p.col_blocks = a.cols / 128;
+    p.blocks = (long)a.rows * p.col_blocks;
+    if (p.blocks >= (1L << 31)) throw std::runtime_error("had_r_128 slabs: too many rows");
+    if (!a.suh_list) {
+        if (a.slabs > kBundleMaxSlices) throw std::runtime_error("had_r_128 slabs: too many slabs for the by-value table");
+        for (int i = 0; i < a.slabs; ++i) {
+            p.tab.suh[i] = (const _Float16*)a.suh_host[i];
+            p.tab.out[i] = a.out_host ? (_Float16*)a.out_host[i] : nullptr;
+        }
+    }
+    const long wgs = (p.blocks + 15) / 16;
+    const dim3 grid((unsigned)(wgs < 4096 ? wgs : 4096), (unsigned)a.slabs);
+    if (a.up) hipLaunchKernelGGL(silu_mul_had_r_128_kernel, grid, dim3(256), 0, a.stream, p);
+    else hipLaunchKernelGGL(had_r_128_slabs_kernel, grid, dim3(256), 0, a.stream, p);
     hip_ok(hipGetLastError(), "had_r_128 slabs launch");
-    return "had_r_128_slabs_kernel grid=" + std::to_string(grid.x) + "x" + std::to_string(grid.y) + " block=256";
+    return std::string(a.up ? "silu_mul_had_r_128_kernel" : "had_r_128_slabs_kernel") + " grid=" + std::to_string(grid.x) +
+           "x" + std::to_string(grid.y) + " block=256";
 }
 
 std::string launch_had_r_128(const void* in, void* out, const void* scale, int pre_scale,
@@ -154,11 +194,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const half2_t* __restrict
             gj = (_Float16)gl;
             uj = (_Float16)ul;
         }
-        _Float16 e = (_Float16)expf(-(float)gj);
-        _Float16 s = (_Float16)1.0f + e;
-        _Float16 r = (_Float16)(1.0f / (float)s);
-        _Float16 t = gj * r;
-        o[j] = t * uj;
+        o[j] = silu_mul_h(gj, uj);
     }
     out[i] = o;
 }

@@ -1,11 +1,13 @@
 // Launchers of the EXL3 MFMA GEMM (exl3_gemm_kernel.cuh): dense rows through
 // berth_prefill_exl3_linear / berth_exl3_linear, grouped MoE problems, and the
 // plain fp16 GEMM of crates/berth-kernels/csrc/prefill_lin/linear.cu:387-418.
-#include "exl3_gemm_kernel.cuh"
+#include "exl3_gemm_rows_kernel.cuh"
 #include "launch.h"
+#include "rows_operand.cuh"
 
 #include <cstdlib>
 #include <cstring>
+#include <optional>
 
 namespace berth {
 
@@ -54,6 +56,106 @@ static int gemm_counter_stride(long tiles)
     int stride = 1;
     while (stride * 2 <= cap && tiles * stride * 2 <= kCounters / 2) stride *= 2;
     return stride;
+}
+
+// ---- few rows (exl3_gemm_rows_kernel): how the launch's units are dealt out, and when it applies
+struct RowsPlan {
+    bool ok = false;
+    int mt = 1;                 // tiles of 16 rows
+    long units = 0;             // 64 x 128 weights each
+    unsigned grid = 0, q = 0, rem = 0, S = 0;
+    size_t lds = 0;
+    size_t operand_at = 0;      // bytes into the partial-sum workspace
+};
+
+static unsigned magic(unsigned d) { return (unsigned)((1ull << 32) / d) + 1u; }
+
+// Fewest units for which the few-row kernel is taken.  Up to 8 rows the alternative is the VALU
+// kernel of exl3_gemv.hip, which rotates the input itself (one launch instead of two) and pays half
+// an instruction per weight and row: 4096 x 2048 (1024 units) takes 9.8 / 13.4 / 16.8 us at 2 / 5
+// / 8 rows there and 10.3 / 10.9 / 11.3 here, 4096 x 8192 (4096 units) 13.4 against 12.8 at two.
+// Above 8 rows it is the 32-row MFMA kernel, whose hand-over and half-empty rounds cost more from
+// the start (2048 x 1024, 256 units: 14.1 -> 10.6 us at 12 rows, 16.0 -> 13.9 at 32).
+// BERTH_GEMM_ROWS_UNITS replaces the rule (0: never).
+static int rows_min_units(int size_m)
+{
+    const int forced = knobs().gemm_rows_units;
+    if (forced >= 0) return forced;
+    return size_m <= 3 ? 3072 : size_m <= 8 ? 1024 : 192;
+}
+
+static RowsPlan plan_rows(const Workspace& ws, int slices, int slabs, int size_m, int size_k, int size_n)
+{
+    RowsPlan pl;
+    const int min_units = rows_min_units(size_m);
+    if (min_units <= 0 || size_m < 2 || size_m > 32 || size_k % 64 != 0 || size_n % 128 != 0) return pl;
+    const unsigned TR4 = (unsigned)size_k / 64;
+    const long blocks = (long)slices * (size_n / 128);
+    const unsigned long long U = (unsigned long long)blocks * TR4;
+    if (U < (unsigned long long)min_units || U >= (1ull << 30) || blocks > kCounters / 2) return pl;
+    if ((unsigned long long)size_m * size_k >= (1ull << 31)) return pl;
+    // one workgroup per compute unit with at least a unit per wave group; several rounds of them
+    // where the column blocks that a range touches would not fit the LDS together
+    for (int rounds = 1; rounds <= 64; rounds *= 2) {
+        unsigned long long G = (unsigned long long)ws.cu_count * rounds;
+        if (G > U / 4) G = U / 4;
+        if (G < 1) return pl;
+        unsigned q = (unsigned)(U / G), rem = (unsigned)(U % G), S = 0;
+        const unsigned most = q + (rem ? 1 : 0);
+        unsigned ncb = (most + TR4 - 2) / TR4 + 1;                  // column blocks a range can touch
+        // At least two workgroups per column block: parts of its own for each block where the
+        // longest part is no more than an eighth above the even share.  A range across two blocks
+        // hands both over (2688 x 4096 at 8 / 32 rows: 12.8 / 22.1 -> 11.1 / 16.1 us with parts of its own).
+        if (G >= 2 * (unsigned long long)blocks) {
+            const unsigned s = (unsigned)(G / blocks);
+            if (TR4 / s >= 4 && ((TR4 + s - 1) / s) * 8ull <= most * 9ull) {
+                S = s;
+                G = (unsigned long long)blocks * s;
+                q = rem = 0;
+                ncb = 1;
+            }
+        }
+        const size_t lds = rows_lds_bytes(size_m, (int)ncb);
+        if (ncb > (unsigned)kRowsWaves || lds > 160 * 1024) continue;
+        // exact division by multiply-high needs dividend * divisor < 2^32
+        if (U * (q + 2) >= (1ull << 32) || U * TR4 >= (1ull << 32)) return pl;
+        // the workspace holds two partial column blocks per workgroup, then the operand copies
+        const int mt = size_m <= 16 ? 1 : 2;
+        pl.operand_at = (size_t)G * 2 * size_m * 512;
+        if (pl.operand_at + slabs * rows_operand_elements(size_k, mt) * 2 > ws.partial_bytes) return pl;
+        pl.ok = true;
+        pl.mt = mt;
+        pl.units = (long)U;
+        pl.grid = (unsigned)G;
+        pl.q = q;
+        pl.rem = rem;
+        pl.S = S;
+        pl.lds = lds;
+        return pl;
+    }
+    return pl;
+}
+
+bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, int size_n)
+{
+    return plan_rows(ws, slices, slices, size_m, size_k, size_n).ok;
+}
+
+static void run_rows(const RowsPlan& pl, GemmParams& p, int k_bits, int codebook, hipStream_t stream, std::string& desc)
+{
+    p.cstride = gemm_counter_stride((long)(p.num_slices > 0 ? p.num_slices : 1) * (p.N / 128));
+    p.units = (int)pl.units;
+    p.unit_q = (int)pl.q;
+    p.unit_r = (int)pl.rem;
+    p.m_tr = magic((unsigned)p.K / 64);
+    p.m_nb = magic((unsigned)p.N / 128);
+    p.S = (int)pl.S;
+    p.m_s = pl.S ? magic(pl.S) : 0;
+    p.m_q = pl.S ? 0 : magic(pl.q);
+    p.m_q1 = magic(pl.q + 1);
+    p.lds_bytes = (unsigned)pl.lds;
+    gemm_bits(p, k_bits, codebook, -pl.mt, stream, desc, dim3(pl.grid));
+    hip_ok(hipGetLastError(), "exl3_gemm_rows_kernel launch");
 }
 
 // Tile shape and work split of a dense launch: `nblocks` column blocks of 256 (all slices of
@@ -120,17 +222,32 @@ static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int c
     hip_ok(hipGetLastError(), "exl3_gemm_kernel launch");
 }
 
-std::string launch_gemm(const LinearArgs& a)
+std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
 {
     if (a.size_k % 128 != 0) throw std::runtime_error("exl3 linear: size_k must be a multiple of 128");
-    LaunchScope scope(a.stream);
-    Workspace& ws = scope.ws;
+    std::optional<LaunchScope> scope;
+    if (!scratch) scope.emplace(a.stream);
+    const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
-    std::string d0 = launch_had_r_128(a.a, a.a_had, a.suh, 1, a.size_m, a.size_k, 0, a.stream);
+    const RowsPlan rows = plan_rows(ws, 1, 1, a.size_m, a.size_k, a.size_n);
+    RotateArgs rot;
+    rot.in = a.a;
+    rot.up = a.a_up;
+    rot.act_out = a.act_out;
+    rot.out = a.a_had;
+    rot.suh_host = &a.suh;
+    rot.rows = a.size_m;
+    rot.cols = a.size_k;
+    rot.stream = a.stream;
+    if (rows.ok) {
+        rot.operand = (char*)ws.partials + rows.operand_at;
+        rot.mt = rows.mt;
+    }
+    std::string d0 = launch_rotate(rot);
     GemmParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
-    p.a_had[0] = (const _Float16*)a.a_had;
+    p.a_had[0] = (const _Float16*)(rows.ok ? rot.operand : a.a_had);
     p.lin.trellis = (const uint32_t*)a.trellis;
     p.lin.svh = (const _Float16*)a.svh;
     p.c[0] = a.c;
@@ -141,7 +258,8 @@ std::string launch_gemm(const LinearArgs& a)
     p.partials = ws.partials;
     p.counters = ws.counters;
     std::string desc;
-    dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (a.size_n + 255) / 256, a.stream, desc);
+    if (rows.ok) run_rows(rows, p, a.k_bits, a.codebook, a.stream, desc);
+    else dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (a.size_n + 255) / 256, a.stream, desc);
     return d0 + " + " + desc + (a.out_fp32 ? " out=f32" : " out=f16");
 }
 
@@ -157,11 +275,14 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
     Workspace& ws = scope.ws;
     throw_pending_device_fault(ws);
     const int slabs = sliced ? m.num_had_src : m.bszm_out;
-    const size_t slab_stride = (size_t)m.size_m * m.size_k;
+    const RowsPlan rows = plan_rows(ws, m.bszm_out, slabs, m.size_m, m.size_k, m.size_n);
+    // what the kernel multiplies: the rotated rows, or their copy in operand order
+    const size_t slab_stride = rows.ok ? rows_operand_elements(m.size_k, rows.mt) : (size_t)m.size_m * m.size_k;
+    const _Float16* const slab0 = (const _Float16*)(rows.ok ? (char*)ws.partials + rows.operand_at : m.a_had);
     GemmParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
-    p.a_had[0] = (const _Float16*)m.a_had;
+    p.a_had[0] = slab0;
     p.c[0] = m.c;
     p.M = m.size_m;
     p.K = m.size_k;
@@ -190,12 +311,12 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
                 g.c = (void*)((const uint64_t*)m.c_ptrs)[i];
                 g.width = m.size_n_list[i];
                 g.n_stride = m.n_stride_list[i];
-                g.a_had = (const _Float16*)m.a_had + (size_t)src * slab_stride;
+                g.a_had = slab0 + (size_t)src * slab_stride;
             } else {
                 g.c = (char*)m.c + (size_t)i * m.size_m * m.size_n * (m.c_fp32 ? 4 : 2);
                 g.width = m.size_n;
                 g.n_stride = m.size_n;
-                g.a_had = (const _Float16*)m.a_had + (size_t)i * slab_stride;
+                g.a_had = slab0 + (size_t)i * slab_stride;
             }
         }
     } else {
@@ -208,13 +329,27 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
             p.had_src_list = m.had_src_list;
         }
     }
-    const size_t in_stride = (!sliced && m.bszm_in > 1) ? slab_stride : 0;
-    std::string d0 = launch_had_r_128_slabs(m.a, in_stride, m.a_had, slab_stride, m.host_lists ? nullptr : m.suh_list,
-                                            suh_host, slabs, m.size_m, m.size_k, m.stream);
+    RotateArgs rot;
+    rot.in = m.a;
+    rot.in_stride = (!sliced && m.bszm_in > 1) ? (size_t)m.size_m * m.size_k : 0;
+    rot.out = m.a_had;
+    rot.out_stride = (size_t)m.size_m * m.size_k;
+    rot.suh_list = m.host_lists ? nullptr : m.suh_list;
+    rot.suh_host = suh_host;
+    rot.slabs = slabs;
+    rot.rows = m.size_m;
+    rot.cols = m.size_k;
+    rot.stream = m.stream;
+    if (rows.ok) {
+        rot.operand = (void*)slab0;
+        rot.mt = rows.mt;
+    }
+    std::string d0 = launch_rotate(rot);
     const long nblocks = (long)m.bszm_out * ((m.size_n + 255) / 256);
     if (nblocks * ((m.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3_mgemm: too many output tiles");
     std::string desc;
-    dispatch_dense(ws, p, m.k_bits, m.codebook, m.size_m, m.size_k, (int)nblocks, m.stream, desc);
+    if (rows.ok) run_rows(rows, p, m.k_bits, m.codebook, m.stream, desc);
+    else dispatch_dense(ws, p, m.k_bits, m.codebook, m.size_m, m.size_k, (int)nblocks, m.stream, desc);
     return std::string(sliced ? "sliced x" : "uniform x") + std::to_string(m.bszm_out) + (m.host_lists ? " by value " : " ") + d0 +
            " + " + desc + (m.c_fp32 ? " out=f32" : " out=f16");
 }
@@ -225,6 +360,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
     LaunchScope scope(a.stream);
     Workspace& ws = scope.ws;
     throw_pending_device_fault(ws);
+    const RowsPlan rows = plan_rows(ws, 2, 2, a.size_m, a.size_k, a.size_n);
     GemmParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
@@ -247,11 +383,26 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
         g.n_stride = a.size_n;
         g.a_had = (const _Float16*)slabs[i];
     }
-    std::string d0 = launch_had_r_128_slabs(a.a, 0, a.a_had, 0, nullptr, a.suh, 2, a.size_m, a.size_k, a.stream, slabs);
+    RotateArgs rot;
+    rot.in = a.a;
+    rot.suh_host = a.suh;
+    rot.out_host = slabs;
+    rot.slabs = 2;
+    rot.rows = a.size_m;
+    rot.cols = a.size_k;
+    rot.stream = a.stream;
+    if (rows.ok) {
+        rot.operand = (char*)ws.partials + rows.operand_at;
+        rot.mt = rows.mt;
+        for (int i = 0; i < 2; ++i)
+            p.slice[i].a_had = (const _Float16*)rot.operand + i * rows_operand_elements(a.size_k, rows.mt);
+    }
+    std::string d0 = launch_rotate(rot);
     const long nblocks = 2L * ((a.size_n + 255) / 256);
     if (nblocks * ((a.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3 linear pair: too many output tiles");
     std::string desc;
-    dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (int)nblocks, a.stream, desc);
+    if (rows.ok) run_rows(rows, p, a.k_bits, a.codebook, a.stream, desc);
+    else dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (int)nblocks, a.stream, desc);
     return "pair " + d0 + " + " + desc + " out=f16";
 }
 

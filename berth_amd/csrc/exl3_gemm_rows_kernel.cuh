@@ -1,0 +1,382 @@
+// EXL3 linear for a few rows (2..32): every weight is decoded once and multiplied on the matrix
+// units, as a single resident round of sixteen-wave workgroups.
+//
+//   c = Hh(a_had @ W) * svh (+ out_add),   a_had = Hh(a * suh) rotated by an earlier launch
+//
+// What bounds it: the decode (about 4.0 vector instructions per weight, 124 for the 32 weights a
+// lane takes per step); the four v_mfma_f32_16x16x32_f16 of a step and 16 rows need 64 of the
+// 496 cycles that the decode takes, so rows up to 32 cost little more than one.
+//
+//   * A unit of work is 64 rows of K x 128 columns, column block major.  The launch's units are
+//     dealt out evenly to the workgroups (one per compute unit), whatever the shape is: no
+//     second round, no tail.  Few column blocks: each is cut into S parts of its own instead,
+//     so that no workgroup hands over two of them.
+//   * Of a workgroup's sixteen waves four share a unit (32 columns each) and four such groups
+//     take a contiguous quarter of the units each.  A wave walks its quarter alone: no barrier
+//     in the loop, two units of trellis and activation in registers, and the walk crosses
+//     column blocks without draining them.
+//   * Operands: 16 lanes cover 2 tiles (32 columns) of one tile row in the octet layout, the
+//     four lane groups four tile rows.  The four register quads a lane decodes (column u or u + 8,
+//     k 0..7 or 8..15 of its tile row) are four B operands of the 16x16x32 form, with k slot
+//     8 * group + i standing for k = 16 * group + 8h + i.  The A operand of the same slots is 16
+//     bytes of a rotated row.  The rotation leaves a second copy of its result in operand order
+//     (rows_operand_offset), so a wave reads an operand as 1 KB in a row; from the row-major copy
+//     the same loads touch a line per lane and cost the launch a third of its time.  All column
+//     groups of a compute unit read the same operands at about the same time, from its L1.
+//   * A wave leaves its part of a column block in LDS, in fp32; the parts are added in k order.
+//     A column block that lies inside one workgroup's units is finished there.  Otherwise the
+//     sharers leave their sums in the workspace and the last to arrive adds them in k order, so
+//     results repeat bit for bit.
+//
+// Measured (27B layer, traced): gate + up at 5 rows and 3 bits 62.6 -> 32.5 us against the VALU
+// kernel, at 24 rows and 4 bits 49.0 -> 40.6 against 32-row tiles (whose 544 workgroups also
+// ran in one and a bit rounds), down 47.4 -> 19.1 and 38 -> 23.0.  Of the 41 us at 24 rows the
+// vector pipes issue for 65 %, the MFMAs take 13 %, 4 us are launch, head and hand-over.
+#pragma once
+
+#include "exl3_gemm_kernel.cuh"
+
+namespace berth {
+
+constexpr int kRowsWaves = 16;
+constexpr int kRowsStride = 132;            // floats per row of a partial column block in LDS
+
+// dynamic LDS of a launch: the pieces, the output scales of the column blocks, two flags
+__host__ __device__ constexpr size_t rows_lds_bytes(int rows, int ncb)
+{
+    return (size_t)(ncb + 3) * rows * kRowsStride * 4 + (size_t)ncb * 256 + 16;
+}
+
+// the tensors of one 128-column block of the launch
+struct RowsBlock {
+    const uint32_t* trellis;    // of the linear (of the whole weight's slice)
+    const _Float16* svh;
+    const _Float16* a_had;      // the rotated input in operand order
+    void* c;
+    int n0;                     // first column inside the linear
+    int ldc;                    // elements between output rows, and columns of the weight
+    bool empty;                 // past the end of a narrower slice: nothing to compute
+};
+__device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsigned cb)
+{
+    RowsBlock b;
+    b.trellis = p.lin.trellis;
+    b.svh = p.lin.svh;
+    b.a_had = p.a_had[0];
+    b.c = p.c[0];
+    b.n0 = (int)cb * 128;
+    b.ldc = p.N;
+    b.empty = false;
+    if (p.num_slices > 0) {
+        const unsigned nb = (unsigned)p.N >> 7;
+        const unsigned sl = __umulhi(cb, p.m_nb);
+        b.n0 = (int)(cb - sl * nb) * 128;
+        int width = p.N;
+        if (p.b_list) {
+            unsigned slab = sl;
+            b.trellis = (const uint32_t*)p.b_list[sl];
+            b.svh = (const _Float16*)p.svh_list[sl];
+            if (p.c_ptrs) {
+                width = p.size_n_list[sl];
+                b.ldc = p.n_stride_list[sl];
+                slab = (unsigned)p.had_src_list[sl];
+                b.c = (void*)p.c_ptrs[sl];
+            } else {
+                b.c = (char*)p.c[0] + (size_t)sl * p.M * p.N * (p.out_fp32 ? 4 : 2);
+            }
+            b.a_had = p.a_had[0] + (size_t)slab * p.slab_stride;
+        } else {
+            const GemmSlice& g = p.slice[sl];
+            b.trellis = g.trellis;
+            b.svh = g.svh;
+            b.c = g.c;
+            width = g.width;
+            b.ldc = g.n_stride;
+            b.a_had = g.a_had;
+        }
+        b.empty = b.n0 >= width;
+    }
+    return b;
+}
+
+template <typename T>
+__device__ __forceinline__ const T* rows_uniform(const T* q)
+{
+    const uint64_t v = (uint64_t)q;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (const T*)(((uint64_t)hi << 32) | lo);
+}
+
+template <int BITS, int CB, int MT>         // MT: tiles of 16 rows
+__global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int tile_dw = 8 * BITS;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cg = wave & 3, kg = wave >> 2;
+    const int l16 = lane & 15, lg = lane >> 4;
+    const unsigned TR4 = (unsigned)p.K >> 6;            // units per column block
+    const int M = p.M;
+
+    // ---- this workgroup's units [u0, u1), this wave's quarter [w0, w1)
+    const unsigned w = blockIdx.x;
+    const unsigned q = (unsigned)p.unit_q, rem = (unsigned)p.unit_r;
+    const unsigned S = (unsigned)p.S;
+    unsigned u0 = w * q + min(w, rem), u1 = (w + 1) * q + min(w + 1, rem);
+    if (S) {
+        const unsigned blk = __umulhi(w, p.m_s), part = w - blk * S;
+        u0 = blk * TR4 + __umulhi(part * TR4, p.m_s);
+        u1 = blk * TR4 + __umulhi((part + 1) * TR4, p.m_s);
+    }
+    const unsigned L = u1 - u0;
+    const unsigned cb_first = __umulhi(u0, p.m_tr), cb_last = __umulhi(u1 - 1, p.m_tr);
+    const unsigned ncb = cb_last - cb_first + 1;
+    const unsigned w0 = u0 + (L * (unsigned)kg >> 2), w1 = u0 + (L * (unsigned)(kg + 1) >> 2);
+
+    float* const red = (float*)smem;
+    uint32_t* const sv_lds = (uint32_t*)(red + (size_t)(ncb + 3) * M * kRowsStride);
+    unsigned* const flags = sv_lds + ncb * 64;
+
+    // ---- the walk's operands: a pointer pair that runs two units ahead of the decode
+    unsigned f_cb = __umulhi(w0, p.m_tr);
+    unsigned f_k = w0 - f_cb * TR4, f_left = w1 - w0;
+    const char* f_t;
+    const char* f_a;
+    long f_step;
+    uint32_t t_off;                                     // bytes, per lane
+    const uint32_t a_off = (uint32_t)lane * 16;
+    constexpr int kUnitA = MT * 2 * 1024;               // bytes of A operands per unit
+    auto seek = [&](unsigned cb, unsigned k) {
+        const RowsBlock b = rows_block(p, cb);
+        if (b.empty) {                                  // read anything valid, use nothing
+            f_t = (const char*)rows_uniform(b.a_had);
+            f_step = 0;
+            t_off = 0;
+        } else {
+            const uint32_t row_bytes = (uint32_t)(b.ldc >> 4) * (tile_dw * 4);
+            f_step = 4 * (long)row_bytes;
+            f_t = (const char*)rows_uniform(b.trellis) + (size_t)(b.n0 >> 4) * (tile_dw * 4) + (size_t)(4 * k) * row_bytes;
+            t_off = (uint32_t)lg * row_bytes + (uint32_t)(cg * 16 + l16) * (BITS * 4);
+        }
+        f_a = (const char*)rows_uniform(b.a_had) + (size_t)k * kUnitA;
+    };
+    seek(f_cb, f_k);
+
+    uint32_t own[2][BITS];
+    half8_t av[2][MT][2];
+    auto fetch_t = [&](int j) { load_tile_dwords<BITS>((global_ptr<const uint32_t>)(as_global(f_t) + t_off), own[j]); };
+    auto fetch_a = [&](int j) {
+        const global_ptr<const half8_t> src = (global_ptr<const half8_t>)(as_global(f_a) + a_off);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            av[j][mt][0] = src[(2 * mt) * 64];
+            av[j][mt][1] = src[(2 * mt + 1) * 64];
+        }
+    };
+    auto advance = [&]() {                              // on the last unit it stays: read again, not used
+        if (f_left > 1) {
+            --f_left;
+            f_t += f_step;
+            f_a += kUnitA;
+            if (++f_k == TR4) {
+                f_k = 0;
+                ++f_cb;
+                seek(f_cb, 0);
+            }
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        fetch_t(j);
+        fetch_a(j);
+        advance();
+    }
+    // the output scales, asked for now: the finish does not wait for them
+    uint32_t sv_mine = 0;
+    if ((unsigned)wave < ncb) {
+        const RowsBlock b = rows_block(p, cb_first + (unsigned)wave);
+        if (!b.empty) sv_mine = as_global((const uint32_t*)(b.svh + b.n0))[lane];
+    }
+
+    float4_t acc[MT][2];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    unsigned cb = __umulhi(w0, p.m_tr);
+    unsigned k = w0 - cb * TR4;
+    // piece of (quarter, column block): the quarters are consecutive runs, so kg + (cb - cb_first)
+    // names each of them once
+    auto flush = [&]() {
+        float* const piece = red + (size_t)((unsigned)kg + cb - cb_first) * M * kRowsStride;
+        const int col = cg * 32 + (l16 >> 3) * 16 + (l16 & 7);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = mt * 16 + 4 * lg + r;
+                if (row < M) {
+                    piece[row * kRowsStride + col] = acc[mt][0][r];
+                    piece[row * kRowsStride + col + 8] = acc[mt][1][r];
+                }
+            }
+    };
+    // The registers of a step are reloaded as soon as they have been used, the trellis behind the
+    // decode and the A operands behind the MFMAs; the barriers keep the compiler from issuing the
+    // loads ahead of that into other registers, which costs a move per register and step.
+    auto stage = [&](int j) {
+        const uint32_t prev = fetch_prev(lane, own[j][BITS - 1]);
+        uint32_t w2[16];
+        decode_lane<BITS, CB>(own[j], prev, w2);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_t(j);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const uint4 bq = {w2[2 * f + h], w2[4 + 2 * f + h], w2[8 + 2 * f + h], w2[12 + 2 * f + h]};
+                const half8_t b = __builtin_bit_cast(half8_t, bq);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    acc[mt][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[j][mt][h], b, acc[mt][f], 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_a(j);
+        advance();
+        if (++k == TR4) {
+            flush();
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            ++cb;
+            k = 0;
+        }
+    };
+    const unsigned pairs = (w1 - w0) >> 1;
+    for (unsigned g = 0; g < pairs; ++g) {
+        stage(0);
+        stage(1);
+    }
+    if ((w1 - w0) & 1) stage(0);
+    if (k != 0) flush();
+    if ((unsigned)wave < ncb) sv_lds[wave * 64 + lane] = sv_mine;
+    __syncthreads();
+
+    // ---- finish: a wave takes (column block, row) vectors, two columns a lane
+    auto store_row = [&](const RowsBlock& b, unsigned cbi, int row, float z0, float z1) {
+        had128_wave(z0, z1, lane);
+        const half2_t sv = as_half2(sv_lds[cbi * 64 + lane]);
+        z0 = (z0 * kRsqrt128) * (float)sv.x;
+        z1 = (z1 * kRsqrt128) * (float)sv.y;
+        const size_t at = (size_t)row * b.ldc + b.n0 + 2 * lane;
+        if (p.out_fp32) {
+            if (p.out_add) {
+                const float2_t add = *(global_ptr<const float2_t>)(as_global(p.out_add) + at);
+                z0 += add.x;
+                z1 += add.y;
+            }
+            *(global_ptr<float2_t>)(as_global((float*)b.c) + at) = float2_t{z0, z1};
+        } else {
+            half2_t o;
+            o.x = (_Float16)z0;
+            o.y = (_Float16)z1;
+            *(global_ptr<half2_t>)(as_global((_Float16*)b.c) + at) = o;
+        }
+    };
+    const bool first_shared = !(u0 == cb_first * TR4 && u1 >= (cb_first + 1) * TR4);
+    const bool last_shared = ncb > 1 && u1 < (cb_last + 1) * TR4;
+    int row = wave;
+    unsigned cbi = 0;
+    const unsigned qs1 = u0 + (L >> 2), qs2 = u0 + (L * 2 >> 2), qs3 = u0 + (L * 3 >> 2);
+    while (true) {
+        while (row >= M) {
+            row -= M;
+            ++cbi;
+        }
+        if (cbi >= ncb) break;
+        const unsigned cbx = cb_first + cbi;
+        const unsigned c0 = cbx * TR4, c1 = c0 + TR4;
+        const RowsBlock b = rows_block(p, cbx);
+        if (!b.empty) {
+            float z0 = 0.0f, z1 = 0.0f;
+            const float* const base = red + (size_t)cbi * M * kRowsStride + row * kRowsStride + 2 * lane;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const unsigned a0 = g == 0 ? u0 : g == 1 ? qs1 : g == 2 ? qs2 : qs3;
+                const unsigned a1 = g == 0 ? qs1 : g == 1 ? qs2 : g == 2 ? qs3 : u1;
+                if (a0 < c1 && a1 > c0) {
+                    const float2_t part = *(const float2_t*)(base + (size_t)g * M * kRowsStride);
+                    z0 += part.x;
+                    z1 += part.y;
+                }
+            }
+            if ((cbi == 0 && first_shared) || (cbi == ncb - 1 && last_shared)) {
+                unsigned long long* const slot =
+                    (unsigned long long*)(p.partials + ((size_t)w * 2 + (cbi == 0 ? 0 : 1)) * M * 128 + row * 128) + lane;
+                __hip_atomic_store(slot, __builtin_bit_cast(unsigned long long, float2_t{z0, z1}), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+                store_row(b, cbi, row, z0, z1);
+            }
+        }
+        row += kRowsWaves;
+    }
+    if (!first_shared && !last_shared) return;
+
+    // ---- shared column blocks (the first and the last of the range at most): count this
+    // workgroup in; the last sharer to arrive adds the parts in k order and finishes the block
+    auto owner = [&](unsigned x) {
+        const unsigned big = rem * (q + 1);
+        if (S) return __umulhi(x, p.m_tr) * S + (x % TR4 ? S - 1 : 0u);     // asked for a block's first or last unit
+        return x < big ? __umulhi(x, p.m_q1) : rem + __umulhi(x - big, p.m_q);
+    };
+    wait_own_stores();
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned done = 0;
+        if (threadIdx.x == 0 ? first_shared : last_shared) {
+            const unsigned cbx = threadIdx.x == 0 ? cb_first : cb_last;
+            const unsigned parts = owner(cbx * TR4 + TR4 - 1) - owner(cbx * TR4) + 1;
+            unsigned* const counter = p.counters + (size_t)cbx * p.cstride;
+            const unsigned old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (old == parts - 1) {
+                __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                done = 1;
+            }
+        }
+        flags[threadIdx.x] = done;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int t = 0; t < 2; ++t) {
+        if (!__builtin_amdgcn_readfirstlane((int)flags[t])) continue;
+        const unsigned cbx = t == 0 ? cb_first : cb_last;
+        const RowsBlock b = rows_block(p, cbx);
+        if (b.empty) continue;
+        const unsigned wa = owner(cbx * TR4), wb = owner(cbx * TR4 + TR4 - 1);
+        // the block is the first of every sharer's range but, unless that starts with it, the first sharer's
+        const unsigned slot_a = S || wa * q + min(wa, rem) >= cbx * TR4 ? 0u : 1u;
+        for (int r = wave; r < M; r += kRowsWaves) {
+            float z0 = 0.0f, z1 = 0.0f;
+            for (unsigned x = wa; x <= wb; x += 8) {
+                float2_t part[8];
+#pragma unroll
+                for (unsigned i = 0; i < 8; ++i) {
+                    const unsigned xi = min(x + i, wb);
+                    const unsigned long long* const src =
+                        (const unsigned long long*)(p.partials + ((size_t)xi * 2 + (xi == wa ? slot_a : 0u)) * M * 128 +
+                                                    r * 128) + lane;
+                    part[i] = __builtin_bit_cast(float2_t, __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                }
+#pragma unroll
+                for (unsigned i = 0; i < 8; ++i)
+                    if (x + i <= wb) {
+                        z0 += part[i].x;
+                        z1 += part[i].y;
+                    }
+            }
+            store_row(b, cbx - cb_first, r, z0, z1);
+        }
+    }
+}
+
+}  // namespace berth

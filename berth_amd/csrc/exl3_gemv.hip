@@ -198,6 +198,15 @@ static void pick_units(const Workspace& ws, GemvParams& p, long units, int mmax)
     p.S = pick_split(ws, units, p.KB, mmax);
 }
 
+// Two to eight rows of a weight large enough for the few-row MFMA kernel go there: it decodes as
+// fast as the one-row kernel and its dot products cost nothing beside that, where the kernel of
+// this file pays half an instruction per weight and row.  A launch width chosen by hand
+// (BERTH_GEMV_WG_PER_CU) keeps the kernel that it tunes.
+static bool rows_on_matrix_units(const Workspace& ws, int problems, int size_m, int size_k, int size_n)
+{
+    return size_m > 1 && knobs().gemv_wg_per_cu <= 0 && gemm_rows_applies(ws, problems, size_m, size_k, size_n);
+}
+
 std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
 {
     if (a.size_m < 1 || a.size_m > 8) throw std::runtime_error("exl3 gemv: rows must be in 1..=8");
@@ -207,6 +216,10 @@ std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
     const int mmax = a.size_m == 1 ? 1 : 8;
+    if (rows_on_matrix_units(ws, 1, a.size_m, a.size_k, a.size_n)) {
+        scope.reset();          // the MFMA launcher holds its own
+        return launch_gemm(a, scratch);
+    }
     if (a.size_m == 1) {
         const StreamPlan pl = plan_stream(ws, 1, a.size_k, a.size_n);
         if (pl.ok) {
@@ -253,6 +266,11 @@ std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
     return "exl3_gemv_kernel<" + std::to_string(a.k_bits) + "," + std::to_string(a.codebook) + "," +
            std::to_string(mmax) + (a.a_up ? ",silu" : "") + "> grid=" + std::to_string(grid) + " block=256 split_k=" +
            std::to_string(p.S) + (p.half_units ? "/half" : "") + (a.out_fp32 ? " out=f32" : " out=f16");
+}
+
+bool gemv_rows_on_matrix_units(int problems, int size_m, int size_k, int size_n)
+{
+    return rows_on_matrix_units(workspace_for_current_device(), problems, size_m, size_k, size_n);
 }
 
 std::string launch_gemv_pair(const PairArgs& a)
@@ -325,6 +343,8 @@ std::string launch_mgemm(const MgemmArgs& m)
 {
     if (m.size_k % 128 != 0) throw std::runtime_error("exl3_mgemm: size_k must be a multiple of 128");
     if (m.size_m > 8) return launch_gemm_bundle(m);
+    if (!m.host_lists && rows_on_matrix_units(workspace_for_current_device(), m.bszm_out, m.size_m, m.size_k, m.size_n))
+        return launch_gemm_bundle(m);
     LaunchScope scope(m.stream);
     Workspace& ws = scope.ws;
     throw_pending_device_fault(ws);

@@ -25,6 +25,7 @@
 #include "exl3_decode.cuh"
 #include "hadamard.cuh"
 #include "moe_route.cuh"
+#include "silu.cuh"
 
 namespace berth {
 
@@ -111,17 +112,6 @@ struct GemvParams {
 };
 
 constexpr int kCombMaxProblems = 16;
-
-// silu(g) * u with every step rounded to fp16: e = exp(-g); s = 1 + e; r = 1 / s;
-// t = g * r; out = t * u (crates/berth-kernels/csrc/ops/act.cu:35-69 and its fixture)
-__device__ __forceinline__ _Float16 silu_mul_h(_Float16 g, _Float16 u)
-{
-    _Float16 e = (_Float16)expf(-(float)g);
-    _Float16 s = (_Float16)1.0f + e;
-    _Float16 r = (_Float16)(1.0f / (float)s);
-    _Float16 t = g * r;
-    return t * u;
-}
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));

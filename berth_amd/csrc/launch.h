@@ -73,6 +73,7 @@ struct Knobs {
     int gemm_wg_per_cu;         // BERTH_GEMM_WG_PER_CU
     int gemm_balanced;          // BERTH_GEMM_BALANCED
     int gemm_rows256;           // BERTH_GEMM_ROWS256
+    int gemm_rows_units;        // BERTH_GEMM_ROWS_UNITS        fewest units for which the few-row kernel is taken (0: never, -1: by row count)
     int counter_stride;         // BERTH_COUNTER_STRIDE         cap on the words between arrival counters (1..32)
     int moe_big_min;            // BERTH_MOE_BIG_MIN
     int moe_route_slab;         // BERTH_MOE_ROUTE_SLAB: 0 keeps the two-launch routing of many tokens
@@ -133,7 +134,8 @@ struct LinearArgs {
     const void* svh;
     int size_m, size_k, size_n, k_bits, codebook, out_fp32;
     hipStream_t stream;
-    const void* a_up = nullptr;   // VALU kernel only: the input is silu(a) * a_up, element by element
+    const void* a_up = nullptr;   // the input is silu(a) * a_up, element by element
+    void* act_out = nullptr;      // with a_up, MFMA kernels only: where that input also goes (may be a_up)
     const float* out_add = nullptr;   // streaming kernel only (one row, fp32 output): a row added to the output
 };
 
@@ -164,6 +166,9 @@ std::string launch_gemv_pair(const PairArgs& args);
 // whether a one-row launch of `problems` linears of this shape takes the streaming kernel (and,
 // with whole_rows, whether every workgroup of it then holds the whole input row)
 bool gemv_stream_applies(int problems, int size_k, int size_n, bool whole_rows);
+
+// whether 2..8 rows of `problems` linears of this shape run on the few-row MFMA kernel
+bool gemv_rows_on_matrix_units(int problems, int size_m, int size_k, int size_n);
 
 // grouped (MoE) launches: problems, experts and num_problems are device memory
 struct GroupedArgs {
@@ -238,12 +243,27 @@ struct MgemmArgs {
 std::string launch_mgemm(const MgemmArgs& args);
 // more than 8 rows: the bundle as one dense MFMA launch
 std::string launch_gemm_bundle(const MgemmArgs& args);
-// out slab s = Hh(in(s) * suh(s)) for s < slabs (fp16; in(s) = in + s * in_stride, out slabs
-// out_stride elements apart, or at out_host[s] when that is given with a null list); suh(s) from
-// the device list, or from the host array when the list is null
-std::string launch_had_r_128_slabs(const void* in, size_t in_stride, void* out, size_t out_stride, const void* suh_list,
-                                   const void* const* suh_host, int slabs, int rows, int cols, hipStream_t stream,
-                                   void* const* out_host = nullptr);
+// Rotated inputs in one launch: out slab s = Hh(in(s) * suh(s)) for s < slabs, with in(s) = in +
+// s * in_stride and the slabs out_stride elements apart (or at out_host[s], by-value scales only);
+// suh(s) from the device list, or from the host array when the list is null.  With `up` the input
+// is silu(in) * up, which also goes to act_out unless null.  `operand` (optional): a second copy in
+// the operand order of the few-row kernel, for mt tiles of 16 rows.
+struct RotateArgs {
+    const void* in = nullptr;
+    size_t in_stride = 0;
+    void* out = nullptr;
+    size_t out_stride = 0;
+    const void* suh_list = nullptr;
+    const void* const* suh_host = nullptr;
+    void* const* out_host = nullptr;
+    int slabs = 1, rows = 0, cols = 0;
+    hipStream_t stream = nullptr;
+    const void* up = nullptr;
+    void* act_out = nullptr;
+    void* operand = nullptr;
+    int mt = 1;
+};
+std::string launch_rotate(const RotateArgs& args);
 // gate and up of an MLP above 8 rows as one bundle: two linears of one shape on one input, each
 // with its own output and its own buffer for the rotated input
 std::string launch_gemm_pair(const PairArgs& pair, void* a_had_second);
@@ -253,7 +273,9 @@ constexpr int kBundleMaxSlices = 16;    // slices of a bundle whose lists travel
 // split-K scratch to use instead of the device's lazily allocated workspace.
 std::string launch_gemv(const LinearArgs& args, const Workspace* scratch = nullptr);
 // any row count: fp16 MFMA kernel (rows padded to 32 inside the kernel).
-std::string launch_gemm(const LinearArgs& args);
+std::string launch_gemm(const LinearArgs& args, const Workspace* scratch = nullptr);
+// whether a launch of this many linears of one shape takes the few-row kernel (2..32 rows)
+bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, int size_n);
 // trellis -> fp16 [K][slice_n] (row stride slice_n), columns n_offset.. of a
 // [K][full_n] weight
 std::string launch_reconstruct(void* unpacked, const void* packed, int size_k, int slice_n,

@@ -1,0 +1,79 @@
+"""The few-row MFMA kernel (2..32 rows, units of 64 x 128 weights dealt out evenly) at the sizes
+where its split can go wrong, against the oracle: one and two tiles of 16 rows with and without
+a remainder, the smallest launch there is, ranges that start or end on a column block, ranges
+that touch many column blocks (shallow weights, several rounds of workgroups), odd numbers of
+k-blocks, narrower slices of a bundle.  Bar: rtol 2e-3 / atol 1e-3 of the oracle's fp32 sums;
+a second call gives the same bits."""
+import numpy as np
+import pytest
+import torch
+
+from berth_amd import kernels as K
+from berth_amd import synth
+from berth_amd.kernels import Codebook, OutDtype
+from oracle import oracle as O
+from tests.gpu_util import DEV, close, dev, host_f16, host_u16, knobs
+from tests.test_gpu_linear import _run_linear
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _every_size():
+    """The kernel at every size it can serve, not only where it is the faster one."""
+    with knobs(BERTH_GEMM_ROWS_UNITS=1):
+        yield
+
+
+@pytest.mark.parametrize("rows,Kk,N,bits,cb", [
+    (2, 128, 256, 4, 2),            # four units: one workgroup, one unit per wave group
+    (3, 1408, 640, 4, 2),           # 110 units
+    (5, 5120, 1024, 3, 1),          # ranges shared by many workgroups
+    (8, 1152, 4864, 5, 0),          # nine k-blocks
+    (16, 4096, 2048, 2, 2),         # a full tile; every range starts and ends on a unit of its own block
+    (17, 2176, 3200, 6, 2),         # second tile with one row
+    (32, 2048, 4096, 8, 2),
+    (31, 128, 128 * 2600, 1, 2),    # shallow: ranges of many column blocks, two rounds of workgroups
+    (9, 16384, 512, 7, 1),          # deep and narrow: one column block over most of the launch
+])
+def test_few_rows_match_the_oracle_and_repeat(rows, Kk, N, bits, cb):
+    got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, bits, cb, True, 40 + rows, prefill=True)
+    assert "exl3_gemm_kernel/rows" in launch, launch
+    assert np.array_equal(ah, want_ah), launch
+    bad, worst = close(got, want)
+    assert bad == 0, (bad, worst, launch)
+    again = _run_linear(rows, Kk, N, bits, cb, True, 40 + rows, prefill=True)[0]
+    assert np.array_equal(got.view(np.uint8), again.view(np.uint8)), launch
+
+
+@pytest.mark.parametrize("rows", [3, 20])
+def test_bundle_with_narrower_slices(rows):
+    """Sliced lists whose widths differ (the last one a single column block): blocks past a
+    slice's end are empty and touch nothing."""
+    Kk, width, widths, bits = 1024, 1664, (1664, 640, 128, 1664), 4
+    lins = [synth.linear(600 + i, Kk, n, bits) for i, n in enumerate(widths)]
+    d = [[dev(t.view(np.uint16)) for t in lin] for lin in lins]
+    x = synth.activations(610 + rows, rows, Kk)
+    outs = [torch.full((rows, n), 5.0, dtype=torch.float16, device=DEV) for n in widths]
+    i64 = lambda v: torch.tensor(v, dtype=torch.int64, device=DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    lists = [i64([dd[j].data_ptr() for dd in d]) for j in range(3)]
+    c_ptrs, n_list, src = i64([o.data_ptr() for o in outs]), i32(list(widths)), i32([0, 1, 2, 3])
+    a_had = torch.zeros((4, rows, Kk), dtype=torch.float16, device=DEV)
+    d_x = dev(x.view(np.uint16))
+    K.ops.exl3_mgemm(d_x.data_ptr(), lists[0].data_ptr(), outs[0].data_ptr(), lists[1].data_ptr(), a_had.data_ptr(),
+                     lists[2].data_ptr(), rows, Kk, width, bits, Codebook.MUL1, OutDtype.F16, 1, 4, n_list.data_ptr(),
+                     c_ptrs.data_ptr(), n_list.data_ptr(), src.data_ptr(), 4)
+    torch.cuda.synchronize()
+    assert "exl3_gemm_kernel/rows" in K.ops.last_launch(), K.ops.last_launch()
+    for i, (tr, suh, svh) in enumerate(lins):
+        want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=False)
+        assert close(host_f16(outs[i]), want)[0] == 0, i
+        assert np.array_equal(host_u16(a_had).reshape(4, -1)[i], want_had.view(np.uint16).reshape(-1)), i
+
+
+@pytest.mark.parametrize("rows", [4, 12])
+def test_mlp_of_few_rows_stage_by_stage(rows):
+    from tests.test_gpu_mlp import run_mlp_block
+    launch = run_mlp_block(rows, 1536, 4096, 4)
+    assert launch.count("exl3_gemm_kernel/rows") == 2 and "silu_mul_had_r_128_kernel" in launch, launch
