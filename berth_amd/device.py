@@ -12,6 +12,10 @@ import torch
 from . import kernels as K
 from .kernels import Codebook, OutDtype
 
+# torch's handle of a device's current stream, without the Stream object around it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+    (lambda index: torch.cuda.current_stream(index).cuda_stream)
+
 MAX_RECONSTRUCT_N = 32768   # crates/berth-engine/src/device.rs:193
 
 
@@ -53,12 +57,15 @@ class Gpu:
         self.device = torch.device("cuda", device)
         torch.cuda.set_device(self.device)
         self.stream = torch.cuda.current_stream(self.device)
+        self._index = device
         self.sm_count = K.device_sms(device)
 
     def raw_stream(self):
         """The stream launches go on: torch's current stream of the device (the one
-        captured when a HIP graph is being recorded)."""
-        return torch.cuda.current_stream(self.device).cuda_stream or None
+        captured when a HIP graph is being recorded).  The handle straight from torch: a
+        Stream object made for every launch costs 1.8 us of host time, a quarter of what a
+        one-row linear takes to issue."""
+        return _raw_stream(self._index) or None
 
     def zeroed(self, nbytes: int) -> torch.Tensor:
         return torch.zeros(nbytes, dtype=torch.uint8, device=self.device)
@@ -286,6 +293,8 @@ class Exl3MultiLinear:
                    "size_n": np.array([width] * len(b), dtype=np.int32), "stride": np.array(stride, dtype=np.int32),
                    "src": np.array(src, dtype=np.int32)}
         self._h_c = None
+        self._h_at = {name: array.ctypes.data for name, array in self._h.items()}    # addresses, looked up once
+        self._h_c_at = 0
         self.host_lists = self.slices <= 16
 
     def forward(self, gpu: Gpu, a: torch.Tensor, outs: list[torch.Tensor], out: OutDtype, rows: int = 1,
@@ -302,16 +311,16 @@ class Exl3MultiLinear:
             ptrs = [outs[s].data_ptr() + n0 * esz for s, n0 in zip(self._src, self._n0)]
             self._c_ptrs = torch.tensor(ptrs, dtype=torch.int64, device=gpu.device)
             self._h_c = np.array(ptrs, dtype=np.uint64)
+            self._h_c_at = self._h_c.ctypes.data
             self._c_key = key
         # lists by value: one row through the streaming kernel, more than 8 rows through the MFMA
         # kernels (2..8 rows read the device lists)
         if by_value and ((rows == 1 and self.host_lists) or (rows > 8 and self.slices <= 16)):
-            h = self._h
+            h = self._h_at
             try:
-                K.ops.exl3_mgemm_hostlists(ptr(a), h["b"].ctypes.data, ptr(outs[0]), h["suh"].ctypes.data, ptr(self.a_had),
-                                           h["svh"].ctypes.data, rows, self.size_k, self.width, self.k_bits, self.codebook,
-                                           out, 1, self.slices, h["size_n"].ctypes.data, self._h_c.ctypes.data,
-                                           h["stride"].ctypes.data, h["src"].ctypes.data, len(self.sources),
+                K.ops.exl3_mgemm_hostlists(ptr(a), h["b"], ptr(outs[0]), h["suh"], ptr(self.a_had), h["svh"], rows,
+                                           self.size_k, self.width, self.k_bits, self.codebook, out, 1, self.slices,
+                                           h["size_n"], self._h_c_at, h["stride"], h["src"], len(self.sources),
                                            gpu.raw_stream())
                 return
             except K.LaunchError as err:
@@ -337,6 +346,9 @@ class MlpLayer:
         self.g = torch.zeros(max_rows * self.intermediate, dtype=torch.float16, device=gpu.device)
         self.u = torch.zeros(max_rows * self.intermediate, dtype=torch.float16, device=gpu.device)
         self.x_had = self.act_had = None      # rotated inputs of the fused call, allocated on first use
+        self.h_norm = None                    # normed input of the block call, likewise
+        self._lins_key = self._lins = None    # the argument table of the one-call paths, kept between calls
+        self._norm_key = self._norm = None
         # the one-call path takes one bit rate and codebook for the three linears
         self.uniform = gate.k_bits == up.k_bits == down.k_bits and gate.codebook == up.codebook == down.codebook
         self.has_bias = any(l.bias is not None for l in (gate, up, down))
@@ -361,6 +373,15 @@ class MlpLayer:
             raise WeightsError(f"{prefix}: intermediate {gate.size_n} must be positive and even")
         return cls(gpu, gate, up, down, max_rows)
 
+    def _lin_table(self):
+        g, u, d = self.gate, self.up, self.down
+        key = (ptr(g.trellis), ptr(g.suh), ptr(g.svh), ptr(u.trellis), ptr(u.suh), ptr(u.svh),
+               ptr(d.trellis), ptr(d.suh), ptr(d.svh))
+        if key != self._lins_key:
+            self._lins_key = key
+            self._lins = K.lin_table((key[0:3], key[3:6], key[6:9]))
+        return self._lins
+
     def forward(self, gpu: Gpu, x: torch.Tensor, y: torch.Tensor, fused: bool = True, rows: int = 1) -> None:
         """x fp16 [rows][hidden] -> y fp32 [rows][hidden].  fused: one `berth_exl3_mlp` call (two
         launches up to 8 rows); otherwise the reference's four calls for one row (mlp.rs:118-150)."""
@@ -371,8 +392,7 @@ class MlpLayer:
             if self.x_had is None or self.x_had.numel() < rows * self.hidden:
                 self.x_had = torch.zeros(rows * self.hidden, dtype=torch.float16, device=x.device)
                 self.act_had = torch.zeros(self.g.numel(), dtype=torch.float16, device=x.device)
-            lins = [(ptr(l.trellis), ptr(l.suh), ptr(l.svh)) for l in (self.gate, self.up, self.down)]
-            K.exl3_mlp(ptr(x), lins, ptr(self.g), ptr(self.u), ptr(self.x_had), ptr(self.act_had), ptr(y), rows,
+            K.exl3_mlp(ptr(x), self._lin_table(), ptr(self.g), ptr(self.u), ptr(self.x_had), ptr(self.act_had), ptr(y), rows,
                        self.hidden, self.intermediate, self.gate.k_bits, self.gate.codebook, gpu.raw_stream())
             return
         self.gate.forward(gpu, x, self.g, OutDtype.F16)
@@ -393,11 +413,12 @@ class MlpLayer:
         if self.x_had is None or self.x_had.numel() < rows * self.hidden:
             self.x_had = torch.zeros(rows * self.hidden, dtype=torch.float16, device=x.device)
             self.act_had = torch.zeros(self.g.numel(), dtype=torch.float16, device=x.device)
-        if getattr(self, "h_norm", None) is None or self.h_norm.numel() < rows * self.hidden:
+        if self.h_norm is None or self.h_norm.numel() < rows * self.hidden:
             self.h_norm = torch.zeros(rows * self.hidden, dtype=torch.float16, device=x.device)
-        norm = K.RmsNorm(ptr(norm_weight), epsilon, constant_bias, constant_scale, int(weight_bf16))
-        lins = [(ptr(l.trellis), ptr(l.suh), ptr(l.svh)) for l in (self.gate, self.up, self.down)]
-        K.exl3_mlp_block(ptr(x), ptr(residual), ptr(residual_out), norm, lins, ptr(self.h_norm), ptr(self.g), ptr(self.u),
+        key = (ptr(norm_weight), epsilon, constant_bias, constant_scale, int(weight_bf16))
+        if key != self._norm_key:
+            self._norm_key, self._norm = key, K.RmsNorm(*key)
+        K.exl3_mlp_block(ptr(x), ptr(residual), ptr(residual_out), self._norm, self._lin_table(), ptr(self.h_norm), ptr(self.g), ptr(self.u),
                          ptr(self.x_had), ptr(self.act_had), ptr(y), rows, self.hidden, self.intermediate,
                          self.gate.k_bits, self.gate.codebook, gpu.raw_stream())
 

@@ -136,12 +136,17 @@ class Exl3Lin(C.Structure):
     _fields_ = [("trellis", C.c_void_p), ("suh", C.c_void_p), ("svh", C.c_void_p)]
 
 
+def lin_table(lins):
+    """Three (trellis, suh, svh) address triples as the array the MLP entries take; a caller that
+    keeps the result passes it instead of the triples."""
+    return lins if isinstance(lins, C.Array) else (Exl3Lin * 3)(*[Exl3Lin(*t) for t in lins])
+
+
 def exl3_mlp(x, lins, gate_out, up_out, a_had, act_had, y, size_m, hidden, intermediate, k_bits,
              codebook: Codebook, stream=None) -> None:
     """y = down(silu(gate(x)) * up(x)): the four calls of crates/berth-engine/src/mlp.rs:118-150
     in one entry (two launches up to 8 rows).  lins: three (trellis, suh, svh) address triples."""
-    table = (Exl3Lin * 3)(*[Exl3Lin(*t) for t in lins])
-    rc = load().berth_exl3_mlp(x, table, gate_out, up_out, a_had, act_had, y, size_m, hidden, intermediate, k_bits,
+    rc = load().berth_exl3_mlp(x, lin_table(lins), gate_out, up_out, a_had, act_had, y, size_m, hidden, intermediate, k_bits,
                                int(codebook), stream)
     if rc != 0:
         raise LaunchError(last_error() or f"exl3 mlp launch failed ({rc})")
@@ -157,8 +162,7 @@ def exl3_mlp_block(x, residual, residual_out, norm: RmsNorm, lins, h_norm, gate_
                    size_m, hidden, intermediate, k_bits, codebook: Codebook, stream=None) -> None:
     """berth_exl3_mlp_block: residual add + RMS norm, the MLP, and the residual add behind it
     (two launches for one row of streaming-kernel sizes)."""
-    arr = (Exl3Lin * 3)(*[Exl3Lin(*l) for l in lins])
-    rc = load().berth_exl3_mlp_block(x, residual, residual_out, C.byref(norm), arr, h_norm, gate_out, up_out, a_had,
+    rc = load().berth_exl3_mlp_block(x, residual, residual_out, C.byref(norm), lin_table(lins), h_norm, gate_out, up_out, a_had,
                                      act_had, y, size_m, hidden, intermediate, k_bits, int(codebook), stream)
     if rc != 0:
         raise LaunchError(last_error() or f"exl3 mlp block launch failed ({rc})")

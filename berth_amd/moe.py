@@ -91,11 +91,13 @@ class MoeLayer:
         self.shared = shared
         self.shared_I = shared[0].size_n if shared else 0
         self._shared_host = None
+        self._shared_at = None
         if shared:
             arr = (ExpertLinStruct * 3)()
             for i, lin in enumerate(shared):
                 arr[i] = ExpertLinStruct(lin.trellis.data_ptr(), lin.suh.data_ptr(), lin.svh.data_ptr())
             self._shared_host = arr
+            self._shared_at = C.addressof(arr)
         self.shared_gate = None
         if shared_gate is not None:
             if not shared:
@@ -197,7 +199,7 @@ class MoeLayer:
         ws = self._workspace(gpu, T)
         K.moe.layer(x.data_ptr(), self.router.data_ptr(), None if self.bias is None else self.bias.data_ptr(),
                     self.table.data_ptr(),
-                    None if self._shared_host is None else C.cast(self._shared_host, C.c_void_p),
+                    self._shared_at,
                     out.data_ptr(), None if idx_out is None else idx_out.data_ptr(),
                     None if w_out is None else w_out.data_ptr(), ws.data_ptr(), ws.numel(),
                     T, self.hidden, self.num_experts, self.top_k, self.intermediate, self.shared_I,
