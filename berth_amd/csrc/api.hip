@@ -568,13 +568,38 @@ extern "C" int berth_prefill_had_r_128(const void* input, void* output, const vo
 extern "C" const char* berth_prefill_last_error(void) { return g_prefill_err.c_str(); }
 extern "C" const char* berth_prefill_last_launch(void) { return g_prefill_launch.c_str(); }
 
-// gate and up of an MLP for 1..8 rows: on the few-row MFMA kernel where that serves them (the up
-// projection's rotated copy of the input waits in act_had, as above 8 rows), else in one VALU launch
-static std::string launch_pair_few_rows(const PairArgs& pair, void* act_had)
+// Whether gate and up of an MLP run on the MFMA kernels as one bundle: one launch rotates the input
+// with either linear's scales (the up projection's copy waits in act_had, which the down projection
+// fills only afterwards), one dense launch runs both.
+static bool mlp_pair_on_matrix_units(int size_m, int hidden, int intermediate)
 {
-    if (pair.size_n >= pair.size_k && gemv_rows_on_matrix_units(2, pair.size_m, pair.size_k, pair.size_n))
-        return launch_gemm_pair(pair, act_had);
-    return launch_gemv_pair(pair);
+    return intermediate >= hidden && (size_m > 8 || gemv_rows_on_matrix_units(2, size_m, hidden, intermediate));
+}
+
+// gate and up; `norm`: the input is that norm's rows instead of pair.a
+static std::string mlp_gate_up(const PairArgs& pair, void* act_had)
+{
+    if (mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n)) return launch_gemm_pair(pair, act_had);
+    if (pair.size_m <= 8) return launch_gemv_pair(pair);
+    std::string desc;
+    for (int i = 0; i < 2; ++i) {
+        const LinearArgs lin{pair.a, pair.trellis[i], pair.c[i], pair.suh[i], pair.a_had, pair.svh[i], pair.size_m, pair.size_k,
+                             pair.size_n, pair.k_bits, pair.codebook, 0, pair.stream};
+        desc += (i ? " ; " : "") + launch_gemm(lin);
+    }
+    return desc;
+}
+
+// down(silu(gate) * up), with out_add added to its output.  Above 8 rows up_out ends up holding the
+// activation, which is formed where it is rotated.
+static std::string mlp_down(LinearArgs down, void* gate_out, void* up_out, const float* out_add)
+{
+    down.a = gate_out;
+    down.a_up = up_out;
+    down.out_add = out_add;
+    if (down.size_m <= 8) return launch_gemv(down);
+    down.act_out = up_out;
+    return launch_gemm(down);
 }
 
 extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* gate_out, void* up_out, void* a_had,
@@ -596,37 +621,10 @@ extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* g
                         k_bits, codebook, 0, st};
         check_shape("exl3 mlp", gate);
         check_shape("exl3 mlp", down);
-        if (size_m <= 8) {
-            PairArgs pair{x, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh}, {lins[0].svh, lins[1].svh},
-                          {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits, codebook, st};
-            std::string desc = launch_pair_few_rows(pair, act_had);
-            down.a = gate_out;
-            down.a_up = up_out;
-            g_exl3_launch = desc + " ; " + launch_gemv(down);
-            return 0;
-        }
-        std::string desc;
-        if (intermediate >= hidden) {
-            // gate and up as one bundle: one launch rotates the input with either linear's scales (the
-            // up projection's copy waits in act_had, which the down projection fills only afterwards),
-            // one dense launch runs both
-            PairArgs pair{x, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh}, {lins[0].svh, lins[1].svh},
-                          {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits, codebook, st};
-            desc = launch_gemm_pair(pair, act_had);
-        } else {
-            LinearArgs up = gate;
-            up.trellis = lins[1].trellis;
-            up.suh = lins[1].suh;
-            up.svh = lins[1].svh;
-            up.c = up_out;
-            desc = launch_gemm(gate);
-            desc += " ; " + launch_gemm(up);
-        }
-        // the gated activation and its rotation in one launch; up_out ends up holding the activation
-        down.a = gate_out;
-        down.a_up = up_out;
-        down.act_out = up_out;
-        g_exl3_launch = desc + " ; " + launch_gemm(down);
+        PairArgs pair{x, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh}, {lins[0].svh, lins[1].svh},
+                      {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits, codebook, st};
+        const std::string desc = mlp_gate_up(pair, act_had);
+        g_exl3_launch = desc + " ; " + mlp_down(down, gate_out, up_out, nullptr);
         return 0;
     } catch (const std::exception& err) {
         g_exl3_err = err.what();
@@ -641,6 +639,8 @@ extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* g
 // it (ops.rs:522-552, add_f32), as crates/berth-engine/src/mlp.rs:118-150 is called from the
 // block.  One row whose linears take the streaming kernel: two launches, the norm formed while
 // the gate / up launch rotates its input, the sum added where the down launch writes its output.
+// Rows on the MFMA kernels: four launches, the norm formed where the input is rotated, the
+// activation likewise, the sum added where the down launch writes.
 extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* residual_out, const berth_rms_norm* norm,
                                     const berth_exl3_lin* lins, void* h_norm, void* gate_out, void* up_out, void* a_had,
                                     void* act_had, void* y, int size_m, int hidden, int intermediate, int k_bits,
@@ -667,40 +667,31 @@ extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* r
         check_shape("exl3 mlp block", gate);
         check_shape("exl3 mlp block", down);
         const int n = size_m * hidden;
-        const bool fuse_norm = size_m == 1 && gemv_stream_applies(2, hidden, intermediate, false);
-        const bool fuse_add = size_m == 1 && gemv_stream_applies(1, intermediate, hidden, false);
+        const NormInput ni{(const float*)x, (const float*)residual, (float*)residual_out, norm->weight, norm->epsilon,
+                           norm->constant_bias, norm->constant_scale, norm->weight_bf16};
+        PairArgs pair{h_norm, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh}, {lins[0].svh, lins[1].svh},
+                      {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits, codebook, st};
+        // (the fused forms read and write 16 bytes at a time)
+        const bool aligned = (((uintptr_t)x | (uintptr_t)residual | (uintptr_t)residual_out | (uintptr_t)norm->weight) & 15) == 0;
+        const bool fuse_norm = size_m == 1 ? gemv_stream_applies(2, hidden, intermediate, false)
+                                           : aligned && mlp_pair_on_matrix_units(size_m, hidden, intermediate) &&
+                                                 hidden <= kNormRotateMaxCols;
+        const bool fuse_add = size_m == 1 ? gemv_stream_applies(1, intermediate, hidden, false)
+                                          : aligned && (size_m > 8 || gemv_rows_on_matrix_units(1, size_m, intermediate, hidden));
         std::string desc;
         if (fuse_norm) {
-            const NormInput ni{(const float*)x, (const float*)residual, (float*)residual_out, norm->weight, norm->epsilon,
-                               norm->constant_bias, norm->constant_scale, norm->weight_bf16};
-            PairArgs pair{nullptr, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh},
-                          {lins[0].svh, lins[1].svh}, {gate_out, up_out}, a_had, 1, hidden, intermediate, k_bits, codebook, st};
+            pair.a = nullptr;
             pair.norm = &ni;
-            desc = launch_gemv_pair(pair);
         } else {
             // the same arithmetic as separate launches
             desc = launch_add_f32(residual, x, residual_out, n, st);
             desc += " ; " + launch_rms_norm(residual_out, norm->weight, h_norm, nullptr, size_m, hidden, norm->epsilon,
-                                            norm->constant_bias, norm->constant_scale, norm->weight_bf16, st);
+                                            norm->constant_bias, norm->constant_scale, norm->weight_bf16, st) + " ; ";
         }
-        if (size_m <= 8) {
-            if (!fuse_norm) {
-                PairArgs pair{h_norm, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh},
-                              {lins[0].svh, lins[1].svh}, {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits,
-                              codebook, st};
-                desc += " ; " + launch_pair_few_rows(pair, act_had);
-            }
-            down.a = gate_out;
-            down.a_up = up_out;
-            if (fuse_add) down.out_add = (const float*)residual_out;
-            desc += " ; " + launch_gemv(down) + (fuse_add ? " +residual" : "");
-        } else {
-            if (berth_exl3_mlp(h_norm, lins, gate_out, up_out, a_had, act_had, y, size_m, hidden, intermediate, k_bits,
-                               codebook, stream) != 0)
-                throw std::runtime_error(g_exl3_err);
-            desc += " ; " + g_exl3_launch;
-        }
-        if (!fuse_add) desc += " ; " + launch_add_f32(y, residual_out, y, n, st);
+        desc += mlp_gate_up(pair, act_had);
+        desc += " ; " + mlp_down(down, gate_out, up_out, fuse_add ? (const float*)residual_out : nullptr);
+        if (fuse_add) desc += size_m == 1 ? " +residual" : " +add";
+        else desc += " ; " + launch_add_f32(y, residual_out, y, n, st);
         g_exl3_launch = desc;
         return 0;
     } catch (const std::exception& err) {

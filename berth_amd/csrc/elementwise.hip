@@ -120,6 +120,105 @@ __device__ __forceinline__ void rotate_rows(const RotateParams& p)
 __global__ __launch_bounds__(256) void had_r_128_slabs_kernel(RotateParams p) { rotate_rows<false>(p); }
 __global__ __launch_bounds__(256) void silu_mul_had_r_128_kernel(RotateParams p) { rotate_rows<true>(p); }
 
+// The input of an MLP block's gate and up projections in one pass over the rows: residual add,
+// RMS norm (the steps of rms_norm_kernel) and the rotation with each projection's scales.  One
+// workgroup per row, eight values a thread and chunk held in registers between the passes, so
+// a row is read once and only the residual stream and the rotated rows are written: 20 bytes an
+// element against 42 of the four launches (residual add, norm, two rotations).
+struct NormParams {
+    const float* x;
+    const float* res;
+    float* res_out;
+    const uint16_t* weight;
+    int dim, slabs;
+    float epsilon, constant_bias, constant_scale;
+    int weight_bf16;
+};
+template <int CHUNKS>
+__global__ __launch_bounds__(1024) void add_rms_norm_had_r_128_kernel(NormParams n, RotateParams p)
+{
+    __shared__ double s_part[16];
+    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, l16 = lane & 15;
+    const int threads = blockDim.x;
+    const size_t base = (size_t)row * n.dim;
+    float v[CHUNKS][8];
+    double ss = 0.0;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int e = 8 * (tid + c * threads);
+        if (e < n.dim) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4_t xv = *(const float4_t*)(n.x + base + e + 4 * h), rv = *(const float4_t*)(n.res + base + e + 4 * h);
+                const float4_t sum = {rv.x + xv.x, rv.y + xv.y, rv.z + xv.z, rv.w + xv.w};
+                *(float4_t*)(n.res_out + base + e + 4 * h) = sum;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[c][4 * h + j] = sum[j];
+                    ss += (double)sum[j] * (double)sum[j];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[c][j] = 0.0f;
+        }
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) ss += __shfl_xor(ss, d, 64);
+    if (lane == 0) s_part[tid >> 6] = ss;
+    __syncthreads();
+    double total = 0.0;
+    for (int w = 0; w < (threads >> 6); ++w) total += s_part[w];
+    const float rmf = (float)(1.0 / sqrt(total / n.dim + (double)n.epsilon));
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int e = 8 * (tid + c * threads);
+        if (e - 8 * l16 >= n.dim) continue;             // the sixteen lanes of a 128 block stay together
+        const half8_t wb = *(const half8_t*)(n.weight + e);
+        _Float16 y[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint16_t bits = __builtin_bit_cast(uint16_t, (_Float16)wb[j]);
+            const float w = n.weight_bf16 ? __builtin_bit_cast(float, (uint32_t)bits << 16) : (float)(_Float16)wb[j];
+            float t = v[c][j] * rmf;
+            t = t * (w + n.constant_bias);
+            t = t * n.constant_scale;
+            y[j] = (_Float16)t;
+        }
+        for (int s = 0; s < n.slabs; ++s) {
+            const half8_t s8 = *(const half8_t*)(p.tab.suh[s] + e);
+            float r[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) r[j] = (float)y[j] * (float)s8[j];
+            had128_row16(r, lane);
+            half8_t o;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o[j] = (_Float16)(r[j] * kRsqrt128);
+            _Float16* out = p.tab.out[s] ? p.tab.out[s] : p.out + (size_t)s * p.out_stride;
+            *(half8_t*)(out + base + e) = o;
+            if (p.operand) *(half8_t*)(p.operand + (size_t)s * p.operand_stride + rows_operand_offset(row, e, p.mt)) = o;
+        }
+    }
+}
+
+static std::string launch_norm_rotate(const RotateArgs& a, const RotateParams& p)
+{
+    if (a.suh_list || a.cols > kNormRotateMaxCols || a.cols % 128)
+        throw std::runtime_error("norm + rotation: by-value scales and at most " + std::to_string(kNormRotateMaxCols) + " columns");
+    const NormInput& in = *a.norm;
+    const NormParams n{in.x, in.res, in.res_out, (const uint16_t*)in.weight, a.cols, a.slabs, in.epsilon, in.constant_bias,
+                       in.constant_scale, in.weight_bf16};
+    const int chunks = (a.cols / 8 + 1023) / 1024;      // 1..4
+    const int threads = ((a.cols / 8 + chunks - 1) / chunks + 63) / 64 * 64;
+    switch (chunks) {
+    case 1: hipLaunchKernelGGL(add_rms_norm_had_r_128_kernel<1>, dim3((unsigned)a.rows), dim3(threads), 0, a.stream, n, p); break;
+    case 2: hipLaunchKernelGGL(add_rms_norm_had_r_128_kernel<2>, dim3((unsigned)a.rows), dim3(threads), 0, a.stream, n, p); break;
+    default: hipLaunchKernelGGL(add_rms_norm_had_r_128_kernel<4>, dim3((unsigned)a.rows), dim3(threads), 0, a.stream, n, p); break;
+    }
+    hip_ok(hipGetLastError(), "add + rms_norm + had_r_128 launch");
+    return "add_rms_norm_had_r_128_kernel grid=" + std::to_string(a.rows) + " block=" + std::to_string(threads);
+}
+
 std::string launch_rotate(const RotateArgs& a)
 {
     if (a.slabs < 1 || a.slabs > 65535) throw std::runtime_error("had_r_128 slabs: between 1 and 65535 slabs");
@@ -144,6 +243,7 @@ std::string launch_rotate(const RotateArgs& a)
             p.tab.out[i] = a.out_host ? (_Float16*)a.out_host[i] : nullptr;
         }
     }
+    if (a.norm) return launch_norm_rotate(a, p);
     const long wgs = (p.blocks + 15) / 16;
     const dim3 grid((unsigned)(wgs < 4096 ? wgs : 4096), (unsigned)a.slabs);
     if (a.up) hipLaunchKernelGGL(silu_mul_had_r_128_kernel, grid, dim3(256), 0, a.stream, p);

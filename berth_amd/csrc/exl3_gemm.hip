@@ -255,6 +255,8 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     p.K = a.size_k;
     p.N = a.size_n;
     p.out_fp32 = a.out_fp32;
+    if (a.out_add && !a.out_fp32) throw std::runtime_error("exl3 gemm: rows are added to an fp32 output only");
+    p.out_add = a.out_add;
     p.partials = ws.partials;
     p.counters = ws.counters;
     std::string desc;
@@ -385,6 +387,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
     }
     RotateArgs rot;
     rot.in = a.a;
+    rot.norm = a.norm;
     rot.suh_host = a.suh;
     rot.out_host = slabs;
     rot.slabs = 2;

@@ -554,6 +554,12 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                 for (int i = 0; i < 8; ++i) v[i] = (v[i] * kRsqrt128) * (float)sv[i];
                 const size_t at = (size_t)(m0 + mb * 32 + row) * ldc + gn + 8 * l16;
                 if (p.out_fp32) {
+                    if (p.out_add) {
+                        const global_ptr<const float4_t> add = (global_ptr<const float4_t>)(as_global(p.out_add) + at);
+                        const float4_t a0 = add[0], a1 = add[1];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) { v[i] += a0[i]; v[4 + i] += a1[i]; }
+                    }
                     global_ptr<float4_t> dst = (global_ptr<float4_t>)(as_global((float*)cout) + at);
                     dst[0] = float4_t{v[0], v[1], v[2], v[3]};
                     dst[1] = float4_t{v[4], v[5], v[6], v[7]};

@@ -239,7 +239,7 @@ std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
             return run_stream(ws, pl, sp, a.k_bits, a.codebook, a.stream);
         }
     }
-    if (a.out_add) throw std::runtime_error("exl3 gemv: the added output row needs the one-row streaming kernel");
+    if (a.out_add) throw std::runtime_error("exl3 gemv: the added output needs the one-row streaming kernel or the MFMA kernels");
 
     GemvParams p{};
     p.a = (const _Float16*)a.a;

@@ -136,15 +136,15 @@ struct LinearArgs {
     hipStream_t stream;
     const void* a_up = nullptr;   // the input is silu(a) * a_up, element by element
     void* act_out = nullptr;      // with a_up, MFMA kernels only: where that input also goes (may be a_up)
-    const float* out_add = nullptr;   // streaming kernel only (one row, fp32 output): a row added to the output
+    const float* out_add = nullptr;   // streaming and MFMA kernels, fp32 output: fp32 [size_m][size_n] added to the output
 };
 
-// RMS norm with the residual added first, as the input of a launch of the streaming kernel
-// (the arithmetic of berth_ops_rms_norm_res_in; the sum goes to res_out, which aliases neither)
+// RMS norm with the residual added first, as the input of a launch of the streaming kernel or of a
+// rotation (the arithmetic of berth_ops_rms_norm_res_in; the sum goes to res_out, which aliases neither)
 struct NormInput {
-    const float* x;             // fp32 [K]
-    const float* res;           // fp32 [K]
-    float* res_out;             // fp32 [K]
+    const float* x;             // fp32 [rows][K]
+    const float* res;           // fp32 [rows][K]
+    float* res_out;             // fp32 [rows][K]
     const void* weight;         // fp16 or bf16 [K]
     float epsilon, constant_bias, constant_scale;
     int weight_bf16;
@@ -160,7 +160,7 @@ struct PairArgs {
     void* a_had;                // [size_m][size_k]
     int size_m, size_k, size_n, k_bits, codebook;
     hipStream_t stream;
-    const NormInput* norm = nullptr;    // one row, streaming kernel only: `a` is then unused
+    const NormInput* norm = nullptr;    // `a` is then unused; one row: the streaming kernel only
 };
 std::string launch_gemv_pair(const PairArgs& args);
 // whether a one-row launch of `problems` linears of this shape takes the streaming kernel (and,
@@ -262,8 +262,11 @@ struct RotateArgs {
     void* act_out = nullptr;
     void* operand = nullptr;
     int mt = 1;
+    const NormInput* norm = nullptr;    // the input of every slab is this norm's (in is then unused)
 };
 std::string launch_rotate(const RotateArgs& args);
+// columns up to which launch_rotate forms a norm
+constexpr int kNormRotateMaxCols = 32768;
 // gate and up of an MLP above 8 rows as one bundle: two linears of one shape on one input, each
 // with its own output and its own buffer for the rotated input
 std::string launch_gemm_pair(const PairArgs& pair, void* a_had_second);

@@ -289,8 +289,9 @@ int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* gate_out, vo
  * one-row streaming kernel the norm is formed while that launch rotates its input (same fp32
  * steps as berth_ops_rms_norm_res_in; the sum of squares in double, whose order of summation
  * differs), and where the down projection takes it the residual is added where it writes its
- * output: two launches when both do.  Anything else runs the same arithmetic as separate
- * launches. */
+ * output: two launches when both do.  More rows where gate and up run on the MFMA kernels as one
+ * bundle: the norm is formed where the input is rotated and the residual added where the down launch
+ * writes (four launches).  Anything else runs the same arithmetic as separate launches. */
 typedef struct {
     const void* weight;         /* fp16 or bf16 [hidden] */
     float epsilon, constant_bias, constant_scale;

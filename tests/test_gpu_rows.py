@@ -77,3 +77,36 @@ def test_mlp_of_few_rows_stage_by_stage(rows):
     from tests.test_gpu_mlp import run_mlp_block
     launch = run_mlp_block(rows, 1536, 4096, 4)
     assert launch.count("exl3_gemm_kernel/rows") == 2 and "silu_mul_had_r_128_kernel" in launch, launch
+
+
+@pytest.mark.parametrize("rows,H,I,bits", [(2, 128, 256, 4),        # one block a row: a quarter of a wave
+                                           (9, 1152, 1280, 3),      # a workgroup with a half-empty wave
+                                           (33, 8320, 8320, 2),     # two chunks a thread, 32-row tiles with one row
+                                           (3, 17408, 17408, 1)])   # three chunks
+def test_block_with_fused_norm_equals_the_separate_calls(rows, H, I, bits):
+    """Residual add, norm and both rotations in one launch, the residual added by the down launch:
+    the residual stream, rotated inputs, gate / up results and the output bit for bit as
+    berth_ops_rms_norm_res_in -> berth_exl3_mlp -> berth_ops_add_f32 give them."""
+    from berth_amd.device import Gpu, ptr
+    from tests.test_gpu_mlp import _block_inputs, _layer
+    gpu = Gpu(0)
+    _, mlp = _layer(gpu, H, I, bits, 9900 + rows, rows)
+    x, res, w = _block_inputs(gpu, H, rows, 9950 + rows)
+    res_ref, h = res.clone(), torch.zeros((rows, H), dtype=torch.float16, device=DEV)
+    K.ops.rms_norm_res_in(ptr(x), ptr(w), ptr(h), ptr(res_ref), rows, H, 1e-6, 1.0, 1.0, True, gpu.raw_stream())
+    y_ref = torch.zeros((rows, H), dtype=torch.float32, device=DEV)
+    mlp.forward(gpu, h, y_ref, rows=rows)
+    K.ops.add_f32(ptr(y_ref), ptr(res_ref), ptr(y_ref), rows * H, gpu.raw_stream())
+    names = ("x_had", "g", "u", "act_had")
+    want = {n: getattr(mlp, n).clone() for n in names}
+    for n in names:
+        getattr(mlp, n).zero_()
+    res_out, y = torch.zeros_like(res), torch.zeros_like(y_ref)
+    mlp.forward_block(gpu, x, res, res_out, w, y, rows=rows)
+    torch.cuda.synchronize()
+    launch = K.last_launch()
+    assert "add_rms_norm_had_r_128_kernel" in launch and "+add" in launch, launch
+    bits_of = lambda t: t.view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+    assert torch.equal(bits_of(res_out), bits_of(res_ref)) and torch.equal(bits_of(y), bits_of(y_ref)), launch
+    for n in names:
+        assert torch.equal(bits_of(getattr(mlp, n)), bits_of(want[n])), (n, launch)
