@@ -151,7 +151,7 @@ Knobs read_knobs()
 {
     Knobs k{};
     k.gemv_stream = env_int("BERTH_GEMV_STREAM", 1);
-    k.gemv_stream_min_units = std::max(2, env_int("BERTH_GEMV_STREAM_MIN_UNITS", 3));
+    k.gemv_stream_min_units = std::max(2, env_int("BERTH_GEMV_STREAM_MIN_UNITS", 2));
     k.gemv_stream_shrink = env_int("BERTH_GEMV_STREAM_SHRINK", 0);
     k.gemv_stream_wgs = env_int("BERTH_GEMV_STREAM_WGS", 0);
     k.gemv_stream_lut = env_int("BERTH_GEMV_STREAM_LUT", -1);

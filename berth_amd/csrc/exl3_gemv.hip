@@ -46,12 +46,12 @@ void launch_gemv_stream_cb2(const StreamParams& p, int bits, int lutmask, dim3 g
 
 // ---- the one-row streaming kernel: the static split and when it applies
 //
-// Of a problem's U = (N/128) * (K/16) units every wave of its Gp workgroups takes q (the
-// first `rem` waves q + 1).  The kernel applies when every wave gets at least
-// `stream_min_units` tile rows (below that the fixed cost of a sixteen-wave workgroup, its
-// table copy and its barriers, is not paid back), when the rotated activation of a
-// workgroup's units fits its LDS region and when the exact-division multipliers are exact
-// for the operands the kernel divides.
+// Of a problem's U = (N/128) * (K/64) units every wave group of its Gp workgroups takes q (the
+// first `rem` groups q + 1).  The kernel applies when the groups get more than
+// `stream_min_units` units each, when the rotated activation of a workgroup's units fits its LDS
+// region and when the exact-division multipliers are exact for the operands the kernel divides.
+// Two units: 4096 x 4096 (two each) takes 7.3 us with either kernel at 4 bits, 2688 x 4096 (1.3)
+// 7.1 with the other one and 7.2 here, 5120 x 4096 (2.5) 9.2 with the other one and 7.9 here.
 struct StreamPlan {
     bool ok = false;
     int problems = 0, Gp = 0;
@@ -78,26 +78,26 @@ static StreamPlan plan_stream(const Workspace& ws, int problems, int K, int N)
     StreamPlan pl;
     const Knobs& kn = knobs();
     if (!kn.gemv_stream || problems < 1 || problems > ws.cu_count || !ws.accum) return pl;
-    const unsigned TR = (unsigned)K / 16, NB = (unsigned)N / 128, KB = (unsigned)K / 128;
+    const unsigned TR = (unsigned)K / 64, NB = (unsigned)N / 128, KB = (unsigned)K / 128;
     const unsigned long long U = (unsigned long long)NB * TR;
     if (U >= (1ull << 31)) return pl;
     const unsigned min_units = (unsigned)kn.gemv_stream_min_units;
     int Gp = ws.cu_count / problems;
     if (kn.gemv_stream_wgs > 0 && Gp > kn.gemv_stream_wgs) Gp = kn.gemv_stream_wgs;
-    if (U / ((unsigned)Gp * kStreamWaves) < min_units) {
+    if (U <= (unsigned long long)Gp * kStreamGroups * min_units) {
         if (!kn.gemv_stream_shrink) return pl;
-        Gp = (int)(U / (min_units * kStreamWaves));
+        Gp = (int)(U / (min_units * kStreamGroups));
         if (Gp < 1) return pl;
     }
-    const unsigned waves = (unsigned)Gp * kStreamWaves;
-    const unsigned q = (unsigned)(U / waves), rem = (unsigned)(U % waves);
+    const unsigned groups = (unsigned)Gp * kStreamGroups;
+    const unsigned q = (unsigned)(U / groups), rem = (unsigned)(U % groups);
     // exact division by multiply-high needs dividend * divisor < 2^32
     if (U * (q + 2) >= (1ull << 32) || U * TR >= (1ull << 32)) return pl;
-    const unsigned L = kStreamWaves * (q + 1);                 // most units of one workgroup
+    const unsigned L = kStreamGroups * (q + 1);                 // most units of one workgroup
     if ((L + TR - 1) / TR + 1 > (unsigned)kStreamMaxCb) return pl;
-    if (KB > (unsigned)kStreamXsBlocks && (L + 16 >= TR || L / 8 + 2 > (unsigned)kStreamXsBlocks)) return pl;
+    if (KB > (unsigned)kStreamXsBlocks && (L + 4 >= TR || L / 2 + 2 > (unsigned)kStreamXsBlocks)) return pl;
     // workgroups that can share a column block: bounded by the accumulator word's count field
-    const unsigned sharers = (TR + kStreamWaves * q - 1) / (kStreamWaves * q) + 1;
+    const unsigned sharers = (TR + kStreamGroups * q - 1) / (kStreamGroups * q) + 1;
     if (sharers > (unsigned)kFixedMaxSharers) return pl;
     if ((unsigned long long)problems * NB > (unsigned long long)ws.accum_slots) return pl;
     pl.ok = true;
@@ -116,19 +116,19 @@ bool gemv_stream_applies(int problems, int size_k, int size_n, bool whole_rows)
     if (size_k % 128 != 0 || size_n % 128 != 0) return false;
     const StreamPlan pl = plan_stream(workspace_for_current_device(), problems, size_k, size_n);
     if (!pl.ok) return false;
-    return !whole_rows || (unsigned)kStreamWaves * pl.q >= (unsigned)size_k / 16;
+    return !whole_rows || (unsigned)kStreamGroups * pl.q >= (unsigned)size_k / 64;
 }
 
 static std::string run_stream(const Workspace& ws, const StreamPlan& pl, StreamParams& p, int bits, int cb,
                               hipStream_t stream)
 {
     throw_pending_device_fault(ws);
-    int mask = stream_lut_mask(bits, (unsigned long long)pl.q * kStreamWaves * 256 * bits);
+    int mask = stream_lut_mask(bits, (unsigned long long)pl.q * kStreamGroups * 1024 * bits);
     if (mask != 0) mask = 0xA;          // the one hybrid mask that is instantiated
     p.accum = ws.accum;
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
-    p.TR = p.K / 16;
+    p.TR = p.K / 64;
     p.NB = p.N / 128;
     p.Gp = pl.Gp;
     p.mgp = magic((unsigned)pl.Gp);

@@ -1,25 +1,30 @@
 // EXL3 linear for ONE row, as a single resident round of workgroups: one workgroup of
-// sixteen waves per compute unit, every wave a contiguous run of tile rows.
+// sixteen waves per compute unit, every wave a contiguous run of units.
 //
 //   c = ( Hh(x * suh) @ W ) -> Hh(.) * svh          (Hh = 128-block Hadamard / sqrt(128))
 //
 // The operator of crates/berth-kernels/csrc/linear.cu:209-286 at m = 1 (and of the m = 1
 // bundles of crates/berth-kernels/csrc/ops/mgemm.cu:125-272), for weights large enough
-// that every wave gets several tile rows.
+// that every wave gets several units.
 //
-//   * Work of a problem (one linear, or one slice of a bundle) = its (column block, tile
-//     row) units, column block major: U = (N/128) * (K/16) units of `32*bits` bytes per
-//     lane-octet, 8 octets (128 columns) per wave.  The problem's waves split the units
-//     evenly: wave W takes q units, the first `rem` waves one more.  No second round, no
-//     tail of half-empty compute units: the grid is at most the number of compute units
-//     and every wave does the same amount of decode.
-//   * A wave keeps a ring of two tile rows in registers; a tile row is reloaded with the
-//     tile row two units ahead as soon as it has been decoded.  The walk crosses column
-//     block boundaries without draining the ring.
+//   * Work of a problem (one linear, or one slice of a bundle) = its units of 64 rows of K x
+//     128 columns, column block major: U = (N/128) * (K/64).  Four waves share a unit, 32 columns
+//     each; the problem's wave groups split the units evenly: group W takes q units, the first
+//     `rem` groups one more.  No second round, no tail of half-empty compute units: the grid is
+//     at most the number of compute units and every wave does the same amount of decode.
+//   * The dot products run on the matrix units (v_mfma_f32_16x16x32_f16 with the one row in all
+//     sixteen row slots): 16 lanes cover 2 tiles of one tile row, the four lane groups four tile
+//     rows, so the register quads a lane decodes are B operands as they are, and the A operand is
+//     16 bytes of the rotated activation per lane group.  Four of them per 32 weights of a lane
+//     take 64 cycles of a pipe that is idle otherwise; the sixteen v_dot2 they replace took 64
+//     of the 560 that the vector pipe was busy.
+//   * A wave keeps a ring of two units in registers; one is reloaded with the unit two ahead
+//     as soon as it has been decoded.  The walk crosses column block boundaries without
+//     draining the ring.
 //   * The workgroup rotates the activation of the k-blocks its units touch once, into
 //     LDS (every wave takes some k-blocks), and writes a_had for the k-blocks whose
 //     column-block-0 units it owns.  Those loads go out first of all, ahead of the split
-//     arithmetic of the wave and of its first tile row: the barrier behind the rotation
+//     arithmetic of the wave and of its first unit: the barrier behind the rotation
 //     is what the whole workgroup waits for.
 //   * Decode is optionally a hybrid: of the four weight pairs of a dword, those selected
 //     by LUTMASK come from a 128 KiB state -> fp16 table in LDS, which the workgroup builds
@@ -27,8 +32,8 @@
 //     arithmetic.  The table read costs address + read + pack (2.5 vector instructions
 //     per weight with the dot product) against 4.4 for the arithmetic; the LDS read rate
 //     bounds how many can go that way.
-//   * Partial sums: a wave writes one 128-column partial per column block it touched
-//     into LDS, and the pieces of a column block are added in wave order.  A column block
+//   * Partial sums: a wave group writes one 128-column partial per column block it touched
+//     into LDS, and the pieces of a column block are added in group order.  A column block
 //     that lies entirely inside the workgroup's units is finished there.  Otherwise every
 //     workgroup that shares it adds its part, converted to 64-bit fixed point, onto the
 //     block's accumulator words with one atomic add that returns the old value: integer
@@ -45,13 +50,14 @@
 namespace berth {
 
 constexpr int kStreamWaves = 16;
+constexpr int kStreamGroups = 4;           // wave groups of a workgroup, four waves each
 constexpr int kStreamXsBlocks = 64;        // k-blocks of rotated activation a workgroup can hold
 constexpr int kStreamMaxCb = 15;           // column blocks one workgroup's units can touch
-constexpr int kStreamPieces = kStreamWaves + kStreamMaxCb - 1;
-// dynamic LDS of a launch: [table 128 KiB, if any][rotated activation][partial pieces][piece bounds]
+constexpr int kStreamPieces = kStreamGroups + kStreamMaxCb - 1;
+// dynamic LDS of a launch: [table 128 KiB, if any][rotated activation][partial pieces][norm sums]
 __host__ __device__ constexpr int stream_lds_bytes(int lutmask)
 {
-    return (lutmask ? 131072 : 0) + kStreamXsBlocks * 256 + kStreamPieces * 512 + 128 + 128;
+    return (lutmask ? 131072 : 0) + kStreamXsBlocks * 256 + kStreamPieces * 512 + 128;
 }
 
 // one problem of a bundle whose lists the host knows (mode 3)
@@ -82,11 +88,11 @@ struct StreamParams {
     _Float16* a_had;            // optional; slab per rotation source
     int mode;                   // 0 by value, 1 uniform lists, 2 sliced lists, 3 slices by value
     int in_stride;              // elements between the inputs of consecutive problems (0: shared)
-    int K, N, NB, TR;           // N: row stride of trellis and output in mode 0 / 1; TR = K / 16
+    int K, N, NB, TR;           // N: row stride of trellis and output in mode 0 / 1; TR = K / 64
     int out_fp32;
     int Gp;                     // workgroups per problem (gridDim.x = problems * Gp)
     unsigned mgp;               // floor(2^32 / Gp) + 1
-    unsigned q, rem;            // units per wave; the first `rem` waves of a problem take q + 1
+    unsigned q, rem;            // units per wave group; the first `rem` groups of a problem take q + 1
     unsigned mq, mq1, mtr;      // floor(2^32 / d) + 1 for d = q, q + 1, TR (exact for the operands used)
     unsigned long long* accum;  // [problem][column block][128] fixed-point sums, zero between launches
     unsigned* fault;            // host-visible word for a finisher that gives up its bounded wait
@@ -124,7 +130,7 @@ __device__ __forceinline__ uint32_t lut_read(uint32_t addr) { return *(lds_u16_p
 
 __host__ __device__ constexpr int popcount4(int m) { return (m & 1) + ((m >> 1) & 1) + ((m >> 2) & 1) + ((m >> 3) & 1); }
 
-// Decode of a lane's 32 weights of one tile row, some pairs through the table, in three
+// Decode of a lane's 32 weights of one unit, some pairs through the table, in three
 // steps so that the table reads are in flight while the other pairs are computed:
 // addresses() fills the table addresses, the caller issues the reads, finish() decodes
 // the arithmetic pairs and packs the table values.
@@ -242,7 +248,7 @@ __device__ __forceinline__ void nested_tail(unsigned count, F&& f)
     }
 }
 
-// Tile rows a wave keeps in flight.  Two: with sixteen waves per compute unit that is what the
+// Units a wave keeps in flight.  Two: with sixteen waves per compute unit that is what the
 // memory's latency takes at the rate the decode consumes them; deeper rings only lengthen the
 // queues that everything else (the first loads of the launch, the hand-over at its end) waits in
 // (27B layer set at 4 bits per weight, four launches: 67.1 us with four, 65.3 with two).
@@ -277,9 +283,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
     constexpr int RING = StreamRing<BITS>::depth;
     uint32_t* const xs = (uint32_t*)(lds + kXsOff);
     float* const red = (float*)(lds + kRedOff);
-    unsigned* const piece_first = (unsigned*)(lds + kMetaOff);
-    unsigned* const piece_last = piece_first + 16;
-    double* const norm_part = (double*)(lds + kMetaOff + 128);         // NORM: one sum of squares per wave
+    double* const norm_part = (double*)(lds + kMetaOff);               // NORM: one sum of squares per wave
 
     // The scalar fields sit in the first six lines of the argument block; the by-value problems
     // behind them are read by the launches that use them (touching all sixteen lines at the
@@ -325,18 +329,19 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
     // (a slice narrower than the bundle's width ends early: its units stop at its last column block)
     const unsigned TR = (unsigned)p.TR;
     const unsigned u_end = (unsigned)(width >> 7) * TR;
-    const unsigned W0 = gl * kStreamWaves;
-    const unsigned u0 = min(W0 * p.q + min(W0, p.rem), u_end);
-    const unsigned u1 = min((W0 + kStreamWaves) * p.q + min(W0 + kStreamWaves, p.rem), u_end);
+    const unsigned W0 = gl * kStreamGroups;
+    auto group_start = [&](unsigned W) { return min(W * p.q + min(W, p.rem), u_end); };
+    const unsigned u0 = group_start(W0);
+    const unsigned u1 = group_start(W0 + kStreamGroups);
     if (u0 >= u1) return;
     const unsigned cb_first = div_magic(u0, p.mtr);
     // The k-blocks these units touch are a cyclic run of nk k-blocks from that of the first
-    // unit (the walk wraps from the last tile row of a column block to tile row 0 of the
+    // unit (the walk wraps from the last unit of a column block to the first of the
     // next); k-block a_lo + i, taken modulo K / 128, is held in slot i of the LDS region.
-    const unsigned KB = TR >> 3;
+    const unsigned KB = TR >> 1;
     const unsigned r_lo = u0 - cb_first * TR;
-    unsigned a_lo = r_lo >> 3;
-    unsigned nk = ((r_lo & 7u) + (u1 - u0) + 7u) >> 3;
+    unsigned a_lo = r_lo >> 1;
+    unsigned nk = ((r_lo & 1u) + (u1 - u0) + 1u) >> 1;
     if (nk >= KB) {
         nk = KB;
         a_lo = 0;
@@ -382,35 +387,40 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         }
     }
 
-    // ---- this wave's units [uw0, uw1) and its first tile row
-    const unsigned Ww = W0 + (unsigned)wave;
-    const unsigned uw0 = min(Ww * p.q + min(Ww, p.rem), u_end);
-    const unsigned uw1 = min((Ww + 1) * p.q + min(Ww + 1, p.rem), u_end);
+    // ---- this wave's units [uw0, uw1) and the first of them
+    const int cg = wave & 3, kg = wave >> 2;
+    const int l16 = lane & 15, lg = lane >> 4;
+    const unsigned uw0 = group_start(W0 + (unsigned)kg);
+    const unsigned uw1 = group_start(W0 + (unsigned)kg + 1);
     constexpr int tile_dw = 8 * BITS;
     const long row_dw = (long)(n_stride >> 4) * tile_dw;
-    const long wrap_dw = (long)(8 * tile_dw) - (long)(TR - 1) * row_dw;
+    const long unit_dw = 4 * row_dw;                        // four tile rows
+    const long wrap_dw = (long)(8 * tile_dw) - (long)(TR - 1) * unit_dw;
     // (a wave without units, possible only behind the end of a narrow slice, reads the
     // workgroup's first unit and never uses it)
     const unsigned ufirst = uw0 < uw1 ? uw0 : u0;
     unsigned cb = div_magic(ufirst, p.mtr);
     unsigned r = ufirst - cb * TR;
-    const int lane_dw = lane * BITS;
+    const uint32_t lane_bytes = ((uint32_t)lg * (uint32_t)row_dw + (uint32_t)((cg * 16 + l16) * BITS)) * 4u;
     // the walk's pointer is the same in every lane: held in scalar registers, so that stepping it
     // costs no vector instruction and the loads take it as their scalar base
     global_ptr<const uint32_t> pbase =
-        uniform_ptr(as_global(lin.trellis) + (long)cb * (8 * tile_dw) + (long)r * row_dw);
-    unsigned p_r = r;                                       // tile row of the unit pbase points at
+        uniform_ptr(as_global(lin.trellis) + (long)cb * (8 * tile_dw) + (long)r * unit_dw);
+    unsigned p_r = r;                                       // place in its column block of the unit pbase points at
     unsigned p_left = uw0 < uw1 ? uw1 - uw0 - 1 : 0u;       // units after it that are still this wave's
     uint32_t own[RING][BITS];
+    auto load_unit = [&](uint32_t (&out)[BITS]) {
+        load_tile_dwords<BITS>((global_ptr<const uint32_t>)((global_ptr<const char>)pbase + lane_bytes), out);
+    };
     auto prologue_row = [&](int j) {
-        load_tile_dwords<BITS>(pbase + lane_dw, own[j]);
-        const long step = p_left == 0 ? 0 : (p_r == TR - 1 ? wrap_dw : row_dw);
+        load_unit(own[j]);
+        const long step = p_left == 0 ? 0 : (p_r == TR - 1 ? wrap_dw : unit_dw);
         pbase += step;
         p_r = p_left == 0 ? p_r : (p_r == TR - 1 ? 0u : p_r + 1);
         p_left = p_left == 0 ? 0u : p_left - 1;
         __builtin_amdgcn_sched_barrier(0);
     };
-    // Only the first tile row goes out ahead of the rotation: whole rings of sixteen waves are
+    // Only the first unit goes out ahead of the rotation: whole rings of sixteen waves are
     // more than the compute unit's request queue holds, the later waves would sit in the
     // issue of their loads until the burst has drained at the memory's rate, and the barrier
     // below waits for the slowest wave.
@@ -425,12 +435,8 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         sv_mine = ((global_ptr<const half2_t>)as_global(lin.svh + (cb_first + (unsigned)wave) * 128))[lane];
         if (p.out_add) add_mine = ((global_ptr<const float2_t>)as_global(p.out_add + (cb_first + (unsigned)wave) * 128))[lane];
     }
-    if (threadIdx.x < 16) {
-        piece_first[threadIdx.x] = 0xffffffffu;
-        piece_last[threadIdx.x] = 0u;
-    }
 
-    // ---- the table: built in place while the first tile rows and the activation are on
+    // ---- the table: built in place while the first units and the activation are on
     // their way (the vector ALU has nothing else to do until they arrive).  Thread t writes
     // the entries of states 2 (t + 1024 j), + 1 as one dword: consecutive lanes, consecutive
     // dwords.
@@ -504,7 +510,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
             rot_x[t].y = (_Float16)t1;
         }
     }
-    // ---- rotate; a_had: the workgroup that owns tile row 8 * kb of column block 0 writes k-block kb
+    // ---- rotate; a_had: the workgroup that owns unit 2 * kb of column block 0 writes k-block kb
     const global_ptr<half2_t> hout = (global_ptr<half2_t>)as_global(p.a_had + (size_t)had_slab * p.K);
 #pragma unroll
     for (int t = 0; t < kRot; ++t) {
@@ -522,7 +528,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         rotated.x = (_Float16)(v0 * kRsqrt128);
         rotated.y = (_Float16)(v1 * kRsqrt128);
         xs[i * 64 + lane] = as_u32(rotated);
-        if (write_had && u0 <= 8 * rot_kb[t] && 8 * rot_kb[t] < u1) hout[rot_kb[t] * 64 + lane] = rotated;
+        if (write_had && u0 <= 2 * rot_kb[t] && 2 * rot_kb[t] < u1) hout[rot_kb[t] * 64 + lane] = rotated;
     }
     __syncthreads();
     // the rest of the ring goes out behind the barrier: a wave whose loads wait for room in
@@ -531,26 +537,24 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
     for (int j = 1; j < RING; ++j) prologue_row(j);
 
     // ---- the walk
-    // LDS byte offset of the rotated activation of tile row r of the current column block
-    const unsigned xoff_wrap = kXsOff + (a_lo ? (KB - a_lo) * 256u : 0u);     // tile row 0 of a later column block
-    unsigned xoff = kXsOff + (r << 5) - a_lo * 256u;
-    if (cb != cb_first) xoff = xoff_wrap + (r << 5);
-    unsigned piece = (unsigned)wave + (cb - cb_first);
+    // LDS byte offset of this lane group's part of the rotated activation of the current unit
+    const unsigned xoff_wrap = kXsOff + (a_lo ? (KB - a_lo) * 256u : 0u);     // first unit of a later column block
+    unsigned xoff = kXsOff + (r << 7) - a_lo * 256u;
+    if (cb != cb_first) xoff = xoff_wrap + (r << 7);
+    unsigned piece = (unsigned)kg + (cb - cb_first);
     unsigned left = uw0 < uw1 ? uw1 - uw0 : 0u;
-    float acc0 = 0.0f, acc1 = 0.0f;
-    const int col = (lane >> 3) * 16 + (lane & 7);
+    float4_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;  // all four elements alike: the row slots hold one row
+    const int col = cg * 32 + (l16 >> 3) * 16 + (l16 & 7);
 
     auto flush = [&](unsigned pc) {
-        red[pc * 128 + col] = acc0;
-        red[pc * 128 + col + 8] = acc1;
-        if (lane == 0) {
-            atomicMin(&piece_first[pc - (unsigned)wave], (unsigned)wave);
-            atomicMax(&piece_last[pc - (unsigned)wave], (unsigned)wave);
+        if (lane < 16) {
+            red[pc * 128 + col] = acc0[0];
+            red[pc * 128 + col + 8] = acc1[0];
         }
     };
 
-    // One tile row: table addresses and reads first, the next tile row's load, the
-    // arithmetic pairs while the table reads are in flight, then the dot products.
+    // One unit: table addresses and reads first, the next unit's load, the arithmetic
+    // pairs while the table reads are in flight, then the dot products.
     auto stage = [&](uint32_t (&mine)[BITS], bool prefetch) {
         using Dec = HybridDecode<BITS, CB, LUTMASK>;
         constexpr int NT = Dec::kTablePairs ? 2 * Dec::kTablePairs : 1;
@@ -558,8 +562,8 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         const uint32_t prev = fetch_prev(lane, mine[BITS - 1]);
         uint32_t addr[NT], t[NT], w2[16];
         dec.addresses(mine, prev, addr);
-        const uint4* xp = (const uint4*)(lds + xoff);
-        const uint4 xa = xp[0], xb = xp[1];
+        const half8_t* xp = (const half8_t*)(lds + xoff + 32 * lg);
+        const half8_t xa = xp[0], xb = xp[1];               // k 0..7 and 8..15 of the lane group's tile row
         if constexpr (Dec::kTablePairs != 0) {
 #pragma unroll
             for (int i = 0; i < NT; ++i) t[i] = lut_read(addr[i]);
@@ -567,14 +571,14 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         __builtin_amdgcn_sched_barrier(0);
         auto reload = [&]() {
             if (prefetch) {
-                load_tile_dwords<BITS>(pbase + lane_dw, mine);
-                const long step = p_left == 0 ? 0 : (p_r == TR - 1 ? wrap_dw : row_dw);
+                load_unit(mine);
+                const long step = p_left == 0 ? 0 : (p_r == TR - 1 ? wrap_dw : unit_dw);
                 pbase += step;
                 p_r = p_left == 0 ? p_r : (p_r == TR - 1 ? 0u : p_r + 1);
                 p_left = p_left == 0 ? 0u : p_left - 1;
             }
         };
-        // the 4-bit hybrid keeps what it still needs of the tile row in its own registers,
+        // the 4-bit hybrid keeps what it still needs of the unit in its own registers,
         // so the reload can go out before the arithmetic pairs
         if constexpr (BITS == 4 && LUTMASK != 0) {
             reload();
@@ -584,17 +588,19 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
             reload();
         }
         __builtin_amdgcn_sched_barrier(0);
-        const uint32_t xk[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
 #pragma unroll
-        for (int qq = 0; qq < 16; ++qq) {
-            if (pair_col_half(qq)) acc1 = __builtin_amdgcn_fdot2(as_half2(w2[qq]), as_half2(xk[pair_kk(qq)]), acc1, false);
-            else acc0 = __builtin_amdgcn_fdot2(as_half2(w2[qq]), as_half2(xk[pair_kk(qq)]), acc0, false);
+        for (int h = 0; h < 2; ++h) {
+            const half8_t x = h ? xb : xa;
+            const uint4 b0 = {w2[h], w2[4 + h], w2[8 + h], w2[12 + h]};
+            const uint4 b1 = {w2[2 + h], w2[6 + h], w2[10 + h], w2[14 + h]};
+            acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8_t, b0), acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8_t, b1), acc1, 0, 0, 0);
         }
         ++r;
-        xoff += 32;
+        xoff += 128;
         if (r == TR) {
             flush(piece);
-            acc0 = acc1 = 0.0f;
+            acc0 = acc1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
             ++piece;
             ++cb;
             r = 0;
@@ -602,10 +608,10 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         }
     };
 
-    // whole rings: straight-line, one exit, so that the wait before each tile row's use
+    // whole rings: straight-line, one exit, so that the wait before each unit's use
     // is exactly "all but the RING - 1 loads issued after it"
     const unsigned groups = left / RING;
-    // A wave runs its tile rows at the highest user priority and steps it down over the
+    // A wave runs its units at the highest user priority and steps it down over the
     // second half of its run (to 2 at a half, 1 at three quarters, 0 for the last eighth).
     // Measured on the four launches of a 27B layer set, interleaved runs on one machine:
     // 66.4 us without, 64.9 with a constant 3, 63.3 with quarter steps, 62.9 with these;
@@ -620,7 +626,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         for (int j = 0; j < RING; ++j) stage(own[j], true);
     }
     __builtin_amdgcn_s_setprio(0);
-    // the remaining tile rows (fewer than RING), nested so that each is reached one way only
+    // the remaining units (fewer than RING), nested so that each is reached one way only
     const unsigned tail = left - groups * RING;
     nested_tail<0, RING - 1>(tail, [&](auto J) { stage(own[decltype(J)::value], false); });
     if (r != 0 && uw0 < uw1) flush(piece);
@@ -633,12 +639,16 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         const unsigned cbx = cb_first + cbi;
         if (cbx * 128u >= (unsigned)width) continue;             // a narrower slice of a bundle: nothing there
         const half2_t sv = sv_mine;
-        const unsigned wf = piece_first[cbi], wl = piece_last[cbi];
         float z0 = 0.0f, z1 = 0.0f;
-        for (unsigned wv = wf; wv <= wl; ++wv) {
-            const float2_t part = *(const float2_t*)&red[(wv + cbi) * 128 + 2 * lane];
-            z0 += part.x;
-            z1 += part.y;
+#pragma unroll
+        for (int g = 0; g < kStreamGroups; ++g) {
+            // the groups whose run touches the column block, in k order
+            if (group_start(W0 + g) < (cbx + 1) * TR && group_start(W0 + g + 1) > cbx * TR &&
+                group_start(W0 + g) < group_start(W0 + g + 1)) {
+                const float2_t part = *(const float2_t*)&red[((unsigned)g + cbi) * 128 + 2 * lane];
+                z0 += part.x;
+                z1 += part.y;
+            }
         }
         const bool whole = u0 <= cbx * TR && (cbx + 1) * TR <= u1;
         if (!whole) {
@@ -648,7 +658,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
             const unsigned big = p.rem * (p.q + 1);
             const unsigned wa = ua < big ? div_magic(ua, p.mq1) : p.rem + div_magic(ua - big, p.mq);
             const unsigned wb = ub < big ? div_magic(ub, p.mq1) : p.rem + div_magic(ub - big, p.mq);
-            const unsigned count = (wb >> 4) - (wa >> 4) + 1;
+            const unsigned count = wb / kStreamGroups - wa / kStreamGroups + 1;
             unsigned long long* const word = p.accum + ((size_t)(pslot + cbx) * 128 + 2 * lane);
             const unsigned long long f0 = to_fixed_tagged(z0), f1 = to_fixed_tagged(z1);
             unsigned long long t0 = __hip_atomic_fetch_add(word, f0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + f0;

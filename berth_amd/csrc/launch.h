@@ -63,7 +63,7 @@ constexpr int kAccumSlots = 16384;     // column blocks of a streaming launch (1
 // process call it after changing the environment).
 struct Knobs {
     int gemv_stream;            // BERTH_GEMV_STREAM            0: never take the streaming kernel
-    int gemv_stream_min_units;  // BERTH_GEMV_STREAM_MIN_UNITS  fewest tile rows per wave for which it is taken
+    int gemv_stream_min_units;  // BERTH_GEMV_STREAM_MIN_UNITS  it is taken for more units of 64 x 128 weights than this per wave group
     int gemv_stream_shrink;     // BERTH_GEMV_STREAM_SHRINK     1: fewer workgroups instead of falling back
     int gemv_stream_wgs;        // BERTH_GEMV_STREAM_WGS        cap on the workgroups per problem (0: none)
     int gemv_stream_lut;        // BERTH_GEMV_STREAM_LUT        table mask of the hybrid decode (-1: by size)
