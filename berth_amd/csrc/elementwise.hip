@@ -77,6 +77,13 @@ struct RotateParams {
     int col_blocks, mt;
     RotateTable tab;
 };
+// values k .. k + 7 of a row of a slab in operand order, row blocks of 16 * mt rows one after the other
+__device__ __forceinline__ void store_operand(const RotateParams& p, int slab, int row, int k, half8_t o)
+{
+    const unsigned block = (unsigned)row / (unsigned)(16 * p.mt);
+    *(half8_t*)(p.operand + (size_t)slab * p.operand_stride + block * rows_operand_elements(p.col_blocks * 128, p.mt) +
+                rows_operand_offset(row - (int)block * 16 * p.mt, k, p.mt)) = o;
+}
 template <bool SILU>
 __device__ __forceinline__ void rotate_rows(const RotateParams& p)
 {
@@ -111,9 +118,7 @@ __device__ __forceinline__ void rotate_rows(const RotateParams& p)
         if (live) {
             if (SILU && p.act_out) *(half8_t*)(p.act_out + at) = x;
             *(half8_t*)(out + at) = o;
-            if (p.operand)
-                *(half8_t*)(p.operand + (size_t)slab * p.operand_stride +
-                            rows_operand_offset((int)row, (int)cb * 128 + 8 * l16, p.mt)) = o;
+            if (p.operand) store_operand(p, slab, (int)row, (int)cb * 128 + 8 * l16, o);
         }
     }
 }
@@ -196,7 +201,7 @@ __global__ __launch_bounds__(1024) void add_rms_norm_had_r_128_kernel(NormParams
             for (int j = 0; j < 8; ++j) o[j] = (_Float16)(r[j] * kRsqrt128);
             _Float16* out = p.tab.out[s] ? p.tab.out[s] : p.out + (size_t)s * p.out_stride;
             *(half8_t*)(out + base + e) = o;
-            if (p.operand) *(half8_t*)(p.operand + (size_t)s * p.operand_stride + rows_operand_offset(row, e, p.mt)) = o;
+            if (p.operand) store_operand(p, s, row, e, o);
         }
     }
 }
@@ -232,7 +237,7 @@ std::string launch_rotate(const RotateArgs& a)
     p.in_stride = a.in_stride;
     p.out_stride = a.out_stride;
     p.mt = a.mt;
-    p.operand_stride = rows_operand_elements(a.cols, a.mt);
+    p.operand_stride = (size_t)((a.rows + 16 * a.mt - 1) / (16 * a.mt)) * rows_operand_elements(a.cols, a.mt);
     p.col_blocks = a.cols / 128;
     p.blocks = (long)a.rows * p.col_blocks;
     if (p.blocks >= (1L << 31)) throw std::runtime_error("had_r_128 slabs: too many rows");

@@ -1,10 +1,11 @@
 // Launchers of the EXL3 MFMA GEMM (exl3_gemm_kernel.cuh): dense rows through
 // berth_prefill_exl3_linear / berth_exl3_linear, grouped MoE problems, and the
 // plain fp16 GEMM of crates/berth-kernels/csrc/prefill_lin/linear.cu:387-418.
-#include "exl3_gemm_rows_kernel.cuh"
+#include "exl3_gemm_block_kernel.cuh"
 #include "launch.h"
 #include "rows_operand.cuh"
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <optional>
@@ -68,7 +69,7 @@ struct RowsPlan {
     size_t operand_at = 0;      // bytes into the partial-sum workspace
 };
 
-static unsigned magic(unsigned d) { return (unsigned)((1ull << 32) / d) + 1u; }
+static unsigned magic(unsigned d) { return d == 1 ? 0u : (unsigned)((1ull << 32) / d) + 1u; }
 
 // Fewest units for which the few-row kernel is taken.  Up to 8 rows the alternative is the VALU
 // kernel of exl3_gemv.hip, which rotates the input itself (one launch instead of two) and pays half
@@ -151,12 +152,130 @@ static void run_rows(const RowsPlan& pl, GemmParams& p, int k_bits, int codebook
     p.m_nb = magic((unsigned)p.N / 128);
     p.S = (int)pl.S;
     p.m_s = pl.S ? magic(pl.S) : 0;
-    p.m_q = pl.S ? 0 : magic(pl.q);
+    p.m_q = pl.S ? 0u : magic(pl.q);
     p.m_q1 = magic(pl.q + 1);
     p.lds_bytes = (unsigned)pl.lds;
     gemm_bits(p, k_bits, codebook, -pl.mt, stream, desc, dim3(pl.grid));
     hip_ok(hipGetLastError(), "exl3_gemm_rows_kernel launch");
 }
+
+// ---- row blocks (exl3_gemm_block_kernel)
+struct BlockPlan {
+    bool ok = false;
+    int rows_per_tile = 0, mt = 0, row_blocks = 0;     // mt: tiles of 16 rows a block has room for
+    long units = 0;             // steps of 256 x 128 weights
+    unsigned grid = 0, q = 0, rem = 0, S = 0, spt = 0;
+    size_t operand_at = 0;      // bytes into the partial-sum workspace
+    size_t operand_stride = 0;  // elements of one slab's copy
+};
+
+// 128-row tiles of 256 columns enough to spread over the chip (dispatch_dense)
+static bool fills_128_row_tiles(const Workspace& ws, long nblocks, int size_m)
+{
+    return nblocks * ((size_m + 127) / 128) * 4 >= ws.cu_count;
+}
+
+// When row blocks are taken (more than 32 rows).  Measured against the tiles of exl3_gemm_kernel.cuh at 4 bits,
+// 40..448 rows (K x N, us, tiles -> row blocks):
+//   * enough steps that the second launch and the hand-over pay: one per compute unit up to 64 rows (512x4096 14.0 ->
+//     14.7, 512x16384 20.4 -> 19.1, 4096x4096 23.5 -> 21.0), 2.25 of them above (4096x4096 at 100 rows 24.8 -> 27.0,
+//     7296x2688 33.8 -> 28.4);
+//   * narrow outputs, which would run as 32-row tiles and decode every weight once per 32 rows: always (17408x5120 at
+//     64, 128, 256 and 384 rows 59, 88, 162, 167 -> 32, 46, 72, 100), up to gemm_block_rows;
+//   * wide outputs: a launch of 128-row or 256-row tiles costs the same for any rows up to a multiple of those, row
+//     blocks go by the row.  One row block (5120x34816 at 64 rows 62 -> 51, at 128 rows even) and several of up to 96
+//     rows (160 rows 112 -> 104), not several of up to 128 (256 rows 123 -> 137).
+static BlockPlan plan_block(const Workspace& ws, int slices, int slabs, int size_m, int size_k, int size_n)
+{
+    BlockPlan pl;
+    if (!knobs().gemm_balanced || size_m <= 32 || size_m > knobs().gemm_block_rows || size_n % 128 != 0) return pl;
+    // row blocks of equal height, as few as 128 rows each allow
+    const int blocks_min = (size_m + 127) / 128;
+    pl.rows_per_tile = ((size_m + blocks_min - 1) / blocks_min + 15) / 16 * 16;
+    pl.row_blocks = (size_m + pl.rows_per_tile - 1) / pl.rows_per_tile;
+    pl.mt = std::max(4, (pl.rows_per_tile + 31) / 32 * 2);
+    const unsigned spt = (unsigned)(size_k / 64 + 3) / 4;
+    const unsigned long long tiles = (unsigned long long)slices * (size_n / 128) * pl.row_blocks;
+    const unsigned long long U = tiles * spt;
+    if (U >= (1ull << 30)) return pl;
+    const int least = knobs().gemm_block_steps;
+    if (U < (unsigned long long)(least >= 0 ? least : size_m <= 64 ? 256 : 576)) return pl;
+    if (least < 0 && pl.row_blocks > 1 && pl.rows_per_tile > 96 && fills_128_row_tiles(ws, (long)slices * ((size_n + 255) / 256), size_m))
+        return pl;
+    unsigned long long G = (unsigned long long)ws.cu_count;
+    if (G > U) G = U;
+    unsigned q = (unsigned)(U / G), rem = (unsigned)(U % G), S = 0;
+    const unsigned most = q + (rem ? 1 : 0);
+    if (G >= 2 * tiles) {       // parts of its own for each tile, as for few rows
+        const unsigned s = (unsigned)(G / tiles);
+        if (((spt + s - 1) / s) * 8ull <= most * 9ull) {
+            S = s;
+            G = tiles * s;
+            q = rem = 0;
+        }
+    }
+    if (U * (q + 2) >= (1ull << 32) || U * spt >= (1ull << 32)) return pl;
+    // the workspace holds two partial tiles per workgroup, then the operand copies
+    pl.operand_at = (size_t)G * 2 * pl.rows_per_tile * 512;
+    pl.operand_stride = (size_t)pl.row_blocks * rows_operand_elements(size_k, pl.rows_per_tile / 16);
+    if (pl.operand_at + slabs * pl.operand_stride * 2 > ws.partial_bytes) return pl;
+    pl.ok = true;
+    pl.units = (long)U;
+    pl.grid = (unsigned)G;
+    pl.q = q;
+    pl.rem = rem;
+    pl.S = S;
+    pl.spt = spt;
+    return pl;
+}
+
+static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebook, hipStream_t stream, std::string& desc)
+{
+    const long tiles = (long)(p.num_slices > 0 ? p.num_slices : 1) * (p.N / 128) * pl.row_blocks;
+    p.units = (int)pl.units;
+    p.unit_q = (int)pl.q;
+    p.unit_r = (int)pl.rem;
+    p.S = (int)pl.S;
+    p.tiles_y = pl.row_blocks;
+    p.rows_per_tile = pl.rows_per_tile;
+    p.m_tr = magic(pl.spt);
+    p.m_rt = magic((unsigned)pl.row_blocks);
+    p.m_nb = magic((unsigned)p.N / 128);
+    p.m_s = pl.S ? magic(pl.S) : 0;
+    p.m_q = pl.S ? 0u : magic(pl.q);
+    p.m_q1 = magic(pl.q + 1);
+    p.lds_bytes = (unsigned)block_lds_bytes(pl.mt);
+    gemm_bits(p, k_bits, codebook, -8 - pl.mt, stream, desc, dim3(pl.grid));
+    hip_ok(hipGetLastError(), "exl3_gemm_block_kernel launch");
+    if (pl.S || pl.rem || pl.q % pl.spt) {              // some tile is shared
+        const dim3 grid((unsigned)tiles, (unsigned)(pl.rows_per_tile / 16));
+        hipLaunchKernelGGL(exl3_gemm_finish_kernel, grid, dim3(256), 0, stream, p);
+        hip_ok(hipGetLastError(), "exl3_gemm_finish_kernel launch");
+        desc += " + exl3_gemm_finish grid=" + std::to_string(grid.x) + "x" + std::to_string(grid.y);
+    }
+}
+
+// Which of the two kernels that read operand-ordered copies a dense launch takes, if any.
+struct OperandPlan {
+    RowsPlan rows;
+    BlockPlan block;
+    OperandPlan(const Workspace& ws, int slices, int slabs, int size_m, int size_k, int size_n)
+        : rows(plan_rows(ws, slices, slabs, size_m, size_k, size_n)),
+          block(rows.ok ? BlockPlan{} : plan_block(ws, slices, slabs, size_m, size_k, size_n))
+    {
+        stride = rows.ok ? rows_operand_elements(size_k, rows.mt) : block.operand_stride;
+        at = (_Float16*)((char*)ws.partials + (rows.ok ? rows.operand_at : block.operand_at));
+    }
+    bool ok() const { return rows.ok || block.ok; }
+    int mt() const { return rows.ok ? rows.mt : block.rows_per_tile / 16; }
+    void run(GemmParams& p, int k_bits, int codebook, hipStream_t stream, std::string& desc) const
+    {
+        if (rows.ok) run_rows(rows, p, k_bits, codebook, stream, desc);
+        else run_block(block, p, k_bits, codebook, stream, desc);
+    }
+    _Float16* at = nullptr;     // the first slab's copy
+    size_t stride = 0;          // elements between slabs
+};
 
 // Tile shape and work split of a dense launch: `nblocks` column blocks of 256 (all slices of
 // a bundle together), size_m rows.  Fills the split fields of p and launches.
@@ -166,8 +285,7 @@ static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int c
     // 128-row tiles decode a weight once per 128 rows, but need enough tiles to spread
     // over the chip; narrow outputs (few column tiles) run as 32-row tiles instead
     p.cstride = gemm_counter_stride((long)nblocks * ((size_m + 31) / 32));
-    const long tiles128 = (long)nblocks * ((size_m + 127) / 128);
-    const int mb_plain = (size_m <= 32 || tiles128 * 4 < ws.cu_count) ? 1 : 4;
+    const int mb_plain = (size_m <= 32 || !fills_128_row_tiles(ws, nblocks, size_m)) ? 1 : 4;
     const int KB = size_k / 128;
     p.tile0 = 0;
     const int balance = knobs().gemm_balanced;
@@ -229,7 +347,7 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     if (!scratch) scope.emplace(a.stream);
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
-    const RowsPlan rows = plan_rows(ws, 1, 1, a.size_m, a.size_k, a.size_n);
+    const OperandPlan plan(ws, 1, 1, a.size_m, a.size_k, a.size_n);
     RotateArgs rot;
     rot.in = a.a;
     rot.up = a.a_up;
@@ -239,15 +357,15 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     rot.rows = a.size_m;
     rot.cols = a.size_k;
     rot.stream = a.stream;
-    if (rows.ok) {
-        rot.operand = (char*)ws.partials + rows.operand_at;
-        rot.mt = rows.mt;
+    if (plan.ok()) {
+        rot.operand = plan.at;
+        rot.mt = plan.mt();
     }
     std::string d0 = launch_rotate(rot);
     GemmParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
-    p.a_had[0] = (const _Float16*)(rows.ok ? rot.operand : a.a_had);
+    p.a_had[0] = (const _Float16*)(plan.ok() ? plan.at : a.a_had);
     p.lin.trellis = (const uint32_t*)a.trellis;
     p.lin.svh = (const _Float16*)a.svh;
     p.c[0] = a.c;
@@ -260,7 +378,7 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     p.partials = ws.partials;
     p.counters = ws.counters;
     std::string desc;
-    if (rows.ok) run_rows(rows, p, a.k_bits, a.codebook, a.stream, desc);
+    if (plan.ok()) plan.run(p, a.k_bits, a.codebook, a.stream, desc);
     else dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (a.size_n + 255) / 256, a.stream, desc);
     return d0 + " + " + desc + (a.out_fp32 ? " out=f32" : " out=f16");
 }
@@ -277,10 +395,10 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
     Workspace& ws = scope.ws;
     throw_pending_device_fault(ws);
     const int slabs = sliced ? m.num_had_src : m.bszm_out;
-    const RowsPlan rows = plan_rows(ws, m.bszm_out, slabs, m.size_m, m.size_k, m.size_n);
+    const OperandPlan plan(ws, m.bszm_out, slabs, m.size_m, m.size_k, m.size_n);
     // what the kernel multiplies: the rotated rows, or their copy in operand order
-    const size_t slab_stride = rows.ok ? rows_operand_elements(m.size_k, rows.mt) : (size_t)m.size_m * m.size_k;
-    const _Float16* const slab0 = (const _Float16*)(rows.ok ? (char*)ws.partials + rows.operand_at : m.a_had);
+    const size_t slab_stride = plan.ok() ? plan.stride : (size_t)m.size_m * m.size_k;
+    const _Float16* const slab0 = (const _Float16*)(plan.ok() ? plan.at : m.a_had);
     GemmParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
@@ -342,15 +460,15 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
     rot.rows = m.size_m;
     rot.cols = m.size_k;
     rot.stream = m.stream;
-    if (rows.ok) {
-        rot.operand = (void*)slab0;
-        rot.mt = rows.mt;
+    if (plan.ok()) {
+        rot.operand = plan.at;
+        rot.mt = plan.mt();
     }
     std::string d0 = launch_rotate(rot);
     const long nblocks = (long)m.bszm_out * ((m.size_n + 255) / 256);
     if (nblocks * ((m.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3_mgemm: too many output tiles");
     std::string desc;
-    if (rows.ok) run_rows(rows, p, m.k_bits, m.codebook, m.stream, desc);
+    if (plan.ok()) plan.run(p, m.k_bits, m.codebook, m.stream, desc);
     else dispatch_dense(ws, p, m.k_bits, m.codebook, m.size_m, m.size_k, (int)nblocks, m.stream, desc);
     return std::string(sliced ? "sliced x" : "uniform x") + std::to_string(m.bszm_out) + (m.host_lists ? " by value " : " ") + d0 +
            " + " + desc + (m.c_fp32 ? " out=f32" : " out=f16");
@@ -362,7 +480,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
     LaunchScope scope(a.stream);
     Workspace& ws = scope.ws;
     throw_pending_device_fault(ws);
-    const RowsPlan rows = plan_rows(ws, 2, 2, a.size_m, a.size_k, a.size_n);
+    const OperandPlan plan(ws, 2, 2, a.size_m, a.size_k, a.size_n);
     GemmParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
@@ -394,17 +512,16 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
     rot.rows = a.size_m;
     rot.cols = a.size_k;
     rot.stream = a.stream;
-    if (rows.ok) {
-        rot.operand = (char*)ws.partials + rows.operand_at;
-        rot.mt = rows.mt;
-        for (int i = 0; i < 2; ++i)
-            p.slice[i].a_had = (const _Float16*)rot.operand + i * rows_operand_elements(a.size_k, rows.mt);
+    if (plan.ok()) {
+        rot.operand = plan.at;
+        rot.mt = plan.mt();
+        for (int i = 0; i < 2; ++i) p.slice[i].a_had = plan.at + i * plan.stride;
     }
     std::string d0 = launch_rotate(rot);
     const long nblocks = 2L * ((a.size_n + 255) / 256);
     if (nblocks * ((a.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3 linear pair: too many output tiles");
     std::string desc;
-    if (rows.ok) run_rows(rows, p, a.k_bits, a.codebook, a.stream, desc);
+    if (plan.ok()) plan.run(p, a.k_bits, a.codebook, a.stream, desc);
     else dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (int)nblocks, a.stream, desc);
     return "pair " + d0 + " + " + desc + " out=f16";
 }

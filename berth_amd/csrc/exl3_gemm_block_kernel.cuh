@@ -1,0 +1,346 @@
+// EXL3 linear for more than 32 rows: row blocks of up to 128 rows, every weight decoded once per
+// block and multiplied on the matrix units while other waves decode.
+//
+//   c = Hh(a_had @ W) * svh (+ out_add),   a_had = Hh(a * suh) rotated by an earlier launch
+//
+// What bounds it: issue and power.  Per step a wave decodes 32 weights a lane (about 140 vector
+// instructions) and issues 4 * MT v_mfma_f32_16x16x32_f16.  In loops of nothing else the decode of a
+// step takes 1.15 us (at 2.16 GHz, what the card holds under it) and the MFMAs of 128 rows 1.36 us
+// (1.66 GHz); both, interleaved in their proportion, 1.65 us; the kernel 1.9.  (Eight waves of
+// 32x32x16 MFMAs, decode interleaved by the instruction, loads three half steps ahead: 2.05.)
+//
+//   * Tile: rows_per_tile rows (a multiple of 16, at most 16 * MT) x 128 columns.  Tiles of one
+//     column block are neighbours, so their weights are in the caches for the next row block.
+//   * Sixteen waves: four column groups of 32 columns x four k groups.  A step is 256 rows of K,
+//     64 per k group (octet layout and operand assignment as in the few-row kernel).
+//   * The k groups 0, 1 and 2, 3 run half a step apart, a barrier between the halves: while one
+//     pair decodes, the other multiplies.  A SIMD holds one wave of each k group, so both of its
+//     pipes always have two waves to choose from; left to themselves, waves that meet at one
+//     barrier per step decode together and then queue for the matrix pipe.
+//   * A tile, double-buffered: 256 k of every row, from the copy of the rotated rows in operand
+//     order (rows_operand_offset) by direct global-to-LDS loads of 1 KB.  In memory a step is one
+//     contiguous run, so the workgroups of a die draw on all channels of its L2, and operand
+//     reads from LDS are lane-linear.
+//   * The steps of the launch, tile-major, are dealt out evenly to one workgroup per compute unit
+//     (or, with few tiles, each tile is cut into S parts).  At the end of a tile the k groups' sums
+//     meet in LDS.  A tile inside one workgroup's steps is finished there; of a shared one every
+//     sharer leaves its sums in the workspace, and a second launch adds them in k order and
+//     finishes it (exl3_gemm_finish_kernel: inside the first launch the same work falls to the
+//     last sharer alone, which reads half a megabyte per tile through one compute unit: 28 us
+//     instead of 13 outside the steps).
+//
+// Measured (27B layer, 4 bits, whole layer on the host clock, against 32-row and 128-row tiles): 33
+// rows 181 -> 135 us, 64 rows 196 -> 151, 100 rows 245 -> 190, 256 rows 420 -> 311, 384 rows 548 -> 441.
+#pragma once
+
+#include "exl3_gemm_rows_kernel.cuh"
+
+namespace berth {
+
+__host__ __device__ constexpr size_t block_lds_bytes(int mt)
+{
+    // A buffers / the k groups' register dumps (16 KB per 16 rows), or half of that and the
+    // row-major tile behind it; then the output scales
+    return (size_t)mt * (8192 + 16 * kRowsStride * 4) + 256;
+}
+
+// sixteen bytes a lane from base + offset to LDS at lds_at + 16 * lane
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, uint32_t lds_at)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 : : "s"(lds_at), "v"(offset), "s"(base) : "m0", "memory");
+}
+
+// The end of one output row of a 128-column block, sixteen lanes with eight sums each: Hadamard, svh,
+// the optional addend, the store (`live` false: a lane group past the last row, which only takes part
+// in the exchanges).
+__device__ __forceinline__ void block_finish_row(const GemmParams& p, const RowsBlock& b, float (&v)[8], const half8_t sv,
+                                                 const int row, const bool live, const int lane)
+{
+    had128_row16(v, lane);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (v[e] * kRsqrt128) * (float)sv[e];
+    if (!live) return;
+    const size_t at = (size_t)row * b.ldc + b.n0 + 8 * (lane & 15);
+    if (p.out_fp32) {
+        if (p.out_add) {
+            const global_ptr<const float4_t> add = (global_ptr<const float4_t>)(as_global(p.out_add) + at);
+            const float4_t a0 = add[0], a1 = add[1];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { v[e] += a0[e]; v[4 + e] += a1[e]; }
+        }
+        const global_ptr<float4_t> dst = (global_ptr<float4_t>)(as_global((float*)b.c) + at);
+        dst[0] = float4_t{v[0], v[1], v[2], v[3]};
+        dst[1] = float4_t{v[4], v[5], v[6], v[7]};
+    } else {
+        half8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (_Float16)v[e];
+        *(global_ptr<half8_t>)(as_global((_Float16*)b.c) + at) = o;
+    }
+}
+
+template <int BITS, int CB, int MT>         // MT (even): tiles of 16 rows a block can hold
+__global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int tile_dw = 8 * BITS;
+    constexpr int kBuf = MT * 8192;                     // bytes of one A buffer: [k group][row tile][k half][lane][16]
+    constexpr int kLoads = MT / 2;                      // A loads of a wave per step
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cg = wave & 3, kg = wave >> 2;
+    const int l16 = lane & 15, lg = lane >> 4;
+    const unsigned TR4 = (unsigned)p.K >> 6;
+    const unsigned SPT = (TR4 + 3) >> 2;                // steps per tile
+    const unsigned RT = (unsigned)p.tiles_y;            // row blocks
+    const int BM = p.rows_per_tile;
+
+    // ---- this workgroup's steps [u0, u1)
+    const unsigned w = blockIdx.x;
+    const unsigned q = (unsigned)p.unit_q, rem = (unsigned)p.unit_r;
+    const unsigned S = (unsigned)p.S;
+    unsigned u0 = w * q + min(w, rem), u1 = (w + 1) * q + min(w + 1, rem);
+    if (S) {
+        const unsigned tile = div_exact(w, p.m_s), part = w - tile * S;
+        u0 = tile * SPT + div_exact(part * SPT, p.m_s);
+        u1 = tile * SPT + div_exact((part + 1) * SPT, p.m_s);
+    }
+    const unsigned t_first = div_exact(u0, p.m_tr), t_last = div_exact(u1 - 1, p.m_tr);
+
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    float* const dump = (float*)smem;                   // [2][4 column groups][8 * MT][64]
+    float* const z = (float*)(smem + MT * 8192);        // [16 * MT][kRowsStride]
+    uint32_t* const sv_lds = (uint32_t*)(z + 16 * MT * kRowsStride);
+
+    // ---- operands
+    uint32_t own[2][BITS];
+    const char* t_base = nullptr;                       // trellis of the segment's tile, this wave's k group, step 0
+    long t_step = 0;                                    // bytes per step
+    uint32_t t_off = 0, t_kg = 0;                       // per lane; bytes from k group 0 to this one
+    const char* a_base = nullptr;                       // rotated rows of the tile
+    const uint32_t a_unit = (uint32_t)BM * 128;         // bytes of 64 k of the block
+    auto seek = [&](unsigned tile) {
+        const unsigned cb = div_exact(tile, p.m_rt);
+        const RowsBlock b = rows_block(p, cb);
+        a_base = (const char*)rows_uniform(b.a_had + (size_t)((tile - cb * RT) * (unsigned)BM) * p.K);
+        if (b.empty) {                                  // read anything valid, use nothing
+            t_base = a_base;
+            t_step = 0;
+            t_off = t_kg = 0;
+        } else {
+            const uint32_t row_bytes = (uint32_t)(b.ldc >> 4) * (tile_dw * 4);
+            t_step = 16 * (long)row_bytes;
+            t_kg = (uint32_t)kg * 4 * row_bytes;
+            t_base = (const char*)rows_uniform(b.trellis) + (size_t)(b.n0 >> 4) * (tile_dw * 4) + t_kg;
+            t_off = (uint32_t)lg * row_bytes + (uint32_t)(cg * 16 + l16) * (BITS * 4);
+        }
+    };
+    auto fetch_t = [&](int j, unsigned s) {
+        // (in the last step of a K that is no multiple of 256 a k group may have no rows: it reads those of group 0)
+        const char* src = t_base + (size_t)s * t_step - (s * 4 + (unsigned)kg < TR4 ? 0u : t_kg);
+        load_tile_dwords<BITS>((global_ptr<const uint32_t>)(as_global(src) + t_off), own[j]);
+    };
+    auto a_source = [&](unsigned s) {
+        return a_base + (size_t)(s * 4 + (s * 4 + (unsigned)kg < TR4 ? (unsigned)kg : 0u)) * a_unit;
+    };
+    auto fetch_a = [&](const char* src, int buf, int j) {       // (a lower block than 16 * MT rows: the last piece again)
+        const uint32_t at = min((uint32_t)(cg * kLoads + j) * 1024u, a_unit - 1024u);
+        load_to_lds(src + at, (uint32_t)lane * 16, lds0 + (uint32_t)(buf * kBuf + kg * 2048 * MT) + at);
+    };
+    const uint32_t ra = (uint32_t)(kg * 2048 * MT + lane * 16);     // this lane's part of its k group's first operand
+
+    float4_t acc[MT][2];
+    auto stage = [&](int j, unsigned s, unsigned last) {
+        const uint32_t prev = fetch_prev(lane, own[j][BITS - 1]);
+        uint32_t w2[16];
+        decode_lane<BITS, CB>(own[j], prev, w2);
+        if (s * 4 + (unsigned)kg >= TR4) {              // a k group past the end of K multiplies zeros
+#pragma unroll
+            for (int i = 0; i < 16; ++i) w2[i] = 0;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(w2[i]));       // decoded here, not behind the barrier
+        // this step's A loads of this wave are older than the next step's trellis loads (one or
+        // more), so they have landed when at most one load is outstanding; behind the barrier the
+        // other three waves' have, too, and everybody has left the other buffer
+        asm volatile("s_waitcnt vmcnt(1)\n\ts_barrier" ::: "memory");
+        // (on the segment's last step the loads bring in the same step again, unused: no branch)
+        const char* const next = a_source(min(s + 1, last));
+        half8_t b[2][2];                                // [k half][column half]
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const uint4 v = {w2[2 * f + h], w2[4 + 2 * f + h], w2[8 + 2 * f + h], w2[12 + 2 * f + h]};
+                b[h][f] = __builtin_bit_cast(half8_t, v);
+            }
+        // the operands of the next sixteen rows are read behind the MFMAs of these
+        const unsigned char* const a0 = smem + j * kBuf + ra;
+        const unsigned char* const a1 = a0 + 1024;
+        half8_t x[2][2];
+        x[0][0] = *(const half8_t*)a0;
+        x[0][1] = *(const half8_t*)a1;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            if (mt + 1 < MT) {
+                x[(mt + 1) & 1][0] = *(const half8_t*)(a0 + (mt + 1) * 2048);
+                x[(mt + 1) & 1][1] = *(const half8_t*)(a1 + (mt + 1) * 2048);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int f = 0; f < 2; ++f)
+                    acc[mt][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[mt & 1][h], b[h][f], acc[mt][f], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            // the next step's loads go out one at a time behind MFMAs: issued together ahead of
+            // them they hold every wave of the group up at the memory pipe
+            if (mt < kLoads) fetch_a(next, j ^ 1, mt);
+            else if (mt == kLoads) fetch_t(j, min(s + 2, last));
+        }
+        asm volatile("s_barrier" ::: "memory");
+    };
+
+    seek(t_first);
+    {
+        const unsigned s0 = u0 - t_first * SPT, s1 = min(SPT, s0 + (u1 - u0));
+        fetch_t(0, s0);
+        fetch_t(1, min(s0 + 1, s1 - 1));
+    }
+    for (unsigned tile = t_first; tile <= t_last; ++tile) {
+        const unsigned base = tile * SPT;
+        const unsigned s0 = u0 > base ? u0 - base : 0u, s1 = min(SPT, u1 - base);
+        const unsigned cb = div_exact(tile, p.m_rt);
+        const RowsBlock b = rows_block(p, cb);
+        const int m0 = (int)(tile - cb * RT) * BM;
+        const int rows = min(BM, p.M - m0);
+        uint32_t sv_mine = 0;
+        if (wave == 0 && !b.empty) sv_mine = as_global((const uint32_t*)(b.svh + b.n0))[lane];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) fetch_a(a_source(s0), 0, j);
+        // (the segment's first trellis loads are older than these: its first step waits for everything)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (kg >= 2) asm volatile("s_barrier" ::: "memory");       // half a step behind
+        unsigned s = s0;
+        for (; s + 1 < s1; s += 2) {
+            stage(0, s, s1 - 1);
+            stage(1, s + 1, s1 - 1);
+        }
+        if (s < s1) stage(0, s, s1 - 1);
+        if (kg < 2) asm volatile("s_barrier" ::: "memory");
+        if (tile < t_last) {                            // the next tile's first steps, behind the finish of this one
+            seek(tile + 1);
+            fetch_t(0, 0);
+            fetch_t(1, min(1u, min(SPT, u1 - base - SPT) - 1));
+        }
+        // ---- the k groups' sums: (0 + 2) + (1 + 3), through register dumps
+        float* const mine = dump + ((size_t)(kg & 1) * 4 + cg) * (8 * MT * 64) + lane;
+        __syncthreads();
+        if (kg >= 2) {
+#pragma unroll
+            for (int i = 0; i < 8 * MT; ++i) mine[i * 64] = acc[i >> 3][(i >> 2) & 1][i & 3];
+        }
+        __syncthreads();
+        if (kg < 2) {
+#pragma unroll
+            for (int i = 0; i < 8 * MT; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] += mine[i * 64];
+        }
+        if (kg == 1) {                                  // its own region has been read by nobody else
+#pragma unroll
+            for (int i = 0; i < 8 * MT; ++i) mine[i * 64] = acc[i >> 3][(i >> 2) & 1][i & 3];
+        }
+        __syncthreads();
+        if (kg == 0) {
+            const float* const other = dump + ((size_t)4 + cg) * (8 * MT * 64) + lane;
+#pragma unroll
+            for (int i = 0; i < 8 * MT; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] += other[i * 64];
+        }
+        if (wave == 0) sv_lds[lane] = sv_mine;
+        __syncthreads();                                // the row-major tile lies over the second dump
+        if (kg == 0) {
+            const int col = cg * 32 + (l16 >> 3) * 16 + (l16 & 7);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float* const row = z + (mt * 16 + 4 * lg + r) * kRowsStride + col;
+                    row[0] = acc[mt][0][r];
+                    row[8] = acc[mt][1][r];
+                }
+        }
+        __syncthreads();
+        if (!b.empty) {
+            // sixteen lanes a row, eight columns each: a wave takes four rows at a time
+            const bool whole = s0 == 0 && s1 == SPT;
+            float* const part = p.partials + ((size_t)w * 2 + (tile == t_first ? 0 : 1)) * BM * 128;
+#pragma unroll
+            for (int pass = 0; pass < MT / 4 + (MT % 4 != 0); ++pass) {
+                const int r = pass * 64 + wave * 4 + lg;
+                if (pass * 64 + wave * 4 >= rows) break;
+                const float4_t* const zr = (const float4_t*)&z[min(r, 16 * MT - 1) * kRowsStride + 8 * l16];
+                const float4_t v0 = zr[0], v1 = zr[1];
+                if (whole) {
+                    float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+                    block_finish_row(p, b, v, ((const half8_t*)sv_lds)[l16], m0 + r, r < rows, lane);
+                } else if (r < rows) {
+                    const global_ptr<float4_t> dst = (global_ptr<float4_t>)as_global(part + r * 128 + 8 * l16);
+                    dst[0] = v0;
+                    dst[1] = v1;
+                }
+            }
+        }
+        __syncthreads();                                // the next tile's A loads land here
+    }
+}
+
+// Finishes the tiles that several workgroups of the launch before share: adds their sums in k order,
+// then output Hadamard, svh, the optional addend and the store.  blockIdx.x = tile, blockIdx.y =
+// sixteen rows of it; sixteen lanes a row, eight columns each.  Bound by the bytes of the sums,
+// which are still in the caches.
+static __global__ __launch_bounds__(256) void exl3_gemm_finish_kernel(GemmParams p)
+{
+    const unsigned SPT = (((unsigned)p.K >> 6) + 3) >> 2, RT = (unsigned)p.tiles_y;
+    const unsigned q = (unsigned)p.unit_q, rem = (unsigned)p.unit_r, S = (unsigned)p.S;
+    const unsigned tile = blockIdx.x;
+    auto owner = [&](unsigned x) {
+        const unsigned big = rem * (q + 1);
+        return x < big ? div_exact(x, p.m_q1) : rem + div_exact(x - big, p.m_q);
+    };
+    const unsigned wa = S ? tile * S : owner(tile * SPT), wb = S ? tile * S + S - 1 : owner(tile * SPT + SPT - 1);
+    if (wa == wb) return;                               // finished by its only workgroup
+    const unsigned cb = div_exact(tile, p.m_rt);
+    const RowsBlock b = rows_block(p, cb);
+    if (b.empty) return;
+    const int lane = threadIdx.x & 63, l16 = lane & 15;
+    const int BM = p.rows_per_tile, m0 = (int)(tile - cb * RT) * BM;
+    const int row = (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4);
+    const int rows = min(BM, p.M - m0);
+    if ((int)blockIdx.y * 16 + (int)(threadIdx.x >> 6) * 4 >= rows) return;
+    const int r = min(row, rows - 1);
+    // the tile is the first of every sharer's range but, unless that starts with it, the first sharer's
+    const unsigned slot_a = S || wa * q + min(wa, rem) >= tile * SPT ? 0u : 1u;
+    const half8_t sv = ((global_ptr<const half8_t>)as_global(b.svh + b.n0))[l16];
+    float v[8] = {};
+    for (unsigned x = wa; x <= wb; x += 4) {
+        float4_t part[4][2];
+#pragma unroll
+        for (unsigned i = 0; i < 4; ++i) {
+            const unsigned xi = min(x + i, wb);
+            const global_ptr<const float4_t> src = (global_ptr<const float4_t>)as_global(
+                p.partials + ((size_t)xi * 2 + (xi == wa ? slot_a : 0u)) * BM * 128 + r * 128 + 8 * l16);
+            part[i][0] = src[0];
+            part[i][1] = src[1];
+        }
+#pragma unroll
+        for (unsigned i = 0; i < 4; ++i)
+            if (x + i <= wb) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] += part[i][e >> 2][e & 3];
+            }
+    }
+    block_finish_row(p, b, v, sv, m0 + row, row < rows, lane);
+}
+
+}  // namespace berth

@@ -2,7 +2,7 @@
 // exl3_gemm_cb{0,1,2}.hip with BERTH_GEMM_CB defined): 32-row and 128-row tiles for
 // every bit rate, the balanced variant of the 128-row kernel, and the 256-row kernel.
 #include "exl3_gemm_kernel.cuh"
-#include "exl3_gemm_rows_kernel.cuh"
+#include "exl3_gemm_block_kernel.cuh"
 #include "exl3_gemm_wide_kernel.cuh"
 #include "launch.h"
 
@@ -81,12 +81,28 @@ static void gemm_launch_rows(const GemmParams& p, hipStream_t stream, std::strin
            (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
 }
 
+// row blocks of up to 16 * MT rows; mb = -8 - MT
+template <int BITS, int CB, int MT>
+static void gemm_launch_block(const GemmParams& p, hipStream_t stream, std::string& desc, dim3 grid)
+{
+    static bool raised[64] = {};
+    raise_dynamic_lds_limit((const void*)exl3_gemm_block_kernel<BITS, CB, MT>, 160 * 1024, raised,
+                            "exl3_gemm_block_kernel shared-memory attribute");
+    hipLaunchKernelGGL((exl3_gemm_block_kernel<BITS, CB, MT>), grid, dim3(1024), p.lds_bytes, stream, p);
+    desc = "exl3_gemm_kernel/block<" + std::to_string(BITS) + "," + std::to_string(CB) + "," +
+           std::to_string(p.rows_per_tile) + "x128> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
+           (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
+}
+
 template <int BITS, int CB>
 static void gemm_launch(const GemmParams& p, int mb, hipStream_t stream, std::string& desc, dim3 grid)
 {
     if (p.max_big > 0) gemm_launch_mixed<BITS, CB>(p, stream, desc, grid);
     else if (mb == -1) gemm_launch_rows<BITS, CB, 1>(p, stream, desc, grid);
     else if (mb == -2) gemm_launch_rows<BITS, CB, 2>(p, stream, desc, grid);
+    else if (mb == -12) gemm_launch_block<BITS, CB, 4>(p, stream, desc, grid);
+    else if (mb == -14) gemm_launch_block<BITS, CB, 6>(p, stream, desc, grid);
+    else if (mb == -16) gemm_launch_block<BITS, CB, 8>(p, stream, desc, grid);
     else if (mb == 1) gemm_launch_mb<BITS, CB, 1>(p, stream, desc, grid);
     else if (mb == 8) gemm_launch_wide<BITS, CB>(p, stream, desc, grid);
     else gemm_launch_mb<BITS, CB, 4>(p, stream, desc, grid);

@@ -95,9 +95,13 @@ struct GemmParams {
     const int* n_stride_list;
     const int* had_src_list;
     // few-row launches (exl3_gemm_rows_kernel): unit_q / unit_r deal out units of 64 x 128 weights;
-    // or, with S > 0, cut every column block into S parts; floor(2^32 / d) + 1 for d = K / 64,
+    // or, with S > 0, cut every column block into S parts; floor(2^32 / d) + 1 (0 for d = 1) for d = K / 64,
     // N / 128, unit_q, unit_q + 1, S (exact for the operands used)
-    unsigned m_tr, m_nb, m_q, m_q1, m_s;
+    // The row-block launches (exl3_gemm_block_kernel) deal out steps of 256 x 128 weights of tiles
+    // of rows_per_tile rows, tiles_y row blocks per column block: m_tr for the steps of a tile,
+    // m_rt for tiles_y.
+    unsigned m_tr, m_nb, m_q, m_q1, m_s, m_rt;
+    int rows_per_tile;
     unsigned lds_bytes;         // dynamic LDS of the launch
     const float* out_add;       // optional fp32 [M][N] (one linear, fp32 output): added to the output
     GemmSlice slice[kGemmMaxSlices];

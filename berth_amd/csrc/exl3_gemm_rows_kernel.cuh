@@ -47,6 +47,9 @@ __host__ __device__ constexpr size_t rows_lds_bytes(int rows, int ncb)
     return (size_t)(ncb + 3) * rows * kRowsStride * 4 + (size_t)ncb * 256 + 16;
 }
 
+// x / d for the launch's exact divisors, m = floor(2^32 / d) + 1 (0 for d = 1)
+__device__ __forceinline__ unsigned div_exact(unsigned x, unsigned m) { return m ? __umulhi(x, m) : x; }
+
 // the tensors of one 128-column block of the launch
 struct RowsBlock {
     const uint32_t* trellis;    // of the linear (of the whole weight's slice)
@@ -69,7 +72,7 @@ __device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsig
     b.empty = false;
     if (p.num_slices > 0) {
         const unsigned nb = (unsigned)p.N >> 7;
-        const unsigned sl = __umulhi(cb, p.m_nb);
+        const unsigned sl = div_exact(cb, p.m_nb);
         b.n0 = (int)(cb - sl * nb) * 128;
         int width = p.N;
         if (p.b_list) {
@@ -126,12 +129,12 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     const unsigned S = (unsigned)p.S;
     unsigned u0 = w * q + min(w, rem), u1 = (w + 1) * q + min(w + 1, rem);
     if (S) {
-        const unsigned blk = __umulhi(w, p.m_s), part = w - blk * S;
-        u0 = blk * TR4 + __umulhi(part * TR4, p.m_s);
-        u1 = blk * TR4 + __umulhi((part + 1) * TR4, p.m_s);
+        const unsigned blk = div_exact(w, p.m_s), part = w - blk * S;
+        u0 = blk * TR4 + div_exact(part * TR4, p.m_s);
+        u1 = blk * TR4 + div_exact((part + 1) * TR4, p.m_s);
     }
     const unsigned L = u1 - u0;
-    const unsigned cb_first = __umulhi(u0, p.m_tr), cb_last = __umulhi(u1 - 1, p.m_tr);
+    const unsigned cb_first = div_exact(u0, p.m_tr), cb_last = div_exact(u1 - 1, p.m_tr);
     const unsigned ncb = cb_last - cb_first + 1;
     const unsigned w0 = u0 + (L * (unsigned)kg >> 2), w1 = u0 + (L * (unsigned)(kg + 1) >> 2);
 
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     unsigned* const flags = sv_lds + ncb * 64;
 
     // ---- the walk's operands: a pointer pair that runs two units ahead of the decode
-    unsigned f_cb = __umulhi(w0, p.m_tr);
+    unsigned f_cb = div_exact(w0, p.m_tr);
     unsigned f_k = w0 - f_cb * TR4, f_left = w1 - w0;
     const char* f_t;
     const char* f_a;
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     float4_t acc[MT][2];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    unsigned cb = __umulhi(w0, p.m_tr);
+    unsigned cb = div_exact(w0, p.m_tr);
     unsigned k = w0 - cb * TR4;
     // piece of (quarter, column block): the quarters are consecutive runs, so kg + (cb - cb_first)
     // names each of them once
@@ -326,8 +329,8 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     // workgroup in; the last sharer to arrive adds the parts in k order and finishes the block
     auto owner = [&](unsigned x) {
         const unsigned big = rem * (q + 1);
-        if (S) return __umulhi(x, p.m_tr) * S + (x % TR4 ? S - 1 : 0u);     // asked for a block's first or last unit
-        return x < big ? __umulhi(x, p.m_q1) : rem + __umulhi(x - big, p.m_q);
+        if (S) return div_exact(x, p.m_tr) * S + (x % TR4 ? S - 1 : 0u);     // asked for a block's first or last unit
+        return x < big ? div_exact(x, p.m_q1) : rem + div_exact(x - big, p.m_q);
     };
     wait_own_stores();
     __syncthreads();

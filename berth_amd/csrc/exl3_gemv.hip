@@ -89,6 +89,7 @@ static StreamPlan plan_stream(const Workspace& ws, int problems, int K, int N)
         Gp = (int)(U / (min_units * kStreamGroups));
         if (Gp < 1) return pl;
     }
+    if (Gp == 1 && problems > 1) return pl;             // the multiplier below has no form for a divisor of one
     const unsigned groups = (unsigned)Gp * kStreamGroups;
     const unsigned q = (unsigned)(U / groups), rem = (unsigned)(U % groups);
     // exact division by multiply-high needs dividend * divisor < 2^32

@@ -73,6 +73,8 @@ struct Knobs {
     int gemm_wg_per_cu;         // BERTH_GEMM_WG_PER_CU
     int gemm_balanced;          // BERTH_GEMM_BALANCED
     int gemm_rows256;           // BERTH_GEMM_ROWS256
+    int gemm_block_steps;       // BERTH_GEMM_BLOCK_STEPS       fewest steps for the row-block kernel, whatever the shape (-1: by shape)
+    int gemm_block_rows;        // BERTH_GEMM_BLOCK_ROWS        most rows for which the row-block kernel is taken (0: never)
     int gemm_rows_units;        // BERTH_GEMM_ROWS_UNITS        fewest units for which the few-row kernel is taken (0: never, -1: by row count)
     int counter_stride;         // BERTH_COUNTER_STRIDE         cap on the words between arrival counters (1..32)
     int moe_big_min;            // BERTH_MOE_BIG_MIN
@@ -247,7 +249,7 @@ std::string launch_gemm_bundle(const MgemmArgs& args);
 // s * in_stride and the slabs out_stride elements apart (or at out_host[s], by-value scales only);
 // suh(s) from the device list, or from the host array when the list is null.  With `up` the input
 // is silu(in) * up, which also goes to act_out unless null.  `operand` (optional): a second copy in
-// the operand order of the few-row kernel, for mt tiles of 16 rows.
+// the operand order of the MFMA kernels, row blocks of mt tiles of 16 rows.
 struct RotateArgs {
     const void* in = nullptr;
     size_t in_stride = 0;

@@ -1,0 +1,74 @@
+"""The row-block MFMA kernel (more than 32 rows; blocks of up to 128 rows x 128 columns, steps of
+256 rows of K dealt out evenly) at the sizes where it can go wrong, against the oracle: blocks
+that are full, of one row more than a tile of sixteen, of every height class; K that leaves
+k groups of the last step empty; tiles inside one workgroup and shared by many; bundles with
+narrower slices.  Bar: rtol 2e-3 / atol 1e-3 of the oracle's fp32 sums; a second call gives the
+same bits."""
+import numpy as np
+import pytest
+import torch
+
+from berth_amd import kernels as K
+from berth_amd import synth
+from berth_amd.kernels import Codebook, OutDtype
+from oracle import oracle as O
+from tests.gpu_util import DEV, close, dev, host_f16, host_u16, knobs
+from tests.test_gpu_linear import _run_linear
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _every_size():
+    with knobs(BERTH_GEMM_BLOCK_ROWS=1 << 30, BERTH_GEMM_BLOCK_STEPS=0):
+        yield
+
+
+@pytest.mark.parametrize("rows,Kk,N,bits,cb,fp32", [
+    (33, 128, 128, 4, 2, True),         # one step with two of four k groups, one workgroup
+    (48, 256, 256, 3, 1, False),        # one full step
+    (49, 384, 1280, 5, 0, True),        # two steps, the second half empty
+    (64, 4096, 384, 2, 2, False),       # three tiles cut into many parts
+    (65, 1408, 640, 6, 2, True),        # 80-row blocks
+    (97, 2176, 256, 8, 2, False),       # 112-row blocks
+    (128, 1024, 1024, 4, 2, True),
+    (129, 1024, 1152, 7, 1, True),      # two blocks of 80 rows, the second short
+    (300, 640, 4352, 1, 2, False),      # three blocks; more tiles than fit the parts: ranges across tiles
+    (520, 256, 8192, 4, 2, True),       # five blocks, several whole tiles per workgroup
+])
+def test_row_blocks_match_the_oracle_and_repeat(rows, Kk, N, bits, cb, fp32):
+    got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, bits, cb, fp32, 60 + rows, prefill=True)
+    assert "exl3_gemm_kernel/block" in launch, launch
+    assert np.array_equal(ah, want_ah), launch
+    bad, worst = close(got, want)
+    assert bad == 0, (bad, worst, launch)
+    again = _run_linear(rows, Kk, N, bits, cb, fp32, 60 + rows, prefill=True)[0]
+    assert np.array_equal(got.view(np.uint8), again.view(np.uint8)), launch
+
+
+@pytest.mark.parametrize("rows,unit", [(40, 128), (150, 128), (70, 0)])
+def test_bundle_with_narrower_slices(rows, unit):
+    """Sliced lists whose widths differ: blocks past a slice's end are empty and touch nothing.  unit 0: four slices of one
+    column block each."""
+    Kk, width, widths, bits = 640, 640, (640, 256, 128, 640), 4
+    if not unit:
+        width, widths = 128, (128, 128, 128, 128)
+    lins = [synth.linear(640 + i, Kk, n, bits) for i, n in enumerate(widths)]
+    d = [[dev(t.view(np.uint16)) for t in lin] for lin in lins]
+    x = synth.activations(650 + rows, rows, Kk)
+    outs = [torch.full((rows, n), 5.0, dtype=torch.float16, device=DEV) for n in widths]
+    i64 = lambda v: torch.tensor(v, dtype=torch.int64, device=DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    lists = [i64([dd[j].data_ptr() for dd in d]) for j in range(3)]
+    c_ptrs, n_list, src = i64([o.data_ptr() for o in outs]), i32(list(widths)), i32([0, 1, 2, 3])
+    a_had = torch.zeros((4, rows, Kk), dtype=torch.float16, device=DEV)
+    d_x = dev(x.view(np.uint16))
+    K.ops.exl3_mgemm(d_x.data_ptr(), lists[0].data_ptr(), outs[0].data_ptr(), lists[1].data_ptr(), a_had.data_ptr(),
+                     lists[2].data_ptr(), rows, Kk, width, bits, Codebook.MUL1, OutDtype.F16, 1, 4, n_list.data_ptr(),
+                     c_ptrs.data_ptr(), n_list.data_ptr(), src.data_ptr(), 4)
+    torch.cuda.synchronize()
+    assert "exl3_gemm_kernel/block" in K.ops.last_launch(), K.ops.last_launch()
+    for i, (tr, suh, svh) in enumerate(lins):
+        want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=False)
+        assert close(host_f16(outs[i]), want)[0] == 0, i
+        assert np.array_equal(host_u16(a_had).reshape(4, -1)[i], want_had.view(np.uint16).reshape(-1)), i

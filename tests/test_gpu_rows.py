@@ -46,11 +46,14 @@ def test_few_rows_match_the_oracle_and_repeat(rows, Kk, N, bits, cb):
     assert np.array_equal(got.view(np.uint8), again.view(np.uint8)), launch
 
 
-@pytest.mark.parametrize("rows", [3, 20])
-def test_bundle_with_narrower_slices(rows):
+@pytest.mark.parametrize("rows,unit", [(3, 128), (20, 128), (5, 0)])
+def test_bundle_with_narrower_slices(rows, unit):
     """Sliced lists whose widths differ (the last one a single column block): blocks past a
-    slice's end are empty and touch nothing."""
+    slice's end are empty and touch nothing.  unit 0: four slices of one
+    column block each."""
     Kk, width, widths, bits = 1024, 1664, (1664, 640, 128, 1664), 4
+    if not unit:
+        width, widths = 128, (128, 128, 128, 128)
     lins = [synth.linear(600 + i, Kk, n, bits) for i, n in enumerate(widths)]
     d = [[dev(t.view(np.uint16)) for t in lin] for lin in lins]
     x = synth.activations(610 + rows, rows, Kk)
