@@ -926,7 +926,8 @@ void check_route_shape(int T, int H, int E, int k)
 
 std::string run_route(const void* x, const void* wr, const float* bias, int32_t* idx, float* w,
                       float* logits, float* parts, int T, int H, int E, int k, int renorm,
-                      hipStream_t stream, const PermuteParams* sort = nullptr)
+                      hipStream_t stream, const PermuteParams* sort = nullptr, int32_t* idx_out = nullptr,
+                      float* w_out = nullptr)
 {
     LaunchScope scope(stream);
     Workspace& ws = scope.ws;
@@ -939,6 +940,8 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
     p.idx = idx;
     p.w = w;
     p.logits = logits;
+    p.idx_out = idx_out;
+    p.w_out = w_out;
     p.T = T; p.H = H; p.E = E; p.k = k; p.renorm = renorm;
     p.nseg = (H + kRouteSeg - 1) / kRouteSeg;
     if (sort && T == 1) p.sort = *sort;
@@ -1274,6 +1277,8 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         r.parts = (float*)(wsb + L.parts);
         r.idx = idx;
         r.w = w;
+        r.idx_out = idx_out;
+        r.w_out = w_out;
         r.T = 1; r.H = H; r.E = E; r.k = k; r.renorm = renorm;
         r.nseg = L.nseg;
         r.sort = pp;
@@ -1281,7 +1286,7 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         hip_ok(hipGetLastError(), "moe_route_segments_kernel launch");
         desc += "moe_route_segments_kernel grid=" + std::to_string(L.nseg) + " (top-k and sort inside the next launch)";
     } else {
-        desc += run_route(x, wr, bias, idx, w, nullptr, (float*)(wsb + L.parts), T, H, E, k, renorm, stream, &pp);
+        desc += run_route(x, wr, bias, idx, w, nullptr, (float*)(wsb + L.parts), T, H, E, k, renorm, stream, &pp, idx_out, w_out);
         if (T > 1) desc += " + " + run_permute(pp, stream);
     }
 
@@ -1461,8 +1466,6 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
                        (const int32_t*)(wsb + L.inv), (float*)out, T, H, k, stream);
         desc += " + moe_combine_kernel";
     }
-    if (idx_out) hip_ok(hipMemcpyAsync(idx_out, idx, (size_t)P * 4, hipMemcpyDeviceToDevice, stream), "idx copy");
-    if (w_out) hip_ok(hipMemcpyAsync(w_out, w, (size_t)P * 4, hipMemcpyDeviceToDevice, stream), "w copy");
     g_moe_launch = desc;
     MOE_TRY_END
 }

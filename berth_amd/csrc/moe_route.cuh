@@ -55,6 +55,8 @@ struct RouteParams {
     int32_t* idx;           // [T][k]
     float* w;               // [T][k]
     float* logits;          // [T][E] or null
+    int32_t* idx_out;       // [T][k], [T][k] or null: the caller's own copies of idx and w, written with them (two
+    float* w_out;           // copy launches behind the layer cost 4 us of a one-token layer's 30, 8 under a profiler)
     int T, H, E, k, nseg, renorm;
     // one token only: the wave that selected the experts also sorts them and writes
     // what the permute kernel would (sort.perm != nullptr), saving its launch
@@ -127,8 +129,12 @@ __device__ __forceinline__ int route_topk_n(const float (&lg)[kRoutePer], int la
         denom = loc;
     }
     if (store && lane < p.k) {
-        p.idx[(size_t)t * p.k + lane] = sel_idx;
-        p.w[(size_t)t * p.k + lane] = ev / denom;
+        const size_t at = (size_t)t * p.k + lane;
+        const float weight = ev / denom;
+        p.idx[at] = sel_idx;
+        p.w[at] = weight;
+        if (p.idx_out) p.idx_out[at] = sel_idx;
+        if (p.w_out) p.w_out[at] = weight;
     }
     return sel_idx;     // lane j < k: expert of slot j
 }
