@@ -18,7 +18,7 @@ __global__ __launch_bounds__(256) void had_r_128_kernel(const T* __restrict__ in
     // accesses): a wave takes four neighbouring blocks at a time and strides over the tensor
     typedef T vec8_t __attribute__((ext_vector_type(8)));
     const int lane = threadIdx.x & 63;
-    const int l16 = lane & 15;
+    const int chunk = had_chunk(lane);
     const long waves = (long)gridDim.x * 4;
     const long groups = (blocks + 3) / 4;
     for (long g = (long)blockIdx.x * 4 + (threadIdx.x >> 6); g < groups; g += waves) {
@@ -26,11 +26,11 @@ __global__ __launch_bounds__(256) void had_r_128_kernel(const T* __restrict__ in
         const bool live = blk < blocks;
         const long b = live ? blk : blocks - 1;             // lanes past the end redo the last block and store nothing
         const int cb = (int)(b % col_blocks);
-        const size_t at = (size_t)b * 128 + 8 * l16;
+        const size_t at = (size_t)b * 128 + 8 * chunk;
         const vec8_t x = *(const vec8_t*)(in + at);
         float v[8], sc[8];
         if (scale) {
-            const half8_t s8 = *(const half8_t*)(scale + cb * 128 + 8 * l16);
+            const half8_t s8 = *(const half8_t*)(scale + cb * 128 + 8 * chunk);
 #pragma unroll
             for (int i = 0; i < 8; ++i) sc[i] = (float)s8[i];
         } else {
@@ -42,12 +42,12 @@ __global__ __launch_bounds__(256) void had_r_128_kernel(const T* __restrict__ in
             v[i] = (float)x[i];
             if (PRE) v[i] *= sc[i];
         }
-        had128_row16(v, lane);
+        const float unit = had128_row16(v, lane) * kRsqrt128;
         vec8_t o;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            float r = v[i] * kRsqrt128;
-            if (!PRE) r *= sc[i];
+            float r = had_scale(v[i], unit);
+            if (!PRE) r = rounded(r * sc[i]);
             o[i] = (T)r;
         }
         if (live) *(vec8_t*)(out + at) = o;
@@ -92,7 +92,7 @@ __device__ __forceinline__ void rotate_rows(const RotateParams& p)
     const _Float16* in = p.in + (size_t)slab * p.in_stride;
     _Float16* out = (!p.suh_list && p.tab.out[slab]) ? p.tab.out[slab] : p.out + (size_t)slab * p.out_stride;
     const int lane = threadIdx.x & 63;
-    const int l16 = lane & 15;
+    const int chunk = had_chunk(lane);
     const long waves = (long)gridDim.x * 4;
     const long groups = (p.blocks + 3) / 4;
     for (long g = (long)blockIdx.x * 4 + (threadIdx.x >> 6); g < groups; g += waves) {
@@ -100,25 +100,24 @@ __device__ __forceinline__ void rotate_rows(const RotateParams& p)
         const bool live = blk < p.blocks;
         const unsigned b = (unsigned)(live ? blk : p.blocks - 1);   // lanes past the end redo the last block and store nothing
         const unsigned row = b / (unsigned)p.col_blocks, cb = b - row * (unsigned)p.col_blocks;
-        const size_t at = (size_t)b * 128 + 8 * l16;
+        const size_t at = (size_t)b * 128 + 8 * chunk;
         half8_t x = *(const half8_t*)(in + at);
-        const half8_t s8 = *(const half8_t*)(scale + cb * 128 + 8 * l16);
+        const half8_t s8 = *(const half8_t*)(scale + cb * 128 + 8 * chunk);
         if (SILU) {
             const half8_t u = *(const half8_t*)(p.up + at);
 #pragma unroll
             for (int i = 0; i < 8; ++i) x[i] = silu_mul_h(x[i], u[i]);
         }
         float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = (float)x[i] * (float)s8[i];
-        had128_row16(v, lane);
+        mul_half8(x, s8, v);
+        const float unit = had128_row16(v, lane) * kRsqrt128;
         half8_t o;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = (_Float16)(v[i] * kRsqrt128);
+        for (int i = 0; i < 8; ++i) o[i] = (_Float16)had_scale(v[i], unit);
         if (live) {
             if (SILU && p.act_out) *(half8_t*)(p.act_out + at) = x;
             *(half8_t*)(out + at) = o;
-            if (p.operand) store_operand(p, slab, (int)row, (int)cb * 128 + 8 * l16, o);
+            if (p.operand) store_operand(p, slab, (int)row, (int)cb * 128 + 8 * chunk, o);
         }
     }
 }
@@ -143,14 +142,15 @@ template <int CHUNKS>
 __global__ __launch_bounds__(1024) void add_rms_norm_had_r_128_kernel(NormParams n, RotateParams p)
 {
     __shared__ double s_part[16];
-    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, l16 = lane & 15;
+    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int mine = (tid & ~15) | had_chunk(lane);        // which eight values of a chunk this thread holds
     const int threads = blockDim.x;
     const size_t base = (size_t)row * n.dim;
     float v[CHUNKS][8];
     double ss = 0.0;
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
-        const int e = 8 * (tid + c * threads);
+        const int e = 8 * (mine + c * threads);
         if (e < n.dim) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -168,6 +168,7 @@ __global__ __launch_bounds__(1024) void add_rms_norm_had_r_128_kernel(NormParams
             for (int j = 0; j < 8; ++j) v[c][j] = 0.0f;
         }
     }
+    ss = __shfl(ss, (lane & ~15) | had_chunk(lane), 64);    // summed in the order of the row
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) ss += __shfl_xor(ss, d, 64);
     if (lane == 0) s_part[tid >> 6] = ss;
@@ -177,10 +178,10 @@ __global__ __launch_bounds__(1024) void add_rms_norm_had_r_128_kernel(NormParams
     const float rmf = (float)(1.0 / sqrt(total / n.dim + (double)n.epsilon));
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
-        const int e = 8 * (tid + c * threads);
-        if (e - 8 * l16 >= n.dim) continue;             // the sixteen lanes of a 128 block stay together
+        const int e = 8 * (mine + c * threads);
+        if (e - 8 * had_chunk(lane) >= n.dim) continue;             // the sixteen lanes of a 128 block stay together
         const half8_t wb = *(const half8_t*)(n.weight + e);
-        _Float16 y[8];
+        half8_t y;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const uint16_t bits = __builtin_bit_cast(uint16_t, (_Float16)wb[j]);
@@ -193,12 +194,11 @@ __global__ __launch_bounds__(1024) void add_rms_norm_had_r_128_kernel(NormParams
         for (int s = 0; s < n.slabs; ++s) {
             const half8_t s8 = *(const half8_t*)(p.tab.suh[s] + e);
             float r[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) r[j] = (float)y[j] * (float)s8[j];
-            had128_row16(r, lane);
+            mul_half8(y, s8, r);
+            const float unit = had128_row16(r, lane) * kRsqrt128;
             half8_t o;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] = (_Float16)(r[j] * kRsqrt128);
+            for (int j = 0; j < 8; ++j) o[j] = (_Float16)had_scale(r[j], unit);
             _Float16* out = p.tab.out[s] ? p.tab.out[s] : p.out + (size_t)s * p.out_stride;
             *(half8_t*)(out + base + e) = o;
             if (p.operand) store_operand(p, s, row, e, o);

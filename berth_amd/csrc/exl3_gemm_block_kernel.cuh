@@ -57,11 +57,11 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, u
 __device__ __forceinline__ void block_finish_row(const GemmParams& p, const RowsBlock& b, float (&v)[8], const half8_t sv,
                                                  const int row, const bool live, const int lane)
 {
-    had128_row16(v, lane);
+    const float unit = had128_row16(v, lane) * kRsqrt128;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (v[e] * kRsqrt128) * (float)sv[e];
+    for (int e = 0; e < 8; ++e) v[e] = had_scale(v[e], unit) * (float)sv[e];
     if (!live) return;
-    const size_t at = (size_t)row * b.ldc + b.n0 + 8 * (lane & 15);
+    const size_t at = (size_t)row * b.ldc + b.n0 + 8 * had_chunk(lane);
     if (p.out_fp32) {
         if (p.out_add) {
             const global_ptr<const float4_t> add = (global_ptr<const float4_t>)(as_global(p.out_add) + at);
@@ -273,19 +273,20 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
         __syncthreads();
         if (!b.empty) {
             // sixteen lanes a row, eight columns each: a wave takes four rows at a time
+            const int chunk = had_chunk(lane);
             const bool whole = s0 == 0 && s1 == SPT;
             float* const part = p.partials + ((size_t)w * 2 + (tile == t_first ? 0 : 1)) * BM * 128;
 #pragma unroll
             for (int pass = 0; pass < MT / 4 + (MT % 4 != 0); ++pass) {
                 const int r = pass * 64 + wave * 4 + lg;
                 if (pass * 64 + wave * 4 >= rows) break;
-                const float4_t* const zr = (const float4_t*)&z[min(r, 16 * MT - 1) * kRowsStride + 8 * l16];
+                const float4_t* const zr = (const float4_t*)&z[min(r, 16 * MT - 1) * kRowsStride + 8 * chunk];
                 const float4_t v0 = zr[0], v1 = zr[1];
                 if (whole) {
                     float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-                    block_finish_row(p, b, v, ((const half8_t*)sv_lds)[l16], m0 + r, r < rows, lane);
+                    block_finish_row(p, b, v, ((const half8_t*)sv_lds)[chunk], m0 + r, r < rows, lane);
                 } else if (r < rows) {
-                    const global_ptr<float4_t> dst = (global_ptr<float4_t>)as_global(part + r * 128 + 8 * l16);
+                    const global_ptr<float4_t> dst = (global_ptr<float4_t>)as_global(part + r * 128 + 8 * chunk);
                     dst[0] = v0;
                     dst[1] = v1;
                 }
@@ -313,7 +314,7 @@ static __global__ __launch_bounds__(256) void exl3_gemm_finish_kernel(GemmParams
     const unsigned cb = div_exact(tile, p.m_rt);
     const RowsBlock b = rows_block(p, cb);
     if (b.empty) return;
-    const int lane = threadIdx.x & 63, l16 = lane & 15;
+    const int lane = threadIdx.x & 63, chunk = had_chunk(lane);
     const int BM = p.rows_per_tile, m0 = (int)(tile - cb * RT) * BM;
     const int row = (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4);
     const int rows = min(BM, p.M - m0);
@@ -321,7 +322,7 @@ static __global__ __launch_bounds__(256) void exl3_gemm_finish_kernel(GemmParams
     const int r = min(row, rows - 1);
     // the tile is the first of every sharer's range but, unless that starts with it, the first sharer's
     const unsigned slot_a = S || wa * q + min(wa, rem) >= tile * SPT ? 0u : 1u;
-    const half8_t sv = ((global_ptr<const half8_t>)as_global(b.svh + b.n0))[l16];
+    const half8_t sv = ((global_ptr<const half8_t>)as_global(b.svh + b.n0))[chunk];
     float v[8] = {};
     for (unsigned x = wa; x <= wb; x += 4) {
         float4_t part[4][2];
@@ -329,7 +330,7 @@ static __global__ __launch_bounds__(256) void exl3_gemm_finish_kernel(GemmParams
         for (unsigned i = 0; i < 4; ++i) {
             const unsigned xi = min(x + i, wb);
             const global_ptr<const float4_t> src = (global_ptr<const float4_t>)as_global(
-                p.partials + ((size_t)xi * 2 + (xi == wa ? slot_a : 0u)) * BM * 128 + r * 128 + 8 * l16);
+                p.partials + ((size_t)xi * 2 + (xi == wa ? slot_a : 0u)) * BM * 128 + r * 128 + 8 * chunk);
             part[i][0] = src[0];
             part[i][1] = src[1];
         }

@@ -281,12 +281,12 @@ __device__ __forceinline__ void gemm_tile_wide(const GemmParams& p, const int ti
     // ---- epilogue, 32 rows at a time per row half: stage the fp32 tile, output Hadamard, svh,
     // store.  Both halves take the barriers as often as the first half needs them.
     float* z_tile = (float*)(smem + (size_t)rh * 32 * kZStride * sizeof(float));
-    const int l16 = lane & 15;
+    const int chunk = had_chunk(lane);
     half8_t sv_blk[2];
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
         const int gn = n0 + blk * 128;
-        sv_blk[blk] = gn < N ? ((global_ptr<const half8_t>)as_global(lin.svh + gn))[l16] : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        sv_blk[blk] = gn < N ? ((global_ptr<const half8_t>)as_global(lin.svh + gn))[chunk] : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
     }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
@@ -310,15 +310,15 @@ __device__ __forceinline__ void gemm_tile_wide(const GemmParams& p, const int ti
             const int gn = n0 + blk * 128;
             if (row < rows_blk && gn < N) {
                 float v[8];
-                const float4_t* zp = (const float4_t*)&z_tile[row * kZStride + blk * 128 + 8 * l16];
+                const float4_t* zp = (const float4_t*)&z_tile[row * kZStride + blk * 128 + 8 * chunk];
                 const float4_t z0 = zp[0], z1 = zp[1];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) { v[i] = z0[i]; v[4 + i] = z1[i]; }
-                had128_row16(v, lane);
+                const float unit = had128_row16(v, lane) * kRsqrt128;
                 const half8_t sv = blk ? sv_blk[1] : sv_blk[0];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = (v[i] * kRsqrt128) * (float)sv[i];
-                const size_t at = (size_t)(m0 + mb * 32 + row) * ldc + gn + 8 * l16;
+                for (int i = 0; i < 8; ++i) v[i] = had_scale(v[i], unit) * (float)sv[i];
+                const size_t at = (size_t)(m0 + mb * 32 + row) * ldc + gn + 8 * chunk;
                 if (p.out_fp32) {
                     if (p.out_add) {
                         const global_ptr<const float4_t> add = (global_ptr<const float4_t>)(as_global(p.out_add) + at);

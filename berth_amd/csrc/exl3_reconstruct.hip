@@ -97,16 +97,16 @@ __global__ __launch_bounds__(256) void exl3_reconstruct_had_kernel(
 
     // down the columns: wave w takes columns 32w .. 32w + 31, four at a time (one per
     // 16-lane row of the wave), a lane holds eight consecutive k of its column
-    const int sub = lane >> 4, l16 = lane & 15;
+    const int sub = lane >> 4, chunk = had_chunk(lane);
 #pragma unroll 1
     for (int pass = 0; pass < 8; ++pass) {
         const int n = wave * 32 + pass * 4 + sub;
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = blk[8 * l16 + i][n];
-        had128_row16(v, lane);
+        for (int i = 0; i < 8; ++i) v[i] = blk[8 * chunk + i][n];
+        const float sign = had128_row16(v, lane);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) blk[8 * l16 + i][n] = v[i];
+        for (int i = 0; i < 8; ++i) blk[8 * chunk + i][n] = had_scale(v[i], sign);
     }
     __syncthreads();
 
@@ -114,20 +114,20 @@ __global__ __launch_bounds__(256) void exl3_reconstruct_had_kernel(
     const global_ptr<const _Float16> g_suh = as_global(suh), g_svh = as_global(svh);
     float sv[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sv[i] = (float)g_svh[nb * 128 + 8 * l16 + i];
+    for (int i = 0; i < 8; ++i) sv[i] = (float)g_svh[nb * 128 + 8 * chunk + i];
 #pragma unroll 1
     for (int pass = 0; pass < 8; ++pass) {
         const int r = wave * 32 + pass * 4 + sub;
         float v[8];
-        const float4_t lo = *(const float4_t*)&blk[r][8 * l16], hi = *(const float4_t*)&blk[r][8 * l16 + 4];
+        const float4_t lo = *(const float4_t*)&blk[r][8 * chunk], hi = *(const float4_t*)&blk[r][8 * chunk + 4];
         v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
         v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-        had128_row16(v, lane);
+        const float unit = had128_row16(v, lane) * kRsqrt128;
         const float su = (float)g_suh[kb * 128 + r];
         half8_t o;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = (_Float16)((((v[i] * kRsqrt128) * kRsqrt128) * su) * sv[i]);
-        *(half8_t*)(out + (size_t)(kb * 128 + r) * slice_n + nb * 128 + 8 * l16) = o;
+        for (int i = 0; i < 8; ++i) o[i] = (_Float16)rounded(((had_scale(v[i], unit) * kRsqrt128) * su) * sv[i]);
+        *(half8_t*)(out + (size_t)(kb * 128 + r) * slice_n + nb * 128 + 8 * chunk) = o;
     }
 }
 

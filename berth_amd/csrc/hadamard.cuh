@@ -102,11 +102,25 @@ __device__ __forceinline__ void had128_wave(float& v0, float& v1, int lane)
     v0 = had_stage_swap32(v0, s32);  v1 = had_stage_swap32(v1, s32);
 }
 
-// 128-point Hadamard with eight consecutive elements per lane and sixteen lanes
-// (one DPP row) per vector, so a wave rotates four vectors at once: stages 1, 2, 4
-// stay inside the lane, stages 8 .. 64 are DPP exchanges inside the row.  Same
-// butterfly order and the same exact sums as had128_wave.
-__device__ __forceinline__ void had128_row16(float (&v)[8], int lane)
+// 128-point Hadamard with eight consecutive elements per lane and sixteen lanes (one DPP row) per
+// vector, so a wave rotates four vectors at once: stages 1, 2, 4 stay inside the lane, stages
+// 8 .. 64 are exchanges inside the row, one v_fmac_f32 with a DPP operand per element and stage.
+//
+//   * Lane l of a row holds the elements 8 * had_chunk(l) .. + 7.  One DPP control reaches the lane
+//     at distance 1, 2 or 8, none the one at distance 4; the mirror of half a row reaches l ^ 7.
+//     With the lanes of the upper half of eight in reversed order inside their four, l ^ 7 is the
+//     lane whose elements are 32 away.
+//   * own + sgn * partner is the butterfly's result in the lower lane and its negative in the upper
+//     one.  Later stages meet both lanes of a pair with the same sign, so it is left on: the
+//     values come back times the returned +1 or -1, which had_scale takes off.
+//
+// Same butterfly order and the same sums as had128_wave (a zero leaves had_scale as +0).  What bounds the
+// launches around it is the vector pipe: with a move, an fma and, for distance 4, another move per
+// stage, and two conversions before every product, an element took 17 vector instructions instead of
+// 10.5.
+__device__ __forceinline__ int had_chunk(int lane) { return (lane & 15) ^ ((lane & 4) ? 3 : 0); }
+
+__device__ __forceinline__ float had128_row16(float (&v)[8], int lane)
 {
 #pragma unroll
     for (int h = 1; h < 8; h <<= 1) {
@@ -119,18 +133,56 @@ __device__ __forceinline__ void had128_row16(float (&v)[8], int lane)
             }
         }
     }
-    const float s1 = (lane & 1) ? -1.0f : 1.0f;
-    const float s2 = (lane & 2) ? -1.0f : 1.0f;
-    const float s4 = (lane & 4) ? -1.0f : 1.0f;
-    const float s8 = (lane & 8) ? -1.0f : 1.0f;
+    const int c = had_chunk(lane);
+    const float s1 = (c & 1) ? -1.0f : 1.0f;
+    const float s2 = (c & 2) ? -1.0f : 1.0f;
+    const float s4 = (c & 4) ? -1.0f : 1.0f;
+    const float s8 = (c & 8) ? -1.0f : 1.0f;
+    // a DPP operand may be read two instructions after it was written at the earliest: the s_nop
+    // covers the compiler's last write, inside a register is read again eight instructions later
+#define BERTH_HAD_STAGE(sgn, ctrl)                                                            \
+    "v_fmac_f32_dpp %0, %0, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"                  \
+    "v_fmac_f32_dpp %1, %1, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"                  \
+    "v_fmac_f32_dpp %2, %2, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"                  \
+    "v_fmac_f32_dpp %3, %3, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"                  \
+    "v_fmac_f32_dpp %4, %4, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"                  \
+    "v_fmac_f32_dpp %5, %5, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"                  \
+    "v_fmac_f32_dpp %6, %6, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"                  \
+    "v_fmac_f32_dpp %7, %7, " sgn " " ctrl " row_mask:0xf bank_mask:0xf\n\t"
+    asm volatile("s_nop 1\n\t"
+                 BERTH_HAD_STAGE("%8", "quad_perm:[1,0,3,2]") BERTH_HAD_STAGE("%9", "quad_perm:[2,3,0,1]")
+                 BERTH_HAD_STAGE("%10", "row_half_mirror") BERTH_HAD_STAGE("%11", "row_ror:8")
+                 "s_nop 1"
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+                 : "v"(s1), "v"(s2), "v"(s4), "v"(s8));
+#undef BERTH_HAD_STAGE
+    return (s1 * s2) * (s4 * s8);
+}
+
+// a value that has been rounded to fp32: keeps a multiplication and the conversion of its result to
+// fp16 two roundings, as the oracle has them (the compiler may make them one v_fma_mixlo_f16)
+__device__ __forceinline__ float rounded(float v)
+{
+    asm("" : "+v"(v));
+    return v;
+}
+
+// v times `unit` (the sign that had128_row16 returned, / sqrt(128) where that is wanted) with one
+// rounding; the sum with +0 keeps the sign from turning a zero into -0
+__device__ __forceinline__ float had_scale(float v, float unit) { return rounded(__builtin_fmaf(v, unit, 0.0f)); }
+
+// a[i] * b[i] of eight fp16 pairs in fp32 (exact; a zero is +0), one instruction each
+typedef _Float16 had_half8_t __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ void mul_half8(const had_half8_t a, const had_half8_t b, float (&v)[8])
+{
+    typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+    const u4_t x = __builtin_bit_cast(u4_t, a), y = __builtin_bit_cast(u4_t, b);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = had_stage_dpp<1>(v[i], s1);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = had_stage_dpp<2>(v[i], s2);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = had_stage_dpp<4>(v[i], s4);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = had_stage_dpp<8>(v[i], s8);
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t xi = x[i], yi = y[i];
+        asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(v[2 * i]) : "v"(xi), "v"(yi));
+        asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(v[2 * i + 1]) : "v"(xi), "v"(yi));
+    }
 }
 
 }  // namespace berth

@@ -661,7 +661,6 @@ struct HadRowsParams {
 __global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
 {
     const int lane = threadIdx.x & 63;
-    const int l16 = lane & 15;
     const int which = blockIdx.y;
     const int nkb = p.K >> 7;
     const int total = p.P * nkb;
@@ -669,7 +668,7 @@ __global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
     const bool live = first < total;
     const int item = live ? first : total - 1;              // groups past the end redo the last item, store nothing
     const int row = item / nkb;
-    const int at = (item - row * nkb) * 128 + 8 * l16;
+    const int at = (item - row * nkb) * 128 + 8 * had_chunk(lane);
     const int ex = p.row_expert[row];
     const int src = p.gather ? p.gather[row] / p.gather_div : row;
     const _Float16* scale = ex == p.shared_expert ? p.shared[p.lin_base + which].suh
@@ -682,12 +681,11 @@ __global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
         for (int i = 0; i < 8; ++i) x[i] = silu_mul_h(x[i], u[i]);
     }
     float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = (float)x[i] * (float)sc[i];
-    had128_row16(v, lane);
+    mul_half8(x, sc, v);
+    const float unit = had128_row16(v, lane) * kRsqrt128;
     half8_t o;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = (_Float16)(v[i] * kRsqrt128);
+    for (int i = 0; i < 8; ++i) o[i] = (_Float16)had_scale(v[i], unit);
     if (live) *(half8_t*)(p.out[which] + (size_t)row * p.K + at) = o;
 }
 
