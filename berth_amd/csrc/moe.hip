@@ -652,16 +652,16 @@ struct HadRowsParams {
     int P, K;
 };
 
-// An item is one 128 block of one row under one linear's scales; sixteen lanes (one DPP row)
-// rotate it, eight consecutive elements per lane (16-byte accesses).  blockIdx.x walks the
-// (row, block) items, sixteen per workgroup, so that a narrow K does not leave waves idle;
-// blockIdx.y is the linear.  Measured on 2816 rows (K 2048 under two linears / K 512 under one):
-// 14.4 / 5.0 us; with both linears in one thread 14.4 / 5.9 us, with two or four items per lane
-// group on top of that 13.7 / 6.4 and 15.9 / 7.9 us.  The K 2048 pair writes 23 MB.
+// An item is one 128 block of one row, under the scales of the launch's one or two linears; sixteen
+// lanes (one DPP row) rotate it, eight consecutive elements per lane (16-byte accesses).  blockIdx.x
+// walks the (row, block) items, sixteen per workgroup, so that a narrow K does not leave waves idle.
+// What bounds the launch is the writes: 12000 rows of K 2048 under two linears 33.5 us for 98 MB (40.9
+// with a thread per linear, which walks the chain row -> expert -> pointer -> scales twice; two rows
+// per lane group 33.0), 2816 rows 9.5 us (13).
+template <int LINS>
 __global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
 {
     const int lane = threadIdx.x & 63;
-    const int which = blockIdx.y;
     const int nkb = p.K >> 7;
     const int total = p.P * nkb;
     const int first = blockIdx.x * 16 + (threadIdx.x >> 4);
@@ -671,28 +671,37 @@ __global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
     const int at = (item - row * nkb) * 128 + 8 * had_chunk(lane);
     const int ex = p.row_expert[row];
     const int src = p.gather ? p.gather[row] / p.gather_div : row;
-    const _Float16* scale = ex == p.shared_expert ? p.shared[p.lin_base + which].suh
-                                                  : p.experts[(size_t)ex * p.lins_per_expert + p.lin_base + which].suh;
+    half8_t sc[LINS];
+#pragma unroll
+    for (int l = 0; l < LINS; ++l) {
+        const _Float16* scale = ex == p.shared_expert ? p.shared[p.lin_base + l].suh
+                                                      : p.experts[(size_t)ex * p.lins_per_expert + p.lin_base + l].suh;
+        sc[l] = *(const half8_t*)(scale + at);
+    }
     half8_t x = *(const half8_t*)(p.a + (size_t)src * p.K + at);
-    const half8_t sc = *(const half8_t*)(scale + at);
     if (p.a_up) {
         const half8_t u = *(const half8_t*)(p.a_up + (size_t)src * p.K + at);
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = silu_mul_h(x[i], u[i]);
     }
-    float v[8];
-    mul_half8(x, sc, v);
-    const float unit = had128_row16(v, lane) * kRsqrt128;
-    half8_t o;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = (_Float16)had_scale(v[i], unit);
-    if (live) *(half8_t*)(p.out[which] + (size_t)row * p.K + at) = o;
+    for (int l = 0; l < LINS; ++l) {
+        float v[8];
+        mul_half8(x, sc[l], v);
+        const float unit = had128_row16(v, lane) * kRsqrt128;
+        half8_t o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = (_Float16)had_scale(v[i], unit);
+        if (live) *(half8_t*)(p.out[l] + (size_t)row * p.K + at) = o;
+    }
 }
 
 inline void launch_had_rows(const HadRowsParams& h, hipStream_t stream)
 {
     const long items = (long)h.P * (h.K >> 7);
-    hipLaunchKernelGGL(moe_had_rows_kernel, dim3((unsigned)((items + 15) / 16), h.num_lins), dim3(256), 0, stream, h);
+    const dim3 grid((unsigned)((items + 15) / 16));
+    if (h.num_lins == 2) hipLaunchKernelGGL(moe_had_rows_kernel<2>, grid, dim3(256), 0, stream, h);
+    else hipLaunchKernelGGL(moe_had_rows_kernel<1>, grid, dim3(256), 0, stream, h);
     hip_ok(hipGetLastError(), "moe_had_rows_kernel launch");
 }
 
