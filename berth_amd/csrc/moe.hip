@@ -954,26 +954,35 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
     if (sort && T == 1) p.sort = *sort;
     const int groups = (T + kRouteTT - 1) / kRouteTT;
     if (T >= kRouteBigT && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && knobs().moe_route_slab) {
-        // one launch: tokens per workgroup as many as the segment sums leave room for in 64 KiB
-        // of LDS, fewer while that leaves compute units without a workgroup
+        // One launch.  Tokens per workgroup: one workgroup of sixteen waves runs per compute unit, and its
+        // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 12.8, 19.5 and
+        // 25 us), so the count with the fewest whole rounds of the chip wins.  1500 tokens x 128 experts:
+        // six tokens in one round of 250 workgroups 39 -> 26 us against four in 375.
         const int nslab = (E + kSlabExperts - 1) / kSlabExperts;
-        int tt = 4;
         constexpr int kSlabLdsMax = 144 * 1024;
-        while (tt > 1 && (route_slab_lds_bytes(p.nseg, tt) > kSlabLdsMax || (long)nslab * ((T + tt - 1) / tt) < ws.cu_count / 2)) tt /= 2;
+        int tt = 1;
+        long best = -1;
+        for (const int c : {1, 2, 3, 4, 6}) {
+            const long groups_c = (T + c - 1) / c;
+            if (route_slab_lds_bytes(p.nseg, c) > kSlabLdsMax || groups_c * kRouteCounterStride > kCounters) continue;
+            const long cost = ((long)nslab * groups_c + ws.cu_count - 1) / ws.cu_count * (4 + c);
+            if (best < 0 || cost < best) { best = cost; tt = c; }
+        }
         const int tgroups = (T + tt - 1) / tt;
         if (route_slab_lds_bytes(p.nseg, tt) <= kSlabLdsMax && (long)tgroups * kRouteCounterStride <= kCounters) {
             dim3 grid(tgroups, nslab);
             const size_t lds = (size_t)route_slab_lds_bytes(p.nseg, tt);
-            static bool raised[3][64] = {};
-            if (tt == 4) {
-                raise_dynamic_lds_limit((const void*)moe_route_slab_kernel<4>, kSlabLdsMax, raised[0], "moe_route_slab_kernel shared-memory attribute");
-                hipLaunchKernelGGL(moe_route_slab_kernel<4>, grid, dim3(1024), lds, stream, p);
-            } else if (tt == 2) {
-                raise_dynamic_lds_limit((const void*)moe_route_slab_kernel<2>, kSlabLdsMax, raised[1], "moe_route_slab_kernel shared-memory attribute");
-                hipLaunchKernelGGL(moe_route_slab_kernel<2>, grid, dim3(1024), lds, stream, p);
-            } else {
-                raise_dynamic_lds_limit((const void*)moe_route_slab_kernel<1>, kSlabLdsMax, raised[2], "moe_route_slab_kernel shared-memory attribute");
-                hipLaunchKernelGGL(moe_route_slab_kernel<1>, grid, dim3(1024), lds, stream, p);
+            auto launch = [&](auto kernel, bool (&raised)[64]) {
+                raise_dynamic_lds_limit((const void*)kernel, kSlabLdsMax, raised, "moe_route_slab_kernel shared-memory attribute");
+                hipLaunchKernelGGL(kernel, grid, dim3(1024), lds, stream, p);
+            };
+            static bool raised[7][64] = {};
+            switch (tt) {
+            case 1: launch(moe_route_slab_kernel<1>, raised[1]); break;
+            case 2: launch(moe_route_slab_kernel<2>, raised[2]); break;
+            case 3: launch(moe_route_slab_kernel<3>, raised[3]); break;
+            case 4: launch(moe_route_slab_kernel<4>, raised[4]); break;
+            default: launch(moe_route_slab_kernel<6>, raised[6]); break;
             }
             hip_ok(hipGetLastError(), "moe_route_slab_kernel launch");
             return "moe_route_slab_kernel<" + std::to_string(tt) + "> grid=" + std::to_string(nslab) + "x" +
