@@ -527,27 +527,63 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
 // ---------------------------------------------------------------- permute
 
 
-// One workgroup.  Counting sort by expert, stable in pair order: the pairs of one
-// expert come from distinct tokens, so the rank of pair (t, slot) inside its expert
-// is the number of earlier tokens that chose the expert.  Tokens are taken 64 at a
-// time: a 64-bit mask per expert records which of them chose it, and the rank is a
-// population count below the token's bit.  Nothing depends on scheduling.
-__global__ __launch_bounds__(1024) void moe_permute_kernel(PermuteParams p)
+// Counting sort by expert, stable in pair order.  Every wave takes a contiguous run of the pairs: it
+// counts them per expert (hist[wave][expert]), the counts are summed over the waves and the experts,
+// and then each wave places its own run, 64 pairs at a time, without meeting the others again: the
+// lanes with the same expert find each other by one ballot per bit of the expert's number, a lane's
+// rank among them is a population count, and the wave's next free row of the expert stands in hist.
+// With many pairs several workgroups count all of them, each for itself, and workgroup g places the
+// runs g, g + G, ...: a placed pair is two 4-byte stores at lines of their own, 64 cycles of one
+// compute unit's address unit per wave and store.  Nothing depends on scheduling.
+// What bounds it is latency, a few dependent steps.  1500 tokens x 8: 28 us when one workgroup took
+// 64 tokens at a time behind three barriers each, 20 with runs in one workgroup, 11.5 in sixteen.
+constexpr int kPermuteWaves = 16;
+inline unsigned permute_workgroups(long P) { return (unsigned)std::max(1l, std::min((long)kPermuteWaves, P / 512)); }
+inline size_t permute_lds_bytes(int E) { return (size_t)kPermuteWaves * E * sizeof(int); }
+
+__global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(PermuteParams p)
 {
+    extern __shared__ __align__(16) int hist[];             // [wave][E]: counts, then the next free row
     __shared__ int tot[kMaxExperts + 1];                    // rows per expert
     __shared__ int off[kMaxExperts + 2];                    // first sorted row of each expert
     __shared__ int pfirst[kMaxExperts + 2];                 // first (small or VALU) problem of each expert
     __shared__ int bfirst[kMaxExperts + 2];                 // first big problem of each expert
-    __shared__ int done[kMaxExperts + 1];                   // rows of the expert placed so far
-    __shared__ unsigned long long mask[kMaxExperts + 1];
-    __shared__ unsigned long long wave_sum[16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ unsigned long long wave_sum[kPermuteWaves];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int P = p.T * p.k;
     const int E1 = p.E + (p.shared_rows ? 1 : 0);           // experts including the always-on one
+    const int run = ((P + kPermuteWaves - 1) / kPermuteWaves + 63) & ~63;
+    const int q_begin = min(P, wave * run), q_end = min(P, q_begin + run);
+    constexpr int kAhead = 8;                               // groups of 64 pairs whose experts are requested together
+    // (lanes past the end of the run read its last pair and do not count)
+    auto experts_of = [&](int q0, int (&e)[kAhead]) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) e[j] = p.idx[min(q0 + 64 * j + lane, q_end - 1)];
+    };
 
-    for (int e = tid; e <= p.E; e += 1024) { tot[e] = 0; done[e] = 0; mask[e] = 0; }
+    for (int e = tid; e < kPermuteWaves * p.E; e += 64 * kPermuteWaves) hist[e] = 0;
     __syncthreads();
-    for (int q = tid; q < P; q += 1024) atomicAdd(&tot[p.idx[q]], 1);
+    int* const mine_hist = hist + wave * p.E;
+    for (int q0 = q_begin; q0 < q_end; q0 += 64 * kAhead) {
+        int e[kAhead];
+        experts_of(q0, e);
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j)
+            if (q0 + 64 * j + lane < q_end) atomicAdd(&mine_hist[e[j]], 1);
+    }
+    __syncthreads();
+    if (tid < p.E) {                                        // (at most 1024 experts)
+        int before = 0, c[kPermuteWaves];
+#pragma unroll
+        for (int w = 0; w < kPermuteWaves; ++w) c[w] = hist[w * p.E + tid];
+#pragma unroll
+        for (int w = 0; w < kPermuteWaves; ++w) {
+            hist[w * p.E + tid] = before;
+            before += c[w];
+        }
+        tot[tid] = before;
+    }
     if (p.shared_rows && tid == 0) tot[p.E] = p.T;
     __syncthreads();
 
@@ -582,9 +618,8 @@ __global__ __launch_bounds__(1024) void moe_permute_kernel(PermuteParams p)
             pfirst[tid] = (int)((excl >> 22) & 0x1fffffu);
             bfirst[tid] = (int)(excl >> 43);
         }
-        if (tid == E1 - 1) {
+        if (tid == E1 - 1 && blockIdx.x == 0) {
             const unsigned long long all = excl + mine;
-            off[E1] = (int)(all & 0x3fffffu);
             const int total_small = (int)((all >> 22) & 0x1fffffu);
             p.counts[0] = p.use_valu ? total_small : 0;
             p.counts[1] = p.use_valu ? 0 : total_small;
@@ -592,8 +627,10 @@ __global__ __launch_bounds__(1024) void moe_permute_kernel(PermuteParams p)
         }
     }
     __syncthreads();
-    for (int x = tid; x <= p.E; x += 1024) p.offsets[x] = off[x];
-    if (tid < E1) {
+    if (blockIdx.x == 0) {
+        for (int x = tid; x <= p.E; x += 1024) p.offsets[x] = x < E1 ? off[x] : P;
+    }
+    if (tid < E1 && blockIdx.x == 0) {
         const int m = tot[tid];
         if (m > 0) {
             if (p.use_valu) {
@@ -608,29 +645,40 @@ __global__ __launch_bounds__(1024) void moe_permute_kernel(PermuteParams p)
         }
     }
 
-    for (int t0 = 0; t0 < p.T; t0 += 64) {
-        const int nq = min(64, p.T - t0) * p.k;
-        const int q0 = t0 * p.k;
-        for (int i = tid; i < nq; i += 1024) atomicOr(&mask[p.idx[q0 + i]], 1ull << (i / p.k));
-        __syncthreads();
-        for (int i = tid; i < nq; i += 1024) {
-            const int q = q0 + i, e = p.idx[q];
-            const int at = off[e] + done[e] + __popcll(mask[e] & ((1ull << (i / p.k)) - 1ull));
-            p.perm[at] = q;
-            p.inv[q] = at;
-            p.row_expert[at] = e;
-        }
-        __syncthreads();
-        for (int e = tid; e < p.E; e += 1024) {
-            done[e] += __popcll(mask[e]);
-            mask[e] = 0;
-        }
-        __syncthreads();
-    }
-    if (p.shared_rows) {
+    if (p.shared_rows && blockIdx.x == 0) {
         for (int t = tid; t < p.T; t += 1024) {
             p.perm[P + t] = t * p.k;
             p.row_expert[P + t] = p.E;
+        }
+    }
+    if (wave % (int)gridDim.x != (int)blockIdx.x) return;
+    static_assert(kMaxExperts == 1 << 10, "ten bits of an expert's number");
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (int q0 = q_begin; q0 < q_end; q0 += 64 * kAhead) {
+        int ex[kAhead];
+        experts_of(q0, ex);
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            if (q0 + 64 * j >= q_end) break;                // wave-uniform
+            const int q = q0 + 64 * j + lane, e = ex[j];
+            const bool live = q < q_end;
+            unsigned long long same = __builtin_amdgcn_ballot_w64(live);    // the lanes with this lane's expert
+#pragma unroll
+            for (int b = 0; b < 10; ++b) {
+                const unsigned long long set = __builtin_amdgcn_ballot_w64((e >> b) & 1);
+                same &= set ^ ((unsigned long long)((e >> b) & 1) - 1ull);      // ~set in the lanes without the bit
+            }
+            // the wave's LDS accesses run in order; the fences keep the compiler to that across lanes
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (live) {
+                const int next = mine_hist[e];
+                const int at = off[e] + next + __popcll(same & below);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if ((same & ~below) == (1ull << lane)) mine_hist[e] = next + __popcll(same);      // the last of them
+                p.perm[at] = q;
+                p.inv[q] = at;
+                p.row_expert[at] = e;
+            }
         }
     }
 }
@@ -1036,7 +1084,10 @@ PermuteParams permute_params(const int32_t* idx, unsigned char* wsb, const MoeLa
 
 std::string run_permute(const PermuteParams& p, hipStream_t stream)
 {
-    hipLaunchKernelGGL(moe_permute_kernel, dim3(1), dim3(1024), 0, stream, p);
+    static bool raised[64] = {};
+    raise_dynamic_lds_limit((const void*)moe_permute_kernel, (int)permute_lds_bytes(kMaxExperts), raised,
+                            "moe_permute_kernel shared-memory attribute");
+    hipLaunchKernelGGL(moe_permute_kernel, dim3(permute_workgroups((long)p.T * p.k)), dim3(64 * kPermuteWaves), permute_lds_bytes(p.E), stream, p);
     hip_ok(hipGetLastError(), "moe_permute_kernel launch");
     return "moe_permute_kernel";
 }
@@ -1121,9 +1172,7 @@ extern "C" int berth_moe_permute(const int32_t* idx, int32_t* offsets, int32_t* 
     p.use_valu = (T == 1 || P <= (size_t)kValuPairs) ? 1 : 0;
     p.shared_rows = 0;
     p.big_min = !p.use_valu && at.big_min > 0 ? at.big_min : (1 << 30);
-    hipLaunchKernelGGL(moe_permute_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, p);
-    hip_ok(hipGetLastError(), "moe_permute_kernel launch");
-    g_moe_launch = "moe_permute_kernel";
+    g_moe_launch = run_permute(p, (hipStream_t)stream);
     MOE_TRY_END
 }
 
