@@ -1003,9 +1003,9 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
     const int groups = (T + kRouteTT - 1) / kRouteTT;
     if (T >= kRouteBigT && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && knobs().moe_route_slab) {
         // One launch.  Tokens per workgroup: one workgroup of sixteen waves runs per compute unit, and its
-        // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 12.8, 19.5 and
-        // 25 us), so the count with the fewest whole rounds of the chip wins.  1500 tokens x 128 experts:
-        // six tokens in one round of 250 workgroups 39 -> 26 us against four in 375.
+        // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 13, 20 and
+        // 30 us), so the count with the fewest whole rounds of the chip wins.  1500 tokens x 128 experts:
+        // six tokens in one round of 250 workgroups 30 us, four in 375 39.5.
         const int nslab = (E + kSlabExperts - 1) / kSlabExperts;
         constexpr int kSlabLdsMax = 144 * 1024;
         int tt = 1;
