@@ -305,28 +305,32 @@ static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int c
         long slots = ws.cu_count;
         if (balance > 1) slots = balance;
         const long G = units < slots ? units : slots;
-        const long per_wg = units / G;                                   // >= 1
-        const long parts = (KB + per_wg - 1) / per_wg + 1;               // workgroups that can share a tile
         const size_t part_bytes = (size_t)4 * mb * 2 * 16 * 64 * sizeof(float);
-        if (!(tiles <= kCounters / 2 && units < (1L << 30) &&
-              (size_t)tiles * parts * part_bytes <= kPartialBytes))
+        if (!(tiles <= kCounters / 2 && units < (1L << 30) && (size_t)G * 2 * part_bytes <= ws.partial_bytes))
             return false;
         p.tiles_y = mtiles;
         p.S = 1;
         p.units = (int)units;
         p.unit_q = (int)(units / G);
         p.unit_r = (int)(units % G);
-        p.max_parts = (int)parts;
         gemm_bits(p, k_bits, codebook, mb, stream, desc, dim3((unsigned)G, 1, 1));
         return true;
     };
     bool done = false;
-    if (balance && mb_plain == 4) {
-        // 256-row tiles pay when there are enough of them that few workgroups share a tile
-        // (measured at 512 rows: gate/up 5120x17408, 136 tiles, 148 -> 139 us; q, o and down
-        // with 40..48 tiles are 5 % slower than with 128-row tiles)
+    const long tiles128 = (long)nblocks * ((size_m + 127) / 128);
+    // (K = 1024 leaves the balanced kernels' single workgroup per compute unit in its epilogue for too
+    // long: 16384 columns at 600 / 768 / 1500 rows 42 / 46 / 70 us as whole tiles, 45 / 51 / 81 dealt out)
+    if (balance && mb_plain == 4 && (KB != 8 || rows256 >= 2 || tiles128 <= ws.cu_count)) {
+        // 256-row or 128-row tiles: a workgroup's k-block of the one takes 4.56 us, of the other 2.55
+        // (rows past the end cost as much as others), and the hand-over and finish of the larger tiles
+        // takes longer by 15 us where every tile is shared, 6 where some are, 3 of epilogue otherwise.
+        // Measured (128-row / 256-row, us): 17408x5120 at 512, 768, 1500 rows 128/135, 178/170, 337/306;
+        // 2048x8192 at 1024 rows 50/65, at 1500 77/74; 4096x17408 at 512, 600, 1500 rows 100/97, 122/131,
+        // 284/240.  A K below 1024 keeps the larger tiles wherever there are enough to go round.
         const long tiles256 = (long)nblocks * ((size_m + 255) / 256);
-        if (size_m > 128 && (rows256 >= 2 || (rows256 == 1 && tiles256 * 2 >= ws.cu_count))) done = balanced(8);
+        const long more = tiles256 >= ws.cu_count ? 300 : tiles256 * 2 > ws.cu_count ? 600 : 1500;
+        const bool wide = KB < 8 ? tiles256 * 2 >= ws.cu_count : (255 * tiles128 - 456 * tiles256) * KB > more * ws.cu_count;
+        if (size_m > 128 && (rows256 >= 2 || (rows256 == 1 && wide))) done = balanced(8);
         if (!done) done = balanced(4);
     }
     if (!done) {

@@ -29,7 +29,7 @@ static void gemm_launch_mb(const GemmParams& p, hipStream_t stream, std::string&
             hipLaunchKernelGGL((exl3_gemm_balanced_kernel<BITS, CB, MB>), grid, dim3(256), smem, stream, p);
             desc = "exl3_gemm_balanced_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + "," +
                    std::to_string(BM) + "x256> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
-                   " max_parts=" + std::to_string(p.max_parts) + " smem=" + std::to_string(smem);
+                   " smem=" + std::to_string(smem);
             return;
         }
         throw std::runtime_error("exl3 gemm: balanced launches use 128-row tiles");
@@ -50,8 +50,7 @@ static void gemm_launch_wide(const GemmParams& p, hipStream_t stream, std::strin
                             "exl3_gemm_wide_kernel shared-memory attribute");
     hipLaunchKernelGGL((exl3_gemm_wide_kernel<BITS, CB>), grid, dim3(512), kWideSmem, stream, p);
     desc = "exl3_gemm_wide_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + ",256x256> grid=" +
-           std::to_string(grid.x) + " units=" + std::to_string(p.units) + " max_parts=" + std::to_string(p.max_parts) +
-           " smem=" + std::to_string(kWideSmem);
+           std::to_string(grid.x) + " units=" + std::to_string(p.units) + " smem=" + std::to_string(kWideSmem);
 }
 
 // two problem lists in one grouped launch: 128-row problems first, 32-row problems behind them

@@ -73,7 +73,6 @@ struct GemmParams {
     // tile-major, are dealt out evenly to gridDim.x workgroups
     int units;                  // tiles * K/128; 0: not a balanced launch
     int unit_q, unit_r;         // units = unit_q * gridDim.x + unit_r
-    int max_parts;              // upper bound of workgroups that share one tile
     // A tile's finisher waits for the other sharers' partial sums with a bound: after
     // spin_limit polls it gives up, zeroes the tile's counters, stores 1 + the tile's counter
     // index to *fault (host-visible memory; may be null) and leaves the tile unwritten.
@@ -176,7 +175,10 @@ __device__ __forceinline__ bool wait_counter_bounded(unsigned* counter, unsigned
 struct KRange {
     int kb0, kb1, step;         // k-blocks kb0, kb0 + step, ... < kb1
     int part, parts;            // this workgroup's position (k order) and the number of sharers
-    size_t slot0;               // first partial-sum slot of the tile
+    size_t slot0;               // partial-sum slot of part 0; part j > 0 has slot_rest + j * slot_step
+    size_t slot_rest;
+    int slot_step;
+    __device__ size_t slot(int j) const { return j == 0 ? slot0 : slot_rest + (size_t)j * slot_step; }
     size_t counter;             // arrival counter of the tile
 };
 
@@ -439,9 +441,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         }
         __syncthreads();
         const bool finisher = s_last != 0;
-        const float* all = p.partials + kr.slot0 * kPerWg + (size_t)wave * MB * 2 * 16 * 64;
+        const float* all = p.partials + (size_t)wave * MB * 2 * 16 * 64;
         if (!(finisher && kr.part == 0)) {
-            float* mine = p.partials + (kr.slot0 + kr.part) * kPerWg + (size_t)wave * MB * 2 * 16 * 64;
+            float* mine = p.partials + kr.slot(kr.part) * kPerWg + (size_t)wave * MB * 2 * 16 * 64;
             if (active) {
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
@@ -486,7 +488,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 #pragma unroll
                     for (int jj = 0; jj < kParts; ++jj) {
                         const int j = j0 + jj < kr.parts ? j0 + jj : kr.parts - 1;      // past the end: ignored
-                        const float* src = all + (size_t)j * kPerWg;
+                        const float* src = all + kr.slot(j) * kPerWg;
 #pragma unroll
                         for (int b = 0; b < kGroup; ++b) {
                             const int blk = g0 + b;             // = mb * 2 + f
@@ -594,19 +596,20 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_kernel(GemmParams p)
     kr.kb0 = split;
     kr.kb1 = p.K >> 7;
     kr.step = p.S;
+    kr.slot_step = 1;
     kr.part = split;
     kr.parts = p.S;
     if (!p.problems) {
         const int tile = p.tile0 + unit;
         kr.counter = (size_t)unit;
-        kr.slot0 = kr.counter * p.S;
+        kr.slot0 = kr.slot_rest = kr.counter * p.S;
         gemm_tile<BITS, CB, MB, true>(p, tile / nblocks, tile % nblocks, kr, 0, smem);
         return;
     }
     if ((int)blockIdx.z >= *p.num_problems) return;
     // grouped: (linear, problem, column block)
     kr.counter = ((size_t)blockIdx.y * p.tiles_y + blockIdx.z) * nblocks + unit;
-    kr.slot0 = kr.counter * p.S;
+    kr.slot0 = kr.slot_rest = kr.counter * p.S;
     gemm_tile<BITS, CB, MB, false>(p, blockIdx.z, unit, kr, blockIdx.y, smem, p.problems);
 }
 
@@ -634,7 +637,8 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
     kr.part = 0;
     kr.parts = 1;
     kr.counter = 0;
-    kr.slot0 = 0;
+    kr.slot0 = kr.slot_rest = 0;
+    kr.slot_step = 0;
     const int z = blockIdx.z;
     if (z < p.max_big) {
         if (z >= *p.num_big) return;
@@ -672,13 +676,13 @@ __device__ __forceinline__ int die_major_index(int i, int n)
     return (n & 7) == 0 ? (i & 7) * (n >> 3) + (i >> 3) : i;
 }
 
-template <int BITS, int CB, int MB>
-__device__ __forceinline__ void gemm_segment(const GemmParams& p, const int w, const int u, const int stop,
-                                             unsigned char* smem)
+// the k-blocks of the tile that unit u lies in, up to `stop`, for workgroup w.  Every workgroup has two
+// partial-sum slots, one for the tile its range starts in and one for the tile it ends in (no other is
+// shared), so that any number of tiles can be dealt out.
+__device__ __forceinline__ KRange range_segment(const GemmParams& p, const int w, const int u, const int stop, int& tile)
 {
-    const int nblocks = ((p.N + 255) >> 8) * (p.num_slices > 0 ? p.num_slices : 1);
     const int KB = p.K >> 7;
-    const int tile = u / KB;
+    tile = u / KB;
     const int t0 = tile * KB;                                   // the tile's first unit
     const int w_first = range_owner(p, t0);
     const int w_last = range_owner(p, t0 + KB - 1);
@@ -689,7 +693,19 @@ __device__ __forceinline__ void gemm_segment(const GemmParams& p, const int w, c
     kr.part = w - w_first;
     kr.parts = w_last - w_first + 1;
     kr.counter = (size_t)tile;
-    kr.slot0 = (size_t)tile * p.max_parts;
+    kr.slot_rest = 2 * (size_t)w_first;
+    kr.slot0 = kr.slot_rest + (range_start(p, w_first) < t0 ? 1 : 0);
+    kr.slot_step = 2;
+    return kr;
+}
+
+template <int BITS, int CB, int MB>
+__device__ __forceinline__ void gemm_segment(const GemmParams& p, const int w, const int u, const int stop,
+                                             unsigned char* smem)
+{
+    const int nblocks = ((p.N + 255) >> 8) * (p.num_slices > 0 ? p.num_slices : 1);
+    int tile;
+    const KRange kr = range_segment(p, w, u, stop, tile);
     const int t = p.tile0 + tile;
     gemm_tile<BITS, CB, MB, true>(p, t / nblocks, t % nblocks, kr, 0, smem);
 }

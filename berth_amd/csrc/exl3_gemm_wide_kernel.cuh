@@ -215,9 +215,9 @@ __device__ __forceinline__ void gemm_tile_wide(const GemmParams& p, const int ti
         __syncthreads();
         const bool finisher = s_last != 0;
         const size_t wave_off = (size_t)wave8 * kPerWave;
-        const float* all = p.partials + kr.slot0 * kPerWg + wave_off;
+        const float* all = p.partials + wave_off;
         if (!(finisher && kr.part == 0)) {
-            float* mine = p.partials + (kr.slot0 + kr.part) * kPerWg + wave_off;
+            float* mine = p.partials + kr.slot(kr.part) * kPerWg + wave_off;
             if (active) {
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
@@ -252,7 +252,7 @@ __device__ __forceinline__ void gemm_tile_wide(const GemmParams& p, const int ti
             constexpr int kGroup = 4;                           // (mb, f) register blocks per batch
             const int first = kr.part == 0 ? 1 : 0;
             for (int j = first; j < kr.parts; ++j) {
-                const float* src = all + (size_t)j * kPerWg;
+                const float* src = all + kr.slot(j) * kPerWg;
 #pragma unroll
                 for (int g0 = 0; g0 < MB * 2; g0 += kGroup) {
                     float tmp[kGroup][16];
@@ -345,19 +345,8 @@ __device__ __forceinline__ void gemm_segment_wide(const GemmParams& p, const int
                                                   unsigned char* smem)
 {
     const int nblocks = ((p.N + 255) >> 8) * (p.num_slices > 0 ? p.num_slices : 1);
-    const int KB = p.K >> 7;
-    const int tile = u / KB;
-    const int t0 = tile * KB;
-    const int w_first = range_owner(p, t0);
-    const int w_last = range_owner(p, t0 + KB - 1);
-    KRange kr;
-    kr.kb0 = u - t0;
-    kr.kb1 = stop - t0;
-    kr.step = 1;
-    kr.part = w - w_first;
-    kr.parts = w_last - w_first + 1;
-    kr.counter = (size_t)tile;
-    kr.slot0 = (size_t)tile * p.max_parts;
+    int tile;
+    const KRange kr = range_segment(p, w, u, stop, tile);
     const int t = p.tile0 + tile;
     gemm_tile_wide<BITS, CB>(p, t / nblocks, t % nblocks, kr, smem);
 }
