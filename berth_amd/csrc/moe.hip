@@ -215,7 +215,7 @@ __global__ __launch_bounds__(64) void moe_route_segments_kernel(RouteParams p)
 // segment; second launch: one workgroup per token adds the segments in order,
 // adds the bias and selects.
 constexpr int kRouteBigGroup = 16;  // most tokens a first-launch workgroup takes
-constexpr int kRouteBigT = 32;      // calls with at least this many tokens take the two-launch path
+constexpr int kRouteBigT = 32;      // where the one-launch form does not apply: from this many tokens on two launches
 
 // How the 256 threads of a first-launch workgroup are used: `lanes` threads cover the expert
 // pairs (64, 128 or 256: a router of up to 128 experts needs one wave), and 256 / lanes token
@@ -1001,7 +1001,9 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
     p.nseg = (H + kRouteSeg - 1) / kRouteSeg;
     if (sort && T == 1) p.sort = *sort;
     const int groups = (T + kRouteTT - 1) / kRouteTT;
-    if (T >= kRouteBigT && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && knobs().moe_route_slab) {
+    // (from two tokens on: 2 .. 31 tokens took moe_route_kernel, whose sums cross memory and a counter before a
+    // token can be finished: 16 us, 13 here; a whole layer of 512 experts at 2 / 16 tokens 66 / 126 -> 58 / 118)
+    if (T > 1 && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && knobs().moe_route_slab) {
         // One launch.  Tokens per workgroup: one workgroup of sixteen waves runs per compute unit, and its
         // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 13, 20 and
         // 30 us), so the count with the fewest whole rounds of the chip wins.  1500 tokens x 128 experts:
