@@ -530,6 +530,36 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
     return "pair " + d0 + " + " + desc + " out=f16";
 }
 
+// Grouped launches of problems of a few rows: room for the column blocks that a workgroup can touch
+// when the list is as long as it can get, in as few rounds of one workgroup per compute unit as that
+// takes.
+struct GroupRowsPlan {
+    bool ok = false;
+    unsigned grid = 0;
+    size_t lds = 0;
+};
+static GroupRowsPlan plan_group_rows(const Workspace& ws, const GroupedArgs& g)
+{
+    GroupRowsPlan pl;
+    if (g.size_k < 256 || g.small_rows > 16) return pl;
+    const unsigned long long TR4 = (unsigned)g.size_k / 64, blocks = (unsigned long long)g.max_problems * g.num_lins * (g.size_n / 128);
+    const unsigned long long U = blocks * TR4;
+    if (blocks > (unsigned)kCounters / 2 || U * TR4 >= (1ull << 32) || blocks * blocks >= (1ull << 32)) return pl;
+    for (unsigned rounds = 1; rounds <= 64; rounds *= 2) {
+        const unsigned long long G = (unsigned long long)ws.cu_count * rounds;
+        const unsigned long long most = std::max((U + G - 1) / G, 8ull);        // (a short list: 4..7 units each)
+        const unsigned long long ncb = (most + TR4 - 2) / TR4 + 1;
+        if (ncb > (unsigned)kRowsWaves) continue;
+        const size_t lds = rows_group_lds_bytes(g.small_rows, (int)ncb);
+        if (lds > 160 * 1024 || G * 2 * g.small_rows * 512 > ws.partial_bytes) continue;
+        pl.ok = true;
+        pl.grid = (unsigned)G;
+        pl.lds = lds;
+        return pl;
+    }
+    return pl;
+}
+
 // grouped: problems of at most 32 * g.mb rows each; a_had rows are in problem order
 std::string launch_gemm_grouped(const GroupedArgs& g)
 {
@@ -559,6 +589,23 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
     if (g.shared) std::memcpy(p.shared, g.shared, sizeof(p.shared));
     p.partials = ws.partials;
     p.counters = ws.counters;
+    if (g.small_rows > 0 && g.max_big == 0) {
+        const GroupRowsPlan pl = plan_group_rows(ws, g);
+        if (pl.ok) {
+            const long blocks = (long)g.num_lins * (g.size_n / 128);
+            std::string desc;
+            p.M = g.small_rows;
+            p.cstride = gemm_counter_stride(g.max_problems * blocks);
+            p.group_blocks = (int)blocks;
+            p.m_rt = magic((unsigned)blocks);
+            p.m_tr = magic((unsigned)g.size_k / 64);
+            p.m_nb = magic((unsigned)g.size_n / 128);
+            p.lds_bytes = (unsigned)pl.lds;
+            gemm_bits(p, g.k_bits, g.codebook, -3, g.stream, desc, dim3(pl.grid));
+            hip_ok(hipGetLastError(), "exl3_gemm_rows_kernel grouped launch");
+            return desc + " grouped";
+        }
+    }
     const int nblocks = (g.size_n + 255) / 256;
     const long tiles = (long)g.max_problems * g.num_lins * nblocks;
     p.cstride = gemm_counter_stride(tiles);

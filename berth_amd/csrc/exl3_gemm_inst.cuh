@@ -67,14 +67,15 @@ static void gemm_launch_mixed(const GemmParams& p, hipStream_t stream, std::stri
            std::to_string(grid.z - p.max_big) + ") smem=" + std::to_string(smem);
 }
 
-// few rows (2..32), units dealt out evenly; mb = -1 / -2: one or two tiles of 16 rows
-template <int BITS, int CB, int MT>
+// few rows (2..32), units dealt out evenly; mb = -1 / -2: one or two tiles of 16 rows, -3: a list of
+// problems of up to 16 rows
+template <int BITS, int CB, int MT, bool GROUPED = false>
 static void gemm_launch_rows(const GemmParams& p, hipStream_t stream, std::string& desc, dim3 grid)
 {
     static bool raised[64] = {};
-    raise_dynamic_lds_limit((const void*)exl3_gemm_rows_kernel<BITS, CB, MT>, 160 * 1024, raised,
+    raise_dynamic_lds_limit((const void*)exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED>, 160 * 1024, raised,
                             "exl3_gemm_rows_kernel shared-memory attribute");
-    hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT>), grid, dim3(1024), p.lds_bytes, stream, p);
+    hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED>), grid, dim3(1024), p.lds_bytes, stream, p);
     desc = "exl3_gemm_kernel/rows<" + std::to_string(BITS) + "," + std::to_string(CB) + "," + std::to_string(16 * MT) +
            "x128> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
            (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
@@ -99,6 +100,7 @@ static void gemm_launch(const GemmParams& p, int mb, hipStream_t stream, std::st
     if (p.max_big > 0) gemm_launch_mixed<BITS, CB>(p, stream, desc, grid);
     else if (mb == -1) gemm_launch_rows<BITS, CB, 1>(p, stream, desc, grid);
     else if (mb == -2) gemm_launch_rows<BITS, CB, 2>(p, stream, desc, grid);
+    else if (mb == -3) gemm_launch_rows<BITS, CB, 1, true>(p, stream, desc, grid);
     else if (mb == -12) gemm_launch_block<BITS, CB, 4>(p, stream, desc, grid);
     else if (mb == -14) gemm_launch_block<BITS, CB, 6>(p, stream, desc, grid);
     else if (mb == -16) gemm_launch_block<BITS, CB, 8>(p, stream, desc, grid);

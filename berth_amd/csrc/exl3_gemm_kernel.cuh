@@ -101,6 +101,7 @@ struct GemmParams {
     // m_rt for tiles_y.
     unsigned m_tr, m_nb, m_q, m_q1, m_s, m_rt;
     int rows_per_tile;
+    int group_blocks;           // grouped few-row launches: column blocks of 128 per problem, all linears (m_rt divides by it)
     unsigned lds_bytes;         // dynamic LDS of the launch
     const float* out_add;       // optional fp32 [M][N] (one linear, fp32 output): added to the output
     GemmSlice slice[kGemmMaxSlices];

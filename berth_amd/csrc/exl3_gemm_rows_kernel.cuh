@@ -27,6 +27,11 @@
 //     A column block that lies inside one workgroup's units is finished there.  Otherwise the
 //     sharers leave their sums in the workspace and the last to arrive adds them in k order, so
 //     results repeat bit for bit.
+//   * GROUPED: the column blocks are those of a list of problems (up to 16 expert-sorted rows each,
+//     problem-major, then the launch's one or two linears).  The list's length is only known on the
+//     device, so the deal is worked out there.  A workgroup looks its few blocks up once, into LDS.
+//     A operands come straight from the row-major rotated rows: a problem has few of them, and the
+//     lanes past the last repeat it, so that a load touches as many lines as there are rows.
 //
 // Measured (27B layer, traced): gate + up at 5 rows and 3 bits 62.6 -> 32.5 us against the VALU
 // kernel, at 24 rows and 4 bits 49.0 -> 40.6 against 32-row tiles (whose 544 workgroups also
@@ -46,6 +51,18 @@ __host__ __device__ constexpr size_t rows_lds_bytes(int rows, int ncb)
 {
     return (size_t)(ncb + 3) * rows * kRowsStride * 4 + (size_t)ncb * 256 + 16;
 }
+// of a GROUPED launch, behind that: the column blocks' tensors
+struct RowsGroupBlock {
+    const uint32_t* trellis;
+    const _Float16* svh;
+    const _Float16* a_had;
+    void* c;
+    int rows, pad;
+};
+__host__ __device__ constexpr size_t rows_group_lds_bytes(int rows, int ncb)
+{
+    return rows_lds_bytes(rows, ncb) + (size_t)ncb * sizeof(RowsGroupBlock);
+}
 
 // x / d for the launch's exact divisors, m = floor(2^32 / d) + 1 (0 for d = 1)
 __device__ __forceinline__ unsigned div_exact(unsigned x, unsigned m) { return m ? __umulhi(x, m) : x; }
@@ -59,6 +76,7 @@ struct RowsBlock {
     int n0;                     // first column inside the linear
     int ldc;                    // elements between output rows, and columns of the weight
     bool empty;                 // past the end of a narrower slice: nothing to compute
+    int rows;                   // of the block (GROUPED only)
 };
 __device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsigned cb)
 {
@@ -70,6 +88,7 @@ __device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsig
     b.n0 = (int)cb * 128;
     b.ldc = p.N;
     b.empty = false;
+    b.rows = p.M;
     if (p.num_slices > 0) {
         const unsigned nb = (unsigned)p.N >> 7;
         const unsigned sl = div_exact(cb, p.m_nb);
@@ -111,7 +130,7 @@ __device__ __forceinline__ const T* rows_uniform(const T* q)
     return (const T*)(((uint64_t)hi << 32) | lo);
 }
 
-template <int BITS, int CB, int MT>         // MT: tiles of 16 rows
+template <int BITS, int CB, int MT, bool GROUPED>       // MT: tiles of 16 rows
 __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -121,12 +140,19 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     const int cg = wave & 3, kg = wave >> 2;
     const int l16 = lane & 15, lg = lane >> 4;
     const unsigned TR4 = (unsigned)p.K >> 6;            // units per column block
-    const int M = p.M;
+    const int M = p.M;                                  // rows of the input; GROUPED: most rows of a problem
 
     // ---- this workgroup's units [u0, u1), this wave's quarter [w0, w1)
     const unsigned w = blockIdx.x;
-    const unsigned q = (unsigned)p.unit_q, rem = (unsigned)p.unit_r;
-    const unsigned S = (unsigned)p.S;
+    unsigned q = (unsigned)p.unit_q, rem = (unsigned)p.unit_r;
+    const unsigned S = GROUPED ? 0u : (unsigned)p.S;
+    if constexpr (GROUPED) {
+        const unsigned U = (unsigned)*p.num_problems * (unsigned)p.group_blocks * TR4;
+        const unsigned G = min((unsigned)gridDim.x, U >> 2);            // a unit for each k group at least
+        if (w >= G) return;
+        q = U / G;
+        rem = U - q * G;
+    }
     unsigned u0 = w * q + min(w, rem), u1 = (w + 1) * q + min(w + 1, rem);
     if (S) {
         const unsigned blk = div_exact(w, p.m_s), part = w - blk * S;
@@ -141,6 +167,44 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     float* const red = (float*)smem;
     uint32_t* const sv_lds = (uint32_t*)(red + (size_t)(ncb + 3) * M * kRowsStride);
     unsigned* const flags = sv_lds + ncb * 64;
+    RowsGroupBlock* const table = (RowsGroupBlock*)(flags + 4);
+    if constexpr (GROUPED) {
+        if (threadIdx.x < ncb) {
+            const unsigned cb = cb_first + threadIdx.x;
+            const unsigned prob = div_exact(cb, p.m_rt), in_prob = cb - prob * (unsigned)p.group_blocks;
+            const int which = (int)div_exact(in_prob, p.m_nb);
+            const GroupProblem gp = p.problems[prob];
+            const ExpertLin lin = gp.expert == p.shared_expert ? p.shared[p.lin_base + which]
+                                                               : p.experts[gp.expert * p.lins_per_expert + p.lin_base + which];
+            RowsGroupBlock g;
+            g.trellis = lin.trellis;
+            g.svh = lin.svh;
+            g.a_had = p.a_had[which] + (size_t)gp.row0 * p.K;
+            g.c = (char*)p.c[which] + (size_t)gp.row0 * p.N * (p.out_fp32 ? 4 : 2);
+            g.rows = gp.nrows;
+            g.pad = 0;
+            table[threadIdx.x] = g;
+        }
+        __syncthreads();
+    }
+    auto block = [&](const unsigned cb) -> RowsBlock {
+        if constexpr (GROUPED) {
+            const RowsGroupBlock& g = table[cb - cb_first];
+            const unsigned nb = (unsigned)p.N >> 7;
+            RowsBlock b;
+            b.trellis = rows_uniform(g.trellis);
+            b.svh = rows_uniform(g.svh);
+            b.a_had = rows_uniform(g.a_had);
+            b.c = (void*)rows_uniform((const char*)g.c);
+            b.n0 = (int)(cb - div_exact(cb, p.m_nb) * nb) * 128;
+            b.ldc = p.N;
+            b.empty = false;
+            b.rows = __builtin_amdgcn_readfirstlane(g.rows);
+            return b;
+        } else {
+            return rows_block(p, cb);
+        }
+    };
 
     // ---- the walk's operands: a pointer pair that runs two units ahead of the decode
     unsigned f_cb = div_exact(w0, p.m_tr);
@@ -149,10 +213,12 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     const char* f_a;
     long f_step;
     uint32_t t_off;                                     // bytes, per lane
-    const uint32_t a_off = (uint32_t)lane * 16;
-    constexpr int kUnitA = MT * 2 * 1024;               // bytes of A operands per unit
+    uint32_t a_off = (uint32_t)lane * 16;
+    constexpr int kUnitA = GROUPED ? 128 : MT * 2 * 1024;   // bytes of A operands per unit (GROUPED: of one row)
+    constexpr int kNextA = GROUPED ? 1 : 64;            // from a lane's operand to its next, in 16 bytes
     auto seek = [&](unsigned cb, unsigned k) {
-        const RowsBlock b = rows_block(p, cb);
+        const RowsBlock b = block(cb);
+        if constexpr (GROUPED) a_off = (uint32_t)min(l16, b.rows - 1) * (uint32_t)p.K * 2 + (uint32_t)lg * 32;
         if (b.empty) {                                  // read anything valid, use nothing
             f_t = (const char*)rows_uniform(b.a_had);
             f_step = 0;
@@ -174,8 +240,8 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
         const global_ptr<const half8_t> src = (global_ptr<const half8_t>)(as_global(f_a) + a_off);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            av[j][mt][0] = src[(2 * mt) * 64];
-            av[j][mt][1] = src[(2 * mt + 1) * 64];
+            av[j][mt][0] = src[(2 * mt) * kNextA];
+            av[j][mt][1] = src[(2 * mt + 1) * kNextA];
         }
     };
     auto advance = [&]() {                              // on the last unit it stays: read again, not used
@@ -199,7 +265,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     // the output scales, asked for now: the finish does not wait for them
     uint32_t sv_mine = 0;
     if ((unsigned)wave < ncb) {
-        const RowsBlock b = rows_block(p, cb_first + (unsigned)wave);
+        const RowsBlock b = block(cb_first + (unsigned)wave);
         if (!b.empty) sv_mine = as_global((const uint32_t*)(b.svh + b.n0))[lane];
     }
 
@@ -291,14 +357,18 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     unsigned cbi = 0;
     const unsigned qs1 = u0 + (L >> 2), qs2 = u0 + (L * 2 >> 2), qs3 = u0 + (L * 3 >> 2);
     while (true) {
-        while (row >= M) {
-            row -= M;
-            ++cbi;
+        if constexpr (GROUPED) {
+            for (int n; cbi < ncb && row >= (n = __builtin_amdgcn_readfirstlane(table[cbi].rows)); ++cbi) row -= n;
+        } else {
+            while (row >= M) {
+                row -= M;
+                ++cbi;
+            }
         }
         if (cbi >= ncb) break;
         const unsigned cbx = cb_first + cbi;
         const unsigned c0 = cbx * TR4, c1 = c0 + TR4;
-        const RowsBlock b = rows_block(p, cbx);
+        const RowsBlock b = block(cbx);
         if (!b.empty) {
             float z0 = 0.0f, z1 = 0.0f;
             const float* const base = red + (size_t)cbi * M * kRowsStride + row * kRowsStride + 2 * lane;
@@ -329,6 +399,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     // workgroup in; the last sharer to arrive adds the parts in k order and finishes the block
     auto owner = [&](unsigned x) {
         const unsigned big = rem * (q + 1);
+        if constexpr (GROUPED) return x < big ? x / (q + 1) : rem + (x - big) / q;
         if (S) return div_exact(x, p.m_tr) * S + (x % TR4 ? S - 1 : 0u);     // asked for a block's first or last unit
         return x < big ? div_exact(x, p.m_q1) : rem + div_exact(x - big, p.m_q);
     };
@@ -353,12 +424,12 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     for (int t = 0; t < 2; ++t) {
         if (!__builtin_amdgcn_readfirstlane((int)flags[t])) continue;
         const unsigned cbx = t == 0 ? cb_first : cb_last;
-        const RowsBlock b = rows_block(p, cbx);
+        const RowsBlock b = block(cbx);
         if (b.empty) continue;
         const unsigned wa = owner(cbx * TR4), wb = owner(cbx * TR4 + TR4 - 1);
         // the block is the first of every sharer's range but, unless that starts with it, the first sharer's
         const unsigned slot_a = S || wa * q + min(wa, rem) >= cbx * TR4 ? 0u : 1u;
-        for (int r = wave; r < M; r += kRowsWaves) {
+        for (int r = wave; r < (GROUPED ? b.rows : M); r += kRowsWaves) {
             float z0 = 0.0f, z1 = 0.0f;
             for (unsigned x = wa; x <= wb; x += 8) {
                 float2_t part[8];

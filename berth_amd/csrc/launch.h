@@ -78,6 +78,7 @@ struct Knobs {
     int gemm_rows_units;        // BERTH_GEMM_ROWS_UNITS        fewest units for which the few-row kernel is taken (0: never, -1: by row count)
     int counter_stride;         // BERTH_COUNTER_STRIDE         cap on the words between arrival counters (1..32)
     int moe_big_min;            // BERTH_MOE_BIG_MIN
+    int moe_few_tokens;         // BERTH_MOE_FEW_TOKENS
     int moe_route_slab;         // BERTH_MOE_ROUTE_SLAB: 0 keeps the two-launch routing of many tokens
     int moe_fold_combine;       // BERTH_MOE_FOLD_COMBINE
     int moe_inline_route;       // BERTH_MOE_INLINE_ROUTE
@@ -183,6 +184,7 @@ struct GroupedArgs {
     int shared_expert;          // expert index the problem list uses for it (-1: none)
     int single_row;             // every problem has exactly one row
     int mb;                     // MFMA path: rows per problem / 32 (1 or 4)
+    int small_rows = 0;         // MFMA path: every problem has at most this many rows, 16 or fewer (0: up to 32 * mb)
     const void* problems;       // GroupProblem[max_problems]
     const int* num_problems;
     int max_problems;

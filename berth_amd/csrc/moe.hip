@@ -598,7 +598,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(Permute
                 nbig = p.big_min <= kGemmBigRows ? c / kGemmBigRows : 0;
                 int rem = c - nbig * kGemmBigRows;
                 if (rem >= p.big_min) { ++nbig; rem = 0; }
-                nsmall = (rem + kGemmRows - 1) / kGemmRows;
+                nsmall = (rem + p.small_rows - 1) / p.small_rows;
             }
         }
         const unsigned long long mine = ((unsigned long long)nbig << 43) | ((unsigned long long)nsmall << 22) | (unsigned)c;
@@ -639,8 +639,8 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(Permute
                 int r = 0;
                 for (int j = bfirst[tid]; m - r >= p.big_min; r += kGemmBigRows, ++j)
                     p.bprob[j] = GroupProblem{tid, off[tid] + r, min(kGemmBigRows, m - r), 0};
-                for (int j = pfirst[tid]; r < m; r += kGemmRows, ++j)
-                    p.mprob[j] = GroupProblem{tid, off[tid] + r, min(kGemmRows, m - r), 0};
+                for (int j = pfirst[tid]; r < m; r += p.small_rows, ++j)
+                    p.mprob[j] = GroupProblem{tid, off[tid] + r, min(p.small_rows, m - r), 0};
             }
         }
     }
@@ -857,7 +857,7 @@ size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 // problem counts, one-row (VALU) problems and 32-row (MFMA) problems
 struct PermuteScratch {
     size_t row_expert, counts, vprob, mprob, bprob, total;
-    int max_m, max_b, big_min;
+    int max_m, max_b, big_min, small_rows;
 };
 
 // An expert's rows beyond 32 go to MFMA problems of up to 128 rows (the weights are decoded
@@ -866,19 +866,27 @@ struct PermuteScratch {
 // Calls with few rows keep them too: there the launch splits K over several workgroups,
 // which the mixed launch does not.
 constexpr int kBigMinRows = 256;
-int moe_big_min(size_t rows)
+// Calls of up to 16 tokens: problems of 16 rows (an expert has at most one per token, so one each) for
+// the grouped few-row kernel, which deals the work out evenly however many problems there are.  Layer of
+// 128 experts x 768, top 8, 4 bits, at 2 / 8 / 16 tokens 55.6 / 83.1 / 106 -> 49.5 / 72.4 / 91.5 us; 512
+// experts x 512 at 3 bits 58 / 89 / 118 -> 55 / 82 / 115.  With more tokens an expert's rows may need
+// several problems, each with a decode of its own: 64 tokens with even choices 136 -> 131, with a few
+// popular experts 95 -> 126.
+int moe_small_rows(int T) { return T <= knobs().moe_few_tokens ? 16 : kGemmRows; }
+int moe_big_min(size_t rows, int small_rows)
 {
+    if (small_rows != kGemmRows) return 0;
     const int v = knobs().moe_big_min;
     return v > 0 && v <= kGemmBigRows && rows >= (size_t)kBigMinRows ? v : 0;
 }
 // capacities of the two problem lists of `rows` rows over `experts` experts
-void problem_capacity(size_t rows, size_t experts, int big_min, int& max_m, int& max_b)
+void problem_capacity(size_t rows, size_t experts, int big_min, int small_rows, int& max_m, int& max_b)
 {
     if (big_min > 0) {
         max_m = (int)std::min<size_t>(((size_t)(big_min + kGemmRows - 2) / kGemmRows) * experts, rows);
         max_b = (int)(rows / big_min);
     } else {
-        max_m = (int)(std::min<size_t>(experts, rows) + rows / kGemmRows + 1);
+        max_m = (int)(std::min<size_t>(experts, rows) + rows / small_rows + 1);
         max_b = 0;
     }
 }
@@ -892,8 +900,9 @@ PermuteScratch permute_scratch_layout(int T, int k, int E)
     s.counts = at; at = align_up(at + 16);
     s.vprob = at; at = align_up(at + small * sizeof(GroupProblem));
     s.mprob = at;
-    s.big_min = moe_big_min(P);
-    problem_capacity(P, (size_t)E, s.big_min, s.max_m, s.max_b);
+    s.small_rows = moe_small_rows(T);
+    s.big_min = moe_big_min(P, s.small_rows);
+    problem_capacity(P, (size_t)E, s.big_min, s.small_rows, s.max_m, s.max_b);
     at = align_up(at + (size_t)std::max(s.max_m, 1) * sizeof(GroupProblem));
     s.bprob = at;
     s.total = align_up(at + (size_t)std::max(s.max_b, 1) * sizeof(GroupProblem));
@@ -903,7 +912,7 @@ PermuteScratch permute_scratch_layout(int T, int k, int E)
 struct MoeLayout {
     size_t idx, w, parts, offsets, perm, inv, row_expert, counts, vprob, mprob, bprob;
     size_t ah0, ah1, g, u, ahd, slot_out, sg, su, s_ahad, shared_out, vlin, gate_scale, total;
-    int max_v, max_m, max_b, big_min, nseg;
+    int max_v, max_m, max_b, big_min, small_rows, nseg;
 };
 
 // One token: the down projection's last arrival per column block also combines the block.
@@ -935,8 +944,9 @@ MoeLayout moe_layout(int T, int H, int E, int k, int I, int shared_I)
     const bool use_valu = T == 1 || R <= (size_t)kValuPairs;      // one row per problem, or very few rows
     L.max_v = use_valu ? (int)(std::min<size_t>((size_t)E, P) + (fold ? 1 : 0)) : 0;
     const size_t E1 = (size_t)E + (fold ? 1 : 0);
-    L.big_min = use_valu ? 0 : moe_big_min(R);
-    if (!use_valu) problem_capacity(R, E1, L.big_min, L.max_m, L.max_b);
+    L.small_rows = moe_small_rows(T);
+    L.big_min = use_valu ? 0 : moe_big_min(R, L.small_rows);
+    if (!use_valu) problem_capacity(R, E1, L.big_min, L.small_rows, L.max_m, L.max_b);
     size_t at = 0;
     auto take = [&](size_t bytes) { size_t r = at; at = align_up(at + bytes); return r; };
     L.idx = take(P * 4);
@@ -1055,8 +1065,8 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
         hip_ok(hipGetLastError(), "moe_route_one_token_kernel launch");
         return std::string("moe_route_one_token_kernel grid=1") + (p.sort.perm ? " (with the sort of the one token)" : "");
     }
-    if ((long)groups * kRouteCounterStride > kCounters) throw std::runtime_error("moe route: too many tokens for the counter table");
     dim3 grid(p.nseg, groups);
+    if ((long)groups * kRouteCounterStride > kCounters) throw std::runtime_error("moe route: too many tokens for the counter table");
     hipLaunchKernelGGL(moe_route_kernel, grid, dim3(256), 0, stream, p);
     hip_ok(hipGetLastError(), "moe_route_kernel launch");
     return "moe_route_kernel grid=" + std::to_string(grid.x) + "x" + std::to_string(grid.y) +
@@ -1080,6 +1090,7 @@ PermuteParams permute_params(const int32_t* idx, unsigned char* wsb, const MoeLa
     p.E = E;
     p.use_valu = L.max_v > 0 ? 1 : 0;
     p.shared_rows = fold ? 1 : 0;
+    p.small_rows = L.small_rows;
     p.big_min = L.big_min > 0 ? L.big_min : (1 << 30);
     return p;
 }
@@ -1173,6 +1184,7 @@ extern "C" int berth_moe_permute(const int32_t* idx, int32_t* offsets, int32_t* 
     p.E = E;
     p.use_valu = (T == 1 || P <= (size_t)kValuPairs) ? 1 : 0;
     p.shared_rows = 0;
+    p.small_rows = at.small_rows;
     p.big_min = !p.use_valu && at.big_min > 0 ? at.big_min : (1 << 30);
     g_moe_launch = run_permute(p, (hipStream_t)stream);
     MOE_TRY_END
@@ -1263,6 +1275,7 @@ extern "C" int berth_moe_grouped_exl3(const void* a, const void* a_up, const int
         g.num_problems = (const int*)(sb + at.counts) + 1;
         g.max_problems = at.max_m;
         g.mb = 1;
+        g.small_rows = at.small_rows < kGemmRows ? at.small_rows : 0;
         if (at.max_b > 0) {
             g.big_problems = sb + at.bprob;
             g.num_big = (const int*)(sb + at.counts) + 2;
@@ -1421,6 +1434,7 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.num_problems = (const int*)(wsb + L.counts) + 1;
         g.max_problems = L.max_m;
         g.mb = 1;
+        g.small_rows = L.small_rows < kGemmRows ? L.small_rows : 0;
         desc += " + " + launch_gemm_grouped(g);
     }
 
@@ -1517,6 +1531,7 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.num_problems = (const int*)(wsb + L.counts) + 1;
         g.max_problems = L.max_m;
         g.mb = 1;
+        g.small_rows = L.small_rows < kGemmRows ? L.small_rows : 0;
         desc += " + " + launch_gemm_grouped(g);
     }
 

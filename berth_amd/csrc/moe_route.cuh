@@ -37,12 +37,13 @@ struct PermuteParams {
     int32_t* row_expert;    // [R] sorted position -> expert
     int32_t* counts;        // [3] number of VALU problems, small MFMA problems, big MFMA problems
     GroupProblem* vprob;
-    GroupProblem* mprob;    // <= 32 rows each
+    GroupProblem* mprob;    // <= small_rows rows each
     GroupProblem* bprob;    // <= 128 rows each
     int T, k, E;
     int use_valu;           // 1: every expert is one VALU problem (<= 8 rows each); 0: MFMA problems: an
                             // expert's rows go to big problems of 128 and the rest to small ones of <= 32
     int shared_rows;        // 1: rows P .. P + T - 1 belong to an always-on expert with index E (token order)
+    int small_rows;         // rows of a small problem: 32, or 16
     int big_min;            // a remainder of at least this many rows becomes a (partial) big problem
 };
 

@@ -1,15 +1,18 @@
-"""Routing and permutation of many tokens: every token count per workgroup that the one-launch
-routing chooses between, and the permutation on either side of where it takes more workgroups
-and where the waves' runs end.  Bit-exact against the oracle."""
+"""MoE launches by token count.  Routing and permutation of many tokens: every token count per
+workgroup that the one-launch routing chooses between, and the permutation on either side of where
+it takes more workgroups and where the waves' runs end, bit-exact against the oracle.  Layers of up
+to 16 tokens: the grouped few-row kernel, stage by stage."""
 import numpy as np
 import pytest
 import torch
 
 from berth_amd import kernels as K
 from berth_amd import synth
+from berth_amd.device import Gpu
+from berth_amd.moe import MoeLayer
 from oracle import oracle as O
-from tests.gpu_util import DEV
-from tests.test_gpu_moe import _route
+from tests.gpu_util import DEV, dev
+from tests.test_gpu_moe import _check_stages, _make_layer, _route
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +46,32 @@ def test_permutation_of_many_pairs(T, k, E, hot):
     assert np.array_equal(off.cpu().numpy(), ooff)
     assert np.array_equal(perm.cpu().numpy(), operm)
     assert np.array_equal(inv.cpu().numpy()[operm], np.arange(T * k))
+
+
+@pytest.mark.parametrize("T,H,E,k,I,bits,shared_I", [
+    (16, 256, 2, 1, 256, 4, 256),       # sixteen rows in one problem, four units a column block, the shared expert among them
+    (9, 1024, 20, 8, 128, 3, 0),        # down projection of one k-block: the 32-row kernel on 16-row problems
+    (16, 2048, 128, 8, 768, 4, 0),
+    (5, 512, 300, 7, 384, 6, 0),        # three column blocks, ranges of one and a bit of them
+    (3, 256, 4, 3, 256, 2, 128),        # fewer units than four for every compute unit
+    (12, 640, 40, 8, 512, 5, 512),
+])
+def test_few_token_layers_on_the_grouped_few_row_kernel(T, H, E, k, I, bits, shared_I):
+    gpu = Gpu(0)
+    wr, experts_np, experts, shared_np, shared = _make_layer(gpu, 9100 + T + H, H, E, I, bits, shared_I, 10.0)
+    layer = MoeLayer(gpu, wr, experts, k, shared=shared)
+    x = (synth.activations(T + H, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
+    out, again = (torch.zeros((T, H), dtype=torch.float32, device=DEV) for _ in range(2))
+    idx = torch.zeros((T, k), dtype=torch.int32, device=DEV)
+    w = torch.zeros((T, k), dtype=torch.float32, device=DEV)
+    d_x = dev(x.view(np.uint16))
+    layer.forward(gpu, d_x, out, T, idx, w)
+    torch.cuda.synchronize()
+    assert "exl3_gemm_kernel/rows" in K.moe.last_launch(), K.moe.last_launch()
+    want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, 2, shared=shared_np, shared_I=shared_I)
+    assert np.array_equal(idx.cpu().numpy(), oi)
+    _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I)
+    for _ in range(3):
+        layer.forward(gpu, d_x, again, T)
+        torch.cuda.synchronize()
+        assert torch.equal(again, out)
