@@ -864,8 +864,12 @@ struct PermuteScratch {
 // once per problem, so once per 128 rows instead of once per 32); a remainder of fewer than
 // `big_min` rows stays a 32-row problem.  BERTH_MOE_BIG_MIN: 0 keeps 32-row problems only.
 // Calls with few rows keep them too: there the launch splits K over several workgroups,
-// which the mixed launch does not.
+// which the mixed launch does not.  So do calls of up to 128 tokens, where an expert has at most
+// four of them: a 128-row problem is then the launch's longest workgroup and the rest waits for it
+// (with / without, few popular experts: 512 experts at 64 tokens 95.5 / 79 us, at 128 109 / 110, 60
+// experts at 128 77 / 57; 128 experts at 256 tokens 107 / 125).
 constexpr int kBigMinRows = 256;
+constexpr int kBigMinTokens = 129;
 // Calls of up to 16 tokens: problems of 16 rows (an expert has at most one per token, so one each) for
 // the grouped few-row kernel, which deals the work out evenly however many problems there are.  Layer of
 // 128 experts x 768, top 8, 4 bits, at 2 / 8 / 16 tokens 55.6 / 83.1 / 106 -> 49.5 / 72.4 / 91.5 us; 512
@@ -873,9 +877,9 @@ constexpr int kBigMinRows = 256;
 // several problems, each with a decode of its own: 64 tokens with even choices 136 -> 131, with a few
 // popular experts 95 -> 126.
 int moe_small_rows(int T) { return T <= knobs().moe_few_tokens ? 16 : kGemmRows; }
-int moe_big_min(size_t rows, int small_rows)
+int moe_big_min(int T, size_t rows)
 {
-    if (small_rows != kGemmRows) return 0;
+    if (T < kBigMinTokens) return 0;
     const int v = knobs().moe_big_min;
     return v > 0 && v <= kGemmBigRows && rows >= (size_t)kBigMinRows ? v : 0;
 }
@@ -901,7 +905,7 @@ PermuteScratch permute_scratch_layout(int T, int k, int E)
     s.vprob = at; at = align_up(at + small * sizeof(GroupProblem));
     s.mprob = at;
     s.small_rows = moe_small_rows(T);
-    s.big_min = moe_big_min(P, s.small_rows);
+    s.big_min = moe_big_min(T, P);
     problem_capacity(P, (size_t)E, s.big_min, s.small_rows, s.max_m, s.max_b);
     at = align_up(at + (size_t)std::max(s.max_m, 1) * sizeof(GroupProblem));
     s.bprob = at;
@@ -945,7 +949,7 @@ MoeLayout moe_layout(int T, int H, int E, int k, int I, int shared_I)
     L.max_v = use_valu ? (int)(std::min<size_t>((size_t)E, P) + (fold ? 1 : 0)) : 0;
     const size_t E1 = (size_t)E + (fold ? 1 : 0);
     L.small_rows = moe_small_rows(T);
-    L.big_min = use_valu ? 0 : moe_big_min(R, L.small_rows);
+    L.big_min = use_valu ? 0 : moe_big_min(T, R);
     if (!use_valu) problem_capacity(R, E1, L.big_min, L.small_rows, L.max_m, L.max_b);
     size_t at = 0;
     auto take = [&](size_t bytes) { size_t r = at; at = align_up(at + bytes); return r; };
@@ -1013,7 +1017,8 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
     const int groups = (T + kRouteTT - 1) / kRouteTT;
     // (from two tokens on: 2 .. 31 tokens took moe_route_kernel, whose sums cross memory and a counter before a
     // token can be finished: 16 us, 13 here; a whole layer of 512 experts at 2 / 16 tokens 66 / 126 -> 58 / 118)
-    if (T > 1 && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && knobs().moe_route_slab) {
+    if (T > 1 && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && ((uintptr_t)x | (uintptr_t)wr) % 4 == 0 &&
+        knobs().moe_route_slab) {
         // One launch.  Tokens per workgroup: one workgroup of sixteen waves runs per compute unit, and its
         // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 13, 20 and
         // 30 us), so the count with the fewest whole rounds of the chip wins.  1500 tokens x 128 experts:
