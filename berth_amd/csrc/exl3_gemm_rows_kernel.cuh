@@ -32,6 +32,7 @@
 //     device, so the deal is worked out there.  A workgroup looks its few blocks up once, into LDS.
 //     A operands come straight from the row-major rotated rows: a problem has few of them, and the
 //     lanes past the last repeat it, so that a load touches as many lines as there are rows.
+//     Gate and up, 2048 x 768 at 4 bits, 2 / 8 / 16 tokens that choose 8 of 128 experts: 15 / 30 / 45 us.
 //
 // Measured (27B layer, traced): gate + up at 5 rows and 3 bits 62.6 -> 32.5 us against the VALU
 // kernel, at 24 rows and 4 bits 49.0 -> 40.6 against 32-row tiles (whose 544 workgroups also
