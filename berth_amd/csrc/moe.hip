@@ -494,7 +494,8 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
             if (lane + 64 * i < p.E) lg[i] = s_parts[wave * kSlabExperts + lane + 64 * i];
-        route_topk_n<2>(lg, lane, p, t0 + wave);
+        const int sel = route_topk_n<2>(lg, lane, p, t0 + wave);
+        if (p.sort.perm) route_sort_one_token(p.sort, lane, sel);       // (one token: one wave gets here)
         return;
     }
     // ---- several slabs: logits to memory ([T][E], the head of the segment-sum scratch), the last
@@ -521,7 +522,8 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
         const int e = lane + 64 * i;
         if (e < p.E) lg[i] = __hip_atomic_load(all + (size_t)t * p.E + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    route_topk(lg, lane, p, t);
+    const int sel = route_topk(lg, lane, p, t);
+    if (p.sort.perm) route_sort_one_token(p.sort, lane, sel);
 }
 
 // ---------------------------------------------------------------- permute
@@ -1015,9 +1017,9 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
     p.nseg = (H + kRouteSeg - 1) / kRouteSeg;
     if (sort && T == 1) p.sort = *sort;
     const int groups = (T + kRouteTT - 1) / kRouteTT;
-    // (from two tokens on: 2 .. 31 tokens took moe_route_kernel, whose sums cross memory and a counter before a
+    // (one token only where its own kernels do not apply; 2 .. 31 tokens took moe_route_kernel, whose sums cross memory and a counter before a
     // token can be finished: 16 us, 13 here; a whole layer of 512 experts at 2 / 16 tokens 66 / 126 -> 58 / 118)
-    if (T > 1 && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && ((uintptr_t)x | (uintptr_t)wr) % 4 == 0 &&
+    if ((T > 1 || E > kRouteOneMaxE) && E % 2 == 0 && H % kRouteSeg == 0 && p.nseg <= 128 && ((uintptr_t)x | (uintptr_t)wr) % 4 == 0 &&
         knobs().moe_route_slab) {
         // One launch.  Tokens per workgroup: one workgroup of sixteen waves runs per compute unit, and its
         // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 13, 20 and
@@ -1051,7 +1053,7 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
             }
             hip_ok(hipGetLastError(), "moe_route_slab_kernel launch");
             return "moe_route_slab_kernel<" + std::to_string(tt) + "> grid=" + std::to_string(nslab) + "x" +
-                   std::to_string(tgroups);
+                   std::to_string(tgroups) + (p.sort.perm ? " (with the sort of the one token)" : "");
         }
     }
     if (T >= kRouteBigT) {

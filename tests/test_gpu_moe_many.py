@@ -17,7 +17,7 @@ from tests.test_gpu_moe import _check_stages, _make_layer, _route
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("T,H,E,k,per_workgroup", [(256, 256, 128, 4, 1), (257, 256, 66, 4, 2), (700, 128, 128, 8, 3),
+@pytest.mark.parametrize("T,H,E,k,per_workgroup", [(256, 256, 128, 4, 1), (257, 256, 66, 4, 2), (700, 128, 128, 8, 3), (1, 2048, 512, 10, 1), (1, 64, 130, 3, 1),
                                                    (1021, 64, 60, 5, 4), (1501, 2048, 128, 8, 6), (200, 128, 1024, 10, 4)])
 def test_routing_of_many_tokens(T, H, E, k, per_workgroup):
     x, wr = synth.activations(T, T, H), synth.router_weight(E, H, E)
@@ -75,3 +75,21 @@ def test_few_token_layers_on_the_grouped_few_row_kernel(T, H, E, k, I, bits, sha
         layer.forward(gpu, d_x, again, T)
         torch.cuda.synchronize()
         assert torch.equal(again, out)
+
+
+def test_one_token_of_many_experts():
+    """More experts than the one-token kernels take: the one-launch routing sorts the choices too."""
+    gpu = Gpu(0)
+    T, H, E, k, I, bits, shared_I = 1, 256, 300, 7, 128, 4, 128
+    wr, experts_np, experts, shared_np, shared = _make_layer(gpu, 9300, H, E, I, bits, shared_I, 10.0)
+    layer = MoeLayer(gpu, wr, experts, k, shared=shared)
+    x = (synth.activations(9301, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
+    out = torch.zeros((T, H), dtype=torch.float32, device=DEV)
+    idx = torch.zeros((T, k), dtype=torch.int32, device=DEV)
+    w = torch.zeros((T, k), dtype=torch.float32, device=DEV)
+    layer.forward(gpu, dev(x.view(np.uint16)), out, T, idx, w)
+    torch.cuda.synchronize()
+    assert "moe_route_slab_kernel<1>" in K.moe.last_launch() and "sort" in K.moe.last_launch(), K.moe.last_launch()
+    want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, 2, shared=shared_np, shared_I=shared_I)
+    assert np.array_equal(idx.cpu().numpy(), oi)
+    _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I)
