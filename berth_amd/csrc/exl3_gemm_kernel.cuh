@@ -406,7 +406,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                         else if (hs < 7) a_op = a_operand(hs + 1, 0);
                         acc[mb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_now, b0, acc[mb][0], 0, 0, 0);
                         acc[mb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_now, b1, acc[mb][1], 0, 0, 0);
-                        decode_pairs(win, h ^ 1, mb * (8 / MB), 8 / MB, b_nx);
+                        decode_pairs(win, h ^ 1, mb * 8 / MB, (mb + 1) * 8 / MB - mb * 8 / MB, b_nx);
                     }
                     // the step's dwords are decoded once its odd pairs exist: request the next k-block's
                     if (h == 0) load_b_step(nkb, st);
@@ -416,8 +416,15 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         __builtin_amdgcn_sched_group_barrier(0x002, valu0, 0);                          \
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                              \
         __builtin_amdgcn_sched_group_barrier(0x002, valu1, 0);
-                    static_assert(MB == 4, "the groups below describe eight MFMAs per half-step");
-                    BERTH_GEMM_CHUNK(9, 9) BERTH_GEMM_CHUNK(9, 9) BERTH_GEMM_CHUNK(9, 9) BERTH_GEMM_CHUNK(9, 9)
+                    // (the decode of a half-step spread over its 2 * MB MFMAs)
+                    static_assert(MB >= 2 && MB <= 4, "the groups below describe four to eight MFMAs per half-step");
+                    if constexpr (MB == 4) {
+                        BERTH_GEMM_CHUNK(9, 9) BERTH_GEMM_CHUNK(9, 9) BERTH_GEMM_CHUNK(9, 9) BERTH_GEMM_CHUNK(9, 9)
+                    } else if constexpr (MB == 3) {
+                        BERTH_GEMM_CHUNK(12, 12) BERTH_GEMM_CHUNK(12, 12) BERTH_GEMM_CHUNK(12, 12)
+                    } else {
+                        BERTH_GEMM_CHUNK(18, 18) BERTH_GEMM_CHUNK(18, 18)
+                    }
     #undef BERTH_GEMM_CHUNK
                 }
             }
@@ -479,7 +486,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
             // part 0 first (from memory unless it is this workgroup's own), then parts 1, 2, ...
             // added in order.  64 (128-row tiles) or 128 (32-row tiles) loads a lane are in
             // flight at a time: half of a part's register blocks, or four whole parts.
-            constexpr int kGroup = MB == 1 ? 2 : 4;             // (mb, f) register blocks per batch
+            constexpr int kGroup = MB & 1 ? 2 : 4;              // (mb, f) register blocks per batch
             constexpr int kParts = MB == 1 ? 4 : 1;             // parts per batch
             const int first = kr.part == 0 ? 1 : 0;
             for (int j0 = first; j0 < kr.parts; j0 += kParts) {
@@ -620,6 +627,9 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_kernel(GemmParams p)
 // rows.  Both kinds sit in one launch, the long tiles first, so the short ones fill in around
 // them (as two launches the 128-row tiles would run alone on a fraction of the compute units).
 // blockIdx.x = column block (whole K per workgroup: no hand-over), blockIdx.y the linear.
+// A problem of up to 64 or 96 rows runs as two or three 32-row blocks (the loop multiplies all the blocks
+// it has, needed or not): gate + up and down of 800 tokens that choose 8 of 128 experts 137 + 82 -> 119 +
+// 70 us, of 1500 tokens (94 rows an expert) 133 + 89 -> 131 + 85.
 // Measured and dropped: cutting K in two with the split-K hand-over, for every tile or for the
 // 128-row tiles only (the shorter units pack better, the hand-over of 128 KB of partial sums per
 // tile costs far more than that gains: 150 -> 183 us per layer), 128-column units whose four waves
@@ -643,7 +653,10 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
     const int z = blockIdx.z;
     if (z < p.max_big) {
         if (z >= *p.num_big) return;
-        gemm_tile<BITS, CB, 4, false>(p, z, blockIdx.x, kr, blockIdx.y, smem, p.big_problems);
+        const int rows = p.big_problems[z].nrows;               // as many 32-row blocks as the problem has
+        if (rows > 96) gemm_tile<BITS, CB, 4, false>(p, z, blockIdx.x, kr, blockIdx.y, smem, p.big_problems);
+        else if (rows > 64) gemm_tile<BITS, CB, 3, false>(p, z, blockIdx.x, kr, blockIdx.y, smem, p.big_problems);
+        else gemm_tile<BITS, CB, 2, false>(p, z, blockIdx.x, kr, blockIdx.y, smem, p.big_problems);
         return;
     }
     if (z - p.max_big >= *p.num_problems) return;

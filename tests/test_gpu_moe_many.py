@@ -11,7 +11,7 @@ from berth_amd import synth
 from berth_amd.device import Gpu
 from berth_amd.moe import MoeLayer
 from oracle import oracle as O
-from tests.gpu_util import DEV, dev
+from tests.gpu_util import DEV, dev, knobs
 from tests.test_gpu_moe import _check_stages, _make_layer, _route
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +93,23 @@ def test_one_token_of_many_experts():
     want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, 2, shared=shared_np, shared_I=shared_I)
     assert np.array_equal(idx.cpu().numpy(), oi)
     _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I)
+
+
+@pytest.mark.parametrize("T,bits", [(150, 4), (150, 3), (240, 4), (240, 6), (330, 4), (330, 2)])
+def test_problems_of_two_three_and_four_row_blocks(T, bits):
+    """About 50, 80 and 110 rows an expert: the 128-row problems run as many 32-row blocks as they
+    have rows for, with the bits of 32-row problems."""
+    gpu = Gpu(0)
+    H, E, k, I = 256, 6, 2, 384
+    wr, _, experts, _, _ = _make_layer(gpu, 9400 + T + bits, H, E, I, bits, 0, 1.0)
+    x = (synth.activations(9401 + T, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
+    d_x, res = dev(x.view(np.uint16)), []
+    for big_min in (0, 33):
+        with knobs(BERTH_MOE_BIG_MIN=big_min):
+            layer = MoeLayer(gpu, wr, experts, k)
+            out = torch.zeros((T, H), dtype=torch.float32, device=DEV)
+            layer.forward(gpu, d_x, out, T)
+            torch.cuda.synchronize()
+            assert ("exl3_gemm_mixed_kernel" in K.moe.last_launch()) == (big_min > 0), K.moe.last_launch()
+            res.append(out)
+    assert torch.equal(res[0], res[1])
