@@ -44,11 +44,14 @@ __host__ __device__ constexpr size_t block_lds_bytes(int mt)
     return (size_t)mt * (8192 + 16 * kRowsStride * 4) + 256;
 }
 
-// sixteen bytes a lane from base + offset to LDS at lds_at + 16 * lane
+// Sixteen bytes a lane from base + offset to LDS at lds_at + 16 * lane (m0: an operand, so that the
+// compiler sets it and knows; the s_nop is the wait state between that and the load).  The compiler
+// sees neither a load here nor what it writes: whoever reads or overwrites the bytes waits first.
+// (__builtin_amdgcn_global_load_lds from an LDS offset gets no waits either, and takes its address in
+// a pair of vector registers instead of the scalar base.)
 __device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, uint32_t lds_at)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 : : "s"(lds_at), "v"(offset), "s"(base) : "m0", "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(lds_at), "v"(offset), "s"(base) : "memory");
 }
 
 // The end of one output row of a 128-column block, sixteen lanes with eight sums each: Hadamard, svh,
@@ -229,6 +232,10 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
             stage(1, s + 1, s1 - 1);
         }
         if (s < s1) stage(0, s, s1 - 1);
+        // The last step's A loads bring nothing that is used, but they land in the buffers that the register
+        // dumps lie over, some of them in another wave's dump: every wave has its own behind it before
+        // the first barrier of the finish.  Ahead of the next tile's trellis loads, which go on.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (kg < 2) asm volatile("s_barrier" ::: "memory");
         if (tile < t_last) {                            // the next tile's first steps, behind the finish of this one
             seek(tile + 1);

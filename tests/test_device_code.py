@@ -1,0 +1,135 @@
+"""What the compiler cannot see around inline assembly, checked in the gfx950 assembly of the kernels themselves.
+
+Loads that write LDS directly are issued as inline assembly, so the compiler inserts no wait for them: a
+kernel has to wait itself before anything else uses the bytes they land in.  The kernels are compiled
+here (no GPU), and every path through their control flow is followed.
+"""
+import re
+import subprocess
+
+import pytest
+
+from berth_amd import build as B
+
+# the row-block kernel at every height and over the bit rates' load shapes
+BLOCK_KERNELS = [f"exl3_gemm_block_kernel<{bits}, {cb}, {mt}>" for bits, cb, mt in
+                 ((4, 2, 4), (4, 2, 6), (4, 2, 8), (1, 2, 4), (3, 1, 8), (8, 0, 6))]
+
+
+def _operands(text):
+    """Registers of one operand list, operand by operand: [('v', 3), ...] each."""
+    out = []
+    for op in re.split(r",(?![^\[]*\])", text):
+        m = re.match(r"\s*[-|]*([vas])\[(\d+):(\d+)\]", op) or re.match(r"\s*[-|]*([vas])(\d+)\b", op)
+        out.append([] if not m else [(m[1], i) for i in range(int(m[2]), int(m[m.lastindex]) + 1)])
+    return out
+
+
+class Function:
+    """Instructions of one kernel as (opcode, operand text, inside inline assembly), with successors."""
+
+    def __init__(self, name, lines):
+        self.name, self.code, labels = name, [], {}
+        in_asm = False
+        for line in lines:
+            if "#ASMSTART" in line or "#ASMEND" in line:
+                in_asm = "#ASMSTART" in line
+            text = line.split(";")[0].strip()
+            if m := re.match(r"(\.LBB\w+):", text):
+                labels[m[1]] = len(self.code)
+            elif text and not text.startswith(".") and not text.endswith(":"):
+                op, _, rest = text.partition(" ")
+                self.code.append((op, rest.strip(), in_asm))
+        self.next = []
+        for i, (op, rest, _) in enumerate(self.code):
+            after = [] if op in ("s_endpgm", "s_branch") else [i + 1]
+            if op == "s_branch" or op.startswith("s_cbranch"):
+                after.append(labels[rest])
+            assert op not in ("s_setpc_b64", "s_swappc_b64"), "an indirect branch cannot be followed"
+            self.next.append(after)
+
+    def states(self, entry, step, join):
+        """The state before every instruction, as the join over all paths that reach it."""
+        before = {0: entry}
+        work = [0]
+        while work:
+            i = work.pop()
+            out = step(before[i], *self.code[i])
+            for j in self.next[i]:
+                new = out if j not in before else join(before[j], out)
+                if j not in before or new != before[j]:
+                    before[j] = new
+                    work.append(j)
+        return before
+
+
+def _compile(tmp_path, kernels, headers=("exl3_gemm_block_kernel.cuh", "exl3_gemm_wide_kernel.cuh")):
+    source = tmp_path / "kernels.hip"
+    source.write_text("".join(f'#include "{h}"\n' for h in headers) + "namespace berth {\n" +
+                      "".join(f"template __global__ void {k}(GemmParams);\n" for k in kernels) + "}\n")
+    out = tmp_path / "kernels.gfx950"
+    r = subprocess.run([B.HIPCC, *B.FLAGS, "--offload-device-only", "-S", "-I" + B.CSRC, str(source), "-o", str(out)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-4000:]
+    functions, lines = [], None
+    for line in out.read_text().splitlines():
+        if m := re.match(r"(_Z\w+):", line):
+            name, lines = m[1], []
+        elif lines is not None and line.startswith(".Lfunc_end"):
+            functions.append(Function(name, lines))
+            lines = None
+        elif lines is not None:
+            lines.append(line)
+    return functions
+
+
+def _is_vector_load(op):
+    return op.startswith(("global_load", "buffer_load", "scratch_load"))
+
+
+def _lds_loads_step(younger, op, rest, in_asm):
+    """State: None when every load to LDS has landed, else the fewest vector loads issued behind the
+    youngest of them.  Loads come back in order, so vmcnt(n) covers it from n younger loads on."""
+    if "load_lds" in op:
+        return 0
+    if younger is not None and _is_vector_load(op):
+        return min(younger + 1, 64)
+    if younger is not None and op == "s_waitcnt" and (m := re.search(r"vmcnt\((\d+)\)", rest)):
+        return None if younger >= int(m[1]) else younger
+    return younger
+
+
+def _fewest(a, b):
+    return b if a is None else a if b is None else min(a, b)
+
+
+@pytest.fixture(scope="module")
+def block_kernels(tmp_path_factory):
+    found = _compile(tmp_path_factory.mktemp("block"), BLOCK_KERNELS)
+    found = [f for f in found if "exl3_gemm_block_kernel" in f.name]
+    assert len(found) == len(BLOCK_KERNELS)
+    return found
+
+
+def test_loads_to_lds_have_landed_before_their_bytes_are_used_again(block_kernels):
+    """The register dumps at the end of a tile lie over the operand buffers, some of them over what another
+    wave loaded: no load to LDS may be outstanding at a barrier of the finish (the loop's own barriers are
+    inline assembly), where LDS is written, or where the workgroup gives its LDS back."""
+    for f in block_kernels:
+        before = f.states(None, _lds_loads_step, _fewest)
+        assert any("load_lds" in op for op, _, _ in f.code), f.name
+        late = [(i, op) for i, (op, _, in_asm) in enumerate(f.code)
+                if ((op == "s_barrier" and not in_asm) or op.startswith("ds_write") or op == "s_endpgm")
+                and before.get(i) is not None]
+        assert not late, f"{f.name}: loads to LDS outstanding at {late[:4]} ({len(late)} in all)"
+
+
+def test_the_loops_wait_covers_the_loads_of_its_step(block_kernels):
+    """`s_waitcnt vmcnt(n)` + `s_barrier` in the loop: on every path the loads to LDS are older than at
+    least n other loads, so the operands that are read behind the barrier are there."""
+    for f in block_kernels:
+        before = f.states(None, _lds_loads_step, _fewest)
+        waits = [i for i, (op, rest, in_asm) in enumerate(f.code) if in_asm and op == "s_waitcnt" and "vmcnt" in rest]
+        assert waits, f.name
+        for i in waits:
+            assert _lds_loads_step(before[i], *f.code[i]) is None, (f.name, i, f.code[i])
