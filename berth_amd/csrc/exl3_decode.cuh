@@ -163,6 +163,22 @@ __device__ __forceinline__ uint32_t decode_pair(uint32_t s0, uint32_t s1)
     }
 }
 
+// MFMA operands that decode_pair has just written.  A matrix instruction may read a vector register
+// two wait states after a vector instruction wrote it at the earliest; the compiler keeps that
+// distance behind its own instructions, but of the inline assembly of inst3_pair it knows only the
+// registers (it left one wait state in the 128-row tiles with the MCG codebook).  Between the last
+// pair and the first MFMA; no code for the codebook whose decode is the compiler's own.
+template <int CB>
+__device__ __forceinline__ void settle(half8_t& b0, half8_t& b1)
+{
+    if constexpr (CB != 2) asm("s_nop 1" : "+v"(b0), "+v"(b1));
+}
+template <int CB>
+__device__ __forceinline__ void settle(half8_t& b0, half8_t& b1, half8_t& b2, half8_t& b3)
+{
+    if constexpr (CB != 2) asm("s_nop 1" : "+v"(b0), "+v"(b1), "+v"(b2), "+v"(b3));
+}
+
 // ---- window extraction
 // `own` are the lane's BITS dwords as loaded (little-endian pairs of u16 words),
 // `prev` is the dword just before them in the tile (the last dword of the previous

@@ -164,6 +164,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(w2[i]));       // decoded here, not behind the barrier
+        // (the wait and the barrier are also the two wait states that `settle` puts before an MFMA)
         // this step's A loads of this wave are older than the next step's trellis loads (one or
         // more), so they have landed when at most one load is outstanding; behind the barrier the
         // other three waves' have, too, and everybody has left the other buffer

@@ -290,6 +290,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                             const uint4 q = {w2[2 * f + h], w2[4 + 2 * f + h], w2[8 + 2 * f + h], w2[12 + 2 * f + h]};
                             b[f][h] = __builtin_bit_cast(half8_t, q);
                         }
+                    settle<CB>(b[0][0], b[1][0], b[0][1], b[1][1]);
                     const half8_t a0 = av[st][0], a1 = av[st][1];
                     av[st][0] = anx[4 * st];
                     av[st][1] = anx[4 * st + 1];
@@ -392,8 +393,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                     __builtin_amdgcn_sched_barrier(0);
                     uint32_t (&b_cur)[2][4] = b_half[h];
                     uint32_t (&b_nx)[2][4] = b_half[h ^ 1];
-                    const half8_t b0 = __builtin_bit_cast(half8_t, uint4{b_cur[0][0], b_cur[0][1], b_cur[0][2], b_cur[0][3]});
-                    const half8_t b1 = __builtin_bit_cast(half8_t, uint4{b_cur[1][0], b_cur[1][1], b_cur[1][2], b_cur[1][3]});
+                    half8_t b0 = __builtin_bit_cast(half8_t, uint4{b_cur[0][0], b_cur[0][1], b_cur[0][2], b_cur[0][3]});
+                    half8_t b1 = __builtin_bit_cast(half8_t, uint4{b_cur[1][0], b_cur[1][1], b_cur[1][2], b_cur[1][3]});
+                    settle<CB>(b0, b1);
                     if (h == 1) {
                         // the step after this one: its windows, then (below) its even pairs
                         const int ns = (st + 1) & 3;

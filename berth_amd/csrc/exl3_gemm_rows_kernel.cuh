@@ -300,16 +300,22 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
         decode_lane<BITS, CB>(own[j], prev, w2);
         __builtin_amdgcn_sched_barrier(0);
         fetch_t(j);
+        half8_t b[2][2];                                // [k half][column half]
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
                 const uint4 bq = {w2[2 * f + h], w2[4 + 2 * f + h], w2[8 + 2 * f + h], w2[12 + 2 * f + h]};
-                const half8_t b = __builtin_bit_cast(half8_t, bq);
+                b[h][f] = __builtin_bit_cast(half8_t, bq);
+            }
+        settle<CB>(b[0][0], b[0][1], b[1][0], b[1][1]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[mt][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[j][mt][h], b, acc[mt][f], 0, 0, 0);
-            }
+                    acc[mt][f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[j][mt][h], b[h][f], acc[mt][f], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         fetch_a(j);
         advance();

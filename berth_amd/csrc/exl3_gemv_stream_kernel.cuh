@@ -588,13 +588,18 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
             reload();
         }
         __builtin_amdgcn_sched_barrier(0);
+        half8_t b[2][2];                                    // [k half][column half]
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            b[h][0] = __builtin_bit_cast(half8_t, uint4{w2[h], w2[4 + h], w2[8 + h], w2[12 + h]});
+            b[h][1] = __builtin_bit_cast(half8_t, uint4{w2[2 + h], w2[6 + h], w2[10 + h], w2[14 + h]});
+        }
+        settle<CB>(b[0][0], b[0][1], b[1][0], b[1][1]);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const half8_t x = h ? xb : xa;
-            const uint4 b0 = {w2[h], w2[4 + h], w2[8 + h], w2[12 + h]};
-            const uint4 b1 = {w2[2 + h], w2[6 + h], w2[10 + h], w2[14 + h]};
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8_t, b0), acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, __builtin_bit_cast(half8_t, b1), acc1, 0, 0, 0);
+            acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[h][0], acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[h][1], acc1, 0, 0, 0);
         }
         ++r;
         xoff += 128;

@@ -1,8 +1,9 @@
 """What the compiler cannot see around inline assembly, checked in the gfx950 assembly of the kernels themselves.
 
 Loads that write LDS directly are issued as inline assembly, so the compiler inserts no wait for them: a
-kernel has to wait itself before anything else uses the bytes they land in.  The kernels are compiled
-here (no GPU), and every path through their control flow is followed.
+kernel has to wait itself before anything else uses the bytes they land in.  The decode of two codebooks
+is inline assembly, so the compiler does not keep a matrix instruction away from its results.  The kernels
+are compiled here (no GPU), and every path through their control flow is followed.
 """
 import re
 import subprocess
@@ -14,6 +15,14 @@ from berth_amd import build as B
 # the row-block kernel at every height and over the bit rates' load shapes
 BLOCK_KERNELS = [f"exl3_gemm_block_kernel<{bits}, {cb}, {mt}>" for bits, cb, mt in
                  ((4, 2, 4), (4, 2, 6), (4, 2, 8), (1, 2, 4), (3, 1, 8), (8, 0, 6))]
+
+# every loop that multiplies freshly decoded weights, with the codebooks whose decode is inline assembly
+DECODING_KERNELS = (["exl3_gemm_kernel<3, 1, 4>", "exl3_gemm_balanced_kernel<3, 1, 4>", "exl3_gemm_kernel<4, 0, 1>",
+                     "exl3_gemm_wide_kernel<4, 1>"] +
+                    [f"exl3_gemm_mixed_kernel<{bits}, {cb}>" for bits, cb in ((1, 1), (2, 1), (3, 1), (4, 0))] +
+                    [f"exl3_gemm_rows_kernel<3, 1, {mt}, {grouped}>" for mt, grouped in ((1, "false"), (2, "false"), (1, "true"))] +
+                    ["exl3_gemm_block_kernel<3, 1, 4>", "exl3_gemm_block_kernel<5, 0, 8>"])
+STREAM_KERNELS = ["exl3_gemv_stream_kernel<4, 1, kInPlain, 0>", "exl3_gemv_stream_kernel<5, 0, kInPlain, 0>"]
 
 
 def _operands(text):
@@ -63,10 +72,10 @@ class Function:
         return before
 
 
-def _compile(tmp_path, kernels, headers=("exl3_gemm_block_kernel.cuh", "exl3_gemm_wide_kernel.cuh")):
+def _compile(tmp_path, kernels, headers, params="GemmParams"):
     source = tmp_path / "kernels.hip"
     source.write_text("".join(f'#include "{h}"\n' for h in headers) + "namespace berth {\n" +
-                      "".join(f"template __global__ void {k}(GemmParams);\n" for k in kernels) + "}\n")
+                      "".join(f"template __global__ void {k}({params});\n" for k in sorted(set(kernels))) + "}\n")
     out = tmp_path / "kernels.gfx950"
     r = subprocess.run([B.HIPCC, *B.FLAGS, "--offload-device-only", "-S", "-I" + B.CSRC, str(source), "-o", str(out)],
                        capture_output=True, text=True)
@@ -105,7 +114,7 @@ def _fewest(a, b):
 
 @pytest.fixture(scope="module")
 def block_kernels(tmp_path_factory):
-    found = _compile(tmp_path_factory.mktemp("block"), BLOCK_KERNELS)
+    found = _compile(tmp_path_factory.mktemp("block"), BLOCK_KERNELS, ["exl3_gemm_block_kernel.cuh"])
     found = [f for f in found if "exl3_gemm_block_kernel" in f.name]
     assert len(found) == len(BLOCK_KERNELS)
     return found
@@ -133,3 +142,42 @@ def test_the_loops_wait_covers_the_loads_of_its_step(block_kernels):
         assert waits, f.name
         for i in waits:
             assert _lds_loads_step(before[i], *f.code[i]) is None, (f.name, i, f.code[i])
+
+
+VALU_TO_MFMA = 2        # wait states; what the compiler leaves between its own instructions
+
+
+def _asm_results_step(ages, op, rest, in_asm):
+    """State: wait states since inline assembly wrote a vector register, while fewer than VALU_TO_MFMA."""
+    passed = int(rest, 0) + 1 if op == "s_nop" else 1
+    ages = {reg: age + passed for reg, age in ages if age + passed < VALU_TO_MFMA}
+    if op.startswith(("v_", "ds_read", "global_load", "buffer_load", "scratch_load")):
+        for reg in _operands(rest)[0]:
+            ages.pop(reg, None)
+            if in_asm and op.startswith("v_"):
+                ages[reg] = 0
+    return frozenset(ages.items())
+
+
+def _youngest(a, b):
+    joined = dict(a)
+    for reg, age in b:
+        joined[reg] = min(age, joined.get(reg, age))
+    return frozenset(joined.items())
+
+
+@pytest.mark.parametrize("kernels,headers,params", [
+    (DECODING_KERNELS, ("exl3_gemm_block_kernel.cuh", "exl3_gemm_wide_kernel.cuh"), "GemmParams"),
+    (STREAM_KERNELS, ("exl3_gemv_stream_kernel.cuh",), "StreamParams")])
+def test_matrix_instructions_keep_their_distance_from_inline_assembly(tmp_path, kernels, headers, params):
+    functions = [f for f in _compile(tmp_path, kernels, headers, params) if "finish_kernel" not in f.name]
+    assert len(functions) == len(set(kernels))
+    for f in functions:
+        before = f.states(frozenset(), _asm_results_step, _youngest)
+        assert any(op.startswith("v_mfma") for op, _, _ in f.code), f.name
+        assert any(a and op.startswith("v_") for op, _, a in f.code), f"{f.name}: no inline assembly left to check"
+        for i, (op, rest, _) in enumerate(f.code):
+            if op.startswith("v_mfma") and i in before:
+                fresh = dict(before[i])
+                close = [reg for operand in _operands(rest)[1:4] for reg in operand if reg in fresh]
+                assert not close, f"{f.name}: {op} {rest} reads {close} too soon"
