@@ -169,9 +169,14 @@ __device__ __forceinline__ uint32_t decode_pair(uint32_t s0, uint32_t s1)
 // registers (it left one wait state in the 128-row tiles with the MCG codebook).  Between the last
 // pair and the first MFMA; no code for the codebook whose decode is the compiler's own.
 template <int CB>
-__device__ __forceinline__ void settle(half8_t& b0, half8_t& b1)
+__device__ __forceinline__ void settle(half8_t& b)
 {
-    if constexpr (CB != 2) asm("s_nop 1" : "+v"(b0), "+v"(b1));
+    if constexpr (CB != 2) asm("s_nop 1" : "+v"(b));
+}
+template <int CB>
+__device__ __forceinline__ void settle(uint32_t (&w)[4])
+{
+    if constexpr (CB != 2) asm("s_nop 1" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
 }
 template <int CB>
 __device__ __forceinline__ void settle(half8_t& b0, half8_t& b1, half8_t& b2, half8_t& b3)

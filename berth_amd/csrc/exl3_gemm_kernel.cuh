@@ -362,6 +362,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                 for (int st = 0; st < 4; ++st) load_b_step(kr.kb0, st);
                 win = LaneWindows<BITS>(ring[0], fetch_prev(lane, ring[0][BITS - 1]));
                 decode_pairs(win, 0, 0, 8, b_half[0]);
+                settle<CB>(b_half[0][0]);
             }
         }
 
@@ -395,7 +396,6 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                     uint32_t (&b_nx)[2][4] = b_half[h ^ 1];
                     half8_t b0 = __builtin_bit_cast(half8_t, uint4{b_cur[0][0], b_cur[0][1], b_cur[0][2], b_cur[0][3]});
                     half8_t b1 = __builtin_bit_cast(half8_t, uint4{b_cur[1][0], b_cur[1][1], b_cur[1][2], b_cur[1][3]});
-                    settle<CB>(b0, b1);
                     if (h == 1) {
                         // the step after this one: its windows, then (below) its even pairs
                         const int ns = (st + 1) & 3;
@@ -407,8 +407,10 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                         if (mb + 1 < MB) a_op = a_operand(hs, mb + 1);
                         else if (hs < 7) a_op = a_operand(hs + 1, 0);
                         acc[mb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_now, b0, acc[mb][0], 0, 0, 0);
+                        if (mb == 0) settle<CB>(b1);
                         acc[mb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_now, b1, acc[mb][1], 0, 0, 0);
                         decode_pairs(win, h ^ 1, mb * 8 / MB, (mb + 1) * 8 / MB - mb * 8 / MB, b_nx);
+                        if ((mb + 1) * 8 / MB >= 4 && mb * 8 / MB < 4) settle<CB>(b_nx[0]);
                     }
                     // the step's dwords are decoded once its odd pairs exist: request the next k-block's
                     if (h == 0) load_b_step(nkb, st);
