@@ -277,6 +277,41 @@ struct OperandPlan {
     size_t stride = 0;          // elements between slabs
 };
 
+// How a dense launch of 128-row tiles or larger is cut up.  Whole tiles: a workgroup of four waves per
+// 128 x 256 tile, two of them on a compute unit.  Dealt out: one workgroup per compute unit with an even
+// share of the (tile, k-block) units, the workgroups of a shared tile adding their parts in k order;
+// of 128-row tiles, or of 256-row tiles (eight waves, every weight decoded once per 256 rows).
+enum class DenseTiles { kWhole128, kDealt128, kDealt256 };
+
+// The cheapest by what a compute unit spends, in 10 ns: k-blocks, the epilogue of every tile, and the
+// hand-over of shared ones, which takes longer the more workgroups share a tile.
+//   * Whole tiles hide part of an epilogue behind the other workgroup's k-loop, but come in rounds; a
+//     round with r of its tiles takes about (1 + r) / 2 of a full one, the first a whole one.
+//   * Dealt-out tiles have no partial round; their epilogue and hand-over are in nobody's shadow.  So a
+//     short K, where those weigh against few k-blocks, takes whole tiles, and a long one is dealt out.
+//   * The decode of 128-row tiles does not quite fit behind their MFMAs, so a k-block costs more with the
+//     codebooks of longer decode; with 256-row tiles it does fit (6144 columns of 4096 at 1500 rows, dealt 128 /
+//     dealt 256 us: MUL1 108/105, MCG 112/103, 3INST 123/105; the bit rate matters less).
+// Fitted to 499 launches at 4 bits (K 128 .. 10240, 2048 .. 32768 columns, 460 .. 1500 rows): the choice costs
+// 0.7 % over the fastest of the three on average, 14 % at most.  Examples, K x N at rows: whole / dealt
+// 128 / dealt 256 us: 256x8192 at 512 16/26/31, 512x16384 at 1500 46/59/59, 1024x4096 at 512 27/31/50,
+// 1024x16384 at 1500 72/88/81, 2048x4096 at 512 43/36/54, 2048x16384 at 1024 87/96/83, 5120x12288 at 600
+// 99/106/121, 4096x16384 at 600 128/111/122 and at 1500 231/254/225.
+static DenseTiles cheapest_tiles(long cus, int codebook, long KB, long tiles128, long tiles256, bool whole_allowed, bool wide_allowed)
+{
+    const long whole_kb = codebook == 0 ? 250 : codebook == 1 ? 236 : 230;
+    const long dealt_kb = codebook == 0 ? 260 : codebook == 1 ? 243 : 235;
+    const long n = tiles128 / cus, r = tiles128 % cus;          // full rounds, tiles of the last one
+    const long m = tiles256 / cus, s = tiles256 % cus;
+    // (one workgroup on a compute unit has no other to hide its epilogue behind)
+    const long whole = n == 0 || tiles128 == cus ? KB * whole_kb + 500 + 400 * tiles128 / cus
+                                                 : (2 * n * cus + (r ? cus + r : 0)) * (KB * whole_kb + 500) / (2 * cus);
+    const long dealt128 = tiles128 * KB * dealt_kb / cus + 800 * n + (r == 0 ? 0 : n ? 800 : 2500 - 1600 * r / cus);
+    const long dealt256 = tiles256 * KB * 415 / cus + 900 * m + (s == 0 ? 0 : m ? 1900 : 3700 - 2200 * s / cus);
+    if (whole_allowed && whole < dealt128 && (!wide_allowed || whole <= dealt256)) return DenseTiles::kWhole128;
+    return wide_allowed && dealt256 < dealt128 ? DenseTiles::kDealt256 : DenseTiles::kDealt128;
+}
+
 // Tile shape and work split of a dense launch: `nblocks` column blocks of 256 (all slices of
 // a bundle together), size_m rows.  Fills the split fields of p and launches.
 static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int codebook, int size_m, int size_k,
@@ -288,16 +323,13 @@ static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int c
     const int mb_plain = (size_m <= 32 || !fills_128_row_tiles(ws, nblocks, size_m)) ? 1 : 4;
     const int KB = size_k / 128;
     p.tile0 = 0;
+    // 0: whole tiles, K split by gemm_split; 1 (default): by cost; more: dealt out to this many workgroups
     const int balance = knobs().gemm_balanced;
     // 0: never 256-row tiles; 1 (default): where they are faster; 2: wherever they are possible
     const int rows256 = knobs().gemm_rows256;
-    // 128-row tiles rarely divide over the compute units (272 tiles on 256 units leave most of
-    // the chip idle for the second half of the launch): deal the (tile, k-block) units out evenly.
-    // 128-row tiles: one workgroup per compute unit (a wave interleaves its own decode with its
-    // MFMAs, so a second workgroup per unit adds nothing and more workgroups share a tile: the 27B
-    // down projection at 512 rows takes 147 us with 256 workgroups, 160 with 512).  256-row tiles
-    // (more than 128 rows, wide outputs): a weight is decoded once per 256 rows; one workgroup of
-    // eight waves fills a compute unit.
+    // over more workgroups than compute units the dealt-out 128-row tiles lose (the 27B down projection at
+    // 512 rows takes 147 us with 256 workgroups, 160 with 512): a wave interleaves its own decode with
+    // its MFMAs, and more workgroups share a tile
     auto balanced = [&](int mb) {
         const int mtiles = (size_m + mb * 32 - 1) / (mb * 32);
         const long tiles = (long)nblocks * mtiles;
@@ -314,33 +346,24 @@ static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int c
         p.unit_q = (int)(units / G);
         p.unit_r = (int)(units % G);
         gemm_bits(p, k_bits, codebook, mb, stream, desc, dim3((unsigned)G, 1, 1));
+        hip_ok(hipGetLastError(), "exl3_gemm_kernel launch");
         return true;
     };
-    bool done = false;
-    const long tiles128 = (long)nblocks * ((size_m + 127) / 128);
-    // (K = 1024 leaves the balanced kernels' single workgroup per compute unit in its epilogue for too
-    // long: 16384 columns at 600 / 768 / 1500 rows 42 / 46 / 70 us as whole tiles, 45 / 51 / 81 dealt out)
-    if (balance && mb_plain == 4 && (KB != 8 || rows256 >= 2 || tiles128 <= ws.cu_count)) {
-        // 256-row or 128-row tiles: a workgroup's k-block of the one takes 4.56 us, of the other 2.55
-        // (rows past the end cost as much as others), and the hand-over and finish of the larger tiles
-        // takes longer by 15 us where every tile is shared, 6 where some are, 3 of epilogue otherwise.
-        // Measured (128-row / 256-row, us): 17408x5120 at 512, 768, 1500 rows 128/135, 178/170, 337/306;
-        // 2048x8192 at 1024 rows 50/65, at 1500 77/74; 4096x17408 at 512, 600, 1500 rows 100/97, 122/131,
-        // 284/240.  A K below 1024 keeps the larger tiles wherever there are enough to go round.
-        const long tiles256 = (long)nblocks * ((size_m + 255) / 256);
-        const long more = tiles256 >= ws.cu_count ? 300 : tiles256 * 2 > ws.cu_count ? 600 : 1500;
-        const bool wide = KB < 8 ? tiles256 * 2 >= ws.cu_count : (255 * tiles128 - 456 * tiles256) * KB > more * ws.cu_count;
-        if (size_m > 128 && (rows256 >= 2 || (rows256 == 1 && wide))) done = balanced(8);
-        if (!done) done = balanced(4);
+    bool whole = false;
+    if (mb_plain == 4 && balance) {
+        const long tiles128 = (long)nblocks * ((size_m + 127) / 128), tiles256 = (long)nblocks * ((size_m + 255) / 256);
+        const DenseTiles cheapest = cheapest_tiles(ws.cu_count, codebook, KB, tiles128, tiles256, balance == 1, rows256 > 0 && size_m > 128);
+        const bool wide = size_m > 128 && (rows256 >= 2 || cheapest == DenseTiles::kDealt256);
+        if (wide && balanced(8)) return;
+        whole = cheapest == DenseTiles::kWhole128;
+        if (!whole && balanced(4)) return;
     }
-    if (!done) {
-        const int mtiles = (size_m + mb_plain * 32 - 1) / (mb_plain * 32);
-        const long tiles = (long)nblocks * mtiles;
-        p.tiles_y = mtiles;
-        p.units = 0;
-        p.S = gemm_split(ws, tiles, KB, mb_plain, size_m <= 32);
-        gemm_bits(p, k_bits, codebook, mb_plain, stream, desc, dim3((unsigned)(tiles * p.S), 1, 1));
-    }
+    const int mtiles = (size_m + mb_plain * 32 - 1) / (mb_plain * 32);
+    const long tiles = (long)nblocks * mtiles;
+    p.tiles_y = mtiles;
+    p.units = 0;
+    p.S = whole ? 1 : gemm_split(ws, tiles, KB, mb_plain, size_m <= 32);
+    gemm_bits(p, k_bits, codebook, mb_plain, stream, desc, dim3((unsigned)(tiles * p.S), 1, 1));
     hip_ok(hipGetLastError(), "exl3_gemm_kernel launch");
 }
 

@@ -14,7 +14,7 @@ from berth_amd import synth
 from berth_amd.device import Exl3Linear, Gpu
 from berth_amd.kernels import Codebook, OutDtype
 from oracle import oracle as O
-from tests.gpu_util import DEV, close, dev, host_f16, host_u16
+from tests.gpu_util import DEV, close, dev, host_f16, host_u16, knobs
 
 pytestmark = pytest.mark.gpu
 
@@ -296,6 +296,12 @@ def test_gemm_split_k(m, Kk, N):
 
 
 def _check_balanced(m, Kk, N, fp32, tile, bits=4, cb=2):
+    """Tiles dealt out to 256 workgroups whatever they cost (short K and few rows keep the oracle quick)."""
+    with knobs(BERTH_GEMM_BALANCED=256, **({"BERTH_GEMM_ROWS256": 2} if tile == 256 else {})):
+        _check_dealt_out(m, Kk, N, fp32, tile, bits, cb)
+
+
+def _check_dealt_out(m, Kk, N, fp32, tile, bits, cb):
     got, want, ah, want_ah, launch = _run_linear(m, Kk, N, bits, cb, fp32, 700 + m, prefill=True)
     name = "exl3_gemm_wide_kernel" if tile == 256 else "exl3_gemm_balanced_kernel"
     assert f"{name}<{bits},{cb},{tile}x256>" in launch, launch
@@ -316,9 +322,9 @@ def test_gemm_128_row_tiles_dealt_out_evenly(m, Kk, N, fp32):
 @pytest.mark.parametrize("m,Kk,N,fp32,bits", [(512, 512, 16384, True, 4), (300, 256, 16640, False, 4),
                                               (640, 256, 11008, True, 3)])
 def test_gemm_256_row_tiles_dealt_out_evenly(m, Kk, N, fp32, bits):
-    """More than 128 rows and at least half as many 256 x 256 tiles as compute units: tiles
-    of eight waves; every weight is decoded once per tile and reaches the MFMA waves through
-    LDS.  Dealt out the same way.  The last row tile may be short (44 or 128 rows)."""
+    """More than 128 rows, 256 x 256 tiles: tiles of eight waves; every weight is decoded once per
+    tile and reaches the MFMA waves through LDS.  Dealt out the same way.  The last row tile may
+    be short (44 or 128 rows)."""
     _check_balanced(m, Kk, N, fp32, 256, bits)
 
 
