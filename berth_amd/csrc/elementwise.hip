@@ -274,7 +274,7 @@ std::string launch_had_r_128(const void* in, void* out, const void* scale, int p
         else hipLaunchKernelGGL((had_r_128_kernel<_Float16, false>), grid, dim3(256), 0, stream, (const _Float16*)in, (_Float16*)out, sc, blocks, col_blocks);
     }
     hip_ok(hipGetLastError(), "had_r_128 launch");
-    return std::string(fp32 ? "had_ff_r_128_kernel<" : "had_hf_r_128_kernel<") + (pre_scale ? "1,0>" : "0,1>") +
+    return std::string(fp32 ? "had_r_128_kernel<float," : "had_r_128_kernel<half,") + (pre_scale ? "1,0>" : "0,1>") +
            " grid=" + std::to_string(grid.x) + " block=256";
 }
 
@@ -327,7 +327,7 @@ std::string launch_add_f32(const void* a, const void* b, void* c, int n, hipStre
     const unsigned blocks = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(add_f32_kernel, dim3(blocks), dim3(256), 0, stream, (const float*)a, (const float*)b, (float*)c, n);
     hip_ok(hipGetLastError(), "add_f32 launch");
-    return "add_f32 block=256 grid=" + std::to_string(blocks);
+    return "add_f32_kernel block=256 grid=" + std::to_string(blocks);
 }
 
 // c[r][j] += bias[j] for a linear that carries a bias (crates/berth-exl3/src/linear.rs:131-133; the
@@ -356,7 +356,7 @@ std::string launch_add_bias(void* c, const void* bias, int rows, int n, int c_fp
     else
         hipLaunchKernelGGL(add_bias_kernel<false>, dim3(blocks), dim3(256), 0, stream, c, (const float*)bias, n, total);
     hip_ok(hipGetLastError(), "add_bias launch");
-    return std::string("add_bias ") + (c_fp32 ? "f32" : "f16") + " block=256 grid=" + std::to_string(blocks);
+    return std::string(c_fp32 ? "add_bias_kernel<f32>" : "add_bias_kernel<f16>") + " block=256 grid=" + std::to_string(blocks);
 }
 
 // RMS norm of fp32 rows to fp16, optionally with the fused residual
@@ -496,7 +496,8 @@ std::string launch_rms_norm(const void* x, const void* weight, void* y, void* re
     float* r = (float*)residual;
     // rows of eight values a thread, sixteen bytes at a time; what does not divide or align takes
     // the four-value kernel
-    if (dim % 8 == 0 && dim <= 32768 && (((uintptr_t)x | (uintptr_t)weight | (uintptr_t)y | (uintptr_t)residual) & 15) == 0) {
+    const bool by_row = dim % 8 == 0 && dim <= 32768 && (((uintptr_t)x | (uintptr_t)weight | (uintptr_t)y | (uintptr_t)residual) & 15) == 0;
+    if (by_row) {
         if (residual) {
             if (weight_bf16) launch_rms_norm_row<true, true>(xf, w, yh, r, rows, dim, epsilon, constant_bias, constant_scale, stream);
             else launch_rms_norm_row<true, false>(xf, w, yh, r, rows, dim, epsilon, constant_bias, constant_scale, stream);
@@ -512,7 +513,7 @@ std::string launch_rms_norm(const void* x, const void* weight, void* y, void* re
         else hipLaunchKernelGGL((rms_norm_kernel<false, false>), grid, block, 0, stream, xf, w, yh, r, dim, epsilon, constant_bias, constant_scale);
     }
     hip_ok(hipGetLastError(), "rms_norm launch");
-    return std::string("rms_norm_kernel<") + (residual ? "2" : "0") + ",float,half," + (weight_bf16 ? "bfloat16" : "half") +
+    return std::string(by_row ? "rms_norm_row_kernel<" : "rms_norm_kernel<") + (residual ? "2" : "0") + ",float,half," + (weight_bf16 ? "bfloat16" : "half") +
            ",float> grid=" + std::to_string(rows);
 }
 
@@ -565,7 +566,7 @@ std::string launch_rms_norm_f16(const void* x, const void* weight, void* y, int 
     hipLaunchKernelGGL(rms_norm_f16_kernel, dim3((unsigned)rows), dim3(256), 0, stream, (const _Float16*)x,
                        (const uint16_t*)weight, (_Float16*)y, dim, epsilon, constant_bias, constant_scale);
     hip_ok(hipGetLastError(), "rms_norm_f16 launch");
-    return "rms_norm_kernel<0,half,half,bfloat16,half> block=256 grid=" + std::to_string(rows);
+    return "rms_norm_f16_kernel<0,half,half,bfloat16,half> block=256 grid=" + std::to_string(rows);
 }
 
 // Embedding rows (crates/berth-kernels/src/ops.rs:99-127, csrc/ops/embed.cu): out[t] =
@@ -590,7 +591,7 @@ std::string launch_embed_tokens(const void* weight, const int* ids, void* out, i
     if (f16) hipLaunchKernelGGL(embed_bf16_kernel<true>, dim3((unsigned)n), dim3(256), 0, stream, (const uint16_t*)weight, ids, out, hidden);
     else hipLaunchKernelGGL(embed_bf16_kernel<false>, dim3((unsigned)n), dim3(256), 0, stream, (const uint16_t*)weight, ids, out, hidden);
     hip_ok(hipGetLastError(), f16 ? "embed_tokens_f16 launch" : "embed_tokens launch");
-    return std::string(f16 ? "embed_bf16_f16" : "embed_bf16_f32") + " block=256 grid=" + std::to_string(n);
+    return std::string(f16 ? "embed_bf16_kernel<f16>" : "embed_bf16_kernel<f32>") + " block=256 grid=" + std::to_string(n);
 }
 
 // out[row] = embedding[row] followed by hidden[row], fp16 (crates/berth-kernels/src/ops.rs:136-143,
@@ -612,7 +613,7 @@ std::string launch_cat_f16_last(const void* embedding, const void* hidden, void*
     hipLaunchKernelGGL(cat_f16_last_kernel, dim3((unsigned)rows), dim3(256), 0, stream, (const uint16_t*)embedding,
                        (const uint16_t*)hidden, (uint16_t*)out, width);
     hip_ok(hipGetLastError(), "cat_f16_last launch");
-    return "cat_f16_last block=256 grid=" + std::to_string(rows);
+    return "cat_f16_last_kernel block=256 grid=" + std::to_string(rows);
 }
 
 // crates/berth-exl3/src/signs.rs:25-46: packed su / sv -> fp16 signs.  Little-endian

@@ -251,7 +251,7 @@ static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebo
         const dim3 grid((unsigned)tiles, (unsigned)(pl.rows_per_tile / 16));
         hipLaunchKernelGGL(exl3_gemm_finish_kernel, grid, dim3(256), 0, stream, p);
         hip_ok(hipGetLastError(), "exl3_gemm_finish_kernel launch");
-        desc += " + exl3_gemm_finish grid=" + std::to_string(grid.x) + "x" + std::to_string(grid.y);
+        desc += " + exl3_gemm_finish_kernel grid=" + std::to_string(grid.x) + "x" + std::to_string(grid.y);
     }
 }
 

@@ -21,7 +21,7 @@ static void gemm_launch_mb(const GemmParams& p, hipStream_t stream, std::string&
                                 "exl3_gemm_kernel shared-memory attribute");
     }
     if (p.units > 0) {
-        // balanced dense launch (128-row tiles only): two workgroups per compute unit
+        // dealt-out dense launch (128-row tiles only)
         if constexpr (MB == 4) {
             static bool raised2[64] = {};
             raise_dynamic_lds_limit((const void*)exl3_gemm_balanced_kernel<BITS, CB, MB>, (int)smem, raised2,
@@ -76,7 +76,7 @@ static void gemm_launch_rows(const GemmParams& p, hipStream_t stream, std::strin
     raise_dynamic_lds_limit((const void*)exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED>, 160 * 1024, raised,
                             "exl3_gemm_rows_kernel shared-memory attribute");
     hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED>), grid, dim3(1024), p.lds_bytes, stream, p);
-    desc = "exl3_gemm_kernel/rows<" + std::to_string(BITS) + "," + std::to_string(CB) + "," + std::to_string(16 * MT) +
+    desc = "exl3_gemm_rows_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + "," + std::to_string(16 * MT) +
            "x128> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
            (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
 }
@@ -89,7 +89,7 @@ static void gemm_launch_block(const GemmParams& p, hipStream_t stream, std::stri
     raise_dynamic_lds_limit((const void*)exl3_gemm_block_kernel<BITS, CB, MT>, 160 * 1024, raised,
                             "exl3_gemm_block_kernel shared-memory attribute");
     hipLaunchKernelGGL((exl3_gemm_block_kernel<BITS, CB, MT>), grid, dim3(1024), p.lds_bytes, stream, p);
-    desc = "exl3_gemm_kernel/block<" + std::to_string(BITS) + "," + std::to_string(CB) + "," +
+    desc = "exl3_gemm_block_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + "," +
            std::to_string(p.rows_per_tile) + "x128> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
            (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
 }

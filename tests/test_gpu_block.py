@@ -38,7 +38,7 @@ def _every_size():
 ])
 def test_row_blocks_match_the_oracle_and_repeat(rows, Kk, N, bits, cb, fp32):
     got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, bits, cb, fp32, 60 + rows, prefill=True)
-    assert "exl3_gemm_kernel/block" in launch, launch
+    assert "exl3_gemm_block_kernel" in launch, launch
     assert np.array_equal(ah, want_ah), launch
     bad, worst = close(got, want)
     assert bad == 0, (bad, worst, launch)
@@ -67,7 +67,7 @@ def test_bundle_with_narrower_slices(rows, unit):
                      lists[2].data_ptr(), rows, Kk, width, bits, Codebook.MUL1, OutDtype.F16, 1, 4, n_list.data_ptr(),
                      c_ptrs.data_ptr(), n_list.data_ptr(), src.data_ptr(), 4)
     torch.cuda.synchronize()
-    assert "exl3_gemm_kernel/block" in K.ops.last_launch(), K.ops.last_launch()
+    assert "exl3_gemm_block_kernel" in K.ops.last_launch(), K.ops.last_launch()
     for i, (tr, suh, svh) in enumerate(lins):
         want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=False)
         assert close(host_f16(outs[i]), want)[0] == 0, i

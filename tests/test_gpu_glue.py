@@ -40,7 +40,7 @@ def test_rms_norm_fixture(yfile):
     x, y = load("norm.x.bin", np.float32), load(yfile, np.float16)
     got, _ = _rms(x.reshape(1, -1), recover_weight(x, y), EPS, 1.0, 1.0, True)
     assert np.array_equal(got.view(np.uint16).ravel(), y.view(np.uint16))
-    assert "rms_norm_kernel<0,float,half,bfloat16,float>" in K.ops.last_launch()
+    assert "rms_norm_row_kernel<0,float,half,bfloat16,float>" in K.ops.last_launch()
 
 
 def test_rms_norm_res_in_fixture():
@@ -74,7 +74,7 @@ def test_add_f32_fixture_and_alias():
     K.ops.add_f32(d_a.data_ptr(), d_b.data_ptr(), d_c.data_ptr(), a.size)
     torch.cuda.synchronize()
     assert np.array_equal(d_c.cpu().numpy().view(np.uint32), c.view(np.uint32))
-    assert K.ops.last_launch() == "add_f32 block=256 grid=20"
+    assert K.ops.last_launch() == "add_f32_kernel block=256 grid=20"
     K.ops.add_f32(d_a.data_ptr(), d_b.data_ptr(), d_a.data_ptr(), a.size)      # c may alias a
     torch.cuda.synchronize()
     assert np.array_equal(d_a.cpu().numpy().view(np.uint32), c.view(np.uint32))
@@ -93,7 +93,7 @@ def test_rms_norm_f16_matches_the_fp32_input_norm_on_widened_rows():
     y = torch.zeros((rows, dim), dtype=torch.float16, device=DEV)
     K.ops.rms_norm_f16(d_x.data_ptr(), d_w.data_ptr(), y.data_ptr(), rows, dim, 1e-6)
     torch.cuda.synchronize()
-    assert "rms_norm_kernel<0,half,half,bfloat16,half>" in K.ops.last_launch()
+    assert "rms_norm_f16_kernel<0,half,half,bfloat16,half>" in K.ops.last_launch()
     want = O.rms_norm(x.astype(np.float32), w_bf16, 1e-6, 1.0, 1.0, weight_bf16=True)
     assert np.array_equal(host_u16(y).reshape(rows, dim), want.view(np.uint16).reshape(rows, dim))
 
@@ -111,9 +111,9 @@ def test_embed_copy_and_concat_are_exact():
     out32 = torch.zeros((ids.size, hidden), dtype=torch.float32, device=DEV)
     out16 = torch.zeros((ids.size, hidden), dtype=torch.float16, device=DEV)
     K.ops.embed_tokens(d_w.data_ptr(), d_ids.data_ptr(), out32.data_ptr(), hidden, ids.size)
-    assert "embed_bf16_f32" in K.ops.last_launch()
+    assert "embed_bf16_kernel<f32>" in K.ops.last_launch()
     K.ops.embed_tokens(d_w.data_ptr(), d_ids.data_ptr(), out16.data_ptr(), hidden, ids.size, f16=True)
-    assert "embed_bf16_f16" in K.ops.last_launch()
+    assert "embed_bf16_kernel<f16>" in K.ops.last_launch()
     torch.cuda.synchronize()
     assert np.array_equal(out32.cpu().numpy().view(np.uint32), exact[ids].view(np.uint32))
     assert np.array_equal(host_u16(out16), exact[ids].astype(np.float16).view(np.uint16))

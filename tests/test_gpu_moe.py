@@ -192,7 +192,8 @@ def test_moe_layer_matches_oracle(T, H, E, k, I, bits, shared_I, scale):
     err = np.abs(out.cpu().numpy() - want)
     assert err.max() <= 2e-3 * np.abs(want).max(), (err.max(), np.abs(want).max(), launch)
     if T > 1 and T * k + (T if shared_I == I else 0) > 8:
-        assert ("exl3_gemm_kernel" in launch or "exl3_gemm_mixed_kernel" in launch) and "exl3_gemv_kernel" not in launch
+        assert any(k in launch for k in ("exl3_gemm_rows_kernel", "exl3_gemm_kernel", "exl3_gemm_mixed_kernel")), launch
+        assert "exl3_gemv_kernel" not in launch, launch
     else:
         assert "exl3_gemv_kernel" in launch and "exl3_gemm_" not in launch
     # a second call reuses the workspace and the self-resetting counters

@@ -67,7 +67,7 @@ def test_few_token_layers_on_the_grouped_few_row_kernel(T, H, E, k, I, bits, sha
     d_x = dev(x.view(np.uint16))
     layer.forward(gpu, d_x, out, T, idx, w)
     torch.cuda.synchronize()
-    assert "exl3_gemm_kernel/rows" in K.moe.last_launch(), K.moe.last_launch()
+    assert "exl3_gemm_rows_kernel" in K.moe.last_launch(), K.moe.last_launch()
     want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, 2, shared=shared_np, shared_I=shared_I)
     assert np.array_equal(idx.cpu().numpy(), oi)
     _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I)

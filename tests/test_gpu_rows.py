@@ -38,7 +38,7 @@ def _every_size():
 ])
 def test_few_rows_match_the_oracle_and_repeat(rows, Kk, N, bits, cb):
     got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, bits, cb, True, 40 + rows, prefill=True)
-    assert "exl3_gemm_kernel/rows" in launch, launch
+    assert "exl3_gemm_rows_kernel" in launch, launch
     assert np.array_equal(ah, want_ah), launch
     bad, worst = close(got, want)
     assert bad == 0, (bad, worst, launch)
@@ -68,7 +68,7 @@ def test_bundle_with_narrower_slices(rows, unit):
                      lists[2].data_ptr(), rows, Kk, width, bits, Codebook.MUL1, OutDtype.F16, 1, 4, n_list.data_ptr(),
                      c_ptrs.data_ptr(), n_list.data_ptr(), src.data_ptr(), 4)
     torch.cuda.synchronize()
-    assert "exl3_gemm_kernel/rows" in K.ops.last_launch(), K.ops.last_launch()
+    assert "exl3_gemm_rows_kernel" in K.ops.last_launch(), K.ops.last_launch()
     for i, (tr, suh, svh) in enumerate(lins):
         want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=False)
         assert close(host_f16(outs[i]), want)[0] == 0, i
@@ -79,7 +79,7 @@ def test_bundle_with_narrower_slices(rows, unit):
 def test_mlp_of_few_rows_stage_by_stage(rows):
     from tests.test_gpu_mlp import run_mlp_block
     launch = run_mlp_block(rows, 1536, 4096, 4)
-    assert launch.count("exl3_gemm_kernel/rows") == 2 and "silu_mul_had_r_128_kernel" in launch, launch
+    assert launch.count("exl3_gemm_rows_kernel") == 2 and "silu_mul_had_r_128_kernel" in launch, launch
 
 
 @pytest.mark.parametrize("rows,H,I,bits", [(2, 128, 256, 4),        # one block a row: a quarter of a wave
