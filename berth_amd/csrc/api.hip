@@ -212,7 +212,8 @@ void check_shape(const char* who, const LinearArgs& a)
         throw std::runtime_error(w + ": size_k must be a multiple of 128 (one Hadamard block)");
 }
 
-// rows up to this count take the VALU kernel, more rows the MFMA kernel
+// rows up to this count go through launch_gemv (one row: the streaming or the VALU kernel; more: the few-row
+// MFMA kernel, the VALU kernel for small weights), more rows through launch_gemm
 int gemv_max_rows() { return knobs().gemv_max_rows; }
 
 std::string dispatch_linear(const LinearArgs& a)
@@ -255,9 +256,10 @@ extern "C" int berth_exl3_linear(const void* a, const void* trellis, void* c, co
 // copy until the process ends.  In host code the array's name is only a handle for
 // hipGetSymbolAddress; the device address it returns, kept per device, is what kernels get.
 // The array has no initialiser, so it is zero when the code object is loaded, and every launch
-// leaves the counters and accumulators it used at zero again: nothing has to clear it, and
-// the entry point launches nothing but its GEMV (a first call inside a stream capture records
-// that one kernel).
+// leaves the counters and accumulators it used at zero again: nothing has to clear it, and a
+// first call inside a stream capture records only the linear's own launches (one kernel; two for
+// 2..8 rows of a weight large enough for the few-row MFMA kernel, whose input a launch of its own
+// rotates into the partial sums' scratch).
 namespace {
 constexpr size_t kNoAllocPartialBytes = (size_t)8 << 20;
 constexpr int kNoAllocCounters = 65536;
@@ -912,9 +914,9 @@ extern "C" uint64_t berth_ops_mgemm_tune_key(int size_m, int size_k, int size_n,
 
 // Which of the reference's two QTIP GEMV configurations (0 narrow, 1 wide, -1 neither) its
 // rows-2..8 route would take (crates/berth-kernels/csrc/prefill_lin/gemv.cu:71-99: host
-// integer arithmetic; cc 2 = Ampere, 3 = Ada there).  On this device rows 2..8 always take
-// the VALU kernel and nothing consumes the answer; the table is kept so that the crate
-// links and its table test reads the same.
+// integer arithmetic; cc 2 = Ampere, 3 = Ada there).  On this device rows 2..8 take the few-row
+// MFMA kernel or the VALU kernel by the weight's size (rows_min_units) and nothing consumes the
+// answer; the table is kept so that the crate links and its table test reads the same.
 extern "C" int berth_exl3_gemv_cfg(int cc, int size_m, int size_k, int size_n, int k_bits, int cb, int mode,
                                    int narrow_coresident)
 {

@@ -410,8 +410,8 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     return d0 + " + " + desc + (a.out_fp32 ? " out=f32" : " out=f16");
 }
 
-// berth_ops_mgemm with more than 8 rows: the bundle's linears as one dense MFMA launch behind
-// one launch that rotates every distinct input (slab s of a_had = Hh(input(s) * suh[s])).
+// berth_ops_mgemm with more than 8 rows, or 2..8 of large weights: the bundle's linears on the MFMA kernels
+// behind one launch that rotates every distinct input (slab s of a_had = Hh(input(s) * suh[s])).
 std::string launch_gemm_bundle(const MgemmArgs& m)
 {
     if (m.size_k % 128 != 0) throw std::runtime_error("exl3_mgemm: size_k must be a multiple of 128");

@@ -1,4 +1,6 @@
-// EXL3 linear for 1..8 rows: trellis decode fused into a VALU dot product.
+// Launchers of the EXL3 linear for 1..8 rows.  Large weights take the streaming kernel
+// (one row, exl3_gemv_stream_kernel.cuh) or the few-row MFMA kernel (2..8 rows,
+// exl3_gemm_rows_kernel.cuh); the others a trellis decode fused into a VALU dot product:
 //
 //   c = ( Hh(a * suh) @ W ) -> Hh(.) * svh          (Hh = 128-block Hadamard / sqrt(128))
 //

@@ -558,7 +558,7 @@ public:
     bool has_bias() const { return has_bias_; }
 
     // x fp16 [rows][hidden] -> y fp32 [rows][hidden] through berth_exl3_mlp: gate and up in one
-    // launch, silu(g) * u evaluated inside the down projection (two launches up to 8 rows)
+    // launch, silu(g) * u evaluated inside the down projection (one row: two launches in all)
     void forward_fused(const Gpu& gpu, const DeviceBuffer<Half>& x, DeviceBuffer<float>& y, int rows = 1) const
     {
         if (!uniform_) throw InputError("mlp: the one-call path needs one bit rate and codebook");

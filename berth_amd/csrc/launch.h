@@ -69,7 +69,7 @@ struct Knobs {
     int gemv_stream_lut;        // BERTH_GEMV_STREAM_LUT        table mask of the hybrid decode (-1: by size)
     int gemv_wg_per_cu;         // BERTH_GEMV_WG_PER_CU         workgroups per compute unit of the 1..8-row kernel
     int gemv_half_units;        // BERTH_GEMV_HALF_UNITS        0: never walk half k-blocks
-    int gemv_max_rows;          // BERTH_GEMV_MAX_ROWS          rows up to this count take the VALU kernel (1..8)
+    int gemv_max_rows;          // BERTH_GEMV_MAX_ROWS          rows up to this count go through launch_gemv (1..8)
     int gemm_wg_per_cu;         // BERTH_GEMM_WG_PER_CU
     int gemm_balanced;          // BERTH_GEMM_BALANCED
     int gemm_rows256;           // BERTH_GEMM_ROWS256
@@ -276,10 +276,11 @@ constexpr int kNormRotateMaxCols = 32768;
 std::string launch_gemm_pair(const PairArgs& pair, void* a_had_second);
 constexpr int kBundleMaxSlices = 16;    // slices of a bundle whose lists travel by value
 
-// rows 1..8: VALU dot-product kernel.  Returns the launch description.  `scratch`: the
-// split-K scratch to use instead of the device's lazily allocated workspace.
+// rows 1..8: one row on the streaming kernel, 2..8 rows on the few-row MFMA kernel (launch_gemm), small
+// weights on the VALU dot-product kernel.  Returns the launch description.  `scratch`: the split-K
+// scratch to use instead of the device's lazily allocated workspace.
 std::string launch_gemv(const LinearArgs& args, const Workspace* scratch = nullptr);
-// any row count: fp16 MFMA kernel (rows padded to 32 inside the kernel).
+// any row count, fp16 MFMA kernels: few rows, row blocks, or tiles of 32, 128 or 256 rows.
 std::string launch_gemm(const LinearArgs& args, const Workspace* scratch = nullptr);
 // whether a launch of this many linears of one shape takes the few-row kernel (2..32 rows)
 bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, int size_n);

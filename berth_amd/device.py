@@ -251,7 +251,7 @@ class Exl3MultiLinear:
     `exl3_mgemm` (the qkv bundles of crates/berth-engine/src/attn.rs:1934-1973 and
     gdn.rs:1102-1130; list layout from crates/berth-kernels/src/ops.rs:264-293):
     every source is cut into slices of the greatest common width.  Any row count: one
-    row runs the streaming kernel, 2..8 the dot-product kernel, more the MFMA kernels
+    row runs the streaming kernel, 2..8 of small weights the dot-product kernel, the rest the MFMA kernels
     (the reference sends 9..32 rows through the same call, prefill.rs:81-85)."""
 
     def __init__(self, gpu: Gpu, sources: list[Exl3Linear]):
@@ -384,7 +384,7 @@ class MlpLayer:
 
     def forward(self, gpu: Gpu, x: torch.Tensor, y: torch.Tensor, fused: bool = True, rows: int = 1) -> None:
         """x fp16 [rows][hidden] -> y fp32 [rows][hidden].  fused: one `berth_exl3_mlp` call (two
-        launches up to 8 rows); otherwise the reference's four calls for one row (mlp.rs:118-150)."""
+        launches for one row, four or more above); otherwise the reference's four calls for one row (mlp.rs:118-150)."""
         if fused and self.uniform and not self.has_bias:
             if rows * self.intermediate > self.g.numel() or x.numel() < rows * self.hidden or \
                y.numel() < rows * self.hidden:

@@ -145,7 +145,7 @@ def lin_table(lins):
 def exl3_mlp(x, lins, gate_out, up_out, a_had, act_had, y, size_m, hidden, intermediate, k_bits,
              codebook: Codebook, stream=None) -> None:
     """y = down(silu(gate(x)) * up(x)): the four calls of crates/berth-engine/src/mlp.rs:118-150
-    in one entry (two launches up to 8 rows).  lins: three (trellis, suh, svh) address triples."""
+    in one entry (two launches for one row).  lins: three (trellis, suh, svh) address triples."""
     rc = load().berth_exl3_mlp(x, lin_table(lins), gate_out, up_out, a_had, act_had, y, size_m, hidden, intermediate, k_bits,
                                int(codebook), stream)
     if rc != 0:

@@ -205,11 +205,11 @@ int berth_ops_cat_f16_last(const void* embedding, const void* hidden, void* out,
  * size_n_list[s] <= size_n = slice width; had_src_list[s] = source index;
  * a_had holds num_had_src slabs of size_m*size_k.  Uniform mode (lists NULL):
  * bszm_out linears of one shape, inputs a[i] (bszm_in == bszm_out) or a[0]
- * (bszm_in == 1), outputs c[i] contiguous.  Any row count: up to 8 rows run the
- * dot-product kernels (the rotation of the input inside the launch), more rows one
- * launch that rotates the input once per source / linear and one dense MFMA launch
- * over all slices (the reference sends 9..32 rows of its fused q/k/v and gate/up
- * bundles through this call, crates/berth-engine/src/prefill.rs:81-85).  Returns 1
+ * (bszm_in == 1), outputs c[i] contiguous.  Any row count: one row, and 2..8 rows of
+ * small weights, rotate the input inside the one launch; more rows, and 2..8 rows of
+ * larger weights, take one launch that rotates the input once per source / linear and
+ * MFMA launches over all slices (the reference sends 9..32 rows of its fused q/k/v and
+ * gate/up bundles through this call, crates/berth-engine/src/prefill.rs:81-85).  Returns 1
  * on success (the reference returns its kernel-shape tag there), -1 on error. */
 int berth_ops_mgemm(const void* a, const void* b_list, void* c, const void* suh_list, void* a_had,
                     const void* svh_list, int size_m, int size_k, int size_n, int k_bits,
@@ -258,14 +258,16 @@ typedef struct {
  * y = down(silu(gate(x)) * up(x)), the four calls of MlpLayer::forward
  * (crates/berth-engine/src/mlp.rs:118-150: two berth_exl3_linear with fp16
  * output, berth_ops_silu_mul with act_limit 0, berth_exl3_linear with fp32
- * output) in one entry.  Up to 8 rows run as two launches: gate and up share one
- * launch and the rotated input, and the down projection evaluates silu(g) * u
- * while it rotates its input (same fp16 steps as berth_ops_silu_mul, so the
- * activation is bit-identical to the unfused sequence).  More rows run on the MFMA
- * kernels: gate and up as one bundle (one launch rotates the input with either
- * linear's scales, one dense launch runs both; the up projection's rotated copy
- * waits in act_had, so this form needs intermediate >= hidden, else gate and up run
- * one after the other), berth_ops_silu_mul, the down projection.
+ * output) in one entry.  One row, and 2..8 rows of small weights, run as two
+ * launches: gate and up share one launch and the rotated input, and the down
+ * projection evaluates silu(g) * u while it rotates its input (same fp16 steps as
+ * berth_ops_silu_mul, so the activation is bit-identical to the unfused sequence).
+ * More rows, and 2..8 rows of larger weights, run on the MFMA kernels: gate and up as
+ * one bundle (one launch rotates the input with either linear's scales, the next runs
+ * both; the up projection's rotated copy waits in act_had, so this form needs
+ * intermediate >= hidden, else gate and up run one after the other), one launch that
+ * forms silu(g) * u and rotates it, the down projection; the row-block kernel
+ * (33..448 rows) adds a launch that finishes its shared tiles.
  * lins: HOST array {gate, up, down} of device pointers.  x fp16 [m][hidden];
  * gate_out, up_out fp16 [m][intermediate] (written; above 8 rows up_out ends up
  * holding the activation); a_had fp16 [m][hidden] and act_had fp16
@@ -291,7 +293,7 @@ int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* gate_out, vo
  * differs), and where the down projection takes it the residual is added where it writes its
  * output: two launches when both do.  More rows where gate and up run on the MFMA kernels as one
  * bundle: the norm is formed where the input is rotated and the residual added where the down launch
- * writes (four launches).  Anything else runs the same arithmetic as separate launches. */
+ * writes (four launches, and those that finish shared tiles).  Anything else runs the same arithmetic as separate launches. */
 typedef struct {
     const void* weight;         /* fp16 or bf16 [hidden] */
     float epsilon, constant_bias, constant_scale;

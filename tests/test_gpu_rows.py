@@ -84,7 +84,7 @@ def test_mlp_of_few_rows_stage_by_stage(rows):
 
 @pytest.mark.parametrize("rows,H,I,bits", [(2, 128, 256, 4),        # one block a row: a quarter of a wave
                                            (9, 1152, 1280, 3),      # a workgroup with a half-empty wave
-                                           (33, 8320, 8320, 2),     # two chunks a thread, 32-row tiles with one row
+                                           (33, 8320, 8320, 2),     # two chunks a thread, one row block with one row past its first 32
                                            (3, 17408, 17408, 1)])   # three chunks
 def test_block_with_fused_norm_equals_the_separate_calls(rows, H, I, bits):
     """Residual add, norm and both rotations in one launch, the residual added by the down launch:
