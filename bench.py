@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the EXL3 trellis GEMV hot path on one MI355X.
 
-Workload (BASELINE.json configs[1] at the bit rate the metric is quoted on): the
+Workload (at the bit rate the metric is quoted on): the
 dense 27B-shaped decode linear set at batch 1, 4 bpw, mul1 codebook — q_proj
 5120x6144, k/v_proj 5120x1024, o_proj 6144x5120, gate/up 5120x17408, down
 17408x5120 — fp16 activations N(0,1), uniform random trellis words, suh/svh
@@ -87,8 +87,8 @@ def cpu_baseline(bits: int, seconds: float):
             if el >= budget:
                 return el / n, n
 
-    # the other CPU figures of the same port, a few seconds each
-    # (4096 x 4096, 4 bpw) as a GEMV and as a dequantisation, configs[3] at one token
+    # the other CPU figures of the same port, a few seconds each: a 4096 x 4096 linear
+    # at 4 bpw as a GEMV and as a dequantisation, the 128-expert layer at one token
     k0 = 4096
     tr0, suh0, svh0 = synth.linear(13, k0, k0, 4)
     x0 = synth.activations(14, 1, k0)
@@ -328,7 +328,7 @@ def moe_plan_bytes(H: int, E: int, k: int, I: int, bits: int, shared_I: int = 0)
 
 
 def moe_bench(gpu, steps: int, warmup: int):
-    """hidden 2048, 128 experts, top-8 softmax routing,
+    """MoE layer: hidden 2048, 128 experts, top-8 softmax routing,
     expert intermediate 768, 4 bpw, router fp16 N(0, 0.02); batch 1 and 64.  One
     call = route + permute + grouped gate/up + SiLU gate + grouped down + combine."""
     import torch
@@ -404,7 +404,7 @@ def moe_bench(gpu, steps: int, warmup: int):
 
 
 def moe_large_bench(gpu, steps: int, resident_layers: int = 48):
-    """hidden 2048, 512 experts top-10 plus one always-on
+    """Large MoE layer: hidden 2048, 512 experts top-10 plus one always-on
     shared expert, intermediate 512, 3 bpw, 256 tokens, router logits biased so
     that expert popularity is Zipf(1.1); the weights of 48 such layers (29 GB)
     stay resident in HBM and the steps rotate over them.  Weights are generated
@@ -496,7 +496,7 @@ def moe_large_bench(gpu, steps: int, resident_layers: int = 48):
 
 
 def bpw_sweep(gpu, rates, steps: int, nlayers: int = 8):
-    """BASELINE.json configs[1] at the other bit rates of its sweep: the same four
+    """The decode linear set at the other bit rates: the same four
     launches per step over device-generated weights, GB/s of algorithmic bytes."""
     import torch
 
@@ -652,7 +652,7 @@ def mlp_block_bench(gpu, layers, bits: int, steps: int):
 
 
 def prefill_bench(gpu, layers, bits: int, rows: int, steps: int):
-    """the same 27B-shaped linears at `rows` = 512 tokens,
+    """The same 27B-shaped linears at `rows` = 512 tokens,
     fp16 activations N(0,1), fp16/fp32 outputs with fp32 accumulation: seven calls of
     berth_prefill_exl3_linear (Hadamard pre-pass + decode-in-GEMM MFMA kernel), and the same
     work with q/k/v and gate/up as bundles (berth_ops_mgemm: one rotation launch and one dense

@@ -514,7 +514,7 @@ def test_very_wide_output_uses_closer_counters(rows):
                                          ("o_proj", "exl3_gemm_balanced_kernel<4,2,128x256>"),
                                          ("k_proj", "exl3_gemm_kernel<4,2,32x256>")])
 def test_prefill_27b_shapes_at_512_rows_slices_match_oracle(name, kernel):
-    """BASELINE configs[2] at full size (512 rows, 4 bpw, the 27B shapes): each of the four
+    """Prefill at full size (512 rows, 4 bpw, the 27B shapes): each of the four
     launch forms the dispatcher picks there, with 256-column windows (first, an odd middle
     one, last) of all 512 rows checked against the oracle on the matching trellis slice."""
     Kk, N = synth.SHAPES_27B[name]
@@ -653,7 +653,7 @@ def _window_check(name, Kk, N, bits, out_fp32, seed):
 
 @pytest.mark.parametrize("name", ["q_proj", "o_proj", "down_proj"])
 def test_27b_shapes_batch1_4bpw_windows_match_oracle(name):
-    """BASELINE configs[1] at 4 bpw, the shapes the other full-size tests leave out."""
+    """The decode linear set at 4 bpw, the shapes the other full-size tests leave out."""
     Kk, N = synth.SHAPES_27B[name]
     _window_check(name, Kk, N, 4, name != "q_proj", 7100 + Kk % 97)
 
@@ -661,6 +661,6 @@ def test_27b_shapes_batch1_4bpw_windows_match_oracle(name):
 @pytest.mark.parametrize("bits", [2, 3, 5])
 @pytest.mark.parametrize("name", ["gate_proj", "down_proj", "q_proj", "o_proj", "k_proj"])
 def test_27b_shapes_batch1_other_rates_windows_match_oracle(name, bits):
-    """BASELINE configs[1] at 2, 3 and 5 bpw on every shape of the set (v_proj has k_proj's)."""
+    """The decode linear set at 2, 3 and 5 bpw on every shape of the set (v_proj has k_proj's)."""
     Kk, N = synth.SHAPES_27B[name]
     _window_check(name, Kk, N, bits, name in ("down_proj", "o_proj"), 7200 + 10 * bits + Kk % 97 + len(name))

@@ -222,7 +222,7 @@ def test_moe_config3_shape_decode_token():
 
 
 def test_moe_config3_shape_batch64():
-    """BASELINE configs[3] at 64 tokens (hidden 2048, 128 experts, top-8, intermediate 768,
+    """64 tokens (hidden 2048, 128 experts, top-8, intermediate 768,
     4 bpw) at full size: the whole layer against the oracle, stage by stage and end to end."""
     gpu = Gpu(0)
     T, H, E, k, I, bits = 64, 2048, 128, 8, 768, 4
