@@ -42,7 +42,7 @@ PROFILE = {
                      "exl3_gemv_stream_kernel<4,2,table=0x0>",
                      "sliced x2 by value exl3_gemv_stream_kernel<4,2,table=0x0>",
                      "exl3_gemv_stream_kernel<4,2,table=0x0>"],
-        "traffic_bytes_per_launch": int((42265 + 892) * 1024),
+        "traffic_bytes_per_launch": int((42266 + 892) * 1024),
         "valu_instr_per_weight": 4.64},
 }
 ORDER = ["q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj"]
