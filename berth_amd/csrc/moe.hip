@@ -385,6 +385,21 @@ constexpr int kSlabExperts = 128;
 // LDS of a workgroup: segment sums [nseg][tt][128] fp32, then the tokens' rows [tt][H] as fp32 (H = 64 nseg)
 inline __host__ __device__ int route_slab_lds_bytes(int nseg, int tt) { return nseg * tt * kSlabExperts * 4 + tt * nseg * kRouteSeg * 4; }
 
+// v + src[0] + src[stride] + ... in order, sixteen reads in flight
+__device__ __forceinline__ float route_add_segments(float v, const float* src, int stride, int n)
+{
+    int seg = 0;
+    for (; seg + 16 <= n; seg += 16, src += 16 * stride) {
+        float part[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) part[j] = src[j * stride];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v += part[j];
+    }
+    for (; seg < n; ++seg, src += stride) v += *src;
+    return v;
+}
+
 template <int TT>
 __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
 {
@@ -479,7 +494,7 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
     // ---- thread (token, expert of the slab): segments added in order, bias
     float v = 0.0f;
     if (mine) {
-        for (int seg = 0; seg < p.nseg; ++seg) v += s_parts[((size_t)seg * TT + tt_mine) * kSlabExperts + c];
+        v = route_add_segments(v, s_parts + (size_t)tt_mine * kSlabExperts + c, TT * kSlabExperts, p.nseg);
         if (p.bias) v += bias_mine;
         if (p.logits && t_mine < p.T) p.logits[(size_t)t_mine * p.E + e_mine] = v;
     }

@@ -74,44 +74,79 @@ __device__ __forceinline__ float lane_value(float v, int lane_index)
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane_index));
 }
 
-// the same value in every lane: butterflies over lane distances 1 .. 32
+// the largest value of the wave (no NaN among them): one v_max_f32 with a DPP operand per distance, row
+// sums handed on to the next row, the result read from the last lane.  (A DPP operand may be read two
+// instructions after it was written at the earliest: the s_nop.)
 __device__ __forceinline__ float wave_max(float v)
 {
-    v = fmaxf(v, lane_xor_dpp<1>(v));
-    v = fmaxf(v, lane_xor_dpp<2>(v));
-    v = fmaxf(v, lane_xor_dpp<4>(v));
-    v = fmaxf(v, lane_xor_dpp<8>(v));
-    v = fmaxf(v, lane_xor_swap16(v));
-    return fmaxf(v, lane_xor_swap32(v));
+#define BERTH_MAX_STEP(ctrl) "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 " ctrl "\n\t"
+    asm volatile(BERTH_MAX_STEP("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf")
+                 BERTH_MAX_STEP("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf")
+                 BERTH_MAX_STEP("row_half_mirror row_mask:0xf bank_mask:0xf")
+                 BERTH_MAX_STEP("row_mirror row_mask:0xf bank_mask:0xf")
+                 BERTH_MAX_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf")
+                 BERTH_MAX_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
+                 "s_nop 1"
+                 : "+v"(v));
+#undef BERTH_MAX_STEP
+    return lane_value(v, 63);
 }
-// PER: how many of the lane's registers can hold experts (ceil(E / 64) rounded up to 2, 8 or 16)
+// PER: how many of the lane's registers can hold experts (ceil(E / 64) rounded up to 2, 8 or 16).
+// A lane sorts its own experts once (largest first, ties in order of their index); a round is then the
+// maximum of the lanes' heads, a ballot and one step of the winner's list.  What bounds it is one
+// wave's chain of dependent instructions: looking through all registers for the maximum and again for
+// its holder in every round, the top 8 of 128 took 2.0 us of a routing launch and the top 10 of 512 4.8;
+// 1.4 and 3.3 now.
 template <int PER>
 __device__ __forceinline__ int route_topk_n(const float (&lg)[kRoutePer], int lane, const RouteParams& p, int t,
                                             bool store = true)
 {
-    unsigned taken = 0;
+    float val[PER];
+    int who[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        // registers past the last expert sort behind the lane's real ones and, with a higher index, lose
+        // every tie; a logit that is no number ranks with minus infinity
+        val[i] = lane + 64 * i < p.E && lg[i] == lg[i] ? lg[i] : -INFINITY;
+        who[i] = lane + 64 * i;
+    }
+    // odd-even transposition: swaps neighbours only, so equal values keep their order
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+#pragma unroll
+        for (int i = r & 1; i + 1 < PER; i += 2) {
+            // (values, not elements, to choose from: a choice of elements becomes an indexed read of the array)
+            const float a = val[i], b = val[i + 1];
+            const int wa = who[i], wb = who[i + 1];
+            const bool swap = b > a;
+            val[i] = swap ? b : a;
+            val[i + 1] = swap ? a : b;
+            who[i] = swap ? wb : wa;
+            who[i + 1] = swap ? wa : wb;
+        }
+    }
     float sel_logit = 0.0f;         // lane j keeps the logit of slot j
     int sel_idx = 0;
-    // One slot per round: the largest remaining logit of the wave (max butterflies), then the
-    // lowest expert index among the registers that hold it (ballots).  One short reduction of
-    // one value instead of a reduction of (value, index) pairs with a tie rule.
+#pragma unroll 1
     for (int j = 0; j < p.k; ++j) {
-        float lv = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < PER; ++i)
-            if (lane + 64 * i < p.E && !((taken >> i) & 1u)) lv = fmaxf(lv, lg[i]);
-        const float bv = wave_max(lv);
-        // the lowest expert index that holds it: register i of lane l is expert l + 64 i, so
-        // the first register with a holder wins and, inside it, the lowest lane (a ballot
-        // and a find-first-set on the scalar side instead of a second butterfly chain)
+        const float bv = wave_max(val[0]);
+        // the lowest expert index among the lanes that hold it (nearly always one)
+        unsigned long long holders = __builtin_amdgcn_ballot_w64(val[0] == bv);
         int bi = 0x7fffffff;
+        do {
+            bi = min(bi, __builtin_amdgcn_readlane(who[0], (int)__builtin_ctzll(holders)));
+            holders &= holders - 1;
+        } while (holders);
+        const bool mine = who[0] == bi;
 #pragma unroll
-        for (int i = PER - 1; i >= 0; --i) {
-            const unsigned long long holders =
-                __builtin_amdgcn_ballot_w64(lane + 64 * i < p.E && !((taken >> i) & 1u) && lg[i] == bv);
-            if (holders) bi = 64 * i + __builtin_ctzll(holders);
+        for (int i = 0; i + 1 < PER; ++i) {
+            const float a = val[i], b = val[i + 1];
+            const int wa = who[i], wb = who[i + 1];
+            val[i] = mine ? b : a;
+            who[i] = mine ? wb : wa;
         }
-        if ((bi & 63) == lane) taken |= 1u << (bi >> 6);
+        val[PER - 1] = mine ? -INFINITY : val[PER - 1];     // (an empty list loses every tie)
+        who[PER - 1] = mine ? 0x7fffffff : who[PER - 1];
         if (lane == j) { sel_logit = bv; sel_idx = bi; }
     }
     // lane j is wave-uniform here: v_readlane instead of a round trip through the LDS crossbar

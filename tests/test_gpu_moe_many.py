@@ -113,3 +113,23 @@ def test_problems_of_two_three_and_four_row_blocks(T, bits):
             assert ("exl3_gemm_mixed_kernel" in K.moe.last_launch()) == (big_min > 0), K.moe.last_launch()
             res.append(out)
     assert torch.equal(res[0], res[1])
+
+
+@pytest.mark.parametrize("T,H,E,k", [(3, 128, 128, 8), (2, 128, 300, 10), (5, 128, 512, 32), (2, 64, 1000, 9), (1, 64, 65, 3)])
+@pytest.mark.parametrize("finite", [0, 2, None])
+def test_choice_among_equal_and_minus_infinite_logits(T, H, E, k, finite):
+    """Columns repeat, so that the same logit stands in many lanes and several times in one lane; with a bias
+    of minus infinity fewer than k experts (or none at all) are left and the lowest of the others follow."""
+    x = synth.activations(T + E, T, H)
+    wr = synth.router_weight(E, H, E)[:, np.arange(E) * 7 % 11]
+    bias = None
+    if finite is not None:
+        bias = np.full(E, -np.inf, np.float32)
+        bias[E // 3:E // 3 + finite] = 0.25
+    idx, w, logits = _route(x, wr, k, bias=bias)
+    # the rule on the device's own logits: largest first, ties to the lowest index (a stable sort)
+    want = np.argsort(-logits, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(idx, want)
+    if finite != 0:
+        oi, ow = O.moe_route(x, wr, k, bias=bias)
+        assert np.array_equal(idx, oi) and np.allclose(w, ow, rtol=1e-5, atol=1e-7)
