@@ -541,6 +541,147 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
     if (p.sort.perm) route_sort_one_token(p.sort, lane, sel);
 }
 
+// The same routing with the fma chains on the matrix units: sixteen tokens x a slab of 16 or 32 experts
+// per workgroup.  v_mfma_f32_16x16x4_f32 adds its four products one after the other with an fma each
+// (compared on the device with chains of fmaf over 64 rows of fp16 values and down to denormal
+// products), so the bits are those of the other forms.
+//
+// What bounds the form above is one compute unit's path to its L2: a workgroup reads 128 columns of the
+// router weight, 512 KB at H = 2048, at some 65 GB/s, and converts them row by row on the vector pipe.
+// Here sixteen tokens share what is read and a slab is a quarter as wide or less.  Wave w takes segments
+// w and w + 16 of every 32; their weights are requested at once, ahead of the token rows, which go
+// through LDS (lanes that read sixteen rows from memory cost an address cycle each).  Step i of a segment
+// multiplies its rows 4 i .. 4 i + 3: lane 16 q + j holds row 4 i + q, of token j and of expert j, or of
+// experts 2 j and 2 j + 1 with a tile each for the even and the odd ones.
+constexpr int kTileTokens = 16, kTileSegs = 32;
+constexpr int kTileXStride = kTileSegs * kRouteSeg + 8;             // halves; sixteen rows' same columns in different banks
+inline __host__ __device__ constexpr int route_tile_lds_bytes(int experts)
+{
+    return kTileSegs * kTileTokens * experts * 4 + kTileTokens * kTileXStride * 2;
+}
+
+template <int TOKENS, int EXPERTS>
+__global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
+{
+    static_assert(TOKENS == kTileTokens && (EXPERTS == 16 || EXPERTS == 32), "tiles of sixteen");
+    extern __shared__ __align__(16) float s_parts[];               // [kTileSegs][16][EXPERTS], then the token rows
+    __shared__ unsigned s_last;
+    _Float16* const s_x = (_Float16*)(s_parts + kTileSegs * TOKENS * EXPERTS);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 15, q = lane >> 4;
+    const int grp = blockIdx.x, slab = blockIdx.y, nslab = gridDim.y;
+    const int t0 = grp * TOKENS, e0 = slab * EXPERTS;
+    // (tokens and experts past the end: the last ones again, unused)
+    const int e_pair = e0 + (EXPERTS == 32 ? 2 * j : j & ~1);
+    const uint32_t w_off = ((uint32_t)q * (uint32_t)p.E + (uint32_t)min(e_pair, p.E - 2)) * 2;
+    uint32_t w[2][16];          // two experts' weights of row 4 i + q, for each of the wave's two segments
+    auto load_w = [&](int seg, uint32_t (&dst)[16]) {
+        const char* src = (const char*)p.wr + (size_t)min(seg, p.nseg - 1) * kRouteSeg * p.E * 2;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dst[i] = *(global_ptr<const uint32_t>)(as_global(src + (size_t)i * 8 * p.E) + w_off);
+    };
+    // a wave brings in one token's columns of 32 segments, 1 KB at a time (columns past the end: the last ones)
+    const uint32_t x_row = (uint32_t)min(t0 + wave, p.T - 1) * (uint32_t)p.H * 2;
+    half8_t x[4];
+    auto load_x = [&](int s0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t col = (uint32_t)min(s0 * kRouteSeg + i * 512 + 8 * lane, p.H - 8);
+            x[i] = *(global_ptr<const half8_t>)(as_global((const char*)p.x) + x_row + 2 * col);
+        }
+    };
+    auto store_x = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *(half8_t*)(s_x + wave * kTileXStride + i * 512 + 8 * lane) = x[i];
+    };
+    const int shift = (q & 1) * 16;
+    auto run = [&](int at, const uint32_t (&wv)[16]) {
+        const uint4* const xs = (const uint4*)(s_x + j * kTileXStride + at * kRouteSeg);
+        float4_t even = {0.0f, 0.0f, 0.0f, 0.0f}, odd = even;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const uint4 xd = xs[i >> 1];
+            const uint32_t lo = i & 1 ? xd.z : xd.x, hi = i & 1 ? xd.w : xd.y;
+            const float xa = (float)as_half2((q & 2 ? hi : lo) >> shift).x;
+            if constexpr (EXPERTS == 32) {
+                even = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, (float)as_half2(wv[i]).x, even, 0, 0, 0);
+                odd = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, (float)as_half2(wv[i]).y, odd, 0, 0, 0);
+            } else {
+                even = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, (float)as_half2(wv[i] >> ((j & 1) * 16)).x, even, 0, 0, 0);
+            }
+        }
+        float* const dst = s_parts + (size_t)at * (TOKENS * EXPERTS) + 4 * q * EXPERTS + (EXPERTS / 16) * j;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (EXPERTS == 32) *(float2_t*)(dst + r * EXPERTS) = float2_t{even[r], odd[r]};
+            else dst[r * EXPERTS] = even[r];
+        }
+    };
+    // thread (token, expert) of the ordered sum; its bias is asked for now
+    const int tt = threadIdx.x / EXPERTS, c = threadIdx.x % EXPERTS;
+    const bool mine = tt < TOKENS && t0 + tt < p.T && e0 + c < p.E;
+    const float bias = mine && p.bias ? p.bias[e0 + c] : 0.0f;
+    float v = 0.0f;
+    load_x(0);
+    load_w(wave, w[0]);
+    load_w(wave + 16, w[1]);
+    for (int s0 = 0; s0 < p.nseg; s0 += kTileSegs) {
+        const bool more = s0 + kTileSegs < p.nseg;
+        store_x();
+        __syncthreads();
+        run(wave, w[0]);
+        if (more) load_w(s0 + kTileSegs + wave, w[0]);
+        run(wave + 16, w[1]);
+        if (more) {
+            load_w(s0 + kTileSegs + wave + 16, w[1]);
+            load_x(s0 + kTileSegs);
+        }
+        __syncthreads();
+        if (mine) v = route_add_segments(v, s_parts + threadIdx.x, TOKENS * EXPERTS, min(kTileSegs, p.nseg - s0));
+        if (more) __syncthreads();                                  // the sums have been read
+    }
+    if (p.bias) v += bias;
+    if (mine && p.logits) p.logits[(size_t)(t0 + tt) * p.E + e0 + c] = v;
+
+    // ---- logits to memory ([T][E], the head of the segment-sum scratch); the last slab of the token
+    // group to arrive selects, a wave per token
+    if (nslab > 1) {
+        if (mine)
+            __hip_atomic_store(p.parts + (size_t)(t0 + tt) * p.E + e0 + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        wait_own_stores();
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            unsigned* counter = p.counters + (size_t)grp * kRouteCounterStride;
+            const unsigned old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_last = (old == (unsigned)(nslab - 1)) ? 1u : 0u;
+            if (s_last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (!s_last) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    } else {
+        __syncthreads();                                            // every sum is formed: the segment sums can go
+        if (mine) s_parts[threadIdx.x] = v;
+        __syncthreads();
+    }
+    const int t = t0 + wave;
+    if (t >= p.T) return;
+    float lg[kRoutePer];
+#pragma unroll
+    for (int i = 0; i < kRoutePer; ++i) {
+        const int e = lane + 64 * i;
+        lg[i] = -INFINITY;
+        if (nslab > 1) {
+            if (e < p.E) lg[i] = __hip_atomic_load(p.parts + (size_t)t * p.E + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (i == 0 && lane < min(EXPERTS, p.E)) {
+            lg[i] = s_parts[wave * EXPERTS + lane];
+        }
+    }
+    route_topk(lg, lane, p, t);
+}
+
 // ---------------------------------------------------------------- permute
 
 
@@ -1040,6 +1181,30 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
         // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 13, 20 and
         // 30 us), so the count with the fewest whole rounds of the chip wins.  1500 tokens x 128 experts:
         // six tokens in one round of 250 workgroups 30 us, four in 375 39.5.
+        // More than 128 experts and passes of 32 segments that are nearly full: tiles of sixteen tokens, with
+        // slabs of 16 experts where that is one round of the chip.  us, slabs of 128 -> tiles: H = 2048, 512
+        // experts at 16 / 64 / 256 / 1500 tokens 13.4 / 14.9 / 20.2 / 82.2 -> 12.4 / 13.2 / 16.0 / 62.7; a
+        // short pass does not pay for the hand-over of the narrower slabs (H = 1024, 512 experts at 64 / 1500
+        // tokens 11.6 / 48.7 -> 12.9 / 56.9), up to 128 experts need none without (9.4 at 64 tokens).
+        const long tile_groups = (T + kTileTokens - 1) / kTileTokens;
+        const int tile_experts = tile_groups * ((E + 15) / 16) <= ws.cu_count ? 16 : 32;
+        const long tile_slabs = (E + tile_experts - 1) / tile_experts;
+        const int tile_segs = (p.nseg + kTileSegs - 1) / kTileSegs * kTileSegs;
+        if (T > 1 && E > kSlabExperts && p.nseg >= kTileSegs && tile_segs * 8 <= p.nseg * 9 && (uintptr_t)x % 16 == 0 &&
+            tile_groups * kRouteCounterStride <= kCounters) {
+            const dim3 grid((unsigned)tile_groups, (unsigned)tile_slabs);
+            const int lds = route_tile_lds_bytes(tile_experts);
+            auto launch = [&](void (*kernel)(RouteParams), bool (&raised)[64]) {
+                raise_dynamic_lds_limit((const void*)kernel, lds, raised, "moe_route_slab_kernel shared-memory attribute");
+                hipLaunchKernelGGL(kernel, grid, dim3(1024), lds, stream, p);
+            };
+            static bool raised[2][64] = {};
+            if (tile_experts == 16) launch(moe_route_slab_kernel<kTileTokens, 16>, raised[0]);
+            else launch(moe_route_slab_kernel<kTileTokens, 32>, raised[1]);
+            hip_ok(hipGetLastError(), "moe_route_slab_kernel launch");
+            return "moe_route_slab_kernel<" + std::to_string(kTileTokens) + "," + std::to_string(tile_experts) + "> grid=" +
+                   std::to_string(tile_slabs) + "x" + std::to_string(tile_groups);
+        }
         const int nslab = (E + kSlabExperts - 1) / kSlabExperts;
         constexpr int kSlabLdsMax = 144 * 1024;
         int tt = 1;

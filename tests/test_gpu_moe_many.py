@@ -133,3 +133,19 @@ def test_choice_among_equal_and_minus_infinite_logits(T, H, E, k, finite):
     if finite != 0:
         oi, ow = O.moe_route(x, wr, k, bias=bias)
         assert np.array_equal(idx, oi) and np.allclose(w, ow, rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("T,H,E,k,experts", [(2, 2048, 130, 3, 16), (17, 2048, 512, 10, 16), (33, 4032, 194, 6, 16), (31, 6144, 1000, 8, 16),
+                                             (270, 2048, 512, 10, 32), (513, 2048, 142, 4, 32)])
+def test_routing_tiles_of_sixteen_tokens(T, H, E, k, experts):
+    """Ragged token groups and slabs, a last pass with one segment missing, three passes: the oracle's bits."""
+    x, wr = synth.activations(T, T, H), synth.router_weight(E, H, E)
+    bias = synth.zipf_bias(5, E) if E % 4 == 0 else None
+    idx, w, logits = _route(x, wr, k, bias=bias)
+    assert "moe_route_slab_kernel<16," in K.moe.last_launch(), K.moe.last_launch()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert f"moe_route_slab_kernel<16,{experts}>" in K.moe.last_launch(), K.moe.last_launch()
+    oi, ow, ol = O.moe_route(x, wr, k, bias=bias, want_logits=True)
+    assert np.array_equal(logits.view(np.uint32), ol.view(np.uint32))
+    assert np.array_equal(idx, oi)
+    assert np.allclose(w, ow, rtol=1e-5, atol=1e-7)
