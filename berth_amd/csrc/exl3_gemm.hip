@@ -597,6 +597,7 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
     p.spin_limit = spin_limit();
     p.a_had[0] = (const _Float16*)g.a_had;
     p.a_had[1] = (const _Float16*)g.a_had2;
+    p.a_rows = g.a_rows;
     p.c[0] = g.c0;
     p.c[1] = g.c1;
     p.M = 0;

@@ -54,6 +54,7 @@ struct GemmParams {
     const ExpertLin* experts;
     const GroupProblem* problems;
     const int* num_problems;
+    const int32_t* a_rows;      // optional: where row r of the sorted order lies in a_had (rows of the always-on expert: at r)
     int lins_per_expert, lin_base;
     ExpertLin shared[3];        // an always-on expert passed by value (problem.expert == shared_expert)
     int shared_expert;
@@ -208,6 +209,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     const _Float16* a_had = p.a_had[0];
     void* cout = p.c[0];
     int N = p.N, ldc = p.N, nblk_lin = nblk;
+    const int32_t* a_rows = nullptr;
     if constexpr (DENSE) {
         const TileView v = dense_tile_view(p, nblk);
         if (v.empty) return;                            // the same for every workgroup that shares the tile
@@ -229,7 +231,10 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         m_end = gp.row0 + gp.nrows;
         a_had = p.a_had[which];
         cout = p.c[which];
+        if (gp.expert != p.shared_expert) a_rows = p.a_rows;
     }
+    // row r of the tile in a_had
+    auto a_row_at = [&](int r) { return !DENSE && a_rows ? as_global(a_rows)[m0 + r] : m0 + r; };
     const int rows_here = min(BM, m_end - m0);          // >= 1
     const int nw = n0 + wave * 64;                      // first column of this wave
     const bool active = nw < N;
@@ -256,7 +261,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         if (active && kr.kb0 < kr.kb1) {
             const global_ptr<const uint32_t> tb = as_global(lin.trellis) + (size_t)half_id * row_dw +
                                                  (size_t)((nw >> 4) + (slot >> 3)) * tile_dw + (slot & 7) * BITS;
-            const int arow = m0 + min(slot, rows_here - 1);         // rows past the problem repeat its last row
+            const int arow = a_row_at(min(slot, rows_here - 1));    // rows past the problem repeat its last row
             const global_ptr<const half8_t> ab =
                 (global_ptr<const half8_t>)(as_global(a_had) + (size_t)arow * p.K + 16 * half_id);
             uint32_t cur[4][BITS];
@@ -324,14 +329,19 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         uint32_t ring[4][BITS];
         u32x4_t a_nxt[kAPasses][2];
         const int a_row = threadIdx.x >> 3, a_ch = threadIdx.x & 7;       // + 32 rows per pass
+        int a_at[kAPasses];
+        if constexpr (!DENSE) {
+    #pragma unroll
+            for (int ps = 0; ps < kAPasses; ++ps) a_at[ps] = a_row_at(min(a_row + 32 * ps, rows_here - 1));
+        }
         auto load_a = [&](int kb) {
     #pragma unroll
             for (int ps = 0; ps < kAPasses; ++ps) {
                 const int r = a_row + 32 * ps;
                 u32x4_t v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
                 if (m0 + r < m_end) {
-                    const global_ptr<const u32x4_t> src =
-                        (global_ptr<const u32x4_t>)(as_global(a_had) + (size_t)(m0 + r) * p.K + kb * 128 + a_ch * 16);
+                    const global_ptr<const u32x4_t> src = (global_ptr<const u32x4_t>)(
+                        as_global(a_had) + (size_t)(DENSE ? m0 + r : a_at[ps]) * p.K + kb * 128 + a_ch * 16);
                     v0 = src[0];
                     v1 = src[1];
                 }

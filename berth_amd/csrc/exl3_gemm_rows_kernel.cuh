@@ -58,7 +58,8 @@ struct RowsGroupBlock {
     const _Float16* svh;
     const _Float16* a_had;
     void* c;
-    int rows, pad;
+    int rows;
+    uint32_t row_at[16];        // byte offset of each of its rows (past the last: the last) in a_had
 };
 __host__ __device__ constexpr size_t rows_group_lds_bytes(int rows, int ncb)
 {
@@ -177,14 +178,18 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
             const GroupProblem gp = p.problems[prob];
             const ExpertLin lin = gp.expert == p.shared_expert ? p.shared[p.lin_base + which]
                                                                : p.experts[gp.expert * p.lins_per_expert + p.lin_base + which];
-            RowsGroupBlock g;
+            RowsGroupBlock& g = table[threadIdx.x];
             g.trellis = lin.trellis;
             g.svh = lin.svh;
-            g.a_had = p.a_had[which] + (size_t)gp.row0 * p.K;
+            g.a_had = p.a_had[which];
             g.c = (char*)p.c[which] + (size_t)gp.row0 * p.N * (p.out_fp32 ? 4 : 2);
             g.rows = gp.nrows;
-            g.pad = 0;
-            table[threadIdx.x] = g;
+        }
+        if (threadIdx.x < 16 * ncb) {
+            const GroupProblem gp = p.problems[div_exact(cb_first + (threadIdx.x >> 4), p.m_rt)];
+            const int r = gp.row0 + min((int)threadIdx.x & 15, gp.nrows - 1);
+            const int at = p.a_rows && gp.expert != p.shared_expert ? p.a_rows[r] : r;
+            table[threadIdx.x >> 4].row_at[threadIdx.x & 15] = (uint32_t)at * (uint32_t)p.K * 2;
         }
         __syncthreads();
     }
@@ -219,7 +224,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     constexpr int kNextA = GROUPED ? 1 : 64;            // from a lane's operand to its next, in 16 bytes
     auto seek = [&](unsigned cb, unsigned k) {
         const RowsBlock b = block(cb);
-        if constexpr (GROUPED) a_off = (uint32_t)min(l16, b.rows - 1) * (uint32_t)p.K * 2 + (uint32_t)lg * 32;
+        if constexpr (GROUPED) a_off = table[cb - cb_first].row_at[l16] + (uint32_t)lg * 32;
         if (b.empty) {                                  // read anything valid, use nothing
             f_t = (const char*)rows_uniform(b.a_had);
             f_step = 0;

@@ -699,9 +699,9 @@ constexpr int kPermuteWaves = 16;
 inline unsigned permute_workgroups(long P) { return (unsigned)std::max(1l, std::min((long)kPermuteWaves, P / 512)); }
 inline size_t permute_lds_bytes(int E) { return (size_t)kPermuteWaves * E * sizeof(int); }
 
-__global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(PermuteParams p)
+// workgroup `block` of `blocks`; hist: dynamic LDS, [wave][E]: counts, then the next free row
+__device__ __forceinline__ void permute_pairs(const PermuteParams& p, const int block, const int blocks, int* hist)
 {
-    extern __shared__ __align__(16) int hist[];             // [wave][E]: counts, then the next free row
     __shared__ int tot[kMaxExperts + 1];                    // rows per expert
     __shared__ int off[kMaxExperts + 2];                    // first sorted row of each expert
     __shared__ int pfirst[kMaxExperts + 2];                 // first (small or VALU) problem of each expert
@@ -776,7 +776,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(Permute
             pfirst[tid] = (int)((excl >> 22) & 0x1fffffu);
             bfirst[tid] = (int)(excl >> 43);
         }
-        if (tid == E1 - 1 && blockIdx.x == 0) {
+        if (tid == E1 - 1 && block == 0) {
             const unsigned long long all = excl + mine;
             const int total_small = (int)((all >> 22) & 0x1fffffu);
             p.counts[0] = p.use_valu ? total_small : 0;
@@ -785,10 +785,10 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(Permute
         }
     }
     __syncthreads();
-    if (blockIdx.x == 0) {
+    if (block == 0) {
         for (int x = tid; x <= p.E; x += 1024) p.offsets[x] = x < E1 ? off[x] : P;
     }
-    if (tid < E1 && blockIdx.x == 0) {
+    if (tid < E1 && block == 0) {
         const int m = tot[tid];
         if (m > 0) {
             if (p.use_valu) {
@@ -803,13 +803,13 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(Permute
         }
     }
 
-    if (p.shared_rows && blockIdx.x == 0) {
+    if (p.shared_rows && block == 0) {
         for (int t = tid; t < p.T; t += 1024) {
             p.perm[P + t] = t * p.k;
             p.row_expert[P + t] = p.E;
         }
     }
-    if (wave % (int)gridDim.x != (int)blockIdx.x) return;
+    if (wave % blocks != block) return;
     static_assert(kMaxExperts == 1 << 10, "ten bits of an expert's number");
     const unsigned long long below = (1ull << lane) - 1ull;
     for (int q0 = q_begin; q0 < q_end; q0 += 64 * kAhead) {
@@ -841,6 +841,12 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(Permute
     }
 }
 
+__global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(PermuteParams p)
+{
+    extern __shared__ __align__(16) int hist[];
+    permute_pairs(p, (int)blockIdx.x, (int)gridDim.x, hist);
+}
+
 // ------------------------------------- rotated inputs for the MFMA problems
 
 struct HadRowsParams {
@@ -849,6 +855,8 @@ struct HadRowsParams {
     const int32_t* gather;      // source row = gather[r] / gather_div, or r
     int gather_div;
     const int32_t* row_expert;
+    int pairs;                  // > 0: row r < pairs is the (token, slot) pair r, of token r / gather_div; row pairs + t is token t's
+                                // for the always-on expert, which row_expert does not list
     const ExpertLin* experts;
     ExpertLin shared[3];        // the always-on expert (row_expert == shared_expert)
     int shared_expert;
@@ -865,18 +873,18 @@ struct HadRowsParams {
 // with a thread per linear, which walks the chain row -> expert -> pointer -> scales twice; two rows
 // per lane group 33.0), 2816 rows 10.3 us (13).
 template <int LINS>
-__global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
+__device__ __forceinline__ void had_row_item(const HadRowsParams& p, const int first)
 {
     const int lane = threadIdx.x & 63;
     const int nkb = p.K >> 7;
     const int total = p.P * nkb;
-    const int first = blockIdx.x * 16 + (threadIdx.x >> 4);
     const bool live = first < total;
     const int item = live ? first : total - 1;              // groups past the end redo the last item, store nothing
     const int row = item / nkb;
     const int at = (item - row * nkb) * 128 + 8 * had_chunk(lane);
-    const int ex = p.row_expert[row];
-    const int src = p.gather ? p.gather[row] / p.gather_div : row;
+    const bool always_on = p.pairs > 0 && row >= p.pairs;
+    const int ex = always_on ? p.shared_expert : p.row_expert[row];
+    const int src = always_on ? row - p.pairs : p.pairs > 0 ? row / p.gather_div : p.gather ? p.gather[row] / p.gather_div : row;
     half8_t sc[LINS];
 #pragma unroll
     for (int l = 0; l < LINS; ++l) {
@@ -900,6 +908,25 @@ __global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
         for (int i = 0; i < 8; ++i) o[i] = (_Float16)had_scale(v[i], unit);
         if (live) *(half8_t*)(p.out[l] + (size_t)row * p.K + at) = o;
     }
+}
+
+template <int LINS>
+__global__ __launch_bounds__(256) void moe_had_rows_kernel(HadRowsParams p)
+{
+    had_row_item<LINS>(p, (int)blockIdx.x * 16 + (int)(threadIdx.x >> 4));
+}
+
+// The permutation and the rotated rows of gate and up in one launch: the rows are left in the order of
+// the pairs (the products find theirs through `perm`), so neither waits for the other.  The first
+// perm_blocks workgroups sort, the others rotate 64 items each.
+// The two launches of 5.2 + 5.2 us (64 tokens x 8), 6.4 + 10.6 (256 x 10 of 512) and 11.0 + 33.5 (1500 x 8)
+// are one of 5.9, 10.9 and 29.7; reading the rows through `perm` costs the products nothing (a problem's
+// rows lie 2 K bytes apart either way).
+__global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_rotate_kernel(PermuteParams p, HadRowsParams h, int perm_blocks)
+{
+    extern __shared__ __align__(16) int hist[];
+    if ((int)blockIdx.x < perm_blocks) permute_pairs(p, (int)blockIdx.x, perm_blocks, hist);
+    else had_row_item<2>(h, ((int)blockIdx.x - perm_blocks) * 64 + (int)(threadIdx.x >> 4));
 }
 
 inline void launch_had_rows(const HadRowsParams& h, hipStream_t stream)
@@ -1292,6 +1319,19 @@ std::string run_permute(const PermuteParams& p, hipStream_t stream)
     return "moe_permute_kernel";
 }
 
+std::string run_permute_rotate(const PermuteParams& p, const HadRowsParams& h, hipStream_t stream)
+{
+    static bool raised[64] = {};
+    raise_dynamic_lds_limit((const void*)moe_permute_rotate_kernel, (int)permute_lds_bytes(kMaxExperts), raised,
+                            "moe_permute_rotate_kernel shared-memory attribute");
+    const long items = (long)h.P * (h.K >> 7);
+    const unsigned sort = permute_workgroups((long)p.T * p.k);
+    hipLaunchKernelGGL(moe_permute_rotate_kernel, dim3(sort + (unsigned)((items + 63) / 64)), dim3(64 * kPermuteWaves),
+                       permute_lds_bytes(p.E), stream, p, h, (int)sort);
+    hip_ok(hipGetLastError(), "moe_permute_rotate_kernel launch");
+    return "moe_permute_rotate_kernel";
+}
+
 }  // namespace
 }  // namespace berth
 
@@ -1554,7 +1594,27 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         desc += "moe_route_segments_kernel grid=" + std::to_string(L.nseg) + " (top-k and sort inside the next launch)";
     } else {
         desc += run_route(x, wr, bias, idx, w, nullptr, (float*)(wsb + L.parts), T, H, E, k, renorm, stream, &pp, idx_out, w_out);
-        if (T > 1) desc += " + " + run_permute(pp, stream);
+        if (L.max_m > 0) {
+            // the rotated rows of gate and up: row r is pair r, then the tokens themselves for the always-on expert
+            HadRowsParams h{};
+            h.a = (const _Float16*)x;
+            h.pairs = P;
+            h.gather_div = k;
+            h.row_expert = idx;
+            h.experts = (const ExpertLin*)experts;
+            h.shared_expert = fold ? E : -1;
+            if (fold) for (int i = 0; i < 3; ++i) h.shared[i] = ExpertLin{(const uint32_t*)shared[i].trellis, (const _Float16*)shared[i].suh, (const _Float16*)shared[i].svh};
+            h.lins_per_expert = 3;
+            h.lin_base = 0;
+            h.out[0] = (_Float16*)(wsb + L.ah0);
+            h.out[1] = (_Float16*)(wsb + L.ah1);
+            h.P = R;
+            h.K = H;
+            h.num_lins = 2;
+            desc += " + " + run_permute_rotate(pp, h, stream);
+        } else if (T > 1) {
+            desc += " + " + run_permute(pp, stream);
+        }
     }
 
     GroupedArgs g{};
@@ -1593,25 +1653,9 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.resolved_out = nullptr;
     }
     if (L.max_m > 0) {
-        HadRowsParams h{};
-        h.a = (const _Float16*)x;
-        h.gather = (const int32_t*)(wsb + L.perm);
-        h.gather_div = k;
-        h.row_expert = (const int32_t*)(wsb + L.row_expert);
-        h.experts = (const ExpertLin*)experts;
-        h.shared_expert = g.shared_expert;
-        if (fold) for (int i = 0; i < 3; ++i) h.shared[i] = ExpertLin{(const uint32_t*)shared[i].trellis, (const _Float16*)shared[i].suh, (const _Float16*)shared[i].svh};
-        h.lins_per_expert = 3;
-        h.lin_base = 0;
-        h.out[0] = (_Float16*)(wsb + L.ah0);
-        h.out[1] = (_Float16*)(wsb + L.ah1);
-        h.P = R;
-        h.K = H;
-        h.num_lins = 2;
-        launch_had_rows(h, stream);
         g.a_had = wsb + L.ah0;
         g.a_had2 = wsb + L.ah1;
-        desc += " + moe_had_rows_kernel";
+        g.a_rows = (const int32_t*)(wsb + L.perm);
         if (L.max_b > 0) {
             g.big_problems = wsb + L.bprob;
             g.num_big = (const int*)(wsb + L.counts) + 2;
@@ -1708,6 +1752,7 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         launch_had_rows(h, stream);
         g.a_had = wsb + L.ahd;
         g.a_had2 = nullptr;
+        g.a_rows = nullptr;
         desc += " + moe_had_rows_kernel";
         if (L.max_b > 0) {
             g.big_problems = wsb + L.bprob;

@@ -12,6 +12,7 @@ from berth_amd.device import Gpu
 from berth_amd.moe import MoeLayer
 from oracle import oracle as O
 from tests.gpu_util import DEV, dev, knobs
+import tests.test_gpu_moe as stages
 from tests.test_gpu_moe import _check_stages, _make_layer, _route
 
 pytestmark = pytest.mark.gpu
@@ -149,3 +150,13 @@ def test_routing_tiles_of_sixteen_tokens(T, H, E, k, experts):
     assert np.array_equal(logits.view(np.uint32), ol.view(np.uint32))
     assert np.array_equal(idx, oi)
     assert np.allclose(w, ow, rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("T,H,E,k,I,bits", [
+    (12, 256, 5, 3, 384, 4),         # problems of sixteen rows
+    (40, 384, 3, 2, 128, 5),         # of 32 rows, a last one of fewer
+    (200, 256, 6, 2, 128, 3),        # of two to four row blocks, and the rest of 32
+])
+def test_rows_found_through_the_permutation(T, H, E, k, I, bits):
+    """The layer leaves the rotated rows in the order of the pairs, the stages on their own in sorted order."""
+    stages.test_stage_entry_points_compose_to_the_layer(T, H, E, k, I, bits)
