@@ -630,6 +630,17 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
             return desc + " grouped";
         }
     }
+    if (g.act_had && g.num_lins == 2 && mb == 1 && g.max_big == 0 &&
+        gemm_split(ws, (long)g.max_problems * (g.size_n / 128), g.size_k / 128, 1) == 1) {
+        // whole K in every workgroup: gate, up and the next rotation together
+        if (g.max_problems > 65535) throw std::runtime_error("moe grouped linear: too many problems");
+        p.act_had = (_Float16*)g.act_had;
+        std::string desc;
+        gemm_bits(p, g.k_bits, g.codebook, -4, g.stream, desc, dim3(g.size_n / 128, g.max_problems));
+        hip_ok(hipGetLastError(), "exl3_gemm_pair_kernel launch");
+        *g.act_done = true;
+        return desc + " grouped";
+    }
     const int nblocks = (g.size_n + 255) / 256;
     const long tiles = (long)g.max_problems * g.num_lins * nblocks;
     p.cstride = gemm_counter_stride(tiles);

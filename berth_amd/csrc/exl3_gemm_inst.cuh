@@ -67,6 +67,16 @@ static void gemm_launch_mixed(const GemmParams& p, hipStream_t stream, std::stri
            std::to_string(grid.z - p.max_big) + ") smem=" + std::to_string(smem);
 }
 
+// gate and up of a problem list, and the down projection's rotated input; mb = -4
+template <int BITS, int CB>
+static void gemm_launch_pair(const GemmParams& p, hipStream_t stream, std::string& desc, dim3 grid)
+{
+    const size_t smem = (size_t)32 * (256 + 4) * sizeof(float);
+    hipLaunchKernelGGL((exl3_gemm_pair_kernel<BITS, CB>), grid, dim3(256), smem, stream, p);
+    desc = "exl3_gemm_pair_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + ",32x(128+128)> grid=" +
+           std::to_string(grid.x) + "x" + std::to_string(grid.y) + " smem=" + std::to_string(smem);
+}
+
 // few rows (2..32), units dealt out evenly; mb = -1 / -2: one or two tiles of 16 rows, -3: a list of
 // problems of up to 16 rows
 template <int BITS, int CB, int MT, bool GROUPED = false>
@@ -101,6 +111,7 @@ static void gemm_launch(const GemmParams& p, int mb, hipStream_t stream, std::st
     else if (mb == -1) gemm_launch_rows<BITS, CB, 1>(p, stream, desc, grid);
     else if (mb == -2) gemm_launch_rows<BITS, CB, 2>(p, stream, desc, grid);
     else if (mb == -3) gemm_launch_rows<BITS, CB, 1, true>(p, stream, desc, grid);
+    else if (mb == -4) gemm_launch_pair<BITS, CB>(p, stream, desc, grid);
     else if (mb == -12) gemm_launch_block<BITS, CB, 4>(p, stream, desc, grid);
     else if (mb == -14) gemm_launch_block<BITS, CB, 6>(p, stream, desc, grid);
     else if (mb == -16) gemm_launch_block<BITS, CB, 8>(p, stream, desc, grid);

@@ -27,6 +27,7 @@
 #pragma once
 
 #include "exl3_gemv_kernel.cuh"
+#include "silu.cuh"
 
 namespace berth {
 
@@ -55,6 +56,7 @@ struct GemmParams {
     const GroupProblem* problems;
     const int* num_problems;
     const int32_t* a_rows;      // optional: where row r of the sorted order lies in a_had (rows of the always-on expert: at r)
+    _Float16* act_had;          // exl3_gemm_pair_kernel: the down projection's rotated input, in sorted order
     int lins_per_expert, lin_base;
     ExpertLin shared[3];        // an always-on expert passed by value (problem.expert == shared_expert)
     int shared_expert;
@@ -188,6 +190,67 @@ constexpr int kGemmWrittenBase = 32768;   // second half of the counter table: "
 
 constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: conflict-free b128 reads)
 
+// The k-loop of a 32-row tile, 64 columns from nw on: every wave is on its own.  The A operand of a lane (row
+// `slot`, 8 k values) is one 16-byte load straight from the rotated rows, so
+// there is no LDS tile and no barrier in the loop.  Trellis and A registers are
+// reloaded for the wave's next k-block as soon as a step has consumed them
+// (rolling prefetch, one k-block ahead); on the last k-block the reload reads
+// the same addresses again and is ignored, which keeps the loop free of branches.
+template <int BITS, int CB>
+__device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
+                                                   const int arow, const int K, const int kb0, const int kb1, const int step,
+                                                   const int lane, float16_t (&acc)[2])
+{
+    constexpr int tile_dw = 8 * BITS;
+    const int half_id = lane >> 5, slot = lane & 31;
+    const global_ptr<const uint32_t> tb = as_global(trellis) + (size_t)half_id * row_dw +
+                                         (size_t)((nw >> 4) + (slot >> 3)) * tile_dw + (slot & 7) * BITS;
+    const global_ptr<const half8_t> ab =
+        (global_ptr<const half8_t>)(as_global(a_had) + (size_t)arow * K + 16 * half_id);
+    uint32_t cur[4][BITS];
+    half8_t av[4][2];
+    {
+        const global_ptr<const uint32_t> t0 = tb + (size_t)(kb0 * 8) * row_dw;
+        const global_ptr<const half8_t> a0 = ab + kb0 * 16;
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            load_tile_dwords<BITS>(t0 + (size_t)(2 * st) * row_dw, cur[st]);
+            av[st][0] = a0[4 * st];
+            av[st][1] = a0[4 * st + 1];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    for (int kb = kb0; kb < kb1; kb += step) {
+        const int nkb = kb + step < kb1 ? kb + step : kb;
+        const global_ptr<const uint32_t> tnx = tb + (size_t)(nkb * 8) * row_dw;
+        const global_ptr<const half8_t> anx = ab + nkb * 16;
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            uint32_t prev = fetch_prev(lane, cur[st][BITS - 1]);
+            uint32_t w2[16];
+            decode_lane<BITS, CB>(cur[st], prev, w2);
+            load_tile_dwords<BITS>(tnx + (size_t)(2 * st) * row_dw, cur[st]);
+            half8_t b[2][2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint4 q = {w2[2 * f + h], w2[4 + 2 * f + h], w2[8 + 2 * f + h], w2[12 + 2 * f + h]};
+                    b[f][h] = __builtin_bit_cast(half8_t, q);
+                }
+            settle<CB>(b[0][0], b[1][0], b[0][1], b[1][1]);
+            const half8_t a0 = av[st][0], a1 = av[st][1];
+            av[st][0] = anx[4 * st];
+            av[st][1] = anx[4 * st + 1];
+            __builtin_amdgcn_sched_barrier(0);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b[0][0], acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b[1][0], acc[1], 0, 0, 0);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b[0][1], acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b[1][1], acc[1], 0, 0, 0);
+        }
+    }
+}
+
 // one output tile: rows of problem / row block `tile_y`, 256 columns
 template <int BITS, int CB, int MB, bool DENSE>  // MB = 32-row blocks per workgroup; DENSE: never a problem list
 __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y, const int nblk, const KRange kr,
@@ -252,61 +315,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
             for (int r = 0; r < 16; ++r) acc[mb][f][r] = 0.0f;
 
     if constexpr (MB == 1) {
-        // ---- 32-row tile: every wave is on its own.  The A operand of a lane (row
-        // `slot`, 8 k values) is one 16-byte load straight from the rotated rows, so
-        // there is no LDS tile and no barrier in the loop.  Trellis and A registers are
-        // reloaded for the wave's next k-block as soon as a step has consumed them
-        // (rolling prefetch, one k-block ahead); on the last k-block the reload reads
-        // the same addresses again and is ignored, which keeps the loop free of branches.
-        if (active && kr.kb0 < kr.kb1) {
-            const global_ptr<const uint32_t> tb = as_global(lin.trellis) + (size_t)half_id * row_dw +
-                                                 (size_t)((nw >> 4) + (slot >> 3)) * tile_dw + (slot & 7) * BITS;
-            const int arow = a_row_at(min(slot, rows_here - 1));    // rows past the problem repeat its last row
-            const global_ptr<const half8_t> ab =
-                (global_ptr<const half8_t>)(as_global(a_had) + (size_t)arow * p.K + 16 * half_id);
-            uint32_t cur[4][BITS];
-            half8_t av[4][2];
-            {
-                const global_ptr<const uint32_t> t0 = tb + (size_t)(kr.kb0 * 8) * row_dw;
-                const global_ptr<const half8_t> a0 = ab + kr.kb0 * 16;
-#pragma unroll
-                for (int st = 0; st < 4; ++st) {
-                    load_tile_dwords<BITS>(t0 + (size_t)(2 * st) * row_dw, cur[st]);
-                    av[st][0] = a0[4 * st];
-                    av[st][1] = a0[4 * st + 1];
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            for (int kb = kr.kb0; kb < kr.kb1; kb += kr.step) {
-                const int nkb = kb + kr.step < kr.kb1 ? kb + kr.step : kb;
-                const global_ptr<const uint32_t> tnx = tb + (size_t)(nkb * 8) * row_dw;
-                const global_ptr<const half8_t> anx = ab + nkb * 16;
-#pragma unroll
-                for (int st = 0; st < 4; ++st) {
-                    uint32_t prev = fetch_prev(lane, cur[st][BITS - 1]);
-                    uint32_t w2[16];
-                    decode_lane<BITS, CB>(cur[st], prev, w2);
-                    load_tile_dwords<BITS>(tnx + (size_t)(2 * st) * row_dw, cur[st]);
-                    half8_t b[2][2];
-#pragma unroll
-                    for (int f = 0; f < 2; ++f)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const uint4 q = {w2[2 * f + h], w2[4 + 2 * f + h], w2[8 + 2 * f + h], w2[12 + 2 * f + h]};
-                            b[f][h] = __builtin_bit_cast(half8_t, q);
-                        }
-                    settle<CB>(b[0][0], b[1][0], b[0][1], b[1][1]);
-                    const half8_t a0 = av[st][0], a1 = av[st][1];
-                    av[st][0] = anx[4 * st];
-                    av[st][1] = anx[4 * st + 1];
-                    __builtin_amdgcn_sched_barrier(0);
-                    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b[0][0], acc[0][0], 0, 0, 0);
-                    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b[1][0], acc[0][1], 0, 0, 0);
-                    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b[0][1], acc[0][0], 0, 0, 0);
-                    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b[1][1], acc[0][1], 0, 0, 0);
-                }
-            }
-        }
+        if (active && kr.kb0 < kr.kb1)
+            accumulate_32_rows<BITS, CB>(lin.trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
+                                         kr.step, lane, acc[0]);      // (rows past the problem repeat its last row)
     } else {
         // lane's trellis position inside a k-block: tile row 2*step + half_id, tile (nw/16 + slot/8)
         const uint32_t* tbase = lin.trellis + (size_t)half_id * row_dw +
@@ -637,6 +648,84 @@ __global__ __launch_bounds__(256, MB == 1 ? 3 : 2) void exl3_gemm_kernel(GemmPar
     kr.counter = ((size_t)blockIdx.y * p.tiles_y + blockIdx.z) * nblocks + unit;
     kr.slot0 = kr.slot_rest = kr.counter * p.S;
     gemm_tile<BITS, CB, MB, false>(p, blockIdx.z, unit, kr, blockIdx.y, smem, p.problems);
+}
+
+// Gate and up of a list of problems of up to 32 rows, and the input of their down projections: waves 0
+// and 1 take 128 columns of gate, waves 2 and 3 the same columns of up, so that the workgroup holds both
+// factors of silu(g) * u and a whole block of the next rotation when its k-loops end.  blockIdx.x =
+// column block, blockIdx.y the problem; linears lin_base, lin_base + 1 and, for its input scales,
+// lin_base + 2 of an expert.  Gate and up are written too (fp16, c[0] and c[1]).
+// The values are those of the 32-row tiles and of moe_had_rows_kernel behind them.
+// What bounds it: the decode, as there; the end of a row is three rotations (of 128 values by sixteen
+// lanes) instead of two, against a launch that reads both factors back: layer of 64 tokens x 128 experts
+// x 768 122.6 -> 121.4 us, of 20 tokens x 128 experts x 896 (seven column blocks, which 256-column tiles
+// cover as eight) 107 -> 94.
+template <int BITS, int CB>
+__global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    if ((int)blockIdx.y >= *p.num_problems) return;
+    constexpr int kZStride = 256 + 4;
+    float* const z_tile = (float*)smem;                 // [32][kZStride]: gate's 128 columns, up's
+    const int lane = threadIdx.x & 63, slot = lane & 31, half_id = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int which = wave >> 1;
+    const int n0 = (int)blockIdx.x * 128;
+    const GroupProblem gp = p.problems[blockIdx.y];
+    const bool shared = gp.expert == p.shared_expert;
+    auto linear = [&](int l) { return shared ? p.shared[p.lin_base + l] : p.experts[gp.expert * p.lins_per_expert + p.lin_base + l]; };
+    const ExpertLin lin = linear(which);
+    const int rows = gp.nrows;
+    int arow = gp.row0 + min(slot, rows - 1);           // rows past the problem repeat its last row
+    if (p.a_rows && !shared) arow = as_global(p.a_rows)[arow];
+
+    float16_t acc[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[f][r] = 0.0f;
+    accumulate_32_rows<BITS, CB>(lin.trellis, (size_t)(p.N >> 4) * (8 * BITS), n0 + (wave & 1) * 64, p.a_had[which], arow, p.K, 0,
+                                 p.K >> 7, 1, lane, acc);
+
+    // sixteen lanes a row, eight columns of both factors each
+    const int at = n0 + 8 * had_chunk(lane);
+    half8_t sv[2];
+#pragma unroll
+    for (int l = 0; l < 2; ++l) sv[l] = *(global_ptr<const half8_t>)(as_global(linear(l).svh) + at);
+    const half8_t su = *(global_ptr<const half8_t>)(as_global(linear(2).suh) + at);
+    const int col = wave * 64 + (slot >> 3) * 16 + (slot & 7);
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z_tile[(8 * (r >> 2) + 4 * half_id + (r & 3)) * kZStride + col + 8 * f] = acc[f][r];
+    __syncthreads();
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+        const int row = pass * 16 + wave * 4 + (lane >> 4);
+        if (row >= rows) break;
+        const size_t out = (size_t)(gp.row0 + row) * p.N + at;
+        half8_t gu[2];
+#pragma unroll
+        for (int l = 0; l < 2; ++l) {
+            const float4_t* const zp = (const float4_t*)&z_tile[row * kZStride + l * 128 + (at - n0)];
+            const float4_t z0 = zp[0], z1 = zp[1];
+            float v[8] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
+            const float unit = had128_row16(v, lane) * kRsqrt128;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) gu[l][i] = (_Float16)rounded(had_scale(v[i], unit) * (float)sv[l][i]);
+            *(global_ptr<half8_t>)(as_global((_Float16*)p.c[l]) + out) = gu[l];
+        }
+        half8_t x;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = silu_mul_h(gu[0][i], gu[1][i]);
+        float v[8];
+        mul_half8(x, su, v);
+        const float unit = had128_row16(v, lane) * kRsqrt128;
+        half8_t o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = (_Float16)had_scale(v[i], unit);
+        *(global_ptr<half8_t>)(as_global(p.act_had) + out) = o;
+    }
 }
 
 // Grouped launch over two problem lists at once: blockIdx.z < max_big takes a problem of up

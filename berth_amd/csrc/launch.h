@@ -199,6 +199,10 @@ struct GroupedArgs {
     const void* a_had;          // MFMA path: rotated input rows [rows][K] of the first linear
     const void* a_had2;         // ... and of the second linear of the launch
     const int32_t* a_rows = nullptr;    // optional: sorted row r is row a_rows[r] of a_had (the always-on expert's rows stay)
+    // MFMA path, two linears, optional: where the rotated input of the expert's next linear goes
+    // (silu(c0) * c1 under its scales, [rows][size_n] in sorted order); *act_done says whether the launch wrote it
+    void* act_had = nullptr;
+    bool* act_done = nullptr;
     int size_k, size_n, k_bits, codebook, out_fp32;
     hipStream_t stream;
     // VALU path, single_row, one linear, fp32 out, silu input: also combine the

@@ -1652,6 +1652,7 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.route_params = nullptr;
         g.resolved_out = nullptr;
     }
+    bool act_done = false;      // the rotated input of the down projections is there already
     if (L.max_m > 0) {
         g.a_had = wsb + L.ah0;
         g.a_had2 = wsb + L.ah1;
@@ -1666,7 +1667,10 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.max_problems = L.max_m;
         g.mb = 1;
         g.small_rows = L.small_rows < kGemmRows ? L.small_rows : 0;
+        g.act_had = wsb + L.ahd;
+        g.act_done = &act_done;
         desc += " + " + launch_gemm_grouped(g);
+        g.act_had = nullptr;
     }
 
     // shared expert: three dense linears on every token (ahead of the routed down
@@ -1735,25 +1739,27 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.resolved = nullptr;
     }
     if (L.max_m > 0) {
-        HadRowsParams h{};
-        h.a = (const _Float16*)(wsb + L.g);
-        h.a_up = (const _Float16*)(wsb + L.u);
-        h.gather_div = 1;
-        h.row_expert = (const int32_t*)(wsb + L.row_expert);
-        h.experts = (const ExpertLin*)experts;
-        h.shared_expert = g.shared_expert;
-        if (fold) for (int i = 0; i < 3; ++i) h.shared[i] = ExpertLin{(const uint32_t*)shared[i].trellis, (const _Float16*)shared[i].suh, (const _Float16*)shared[i].svh};
-        h.lins_per_expert = 3;
-        h.lin_base = 2;
-        h.out[0] = (_Float16*)(wsb + L.ahd);
-        h.P = R;
-        h.K = I;
-        h.num_lins = 1;
-        launch_had_rows(h, stream);
+        if (!act_done) {
+            HadRowsParams h{};
+            h.a = (const _Float16*)(wsb + L.g);
+            h.a_up = (const _Float16*)(wsb + L.u);
+            h.gather_div = 1;
+            h.row_expert = (const int32_t*)(wsb + L.row_expert);
+            h.experts = (const ExpertLin*)experts;
+            h.shared_expert = g.shared_expert;
+            if (fold) for (int i = 0; i < 3; ++i) h.shared[i] = ExpertLin{(const uint32_t*)shared[i].trellis, (const _Float16*)shared[i].suh, (const _Float16*)shared[i].svh};
+            h.lins_per_expert = 3;
+            h.lin_base = 2;
+            h.out[0] = (_Float16*)(wsb + L.ahd);
+            h.P = R;
+            h.K = I;
+            h.num_lins = 1;
+            launch_had_rows(h, stream);
+            desc += " + moe_had_rows_kernel";
+        }
         g.a_had = wsb + L.ahd;
         g.a_had2 = nullptr;
         g.a_rows = nullptr;
-        desc += " + moe_had_rows_kernel";
         if (L.max_b > 0) {
             g.big_problems = wsb + L.bprob;
             g.num_big = (const int*)(wsb + L.counts) + 2;

@@ -160,3 +160,29 @@ def test_routing_tiles_of_sixteen_tokens(T, H, E, k, experts):
 def test_rows_found_through_the_permutation(T, H, E, k, I, bits):
     """The layer leaves the rotated rows in the order of the pairs, the stages on their own in sorted order."""
     stages.test_stage_entry_points_compose_to_the_layer(T, H, E, k, I, bits)
+
+
+@pytest.mark.parametrize("T,H,E,k,I,bits,shared_I", [
+    (17, 128, 40, 3, 128, 4, 0),        # one k-block, one column block
+    (70, 256, 2, 2, 384, 3, 384),       # experts with 32, 32 and 6 rows, the always-on one among them
+    (128, 384, 9, 1, 640, 6, 128),      # an always-on expert of another width
+    (33, 256, 64, 8, 256, 2, 0),
+])
+def test_gate_up_and_the_next_rotation_in_one_launch(T, H, E, k, I, bits, shared_I):
+    """17..128 tokens: every workgroup holds gate and up of its columns and leaves the down projection's rotated input."""
+    gpu = Gpu(0)
+    wr, experts_np, experts, shared_np, shared = _make_layer(gpu, 9500 + T + H, H, E, I, bits, shared_I, 10.0)
+    layer = MoeLayer(gpu, wr, experts, k, shared=shared)
+    x = (synth.activations(T + H, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
+    out, again = (torch.zeros((T, H), dtype=torch.float32, device=DEV) for _ in range(2))
+    idx = torch.zeros((T, k), dtype=torch.int32, device=DEV)
+    w = torch.zeros((T, k), dtype=torch.float32, device=DEV)
+    layer.forward(gpu, dev(x.view(np.uint16)), out, T, idx, w)
+    torch.cuda.synchronize()
+    assert "exl3_gemm_pair_kernel" in K.moe.last_launch() and "had_rows" not in K.moe.last_launch(), K.moe.last_launch()
+    want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, 2, shared=shared_np, shared_I=shared_I)
+    assert np.array_equal(idx.cpu().numpy(), oi)
+    _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I)
+    layer.forward(gpu, dev(x.view(np.uint16)), again, T)
+    torch.cuda.synchronize()
+    assert torch.equal(again, out)
