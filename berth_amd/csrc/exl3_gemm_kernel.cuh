@@ -196,10 +196,11 @@ constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: 
 // reloaded for the wave's next k-block as soon as a step has consumed them
 // (rolling prefetch, one k-block ahead); on the last k-block the reload reads
 // the same addresses again and is ignored, which keeps the loop free of branches.
-template <int BITS, int CB>
+// `requested` is called when the first loads are on their way.
+template <int BITS, int CB, typename F>
 __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
                                                    const int arow, const int K, const int kb0, const int kb1, const int step,
-                                                   const int lane, float16_t (&acc)[2])
+                                                   const int lane, float16_t (&acc)[2], F requested)
 {
     constexpr int tile_dw = 8 * BITS;
     const int half_id = lane >> 5, slot = lane & 31;
@@ -220,6 +221,7 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+    requested();
     for (int kb = kb0; kb < kb1; kb += step) {
         const int nkb = kb + step < kb1 ? kb + step : kb;
         const global_ptr<const uint32_t> tnx = tb + (size_t)(nkb * 8) * row_dw;
@@ -305,6 +307,16 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     constexpr int tile_dw = 8 * BITS;
     const size_t row_dw = (size_t)tn * tile_dw;
     const int KB = p.K >> 7;
+    // The output scales of the tile, eight columns a thread: asked for ahead of the operands and kept in LDS.
+    // They come from memory, and the end of the tile waited for them: layer of 64 tokens x 128 experts 121.4 ->
+    // 119.5 us, whose workgroups all end together.
+    __shared__ __align__(16) half8_t s_scale[32];
+    half8_t scale_mine = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (threadIdx.x < 32 && n0 + 8 * (int)threadIdx.x < N)
+        scale_mine = ((global_ptr<const half8_t>)as_global(lin.svh + n0))[threadIdx.x];
+    auto keep_scale = [&]() {
+        if (threadIdx.x < 32) s_scale[threadIdx.x] = scale_mine;
+    };
 
     float16_t acc[MB][2];
 #pragma unroll
@@ -317,7 +329,8 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     if constexpr (MB == 1) {
         if (active && kr.kb0 < kr.kb1)
             accumulate_32_rows<BITS, CB>(lin.trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
-                                         kr.step, lane, acc[0]);      // (rows past the problem repeat its last row)
+                                         kr.step, lane, acc[0], keep_scale);      // (rows past the problem repeat its last row)
+        else keep_scale();
     } else {
         // lane's trellis position inside a k-block: tile row 2*step + half_id, tile (nw/16 + slot/8)
         const uint32_t* tbase = lin.trellis + (size_t)half_id * row_dw +
@@ -386,6 +399,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
                 settle<CB>(b_half[0][0]);
             }
         }
+        keep_scale();
 
         int buf = 0;
         for (int kb = kr.kb0; kb < kr.kb1; kb += kr.step, buf ^= 1) {
@@ -554,12 +568,6 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     const int col_in_wave = (slot >> 3) * 16 + (slot & 7);     // + 8f
     // output scales: a lane of the epilogue owns columns 8 * had_chunk(lane) .. + 7 of a block
     const int chunk = had_chunk(lane);
-    half8_t sv_blk[2];
-#pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-        const int gn = n0 + blk * 128;
-        sv_blk[blk] = gn < N ? ((global_ptr<const half8_t>)as_global(lin.svh + gn))[chunk] : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         if (mb * 32 >= rows_here) break;                        // workgroup-uniform
@@ -588,7 +596,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 #pragma unroll
                 for (int i = 0; i < 4; ++i) { v[i] = z0[i]; v[4 + i] = z1[i]; }
                 const float unit = had128_row16(v, lane) * kRsqrt128;
-                const half8_t sv = blk ? sv_blk[1] : sv_blk[0];
+                const half8_t sv = s_scale[blk * 16 + chunk];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = had_scale(v[i], unit) * (float)sv[i];
                 const size_t at = (size_t)(m0 + mb * 32 + row) * ldc + gn + 8 * chunk;
@@ -679,20 +687,26 @@ __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
     int arow = gp.row0 + min(slot, rows - 1);           // rows past the problem repeat its last row
     if (p.a_rows && !shared) arow = as_global(p.a_rows)[arow];
 
+    // the output scales of gate and up, the input scales of down: asked for first, as in gemm_tile
+    __shared__ __align__(16) half8_t s_scale[3][16];
+    half8_t scale_mine = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (threadIdx.x < 48) {
+        const ExpertLin l = linear((int)threadIdx.x >> 4);
+        scale_mine = ((global_ptr<const half8_t>)as_global((threadIdx.x < 32 ? l.svh : l.suh) + n0))[threadIdx.x & 15];
+    }
     float16_t acc[2];
 #pragma unroll
     for (int f = 0; f < 2; ++f)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[f][r] = 0.0f;
     accumulate_32_rows<BITS, CB>(lin.trellis, (size_t)(p.N >> 4) * (8 * BITS), n0 + (wave & 1) * 64, p.a_had[which], arow, p.K, 0,
-                                 p.K >> 7, 1, lane, acc);
+                                 p.K >> 7, 1, lane, acc, [&]() {
+        if (threadIdx.x < 48) s_scale[threadIdx.x >> 4][threadIdx.x & 15] = scale_mine;
+    });
 
     // sixteen lanes a row, eight columns of both factors each
-    const int at = n0 + 8 * had_chunk(lane);
-    half8_t sv[2];
-#pragma unroll
-    for (int l = 0; l < 2; ++l) sv[l] = *(global_ptr<const half8_t>)(as_global(linear(l).svh) + at);
-    const half8_t su = *(global_ptr<const half8_t>)(as_global(linear(2).suh) + at);
+    const int chunk = had_chunk(lane);
+    const int at = n0 + 8 * chunk;
     const int col = wave * 64 + (slot >> 3) * 16 + (slot & 7);
 #pragma unroll
     for (int f = 0; f < 2; ++f)
@@ -712,14 +726,14 @@ __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
             float v[8] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
             const float unit = had128_row16(v, lane) * kRsqrt128;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) gu[l][i] = (_Float16)rounded(had_scale(v[i], unit) * (float)sv[l][i]);
+            for (int i = 0; i < 8; ++i) gu[l][i] = (_Float16)rounded(had_scale(v[i], unit) * (float)s_scale[l][chunk][i]);
             *(global_ptr<half8_t>)(as_global((_Float16*)p.c[l]) + out) = gu[l];
         }
         half8_t x;
 #pragma unroll
         for (int i = 0; i < 8; ++i) x[i] = silu_mul_h(gu[0][i], gu[1][i]);
         float v[8];
-        mul_half8(x, su, v);
+        mul_half8(x, s_scale[2][chunk], v);
         const float unit = had128_row16(v, lane) * kRsqrt128;
         half8_t o;
 #pragma unroll
