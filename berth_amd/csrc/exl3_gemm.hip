@@ -65,8 +65,9 @@ struct RowsPlan {
     int mt = 1;                 // tiles of 16 rows
     long units = 0;             // 64 x 128 weights each
     unsigned grid = 0, q = 0, rem = 0, S = 0;
-    size_t lds = 0;
+    size_t lds = 0, lds_rotate = 0;
     size_t operand_at = 0;      // bytes into the partial-sum workspace
+    bool rotate = false;        // the launch can rotate its input itself
 };
 
 static unsigned magic(unsigned d) { return d == 1 ? 0u : (unsigned)((1ull << 32) / d) + 1u; }
@@ -132,6 +133,12 @@ static RowsPlan plan_rows(const Workspace& ws, int slices, int slabs, int size_m
         pl.rem = rem;
         pl.S = S;
         pl.lds = lds;
+        if (S) {
+            unsigned nb = 0;                                        // most 128 blocks that a part touches
+            for (unsigned s = 0; s < S; ++s) nb = std::max(nb, ((s + 1) * TR4 / S + 1) / 2 - s * TR4 / S / 2);
+            pl.lds_rotate = lds + rows_rot_lds_bytes((int)(2 * nb), mt);
+            pl.rotate = nb * (unsigned)size_m <= (unsigned)(slabs > 1 ? kRowsRotItems : kRowsRotItems - 64) && pl.lds_rotate <= 160 * 1024;
+        }
         return pl;
     }
     return pl;
@@ -142,7 +149,8 @@ bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, 
     return plan_rows(ws, slices, slices, size_m, size_k, size_n).ok;
 }
 
-static void run_rows(const RowsPlan& pl, GemmParams& p, int k_bits, int codebook, hipStream_t stream, std::string& desc)
+// rotate: p is a GemmRotateParams
+static void run_rows(const RowsPlan& pl, GemmParams& p, bool rotate, int k_bits, int codebook, hipStream_t stream, std::string& desc)
 {
     p.cstride = gemm_counter_stride((long)(p.num_slices > 0 ? p.num_slices : 1) * (p.N / 128));
     p.units = (int)pl.units;
@@ -154,8 +162,9 @@ static void run_rows(const RowsPlan& pl, GemmParams& p, int k_bits, int codebook
     p.m_s = pl.S ? magic(pl.S) : 0;
     p.m_q = pl.S ? 0u : magic(pl.q);
     p.m_q1 = magic(pl.q + 1);
-    p.lds_bytes = (unsigned)pl.lds;
-    gemm_bits(p, k_bits, codebook, -pl.mt, stream, desc, dim3(pl.grid));
+    p.lds_bytes = (unsigned)(rotate ? pl.lds_rotate : pl.lds);
+    if (rotate) static_cast<GemmRotateParams&>(p).m_rows = magic((unsigned)p.M);
+    gemm_bits(p, k_bits, codebook, (rotate ? -4 : 0) - pl.mt, stream, desc, dim3(pl.grid));
     hip_ok(hipGetLastError(), "exl3_gemm_rows_kernel launch");
 }
 
@@ -268,9 +277,9 @@ struct OperandPlan {
     }
     bool ok() const { return rows.ok || block.ok; }
     int mt() const { return rows.ok ? rows.mt : block.rows_per_tile / 16; }
-    void run(GemmParams& p, int k_bits, int codebook, hipStream_t stream, std::string& desc) const
+    void run(GemmParams& p, bool rotate, int k_bits, int codebook, hipStream_t stream, std::string& desc) const
     {
-        if (rows.ok) run_rows(rows, p, k_bits, codebook, stream, desc);
+        if (rows.ok) run_rows(rows, p, rotate, k_bits, codebook, stream, desc);
         else run_block(block, p, k_bits, codebook, stream, desc);
     }
     _Float16* at = nullptr;     // the first slab's copy
@@ -367,6 +376,12 @@ static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int c
     hip_ok(hipGetLastError(), "exl3_gemm_kernel launch");
 }
 
+// whether two buffers do not overlap
+static bool apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes)
+{
+    return (uintptr_t)a + a_bytes <= (uintptr_t)b || (uintptr_t)b + b_bytes <= (uintptr_t)a;
+}
+
 std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
 {
     if (a.size_k % 128 != 0) throw std::runtime_error("exl3 linear: size_k must be a multiple of 128");
@@ -388,8 +403,17 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
         rot.operand = plan.at;
         rot.mt = plan.mt();
     }
-    std::string d0 = launch_rotate(rot);
-    GemmParams p{};
+    // (the rotation overlaps the reads of other workgroups then, and the output their reads of the input)
+    const bool rotate = plan.rows.ok && plan.rows.rotate && !a.a_up && !a.act_out &&
+                        apart(a.a, (size_t)a.size_m * a.size_k * 2, a.a_had, (size_t)a.size_m * a.size_k * 2) &&
+                        apart(a.a, (size_t)a.size_m * a.size_k * 2, a.c, (size_t)a.size_m * a.size_n * (a.out_fp32 ? 4 : 2));
+    std::string d0 = rotate ? "" : launch_rotate(rot) + " + ";
+    GemmRotateParams p{};
+    if (rotate) {
+        p.rot_in = (const _Float16*)a.a;
+        p.rot_out = (_Float16*)a.a_had;
+        p.lin.suh = (const _Float16*)a.suh;
+    }
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
     p.a_had[0] = (const _Float16*)(plan.ok() ? plan.at : a.a_had);
@@ -405,9 +429,9 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     p.partials = ws.partials;
     p.counters = ws.counters;
     std::string desc;
-    if (plan.ok()) plan.run(p, a.k_bits, a.codebook, a.stream, desc);
+    if (plan.ok()) plan.run(p, rotate, a.k_bits, a.codebook, a.stream, desc);
     else dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (a.size_n + 255) / 256, a.stream, desc);
-    return d0 + " + " + desc + (a.out_fp32 ? " out=f32" : " out=f16");
+    return d0 + desc + (a.out_fp32 ? " out=f32" : " out=f16");
 }
 
 // berth_ops_mgemm with more than 8 rows, or 2..8 of large weights: the bundle's linears on the MFMA kernels
@@ -426,7 +450,7 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
     // what the kernel multiplies: the rotated rows, or their copy in operand order
     const size_t slab_stride = plan.ok() ? plan.stride : (size_t)m.size_m * m.size_k;
     const _Float16* const slab0 = (const _Float16*)(plan.ok() ? plan.at : m.a_had);
-    GemmParams p{};
+    GemmRotateParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
     p.a_had[0] = slab0;
@@ -491,14 +515,45 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
         rot.operand = plan.at;
         rot.mt = plan.mt();
     }
-    std::string d0 = launch_rotate(rot);
+    const size_t rows_bytes = (size_t)m.size_m * m.size_k * 2;
+    // (More than 8 rows of a short K keep the launch that rotates: it is part of what is tested of such bundles.
+    // A decoder layer of 12 rows and 1024 columns would gain 1 us of 48.)
+    bool rotate = plan.rows.ok && plan.rows.rotate && (m.size_m <= 8 || m.size_k > 1024) &&
+                  apart(m.a, rows_bytes * (rot.in_stride ? slabs : 1), m.a_had, rows_bytes * slabs);
+    // (Lists in device memory cannot be looked at here: their outputs must not overlap the input, as for the
+    // dot-product kernel that bundles of smaller weights take.)
+    if (m.host_lists) {
+        bool used[kGemmMaxSlices] = {};
+        for (int i = 0; i < m.bszm_out; ++i) used[sliced ? m.had_src_list[i] : i] = true;
+        rotate = rotate && std::all_of(used, used + slabs, [](bool u) { return u; });       // every input is some slice's
+        for (int i = 0; i < m.bszm_out; ++i)
+            rotate = rotate && apart(m.a, rows_bytes * (rot.in_stride ? slabs : 1), p.slice[i].c,
+                                     ((size_t)(m.size_m - 1) * p.slice[i].n_stride + p.slice[i].width) * (m.c_fp32 ? 4 : 2));
+    }
+    if (rotate && m.host_lists) {
+        bool left[kGemmMaxSlices] = {};
+        for (int i = 0; i < m.bszm_out; ++i) {
+            const int src = sliced ? m.had_src_list[i] : i;
+            GemmRotation& g = p.rotation[i];
+            g.suh = (const _Float16*)suh_host[src];
+            g.in = (const _Float16*)m.a + (size_t)src * rot.in_stride;
+            g.had_out = left[src] ? nullptr : (_Float16*)m.a_had + (size_t)src * rot.out_stride;
+            left[src] = true;
+        }
+    } else if (rotate) {
+        p.rot_in = (const _Float16*)m.a;
+        p.rot_in_stride = rot.in_stride;
+        p.rot_out = (_Float16*)m.a_had;
+        p.suh_list = (const uint64_t*)m.suh_list;
+    }
+    std::string d0 = rotate ? "" : launch_rotate(rot) + " + ";
     const long nblocks = (long)m.bszm_out * ((m.size_n + 255) / 256);
     if (nblocks * ((m.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3_mgemm: too many output tiles");
     std::string desc;
-    if (plan.ok()) plan.run(p, m.k_bits, m.codebook, m.stream, desc);
+    if (plan.ok()) plan.run(p, rotate, m.k_bits, m.codebook, m.stream, desc);
     else dispatch_dense(ws, p, m.k_bits, m.codebook, m.size_m, m.size_k, (int)nblocks, m.stream, desc);
     return std::string(sliced ? "sliced x" : "uniform x") + std::to_string(m.bszm_out) + (m.host_lists ? " by value " : " ") + d0 +
-           " + " + desc + (m.c_fp32 ? " out=f32" : " out=f16");
+           desc + (m.c_fp32 ? " out=f32" : " out=f16");
 }
 
 std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
@@ -548,7 +603,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
     const long nblocks = 2L * ((a.size_n + 255) / 256);
     if (nblocks * ((a.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3 linear pair: too many output tiles");
     std::string desc;
-    if (plan.ok()) plan.run(p, a.k_bits, a.codebook, a.stream, desc);
+    if (plan.ok()) plan.run(p, false, a.k_bits, a.codebook, a.stream, desc);
     else dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (int)nblocks, a.stream, desc);
     return "pair " + d0 + " + " + desc + " out=f16";
 }
@@ -583,10 +638,11 @@ static GroupRowsPlan plan_group_rows(const Workspace& ws, const GroupedArgs& g)
     return pl;
 }
 
-// grouped: problems of at most 32 * g.mb rows each; a_had rows are in problem order
+// grouped: problems of at most 32 rows each (and, in a list of their own, of up to 128); a_had rows are in problem
+// order, or found through a_rows
 std::string launch_gemm_grouped(const GroupedArgs& g)
 {
-    const int mb = g.mb == 4 ? 4 : 1;
+    constexpr int mb = 1;
     if (g.size_k % 128 != 0 || g.size_n % 128 != 0)
         throw std::runtime_error("moe grouped linear: sizes must be multiples of 128");
     LaunchScope scope(g.stream);
@@ -630,7 +686,7 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
             return desc + " grouped";
         }
     }
-    if (g.act_had && g.num_lins == 2 && mb == 1 && g.max_big == 0 &&
+    if (g.act_had && g.num_lins == 2 && g.max_big == 0 &&
         gemm_split(ws, (long)g.max_problems * (g.size_n / 128), g.size_k / 128, 1) == 1) {
         // whole K in every workgroup: gate, up and the next rotation together
         if (g.max_problems > 65535) throw std::runtime_error("moe grouped linear: too many problems");

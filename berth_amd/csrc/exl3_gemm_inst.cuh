@@ -8,7 +8,7 @@
 
 namespace berth {
 
-template <int BITS, int CB, int MB>
+template <int BITS, int CB, int MB, bool DENSE>
 static void gemm_launch_mb(const GemmParams& p, hipStream_t stream, std::string& desc, dim3 grid)
 {
     constexpr int BM = MB * 32;
@@ -17,12 +17,12 @@ static void gemm_launch_mb(const GemmParams& p, hipStream_t stream, std::string&
     const size_t smem = smem_a > smem_z ? smem_a : smem_z;
     if (smem > 64 * 1024) {
         static bool raised[64] = {};
-        raise_dynamic_lds_limit((const void*)exl3_gemm_kernel<BITS, CB, MB>, (int)smem, raised,
+        raise_dynamic_lds_limit((const void*)exl3_gemm_kernel<BITS, CB, MB, DENSE>, (int)smem, raised,
                                 "exl3_gemm_kernel shared-memory attribute");
     }
     if (p.units > 0) {
         // dealt-out dense launch (128-row tiles only)
-        if constexpr (MB == 4) {
+        if constexpr (MB == 4 && DENSE) {
             static bool raised2[64] = {};
             raise_dynamic_lds_limit((const void*)exl3_gemm_balanced_kernel<BITS, CB, MB>, (int)smem, raised2,
                                     "exl3_gemm_balanced_kernel shared-memory attribute");
@@ -34,7 +34,7 @@ static void gemm_launch_mb(const GemmParams& p, hipStream_t stream, std::string&
         }
         throw std::runtime_error("exl3 gemm: balanced launches use 128-row tiles");
     }
-    hipLaunchKernelGGL((exl3_gemm_kernel<BITS, CB, MB>), grid, dim3(256), smem, stream, p);
+    hipLaunchKernelGGL((exl3_gemm_kernel<BITS, CB, MB, DENSE>), grid, dim3(256), smem, stream, p);
     desc = "exl3_gemm_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + "," + std::to_string(BM) +
            "x256> grid=" + std::to_string(grid.x) + "x" + std::to_string(grid.y) + "x" + std::to_string(grid.z) +
            " split_k=" + std::to_string(p.S) + " smem=" + std::to_string(smem);
@@ -77,17 +77,21 @@ static void gemm_launch_pair(const GemmParams& p, hipStream_t stream, std::strin
            std::to_string(grid.x) + "x" + std::to_string(grid.y) + " smem=" + std::to_string(smem);
 }
 
-// few rows (2..32), units dealt out evenly; mb = -1 / -2: one or two tiles of 16 rows, -3: a list of
-// problems of up to 16 rows
-template <int BITS, int CB, int MT, bool GROUPED = false>
+// few rows (2..32), units dealt out evenly; mb = -1 / -2: one or two tiles of 16 rows (-5 / -6: which the launch
+// rotates itself, p a GemmRotateParams), -3: a list of problems of up to 16 rows
+template <int BITS, int CB, int MT, bool GROUPED = false, bool ROT = false>
 static void gemm_launch_rows(const GemmParams& p, hipStream_t stream, std::string& desc, dim3 grid)
 {
     static bool raised[64] = {};
-    raise_dynamic_lds_limit((const void*)exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED>, 160 * 1024, raised,
+    raise_dynamic_lds_limit((const void*)exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT>, 160 * 1024, raised,
                             "exl3_gemm_rows_kernel shared-memory attribute");
-    hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED>), grid, dim3(1024), p.lds_bytes, stream, p);
+    if constexpr (ROT)
+        hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT>), grid, dim3(1024), p.lds_bytes, stream,
+                           static_cast<const GemmRotateParams&>(p));
+    else
+        hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT>), grid, dim3(1024), p.lds_bytes, stream, p);
     desc = "exl3_gemm_rows_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + "," + std::to_string(16 * MT) +
-           "x128> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
+           "x128" + (ROT ? ",rotate" : "") + "> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
            (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
 }
 
@@ -111,13 +115,18 @@ static void gemm_launch(const GemmParams& p, int mb, hipStream_t stream, std::st
     else if (mb == -1) gemm_launch_rows<BITS, CB, 1>(p, stream, desc, grid);
     else if (mb == -2) gemm_launch_rows<BITS, CB, 2>(p, stream, desc, grid);
     else if (mb == -3) gemm_launch_rows<BITS, CB, 1, true>(p, stream, desc, grid);
+    else if (mb == -5) gemm_launch_rows<BITS, CB, 1, false, true>(p, stream, desc, grid);
+    else if (mb == -6) gemm_launch_rows<BITS, CB, 2, false, true>(p, stream, desc, grid);
     else if (mb == -4) gemm_launch_pair<BITS, CB>(p, stream, desc, grid);
     else if (mb == -12) gemm_launch_block<BITS, CB, 4>(p, stream, desc, grid);
     else if (mb == -14) gemm_launch_block<BITS, CB, 6>(p, stream, desc, grid);
     else if (mb == -16) gemm_launch_block<BITS, CB, 8>(p, stream, desc, grid);
-    else if (mb == 1) gemm_launch_mb<BITS, CB, 1>(p, stream, desc, grid);
+    else if (p.problems) {
+        if (mb != 1) throw std::runtime_error("exl3 gemm: problem lists of 32-row tiles, alone or with 128-row ones");
+        gemm_launch_mb<BITS, CB, 1, false>(p, stream, desc, grid);
+    } else if (mb == 1) gemm_launch_mb<BITS, CB, 1, true>(p, stream, desc, grid);
     else if (mb == 8) gemm_launch_wide<BITS, CB>(p, stream, desc, grid);
-    else gemm_launch_mb<BITS, CB, 4>(p, stream, desc, grid);
+    else gemm_launch_mb<BITS, CB, 4, true>(p, stream, desc, grid);
 }
 
 #define BERTH_CAT2(a, b) a##b

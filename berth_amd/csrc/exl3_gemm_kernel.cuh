@@ -55,8 +55,6 @@ struct GemmParams {
     const ExpertLin* experts;
     const GroupProblem* problems;
     const int* num_problems;
-    const int32_t* a_rows;      // optional: where row r of the sorted order lies in a_had (rows of the always-on expert: at r)
-    _Float16* act_had;          // exl3_gemm_pair_kernel: the down projection's rotated input, in sorted order
     int lins_per_expert, lin_base;
     ExpertLin shared[3];        // an always-on expert passed by value (problem.expert == shared_expert)
     int shared_expert;
@@ -108,6 +106,26 @@ struct GemmParams {
     unsigned lds_bytes;         // dynamic LDS of the launch
     const float* out_add;       // optional fp32 [M][N] (one linear, fp32 output): added to the output
     GemmSlice slice[kGemmMaxSlices];
+    // grouped: where row r of the sorted order lies in a_had (optional; rows of the always-on expert: at r)
+    const int32_t* a_rows;
+    _Float16* act_had;          // exl3_gemm_pair_kernel: the down projection's rotated input, in sorted order
+};
+
+// Few-row launches that rotate the input themselves: where it comes from and where the rotated rows go, for
+// one linear and lists in device memory, or per slice.  (Arguments of their own: every launch copies its
+// arguments, and these are half a kilobyte.)
+struct GemmRotation {
+    const _Float16* suh;
+    const _Float16* in;
+    _Float16* had_out;          // null: another slice leaves them
+};
+struct GemmRotateParams : GemmParams {
+    const _Float16* rot_in;
+    _Float16* rot_out;          // [slab][M][K]
+    const uint64_t* suh_list;
+    size_t rot_in_stride;       // elements between the slabs' inputs (0: one for all)
+    unsigned m_rows;            // divides by M
+    GemmRotation rotation[kGemmMaxSlices];
 };
 
 // the tensors of the column block `nblk` of a dense launch
@@ -307,15 +325,16 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     constexpr int tile_dw = 8 * BITS;
     const size_t row_dw = (size_t)tn * tile_dw;
     const int KB = p.K >> 7;
-    // The output scales of the tile, eight columns a thread: asked for ahead of the operands and kept in LDS.
-    // They come from memory, and the end of the tile waited for them: layer of 64 tokens x 128 experts 121.4 ->
-    // 119.5 us, whose workgroups all end together.
+    // The output scales of a problem's tile, eight columns a thread: asked for ahead of the operands and kept in
+    // LDS.  They come from memory, and the end of the tile waited for them: layer of 64 tokens x 128 experts
+    // 121.4 -> 119.5 us, whose workgroups all end together.  (Dense tiles ask for them at the end: with
+    // few tiles a head that waits costs more, 76 rows of 1152x3584 15.0 -> 15.4 us, 317 of 2944x8320 47.5 -> 48.5.)
     __shared__ __align__(16) half8_t s_scale[32];
     half8_t scale_mine = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (threadIdx.x < 32 && n0 + 8 * (int)threadIdx.x < N)
+    if (!DENSE && threadIdx.x < 32 && n0 + 8 * (int)threadIdx.x < N)
         scale_mine = ((global_ptr<const half8_t>)as_global(lin.svh + n0))[threadIdx.x];
     auto keep_scale = [&]() {
-        if (threadIdx.x < 32) s_scale[threadIdx.x] = scale_mine;
+        if (!DENSE && threadIdx.x < 32) s_scale[threadIdx.x] = scale_mine;
     };
 
     float16_t acc[MB][2];
@@ -523,10 +542,10 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         if (active) {
             // part 0 first (from memory unless it is this workgroup's own), then parts 1, 2, ...
-            // added in order.  64 loads a lane are in
-            // flight at a time: half of a part's register blocks, or two whole parts.
+            // added in order.  64 (128-row tiles), 128 (32-row tiles) or, for problems, 64 loads a lane are in
+            // flight at a time: half of a part's register blocks, or four or two whole parts.
             constexpr int kGroup = MB & 1 ? 2 : 4;              // (mb, f) register blocks per batch
-            constexpr int kParts = MB == 1 ? 2 : 1;             // parts per batch
+            constexpr int kParts = MB > 1 ? 1 : DENSE ? 4 : 2;  // parts per batch
             const int first = kr.part == 0 ? 1 : 0;
             for (int j0 = first; j0 < kr.parts; j0 += kParts) {
 #pragma unroll
@@ -568,6 +587,14 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     const int col_in_wave = (slot >> 3) * 16 + (slot & 7);     // + 8f
     // output scales: a lane of the epilogue owns columns 8 * had_chunk(lane) .. + 7 of a block
     const int chunk = had_chunk(lane);
+    half8_t sv_blk[2];
+    if constexpr (DENSE) {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            const int gn = n0 + blk * 128;
+            sv_blk[blk] = gn < N ? ((global_ptr<const half8_t>)as_global(lin.svh + gn))[chunk] : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    }
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         if (mb * 32 >= rows_here) break;                        // workgroup-uniform
@@ -596,7 +623,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 #pragma unroll
                 for (int i = 0; i < 4; ++i) { v[i] = z0[i]; v[4 + i] = z1[i]; }
                 const float unit = had128_row16(v, lane) * kRsqrt128;
-                const half8_t sv = s_scale[blk * 16 + chunk];
+                const half8_t sv = !DENSE ? s_scale[blk * 16 + chunk] : blk ? sv_blk[1] : sv_blk[0];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = had_scale(v[i], unit) * (float)sv[i];
                 const size_t at = (size_t)(m0 + mb * 32 + row) * ldc + gn + 8 * chunk;
@@ -627,11 +654,11 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 // blockIdx.y the linear, blockIdx.z the problem, so that the workgroups of the (few)
 // real problems of every linear are dispatched before the empty tail of the list.
 //
-// 32-row tiles: up to four workgroups on a compute unit (126 registers a lane; with four parts in flight at
-// the end of a split tile it was 173 and two of them, so that the 756 workgroups of 64 tokens x 128
+// 32-row problems: up to four workgroups on a compute unit (with four parts in flight at the end of a
+// split tile it was 173 registers a lane and two of them, so that the 756 workgroups of 64 tokens x 128
 // experts ran in two rounds: layer 125.6 -> 122.6 us).
-template <int BITS, int CB, int MB>
-__global__ __launch_bounds__(256, MB == 1 ? 3 : 2) void exl3_gemm_kernel(GemmParams p)
+template <int BITS, int CB, int MB, bool DENSE = true>
+__global__ __launch_bounds__(256, MB == 1 && !DENSE ? 3 : 2) void exl3_gemm_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int unit = blockIdx.x / p.S;
@@ -644,18 +671,18 @@ __global__ __launch_bounds__(256, MB == 1 ? 3 : 2) void exl3_gemm_kernel(GemmPar
     kr.slot_step = 1;
     kr.part = split;
     kr.parts = p.S;
-    if (!p.problems) {
+    if constexpr (DENSE) {
         const int tile = p.tile0 + unit;
         kr.counter = (size_t)unit;
         kr.slot0 = kr.slot_rest = kr.counter * p.S;
         gemm_tile<BITS, CB, MB, true>(p, tile / nblocks, tile % nblocks, kr, 0, smem);
-        return;
+    } else {
+        if ((int)blockIdx.z >= *p.num_problems) return;
+        // grouped: (linear, problem, column block)
+        kr.counter = ((size_t)blockIdx.y * p.tiles_y + blockIdx.z) * nblocks + unit;
+        kr.slot0 = kr.slot_rest = kr.counter * p.S;
+        gemm_tile<BITS, CB, MB, false>(p, blockIdx.z, unit, kr, blockIdx.y, smem, p.problems);
     }
-    if ((int)blockIdx.z >= *p.num_problems) return;
-    // grouped: (linear, problem, column block)
-    kr.counter = ((size_t)blockIdx.y * p.tiles_y + blockIdx.z) * nblocks + unit;
-    kr.slot0 = kr.slot_rest = kr.counter * p.S;
-    gemm_tile<BITS, CB, MB, false>(p, blockIdx.z, unit, kr, blockIdx.y, smem, p.problems);
 }
 
 // Gate and up of a list of problems of up to 32 rows, and the input of their down projections: waves 0

@@ -1,7 +1,7 @@
 // EXL3 linear for a few rows (2..32): every weight is decoded once and multiplied on the matrix
 // units, as a single resident round of sixteen-wave workgroups.
 //
-//   c = Hh(a_had @ W) * svh (+ out_add),   a_had = Hh(a * suh) rotated by an earlier launch
+//   c = Hh(a_had @ W) * svh (+ out_add),   a_had = Hh(a * suh) rotated by an earlier launch, or by this one (ROT)
 //
 // What bounds it: the decode (about 4.0 vector instructions per weight, 124 for the 32 weights a
 // lane takes per step); the four v_mfma_f32_16x16x32_f16 of a step and 16 rows need 64 of the
@@ -41,11 +41,26 @@
 #pragma once
 
 #include "exl3_gemm_kernel.cuh"
+#include "rows_operand.cuh"
+
+#include <type_traits>
 
 namespace berth {
 
 constexpr int kRowsWaves = 16;
 constexpr int kRowsStride = 132;            // floats per row of a partial column block in LDS
+
+// Launches that rotate the input themselves (ROT): the most (row, 128 block) items a workgroup takes, sixteen
+// lanes each, and the LDS of their result, `units` units of 64 k behind everything else.  Where a column
+// block is cut into parts of its own, a workgroup needs a part of K only, so all workgroups of a part of
+// K rotating it cost less than the launch that did it once, as long as it is a few items a lane group:
+// linears of 5 / 8 / 14 / 24 rows, us, two launches -> one: 4096x4096 11.1 / 11.6 / 12.4 / 14.5 -> 9.3 / 9.8 / 10.5 /
+// 13.4 (40 .. 96 items), 6144x5120 13.2 / 13.4 / 14.3 / 16.5 -> 11.2 / 11.5 / 13.1 / 15.8 (40 .. 192),
+// 17408x5120 20.8 / 20.8 -> 19.2 / 19.8 (115, 184); 196 items (10240x5120 at 14) 17.0 -> 17.1.  A fourth item a
+// lane group is worth it for bundles, whose launch for the rotation has several inputs (q, k and v of 24
+// rows, 240 items: a layer 115.5 -> 113.9).
+constexpr int kRowsRotItems = 256;
+__host__ __device__ constexpr size_t rows_rot_lds_bytes(int units, int mt) { return (size_t)units * mt * 2048; }
 
 // dynamic LDS of a launch: the pieces, the output scales of the column blocks, two flags
 __host__ __device__ constexpr size_t rows_lds_bytes(int rows, int ncb)
@@ -123,6 +138,23 @@ __device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsig
     return b;
 }
 
+// the input of the column block `cb`, its scales and, for one column block per input, where its rotated rows go
+__device__ __forceinline__ GemmRotation rows_rotation(const GemmRotateParams& p, const unsigned cb)
+{
+    if (p.num_slices == 0) return {p.lin.suh, p.rot_in, cb == 0 ? p.rot_out : nullptr};
+    const unsigned sl = div_exact(cb, p.m_nb);
+    const bool first = cb == sl * ((unsigned)p.N >> 7);
+    if (!p.b_list) {
+        const GemmRotation& r = p.rotation[sl];
+        return {r.suh, r.in, first ? r.had_out : nullptr};
+    }
+    const unsigned slab = p.c_ptrs ? (unsigned)p.had_src_list[sl] : sl;
+    // (slices of one input that are not neighbours: each of them leaves it, the same values)
+    const bool leaves = first && (sl == 0 || !p.c_ptrs || (unsigned)p.had_src_list[sl - 1] != slab);
+    return {(const _Float16*)p.suh_list[slab], p.rot_in + (size_t)slab * p.rot_in_stride,
+            leaves ? p.rot_out + (size_t)slab * p.M * p.K : nullptr};
+}
+
 template <typename T>
 __device__ __forceinline__ const T* rows_uniform(const T* q)
 {
@@ -132,9 +164,10 @@ __device__ __forceinline__ const T* rows_uniform(const T* q)
     return (const T*)(((uint64_t)hi << 32) | lo);
 }
 
-template <int BITS, int CB, int MT, bool GROUPED>       // MT: tiles of 16 rows
-__global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
+template <int BITS, int CB, int MT, bool GROUPED, bool ROT = false>     // MT: tiles of 16 rows
+__global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditional_t<ROT, GemmRotateParams, GemmParams> p)
 {
+    static_assert(!GROUPED || !ROT, "a problem list brings its rows rotated");
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int tile_dw = 8 * BITS;
     const int lane = threadIdx.x & 63;
@@ -221,12 +254,17 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     uint32_t t_off;                                     // bytes, per lane
     uint32_t a_off = (uint32_t)lane * 16;
     constexpr int kUnitA = GROUPED ? 128 : MT * 2 * 1024;   // bytes of A operands per unit (GROUPED: of one row)
+    // ROT: a workgroup's units lie in one column block; the 128 blocks of its rows' input that they need
+    const unsigned rot0 = (u0 - cb_first * TR4) & ~1u;          // first unit in LDS
+    unsigned char* const rot_lds = (unsigned char*)(flags + 4);
+    uint32_t f_lds = 0;                                         // this wave's next unit in it
     constexpr int kNextA = GROUPED ? 1 : 64;            // from a lane's operand to its next, in 16 bytes
     auto seek = [&](unsigned cb, unsigned k) {
         const RowsBlock b = block(cb);
         if constexpr (GROUPED) a_off = table[cb - cb_first].row_at[l16] + (uint32_t)lg * 32;
         if (b.empty) {                                  // read anything valid, use nothing
-            f_t = (const char*)rows_uniform(b.a_had);
+            if constexpr (ROT) f_t = (const char*)rows_uniform(rows_rotation(p, cb).in);
+            else f_t = (const char*)rows_uniform(b.a_had);
             f_step = 0;
             t_off = 0;
         } else {
@@ -235,7 +273,8 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
             f_t = (const char*)rows_uniform(b.trellis) + (size_t)(b.n0 >> 4) * (tile_dw * 4) + (size_t)(4 * k) * row_bytes;
             t_off = (uint32_t)lg * row_bytes + (uint32_t)(cg * 16 + l16) * (BITS * 4);
         }
-        f_a = (const char*)rows_uniform(b.a_had) + (size_t)k * kUnitA;
+        if constexpr (ROT) f_lds = (k - rot0) * (uint32_t)kUnitA;
+        else f_a = (const char*)rows_uniform(b.a_had) + (size_t)k * kUnitA;
     };
     seek(f_cb, f_k);
 
@@ -243,17 +282,30 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
     half8_t av[2][MT][2];
     auto fetch_t = [&](int j) { load_tile_dwords<BITS>((global_ptr<const uint32_t>)(as_global(f_t) + t_off), own[j]); };
     auto fetch_a = [&](int j) {
-        const global_ptr<const half8_t> src = (global_ptr<const half8_t>)(as_global(f_a) + a_off);
+        if constexpr (ROT) {
+            const half8_t* const src = (const half8_t*)(rot_lds + f_lds + a_off);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            av[j][mt][0] = src[(2 * mt) * kNextA];
-            av[j][mt][1] = src[(2 * mt + 1) * kNextA];
+            for (int mt = 0; mt < MT; ++mt) {
+                av[j][mt][0] = src[(2 * mt) * kNextA];
+                av[j][mt][1] = src[(2 * mt + 1) * kNextA];
+            }
+        } else {
+            const global_ptr<const half8_t> src = (global_ptr<const half8_t>)(as_global(f_a) + a_off);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                av[j][mt][0] = src[(2 * mt) * kNextA];
+                av[j][mt][1] = src[(2 * mt + 1) * kNextA];
+            }
         }
     };
     auto advance = [&]() {                              // on the last unit it stays: read again, not used
         if (f_left > 1) {
             --f_left;
             f_t += f_step;
+            if constexpr (ROT) {                        // (all units in one column block)
+                f_lds += kUnitA;
+                return;
+            }
             f_a += kUnitA;
             if (++f_k == TR4) {
                 f_k = 0;
@@ -262,11 +314,57 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
             }
         }
     };
+    if constexpr (ROT) {
+        // The rows' part of the input, rotated into LDS in operand order: all of its loads at once, behind
+        // the first weights of the wave.
+        const GemmRotation r = rows_rotation(p, cb_first);
+        const unsigned nb = ((u1 - cb_first * TR4 + 1) >> 1) - (rot0 >> 1);
+        const unsigned items = nb * (unsigned)M;
+        const int chunk = had_chunk(lane);
+        const uint32_t col0 = rot0 * 64 + 8 * (uint32_t)chunk;
+        half8_t x[kRowsRotItems / 64], sc[kRowsRotItems / 64];
+        unsigned row[kRowsRotItems / 64], blk[kRowsRotItems / 64];
+        const global_ptr<const _Float16> in = as_global(rows_uniform(r.in)), suh = as_global(rows_uniform(r.suh));
+        fetch_t(0);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        fetch_t(j);
-        fetch_a(j);
+        for (int i = 0; i < kRowsRotItems / 64; ++i) {
+            const unsigned it = min(threadIdx.x / 16 + 64u * i, items - 1);     // (past the end: the last one, stored again)
+            blk[i] = div_exact(it, p.m_rows);
+            row[i] = it - blk[i] * (unsigned)M;
+            if (64u * i < items) {                                              // workgroup-uniform
+                x[i] = *(global_ptr<const half8_t>)(in + (size_t)row[i] * p.K + col0 + 128 * blk[i]);
+                sc[i] = *(global_ptr<const half8_t>)(suh + col0 + 128 * blk[i]);
+            }
+        }
+        const unsigned left = f_left;
         advance();
+        fetch_t(1);
+#pragma unroll
+        for (int i = 0; i < kRowsRotItems / 64; ++i) {
+            if (64u * i >= items) break;
+            float v[8];
+            mul_half8(x[i], sc[i], v);
+            const float unit = had128_row16(v, lane) * kRsqrt128;
+            half8_t o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = (_Float16)had_scale(v[e], unit);
+            const uint32_t unit_at = 2 * blk[i] + ((uint32_t)chunk >> 3);
+            *(half8_t*)(rot_lds + unit_at * (uint32_t)kUnitA + 2 * rows_operand_offset((int)row[i], 8 * (chunk & 7), MT)) = o;
+            if (r.had_out) *(global_ptr<half8_t>)(as_global(r.had_out) + (size_t)row[i] * p.K + col0 + 128 * blk[i]) = o;
+        }
+        __syncthreads();
+        f_lds -= left > 1 ? kUnitA : 0;
+        fetch_a(0);
+        f_lds += left > 1 ? kUnitA : 0;
+        fetch_a(1);
+        advance();
+    } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            fetch_t(j);
+            fetch_a(j);
+            advance();
+        }
     }
     // the output scales, asked for now: the finish does not wait for them
     uint32_t sv_mine = 0;
@@ -324,6 +422,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
         __builtin_amdgcn_sched_barrier(0);
         fetch_a(j);
         advance();
+        if constexpr (ROT) return;
         if (++k == TR4) {
             flush();
 #pragma unroll
@@ -338,7 +437,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(GemmParams p)
         stage(1);
     }
     if ((w1 - w0) & 1) stage(0);
-    if (k != 0) flush();
+    if (ROT || k != 0) flush();
     if ((unsigned)wave < ncb) sv_lds[wave * 64 + lane] = sv_mine;
     __syncthreads();
 

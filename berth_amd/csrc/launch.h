@@ -183,8 +183,7 @@ struct GroupedArgs {
     const void* shared;         // host: three {trellis, suh, svh} of the always-on expert, or null
     int shared_expert;          // expert index the problem list uses for it (-1: none)
     int single_row;             // every problem has exactly one row
-    int mb;                     // MFMA path: rows per problem / 32 (1 or 4)
-    int small_rows = 0;         // MFMA path: every problem has at most this many rows, 16 or fewer (0: up to 32 * mb)
+    int small_rows = 0;         // MFMA path: every problem has at most this many rows, 16 or fewer (0: up to 32)
     const void* problems;       // GroupProblem[max_problems]
     const int* num_problems;
     int max_problems;

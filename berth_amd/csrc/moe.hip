@@ -1501,7 +1501,6 @@ extern "C" int berth_moe_grouped_exl3(const void* a, const void* a_up, const int
         g.problems = sb + at.mprob;
         g.num_problems = (const int*)(sb + at.counts) + 1;
         g.max_problems = at.max_m;
-        g.mb = 1;
         g.small_rows = at.small_rows < kGemmRows ? at.small_rows : 0;
         if (at.max_b > 0) {
             g.big_problems = sb + at.bprob;
@@ -1665,7 +1664,6 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.problems = wsb + L.mprob;
         g.num_problems = (const int*)(wsb + L.counts) + 1;
         g.max_problems = L.max_m;
-        g.mb = 1;
         g.small_rows = L.small_rows < kGemmRows ? L.small_rows : 0;
         g.act_had = wsb + L.ahd;
         g.act_done = &act_done;
@@ -1768,7 +1766,6 @@ extern "C" int berth_moe_layer_gated(const void* x, const void* wr, const float*
         g.problems = wsb + L.mprob;
         g.num_problems = (const int*)(wsb + L.counts) + 1;
         g.max_problems = L.max_m;
-        g.mb = 1;
         g.small_rows = L.small_rows < kGemmRows ? L.small_rows : 0;
         desc += " + " + launch_gemm_grouped(g);
     }

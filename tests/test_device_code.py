@@ -181,3 +181,10 @@ def test_matrix_instructions_keep_their_distance_from_inline_assembly(tmp_path, 
                 fresh = dict(before[i])
                 close = [reg for operand in _operands(rest)[1:4] for reg in operand if reg in fresh]
                 assert not close, f"{f.name}: {op} {rest} reads {close} too soon"
+
+
+@pytest.mark.parametrize("kernels,params", [
+    (["exl3_gemm_pair_kernel<3, 1>", "exl3_gemm_pair_kernel<4, 0>", "exl3_gemm_kernel<4, 0, 1, false>"], "GemmParams"),
+    (["exl3_gemm_rows_kernel<3, 1, 1, false, true>", "exl3_gemm_rows_kernel<4, 0, 2, false, true>"], "GemmRotateParams")])
+def test_the_same_of_the_fused_launches(tmp_path, kernels, params):
+    test_matrix_instructions_keep_their_distance_from_inline_assembly(tmp_path, kernels, ("exl3_gemm_rows_kernel.cuh",), params)

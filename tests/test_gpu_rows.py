@@ -113,3 +113,57 @@ def test_block_with_fused_norm_equals_the_separate_calls(rows, H, I, bits):
     assert torch.equal(bits_of(res_out), bits_of(res_ref)) and torch.equal(bits_of(y), bits_of(y_ref)), launch
     for n in names:
         assert torch.equal(bits_of(getattr(mlp, n)), bits_of(want[n])), (n, launch)
+
+
+@pytest.mark.parametrize("rows,Kk,N,bits,cb", [
+    (2, 2048, 2048, 4, 2),          # parts of 4 units: two 128 blocks
+    (5, 4224, 2048, 3, 1),          # 66 units in 16 parts: 4 and 5 units, odd starts
+    (16, 4096, 3968, 5, 0),         # 31 blocks
+    (17, 2176, 3200, 6, 2),         # a second tile with one row
+    (24, 6144, 5120, 4, 2),         # 192 items: three a lane group
+    (32, 1024, 2048, 2, 2),
+    (8, 17408, 1024, 8, 2),
+])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_rotation_inside_the_launch(rows, Kk, N, bits, cb, fp32):
+    """Every column block is cut into parts of its own and a workgroup rotates the part of the input that it needs: the
+    rotated rows as the oracle has them, and the bits of the form with a launch for the rotation (whose input
+    lies in the buffer of the rotated rows, which keeps the two launches)."""
+    tr, suh, svh = synth.linear(rows + Kk, Kk, N, bits)
+    x = synth.activations(rows + N, rows, Kk)
+    d_tr, d_suh, d_svh, d_x = (dev(a.view(np.uint16)) for a in (tr, suh, svh, x))
+    res = []
+    for in_place in (False, True):
+        c = torch.zeros((rows, N), dtype=torch.float32 if fp32 else torch.float16, device=DEV)
+        a_had = d_x.clone() if in_place else torch.zeros_like(d_x)
+        K.prefill_lin.exl3_linear((a_had if in_place else d_x).data_ptr(), d_tr.data_ptr(), c.data_ptr(), d_suh.data_ptr(),
+                                  a_had.data_ptr(), d_svh.data_ptr(), None, rows, Kk, N, bits, Codebook(cb),
+                                  OutDtype.F32 if fp32 else OutDtype.F16)
+        torch.cuda.synchronize()
+        launch = K.prefill_lin.last_launch()
+        assert (",rotate>" in launch) != in_place and ("had_r_128_slabs_kernel" in launch) == in_place, launch
+        res.append((c, a_had))
+    want, want_had = O.linear(x, tr, suh, svh, Kk, N, bits, cb, out_fp32=fp32)
+    assert np.array_equal(host_u16(res[0][1]).reshape(-1), want_had.view(np.uint16).reshape(-1))
+    assert torch.equal(res[0][1], res[1][1]) and torch.equal(res[0][0], res[1][0])
+    assert close(res[0][0].cpu().numpy() if fp32 else host_f16(res[0][0]), want)[0] == 0
+
+
+@pytest.mark.parametrize("rows,by_value", [(3, False), (8, False), (9, True), (20, True), (20, False)])
+def test_bundle_that_rotates_its_input(rows, by_value):
+    """Three sources of one input, two slices of the first: every source's rotated rows are left once."""
+    from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
+    gpu = Gpu(0)
+    Kk, widths, bits = 2304, (1024, 512, 512), 3
+    lins = [synth.linear(700 + i, Kk, n, bits) for i, n in enumerate(widths)]
+    multi = Exl3MultiLinear(gpu, [Exl3Linear(gpu, f"l{i}", *l) for i, l in enumerate(lins)])
+    x = synth.activations(710 + rows, rows, Kk)
+    outs = [torch.zeros((rows, n), dtype=torch.float16, device=DEV) for n in widths]
+    multi.forward(gpu, dev(x.view(np.uint16)), outs, OutDtype.F16, rows, by_value=by_value)
+    torch.cuda.synchronize()
+    assert ",rotate>" in K.ops.last_launch(), K.ops.last_launch()
+    for i, (tr, suh, svh) in enumerate(lins):
+        want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=False)
+        assert close(host_f16(outs[i]), want)[0] == 0, i
+        slab = host_u16(multi.a_had)[i * rows * Kk:(i + 1) * rows * Kk]
+        assert np.array_equal(slab, want_had.view(np.uint16).reshape(-1)), i
