@@ -691,8 +691,9 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         // whole K in every workgroup: gate, up and the next rotation together
         if (g.max_problems > 65535) throw std::runtime_error("moe grouped linear: too many problems");
         p.act_had = (_Float16*)g.act_had;
+        p.group_lins = 1;
         std::string desc;
-        gemm_bits(p, g.k_bits, g.codebook, -4, g.stream, desc, dim3(g.size_n / 128, g.max_problems));
+        gemm_bits(p, g.k_bits, g.codebook, -4, g.stream, desc, group_grid(g.size_n / 128, 1, g.max_problems));
         hip_ok(hipGetLastError(), "exl3_gemm_pair_kernel launch");
         *g.act_done = true;
         return desc + " grouped";
@@ -703,6 +704,7 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
     p.S = gemm_split(ws, tiles, g.size_k / 128, mb);
     if (g.max_problems + g.max_big > 65535) throw std::runtime_error("moe grouped linear: too many problems");
     std::string desc;
+    p.group_lins = g.num_lins;
     p.tiles_y = g.max_problems;
     if (g.max_big > 0) {
         // both lists in one launch, whole K per workgroup
@@ -710,11 +712,11 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         p.num_big = g.num_big;
         p.max_big = g.max_big;
         p.S = 1;
-        gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, dim3(nblocks, g.num_lins, g.max_problems + g.max_big));
+        gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, group_grid(nblocks, g.num_lins, g.max_problems + g.max_big));
         hip_ok(hipGetLastError(), "exl3_gemm_mixed_kernel launch");
         return desc + " grouped";
     }
-    gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, dim3(nblocks * p.S, g.num_lins, g.max_problems));
+    gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, group_grid(nblocks * p.S, g.num_lins, g.max_problems));
     hip_ok(hipGetLastError(), "exl3_gemm_kernel grouped launch");
     return desc + " grouped";
 }

@@ -63,8 +63,8 @@ static void gemm_launch_mixed(const GemmParams& p, hipStream_t stream, std::stri
                             "exl3_gemm_mixed_kernel shared-memory attribute");
     hipLaunchKernelGGL((exl3_gemm_mixed_kernel<BITS, CB>), grid, dim3(256), smem, stream, p);
     desc = "exl3_gemm_mixed_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + ",128x256+32x256> grid=" +
-           std::to_string(grid.x) + "x" + std::to_string(grid.y) + "x(" + std::to_string(p.max_big) + "+" +
-           std::to_string(grid.z - p.max_big) + ") smem=" + std::to_string(smem);
+           std::to_string(grid.x) + "x" + std::to_string(grid.y) + " problems=" + std::to_string(p.max_big) + "+" +
+           std::to_string(p.tiles_y) + " smem=" + std::to_string(smem);
 }
 
 // gate and up of a problem list, and the down projection's rotated input; mb = -4

@@ -108,6 +108,7 @@ struct GemmParams {
     GemmSlice slice[kGemmMaxSlices];
     // grouped: where row r of the sorted order lies in a_had (optional; rows of the always-on expert: at r)
     const int32_t* a_rows;
+    int group_lins;             // linears of a problem that are units of their own (1 or 2)
     _Float16* act_had;          // exl3_gemm_pair_kernel: the down projection's rotated input, in sorted order
 };
 
@@ -648,11 +649,28 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     }
 }
 
+// Grouped launches.  Workgroup i runs on die i % 8, and every die has its own L2: the column blocks of one
+// problem and linear, which read the same rows, go to one die, one after the other.  Of the grid
+// (8 * column blocks, groups / 8) blockIdx.x % 8 and blockIdx.y name the group (problem-major, then the
+// launch's one or two linears, so that the few real problems come ahead of the empty tail of the list)
+// and blockIdx.x / 8 the column block.  XXX
+struct GroupTile {
+    int col, which, problem;
+};
+__device__ __forceinline__ GroupTile group_tile(const GemmParams& p)
+{
+    const int g = (int)blockIdx.y * 8 + ((int)blockIdx.x & 7);
+    const int two = p.group_lins - 1;                   // 0 or 1
+    return {(int)blockIdx.x >> 3, g & two, g >> two};
+}
+inline dim3 group_grid(int cols, int lins, int problems)
+{
+    return dim3((unsigned)(8 * cols), (unsigned)((lins * problems + 7) / 8));
+}
+
 // Dense launches: blockIdx.x = (tile - tile0) * S + split with tiles numbered row
 // block by row block, so that one linear can be issued as several launches with
-// different split factors.  Grouped launches: blockIdx.x = column block * S + split,
-// blockIdx.y the linear, blockIdx.z the problem, so that the workgroups of the (few)
-// real problems of every linear are dispatched before the empty tail of the list.
+// different split factors.  Grouped launches: group_tile, a "column block" being one of S parts of it.
 //
 // 32-row problems: up to four workgroups on a compute unit (with four parts in flight at the end of a
 // split tile it was 173 registers a lane and two of them, so that the 756 workgroups of 64 tokens x 128
@@ -661,8 +679,9 @@ template <int BITS, int CB, int MB, bool DENSE = true>
 __global__ __launch_bounds__(256, MB == 1 && !DENSE ? 3 : 2) void exl3_gemm_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int unit = blockIdx.x / p.S;
-    const int split = blockIdx.x - unit * p.S;
+    const GroupTile gt = DENSE ? GroupTile{(int)blockIdx.x, 0, 0} : group_tile(p);
+    const int unit = gt.col / p.S;
+    const int split = gt.col - unit * p.S;
     const int nblocks = ((p.N + 255) >> 8) * (p.num_slices > 0 ? p.num_slices : 1);
     KRange kr;
     kr.kb0 = split;
@@ -677,18 +696,18 @@ __global__ __launch_bounds__(256, MB == 1 && !DENSE ? 3 : 2) void exl3_gemm_kern
         kr.slot0 = kr.slot_rest = kr.counter * p.S;
         gemm_tile<BITS, CB, MB, true>(p, tile / nblocks, tile % nblocks, kr, 0, smem);
     } else {
-        if ((int)blockIdx.z >= *p.num_problems) return;
+        if (gt.problem >= *p.num_problems) return;
         // grouped: (linear, problem, column block)
-        kr.counter = ((size_t)blockIdx.y * p.tiles_y + blockIdx.z) * nblocks + unit;
+        kr.counter = ((size_t)gt.which * p.tiles_y + gt.problem) * nblocks + unit;
         kr.slot0 = kr.slot_rest = kr.counter * p.S;
-        gemm_tile<BITS, CB, MB, false>(p, blockIdx.z, unit, kr, blockIdx.y, smem, p.problems);
+        gemm_tile<BITS, CB, MB, false>(p, gt.problem, unit, kr, gt.which, smem, p.problems);
     }
 }
 
 // Gate and up of a list of problems of up to 32 rows, and the input of their down projections: waves 0
 // and 1 take 128 columns of gate, waves 2 and 3 the same columns of up, so that the workgroup holds both
-// factors of silu(g) * u and a whole block of the next rotation when its k-loops end.  blockIdx.x =
-// column block, blockIdx.y the problem; linears lin_base, lin_base + 1 and, for its input scales,
+// factors of silu(g) * u and a whole block of the next rotation when its k-loops end.  The grid is
+// group_tile's of one linear; linears lin_base, lin_base + 1 and, for its input scales,
 // lin_base + 2 of an expert.  Gate and up are written too (fp16, c[0] and c[1]).
 // The values are those of the 32-row tiles and of moe_had_rows_kernel behind them.
 // What bounds it: the decode, as there; the end of a row is three rotations (of 128 values by sixteen
@@ -699,14 +718,15 @@ template <int BITS, int CB>
 __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    if ((int)blockIdx.y >= *p.num_problems) return;
+    const GroupTile gt = group_tile(p);
+    if (gt.problem >= *p.num_problems) return;
     constexpr int kZStride = 256 + 4;
     float* const z_tile = (float*)smem;                 // [32][kZStride]: gate's 128 columns, up's
     const int lane = threadIdx.x & 63, slot = lane & 31, half_id = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int which = wave >> 1;
-    const int n0 = (int)blockIdx.x * 128;
-    const GroupProblem gp = p.problems[blockIdx.y];
+    const int n0 = gt.col * 128;
+    const GroupProblem gp = p.problems[gt.problem];
     const bool shared = gp.expert == p.shared_expert;
     auto linear = [&](int l) { return shared ? p.shared[p.lin_base + l] : p.experts[gp.expert * p.lins_per_expert + p.lin_base + l]; };
     const ExpertLin lin = linear(which);
@@ -769,12 +789,12 @@ __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
     }
 }
 
-// Grouped launch over two problem lists at once: blockIdx.z < max_big takes a problem of up
+// Grouped launch over two problem lists at once: the first max_big problems of group_tile are those of up
 // to 128 rows (weights decoded once for all of them, so an expert with many rows costs one
-// decode per 128 rows instead of one per 32), the values after that the problems of up to 32
+// decode per 128 rows instead of one per 32), the ones after them the problems of up to 32
 // rows.  Both kinds sit in one launch, the long tiles first, so the short ones fill in around
 // them (as two launches the 128-row tiles would run alone on a fraction of the compute units).
-// blockIdx.x = column block (whole K per workgroup: no hand-over), blockIdx.y the linear.
+// Whole K per workgroup: no hand-over.
 // A problem of up to 64 or 96 rows runs as two or three 32-row blocks (the loop multiplies all the blocks
 // it has, needed or not): gate + up and down of 800 tokens that choose 8 of 128 experts 137 + 82 -> 119 +
 // 70 us, of 1500 tokens (94 rows an expert) 133 + 89 -> 131 + 85.
@@ -798,17 +818,18 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
     kr.counter = 0;
     kr.slot0 = kr.slot_rest = 0;
     kr.slot_step = 0;
-    const int z = blockIdx.z;
+    const GroupTile gt = group_tile(p);
+    const int z = gt.problem;
     if (z < p.max_big) {
         if (z >= *p.num_big) return;
         const int rows = p.big_problems[z].nrows;               // as many 32-row blocks as the problem has
-        if (rows > 96) gemm_tile<BITS, CB, 4, false>(p, z, blockIdx.x, kr, blockIdx.y, smem, p.big_problems);
-        else if (rows > 64) gemm_tile<BITS, CB, 3, false>(p, z, blockIdx.x, kr, blockIdx.y, smem, p.big_problems);
-        else gemm_tile<BITS, CB, 2, false>(p, z, blockIdx.x, kr, blockIdx.y, smem, p.big_problems);
+        if (rows > 96) gemm_tile<BITS, CB, 4, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
+        else if (rows > 64) gemm_tile<BITS, CB, 3, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
+        else gemm_tile<BITS, CB, 2, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
         return;
     }
     if (z - p.max_big >= *p.num_problems) return;
-    gemm_tile<BITS, CB, 1, false>(p, z - p.max_big, blockIdx.x, kr, blockIdx.y, smem, p.problems);
+    gemm_tile<BITS, CB, 1, false>(p, z - p.max_big, gt.col, kr, gt.which, smem, p.problems);
 }
 
 // Dense launches whose tile count does not divide over the compute units: the
