@@ -582,9 +582,9 @@ static bool mlp_pair_on_matrix_units(int size_m, int hidden, int intermediate)
 }
 
 // gate and up; `norm`: the input is that norm's rows instead of pair.a
-static std::string mlp_gate_up(const PairArgs& pair, void* act_had)
+static std::string mlp_gate_up(const PairArgs& pair, void* act_had, PairNext* next, const Workspace* scratch)
 {
-    if (mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n)) return launch_gemm_pair(pair, act_had);
+    if (mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n)) return launch_gemm_pair(pair, act_had, next, scratch);
     if (pair.size_m <= 8) return launch_gemv_pair(pair);
     std::string desc;
     for (int i = 0; i < 2; ++i) {
@@ -605,6 +605,24 @@ static std::string mlp_down(LinearArgs down, void* gate_out, void* up_out, const
     if (down.size_m <= 8) return launch_gemv(down);
     down.act_out = up_out;
     return launch_gemm(down);
+}
+
+// gate, up and down: the finish of gate and up may leave down its input
+static std::string mlp_linears(const PairArgs& pair, LinearArgs down, const float* out_add)
+{
+    void* const act_had = down.a_had;
+    if (pair.size_m <= 32 || !mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n))
+        return mlp_gate_up(pair, act_had, nullptr, nullptr) + " ; " + mlp_down(down, pair.c[0], pair.c[1], out_add);
+    LaunchScope scope(pair.stream);
+    PairNext next{down.suh, act_had, down.size_n};
+    const std::string desc = mlp_gate_up(pair, act_had, &next, &scope.ws) + " ; ";
+    down.a = pair.c[0];
+    down.a_up = pair.c[1];
+    down.act_out = pair.c[1];
+    down.out_add = out_add;
+    down.rotated = next.done;
+    down.rotated_operand = next.operand;
+    return desc + launch_gemm(down, &scope.ws);
 }
 
 extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* gate_out, void* up_out, void* a_had,
@@ -628,8 +646,7 @@ extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* g
         check_shape("exl3 mlp", down);
         PairArgs pair{x, {lins[0].trellis, lins[1].trellis}, {lins[0].suh, lins[1].suh}, {lins[0].svh, lins[1].svh},
                       {gate_out, up_out}, a_had, size_m, hidden, intermediate, k_bits, codebook, st};
-        const std::string desc = mlp_gate_up(pair, act_had);
-        g_exl3_launch = desc + " ; " + mlp_down(down, gate_out, up_out, nullptr);
+        g_exl3_launch = mlp_linears(pair, down, nullptr);
         return 0;
     } catch (const std::exception& err) {
         g_exl3_err = err.what();
@@ -693,8 +710,7 @@ extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* r
             desc += " ; " + launch_rms_norm(residual_out, norm->weight, h_norm, nullptr, size_m, hidden, norm->epsilon,
                                             norm->constant_bias, norm->constant_scale, norm->weight_bf16, st) + " ; ";
         }
-        desc += mlp_gate_up(pair, act_had);
-        desc += " ; " + mlp_down(down, gate_out, up_out, fuse_add ? (const float*)residual_out : nullptr);
+        desc += mlp_linears(pair, down, fuse_add ? (const float*)residual_out : nullptr);
         if (fuse_add) desc += size_m == 1 ? " +residual" : " +add";
         else desc += " ; " + launch_add_f32(y, residual_out, y, n, st);
         g_exl3_launch = desc;

@@ -238,7 +238,9 @@ static BlockPlan plan_block(const Workspace& ws, int slices, int slabs, int size
     return pl;
 }
 
-static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebook, hipStream_t stream, std::string& desc)
+// next: the two slices are gate and up, finished with what follows them
+static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebook, hipStream_t stream, std::string& desc,
+                      const FinishActivation* next = nullptr)
 {
     const long tiles = (long)(p.num_slices > 0 ? p.num_slices : 1) * (p.N / 128) * pl.row_blocks;
     p.units = (int)pl.units;
@@ -256,7 +258,12 @@ static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebo
     p.lds_bytes = (unsigned)block_lds_bytes(pl.mt);
     gemm_bits(p, k_bits, codebook, -8 - pl.mt, stream, desc, dim3(pl.grid));
     hip_ok(hipGetLastError(), "exl3_gemm_block_kernel launch");
-    if (pl.S || pl.rem || pl.q % pl.spt) {              // some tile is shared
+    if (next) {
+        const dim3 grid((unsigned)(tiles / 2), (unsigned)(pl.rows_per_tile / 16));
+        hipLaunchKernelGGL(exl3_gemm_silu_mul_finish_kernel, grid, dim3(256), 0, stream, p, *next);
+        hip_ok(hipGetLastError(), "exl3_gemm_silu_mul_finish_kernel launch");
+        desc += " + exl3_gemm_silu_mul_finish_kernel grid=" + std::to_string(grid.x) + "x" + std::to_string(grid.y);
+    } else if (pl.S || pl.rem || pl.q % pl.spt) {       // some tile is shared
         const dim3 grid((unsigned)tiles, (unsigned)(pl.rows_per_tile / 16));
         hipLaunchKernelGGL(exl3_gemm_finish_kernel, grid, dim3(256), 0, stream, p);
         hip_ok(hipGetLastError(), "exl3_gemm_finish_kernel launch");
@@ -404,10 +411,10 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
         rot.mt = plan.mt();
     }
     // (the rotation overlaps the reads of other workgroups then, and the output their reads of the input)
-    const bool rotate = plan.rows.ok && plan.rows.rotate && !a.a_up && !a.act_out &&
+    const bool rotate = plan.rows.ok && plan.rows.rotate && !a.a_up && !a.act_out && !a.rotated &&
                         apart(a.a, (size_t)a.size_m * a.size_k * 2, a.a_had, (size_t)a.size_m * a.size_k * 2) &&
                         apart(a.a, (size_t)a.size_m * a.size_k * 2, a.c, (size_t)a.size_m * a.size_n * (a.out_fp32 ? 4 : 2));
-    std::string d0 = rotate ? "" : launch_rotate(rot) + " + ";
+    std::string d0 = rotate || a.rotated ? "" : launch_rotate(rot) + " + ";
     GemmRotateParams p{};
     if (rotate) {
         p.rot_in = (const _Float16*)a.a;
@@ -416,7 +423,7 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     }
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
-    p.a_had[0] = (const _Float16*)(plan.ok() ? plan.at : a.a_had);
+    p.a_had[0] = (const _Float16*)(!plan.ok() ? a.a_had : a.rotated ? a.rotated_operand : plan.at);
     p.lin.trellis = (const uint32_t*)a.trellis;
     p.lin.svh = (const _Float16*)a.svh;
     p.c[0] = a.c;
@@ -556,11 +563,12 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
            desc + (m.c_fp32 ? " out=f32" : " out=f16");
 }
 
-std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
+std::string launch_gemm_pair(const PairArgs& a, void* a_had_second, PairNext* next, const Workspace* scratch)
 {
     if (a.size_k % 128 != 0) throw std::runtime_error("exl3 linear: size_k must be a multiple of 128");
-    LaunchScope scope(a.stream);
-    Workspace& ws = scope.ws;
+    std::optional<LaunchScope> scope;
+    if (!scratch) scope.emplace(a.stream);
+    const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
     const OperandPlan plan(ws, 2, 2, a.size_m, a.size_k, a.size_n);
     GemmParams p{};
@@ -603,7 +611,20 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second)
     const long nblocks = 2L * ((a.size_n + 255) / 256);
     if (nblocks * ((a.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3 linear pair: too many output tiles");
     std::string desc;
-    if (plan.ok()) plan.run(p, false, a.k_bits, a.codebook, a.stream, desc);
+    // Row blocks finish their tiles in a second launch, which can go on to the next linear's input.  Its copy in
+    // operand order lies behind the partial sums that the launch still reads.
+    const OperandPlan after(ws, 1, 1, a.size_m, a.size_n, next ? next->size_n : 128);
+    const size_t operand_at = std::max(plan.block.operand_at, after.block.operand_at);
+    if (next && plan.block.ok && !after.rows.ok && operand_at + after.block.operand_stride * 2 <= ws.partial_bytes) {
+        FinishActivation f{(const _Float16*)next->suh, (_Float16*)next->a_had, nullptr, 1};
+        if (after.block.ok) {
+            f.operand = (_Float16*)((char*)ws.partials + operand_at);
+            f.mt = after.mt();
+        }
+        run_block(plan.block, p, a.k_bits, a.codebook, a.stream, desc, &f);
+        next->operand = f.operand;
+        next->done = true;
+    } else if (plan.ok()) plan.run(p, false, a.k_bits, a.codebook, a.stream, desc);
     else dispatch_dense(ws, p, a.k_bits, a.codebook, a.size_m, a.size_k, (int)nblocks, a.stream, desc);
     return "pair " + d0 + " + " + desc + " out=f16";
 }

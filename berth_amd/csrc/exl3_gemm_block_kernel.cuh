@@ -307,21 +307,63 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
     }
 }
 
+// The workgroups that share a tile of the row-block launch, and the partial-sum slot of the first of them
+// (the tile is the first of every other sharer's range).
+struct TileSharers {
+    unsigned first, last, slot_first;
+};
+__device__ __forceinline__ TileSharers tile_sharers(const GemmParams& p, const unsigned tile)
+{
+    const unsigned SPT = (((unsigned)p.K >> 6) + 3) >> 2;
+    const unsigned q = (unsigned)p.unit_q, rem = (unsigned)p.unit_r, S = (unsigned)p.S;
+    auto owner = [&](unsigned x) {
+        const unsigned big = rem * (q + 1);
+        return x < big ? div_exact(x, p.m_q1) : rem + div_exact(x - big, p.m_q);
+    };
+    TileSharers t;
+    t.first = S ? tile * S : owner(tile * SPT);
+    t.last = S ? tile * S + S - 1 : owner(tile * SPT + SPT - 1);
+    t.slot_first = S || t.first * q + min(t.first, rem) >= tile * SPT ? 0u : 1u;
+    return t;
+}
+// The sums of row r of the tile, columns 8 * chunk .. + 7: those of four sharers from x on (past the last: the last
+// again), added in k order.
+struct SharerSums {
+    float4_t part[4][2];
+};
+__device__ __forceinline__ SharerSums load_sharers(const GemmParams& p, const TileSharers t, const unsigned x, const int r, const int chunk)
+{
+    SharerSums s;
+#pragma unroll
+    for (unsigned i = 0; i < 4; ++i) {
+        const unsigned xi = min(x + i, t.last);
+        const global_ptr<const float4_t> src = (global_ptr<const float4_t>)as_global(
+            p.partials + ((size_t)xi * 2 + (xi == t.first ? t.slot_first : 0u)) * p.rows_per_tile * 128 + r * 128 + 8 * chunk);
+        s.part[i][0] = src[0];
+        s.part[i][1] = src[1];
+    }
+    return s;
+}
+__device__ __forceinline__ void add_sharers(const TileSharers t, const unsigned x, const SharerSums& s, float (&v)[8])
+{
+#pragma unroll
+    for (unsigned i = 0; i < 4; ++i)
+        if (x + i <= t.last) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += s.part[i][e >> 2][e & 3];
+        }
+}
+
 // Finishes the tiles that several workgroups of the launch before share: adds their sums in k order,
 // then output Hadamard, svh, the optional addend and the store.  blockIdx.x = tile, blockIdx.y =
 // sixteen rows of it; sixteen lanes a row, eight columns each.  Bound by the bytes of the sums,
 // which are still in the caches.
 static __global__ __launch_bounds__(256) void exl3_gemm_finish_kernel(GemmParams p)
 {
-    const unsigned SPT = (((unsigned)p.K >> 6) + 3) >> 2, RT = (unsigned)p.tiles_y;
-    const unsigned q = (unsigned)p.unit_q, rem = (unsigned)p.unit_r, S = (unsigned)p.S;
+    const unsigned RT = (unsigned)p.tiles_y;
     const unsigned tile = blockIdx.x;
-    auto owner = [&](unsigned x) {
-        const unsigned big = rem * (q + 1);
-        return x < big ? div_exact(x, p.m_q1) : rem + div_exact(x - big, p.m_q);
-    };
-    const unsigned wa = S ? tile * S : owner(tile * SPT), wb = S ? tile * S + S - 1 : owner(tile * SPT + SPT - 1);
-    if (wa == wb) return;                               // finished by its only workgroup
+    const TileSharers t = tile_sharers(p, tile);
+    if (t.first == t.last) return;                      // finished by its only workgroup
     const unsigned cb = div_exact(tile, p.m_rt);
     const RowsBlock b = rows_block(p, cb);
     if (b.empty) return;
@@ -331,28 +373,82 @@ static __global__ __launch_bounds__(256) void exl3_gemm_finish_kernel(GemmParams
     const int rows = min(BM, p.M - m0);
     if ((int)blockIdx.y * 16 + (int)(threadIdx.x >> 6) * 4 >= rows) return;
     const int r = min(row, rows - 1);
-    // the tile is the first of every sharer's range but, unless that starts with it, the first sharer's
-    const unsigned slot_a = S || wa * q + min(wa, rem) >= tile * SPT ? 0u : 1u;
     const half8_t sv = ((global_ptr<const half8_t>)as_global(b.svh + b.n0))[chunk];
     float v[8] = {};
-    for (unsigned x = wa; x <= wb; x += 4) {
-        float4_t part[4][2];
-#pragma unroll
-        for (unsigned i = 0; i < 4; ++i) {
-            const unsigned xi = min(x + i, wb);
-            const global_ptr<const float4_t> src = (global_ptr<const float4_t>)as_global(
-                p.partials + ((size_t)xi * 2 + (xi == wa ? slot_a : 0u)) * BM * 128 + r * 128 + 8 * chunk);
-            part[i][0] = src[0];
-            part[i][1] = src[1];
-        }
-#pragma unroll
-        for (unsigned i = 0; i < 4; ++i)
-            if (x + i <= wb) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] += part[i][e >> 2][e & 3];
-            }
-    }
+    for (unsigned x = t.first; x <= t.last; x += 4) add_sharers(t, x, load_sharers(p, t, x, r, chunk), v);
     block_finish_row(p, b, v, sv, m0 + row, row < rows, lane);
+}
+
+// Finishes gate and up of an MLP (the two slices of the launch before) and forms the input of the down
+// projection: a workgroup takes the same sixteen rows and 128 columns of both, so that silu(g) * u and its
+// rotation need no launch of their own behind this one that reads both back.  Gate goes to its output,
+// the activation where up would have gone, the rotated rows to act_had and, in operand order, to `operand`
+// (may be null).  blockIdx.x = row block and column block of gate as the tiles are numbered, blockIdx.y = sixteen
+// rows of it.  The values are those of exl3_gemm_finish_kernel and silu_mul_had_r_128_kernel.
+// Bound by latency and the bytes of the sums, 16 to 32 bytes per value of gate and up: everything a row needs is asked
+// for at once (with the loads of gate waited for before those of up a layer of 40 rows took 1 us more).  Decoder
+// layers with an MLP of 5120 x 17408, instead of a finish, silu_mul_had_r_128_kernel and a second entry of the host:
+// 40 rows 132.8 -> 128.5 us, 100 rows 182.8 -> 178.4, 130 rows 232.1 -> 227.3; MLP widths 2048 x 5632, 100 rows
+// 101.6 -> 98.5; where gate and up take another kernel (250 and 400 rows) the same.
+struct FinishActivation {
+    const _Float16* suh;        // input scales of the down projection
+    _Float16* act_had;
+    _Float16* operand;
+    int mt;                     // tiles of 16 rows of a block of the operand copy
+};
+static __global__ __launch_bounds__(256) void exl3_gemm_silu_mul_finish_kernel(GemmParams p, FinishActivation f)
+{
+    const unsigned RT = (unsigned)p.tiles_y, tiles = gridDim.x;
+    const unsigned cb = div_exact(blockIdx.x, p.m_rt);
+    const int lane = threadIdx.x & 63, chunk = had_chunk(lane);
+    const int m0 = (int)(blockIdx.x - cb * RT) * p.rows_per_tile;
+    const int rows = min(p.rows_per_tile, p.M - m0);
+    if ((int)blockIdx.y * 16 + (int)(threadIdx.x >> 6) * 4 >= rows) return;
+    const int row = (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4);
+    const int r = min(row, rows - 1);                   // (lane groups past the last row redo it, and store nothing)
+    const bool live = row < rows;
+    const size_t at = (size_t)(m0 + r) * p.N + cb * 128 + 8 * chunk;
+    const half8_t su = ((global_ptr<const half8_t>)as_global(f.suh + cb * 128))[chunk];
+    half8_t gu[2], sv[2];
+    TileSharers t[2];
+    SharerSums sums[2];
+    float v2[2][8] = {};
+    // everything that is read is asked for together: four sharers of either tile (there are seldom more), or, of a
+    // tile that its only workgroup has finished, the result
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        t[s] = tile_sharers(p, blockIdx.x + (unsigned)s * tiles);
+        sv[s] = ((global_ptr<const half8_t>)as_global(p.slice[s].svh + cb * 128))[chunk];
+        if (t[s].first == t[s].last) gu[s] = *(global_ptr<const half8_t>)(as_global((const _Float16*)p.slice[s].c) + at);
+        else sums[s] = load_sharers(p, t[s], t[s].first, r, chunk);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        if (t[s].first == t[s].last) continue;
+        add_sharers(t[s], t[s].first, sums[s], v2[s]);
+        for (unsigned x = t[s].first + 4; x <= t[s].last; x += 4) add_sharers(t[s], x, load_sharers(p, t[s], x, r, chunk), v2[s]);
+        const float unit = had128_row16(v2[s], lane) * kRsqrt128;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gu[s][e] = (_Float16)rounded(had_scale(v2[s][e], unit) * (float)sv[s][e]);
+        if (s == 0 && live) *(global_ptr<half8_t>)(as_global((_Float16*)p.slice[0].c) + at) = gu[0];
+    }
+    half8_t x;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = silu_mul_h(gu[0][e], gu[1][e]);
+    float v[8];
+    mul_half8(x, su, v);
+    const float unit = had128_row16(v, lane) * kRsqrt128;
+    half8_t o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (_Float16)had_scale(v[e], unit);
+    if (!live) return;
+    *(global_ptr<half8_t>)(as_global((_Float16*)p.slice[1].c) + at) = x;
+    *(global_ptr<half8_t>)(as_global(f.act_had) + at) = o;
+    if (f.operand) {
+        const int R = m0 + row, block = R / (16 * f.mt);
+        *(global_ptr<half8_t>)(as_global(f.operand) + (size_t)block * rows_operand_elements(p.N, f.mt) +
+                               rows_operand_offset(R - block * 16 * f.mt, (int)cb * 128 + 8 * chunk, f.mt)) = o;
+    }
 }
 
 }  // namespace berth

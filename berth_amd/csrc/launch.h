@@ -140,6 +140,10 @@ struct LinearArgs {
     const void* a_up = nullptr;   // the input is silu(a) * a_up, element by element
     void* act_out = nullptr;      // with a_up, MFMA kernels only: where that input also goes (may be a_up)
     const float* out_add = nullptr;   // streaming and MFMA kernels, fp32 output: fp32 [size_m][size_n] added to the output
+    // MFMA kernels: a_had holds the rotated rows already and, where the launch reads a copy in operand order
+    // (launch_gemm_pair's PairNext::operand), so does that place in the workspace
+    bool rotated = false;
+    const void* rotated_operand = nullptr;
 };
 
 // RMS norm with the residual added first, as the input of a launch of the streaming kernel or of a
@@ -277,7 +281,17 @@ std::string launch_rotate(const RotateArgs& args);
 constexpr int kNormRotateMaxCols = 32768;
 // gate and up of an MLP above 8 rows as one bundle: two linears of one shape on one input, each
 // with its own output and its own buffer for the rotated input
-std::string launch_gemm_pair(const PairArgs& pair, void* a_had_second);
+// next, optional: the linear behind silu(c[0]) * c[1].  Where the launch finishes its tiles in a launch of its own
+// that one leaves this activation in c[1] and its rotated rows as LinearArgs::rotated wants them, and sets `done`;
+// the workspace may then serve no other launch in between (scratch: the scope that the caller holds over both).
+struct PairNext {
+    const void* suh;
+    void* a_had;
+    int size_n;
+    bool done = false;
+    const void* operand = nullptr;
+};
+std::string launch_gemm_pair(const PairArgs& pair, void* a_had_second, PairNext* next = nullptr, const Workspace* scratch = nullptr);
 constexpr int kBundleMaxSlices = 16;    // slices of a bundle whose lists travel by value
 
 // rows 1..8: one row on the streaming kernel, 2..8 rows on the few-row MFMA kernel (launch_gemm), small

@@ -72,3 +72,38 @@ def test_bundle_with_narrower_slices(rows, unit):
         want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=False)
         assert close(host_f16(outs[i]), want)[0] == 0, i
         assert np.array_equal(host_u16(a_had).reshape(4, -1)[i], want_had.view(np.uint16).reshape(-1)), i
+
+
+@pytest.mark.parametrize("rows,H,I,bits,steps", [
+    (33, 1024, 4096, 4, -1),            # by the rule of sizes the down projection takes 32-row tiles: no operand-ordered rows
+    (100, 2048, 5632, 3, 0),            # tiles inside one workgroup and shared ones
+    (145, 1152, 4224, 5, 0),            # two row blocks, the second with 65 rows; a ragged last step of K
+    (48, 1280, 3072, 2, 0),             # parts of its own for every tile
+    (64, 128, 17408, 4, 0),             # every tile inside one workgroup
+])
+def test_gate_up_finished_with_the_next_rotation(rows, H, I, bits, steps):
+    """Gate, activation, rotated activation and output of an MLP call, and the rotated activation and output of the block
+    call, whose launch that finishes gate and up forms them."""
+    from berth_amd.device import Gpu
+    from tests.test_gpu_mlp import _block_inputs, _layer, run_mlp_block
+    with knobs(BERTH_GEMM_BLOCK_STEPS=steps):
+        launch = run_mlp_block(rows, H, I, bits)
+    assert "exl3_gemm_silu_mul_finish_kernel" in launch and "silu_mul_had_r_128_kernel" not in launch, launch
+    assert ("exl3_gemm_block_kernel" in launch.split(" ; ")[1]) == (steps == 0), launch
+    gpu = Gpu(0)
+    lins, mlp = _layer(gpu, H, I, bits, 9900 + rows, rows)
+    x, res, w = _block_inputs(gpu, H, rows, 9950 + rows)
+    res_out, y = torch.zeros_like(res), torch.zeros((rows, H), dtype=torch.float32, device=DEV)
+    mlp.forward_block(gpu, x, res, res_out, w, y, rows=rows)
+    torch.cuda.synchronize()
+    act = host_f16(mlp.u)[:rows * I].reshape(rows, I)
+    assert np.array_equal(host_u16(mlp.act_had)[:rows * I], O.had_rows_f16(act, lins[2][1], True).view(np.uint16).ravel())
+    # the output from that activation: the down projection as a call of its own, the residual added behind it
+    d = [dev(t.view(np.uint16)) for t in lins[2]]
+    c, had = torch.zeros_like(y), torch.zeros((rows, I), dtype=torch.float16, device=DEV)
+    with knobs(BERTH_GEMM_BLOCK_STEPS=0):
+        K.prefill_lin.exl3_linear(mlp.u.data_ptr(), d[0].data_ptr(), c.data_ptr(), d[1].data_ptr(), had.data_ptr(), d[2].data_ptr(),
+                                  torch.zeros(I * H, dtype=torch.float16, device=DEV).data_ptr() if rows > 144 else None, rows, I, H,
+                                  bits, Codebook.MUL1, OutDtype.F32)
+    torch.cuda.synchronize()
+    assert torch.equal(y, c + res_out)
