@@ -653,7 +653,8 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 // problem and linear, which read the same rows, go to one die, one after the other.  Of the grid
 // (8 * column blocks, groups / 8) blockIdx.x % 8 and blockIdx.y name the group (problem-major, then the
 // launch's one or two linears, so that the few real problems come ahead of the empty tail of the list)
-// and blockIdx.x / 8 the column block.  XXX
+// and blockIdx.x / 8 the column block.  1500 tokens through 128 experts of 2048 x 768: 283 -> 275 us against column
+// blocks spread over the dies, whose rows every L2 then read for itself.
 struct GroupTile {
     int col, which, problem;
 };
