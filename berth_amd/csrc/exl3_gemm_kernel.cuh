@@ -59,7 +59,7 @@ struct GemmParams {
     ExpertLin shared[3];        // an always-on expert passed by value (problem.expert == shared_expert)
     int shared_expert;
     // mixed grouped launches (exl3_gemm_mixed_kernel): problems of up to 128 rows, whose units
-    // of work come first; those of `problems` follow
+    // of work come first; those of `problems` follow (max_big: the list's capacity)
     const GroupProblem* big_problems;
     const int* num_big;
     int max_big;
@@ -109,6 +109,7 @@ struct GemmParams {
     // grouped: where row r of the sorted order lies in a_had (optional; rows of the always-on expert: at r)
     const int32_t* a_rows;
     int group_lins;             // linears of a problem that are units of their own (1 or 2)
+    int half_tiles;             // exl3_gemm_mixed_kernel: up to this many tiles run as halves of 128 columns
     _Float16* act_had;          // exl3_gemm_pair_kernel: the down projection's rotated input, in sorted order
 };
 
@@ -790,7 +791,174 @@ __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
     }
 }
 
-// Grouped launch over two problem lists at once: the first max_big problems of group_tile are those of up
+// One tile of a problem, 128 columns from n0 on, whole K: half of what gemm_tile's workgroup does, for launches of
+// few tiles.  A wave owns 32 columns instead of 64, so
+// that its 64 lanes decode four tile rows of a k-block at a time instead of two: lane bits 4 and 5 name the
+// tile row (bit 5: which of the step's two, as in gemm_tile; bit 4: which step), and v_permlane16_swap_b32 trades
+// the columns u + 8 of the first step's lanes for the columns u of the second's.  The matrix instructions get
+// the same k values in the same order as gemm_tile's, so the sums are the same bits; column slots map to columns
+// 16 * (slot / 8 % 2) + slot % 8 + 8 * (slot / 16).
+// Bound by the decode and the multiplications, which a wave that is alone on its SIMD does one after the other.  The
+// trades are 16 of the 270 vector instructions of a k-block, and every A operand is read from LDS
+// for one multiplication instead of two.
+template <int BITS, int CB, int MB>
+__device__ __forceinline__ void gemm_half_tile(const GemmParams& p, const GroupProblem gp, const int which, const int n0, unsigned char* smem)
+{
+    constexpr int BM = MB * 32;
+    _Float16* a_tile = (_Float16*)smem;                 // [2][BM][kAStride]
+    float* z_tile = (float*)smem;                       // epilogue: [32][128 + 4]
+    constexpr int kZStride = 128 + 4;
+    if (n0 >= p.N) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int half_id = lane >> 5, slot = lane & 31;
+    const bool shared = gp.expert == p.shared_expert;
+    const ExpertLin lin = shared ? p.shared[p.lin_base + which] : p.experts[gp.expert * p.lins_per_expert + p.lin_base + which];
+    const int rows_here = gp.nrows;
+    constexpr int tile_dw = 8 * BITS;
+    const size_t row_dw = (size_t)(p.N >> 4) * tile_dw;
+    const int KB = p.K >> 7;
+
+    __shared__ __align__(16) half8_t s_scale[16];
+    half8_t scale_mine = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (threadIdx.x < 16) scale_mine = ((global_ptr<const half8_t>)as_global(lin.svh + n0))[threadIdx.x];
+
+    float16_t acc[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mb][r] = 0.0f;
+
+    const global_ptr<const uint32_t> tbase = as_global(lin.trellis) + (size_t)(half_id + 2 * ((lane >> 4) & 1)) * row_dw +
+                                             (size_t)((n0 >> 4) + 2 * wave + ((lane >> 3) & 1)) * tile_dw + (lane & 7) * BITS;
+    uint32_t ring[2][BITS];                             // tile rows 0..3 and 4..7 of a k-block
+    u32x4_t a_nxt[MB][2];
+    const int a_row = threadIdx.x >> 3, a_ch = threadIdx.x & 7;           // + 32 rows per pass
+    global_ptr<const u32x4_t> a_src[MB];
+#pragma unroll
+    for (int ps = 0; ps < MB; ++ps) {
+        int r = gp.row0 + min(a_row + 32 * ps, rows_here - 1);            // rows past the problem repeat its last row
+        if (p.a_rows && !shared) r = as_global(p.a_rows)[r];
+        a_src[ps] = (global_ptr<const u32x4_t>)(as_global(p.a_had[which]) + (size_t)r * p.K + a_ch * 16);
+    }
+    auto load_a = [&](int kb) {
+#pragma unroll
+        for (int ps = 0; ps < MB; ++ps) {
+            a_nxt[ps][0] = a_src[ps][kb * 16];
+            a_nxt[ps][1] = a_src[ps][kb * 16 + 1];
+        }
+    };
+    auto load_b = [&](int kb, int d) { load_tile_dwords<BITS>(tbase + (size_t)(kb * 8 + 4 * d) * row_dw, ring[d]); };
+    // pairs j0 .. j0 + n - 1 of half h, numbered j = 4f + q: out[f][q] = pair 4q + 2f + h
+    auto decode_pairs = [&](const LaneWindows<BITS>& w, int h, int j0, int n, uint32_t (&out)[2][4]) {
+#pragma unroll
+        for (int j = j0; j < j0 + n; ++j) {
+            const int f = j >> 2, q = j & 3;
+            const int pr = 4 * q + 2 * f + h;
+            out[f][q] = decode_pair<CB>(w.state(2 * pr), w.state(2 * pr + 1));
+        }
+    };
+    // [column half][q] of a lane's own step -> [step][q] of its own column half
+    auto trade = [&](uint32_t (&b)[2][4]) {
+        asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %4\n\tv_permlane16_swap_b32 %1, %5\n\t"
+            "v_permlane16_swap_b32 %2, %6\n\tv_permlane16_swap_b32 %3, %7\n\ts_nop 1"
+            : "+v"(b[0][0]), "+v"(b[0][1]), "+v"(b[0][2]), "+v"(b[0][3]), "+v"(b[1][0]), "+v"(b[1][1]), "+v"(b[1][2]), "+v"(b[1][3]));
+    };
+    uint32_t b[2][2][2][4];                             // [two steps' buffer][h][step][q]
+    load_a(0);
+    load_b(0, 0);
+    load_b(0, 1);
+    LaneWindows<BITS> win(ring[0], fetch_prev(lane, ring[0][BITS - 1]));
+    load_b(min(1, KB - 1), 0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        decode_pairs(win, h, 0, 8, b[0][h]);
+        trade(b[0][h]);
+    }
+    if (threadIdx.x < 16) s_scale[threadIdx.x] = scale_mine;
+
+    int buf = 0;
+    for (int kb = 0; kb < KB; ++kb, buf ^= 1) {
+        _Float16* a_buf = a_tile + (size_t)buf * BM * kAStride;
+#pragma unroll
+        for (int ps = 0; ps < MB; ++ps) {
+            u32x4_t* dst = (u32x4_t*)(a_buf + (a_row + 32 * ps) * kAStride + a_ch * 16);
+            dst[0] = a_nxt[ps][0];
+            dst[1] = a_nxt[ps][1];
+        }
+        load_a(min(kb + 1, KB - 1));                    // on the last one the same again: read and ignored
+        __syncthreads();
+        const _Float16* a_lane = a_buf + slot * kAStride + 16 * half_id;
+        // A operand of half-step hs = 2 * st + h, row block mb: k = 32 * st + 16 * half_id + 8 * h .. + 7 of the k-block
+        auto a_operand = [&](int hs, int mb) {
+            return *(const half8_t*)(a_lane + mb * 32 * kAStride + 32 * (hs >> 1) + 8 * (hs & 1));
+        };
+        half8_t a_op = a_operand(0, 0);
+#pragma unroll
+        for (int hs = 0; hs < 8; ++hs) {
+            const int d = hs >> 2, s = (hs >> 1) & 1, h = hs & 1;
+            __builtin_amdgcn_sched_barrier(0);
+            uint32_t (&b_nx)[2][4] = b[d ^ 1][s];       // the half of the next two steps decoded in this one and its neighbour
+            const half8_t b_op = __builtin_bit_cast(half8_t, uint4{b[d][h][s][0], b[d][h][s][1], b[d][h][s][2], b[d][h][s][3]});
+            if (s == 0 && h == 0) {
+                win = LaneWindows<BITS>(ring[d ^ 1], fetch_prev(lane, ring[d ^ 1][BITS - 1]));
+                load_b(min(kb + 1 + d, KB - 1), d ^ 1);
+            }
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                const half8_t a_now = a_op;
+                if (mb + 1 < MB) a_op = a_operand(hs, mb + 1);
+                else if (hs < 7) a_op = a_operand(hs + 1, 0);
+                acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_now, b_op, acc[mb], 0, 0, 0);
+                decode_pairs(win, s, 4 * h + mb * 4 / MB, (mb + 1) * 4 / MB - mb * 4 / MB, b_nx);
+            }
+            if (h == 1) trade(b_nx);
+            // (the decode of a half-step spread over its MB matrix instructions)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 36 / MB, 0);
+            }
+        }
+    }
+
+    const int chunk = had_chunk(lane);
+    const int col = wave * 32 + ((slot >> 3) & 1) * 16 + (slot >> 4) * 8 + (slot & 7);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        if (mb * 32 >= rows_here) break;                        // workgroup-uniform
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z_tile[(8 * (r >> 2) + 4 * half_id + (r & 3)) * kZStride + col] = acc[mb][r];
+        __syncthreads();
+        // 32 vectors; a wave rotates four per pass, sixteen lanes each
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass) {
+            const int row = pass * 16 + wave * 4 + (lane >> 4);
+            if (mb * 32 + row >= rows_here) continue;
+            const float4_t* zp = (const float4_t*)&z_tile[row * kZStride + 8 * chunk];
+            const float4_t z0 = zp[0], z1 = zp[1];
+            float v[8] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
+            const float unit = had128_row16(v, lane) * kRsqrt128;
+            const half8_t sv = s_scale[chunk];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = had_scale(v[i], unit) * (float)sv[i];
+            const size_t at = (size_t)(gp.row0 + mb * 32 + row) * p.N + n0 + 8 * chunk;
+            if (p.out_fp32) {
+                global_ptr<float4_t> dst = (global_ptr<float4_t>)(as_global((float*)p.c[which]) + at);
+                dst[0] = float4_t{v[0], v[1], v[2], v[3]};
+                dst[1] = float4_t{v[4], v[5], v[6], v[7]};
+            } else {
+                half8_t o;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) o[i] = (_Float16)v[i];
+                *(global_ptr<half8_t>)(as_global((_Float16*)p.c[which]) + at) = o;
+            }
+        }
+    }
+}
+
+// Grouped launch over two problem lists at once: the first problems of group_tile are those of up
 // to 128 rows (weights decoded once for all of them, so an expert with many rows costs one
 // decode per 128 rows instead of one per 32), the ones after them the problems of up to 32
 // rows.  Both kinds sit in one launch, the long tiles first, so the short ones fill in around
@@ -799,6 +967,14 @@ __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
 // A problem of up to 64 or 96 rows runs as two or three 32-row blocks (the loop multiplies all the blocks
 // it has, needed or not): gate + up and down of 800 tokens that choose 8 of 128 experts 137 + 82 -> 119 +
 // 70 us, of 1500 tokens (94 rows an expert) 133 + 89 -> 131 + 85.
+// A launch of no more tiles than compute units runs them as halves of 128 columns (gemm_half_tile; bits the same),
+// the second halves behind the first: a workgroup alone on its compute unit takes nearly as long as two
+// that share one.  Layers of 2048 x 768: 200 tokens that choose 4 of 16 experts 69.7 -> 54.4 us (64 and 128 tiles), of
+// 1024 x 512, 300 tokens 58.2 -> 47.0, of 2048 x 1024, 150 tokens that choose 8 of 32 (256 tiles) 84.9 -> 80.8;
+// 400 tokens that choose 6 of 16 (256 tiles, half of them of 128 rows) 104.4 -> 105.
+// Above that whole tiles: up to 384 as halves 1000 tokens that choose 4 of 16 119 -> 126, and with the tiles of a last,
+// half empty round as halves 1500 tokens of 128 experts 278 -> 289 (the whole tiles are the cheaper ones, and the
+// rounds are not in step).
 // Measured and dropped: cutting K in two with the split-K hand-over, for every tile or for the
 // 128-row tiles only (the shorter units pack better, the hand-over of 128 KB of partial sums per
 // tile costs far more than that gains: 150 -> 183 us per layer), 128-column units whose four waves
@@ -819,18 +995,30 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
     kr.counter = 0;
     kr.slot0 = kr.slot_rest = 0;
     kr.slot_step = 0;
+    // problems in order: the first list, the second and, of a launch in halves, both again for the second halves
+    const int big = *p.num_big, problems = big + *p.num_problems;
+    const bool halves = problems * p.group_lins * ((int)gridDim.x >> 3) <= p.half_tiles;
     const GroupTile gt = group_tile(p);
-    const int z = gt.problem;
-    if (z < p.max_big) {
-        if (z >= *p.num_big) return;
+    const int half = gt.problem >= problems;
+    if (half && (!halves || gt.problem >= 2 * problems)) return;
+    const int z = gt.problem - half * problems;
+    if (halves) {
+        const GroupProblem gp = z < big ? p.big_problems[z] : p.problems[z - big];
+        const int n0 = gt.col * 256 + 128 * half;
+        if (gp.nrows > 96) gemm_half_tile<BITS, CB, 4>(p, gp, gt.which, n0, smem);
+        else if (gp.nrows > 64) gemm_half_tile<BITS, CB, 3>(p, gp, gt.which, n0, smem);
+        else if (gp.nrows > 32) gemm_half_tile<BITS, CB, 2>(p, gp, gt.which, n0, smem);
+        else gemm_half_tile<BITS, CB, 1>(p, gp, gt.which, n0, smem);
+        return;
+    }
+    if (z < big) {
         const int rows = p.big_problems[z].nrows;               // as many 32-row blocks as the problem has
         if (rows > 96) gemm_tile<BITS, CB, 4, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
         else if (rows > 64) gemm_tile<BITS, CB, 3, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
         else gemm_tile<BITS, CB, 2, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
         return;
     }
-    if (z - p.max_big >= *p.num_problems) return;
-    gemm_tile<BITS, CB, 1, false>(p, z - p.max_big, gt.col, kr, gt.which, smem, p.problems);
+    gemm_tile<BITS, CB, 1, false>(p, z - big, gt.col, kr, gt.which, smem, p.problems);
 }
 
 // Dense launches whose tile count does not divide over the compute units: the

@@ -116,6 +116,31 @@ def test_problems_of_two_three_and_four_row_blocks(T, bits):
     assert torch.equal(res[0], res[1])
 
 
+@pytest.mark.parametrize("T,H,E,k,I,bits,codebook,shared_I", [
+    (150, 384, 6, 2, 384, 4, 2, 0),         # a column block and a half
+    (330, 256, 6, 2, 384, 5, 0, 384),       # problems of four row blocks and the shared expert's
+    (240, 256, 6, 2, 128, 3, 1, 0),
+    (700, 128, 66, 4, 384, 4, 2, 0),        # at least 264 tiles of gate and up: whole; half that of the down projection
+    (700, 128, 66, 4, 256, 2, 1, 128),      # 132 of either: halves
+])
+def test_launches_of_few_128_row_tiles_run_them_as_halves(T, H, E, k, I, bits, codebook, shared_I):
+    """Either side of one tile per compute unit, against the 32-row problems' bits (which K of up to 384 keeps whole)."""
+    gpu = Gpu(0)
+    wr, _, experts, _, shared = _make_layer(gpu, 9600 + T + bits, H, E, I, bits, shared_I, 1.0)
+    x = (synth.activations(9601 + T, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
+    d_x, res = dev(x.view(np.uint16)), []
+    for big_min in (0, 33):
+        with knobs(BERTH_MOE_BIG_MIN=big_min):
+            layer = MoeLayer(gpu, wr, experts, k, shared=shared, codebook=codebook)
+            out = torch.zeros((T, H), dtype=torch.float32, device=DEV)
+            layer.forward(gpu, d_x, out, T)
+            torch.cuda.synchronize()
+            assert ("exl3_gemm_mixed_kernel" in K.moe.last_launch()) == (big_min > 0), K.moe.last_launch()
+            assert torch.isfinite(out).all() and (out != 0).any()
+            res.append(out)
+    assert torch.equal(res[0], res[1])
+
+
 @pytest.mark.parametrize("T,H,E,k", [(3, 128, 128, 8), (2, 128, 300, 10), (5, 128, 512, 32), (2, 64, 1000, 9), (1, 64, 65, 3)])
 @pytest.mark.parametrize("finite", [0, 2, None])
 def test_choice_among_equal_and_minus_infinite_logits(T, H, E, k, finite):
