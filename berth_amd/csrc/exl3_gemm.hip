@@ -410,10 +410,11 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
         rot.operand = plan.at;
         rot.mt = plan.mt();
     }
-    // (the rotation overlaps the reads of other workgroups then, and the output their reads of the input)
+    // (the rotation overlaps the reads of other workgroups then, the output their reads of the input and their rotated rows)
+    const size_t in_bytes = (size_t)a.size_m * a.size_k * 2, out_bytes = (size_t)a.size_m * a.size_n * (a.out_fp32 ? 4 : 2);
     const bool rotate = plan.rows.ok && plan.rows.rotate && !a.a_up && !a.act_out && !a.rotated &&
-                        apart(a.a, (size_t)a.size_m * a.size_k * 2, a.a_had, (size_t)a.size_m * a.size_k * 2) &&
-                        apart(a.a, (size_t)a.size_m * a.size_k * 2, a.c, (size_t)a.size_m * a.size_n * (a.out_fp32 ? 4 : 2));
+                        apart(a.a, in_bytes, a.a_had, in_bytes) && apart(a.a, in_bytes, a.c, out_bytes) &&
+                        apart(a.a_had, in_bytes, a.c, out_bytes);
     std::string d0 = rotate || a.rotated ? "" : launch_rotate(rot) + " + ";
     GemmRotateParams p{};
     if (rotate) {
@@ -522,20 +523,24 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
         rot.operand = plan.at;
         rot.mt = plan.mt();
     }
-    const size_t rows_bytes = (size_t)m.size_m * m.size_k * 2;
+    const size_t rows_bytes = (size_t)m.size_m * m.size_k * 2, in_bytes = rows_bytes * (rot.in_stride ? slabs : 1);
+    const auto output_apart = [&](const void* c, size_t elements) {
+        const size_t bytes = elements * (m.c_fp32 ? 4 : 2);
+        return apart(m.a, in_bytes, c, bytes) && apart(m.a_had, rows_bytes * slabs, c, bytes);
+    };
     // (More than 8 rows of a short K keep the launch that rotates: it is part of what is tested of such bundles.
     // A decoder layer of 12 rows and 1024 columns would gain 1 us of 48.)
     bool rotate = plan.rows.ok && plan.rows.rotate && (m.size_m <= 8 || m.size_k > 1024) &&
-                  apart(m.a, rows_bytes * (rot.in_stride ? slabs : 1), m.a_had, rows_bytes * slabs);
-    // (Lists in device memory cannot be looked at here: their outputs must not overlap the input, as for the
-    // dot-product kernel that bundles of smaller weights take.)
-    if (m.host_lists) {
+                  apart(m.a, in_bytes, m.a_had, rows_bytes * slabs);
+    // (Lists in device memory cannot be looked at here: the outputs of such slices must not overlap the input, as
+    // for the dot-product kernel that bundles of smaller weights take.)
+    if (!sliced) rotate = rotate && output_apart(m.c, (size_t)m.bszm_out * m.size_m * m.size_n);
+    else if (m.host_lists) {
         bool used[kGemmMaxSlices] = {};
-        for (int i = 0; i < m.bszm_out; ++i) used[sliced ? m.had_src_list[i] : i] = true;
+        for (int i = 0; i < m.bszm_out; ++i) used[m.had_src_list[i]] = true;
         rotate = rotate && std::all_of(used, used + slabs, [](bool u) { return u; });       // every input is some slice's
         for (int i = 0; i < m.bszm_out; ++i)
-            rotate = rotate && apart(m.a, rows_bytes * (rot.in_stride ? slabs : 1), p.slice[i].c,
-                                     ((size_t)(m.size_m - 1) * p.slice[i].n_stride + p.slice[i].width) * (m.c_fp32 ? 4 : 2));
+            rotate = rotate && output_apart(p.slice[i].c, (size_t)(m.size_m - 1) * p.slice[i].n_stride + p.slice[i].width);
     }
     if (rotate && m.host_lists) {
         bool left[kGemmMaxSlices] = {};

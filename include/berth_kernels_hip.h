@@ -205,12 +205,14 @@ int berth_ops_cat_f16_last(const void* embedding, const void* hidden, void* out,
  * size_n_list[s] <= size_n = slice width; had_src_list[s] = source index;
  * a_had holds num_had_src slabs of size_m*size_k.  Uniform mode (lists NULL):
  * bszm_out linears of one shape, inputs a[i] (bszm_in == bszm_out) or a[0]
- * (bszm_in == 1), outputs c[i] contiguous.  Any row count: one row, and 2..8 rows of
- * small weights, rotate the input inside the one launch; more rows, and 2..8 rows of
- * larger weights, take one launch that rotates the input once per source / linear and
- * MFMA launches over all slices (the reference sends 9..32 rows of its fused q/k/v and
- * gate/up bundles through this call, crates/berth-engine/src/prefill.rs:81-85).  Returns 1
- * on success (the reference returns its kernel-shape tag there), -1 on error. */
+ * (bszm_in == 1), outputs c[i] contiguous.  Any row count: one row, 2..8 rows of
+ * small weights, and up to 32 rows where a workgroup needs a part of size_k only, rotate the
+ * input inside the one launch (so neither the input nor a_had may overlap the outputs of
+ * slices whose lists are in device memory); the others take one launch that rotates the
+ * input once per source / linear and MFMA launches over all slices (the reference sends
+ * 9..32 rows of its fused q/k/v and gate/up bundles through this call,
+ * crates/berth-engine/src/prefill.rs:81-85).  Returns 1 on success (the reference returns its
+ * kernel-shape tag there), -1 on error. */
 int berth_ops_mgemm(const void* a, const void* b_list, void* c, const void* suh_list, void* a_had,
                     const void* svh_list, int size_m, int size_k, int size_n, int k_bits,
                     int codebook, int c_fp32, int bszm_in, int bszm_out, const int* size_n_list,

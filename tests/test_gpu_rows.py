@@ -167,3 +167,36 @@ def test_bundle_that_rotates_its_input(rows, by_value):
         assert close(host_f16(outs[i]), want)[0] == 0, i
         slab = host_u16(multi.a_had)[i * rows * Kk:(i + 1) * rows * Kk]
         assert np.array_equal(slab, want_had.view(np.uint16).reshape(-1)), i
+
+
+def test_outputs_over_the_input_or_its_rotated_rows():
+    """Two launches where the output lies over a buffer that the launch would rotate from or into: the bits of
+    buffers of their own (the first launch has read the input and left its copy before anything is stored)."""
+    rows, Kk, N, bits = 6, 2304, 1024, 4
+    lins = [[dev(t.view(np.uint16)) for t in synth.linear(720 + i, Kk, N, bits)] for i in range(2)]
+    d_x = dev(synth.activations(725, rows, Kk).view(np.uint16))
+    tr, suh, svh = lins[0]
+    a_had = torch.zeros_like(d_x)
+    c = torch.zeros((rows, N), dtype=torch.float16, device=DEV)
+    res = []
+    for out in (c, a_had):
+        K.prefill_lin.exl3_linear(d_x.data_ptr(), tr.data_ptr(), out.data_ptr(), suh.data_ptr(), a_had.data_ptr(),
+                                  svh.data_ptr(), None, rows, Kk, N, bits, Codebook.MUL1, OutDtype.F16)
+        torch.cuda.synchronize()
+        assert (",rotate>" in K.prefill_lin.last_launch()) == (out is c), K.prefill_lin.last_launch()
+        res.append(host_u16(out).reshape(-1)[:rows * N].copy())
+    assert np.array_equal(*res)
+
+    # a uniform bundle: its outputs follow from one pointer also where the lists are in device memory
+    lists = [torch.tensor([lin[j].data_ptr() for lin in lins], dtype=torch.int64, device=DEV) for j in range(3)]
+    slabs = torch.zeros((2, rows, Kk), dtype=torch.float16, device=DEV)
+    res = []
+    for over in (False, True):
+        x = d_x.clone()
+        out = x if over else torch.zeros((2, rows, N), dtype=torch.float16, device=DEV)
+        K.ops.exl3_mgemm(x.data_ptr(), lists[0].data_ptr(), out.data_ptr(), lists[1].data_ptr(), slabs.data_ptr(),
+                         lists[2].data_ptr(), rows, Kk, N, bits, Codebook.MUL1, OutDtype.F16, 1, 2)
+        torch.cuda.synchronize()
+        assert (",rotate>" in K.ops.last_launch()) == (not over), K.ops.last_launch()
+        res.append(host_u16(out).reshape(-1)[:2 * rows * N].copy())
+    assert np.array_equal(*res)
