@@ -532,8 +532,8 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
     // A decoder layer of 12 rows and 1024 columns would gain 1 us of 48.)
     bool rotate = plan.rows.ok && plan.rows.rotate && (m.size_m <= 8 || m.size_k > 1024) &&
                   apart(m.a, in_bytes, m.a_had, rows_bytes * slabs);
-    // (Lists in device memory cannot be looked at here: the outputs of such slices must not overlap the input, as
-    // for the dot-product kernel that bundles of smaller weights take.)
+    // The outputs of slices whose lists are in device memory cannot be looked at here: they may lie over the input or
+    // its rotated rows, and a source may have no slice that would leave its slab.  Those keep the two launches.
     if (!sliced) rotate = rotate && output_apart(m.c, (size_t)m.bszm_out * m.size_m * m.size_n);
     else if (m.host_lists) {
         bool used[kGemmMaxSlices] = {};
@@ -541,6 +541,8 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
         rotate = rotate && std::all_of(used, used + slabs, [](bool u) { return u; });       // every input is some slice's
         for (int i = 0; i < m.bszm_out; ++i)
             rotate = rotate && output_apart(p.slice[i].c, (size_t)(m.size_m - 1) * p.slice[i].n_stride + p.slice[i].width);
+    } else {
+        rotate = false;
     }
     if (rotate && m.host_lists) {
         bool left[kGemmMaxSlices] = {};

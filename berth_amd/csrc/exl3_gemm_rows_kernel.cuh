@@ -139,6 +139,7 @@ __device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsig
 }
 
 // the input of the column block `cb`, its scales and, for one column block per input, where its rotated rows go
+// (lists in device memory: of linears with an input each)
 __device__ __forceinline__ GemmRotation rows_rotation(const GemmRotateParams& p, const unsigned cb)
 {
     if (p.num_slices == 0) return {p.lin.suh, p.rot_in, cb == 0 ? p.rot_out : nullptr};
@@ -148,11 +149,8 @@ __device__ __forceinline__ GemmRotation rows_rotation(const GemmRotateParams& p,
         const GemmRotation& r = p.rotation[sl];
         return {r.suh, r.in, first ? r.had_out : nullptr};
     }
-    const unsigned slab = p.c_ptrs ? (unsigned)p.had_src_list[sl] : sl;
-    // (slices of one input that are not neighbours: each of them leaves it, the same values)
-    const bool leaves = first && (sl == 0 || !p.c_ptrs || (unsigned)p.had_src_list[sl - 1] != slab);
-    return {(const _Float16*)p.suh_list[slab], p.rot_in + (size_t)slab * p.rot_in_stride,
-            leaves ? p.rot_out + (size_t)slab * p.M * p.K : nullptr};
+    return {(const _Float16*)p.suh_list[sl], p.rot_in + (size_t)sl * p.rot_in_stride,
+            first ? p.rot_out + (size_t)sl * p.M * p.K : nullptr};
 }
 
 template <typename T>

@@ -205,11 +205,12 @@ int berth_ops_cat_f16_last(const void* embedding, const void* hidden, void* out,
  * size_n_list[s] <= size_n = slice width; had_src_list[s] = source index;
  * a_had holds num_had_src slabs of size_m*size_k.  Uniform mode (lists NULL):
  * bszm_out linears of one shape, inputs a[i] (bszm_in == bszm_out) or a[0]
- * (bszm_in == 1), outputs c[i] contiguous.  Any row count: one row, 2..8 rows of
- * small weights, and up to 32 rows where a workgroup needs a part of size_k only, rotate the
- * input inside the one launch (so neither the input nor a_had may overlap the outputs of
- * slices whose lists are in device memory); the others take one launch that rotates the
- * input once per source / linear and MFMA launches over all slices (the reference sends
+ * (bszm_in == 1), outputs c[i] contiguous.  Any row count: one row and 2..8 rows of
+ * small weights rotate the input inside the one launch (so neither the input nor a_had may
+ * overlap an output there); up to 32 rows where a workgroup needs a part of size_k only do so
+ * in uniform mode, or with lists in host memory, where no output overlaps either; the others take
+ * one launch that rotates the input once per source / linear, whether a slice uses it or
+ * not, and MFMA launches over all slices (the reference sends
  * 9..32 rows of its fused q/k/v and gate/up bundles through this call,
  * crates/berth-engine/src/prefill.rs:81-85).  Returns 1 on success (the reference returns its
  * kernel-shape tag there), -1 on error. */

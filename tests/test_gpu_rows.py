@@ -151,7 +151,8 @@ def test_rotation_inside_the_launch(rows, Kk, N, bits, cb, fp32):
 
 @pytest.mark.parametrize("rows,by_value", [(3, False), (8, False), (9, True), (20, True), (20, False)])
 def test_bundle_that_rotates_its_input(rows, by_value):
-    """Three sources of one input, two slices of the first: every source's rotated rows are left once."""
+    """Three sources of one input, two slices of the first: every source's rotated rows are left once.  With the lists in
+    device memory, which no check of the host sees, a launch of its own rotates."""
     from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
     gpu = Gpu(0)
     Kk, widths, bits = 2304, (1024, 512, 512), 3
@@ -161,7 +162,8 @@ def test_bundle_that_rotates_its_input(rows, by_value):
     outs = [torch.zeros((rows, n), dtype=torch.float16, device=DEV) for n in widths]
     multi.forward(gpu, dev(x.view(np.uint16)), outs, OutDtype.F16, rows, by_value=by_value)
     torch.cuda.synchronize()
-    assert ",rotate>" in K.ops.last_launch(), K.ops.last_launch()
+    launch = K.ops.last_launch()
+    assert (",rotate>" in launch) == by_value and ("had_r_128_slabs_kernel" in launch) != by_value, launch
     for i, (tr, suh, svh) in enumerate(lins):
         want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=False)
         assert close(host_f16(outs[i]), want)[0] == 0, i
@@ -200,3 +202,68 @@ def test_outputs_over_the_input_or_its_rotated_rows():
         assert (",rotate>" in K.ops.last_launch()) == (not over), K.ops.last_launch()
         res.append(host_u16(out).reshape(-1)[:2 * rows * N].copy())
     assert np.array_equal(*res)
+
+
+def _bundle_lists(sources, slices, outs):
+    """The seven lists of a sliced bundle in device memory: slices of (source, first column, width)."""
+    t64, t32 = (lambda v: torch.tensor(v, dtype=torch.int64, device=DEV)), (lambda v: torch.tensor(v, dtype=torch.int32, device=DEV))
+    bits, sizes = sources[0]["bits"], [s["n"] for s in sources]
+    b = t64([sources[s]["d"][0].data_ptr() + n0 // 16 * 16 * bits * 2 for s, n0, _ in slices])
+    svh = t64([sources[s]["d"][2].data_ptr() + 2 * n0 for s, n0, _ in slices])
+    suh = t64([s["d"][1].data_ptr() for s in sources])
+    c = t64([outs[s].data_ptr() + 2 * n0 for s, n0, _ in slices])
+    return b, suh, svh, t32([w for _, _, w in slices]), c, t32([sizes[s] for s, _, _ in slices]), t32([s for s, _, _ in slices])
+
+
+def _sources(seed, Kk, widths, bits):
+    return [{"bits": bits, "n": n, "np": lin, "d": [dev(t.view(np.uint16)) for t in lin]}
+            for n, lin in ((n, synth.linear(seed + i, Kk, n, bits)) for i, n in enumerate(widths))]
+
+
+def _device_bundle(x, a_had, lists, rows, Kk, width, bits, outs, sources):
+    b, suh, svh, n, c, stride, src = lists
+    K.ops.exl3_mgemm(x.data_ptr(), b.data_ptr(), outs[0].data_ptr(), suh.data_ptr(), a_had.data_ptr(), svh.data_ptr(), rows, Kk,
+                     width, bits, Codebook.MUL1, OutDtype.F16, 1, len(src), n.data_ptr(), c.data_ptr(), stride.data_ptr(),
+                     src.data_ptr(), sources)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows", [3, 8, 9, 20, 32])
+@pytest.mark.parametrize("over", ["input", "rotated rows"])
+def test_outputs_of_device_lists_over_the_input(rows, over):
+    """Slices whose lists are in device memory may store over the input or over the rotated rows: both have been read when the
+    first output is stored, so the bits are those of buffers of their own."""
+    Kk, widths, bits = 2304, (1024, 512, 512), 4
+    sources = _sources(730, Kk, widths, bits)
+    slices = [(0, 0, 512), (0, 512, 512), (1, 0, 512), (2, 0, 512)]
+    d_x = dev(synth.activations(735 + rows, rows, Kk).view(np.uint16))
+    res = []
+    for own in (True, False):
+        x, a_had = d_x.clone(), torch.zeros((3, rows, Kk), dtype=torch.float16, device=DEV)
+        outs = [torch.zeros((rows, n), dtype=torch.float16, device=DEV) for n in widths]
+        if not own:         # outputs one behind the other in the input (their columns fit) or in the rotated rows
+            at, flat = 0, (x if over == "input" else a_had).view(torch.float16).reshape(-1)
+            for i, n in enumerate(widths):
+                outs[i] = flat[at:at + rows * n].view(rows, n)
+                at += rows * n
+        _device_bundle(x, a_had, _bundle_lists(sources, slices, outs), rows, Kk, 512, bits, outs, 3)
+        assert ",rotate>" not in K.ops.last_launch(), K.ops.last_launch()
+        res.append([host_u16(o).copy() for o in outs])
+    for i in range(3):
+        assert np.array_equal(res[0][i], res[1][i]), i
+
+
+@pytest.mark.parametrize("rows", [4, 17])
+def test_rotated_rows_of_a_source_without_slices(rows):
+    """A source that no slice of a bundle in device memory uses: its rotated rows are left all the same."""
+    Kk, widths, bits = 2304, (1024, 512, 1024), 3
+    sources = _sources(740, Kk, widths, bits)
+    x = synth.activations(745 + rows, rows, Kk)
+    a_had = torch.zeros((3, rows, Kk), dtype=torch.float16, device=DEV)
+    outs = [torch.zeros((rows, n), dtype=torch.float16, device=DEV) for n in widths]
+    lists = _bundle_lists(sources, [(0, 0, 512), (0, 512, 512), (2, 0, 512), (2, 512, 512)], outs)
+    _device_bundle(dev(x.view(np.uint16)), a_had, lists, rows, Kk, 512, bits, outs, 3)
+    for i, s in enumerate(sources):
+        want, want_had = O.linear(x, *s["np"], Kk, widths[i], bits, 2, out_fp32=False)
+        assert np.array_equal(host_u16(a_had)[i].reshape(-1), want_had.view(np.uint16).reshape(-1)), i
+        assert i == 1 or close(host_f16(outs[i]), want)[0] == 0, i
