@@ -148,14 +148,16 @@ VALU_TO_MFMA = 2        # wait states; what the compiler leaves between its own 
 
 
 def _asm_results_step(ages, op, rest, in_asm):
-    """State: wait states since inline assembly wrote a vector register, while fewer than VALU_TO_MFMA."""
+    """State: wait states since inline assembly wrote a vector register, while fewer than VALU_TO_MFMA.
+    (An exchange of two registers writes both of its operands.)"""
     passed = int(rest, 0) + 1 if op == "s_nop" else 1
     ages = {reg: age + passed for reg, age in ages if age + passed < VALU_TO_MFMA}
     if op.startswith(("v_", "ds_read", "global_load", "buffer_load", "scratch_load")):
-        for reg in _operands(rest)[0]:
-            ages.pop(reg, None)
-            if in_asm and op.startswith("v_"):
-                ages[reg] = 0
+        for operand in _operands(rest)[:2 if re.match(r"v_(permlane\d+_)?swap_b(16|32)", op) else 1]:
+            for reg in operand:
+                ages.pop(reg, None)
+                if in_asm and op.startswith("v_"):
+                    ages[reg] = 0
     return frozenset(ages.items())
 
 
@@ -166,6 +168,16 @@ def _youngest(a, b):
     return frozenset(joined.items())
 
 
+def _read_too_soon(f):
+    """(matrix instruction, register) pairs of a kernel that stand too close to inline assembly."""
+    before, found = f.states(frozenset(), _asm_results_step, _youngest), []
+    for i, (op, rest, _) in enumerate(f.code):
+        if op.startswith("v_mfma") and i in before:
+            fresh = dict(before[i])
+            found += [(f"{op} {rest}", reg) for operand in _operands(rest)[1:4] for reg in operand if reg in fresh]
+    return found
+
+
 @pytest.mark.parametrize("kernels,headers,params", [
     (DECODING_KERNELS, ("exl3_gemm_block_kernel.cuh", "exl3_gemm_wide_kernel.cuh"), "GemmParams"),
     (STREAM_KERNELS, ("exl3_gemv_stream_kernel.cuh",), "StreamParams")])
@@ -173,14 +185,22 @@ def test_matrix_instructions_keep_their_distance_from_inline_assembly(tmp_path, 
     functions = [f for f in _compile(tmp_path, kernels, headers, params) if "finish_kernel" not in f.name]
     assert len(functions) == len(set(kernels))
     for f in functions:
-        before = f.states(frozenset(), _asm_results_step, _youngest)
         assert any(op.startswith("v_mfma") for op, _, _ in f.code), f.name
         assert any(a and op.startswith("v_") for op, _, a in f.code), f"{f.name}: no inline assembly left to check"
-        for i, (op, rest, _) in enumerate(f.code):
-            if op.startswith("v_mfma") and i in before:
-                fresh = dict(before[i])
-                close = [reg for operand in _operands(rest)[1:4] for reg in operand if reg in fresh]
-                assert not close, f"{f.name}: {op} {rest} reads {close} too soon"
+        close = _read_too_soon(f)
+        assert not close, f"{f.name}: too soon: {close[:4]} ({len(close)} in all)"
+
+
+@pytest.mark.parametrize("write,regs", [
+    ("v_permlane16_swap_b32 v4, v12", (4, 12)), ("v_permlane32_swap_b32_e32 v5, v13", (5, 13)), ("v_swap_b32 v6, v14", (6, 14)),
+    ("v_add_u32_e32 v7, v15, v16", (7,))])
+@pytest.mark.parametrize("waits,close", [("s_nop 0", True), ("s_nop 1", False)])
+def test_every_register_that_inline_assembly_writes_counts(write, regs, waits, close):
+    """A matrix instruction right behind inline assembly is found by each register that it writes, and only by those."""
+    for reg in range(4, 17):
+        f = Function("synthetic", [";#ASMSTART", write, waits, ";#ASMEND",
+                                   f"v_mfma_f32_32x32x16_f16 v[32:47], v[20:23], v[{reg}:{reg}], v[32:47]", "s_endpgm"])
+        assert bool(_read_too_soon(f)) == (close and reg in regs), (write, waits, reg)
 
 
 @pytest.mark.parametrize("kernels,params", [
