@@ -650,6 +650,8 @@ static GroupRowsPlan plan_group_rows(const Workspace& ws, const GroupedArgs& g)
     if (g.size_k < 256 || g.small_rows > 16) return pl;
     const unsigned long long TR4 = (unsigned)g.size_k / 64, blocks = (unsigned long long)g.max_problems * g.num_lins * (g.size_n / 128);
     const unsigned long long U = blocks * TR4;
+    // (a row's place in a_had is 32 bits there; the list is long enough for all rows)
+    if ((unsigned long long)g.max_problems * g.small_rows * g.size_k * 2 >= (1ull << 32)) return pl;
     if (blocks > (unsigned)kCounters / 2 || U * TR4 >= (1ull << 32) || blocks * blocks >= (1ull << 32)) return pl;
     for (unsigned rounds = 1; rounds <= 64; rounds *= 2) {
         const unsigned long long G = (unsigned long long)ws.cu_count * rounds;

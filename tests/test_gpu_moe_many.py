@@ -211,3 +211,29 @@ def test_gate_up_and_the_next_rotation_in_one_launch(T, H, E, k, I, bits, shared
     layer.forward(gpu, dev(x.view(np.uint16)), again, T)
     torch.cuda.synchronize()
     assert torch.equal(again, out)
+
+
+def test_rows_beyond_four_gigabytes_of_rotated_input():
+    """16-row problems over 65535 rows of 32896 columns: the rotated rows span more than 32-bit offsets reach, and the last
+    ones are read where they are."""
+    T, Kk, N, E, bits = 65535, 32896, 128, 2, 4
+    tr, suh, svh = synth.linear(9701, Kk, N, bits)
+    x = synth.activations(9702, 8, Kk)
+    d = [dev(t.view(np.uint16)) for t in (tr, suh, svh)]
+    table = torch.tensor([[t.data_ptr() for t in d]] * E, dtype=torch.int64, device=DEV)
+    i32 = lambda *shape: torch.zeros(shape, dtype=torch.int32, device=DEV)
+    idx, off, perm, inv = i32(T), i32(E + 1), i32(T), i32(T)
+    idx[T // 2:] = 1
+    gather = (torch.arange(T, device=DEV) % 8).int()
+    d_x, out = dev(x.view(np.uint16)), torch.zeros((T, N), dtype=torch.float32, device=DEV)
+    a_had = torch.zeros((T, Kk), dtype=torch.float16, device=DEV)
+    with knobs(BERTH_MOE_FEW_TOKENS=T, BERTH_MOE_BIG_MIN=0):
+        scratch = torch.zeros(K.moe.permute_scratch_bytes(T, 1, E), dtype=torch.uint8, device=DEV)
+        K.moe.permute(idx.data_ptr(), off.data_ptr(), perm.data_ptr(), inv.data_ptr(), scratch.data_ptr(), T, 1, E)
+        K.moe.grouped_exl3(d_x.data_ptr(), None, gather.data_ptr(), 1, table.data_ptr(), 1, 0, 1, out.data_ptr(), None,
+                           scratch.data_ptr(), a_had.data_ptr(), T, 1, E, Kk, N, bits, 2, True)
+        torch.cuda.synchronize()
+    want, _ = O.linear(x, tr, suh, svh, Kk, N, bits, 2, out_fp32=True)
+    for r in (0, T // 2, T - 250, T - 1):
+        assert np.abs(out[r].cpu().numpy() - want[r % 8]).max() <= 2e-3 * np.abs(want).max(), r
+    assert torch.equal(out[:8], out[T - 7 - 8:T - 7])
