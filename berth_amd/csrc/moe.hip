@@ -1072,7 +1072,7 @@ int moe_big_min(int T, size_t rows)
 void problem_capacity(size_t rows, size_t experts, int big_min, int small_rows, int& max_m, int& max_b)
 {
     if (big_min > 0) {
-        max_m = (int)std::min<size_t>(((size_t)(big_min + kGemmRows - 2) / kGemmRows) * experts, rows);
+        max_m = (int)std::min<size_t>(((size_t)(big_min + small_rows - 2) / small_rows) * experts, rows);
         max_b = (int)(rows / big_min);
     } else {
         max_m = (int)(std::min<size_t>(experts, rows) + rows / small_rows + 1);

@@ -249,3 +249,22 @@ def test_glue_ops_validate_before_any_device_call():
     with pytest.raises(LaunchError, match="rms_norm: dim must be a multiple of 4"):
         K.ops.rms_norm_f16(P, P, P, 1, 6, 1e-6)
     assert K.ops.last_launch() == ""
+
+
+@pytest.mark.parametrize("few,big_min", [(16, 33), (200, 33), (200, 17), (200, 1), (200, 128), (16, 128)])
+def test_moe_problem_list_holds_the_most_problems_there_can_be(few, big_min):
+    """Both problem lists of berth_moe_permute's scratch (the last two arrays of 16-byte entries, each rounded up to 256
+    bytes), for the distributions of rows over experts that need the longest lists."""
+    from tests.gpu_util import knobs
+    T, k, E, small = 200, 8, 64, 16 if few >= 200 else 32
+    rows = T * k
+    pad = lambda n: (n + 255) // 256 * 256
+    with knobs(BERTH_MOE_FEW_TOKENS=few, BERTH_MOE_BIG_MIN=big_min):
+        total = K.moe.permute_scratch_bytes(T, k, E)
+    lists = total - pad(rows * 4) - pad(16) - pad(min(E, rows) * 16)
+    longest = 0
+    for per in range(1, 129):               # as many experts as there can be with `per` rows each
+        n = min(E, rows // per)
+        longest = max(longest, n * -(-per // small) if per < big_min else 0)
+    big = rows // big_min       # every one of them with the fewest rows
+    assert lists >= pad(longest * 16) + pad(big * 16), (longest, big, lists)

@@ -237,3 +237,28 @@ def test_rows_beyond_four_gigabytes_of_rotated_input():
     for r in (0, T // 2, T - 250, T - 1):
         assert np.abs(out[r].cpu().numpy() - want[r % 8]).max() <= 2e-3 * np.abs(want).max(), r
     assert torch.equal(out[:8], out[T - 7 - 8:T - 7])
+
+
+def test_sixteen_row_problems_beside_128_row_ones():
+    """64 experts with 25 rows each as problems of 16 rows, in a call that may also have 128-row problems: two problems
+    per expert, all of them in the list, and the bits of the 32-row problems."""
+    T, k, E, Kk, N, bits = 200, 8, 64, 256, 384, 4
+    lins = [synth.linear(9800 + e, Kk, N, bits) for e in range(E)]
+    d = [[dev(t.view(np.uint16)) for t in lin] for lin in lins]
+    table = torch.tensor([[t.data_ptr() for t in lin] for lin in d], dtype=torch.int64, device=DEV)
+    i32 = lambda *shape: torch.zeros(shape, dtype=torch.int32, device=DEV)
+    idx = (torch.arange(T * k, device=DEV) % E).int()
+    d_x, res = dev(synth.activations(9801, T, Kk).view(np.uint16)), []
+    for few in (16, T):
+        off, perm, inv = i32(E + 1), i32(T * k), i32(T * k)
+        out = torch.zeros((T * k, N), dtype=torch.float32, device=DEV)
+        a_had = torch.zeros((T * k, Kk), dtype=torch.float16, device=DEV)
+        with knobs(BERTH_MOE_FEW_TOKENS=few):
+            scratch = torch.zeros(K.moe.permute_scratch_bytes(T, k, E), dtype=torch.uint8, device=DEV)
+            K.moe.permute(idx.data_ptr(), off.data_ptr(), perm.data_ptr(), inv.data_ptr(), scratch.data_ptr(), T, k, E)
+            K.moe.grouped_exl3(d_x.data_ptr(), None, perm.data_ptr(), k, table.data_ptr(), 1, 0, 1, out.data_ptr(), None,
+                               scratch.data_ptr(), a_had.data_ptr(), T, k, E, Kk, N, bits, 2, True)
+            torch.cuda.synchronize()
+        assert (out != 0).any(dim=1).all()
+        res.append(out)
+    assert torch.equal(res[0], res[1])
