@@ -1208,17 +1208,38 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
         // time is about that of four tokens plus its own (1, 4 and 6 tokens of H = 2048: 13, 20 and
         // 30 us), so the count with the fewest whole rounds of the chip wins.  1500 tokens x 128 experts:
         // six tokens in one round of 250 workgroups 30 us, four in 375 39.5.
+        const int nslab = (E + kSlabExperts - 1) / kSlabExperts;
+        constexpr int kSlabLdsMax = 144 * 1024;
+        int tt = 1;
+        long best = -1;
+        for (const int c : {1, 2, 3, 4, 6}) {
+            const long groups_c = (T + c - 1) / c;
+            if (route_slab_lds_bytes(p.nseg, c) > kSlabLdsMax || groups_c * kRouteCounterStride > kCounters) continue;
+            const long cost = ((long)nslab * groups_c + ws.cu_count - 1) / ws.cu_count * (4 + c);
+            if (best < 0 || cost < best) { best = cost; tt = c; }
+        }
         // More than 128 experts and passes of 32 segments that are nearly full: tiles of sixteen tokens, with
-        // slabs of 16 experts where that is one round of the chip.  us, slabs of 128 -> tiles: H = 2048, 512
-        // experts at 16 / 64 / 256 / 1500 tokens 13.4 / 14.9 / 20.2 / 82.2 -> 12.4 / 13.2 / 16.0 / 62.7; a
-        // short pass does not pay for the hand-over of the narrower slabs (H = 1024, 512 experts at 64 / 1500
-        // tokens 11.6 / 48.7 -> 12.9 / 56.9), up to 128 experts need none without (9.4 at 64 tokens).
+        // slabs of 16 experts where that is one round of the chip, where they are the quicker form.  The cost above is
+        // about half of the us beyond the first five, also here: 5 for a round of 16 experts and one more per sixteen slabs
+        // that hand over to one workgroup, 2 and 5 per round of 32.  Up to eight tokens the slabs of 128 are too few
+        // to pull the router weight in from memory.  us, slabs of 128 -> tiles, H = 2048, each call a weight of its own:
+        //   512 experts at 2 / 8 / 16 / 64 / 128 tokens  18.6 17.3 16.6 15.9 16.9 -> 15.3 16.4 18.4 17.7 17.4,
+        //               at 256 / 384 / 512 / 1500        19.4 25.6 33.0 81.8 -> 19.5 28.6 29.5 66.4
+        //   256 experts at 8 / 64 / 256 / 384 / 1500     15.9 14.7 15.8 18.6 43.9 -> 15.1 16.1 15.9 17.7 37.2
+        //   160 experts at 8 / 64 / 256 / 384 / 1500     16.2 14.7 15.6 18.1 44.7 -> 13.9 14.8 14.5 14.6 27.0
+        // (H = 1920, 30 segments, and H = 4096 the same way round).  With the weight in the caches, sparser passes: H = 1024, 512
+        // experts at 64 / 1500 tokens 11.5 / 48.9 -> 16.2 / 59.9; H = 2112 at 1500 101 -> 104.  Up to 128 experts need no
+        // hand-over without tiles: H = 2048 at 64 / 1500 tokens 10.6 / 22.4 -> 12.0 / 23.5 (but H = 4096 at 1500 50 -> 39).
+        // BERTH_MOE_ROUTE_SLAB=2: tiles wherever they can serve.
         const long tile_groups = (T + kTileTokens - 1) / kTileTokens;
         const int tile_experts = tile_groups * ((E + 15) / 16) <= ws.cu_count ? 16 : 32;
         const long tile_slabs = (E + tile_experts - 1) / tile_experts;
+        const long tile_cost = tile_experts == 16 ? 5 + tile_slabs / 16
+                                                  : 2 + 5 * ((tile_groups * tile_slabs + ws.cu_count - 1) / ws.cu_count);
         const int tile_segs = (p.nseg + kTileSegs - 1) / kTileSegs * kTileSegs;
-        if (T > 1 && E > kSlabExperts && p.nseg >= kTileSegs && tile_segs * 8 <= p.nseg * 9 && (uintptr_t)x % 16 == 0 &&
-            tile_groups * kRouteCounterStride <= kCounters) {
+        const bool tiles_serve = T > 1 && E > kSlabExperts && (uintptr_t)x % 16 == 0 && tile_groups * kRouteCounterStride <= kCounters;
+        const bool tiles_quicker = tile_segs * 8 <= p.nseg * 9 && (T <= kTileTokens / 2 || best < 0 || tile_cost <= best);
+        if (tiles_serve && (tiles_quicker || knobs().moe_route_slab == 2)) {
             const dim3 grid((unsigned)tile_groups, (unsigned)tile_slabs);
             const int lds = route_tile_lds_bytes(tile_experts);
             auto launch = [&](void (*kernel)(RouteParams), bool (&raised)[64]) {
@@ -1231,16 +1252,6 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
             hip_ok(hipGetLastError(), "moe_route_slab_kernel launch");
             return "moe_route_slab_kernel<" + std::to_string(kTileTokens) + "," + std::to_string(tile_experts) + "> grid=" +
                    std::to_string(tile_slabs) + "x" + std::to_string(tile_groups);
-        }
-        const int nslab = (E + kSlabExperts - 1) / kSlabExperts;
-        constexpr int kSlabLdsMax = 144 * 1024;
-        int tt = 1;
-        long best = -1;
-        for (const int c : {1, 2, 3, 4, 6}) {
-            const long groups_c = (T + c - 1) / c;
-            if (route_slab_lds_bytes(p.nseg, c) > kSlabLdsMax || groups_c * kRouteCounterStride > kCounters) continue;
-            const long cost = ((long)nslab * groups_c + ws.cu_count - 1) / ws.cu_count * (4 + c);
-            if (best < 0 || cost < best) { best = cost; tt = c; }
         }
         const int tgroups = (T + tt - 1) / tt;
         if (route_slab_lds_bytes(p.nseg, tt) <= kSlabLdsMax && (long)tgroups * kRouteCounterStride <= kCounters) {

@@ -167,7 +167,8 @@ def test_routing_tiles_of_sixteen_tokens(T, H, E, k, experts):
     """Ragged token groups and slabs, a last pass with one segment missing, three passes: the oracle's bits."""
     x, wr = synth.activations(T, T, H), synth.router_weight(E, H, E)
     bias = synth.zipf_bias(5, E) if E % 4 == 0 else None
-    idx, w, logits = _route(x, wr, k, bias=bias)
+    with knobs(BERTH_MOE_ROUTE_SLAB=2):         # also where the other form is the quicker one
+        idx, w, logits = _route(x, wr, k, bias=bias)
     assert "moe_route_slab_kernel<16," in K.moe.last_launch(), K.moe.last_launch()
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert f"moe_route_slab_kernel<16,{experts}>" in K.moe.last_launch(), K.moe.last_launch()
@@ -175,6 +176,24 @@ def test_routing_tiles_of_sixteen_tokens(T, H, E, k, experts):
     assert np.array_equal(logits.view(np.uint32), ol.view(np.uint32))
     assert np.array_equal(idx, oi)
     assert np.allclose(w, ow, rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("T,H,E,tokens", [
+    (8, 2048, 512, 16), (9, 2048, 512, 1), (64, 2048, 512, 1), (128, 2048, 512, 2), (256, 2048, 512, 16), (384, 2048, 512, 6),
+    (512, 2048, 512, 16), (128, 2048, 256, 1), (129, 2048, 256, 16), (500, 1856, 160, 16), (500, 1792, 160, 4), (500, 2112, 160, 4)])
+def test_routing_form_by_whole_rounds(T, H, E, tokens):
+    """On either side of the rule's lines: tokens of a workgroup, and the same logits and choices from the other forms."""
+    x, wr = synth.activations(T, T, H), synth.router_weight(E, H, E)
+    res = []
+    for form in (1, 2, 0):
+        with knobs(BERTH_MOE_ROUTE_SLAB=form):
+            res.append(_route(x, wr, 8))
+        if form == 1 and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert f"moe_route_slab_kernel<{tokens}" in K.moe.last_launch(), K.moe.last_launch()
+        if form == 2:
+            assert "moe_route_slab_kernel<16," in K.moe.last_launch(), K.moe.last_launch()
+    for other in res[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(res[0], other))
 
 
 @pytest.mark.parametrize("T,H,E,k,I,bits", [
