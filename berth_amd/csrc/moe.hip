@@ -552,7 +552,8 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
 // w and w + 16 of every 32; their weights are requested at once, ahead of the token rows, which go
 // through LDS (lanes that read sixteen rows from memory cost an address cycle each).  Step i of a segment
 // multiplies its rows 4 i .. 4 i + 3: lane 16 q + j holds row 4 i + q, of token j and of expert j, or of
-// experts 2 j and 2 j + 1 with a tile each for the even and the odd ones.
+// experts 2 j and 2 j + 1 with a tile each for the even and the odd ones.  (More than one slab: the launch
+// takes more than 128 experts.)
 constexpr int kTileTokens = 16, kTileSegs = 32;
 constexpr int kTileXStride = kTileSegs * kRouteSeg + 8;             // halves; sixteen rows' same columns in different banks
 inline __host__ __device__ constexpr int route_tile_lds_bytes(int experts)
@@ -638,46 +639,35 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
             load_x(s0 + kTileSegs);
         }
         __syncthreads();
+        // (the next pass writes only the token rows ahead of its first barrier)
         if (mine) v = route_add_segments(v, s_parts + threadIdx.x, TOKENS * EXPERTS, min(kTileSegs, p.nseg - s0));
-        if (more) __syncthreads();                                  // the sums have been read
     }
     if (p.bias) v += bias;
     if (mine && p.logits) p.logits[(size_t)(t0 + tt) * p.E + e0 + c] = v;
 
     // ---- logits to memory ([T][E], the head of the segment-sum scratch); the last slab of the token
     // group to arrive selects, a wave per token
-    if (nslab > 1) {
-        if (mine)
-            __hip_atomic_store(p.parts + (size_t)(t0 + tt) * p.E + e0 + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        wait_own_stores();
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            unsigned* counter = p.counters + (size_t)grp * kRouteCounterStride;
-            const unsigned old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            s_last = (old == (unsigned)(nslab - 1)) ? 1u : 0u;
-            if (s_last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
-        if (!s_last) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    } else {
-        __syncthreads();                                            // every sum is formed: the segment sums can go
-        if (mine) s_parts[threadIdx.x] = v;
-        __syncthreads();
+    if (mine)
+        __hip_atomic_store(p.parts + (size_t)(t0 + tt) * p.E + e0 + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    wait_own_stores();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned* counter = p.counters + (size_t)grp * kRouteCounterStride;
+        const unsigned old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = (old == (unsigned)(nslab - 1)) ? 1u : 0u;
+        if (s_last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    __syncthreads();
+    if (!s_last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     const int t = t0 + wave;
     if (t >= p.T) return;
     float lg[kRoutePer];
 #pragma unroll
     for (int i = 0; i < kRoutePer; ++i) {
         const int e = lane + 64 * i;
-        lg[i] = -INFINITY;
-        if (nslab > 1) {
-            if (e < p.E) lg[i] = __hip_atomic_load(p.parts + (size_t)t * p.E + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else if (i == 0 && lane < min(EXPERTS, p.E)) {
-            lg[i] = s_parts[wave * EXPERTS + lane];
-        }
+        lg[i] = e < p.E ? __hip_atomic_load(p.parts + (size_t)t * p.E + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
     }
     route_topk(lg, lane, p, t);
 }
