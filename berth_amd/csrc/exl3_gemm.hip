@@ -528,10 +528,7 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
         const size_t bytes = elements * (m.c_fp32 ? 4 : 2);
         return apart(m.a, in_bytes, c, bytes) && apart(m.a_had, rows_bytes * slabs, c, bytes);
     };
-    // (More than 8 rows of a short K keep the launch that rotates: it is part of what is tested of such bundles.
-    // A decoder layer of 12 rows and 1024 columns would gain 1 us of 48.)
-    bool rotate = plan.rows.ok && plan.rows.rotate && (m.size_m <= 8 || m.size_k > 1024) &&
-                  apart(m.a, in_bytes, m.a_had, rows_bytes * slabs);
+    bool rotate = plan.rows.ok && plan.rows.rotate && apart(m.a, in_bytes, m.a_had, rows_bytes * slabs);
     // The outputs of slices whose lists are in device memory cannot be looked at here: they may lie over the input or
     // its rotated rows, and a source may have no slice that would leave its slab.  Those keep the two launches.
     if (!sliced) rotate = rotate && output_apart(m.c, (size_t)m.bszm_out * m.size_m * m.size_n);

@@ -73,8 +73,8 @@ def _many_row_cases():
 
 @pytest.mark.parametrize("rows,Kk,widths,bits,fp32,host_lists", _many_row_cases())
 def test_sliced_bundle_many_rows(rows, Kk, widths, bits, fp32, host_lists):
-    """More than 8 rows: the bundle is one dense MFMA launch (32-, 128- or 256-row tiles by row
-    count and width) behind one launch that rotates the input once per source.  Each source
+    """More than 8 rows: the bundle is one MFMA launch (few-row kernel, 32-, 128- or 256-row tiles by row
+    count and width), as a rule behind one launch that rotates the input once per source.  Each source
     against the oracle's single linear, the rotated slabs bit for bit, lists by value and from
     device memory, and a second call for the same bits."""
     gpu = Gpu(0)
@@ -90,7 +90,9 @@ def test_sliced_bundle_many_rows(rows, Kk, widths, bits, fp32, host_lists):
     want_text = "by value" if by_value else "sliced x"
     torch.cuda.synchronize()
     launch = K.ops.last_launch()
-    assert want_text in launch and "had_r_128_slabs_kernel" in launch and "exl3_gemm" in launch, launch
+    assert want_text in launch and "exl3_gemm" in launch, launch
+    # up to 32 rows with the lists by value the launch may rotate the input itself
+    assert ("had_r_128_slabs_kernel" in launch) != (",rotate>" in launch and by_value and rows <= 32), launch
     first = [o.cpu().numpy().copy() for o in outs]
     for i, (tr, suh, svh) in enumerate(lins_np):
         want, want_had = O.linear(x, tr, suh, svh, Kk, widths[i], bits, 2, out_fp32=fp32)

@@ -149,13 +149,14 @@ def test_rotation_inside_the_launch(rows, Kk, N, bits, cb, fp32):
     assert close(res[0][0].cpu().numpy() if fp32 else host_f16(res[0][0]), want)[0] == 0
 
 
-@pytest.mark.parametrize("rows,by_value", [(3, False), (8, False), (9, True), (20, True), (20, False)])
-def test_bundle_that_rotates_its_input(rows, by_value):
+@pytest.mark.parametrize("rows,by_value,Kk", [(3, False, 2304), (8, False, 2304), (9, True, 2304), (20, True, 2304), (20, False, 2304),
+                                              (9, True, 512), (16, True, 1024), (31, True, 768)])
+def test_bundle_that_rotates_its_input(rows, by_value, Kk):
     """Three sources of one input, two slices of the first: every source's rotated rows are left once.  With the lists in
     device memory, which no check of the host sees, a launch of its own rotates."""
     from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
     gpu = Gpu(0)
-    Kk, widths, bits = 2304, (1024, 512, 512), 3
+    widths, bits = (1024, 512, 512), 3
     lins = [synth.linear(700 + i, Kk, n, bits) for i, n in enumerate(widths)]
     multi = Exl3MultiLinear(gpu, [Exl3Linear(gpu, f"l{i}", *l) for i, l in enumerate(lins)])
     x = synth.activations(710 + rows, rows, Kk)
