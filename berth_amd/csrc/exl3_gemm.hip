@@ -137,7 +137,7 @@ static RowsPlan plan_rows(const Workspace& ws, int slices, int slabs, int size_m
             unsigned nb = 0;                                        // most 128 blocks that a part touches
             for (unsigned s = 0; s < S; ++s) nb = std::max(nb, ((s + 1) * TR4 / S + 1) / 2 - s * TR4 / S / 2);
             pl.lds_rotate = lds + rows_rot_lds_bytes((int)(2 * nb), mt);
-            pl.rotate = nb * (unsigned)size_m <= (unsigned)(slabs > 1 ? kRowsRotItems : kRowsRotItems - 64) && pl.lds_rotate <= 160 * 1024;
+            pl.rotate = nb * (unsigned)size_m <= (unsigned)kRowsRotItems && pl.lds_rotate <= 160 * 1024;
         }
         return pl;
     }

@@ -53,12 +53,16 @@ constexpr int kRowsStride = 132;            // floats per row of a partial colum
 // Launches that rotate the input themselves (ROT): the most (row, 128 block) items a workgroup takes, sixteen
 // lanes each, and the LDS of their result, `units` units of 64 k behind everything else.  Where a column
 // block is cut into parts of its own, a workgroup needs a part of K only, so all workgroups of a part of
-// K rotating it cost less than the launch that did it once, as long as it is a few items a lane group:
-// linears of 5 / 8 / 14 / 24 rows, us, two launches -> one: 4096x4096 11.1 / 11.6 / 12.4 / 14.5 -> 9.3 / 9.8 / 10.5 /
-// 13.4 (40 .. 96 items), 6144x5120 13.2 / 13.4 / 14.3 / 16.5 -> 11.2 / 11.5 / 13.1 / 15.8 (40 .. 192),
-// 17408x5120 20.8 / 20.8 -> 19.2 / 19.8 (115, 184); 196 items (10240x5120 at 14) 17.0 -> 17.1.  A fourth item a
-// lane group is worth it for bundles, whose launch for the rotation has several inputs (q, k and v of 24
-// rows, 240 items: a layer 115.5 -> 113.9).
+// K rotating it cost less than the launch that did it once, as long as it is a few items a lane group.  us, two
+// launches -> one, weights from memory:
+//   linears   4096x4096 at 5 / 16 / 32 rows (20 / 64 / 128 items)     11.7 / 13.4 / 17.2 -> 10.1 / 11.6 / 16.0
+//             6144x5120 at 5 / 24 / 28 / 32 (40 / 192 / 224 / 256)    14.3 / 17.7 / 18.7 / 19.6 -> 12.6 / 16.7 / 17.8 / 19.1
+//             10240x5120 at 8 / 14 / 17 (112 / 196 / 238)             17.8 / 18.9 / 20.8 -> 16.5 / 18.3 / 19.6
+//             17408x5120 at 8 / 11 (184 / 253)                        22.7 / 23.0 -> 21.9 / 22.7
+//   q, k, v   5120 -> 6144 + 2 x 1024 at 9 / 24 (90 / 240)            17.1 / 20.4 -> 15.6 / 19.3
+//             4096 -> 4096 + 2 x 1024 at 16 / 32 (112 / 224)          15.6 / 20.0 -> 13.8 / 18.4
+// Of 100 linears and 47 bundles of up to 256 items, four a lane group, none lost more than 0.1; the gain is 1.6 to 2.2 up to
+// 64 items and 0.2 to 1.6 above 192.
 constexpr int kRowsRotItems = 256;
 __host__ __device__ constexpr size_t rows_rot_lds_bytes(int units, int mt) { return (size_t)units * mt * 2048; }
 

@@ -121,6 +121,8 @@ def test_block_with_fused_norm_equals_the_separate_calls(rows, H, I, bits):
     (16, 4096, 3968, 5, 0),         # 31 blocks
     (17, 2176, 3200, 6, 2),         # a second tile with one row
     (24, 6144, 5120, 4, 2),         # 192 items: three a lane group
+    (32, 6144, 5120, 3, 2),         # 256: four
+    (17, 10240, 5120, 2, 2),        # 238: some lane groups with three
     (32, 1024, 2048, 2, 2),
     (8, 17408, 1024, 8, 2),
 ])
