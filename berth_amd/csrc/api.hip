@@ -258,8 +258,8 @@ extern "C" int berth_exl3_linear(const void* a, const void* trellis, void* c, co
 // The array has no initialiser, so it is zero when the code object is loaded, and every launch
 // leaves the counters and accumulators it used at zero again: nothing has to clear it, and a
 // first call inside a stream capture records only the linear's own launches (one kernel; two for
-// 2..8 rows of a weight large enough for the few-row MFMA kernel, whose input a launch of its own
-// rotates into the partial sums' scratch).
+// 2..8 rows of a weight large enough for the few-row MFMA kernel where that one does not rotate its input
+// itself: a launch ahead of it then leaves the rotated rows in the partial sums' scratch too).
 namespace {
 constexpr size_t kNoAllocPartialBytes = (size_t)8 << 20;
 constexpr int kNoAllocCounters = 65536;
@@ -662,7 +662,8 @@ extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* g
 // block.  One row whose linears take the streaming kernel: two launches, the norm formed while
 // the gate / up launch rotates its input, the sum added where the down launch writes its output.
 // Rows on the MFMA kernels: four launches, the norm formed where the input is rotated, the
-// activation likewise, the sum added where the down launch writes.
+// activation likewise, the sum added where the down launch writes (row blocks: the activation where
+// gate's and up's tiles are finished, and a launch more where down shares tiles).
 extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* residual_out, const berth_rms_norm* norm,
                                     const berth_exl3_lin* lins, void* h_norm, void* gate_out, void* up_out, void* a_had,
                                     void* act_had, void* y, int size_m, int hidden, int intermediate, int k_bits,

@@ -50,8 +50,8 @@ struct GemmParams {
     ExpertLin lin;              // dense mode
     void* c[2];
     int M, K, N, out_fp32;
-    // grouped mode (problems != nullptr): blockIdx.z = problem (<= BM rows),
-    // blockIdx.y = which of the launch's linears
+    // grouped mode (problems != nullptr): group_tile says which problem (<= BM rows), linear of the
+    // launch and column block a workgroup takes
     const ExpertLin* experts;
     const GroupProblem* problems;
     const int* num_problems;
