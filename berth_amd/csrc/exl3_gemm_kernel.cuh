@@ -214,7 +214,9 @@ constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: 
 // `slot`, 8 k values) is one 16-byte load straight from the rotated rows, so
 // there is no LDS tile and no barrier in the loop.  Trellis and A registers are
 // reloaded for the wave's next k-block as soon as a step has consumed them
-// (rolling prefetch, one k-block ahead); on the last k-block the reload reads
+// (rolling prefetch, one k-block ahead; the activation behind the products that read it: asked for ahead of
+// them it lands in other registers and is moved, 16 of the 513 vector instructions of a k-block.  Layers of 64
+// and 20 tokens x 128 experts 120.7 -> 118.3 and 106.4 -> 104.3 us); on the last k-block the reload reads
 // the same addresses again and is ignored, which keeps the loop free of branches.
 // `requested` is called when the first loads are on their way.
 template <int BITS, int CB, typename F>
@@ -261,14 +263,14 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
                     b[f][h] = __builtin_bit_cast(half8_t, q);
                 }
             settle<CB>(b[0][0], b[1][0], b[0][1], b[1][1]);
-            const half8_t a0 = av[st][0], a1 = av[st][1];
+            __builtin_amdgcn_sched_barrier(0);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[st][0], b[0][0], acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[st][0], b[1][0], acc[1], 0, 0, 0);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[st][1], b[0][1], acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[st][1], b[1][1], acc[1], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
             av[st][0] = anx[4 * st];
             av[st][1] = anx[4 * st + 1];
-            __builtin_amdgcn_sched_barrier(0);
-            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b[0][0], acc[0], 0, 0, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b[1][0], acc[1], 0, 0, 0);
-            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b[0][1], acc[0], 0, 0, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b[1][1], acc[1], 0, 0, 0);
         }
     }
 }
