@@ -275,6 +275,81 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
     }
 }
 
+// The same for an expert whose rows all fit into sixteen: v_mfma_f32_16x16x32_f16, half the matrix work of the
+// products above.  A step is 64 rows of K x 32 columns: lanes l and l + 8 of a sixteen take two neighbouring tiles,
+// the four sixteens four tile rows (as in the few-row kernel), and both halves of a wave's columns multiply the
+// same activation.  What the matrix units take there the decode does not get, on a pipe of its own or not: a layer of
+// 64 tokens x 128 experts, four rows an expert, 126 -> 110 us.  The sums of sixteen rows form in another order
+// than those of 32, so that the choice must not depend on how a call cuts its problems: `lone` says that the
+// expert has no more rows, in whichever list it is.
+template <int BITS, int CB, typename F>
+__device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
+                                                   const int arow, const int K, const int lane, float4_t (&acc)[2][2], F requested)
+{
+    constexpr int tile_dw = 8 * BITS;
+    const int l16 = lane & 15, lg = lane >> 4;
+    const global_ptr<const uint32_t> tb = as_global(trellis) + (size_t)lg * row_dw +
+                                         (size_t)((nw >> 4) + (l16 >> 3)) * tile_dw + (l16 & 7) * BITS;
+    const global_ptr<const half8_t> ab = (global_ptr<const half8_t>)(as_global(a_had) + (size_t)arow * K + 16 * lg);
+    uint32_t cur[4][BITS];
+    half8_t av[2][2];
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+        load_tile_dwords<BITS>(tb + (size_t)(st / 2 * 4) * row_dw + st % 2 * 2 * tile_dw, cur[st]);
+        if (st % 2 == 0) {
+            av[st / 2][0] = ab[8 * (st / 2)];
+            av[st / 2][1] = ab[8 * (st / 2) + 1];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    requested();
+    const int KB = K >> 7;
+    for (int kb = 0; kb < KB; ++kb) {
+        const int nkb = min(kb + 1, KB - 1);
+        const global_ptr<const uint32_t> tnx = tb + (size_t)(nkb * 8) * row_dw;
+        const global_ptr<const half8_t> anx = ab + nkb * 16;
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            const int ks = st / 2, cg = st % 2;
+            uint32_t prev = fetch_prev(lane, cur[st][BITS - 1]);
+            uint32_t w2[16];
+            decode_lane<BITS, CB>(cur[st], prev, w2);
+            load_tile_dwords<BITS>(tnx + (size_t)(4 * ks) * row_dw + cg * 2 * tile_dw, cur[st]);
+            half8_t b[2][2];
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint4 q = {w2[2 * f + h], w2[4 + 2 * f + h], w2[8 + 2 * f + h], w2[12 + 2 * f + h]};
+                    b[f][h] = __builtin_bit_cast(half8_t, q);
+                }
+            settle<CB>(b[0][0], b[1][0], b[0][1], b[1][1]);
+            __builtin_amdgcn_sched_barrier(0);
+            acc[cg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[ks][0], b[0][0], acc[cg][0], 0, 0, 0);
+            acc[cg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[ks][0], b[1][0], acc[cg][1], 0, 0, 0);
+            acc[cg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[ks][1], b[0][1], acc[cg][0], 0, 0, 0);
+            acc[cg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[ks][1], b[1][1], acc[cg][1], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (cg == 1) {
+                av[ks][0] = anx[8 * ks];
+                av[ks][1] = anx[8 * ks + 1];
+            }
+        }
+    }
+}
+// its sums to the fp32 tile, 64 columns from z on
+template <int STRIDE>
+__device__ __forceinline__ void stage_16_rows(float* z, const float4_t (&acc)[2][2], const int lane)
+{
+    float* const at = z + 4 * (lane >> 4) * STRIDE + ((lane >> 3) & 1) * 16 + (lane & 7);
+#pragma unroll
+    for (int cg = 0; cg < 2; ++cg)
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) at[r * STRIDE + 32 * cg + 8 * f] = acc[cg][f][r];
+}
+
 // one output tile: rows of problem / row block `tile_y`, 256 columns
 template <int BITS, int CB, int MB, bool DENSE>  // MB = 32-row blocks per workgroup; DENSE: never a problem list
 __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y, const int nblk, const KRange kr,
@@ -297,6 +372,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     void* cout = p.c[0];
     int N = p.N, ldc = p.N, nblk_lin = nblk;
     const int32_t* a_rows = nullptr;
+    bool lone = false;                                  // accumulate_16_rows
     if constexpr (DENSE) {
         const TileView v = dense_tile_view(p, nblk);
         if (v.empty) return;                            // the same for every workgroup that shares the tile
@@ -319,6 +395,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         a_had = p.a_had[which];
         cout = p.c[which];
         if (gp.expert != p.shared_expert) a_rows = p.a_rows;
+        lone = MB == 1 && gp.lone && kr.parts == 1;
     }
     // row r of the tile in a_had
     auto a_row_at = [&](int r) { return !DENSE && a_rows ? as_global(a_rows)[m0 + r] : m0 + r; };
@@ -349,7 +426,12 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[mb][f][r] = 0.0f;
 
-    if constexpr (MB == 1) {
+    float4_t acc16[2][2] = {};
+    if (lone) {
+        if (active)
+            accumulate_16_rows<BITS, CB>(lin.trellis, row_dw, nw, a_had, a_row_at(min(lane & 15, rows_here - 1)), p.K, lane, acc16, keep_scale);
+        else keep_scale();
+    } else if constexpr (MB == 1) {
         if (active && kr.kb0 < kr.kb1)
             accumulate_32_rows<BITS, CB>(lin.trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
                                          kr.step, lane, acc[0], keep_scale);      // (rows past the problem repeat its last row)
@@ -603,7 +685,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     for (int mb = 0; mb < MB; ++mb) {
         if (mb * 32 >= rows_here) break;                        // workgroup-uniform
         __syncthreads();
-        if (active) {
+        if (lone) {
+            if (active) stage_16_rows<kZStride>(z_tile + wave * 64, acc16, lane);
+        } else if (active) {
 #pragma unroll
             for (int f = 0; f < 2; ++f)
 #pragma unroll
@@ -714,7 +798,7 @@ __global__ __launch_bounds__(256, MB == 1 && !DENSE ? 3 : 2) void exl3_gemm_kern
 // group_tile's of one linear; linears lin_base, lin_base + 1 and, for its input scales,
 // lin_base + 2 of an expert.  Gate and up are written too (fp16, c[0] and c[1]).
 // The values are those of the 32-row tiles and of moe_had_rows_kernel behind them.
-// What bounds it: the decode, as there; the end of a row is three rotations (of 128 values by sixteen
+// What bounds it: the decode, as there (experts of up to sixteen rows: accumulate_16_rows); the end of a row is three rotations (of 128 values by sixteen
 // lanes) instead of two, against a launch that reads both factors back: layer of 64 tokens x 128 experts
 // x 768 122.6 -> 121.4 us, of 20 tokens x 128 experts x 896 (seven column blocks, which 256-column tiles
 // cover as eight) 107 -> 94.
@@ -735,7 +819,7 @@ __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
     auto linear = [&](int l) { return shared ? p.shared[p.lin_base + l] : p.experts[gp.expert * p.lins_per_expert + p.lin_base + l]; };
     const ExpertLin lin = linear(which);
     const int rows = gp.nrows;
-    int arow = gp.row0 + min(slot, rows - 1);           // rows past the problem repeat its last row
+    int arow = gp.row0 + min(gp.lone ? slot & 15 : slot, rows - 1);   // rows past the problem repeat its last row
     if (p.a_rows && !shared) arow = as_global(p.a_rows)[arow];
 
     // the output scales of gate and up, the input scales of down: asked for first, as in gemm_tile
@@ -745,24 +829,31 @@ __global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
         const ExpertLin l = linear((int)threadIdx.x >> 4);
         scale_mine = ((global_ptr<const half8_t>)as_global((threadIdx.x < 32 ? l.svh : l.suh) + n0))[threadIdx.x & 15];
     }
-    float16_t acc[2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[f][r] = 0.0f;
-    accumulate_32_rows<BITS, CB>(lin.trellis, (size_t)(p.N >> 4) * (8 * BITS), n0 + (wave & 1) * 64, p.a_had[which], arow, p.K, 0,
-                                 p.K >> 7, 1, lane, acc, [&]() {
+    const size_t row_dw = (size_t)(p.N >> 4) * (8 * BITS);
+    const int nw = n0 + (wave & 1) * 64;
+    auto keep_scale = [&]() {
         if (threadIdx.x < 48) s_scale[threadIdx.x >> 4][threadIdx.x & 15] = scale_mine;
-    });
-
+    };
     // sixteen lanes a row, eight columns of both factors each
     const int chunk = had_chunk(lane);
     const int at = n0 + 8 * chunk;
-    const int col = wave * 64 + (slot >> 3) * 16 + (slot & 7);
+    if (gp.lone) {
+        float4_t acc[2][2] = {};
+        accumulate_16_rows<BITS, CB>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, lane, acc, keep_scale);
+        stage_16_rows<kZStride>(z_tile + wave * 64, acc, lane);
+    } else {
+        float16_t acc[2];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
+        for (int f = 0; f < 2; ++f)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) z_tile[(8 * (r >> 2) + 4 * half_id + (r & 3)) * kZStride + col + 8 * f] = acc[f][r];
+            for (int r = 0; r < 16; ++r) acc[f][r] = 0.0f;
+        accumulate_32_rows<BITS, CB>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, 0, p.K >> 7, 1, lane, acc, keep_scale);
+        const int col = wave * 64 + (slot >> 3) * 16 + (slot & 7);
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z_tile[(8 * (r >> 2) + 4 * half_id + (r & 3)) * kZStride + col + 8 * f] = acc[f][r];
+    }
     __syncthreads();
 #pragma unroll 1
     for (int pass = 0; pass < 2; ++pass) {
@@ -970,7 +1061,7 @@ __device__ __forceinline__ void gemm_half_tile(const GemmParams& p, const GroupP
 // it has, needed or not): gate + up and down of 800 tokens that choose 8 of 128 experts 137 + 82 -> 119 +
 // 70 us, of 1500 tokens (94 rows an expert) 133 + 89 -> 131 + 85.
 // A launch of no more tiles than compute units runs them as halves of 128 columns (gemm_half_tile; bits the same),
-// the second halves behind the first: a workgroup alone on its compute unit takes nearly as long as two
+// the second halves behind the first (experts of up to sixteen rows whole): a workgroup alone on its compute unit takes nearly as long as two
 // that share one.  Layers of 2048 x 768: 200 tokens that choose 4 of 16 experts 69.7 -> 54.4 us (64 and 128 tiles), of
 // 1024 x 512, 300 tokens 58.2 -> 47.0, of 2048 x 1024, 150 tokens that choose 8 of 32 (256 tiles) 84.9 -> 80.8;
 // 400 tokens that choose 6 of 16 (256 tiles, half of them of 128 rows) 104.4 -> 105.
@@ -1004,8 +1095,10 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
     const int half = gt.problem >= problems;
     if (half && (!halves || gt.problem >= 2 * problems)) return;
     const int z = gt.problem - half * problems;
-    if (halves) {
-        const GroupProblem gp = z < big ? p.big_problems[z] : p.problems[z - big];
+    const GroupProblem* const list = z < big ? p.big_problems : p.problems;
+    const int at = z < big ? z : z - big;
+    const GroupProblem gp = list[at];
+    if (halves && !gp.lone) {
         const int n0 = gt.col * 256 + 128 * half;
         if (gp.nrows > 96) gemm_half_tile<BITS, CB, 4>(p, gp, gt.which, n0, smem);
         else if (gp.nrows > 64) gemm_half_tile<BITS, CB, 3>(p, gp, gt.which, n0, smem);
@@ -1013,14 +1106,12 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
         else gemm_half_tile<BITS, CB, 1>(p, gp, gt.which, n0, smem);
         return;
     }
-    if (z < big) {
-        const int rows = p.big_problems[z].nrows;               // as many 32-row blocks as the problem has
-        if (rows > 96) gemm_tile<BITS, CB, 4, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
-        else if (rows > 64) gemm_tile<BITS, CB, 3, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
-        else gemm_tile<BITS, CB, 2, false>(p, z, gt.col, kr, gt.which, smem, p.big_problems);
-        return;
-    }
-    gemm_tile<BITS, CB, 1, false>(p, z - big, gt.col, kr, gt.which, smem, p.problems);
+    if (half) return;                                   // (an expert of at most sixteen rows: whole)
+    // as many 32-row blocks as the problem has
+    if (gp.nrows > 96) gemm_tile<BITS, CB, 4, false>(p, at, gt.col, kr, gt.which, smem, list);
+    else if (gp.nrows > 64) gemm_tile<BITS, CB, 3, false>(p, at, gt.col, kr, gt.which, smem, list);
+    else if (gp.nrows > 32) gemm_tile<BITS, CB, 2, false>(p, at, gt.col, kr, gt.which, smem, list);
+    else gemm_tile<BITS, CB, 1, false>(p, at, gt.col, kr, gt.which, smem, list);
 }
 
 // Dense launches whose tile count does not divide over the compute units: the

@@ -784,11 +784,12 @@ __device__ __forceinline__ void permute_pairs(const PermuteParams& p, const int 
             if (p.use_valu) {
                 p.vprob[pfirst[tid]] = GroupProblem{tid, off[tid], m, 0};
             } else {
+                const int lone = m <= kLoneRows;
                 int r = 0;
                 for (int j = bfirst[tid]; m - r >= p.big_min; r += kGemmBigRows, ++j)
-                    p.bprob[j] = GroupProblem{tid, off[tid] + r, min(kGemmBigRows, m - r), 0};
+                    p.bprob[j] = GroupProblem{tid, off[tid] + r, min(kGemmBigRows, m - r), lone};
                 for (int j = pfirst[tid]; r < m; r += p.small_rows, ++j)
-                    p.mprob[j] = GroupProblem{tid, off[tid] + r, min(p.small_rows, m - r), 0};
+                    p.mprob[j] = GroupProblem{tid, off[tid] + r, min(p.small_rows, m - r), lone};
             }
         }
     }

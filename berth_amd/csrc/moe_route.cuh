@@ -20,8 +20,9 @@ struct GroupProblem {
     int expert;
     int row0;
     int nrows;
-    int pad;
+    int lone;           // 1: all rows of the expert, at most sixteen (whichever list it is in)
 };
+constexpr int kLoneRows = 16;
 
 constexpr int kRouteSeg = 64;       // rows of the router weight per partial sum
 constexpr int kRouteTT = 4;         // tokens per route workgroup

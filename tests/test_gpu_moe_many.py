@@ -232,6 +232,35 @@ def test_gate_up_and_the_next_rotation_in_one_launch(T, H, E, k, I, bits, shared
     assert torch.equal(again, out)
 
 
+@pytest.mark.parametrize("T,H,E,k,I,bits,shared_I", [
+    (140, 256, 20, 2, 384, 4, 0),       # experts on either side of sixteen rows; 240 tiles of gate and up: halves
+    (150, 128, 150, 3, 384, 3, 0),      # nearly all below; whole tiles
+    (16, 384, 2, 1, 128, 5, 128),       # sixteen rows of the always-on expert
+    (60, 384, 5, 1, 640, 2, 0),         # gate, up and the next rotation in one launch
+])
+def test_experts_of_up_to_sixteen_rows(T, H, E, k, I, bits, shared_I):
+    """They take the 16-row matrix instructions whichever list their problem is in (BERTH_MOE_BIG_MIN=9: most of them in
+    that of the 128-row problems): against the oracle, and the same bits for every setting."""
+    gpu, res = Gpu(0), []
+    wr, experts_np, experts, shared_np, shared = _make_layer(gpu, 9900 + T, H, E, I, bits, shared_I, 1.0)
+    x = (synth.activations(9901 + T, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
+    want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, 2, shared=shared_np, shared_I=shared_I)
+    rows = np.bincount(oi.reshape(-1), minlength=E)
+    assert (rows[rows > 0] <= 16).any() or shared_I
+    for big_min in (0, 9, 33):
+        with knobs(BERTH_MOE_BIG_MIN=big_min, BERTH_MOE_FEW_TOKENS=0):
+            layer = MoeLayer(gpu, wr, experts, k, shared=shared)
+            out = torch.zeros((T, H), dtype=torch.float32, device=DEV)
+            idx = torch.zeros((T, k), dtype=torch.int32, device=DEV)
+            w = torch.zeros((T, k), dtype=torch.float32, device=DEV)
+            layer.forward(gpu, dev(x.view(np.uint16)), out, T, idx, w)
+            torch.cuda.synchronize()
+            assert np.array_equal(idx.cpu().numpy(), oi)
+            _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I)
+        res.append(out)
+    assert torch.equal(res[0], res[1]) and torch.equal(res[0], res[2])
+
+
 def test_rows_beyond_four_gigabytes_of_rotated_input():
     """16-row problems over 65535 rows of 32896 columns: the rotated rows span more than 32-bit offsets reach, and the last
     ones are read where they are."""
