@@ -739,8 +739,8 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         p.num_big = g.num_big;
         p.max_big = g.max_big;
         p.S = 1;
-        p.half_tiles = ws.cu_count;
-        const int more = p.half_tiles / (nblocks * g.num_lins);                     // problems whose second halves may come behind
+        p.places = 2 * ws.cu_count;
+        const int more = p.places / (2 * nblocks * g.num_lins);                     // problems that may run as halves
         gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, group_grid(nblocks, g.num_lins, g.max_problems + g.max_big + more));
         hip_ok(hipGetLastError(), "exl3_gemm_mixed_kernel launch");
         return desc + " grouped";

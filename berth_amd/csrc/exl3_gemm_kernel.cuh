@@ -109,7 +109,7 @@ struct GemmParams {
     // grouped: where row r of the sorted order lies in a_had (optional; rows of the always-on expert: at r)
     const int32_t* a_rows;
     int group_lins;             // linears of a problem that are units of their own (1 or 2)
-    int half_tiles;             // exl3_gemm_mixed_kernel: up to this many tiles run as halves of 128 columns
+    int places;                 // exl3_gemm_mixed_kernel: workgroups that run at a time; tiles run as halves of 128 columns up to this many
     _Float16* act_had;          // exl3_gemm_pair_kernel: the down projection's rotated input, in sorted order
 };
 
@@ -1060,14 +1060,18 @@ __device__ __forceinline__ void gemm_half_tile(const GemmParams& p, const GroupP
 // A problem of up to 64 or 96 rows runs as two or three 32-row blocks (the loop multiplies all the blocks
 // it has, needed or not): gate + up and down of 800 tokens that choose 8 of 128 experts 137 + 82 -> 119 +
 // 70 us, of 1500 tokens (94 rows an expert) 133 + 89 -> 131 + 85.
-// A launch of no more tiles than compute units runs them as halves of 128 columns (gemm_half_tile; bits the same),
-// the second halves behind the first (experts of up to sixteen rows whole): a workgroup alone on its compute unit takes nearly as long as two
-// that share one.  Layers of 2048 x 768: 200 tokens that choose 4 of 16 experts 69.7 -> 54.4 us (64 and 128 tiles), of
+// Tiles run as halves of 128 columns (gemm_half_tile; bits the same) where every workgroup of the launch then has a
+// place at once, two on a compute unit: the problems of the first list, or those of both lists (but experts of up to
+// sixteen rows whole).  A launch of one round is as long as its longest workgroup, and a half is the shorter one.
+// Layers of 2048 x 768: 200 tokens that choose 4 of 16 experts 69.7 -> 54.4 us (64 and 128 tiles), of
 // 1024 x 512, 300 tokens 58.2 -> 47.0, of 2048 x 1024, 150 tokens that choose 8 of 32 (256 tiles) 84.9 -> 80.8;
-// 400 tokens that choose 6 of 16 (256 tiles, half of them of 128 rows) 104.4 -> 105.
-// Above that whole tiles: up to 384 as halves 1000 tokens that choose 4 of 16 119 -> 126, and with the tiles of a last,
-// half empty round as halves 1500 tokens of 128 experts 278 -> 289 (the whole tiles are the cheaper ones, and the
-// rounds are not in step).
+// 400 tokens that choose 6 of 16 (256 tiles, half of them of 128 rows) 104.4 -> 105.  The first list alone, popular
+// experts: 512 of 2048 x 512 at 129 / 200 / 256 tokens 102.6 -> 95.5, 111.7 -> 104.2, 116.4 -> 111.2, 128 of 2048 x 768
+// at 150 101.8 -> 94.0, 256 of 1024 x 512 at 600 80.5 -> 70.9.
+// Beyond that whole tiles, which are the cheaper ones: the first list up to 576 and 640 workgroups 110 -> 118 (128
+// experts, 256 tokens) and 139 -> 148 (512, 400), both up to 768 (1000 tokens that choose 4 of 16) 119 -> 126, and
+// with the tiles of a last, half empty round as halves 1500 tokens of 128 experts 278 -> 289 (the rounds are not in
+// step).  Operands asked for two multiplications ahead of their use change nothing there.
 // Measured and dropped: cutting K in two with the split-K hand-over, for every tile or for the
 // 128-row tiles only (the shorter units pack better, the hand-over of 128 KB of partial sums per
 // tile costs far more than that gains: 150 -> 183 us per layer), 128-column units whose four waves
@@ -1088,15 +1092,18 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
     kr.counter = 0;
     kr.slot0 = kr.slot_rest = 0;
     kr.slot_step = 0;
-    // problems in order: the first list, the second and, of a launch in halves, both again for the second halves
-    const int big = *p.num_big, problems = big + *p.num_problems;
-    const bool halves = problems * p.group_lins * ((int)gridDim.x >> 3) <= p.half_tiles;
+    // problems in order: the first list, its second halves, the second list, its second halves
+    const int big = *p.num_big, small = *p.num_problems;
+    const int tiles = p.group_lins * ((int)gridDim.x >> 3);     // per problem
+    const bool big_halves = (2 * big + small) * tiles <= p.places, small_halves = 2 * (big + small) * tiles <= p.places;
     const GroupTile gt = group_tile(p);
-    const int half = gt.problem >= problems;
-    if (half && (!halves || gt.problem >= 2 * problems)) return;
-    const int z = gt.problem - half * problems;
-    const GroupProblem* const list = z < big ? p.big_problems : p.problems;
-    const int at = z < big ? z : z - big;
+    const int first_small = big_halves ? 2 * big : big;
+    const bool in_big = gt.problem < first_small;
+    const bool half = gt.problem >= (in_big ? big : first_small + small);
+    if (half && !in_big && (!small_halves || gt.problem >= first_small + 2 * small)) return;
+    const bool halves = in_big ? big_halves : small_halves;
+    const GroupProblem* const list = in_big ? p.big_problems : p.problems;
+    const int at = in_big ? gt.problem - (half ? big : 0) : gt.problem - first_small - (half ? small : 0);
     const GroupProblem gp = list[at];
     if (halves && !gp.lone) {
         const int n0 = gt.col * 256 + 128 * half;

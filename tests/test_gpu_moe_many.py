@@ -122,6 +122,8 @@ def test_problems_of_two_three_and_four_row_blocks(T, bits):
     (240, 256, 6, 2, 128, 3, 1, 0),
     (700, 128, 66, 4, 384, 4, 2, 0),        # at least 264 tiles of gate and up: whole; half that of the down projection
     (700, 128, 66, 4, 256, 2, 1, 128),      # 132 of either: halves
+    (600, 384, 200, 4, 256, 3, 2, 256),     # 200 small problems whole, the always-on expert's as halves
+    (600, 128, 200, 4, 384, 4, 0, 384),     # too many for that; the down projection's all as halves
 ])
 def test_launches_of_few_128_row_tiles_run_them_as_halves(T, H, E, k, I, bits, codebook, shared_I):
     """Either side of one tile per compute unit, against the 32-row problems' bits (which K of up to 384 keeps whole)."""
