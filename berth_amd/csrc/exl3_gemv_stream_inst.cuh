@@ -24,7 +24,12 @@ static void launch_stream_bits(const StreamParams& p, int lutmask, dim3 grid, hi
         constexpr int M = decltype(mask)::value;
         if (in == kInNorm) launch_stream_one<BITS, CB, kInNorm, M>(p, grid, stream);
         else if (in == kInSilu) launch_stream_one<BITS, CB, kInSilu, M>(p, grid, stream);
-        else launch_stream_one<BITS, CB, kInPlain, M>(p, grid, stream);
+        else {
+            if constexpr (CB != 0) {
+                if (p.q >= kStreamLongUnits) return launch_stream_one<BITS, CB, kInPlainLong, M>(p, grid, stream);
+            }
+            launch_stream_one<BITS, CB, kInPlain, M>(p, grid, stream);
+        }
     };
     switch (lutmask) {
     case 0x0: by_input(std::integral_constant<int, 0x0>{}); break;

@@ -13,7 +13,7 @@
 //     `rem` groups one more.  No second round, no tail of half-empty compute units: the grid is
 //     at most the number of compute units and every wave does the same amount of decode.
 //   * The dot products run on the matrix units (v_mfma_f32_16x16x32_f16 with the one row in all
-//     sixteen row slots): 16 lanes cover 2 tiles of one tile row, the four lane groups four tile
+//     sixteen row slots, or in the first of them): 16 lanes cover 2 tiles of one tile row, the four lane groups four tile
 //     rows, so the register quads a lane decodes are B operands as they are, and the A operand is
 //     16 bytes of the rotated activation per lane group.  Four of them per 32 weights of a lane
 //     take 64 cycles of a pipe that is idle otherwise; the sixteen v_dot2 they replace took 64
@@ -54,10 +54,10 @@ constexpr int kStreamGroups = 4;           // wave groups of a workgroup, four w
 constexpr int kStreamXsBlocks = 64;        // k-blocks of rotated activation a workgroup can hold
 constexpr int kStreamMaxCb = 15;           // column blocks one workgroup's units can touch
 constexpr int kStreamPieces = kStreamGroups + kStreamMaxCb - 1;
-// dynamic LDS of a launch: [table 128 KiB, if any][rotated activation][partial pieces][norm sums]
+// dynamic LDS of a launch: [table 128 KiB, if any][rotated activation][partial pieces][norm sums][32 zeros]
 __host__ __device__ constexpr int stream_lds_bytes(int lutmask)
 {
-    return (lutmask ? 131072 : 0) + kStreamXsBlocks * 256 + kStreamPieces * 512 + 128;
+    return (lutmask ? 131072 : 0) + kStreamXsBlocks * 256 + kStreamPieces * 512 + 128 + 32;
 }
 
 // one problem of a bundle whose lists the host knows (mode 3)
@@ -270,16 +270,25 @@ __device__ __forceinline__ global_ptr<T> uniform_ptr(global_ptr<T> q)
 // down projection, formed with the fp16 steps of berth_ops_silu_mul); or the RMS norm of a
 // fp32 row with the residual added first (the steps of berth_ops_rms_norm_res_in).
 constexpr int kInPlain = 0, kInSilu = 1, kInNorm = 2;
+// The row as given, with zeros in the fifteen empty row slots of the matrix instructions instead of copies: they
+// cost less power, and a long launch runs at the clock that the power leaves it.  us, copies -> zeros, MUL1:
+// 5120 x 248320 at 6 and 4 bits 178.8 -> 175.8 and 152.4 -> 149.0, 5120 x 131072 at 6 95.0 -> 93.7, 5120 x 32768 at 4
+// (20 units a wave group) 24.8 -> 24.2, 17408 x 32768 at 4 79.8 both; MCG 8192 x 32768 at 3 36.2 -> 35.7.
+// From 16 units on: a lane reads one of two LDS addresses then, and short launches lose with that and the zeros at their
+// head (2688 x 7296, 2 units, 7.93 -> 8.05).  3INST keeps the copies (17408 x 32768 at 2 bits 88.8 -> 89.2).
+constexpr int kInPlainLong = 3;
+constexpr unsigned kStreamLongUnits = 16;
 
 template <int BITS, int CB, int IN, int LUTMASK>
 __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams p)
 {
-    constexpr bool SILU = IN == kInSilu, NORM = IN == kInNorm;
+    constexpr bool SILU = IN == kInSilu, NORM = IN == kInNorm, ZEROS = IN == kInPlainLong;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     constexpr int kLutBytes = LUTMASK ? 131072 : 0;       // the table sits at LDS offset 0
     constexpr int kXsOff = kLutBytes;
     constexpr int kRedOff = kXsOff + kStreamXsBlocks * 256;
     constexpr int kMetaOff = kRedOff + kStreamPieces * 512;
+    constexpr int kZeroOff = kMetaOff + 128;
     constexpr int RING = StreamRing<BITS>::depth;
     uint32_t* const xs = (uint32_t*)(lds + kXsOff);
     float* const red = (float*)(lds + kRedOff);
@@ -436,6 +445,8 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         if (p.out_add) add_mine = ((global_ptr<const float2_t>)as_global(p.out_add + (cb_first + (unsigned)wave) * 128))[lane];
     }
 
+    if (ZEROS && wave == kStreamWaves - 1 && lane < 8) ((uint32_t*)(lds + kZeroOff))[lane] = 0;
+
     // ---- the table: built in place while the first units and the activation are on
     // their way (the vector ALU has nothing else to do until they arrive).  Thread t writes
     // the entries of states 2 (t + 1024 j), + 1 as one dword: consecutive lanes, consecutive
@@ -537,13 +548,22 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
     for (int j = 1; j < RING; ++j) prologue_row(j);
 
     // ---- the walk
-    // LDS byte offset of this lane group's part of the rotated activation of the current unit
+    // LDS byte offset of the rotated activation of the current unit.  A lane reads its group's part of it at
+    // x_live * xoff + x_at (one instruction, as the sum alone would be); ZEROS: but those of the fifteen empty row slots zeros.
+    uint32_t x_live = 1u, x_at = 32u * (uint32_t)lg;
+    if constexpr (ZEROS) {
+        if (l16 != 0) {
+            x_live = 0u;
+            x_at = (uint32_t)kZeroOff;
+        }
+        asm volatile("" : "+v"(x_live));                // (a factor, and not a select per unit)
+    }
     const unsigned xoff_wrap = kXsOff + (a_lo ? (KB - a_lo) * 256u : 0u);     // first unit of a later column block
     unsigned xoff = kXsOff + (r << 7) - a_lo * 256u;
     if (cb != cb_first) xoff = xoff_wrap + (r << 7);
     unsigned piece = (unsigned)kg + (cb - cb_first);
     unsigned left = uw0 < uw1 ? uw1 - uw0 : 0u;
-    float4_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;  // all four elements alike: the row slots hold one row
+    float4_t acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;  // the first element of lanes 0..15: the one row
     const int col = cg * 32 + (l16 >> 3) * 16 + (l16 & 7);
 
     auto flush = [&](unsigned pc) {
@@ -562,7 +582,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams 
         const uint32_t prev = fetch_prev(lane, mine[BITS - 1]);
         uint32_t addr[NT], t[NT], w2[16];
         dec.addresses(mine, prev, addr);
-        const half8_t* xp = (const half8_t*)(lds + xoff + 32 * lg);
+        const half8_t* xp = (const half8_t*)(lds + ((ZEROS ? __umul24(xoff, x_live) : xoff) + x_at));
         const half8_t xa = xp[0], xb = xp[1];               // k 0..7 and 8..15 of the lane group's tile row
         if constexpr (Dec::kTablePairs != 0) {
 #pragma unroll

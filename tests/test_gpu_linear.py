@@ -483,6 +483,28 @@ def test_lm_head_shape_6bpw_slices_match_oracle():
         assert close(got[c0:c0 + 256], want.reshape(-1))[0] == 0, c0
 
 
+@pytest.mark.parametrize("blocks,units", [(1638, 15), (1641, 16)])
+@pytest.mark.parametrize("bits,cb,table", [(3, 1, 0), (4, 2, 0), (4, 2, 10), (2, 0, 0)])
+def test_long_launches_of_one_row(blocks, units, bits, cb, table):
+    """Either side of sixteen units a wave group, from which on the empty row slots of the matrix instructions hold zeros."""
+    Kk, N = 640, 128 * blocks
+    tr, suh, svh = synth.linear(68 + bits, Kk, N, bits)
+    x = synth.activations(69 + units, 1, Kk)
+    d_tr, d_suh, d_svh, d_x = dev(tr), dev(suh.view(np.uint16)), dev(svh.view(np.uint16)), dev(x.view(np.uint16))
+    a_had = torch.zeros(Kk, dtype=torch.float16, device=DEV)
+    c = torch.zeros(N, dtype=torch.float32, device=DEV)
+    with knobs(BERTH_GEMV_STREAM_LUT=table):
+        K.exl3_linear(d_x.data_ptr(), d_tr.data_ptr(), c.data_ptr(), d_suh.data_ptr(), a_had.data_ptr(),
+                      d_svh.data_ptr(), 1, Kk, N, bits, cb, OutDtype.F32)
+        torch.cuda.synchronize()
+    assert "exl3_gemv_stream_kernel" in K.last_launch() and f"units_per_wave={units}" in K.last_launch(), K.last_launch()
+    got = c.cpu().numpy()
+    for c0 in (0, 128 * (blocks // 2), N - 256):
+        sub = np.ascontiguousarray(tr[:, c0 // 16:c0 // 16 + 16, :])
+        want, _ = O.linear(x, sub, suh, svh[c0:c0 + 256], Kk, 256, bits, cb, out_fp32=True)
+        assert close(got[c0:c0 + 256], want.reshape(-1))[0] == 0, c0
+
+
 @pytest.mark.parametrize("rows", [1, 3])
 def test_very_wide_output_uses_closer_counters(rows):
     """More column blocks than the arrival-counter table holds at one counter per 128 bytes
