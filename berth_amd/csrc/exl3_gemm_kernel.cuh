@@ -282,6 +282,8 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
 // 64 tokens x 128 experts, four rows an expert, 126 -> 110 us.  The sums of sixteen rows form in another order
 // than those of 32, so that the choice must not depend on how a call cuts its problems: `lone` says that the
 // expert has no more rows, in whichever list it is.
+// Rows past the problem repeat its last row: zeros there, with the loads of their lanes switched off, cost the
+// loop more than the zeros save (that layer 104.2 -> 107.4, of 256 tokens x 512 experts 109.9 -> 112.9).
 template <int BITS, int CB, typename F>
 __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
                                                    const int arow, const int K, const int lane, float4_t (&acc)[2][2], F requested)
@@ -698,8 +700,11 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
         }
         __syncthreads();
         const int rows_blk = min(32, rows_here - mb * 32);
-        // 64 vectors (32 rows x 2 column blocks); a wave rotates four per pass, sixteen lanes each
-#pragma unroll
+        // 64 vectors (32 rows x 2 column blocks); a wave rotates four per pass, sixteen lanes each.  Grouped tiles of
+        // several blocks take two passes at a time: exl3_gemm_mixed_kernel, which holds every kind of them, was 138 KB
+        // long with four (4 bits, 3INST) and needed indirect branches, which reach further than 128 KB
+        constexpr int kPasses = DENSE || MB == 1 ? 4 : 2;
+#pragma unroll kPasses
         for (int pass = 0; pass < 4; ++pass) {
             const int vec = pass * 16 + wave * 4 + (lane >> 4);
             const int row = vec >> 1, blk = vec & 1;
