@@ -208,6 +208,16 @@ struct KRange {
 
 constexpr int kGemmWrittenBase = 32768;   // second half of the counter table: "partial sums written" per tile
 
+// a pointer that every lane of the wave agrees on, in scalar registers
+template <typename T>
+__device__ __forceinline__ const T* rows_uniform(const T* q)
+{
+    const uint64_t v = (uint64_t)q;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (const T*)(((uint64_t)hi << 32) | lo);
+}
+
 constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: conflict-free b128 reads)
 
 // The k-loop of a 32-row tile, 64 columns from nw on: every wave is on its own.  The A operand of a lane (row
@@ -428,14 +438,16 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[mb][f][r] = 0.0f;
 
+    // (the list of linears is read as vectors: the pointer would be two of a lane's 128 registers through the loop)
+    const uint32_t* const trellis = MB == 1 && !DENSE ? rows_uniform(lin.trellis) : lin.trellis;
     float4_t acc16[2][2] = {};
     if (lone) {
         if (active)
-            accumulate_16_rows<BITS, CB>(lin.trellis, row_dw, nw, a_had, a_row_at(min(lane & 15, rows_here - 1)), p.K, lane, acc16, keep_scale);
+            accumulate_16_rows<BITS, CB>(trellis, row_dw, nw, a_had, a_row_at(min(lane & 15, rows_here - 1)), p.K, lane, acc16, keep_scale);
         else keep_scale();
     } else if constexpr (MB == 1) {
         if (active && kr.kb0 < kr.kb1)
-            accumulate_32_rows<BITS, CB>(lin.trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
+            accumulate_32_rows<BITS, CB>(trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
                                          kr.step, lane, acc[0], keep_scale);      // (rows past the problem repeat its last row)
         else keep_scale();
     } else {
@@ -767,9 +779,12 @@ inline dim3 group_grid(int cols, int lins, int problems)
 //
 // 32-row problems: up to four workgroups on a compute unit (with four parts in flight at the end of a
 // split tile it was 173 registers a lane and two of them, so that the 756 workgroups of 64 tokens x 128
-// experts ran in two rounds: layer 125.6 -> 122.6 us).
+// experts ran in two rounds: layer 125.6 -> 122.6 us).  The launch bound keeps 3INST and MCG there as well, whose
+// kernels of 3 and 4 bits had 130..132 registers with both row forms in them: the same time with three workgroups as with
+// four (64 tokens x 128 experts MCG 110.8 -> 109.1 and 111.0 -> 107.8 us at 4 and 3 bits, runs of one side 4 and 8 % apart,
+// 3INST 122.4 -> 122.6 and 120.0 -> 120.5).  8 bits take three, four would need scratch.
 template <int BITS, int CB, int MB, bool DENSE = true>
-__global__ __launch_bounds__(256, MB == 1 && !DENSE ? 3 : 2) void exl3_gemm_kernel(GemmParams p)
+__global__ __launch_bounds__(256, MB > 1 || DENSE ? 2 : BITS < 8 ? 4 : 3) void exl3_gemm_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const GroupTile gt = DENSE ? GroupTile{(int)blockIdx.x, 0, 0} : group_tile(p);
@@ -806,9 +821,9 @@ __global__ __launch_bounds__(256, MB == 1 && !DENSE ? 3 : 2) void exl3_gemm_kern
 // What bounds it: the decode, as there (experts of up to sixteen rows: accumulate_16_rows); the end of a row is three rotations (of 128 values by sixteen
 // lanes) instead of two, against a launch that reads both factors back: layer of 64 tokens x 128 experts
 // x 768 122.6 -> 121.4 us, of 20 tokens x 128 experts x 896 (seven column blocks, which 256-column tiles
-// cover as eight) 107 -> 94.
+// cover as eight) 107 -> 94.  Four workgroups on a compute unit, as exl3_gemm_kernel's 32-row problems.
 template <int BITS, int CB>
-__global__ __launch_bounds__(256, 3) void exl3_gemm_pair_kernel(GemmParams p)
+__global__ __launch_bounds__(256, 4) void exl3_gemm_pair_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const GroupTile gt = group_tile(p);

@@ -157,15 +157,6 @@ __device__ __forceinline__ GemmRotation rows_rotation(const GemmRotateParams& p,
             first ? p.rot_out + (size_t)sl * p.M * p.K : nullptr};
 }
 
-template <typename T>
-__device__ __forceinline__ const T* rows_uniform(const T* q)
-{
-    const uint64_t v = (uint64_t)q;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return (const T*)(((uint64_t)hi << 32) | lo);
-}
-
 template <int BITS, int CB, int MT, bool GROUPED, bool ROT = false>     // MT: tiles of 16 rows
 __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditional_t<ROT, GemmRotateParams, GemmParams> p)
 {

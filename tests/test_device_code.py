@@ -72,7 +72,7 @@ class Function:
         return before
 
 
-def _compile(tmp_path, kernels, headers, params="GemmParams"):
+def _assembly(tmp_path, kernels, headers, params="GemmParams"):
     source = tmp_path / "kernels.hip"
     source.write_text("".join(f'#include "{h}"\n' for h in headers) + "namespace berth {\n" +
                       "".join(f"template __global__ void {k}({params});\n" for k in sorted(set(kernels))) + "}\n")
@@ -80,8 +80,12 @@ def _compile(tmp_path, kernels, headers, params="GemmParams"):
     r = subprocess.run([B.HIPCC, *B.FLAGS, "--offload-device-only", "-S", "-I" + B.CSRC, str(source), "-o", str(out)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-4000:]
+    return out.read_text()
+
+
+def _compile(tmp_path, kernels, headers, params="GemmParams"):
     functions, lines = [], None
-    for line in out.read_text().splitlines():
+    for line in _assembly(tmp_path, kernels, headers, params).splitlines():
         if m := re.match(r"(_Z\w+):", line):
             name, lines = m[1], []
         elif lines is not None and line.startswith(".Lfunc_end"):
@@ -208,3 +212,16 @@ def test_every_register_that_inline_assembly_writes_counts(write, regs, waits, c
     (["exl3_gemm_rows_kernel<3, 1, 1, false, true>", "exl3_gemm_rows_kernel<4, 0, 2, false, true>"], "GemmRotateParams")])
 def test_the_same_of_the_fused_launches(tmp_path, kernels, params):
     test_matrix_instructions_keep_their_distance_from_inline_assembly(tmp_path, kernels, ("exl3_gemm_rows_kernel.cuh",), params)
+
+
+def test_grouped_tiles_of_one_block_leave_room_for_four_workgroups(tmp_path):
+    """Four workgroups of four waves on a compute unit: at most 128 of a SIMD's 512 registers a lane, and no scratch.
+    (8 bits take three outside the pair kernel.)"""
+    kernels = ([f"exl3_gemm_pair_kernel<{bits}, {cb}>" for bits, cb in ((3, 0), (4, 0), (4, 1), (4, 2), (8, 2))] +
+               [f"exl3_gemm_kernel<{bits}, {cb}, 1, false>" for bits, cb in ((3, 0), (3, 1), (3, 2), (4, 0), (7, 1), (7, 2))])
+    found = {}
+    for entry in _assembly(tmp_path, kernels, ("exl3_gemm_kernel.cuh",)).split("  - .agpr_count:")[1:]:
+        found[re.search(r"\.name:\s+(\S+)", entry)[1]] = tuple(int(re.search(rf"\.{key}:\s+(\d+)", entry)[1])
+                                                                for key in ("vgpr_count", "private_segment_fixed_size"))
+    assert len(found) == len(kernels)
+    assert {name: at for name, at in found.items() if at[0] > 128 or at[1]} == {}
