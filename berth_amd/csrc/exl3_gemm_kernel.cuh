@@ -439,7 +439,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
             for (int r = 0; r < 16; ++r) acc[mb][f][r] = 0.0f;
 
     // (the list of linears is read as vectors: the pointer would be two of a lane's 128 registers through the loop)
-    const uint32_t* const trellis = MB == 1 && !DENSE ? rows_uniform(lin.trellis) : lin.trellis;
+    const uint32_t* const trellis = MB == 1 && !DENSE && CB != 2 ? rows_uniform(lin.trellis) : lin.trellis;
     float4_t acc16[2][2] = {};
     if (lone) {
         if (active)
@@ -782,9 +782,11 @@ inline dim3 group_grid(int cols, int lins, int problems)
 // experts ran in two rounds: layer 125.6 -> 122.6 us).  The launch bound keeps 3INST and MCG there as well, whose
 // kernels of 3 and 4 bits had 130..132 registers with both row forms in them: the same time with three workgroups as with
 // four (64 tokens x 128 experts MCG 110.8 -> 109.1 and 111.0 -> 107.8 us at 4 and 3 bits, runs of one side 4 and 8 % apart,
-// 3INST 122.4 -> 122.6 and 120.0 -> 120.5).  8 bits take three, four would need scratch.
+// 3INST 122.4 -> 122.6 and 120.0 -> 120.5).  8 bits take three, four would need scratch.  MUL1 is below 128 up to 6 bits
+// without the bound, and the schedule that the bound gives costs it 0.4 to 0.7 % (150 and 300 tokens x 128 experts 120.5 ->
+// 121.4 and 141.7 -> 142.6).
 template <int BITS, int CB, int MB, bool DENSE = true>
-__global__ __launch_bounds__(256, MB > 1 || DENSE ? 2 : BITS < 8 ? 4 : 3) void exl3_gemm_kernel(GemmParams p)
+__global__ __launch_bounds__(256, MB > 1 || DENSE ? 2 : CB != 2 && BITS < 8 ? 4 : 3) void exl3_gemm_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const GroupTile gt = DENSE ? GroupTile{(int)blockIdx.x, 0, 0} : group_tile(p);
@@ -821,9 +823,9 @@ __global__ __launch_bounds__(256, MB > 1 || DENSE ? 2 : BITS < 8 ? 4 : 3) void e
 // What bounds it: the decode, as there (experts of up to sixteen rows: accumulate_16_rows); the end of a row is three rotations (of 128 values by sixteen
 // lanes) instead of two, against a launch that reads both factors back: layer of 64 tokens x 128 experts
 // x 768 122.6 -> 121.4 us, of 20 tokens x 128 experts x 896 (seven column blocks, which 256-column tiles
-// cover as eight) 107 -> 94.  Four workgroups on a compute unit, as exl3_gemm_kernel's 32-row problems.
+// cover as eight) 107 -> 94.  The launch bound: exl3_gemm_kernel's.
 template <int BITS, int CB>
-__global__ __launch_bounds__(256, 4) void exl3_gemm_pair_kernel(GemmParams p)
+__global__ __launch_bounds__(256, CB != 2 ? 4 : 3) void exl3_gemm_pair_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const GroupTile gt = group_tile(p);
