@@ -740,8 +740,8 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         p.max_big = g.max_big;
         p.S = 1;
         p.places = 2 * ws.cu_count;
-        const int more = p.places / (2 * nblocks * g.num_lins);                     // problems that may run as halves
-        gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, group_grid(nblocks, g.num_lins, g.max_problems + g.max_big + more));
+        gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc,
+                  group_grid(nblocks, g.num_lins, g.max_problems + g.max_big + mixed_extra(nblocks * g.num_lins, p.places)));
         hip_ok(hipGetLastError(), "exl3_gemm_mixed_kernel launch");
         return desc + " grouped";
     }

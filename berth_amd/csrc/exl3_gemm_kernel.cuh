@@ -294,23 +294,24 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
 // expert has no more rows, in whichever list it is.
 // Rows past the problem repeat its last row: zeros there, with the loads of their lanes switched off, cost the
 // loop more than the zeros save (that layer 104.2 -> 107.4, of 256 tokens x 512 experts 109.9 -> 112.9).
-template <int BITS, int CB, typename F>
+template <int BITS, int CB, int CG, typename F>            // CG: column groups of 32 a wave
 __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
-                                                   const int arow, const int K, const int lane, float4_t (&acc)[2][2], F requested)
+                                                   const int arow, const int K, const int lane, float4_t (&acc)[CG][2], F requested)
 {
     constexpr int tile_dw = 8 * BITS;
     const int l16 = lane & 15, lg = lane >> 4;
     const global_ptr<const uint32_t> tb = as_global(trellis) + (size_t)lg * row_dw +
                                          (size_t)((nw >> 4) + (l16 >> 3)) * tile_dw + (l16 & 7) * BITS;
     const global_ptr<const half8_t> ab = (global_ptr<const half8_t>)(as_global(a_had) + (size_t)arow * K + 16 * lg);
-    uint32_t cur[4][BITS];
+    uint32_t cur[2 * CG][BITS];
     half8_t av[2][2];
 #pragma unroll
-    for (int st = 0; st < 4; ++st) {
-        load_tile_dwords<BITS>(tb + (size_t)(st / 2 * 4) * row_dw + st % 2 * 2 * tile_dw, cur[st]);
-        if (st % 2 == 0) {
-            av[st / 2][0] = ab[8 * (st / 2)];
-            av[st / 2][1] = ab[8 * (st / 2) + 1];
+    for (int st = 0; st < 2 * CG; ++st) {
+        const int ks = st / CG, cg = st % CG;
+        load_tile_dwords<BITS>(tb + (size_t)(4 * ks) * row_dw + cg * 2 * tile_dw, cur[st]);
+        if (cg == 0) {
+            av[ks][0] = ab[8 * ks];
+            av[ks][1] = ab[8 * ks + 1];
         }
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -321,8 +322,8 @@ __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, cons
         const global_ptr<const uint32_t> tnx = tb + (size_t)(nkb * 8) * row_dw;
         const global_ptr<const half8_t> anx = ab + nkb * 16;
 #pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            const int ks = st / 2, cg = st % 2;
+        for (int st = 0; st < 2 * CG; ++st) {
+            const int ks = st / CG, cg = st % CG;
             uint32_t prev = fetch_prev(lane, cur[st][BITS - 1]);
             uint32_t w2[16];
             decode_lane<BITS, CB>(cur[st], prev, w2);
@@ -342,20 +343,20 @@ __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, cons
             acc[cg][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[ks][1], b[0][1], acc[cg][0], 0, 0, 0);
             acc[cg][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[ks][1], b[1][1], acc[cg][1], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
-            if (cg == 1) {
+            if (cg == CG - 1) {
                 av[ks][0] = anx[8 * ks];
                 av[ks][1] = anx[8 * ks + 1];
             }
         }
     }
 }
-// its sums to the fp32 tile, 64 columns from z on
-template <int STRIDE>
-__device__ __forceinline__ void stage_16_rows(float* z, const float4_t (&acc)[2][2], const int lane)
+// its sums to the fp32 tile, 32 * CG columns from z on
+template <int STRIDE, int CG>
+__device__ __forceinline__ void stage_16_rows(float* z, const float4_t (&acc)[CG][2], const int lane)
 {
     float* const at = z + 4 * (lane >> 4) * STRIDE + ((lane >> 3) & 1) * 16 + (lane & 7);
 #pragma unroll
-    for (int cg = 0; cg < 2; ++cg)
+    for (int cg = 0; cg < CG; ++cg)
 #pragma unroll
         for (int f = 0; f < 2; ++f)
 #pragma unroll
@@ -906,6 +907,38 @@ __global__ __launch_bounds__(256, CB != 2 ? 4 : 3) void exl3_gemm_pair_kernel(Ge
     }
 }
 
+// Rows 32 * mb .. + 31 of a problem, 128 columns from n0 on: from the fp32 tile through the output rotation to the output.
+constexpr int kHalfZStride = 128 + 4;
+__device__ __forceinline__ void finish_half_rows(const GemmParams& p, const GroupProblem gp, const int which, const int n0, const int mb,
+                                                 const float* z_tile, const half8_t* s_scale)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, chunk = had_chunk(lane);
+    // 32 vectors; a wave rotates four per pass, sixteen lanes each
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+        const int row = pass * 16 + wave * 4 + (lane >> 4);
+        if (mb * 32 + row >= gp.nrows) continue;
+        const float4_t* zp = (const float4_t*)&z_tile[row * kHalfZStride + 8 * chunk];
+        const float4_t z0 = zp[0], z1 = zp[1];
+        float v[8] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
+        const float unit = had128_row16(v, lane) * kRsqrt128;
+        const half8_t sv = s_scale[chunk];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = had_scale(v[i], unit) * (float)sv[i];
+        const size_t at = (size_t)(gp.row0 + mb * 32 + row) * p.N + n0 + 8 * chunk;
+        if (p.out_fp32) {
+            global_ptr<float4_t> dst = (global_ptr<float4_t>)(as_global((float*)p.c[which]) + at);
+            dst[0] = float4_t{v[0], v[1], v[2], v[3]};
+            dst[1] = float4_t{v[4], v[5], v[6], v[7]};
+        } else {
+            half8_t o;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[i] = (_Float16)v[i];
+            *(global_ptr<half8_t>)(as_global((_Float16*)p.c[which]) + at) = o;
+        }
+    }
+}
+
 // One tile of a problem, 128 columns from n0 on, whole K: half of what gemm_tile's workgroup does, for launches of
 // few tiles.  A wave owns 32 columns instead of 64, so
 // that its 64 lanes decode four tile rows of a k-block at a time instead of two: lane bits 4 and 5 name the
@@ -921,8 +954,7 @@ __device__ __forceinline__ void gemm_half_tile(const GemmParams& p, const GroupP
 {
     constexpr int BM = MB * 32;
     _Float16* a_tile = (_Float16*)smem;                 // [2][BM][kAStride]
-    float* z_tile = (float*)smem;                       // epilogue: [32][128 + 4]
-    constexpr int kZStride = 128 + 4;
+    float* z_tile = (float*)smem;                       // epilogue: [32][kHalfZStride]
     if (n0 >= p.N) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int half_id = lane >> 5, slot = lane & 31;
@@ -1037,41 +1069,61 @@ __device__ __forceinline__ void gemm_half_tile(const GemmParams& p, const GroupP
         }
     }
 
-    const int chunk = had_chunk(lane);
     const int col = wave * 32 + ((slot >> 3) & 1) * 16 + (slot >> 4) * 8 + (slot & 7);
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         if (mb * 32 >= rows_here) break;                        // workgroup-uniform
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < 16; ++r) z_tile[(8 * (r >> 2) + 4 * half_id + (r & 3)) * kZStride + col] = acc[mb][r];
+        for (int r = 0; r < 16; ++r) z_tile[(8 * (r >> 2) + 4 * half_id + (r & 3)) * kHalfZStride + col] = acc[mb][r];
         __syncthreads();
-        // 32 vectors; a wave rotates four per pass, sixteen lanes each
-#pragma unroll 1
-        for (int pass = 0; pass < 2; ++pass) {
-            const int row = pass * 16 + wave * 4 + (lane >> 4);
-            if (mb * 32 + row >= rows_here) continue;
-            const float4_t* zp = (const float4_t*)&z_tile[row * kZStride + 8 * chunk];
-            const float4_t z0 = zp[0], z1 = zp[1];
-            float v[8] = {z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
-            const float unit = had128_row16(v, lane) * kRsqrt128;
-            const half8_t sv = s_scale[chunk];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = had_scale(v[i], unit) * (float)sv[i];
-            const size_t at = (size_t)(gp.row0 + mb * 32 + row) * p.N + n0 + 8 * chunk;
-            if (p.out_fp32) {
-                global_ptr<float4_t> dst = (global_ptr<float4_t>)(as_global((float*)p.c[which]) + at);
-                dst[0] = float4_t{v[0], v[1], v[2], v[3]};
-                dst[1] = float4_t{v[4], v[5], v[6], v[7]};
-            } else {
-                half8_t o;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) o[i] = (_Float16)v[i];
-                *(global_ptr<half8_t>)(as_global((_Float16*)p.c[which]) + at) = o;
-            }
-        }
+        finish_half_rows(p, gp, which, n0, mb, z_tile, s_scale);
     }
 }
+
+// The same for an expert of up to sixteen rows (accumulate_16_rows, 32 columns a wave; the bits of a whole tile).  Bound
+// by the decode of a wave that has its SIMD nearly to itself: 60 experts of 1024 x 512 (180 tokens) 44.8 us a layer as halves
+// of 32-row products, 48.2 whole, 42.9 so.
+template <int BITS, int CB>
+__device__ __forceinline__ void gemm_half_tile_16(const GemmParams& p, const GroupProblem gp, const int which, const int n0, unsigned char* smem)
+{
+    float* z_tile = (float*)smem;                       // [16][kHalfZStride]
+    if (n0 >= p.N) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool shared = gp.expert == p.shared_expert;
+    const ExpertLin lin = shared ? p.shared[p.lin_base + which] : p.experts[gp.expert * p.lins_per_expert + p.lin_base + which];
+    __shared__ __align__(16) half8_t s_scale[16];
+    half8_t scale_mine = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (threadIdx.x < 16) scale_mine = ((global_ptr<const half8_t>)as_global(lin.svh + n0))[threadIdx.x];
+    int arow = gp.row0 + min(lane & 15, gp.nrows - 1);  // rows past the problem repeat its last row
+    if (p.a_rows && !shared) arow = as_global(p.a_rows)[arow];
+    float4_t acc[1][2] = {};
+    accumulate_16_rows<BITS, CB>(lin.trellis, (size_t)(p.N >> 4) * (8 * BITS), n0 + 32 * wave, p.a_had[which], arow, p.K, lane, acc, [&]() {
+        if (threadIdx.x < 16) s_scale[threadIdx.x] = scale_mine;
+    });
+    stage_16_rows<kHalfZStride>(z_tile + 32 * wave, acc, lane);
+    __syncthreads();
+    finish_half_rows(p, gp, which, n0, 0, z_tile, s_scale);
+}
+
+// What problem number `problem` of a mixed launch is: the first list, its second halves, the second list, its second
+// halves.  `tiles` of 256 columns a problem; halves where all of the launch then runs at once, in `places`.
+struct MixedPlace {
+    bool first_list, halves, second, empty;     // second: columns 128.. of the tiles
+    int at;                                     // in its list
+};
+constexpr MixedPlace mixed_place(const int problem, const int big, const int small, const int tiles, const int places)
+{
+    const bool big_halves = (2 * big + small) * tiles <= places, small_halves = 2 * (big + small) * tiles <= places;
+    const int first_small = big_halves ? 2 * big : big;
+    const bool first_list = problem < first_small;
+    const bool second = problem >= (first_list ? big : first_small + small);
+    const bool empty = second && !first_list && (!small_halves || problem >= first_small + 2 * small);
+    return {first_list, first_list ? big_halves : small_halves, second, empty,
+            first_list ? problem - (second ? big : 0) : problem - first_small - (second ? small : 0)};
+}
+// problems that may have second halves: the room that a launch needs behind its lists
+constexpr int mixed_extra(const int tiles, const int places) { return places / (2 * tiles); }
 
 // Grouped launch over two problem lists at once: the first problems of group_tile are those of up
 // to 128 rows (weights decoded once for all of them, so an expert with many rows costs one
@@ -1083,13 +1135,15 @@ __device__ __forceinline__ void gemm_half_tile(const GemmParams& p, const GroupP
 // it has, needed or not): gate + up and down of 800 tokens that choose 8 of 128 experts 137 + 82 -> 119 +
 // 70 us, of 1500 tokens (94 rows an expert) 133 + 89 -> 131 + 85.
 // Tiles run as halves of 128 columns (gemm_half_tile; bits the same) where every workgroup of the launch then has a
-// place at once, two on a compute unit: the problems of the first list, or those of both lists (but experts of up to
-// sixteen rows whole).  A launch of one round is as long as its longest workgroup, and a half is the shorter one.
+// place at once, two on a compute unit: the problems of the first list, or those of both lists.  A launch of one round
+// is as long as its longest workgroup, and a half is the shorter one.
 // Layers of 2048 x 768: 200 tokens that choose 4 of 16 experts 69.7 -> 54.4 us (64 and 128 tiles), of
 // 1024 x 512, 300 tokens 58.2 -> 47.0, of 2048 x 1024, 150 tokens that choose 8 of 32 (256 tiles) 84.9 -> 80.8;
 // 400 tokens that choose 6 of 16 (256 tiles, half of them of 128 rows) 104.4 -> 105.  The first list alone, popular
 // experts: 512 of 2048 x 512 at 129 / 200 / 256 tokens 102.6 -> 95.5, 111.7 -> 104.2, 116.4 -> 111.2, 128 of 2048 x 768
-// at 150 101.8 -> 94.0, 256 of 1024 x 512 at 600 80.5 -> 70.9.
+// at 150 101.8 -> 94.0, 256 of 1024 x 512 at 600 80.5 -> 70.9.  Experts of up to sixteen rows too (gemm_half_tile_16):
+// 60 experts of 2048 x 512 at 150 and 180 tokens 66.2 -> 61.7 and 70.9 -> 64.7 against whole ones, of 1024 x 512 at 180
+// 48.2 -> 42.9.
 // Beyond that whole tiles, which are the cheaper ones: the first list up to 576 and 640 workgroups 110 -> 118 (128
 // experts, 256 tokens) and 139 -> 148 (512, 400), both up to 768 (1000 tokens that choose 4 of 16) 119 -> 126, and
 // with the tiles of a last, half empty round as halves 1500 tokens of 128 experts 278 -> 289 (the rounds are not in
@@ -1114,28 +1168,21 @@ __global__ __launch_bounds__(256, 2) void exl3_gemm_mixed_kernel(GemmParams p)
     kr.counter = 0;
     kr.slot0 = kr.slot_rest = 0;
     kr.slot_step = 0;
-    // problems in order: the first list, its second halves, the second list, its second halves
-    const int big = *p.num_big, small = *p.num_problems;
-    const int tiles = p.group_lins * ((int)gridDim.x >> 3);     // per problem
-    const bool big_halves = (2 * big + small) * tiles <= p.places, small_halves = 2 * (big + small) * tiles <= p.places;
     const GroupTile gt = group_tile(p);
-    const int first_small = big_halves ? 2 * big : big;
-    const bool in_big = gt.problem < first_small;
-    const bool half = gt.problem >= (in_big ? big : first_small + small);
-    if (half && !in_big && (!small_halves || gt.problem >= first_small + 2 * small)) return;
-    const bool halves = in_big ? big_halves : small_halves;
-    const GroupProblem* const list = in_big ? p.big_problems : p.problems;
-    const int at = in_big ? gt.problem - (half ? big : 0) : gt.problem - first_small - (half ? small : 0);
+    const MixedPlace place = mixed_place(gt.problem, *p.num_big, *p.num_problems, p.group_lins * ((int)gridDim.x >> 3), p.places);
+    if (place.empty) return;
+    const GroupProblem* const list = place.first_list ? p.big_problems : p.problems;
+    const int at = place.at;
     const GroupProblem gp = list[at];
-    if (halves && !gp.lone) {
-        const int n0 = gt.col * 256 + 128 * half;
-        if (gp.nrows > 96) gemm_half_tile<BITS, CB, 4>(p, gp, gt.which, n0, smem);
+    if (place.halves) {
+        const int n0 = gt.col * 256 + 128 * place.second;
+        if (gp.lone) gemm_half_tile_16<BITS, CB>(p, gp, gt.which, n0, smem);
+        else if (gp.nrows > 96) gemm_half_tile<BITS, CB, 4>(p, gp, gt.which, n0, smem);
         else if (gp.nrows > 64) gemm_half_tile<BITS, CB, 3>(p, gp, gt.which, n0, smem);
         else if (gp.nrows > 32) gemm_half_tile<BITS, CB, 2>(p, gp, gt.which, n0, smem);
         else gemm_half_tile<BITS, CB, 1>(p, gp, gt.which, n0, smem);
         return;
     }
-    if (half) return;                                   // (an expert of at most sixteen rows: whole)
     // as many 32-row blocks as the problem has
     if (gp.nrows > 96) gemm_tile<BITS, CB, 4, false>(p, at, gt.col, kr, gt.which, smem, list);
     else if (gp.nrows > 64) gemm_tile<BITS, CB, 3, false>(p, at, gt.col, kr, gt.which, smem, list);

@@ -225,3 +225,35 @@ def test_grouped_tiles_of_one_block_leave_room_for_four_workgroups(tmp_path):
                                                                 for key in ("vgpr_count", "private_segment_fixed_size"))
     assert len(found) == len(kernels)
     assert {name: at for name, at in found.items() if at[0] > 128 or at[1]} == {}
+
+
+def test_every_tile_of_a_mixed_launch_is_taken_once(tmp_path):
+    """mixed_place over two lists of any length within their room: each problem whole, or both of its halves, once each
+    and within the grid; all of the second list (few rows or many) as halves where twice its tiles have places."""
+    source, program = tmp_path / "places.hip", tmp_path / "places"
+    source.write_text("""#include "exl3_gemm_kernel.cuh"
+#include <cstdio>
+#include <map>
+#include <tuple>
+using namespace berth;
+int main() {
+    for (int tiles : {1, 2, 3, 4, 8, 14, 64}) for (int places : {32, 64, 512, 608})
+    for (int big = 0; big <= 70; big += big < 4 ? 1 : 11) for (int small = 0; small <= 300; small += small < 4 ? 1 : 37) {
+        const bool all = 2 * (big + small) * tiles <= places, first = (2 * big + small) * tiles <= places;
+        std::map<std::tuple<bool, int, bool>, int> seen;
+        const int grid = 8 * (int)group_grid(tiles, 1, big + small + mixed_extra(tiles, places)).y;     // full lists: the tightest
+        for (int i = 0; i < grid; ++i) {
+            const MixedPlace m = mixed_place(i, big, small, tiles, places);
+            if (m.empty) continue;
+            if (m.halves != (m.first_list ? first : all) || (m.second && !m.halves)) return 1;
+            ++seen[{m.first_list, m.at, m.second}];
+        }
+        if ((int)seen.size() != big * (first ? 2 : 1) + small * (all ? 2 : 1)) return 2;
+        for (auto& [place, times] : seen)
+            if (times != 1 || std::get<1>(place) < 0 || std::get<1>(place) >= (std::get<0>(place) ? big : small)) return 3;
+    }
+    std::puts("ok");
+}
+""")
+    subprocess.run([B.HIPCC, *B.FLAGS, "-I" + B.CSRC, str(source), "-o", str(program)], check=True, capture_output=True)
+    assert subprocess.run([str(program)], capture_output=True, text=True).stdout == "ok\n"

@@ -237,6 +237,7 @@ def test_gate_up_and_the_next_rotation_in_one_launch(T, H, E, k, I, bits, shared
 @pytest.mark.parametrize("T,H,E,k,I,bits,shared_I", [
     (140, 256, 20, 2, 384, 4, 0),       # experts on either side of sixteen rows; 240 tiles of gate and up: halves
     (150, 128, 150, 3, 384, 3, 0),      # nearly all below; whole tiles
+    (150, 384, 60, 2, 384, 3, 0),       # 240 tiles of gate and up, 120 of the down projection: both launches in halves, the last odd
     (16, 384, 2, 1, 128, 5, 128),       # sixteen rows of the always-on expert
     (60, 384, 5, 1, 640, 2, 0),         # gate, up and the next rotation in one launch
 ])
