@@ -92,7 +92,7 @@ def _make_layer(gpu, seed, H, E, I, bits, shared_I=0, router_scale=1.0):
     return wr, experts_np, experts, shared_np, shared
 
 
-def _check_stages(layer, x, experts_np, shared_np, idx, w, out, T, H, E, k, I, bits, shared_I):
+def _check_stages(layer, x, experts_np, shared_np, idx, w, out, T, H, E, k, I, bits, shared_I, codebook=2):
     """Each stage against the oracle on the SAME inputs the GPU stage consumed:
     gate/up outputs from the gathered tokens, down outputs from the GPU's own
     gate/up outputs, and the combine from the GPU's own down outputs."""
@@ -118,12 +118,12 @@ def _check_stages(layer, x, experts_np, shared_np, idx, w, out, T, H, E, k, I, b
             continue
         xe = x[perm[r0:r1] // k]
         (gt, gs, gv), (ut, us, uv), (dt, ds, dv) = experts_np[e]
-        want_g, _ = O.linear(xe, gt, gs, gv, H, I, bits, 2)
-        want_u, _ = O.linear(xe, ut, us, uv, H, I, bits, 2)
+        want_g, _ = O.linear(xe, gt, gs, gv, H, I, bits, codebook)
+        want_u, _ = O.linear(xe, ut, us, uv, H, I, bits, codebook)
         assert close(g[r0:r1], want_g)[0] == 0, ("gate", e)
         assert close(u[r0:r1], want_u)[0] == 0, ("up", e)
         a = O.silu_mul(g[r0:r1], u[r0:r1]).reshape(r1 - r0, I)
-        want_d, _ = O.linear(a, dt, ds, dv, I, H, bits, 2, out_fp32=True)
+        want_d, _ = O.linear(a, dt, ds, dv, I, H, bits, codebook, out_fp32=True)
         assert close(slot[r0:r1], want_d)[0] == 0, ("down", e)
     base = np.zeros((T, H), dtype=np.float32)
     if shared_np is not None:
@@ -131,8 +131,8 @@ def _check_stages(layer, x, experts_np, shared_np, idx, w, out, T, H, E, k, I, b
         # the always-on expert, stage by stage like the routed ones: its gate / up rows
         # (where the layer keeps them) against the oracle, its down row from the GPU's own
         # gate / up outputs
-        sg_want, _ = O.linear(x, *shared_np[0], H, shared_I, bits, 2)
-        su_want, _ = O.linear(x, *shared_np[1], H, shared_I, bits, 2)
+        sg_want, _ = O.linear(x, *shared_np[0], H, shared_I, bits, codebook)
+        su_want, _ = O.linear(x, *shared_np[1], H, shared_I, bits, codebook)
         if shared_I == I:           # one more expert of the grouped launches: rows P .. P + T - 1
             sg = ws[offs["gate_out"] + P * I * 2:offs["gate_out"] + (P + T) * I * 2].view(np.float16).reshape(T, I)
             su = ws[offs["up_out"] + P * I * 2:offs["up_out"] + (P + T) * I * 2].view(np.float16).reshape(T, I)
@@ -150,7 +150,7 @@ def _check_stages(layer, x, experts_np, shared_np, idx, w, out, T, H, E, k, I, b
                 act = su
                 assert close(act, O.silu_mul(sg, su_want.astype(np.float16)).reshape(T, shared_I),
                              rtol=4e-3, atol=2e-3)[0] == 0, "shared activation"
-        sd_want, _ = O.linear(act, *shared_np[2], shared_I, H, bits, 2, out_fp32=True)
+        sd_want, _ = O.linear(act, *shared_np[2], shared_I, H, bits, codebook, out_fp32=True)
         assert close(base, sd_want)[0] == 0, ("shared down", close(base, sd_want))
     acc = base.astype(np.float32)
     for j in range(k):

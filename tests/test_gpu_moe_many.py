@@ -116,31 +116,52 @@ def test_problems_of_two_three_and_four_row_blocks(T, bits):
     assert torch.equal(res[0], res[1])
 
 
-@pytest.mark.parametrize("T,H,E,k,I,bits,codebook,shared_I", [
-    (150, 384, 6, 2, 384, 4, 2, 0),         # a column block and a half
-    (330, 256, 6, 2, 384, 5, 0, 384),       # problems of four row blocks and the shared expert's
-    (240, 256, 6, 2, 128, 3, 1, 0),
-    (700, 128, 66, 4, 384, 4, 2, 0),        # at least 264 tiles of gate and up: whole; half that of the down projection
-    (700, 128, 66, 4, 256, 2, 1, 128),      # 132 of either: halves
-    (600, 384, 200, 4, 256, 3, 2, 256),     # 200 small problems whole, the always-on expert's as halves
-    (600, 128, 200, 4, 384, 4, 0, 384),     # too many for that; the down projection's all as halves
+def _tiles_in_halves(rows, tiles):
+    """Which problems of a mixed launch run as halves, from the rows of each expert (the kernel's rule for 256 compute units)."""
+    big = small = 0
+    for m in rows:
+        left = m % 128
+        big += m // 128 + (left >= 33)
+        small += 0 < left < 33
+    return "both" if 2 * (big + small) * tiles <= 512 else "first" if (2 * big + small) * tiles <= 512 else "none"
+
+
+@pytest.mark.parametrize("T,H,E,k,I,bits,codebook,shared_I,gate_up,down", [
+    (150, 384, 6, 2, 384, 4, 2, 0, "both", "both"),         # a column block and a half
+    (330, 256, 6, 2, 384, 5, 0, 384, "both", "both"),       # problems of four row blocks and the shared expert's
+    (240, 256, 6, 2, 128, 3, 1, 0, "both", "both"),
+    (700, 128, 66, 4, 384, 4, 2, 0, "first", "both"),       # few problems in the second list
+    (700, 128, 66, 4, 256, 2, 1, 128, "both", "both"),
+    (600, 384, 200, 4, 256, 3, 2, 256, "first", "first"),   # nearly all experts of up to sixteen rows, whole
+    (600, 128, 200, 4, 384, 4, 0, 384, "none", "both"),     # as halves in the down projection
+    (360, 384, 60, 4, 384, 3, 0, 0, "both", "both"),        # nearly all of 17..32 rows, on either side of both rules
+    (560, 256, 100, 4, 384, 3, 1, 384, "first", "both"),
+    (900, 384, 150, 4, 384, 3, 2, 0, "none", "first"),
 ])
-def test_launches_of_few_128_row_tiles_run_them_as_halves(T, H, E, k, I, bits, codebook, shared_I):
-    """Either side of one tile per compute unit, against the 32-row problems' bits (which K of up to 384 keeps whole)."""
+def test_launches_of_few_128_row_tiles_run_them_as_halves(T, H, E, k, I, bits, codebook, shared_I, gate_up, down):
+    """Halves of both lists, of the first alone and of none, against the bits of a launch of 32-row problems only (whole
+    tiles; K of up to 384 is not cut there either)."""
     gpu = Gpu(0)
     wr, _, experts, _, shared = _make_layer(gpu, 9600 + T + bits, H, E, I, bits, shared_I, 1.0)
     x = (synth.activations(9601 + T, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
     d_x, res = dev(x.view(np.uint16)), []
+    idx = torch.zeros((T, k), dtype=torch.int32, device=DEV)
+    w = torch.zeros((T, k), dtype=torch.float32, device=DEV)
     for big_min in (0, 33):
         with knobs(BERTH_MOE_BIG_MIN=big_min):
             layer = MoeLayer(gpu, wr, experts, k, shared=shared, codebook=codebook)
             out = torch.zeros((T, H), dtype=torch.float32, device=DEV)
-            layer.forward(gpu, d_x, out, T)
+            layer.forward(gpu, d_x, out, T, idx, w)
             torch.cuda.synchronize()
             assert ("exl3_gemm_mixed_kernel" in K.moe.last_launch()) == (big_min > 0), K.moe.last_launch()
             assert torch.isfinite(out).all() and (out != 0).any()
             res.append(out)
     assert torch.equal(res[0], res[1])
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        return
+    rows = [int(r) for r in torch.bincount(idx.flatten().long(), minlength=E).cpu()] + ([T] if shared_I == I else [])
+    assert _tiles_in_halves(rows, 2 * -(-I // 256)) == gate_up
+    assert _tiles_in_halves(rows, -(-H // 256)) == down
 
 
 @pytest.mark.parametrize("T,H,E,k", [(3, 128, 128, 8), (2, 128, 300, 10), (5, 128, 512, 32), (2, 64, 1000, 9), (1, 64, 65, 3)])
@@ -235,33 +256,38 @@ def test_gate_up_and_the_next_rotation_in_one_launch(T, H, E, k, I, bits, shared
 
 
 @pytest.mark.parametrize("T,H,E,k,I,bits,shared_I", [
-    (140, 256, 20, 2, 384, 4, 0),       # experts on either side of sixteen rows; 240 tiles of gate and up: halves
-    (150, 128, 150, 3, 384, 3, 0),      # nearly all below; whole tiles
-    (150, 384, 60, 2, 384, 3, 0),       # 240 tiles of gate and up, 120 of the down projection: both launches in halves, the last odd
+    (140, 256, 20, 2, 384, 4, 0),       # experts on either side of sixteen rows; 80 tiles of gate and up: halves
+    (150, 128, 150, 3, 384, 3, 0),      # nearly all below; 150 x 4 tiles whole, 150 of the down projection as halves
+    (150, 384, 60, 2, 384, 3, 0),       # both launches as halves, of a column block and a half
     (16, 384, 2, 1, 128, 5, 128),       # sixteen rows of the always-on expert
     (60, 384, 5, 1, 640, 2, 0),         # gate, up and the next rotation in one launch
 ])
-def test_experts_of_up_to_sixteen_rows(T, H, E, k, I, bits, shared_I):
-    """They take the 16-row matrix instructions whichever list their problem is in (BERTH_MOE_BIG_MIN=9: most of them in
-    that of the 128-row problems): against the oracle, and the same bits for every setting."""
+@pytest.mark.parametrize("codebook", [0, 1, 2])
+def test_experts_of_up_to_sixteen_rows(T, H, E, k, I, bits, shared_I, codebook):
+    """They take the 16-row matrix instructions: against the oracle, stage by stage.  From 129 tokens on whichever list
+    their problem is in (BERTH_MOE_BIG_MIN=9: most of them in that of the 128-row problems), with the same bits (K of
+    up to 384 is not cut)."""
     gpu, res = Gpu(0), []
     wr, experts_np, experts, shared_np, shared = _make_layer(gpu, 9900 + T, H, E, I, bits, shared_I, 1.0)
     x = (synth.activations(9901 + T, T, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
-    want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, 2, shared=shared_np, shared_I=shared_I)
+    want, oi, _ = O.moe_layer(x, wr, experts_np, k, I, bits, codebook, shared=shared_np, shared_I=shared_I)
     rows = np.bincount(oi.reshape(-1), minlength=E)
     assert (rows[rows > 0] <= 16).any() or shared_I
-    for big_min in (0, 9, 33):
+    for big_min in (0, 9, 33) if T >= 129 and T * k >= 256 else (0,):
         with knobs(BERTH_MOE_BIG_MIN=big_min, BERTH_MOE_FEW_TOKENS=0):
-            layer = MoeLayer(gpu, wr, experts, k, shared=shared)
+            layer = MoeLayer(gpu, wr, experts, k, shared=shared, codebook=codebook)
             out = torch.zeros((T, H), dtype=torch.float32, device=DEV)
             idx = torch.zeros((T, k), dtype=torch.int32, device=DEV)
             w = torch.zeros((T, k), dtype=torch.float32, device=DEV)
             layer.forward(gpu, dev(x.view(np.uint16)), out, T, idx, w)
             torch.cuda.synchronize()
+            assert ("exl3_gemm_mixed_kernel" in K.moe.last_launch()) == (big_min > 0), K.moe.last_launch()
+            assert ("exl3_gemm_pair_kernel" in K.moe.last_launch()) == (big_min == 0), K.moe.last_launch()
             assert np.array_equal(idx.cpu().numpy(), oi)
-            _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I)
+            _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), T, H, E, k, I, bits, shared_I,
+                          codebook)
         res.append(out)
-    assert torch.equal(res[0], res[1]) and torch.equal(res[0], res[2])
+    assert all(torch.equal(res[0], other) for other in res[1:])
 
 
 def test_rows_beyond_four_gigabytes_of_rotated_input():
