@@ -150,7 +150,8 @@ static std::string run_stream(const Workspace& ws, const StreamPlan& pl, StreamP
     char m[16];
     std::snprintf(m, sizeof m, "0x%x", mask);
     return "exl3_gemv_stream_kernel<" + std::to_string(bits) + "," + std::to_string(cb) + (p.a_up ? ",silu" : "") +
-           ",table=" + m + "> grid=" + std::to_string(grid.x) + " block=1024 units_per_wave=" + std::to_string(pl.q) +
+           (stream_input(p, cb) == kInPlainLong ? ",zeros" : "") + ",table=" + m + "> grid=" + std::to_string(grid.x) +
+           " block=1024 units_per_wave=" + std::to_string(pl.q) +
            (p.out_fp32 ? " out=f32" : " out=f16");
 }
 

@@ -19,17 +19,13 @@ static void launch_stream_one(const StreamParams& p, dim3 grid, hipStream_t stre
 template <int BITS, int CB>
 static void launch_stream_bits(const StreamParams& p, int lutmask, dim3 grid, hipStream_t stream)
 {
-    const int in = p.norm_x ? kInNorm : (p.a_up ? kInSilu : kInPlain);
+    const int in = stream_input(p, CB);
     auto by_input = [&](auto mask) {
         constexpr int M = decltype(mask)::value;
         if (in == kInNorm) launch_stream_one<BITS, CB, kInNorm, M>(p, grid, stream);
         else if (in == kInSilu) launch_stream_one<BITS, CB, kInSilu, M>(p, grid, stream);
-        else {
-            if constexpr (CB != 0) {
-                if (p.q >= kStreamLongUnits) return launch_stream_one<BITS, CB, kInPlainLong, M>(p, grid, stream);
-            }
-            launch_stream_one<BITS, CB, kInPlain, M>(p, grid, stream);
-        }
+        else if (in == kInPlain) launch_stream_one<BITS, CB, kInPlain, M>(p, grid, stream);
+        else if constexpr (CB != 0) launch_stream_one<BITS, CB, kInPlainLong, M>(p, grid, stream);
     };
     switch (lutmask) {
     case 0x0: by_input(std::integral_constant<int, 0x0>{}); break;

@@ -278,6 +278,10 @@ constexpr int kInPlain = 0, kInSilu = 1, kInNorm = 2;
 // head (2688 x 7296, 2 units, 7.93 -> 8.05).  3INST keeps the copies (17408 x 32768 at 2 bits 88.8 -> 89.2).
 constexpr int kInPlainLong = 3;
 constexpr unsigned kStreamLongUnits = 16;
+inline int stream_input(const StreamParams& p, const int cb)
+{
+    return p.norm_x ? kInNorm : p.a_up ? kInSilu : cb != 0 && p.q >= kStreamLongUnits ? kInPlainLong : kInPlain;
+}
 
 template <int BITS, int CB, int IN, int LUTMASK>
 __global__ __launch_bounds__(1024, 1) void exl3_gemv_stream_kernel(StreamParams p)

@@ -22,7 +22,8 @@ DECODING_KERNELS = (["exl3_gemm_kernel<3, 1, 4>", "exl3_gemm_balanced_kernel<3, 
                     [f"exl3_gemm_mixed_kernel<{bits}, {cb}>" for bits, cb in ((1, 1), (2, 1), (3, 1), (4, 0))] +
                     [f"exl3_gemm_rows_kernel<3, 1, {mt}, {grouped}>" for mt, grouped in ((1, "false"), (2, "false"), (1, "true"))] +
                     ["exl3_gemm_block_kernel<3, 1, 4>", "exl3_gemm_block_kernel<5, 0, 8>"])
-STREAM_KERNELS = ["exl3_gemv_stream_kernel<4, 1, kInPlain, 0>", "exl3_gemv_stream_kernel<5, 0, kInPlain, 0>"]
+STREAM_KERNELS = ["exl3_gemv_stream_kernel<4, 1, kInPlain, 0>", "exl3_gemv_stream_kernel<5, 0, kInPlain, 0>",
+                  "exl3_gemv_stream_kernel<4, 1, kInPlainLong, 0>"]
 
 
 def _operands(text):

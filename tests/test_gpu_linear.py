@@ -483,11 +483,15 @@ def test_lm_head_shape_6bpw_slices_match_oracle():
         assert close(got[c0:c0 + 256], want.reshape(-1))[0] == 0, c0
 
 
-@pytest.mark.parametrize("blocks,units", [(1638, 15), (1641, 16)])
+@pytest.mark.parametrize("units", [15, 16])
 @pytest.mark.parametrize("bits,cb,table", [(3, 1, 0), (4, 2, 0), (4, 2, 10), (2, 0, 0)])
-def test_long_launches_of_one_row(blocks, units, bits, cb, table):
-    """Either side of sixteen units a wave group, from which on the empty row slots of the matrix instructions hold zeros."""
-    Kk, N = 640, 128 * blocks
+def test_long_launches_of_one_row(units, bits, cb, table):
+    """Either side of sixteen units a wave group, from which on the empty row slots of the matrix instructions hold zeros
+    (MUL1 and MCG)."""
+    groups = 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    Kk = 640                                            # ten units a column block
+    blocks = -(-16 * groups // 10) - (units == 15)
+    N = 128 * blocks
     tr, suh, svh = synth.linear(68 + bits, Kk, N, bits)
     x = synth.activations(69 + units, 1, Kk)
     d_tr, d_suh, d_svh, d_x = dev(tr), dev(suh.view(np.uint16)), dev(svh.view(np.uint16)), dev(x.view(np.uint16))
@@ -498,6 +502,7 @@ def test_long_launches_of_one_row(blocks, units, bits, cb, table):
                       d_svh.data_ptr(), 1, Kk, N, bits, cb, OutDtype.F32)
         torch.cuda.synchronize()
     assert "exl3_gemv_stream_kernel" in K.last_launch() and f"units_per_wave={units}" in K.last_launch(), K.last_launch()
+    assert (",zeros" in K.last_launch()) == (units == 16 and cb != 0), K.last_launch()
     got = c.cpu().numpy()
     for c0 in (0, 128 * (blocks // 2), N - 256):
         sub = np.ascontiguousarray(tr[:, c0 // 16:c0 // 16 + 16, :])
