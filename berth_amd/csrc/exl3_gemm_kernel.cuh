@@ -290,8 +290,9 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
 // the four sixteens four tile rows (as in the few-row kernel), and both halves of a wave's columns multiply the
 // same activation.  What the matrix units take there the decode does not get, on a pipe of its own or not: a layer of
 // 64 tokens x 128 experts, four rows an expert, 126 -> 110 us.  The sums of sixteen rows form in another order
-// than those of 32, so that the choice must not depend on how a call cuts its problems: `lone` says that the
-// expert has no more rows, in whichever list it is.
+// than those of 32, so that the choice must not depend on how a call cuts its rows into problems: `lone` says that
+// the expert has no more rows, in whichever list it is.  Whole K only: launches that cut K (gemm_split) keep the 32-row
+// products, whose partial sums they exchange.
 // Rows past the problem repeat its last row: zeros there, with the loads of their lanes switched off, cost the
 // loop more than the zeros save (that layer 104.2 -> 107.4, of 256 tokens x 512 experts 109.9 -> 112.9).
 template <int BITS, int CB, int CG, typename F>            // CG: column groups of 32 a wave
@@ -385,7 +386,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     void* cout = p.c[0];
     int N = p.N, ldc = p.N, nblk_lin = nblk;
     const int32_t* a_rows = nullptr;
-    bool lone = false;                                  // accumulate_16_rows
+    bool lone = false;                                  // accumulate_16_rows (whole K)
     if constexpr (DENSE) {
         const TileView v = dense_tile_view(p, nblk);
         if (v.empty) return;                            // the same for every workgroup that shares the tile

@@ -270,12 +270,16 @@ __device__ __forceinline__ global_ptr<T> uniform_ptr(global_ptr<T> q)
 // down projection, formed with the fp16 steps of berth_ops_silu_mul); or the RMS norm of a
 // fp32 row with the residual added first (the steps of berth_ops_rms_norm_res_in).
 constexpr int kInPlain = 0, kInSilu = 1, kInNorm = 2;
-// The row as given, with zeros in the fifteen empty row slots of the matrix instructions instead of copies: they
-// cost less power, and a long launch runs at the clock that the power leaves it.  us, copies -> zeros, MUL1:
-// 5120 x 248320 at 6 and 4 bits 178.8 -> 175.8 and 152.4 -> 149.0, 5120 x 131072 at 6 95.0 -> 93.7, 5120 x 32768 at 4
-// (20 units a wave group) 24.8 -> 24.2, 17408 x 32768 at 4 79.8 both; MCG 8192 x 32768 at 3 36.2 -> 35.7.
-// From 16 units on: a lane reads one of two LDS addresses then, and short launches lose with that and the zeros at their
-// head (2688 x 7296, 2 units, 7.93 -> 8.05).  3INST keeps the copies (17408 x 32768 at 2 bits 88.8 -> 89.2).
+// The row as given, with zeros in the fifteen empty row slots of the matrix instructions instead of copies.  The gain
+// grows with the launch and is not one of instructions; that zeros cost less power, which leaves a long launch more
+// clock, is what fits it (neither was read).  us, copies -> zeros, MUL1: 5120 x 248320 at 6 and 4 bits 178.8 -> 175.8 and
+// 152.4 -> 149.0; 5120 x 131072, 65536, 49152 (80, 40, 30 units a wave group) at 6 97.6 -> 96.5, 50.9 -> 50.3, 40.1 -> 39.8,
+// at 4 83.9 -> 82.9, 44.8 -> 44.2, 35.5 -> 34.5; 17408 x 32768 at 4 79.8 both; MCG at 3 84.6 -> 83.0, 43.9 -> 43.3, 34.1 both.
+// Nothing from 10 to 20 units: at 4 bits 14.8, 18.0, 20.5, 21.1, 22.1, 22.9 us at 10, 13, 15, 16, 17 and 20 either way, at
+// 6 the same to 1 % less, MCG up to 0.4 % more.  Below that the second LDS address of a lane and the zeros at the head cost
+// 0.5 to 1 % (4 and 6 units 9.30 -> 9.39 and 11.56 -> 11.65, 2 units 7.93 -> 8.05).  The line of 16 lies where neither counts.
+// 3INST keeps the copies (17408 x 32768 at 2 bits 88.8 -> 89.2), and so does a normed input: gate and up of a 27B-shaped
+// layer, 21 units, the layer 68.0 -> 68.1 with zeros (MCG, 3 bits, 68.7 -> 68.5).
 constexpr int kInPlainLong = 3;
 constexpr unsigned kStreamLongUnits = 16;
 inline int stream_input(const StreamParams& p, const int cb)
