@@ -365,7 +365,8 @@ __device__ __forceinline__ void stage_16_rows(float* z, const float4_t (&acc)[CG
 }
 
 // one output tile: rows of problem / row block `tile_y`, 256 columns
-template <int BITS, int CB, int MB, bool DENSE>  // MB = 32-row blocks per workgroup; DENSE: never a problem list
+// MB = 32-row blocks per workgroup; DENSE: never a problem list; SCALAR: the weights' pointer in scalar registers
+template <int BITS, int CB, int MB, bool DENSE, bool SCALAR = false>
 __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y, const int nblk, const KRange kr,
                                           const int which, unsigned char* smem, const GroupProblem* problems = nullptr)
 {
@@ -440,8 +441,8 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[mb][f][r] = 0.0f;
 
-    // (the list of linears is read as vectors: the pointer would be two of a lane's 128 registers through the loop)
-    const uint32_t* const trellis = MB == 1 && !DENSE && CB != 2 ? rows_uniform(lin.trellis) : lin.trellis;
+    // (the list of linears is read as vectors: the pointer would be two of a lane's registers through the loop)
+    const uint32_t* const trellis = SCALAR ? rows_uniform(lin.trellis) : lin.trellis;
     float4_t acc16[2][2] = {};
     if (lone) {
         if (active)
@@ -812,7 +813,7 @@ __global__ __launch_bounds__(256, MB > 1 || DENSE ? 2 : CB != 2 && BITS < 8 ? 4 
         // grouped: (linear, problem, column block)
         kr.counter = ((size_t)gt.which * p.tiles_y + gt.problem) * nblocks + unit;
         kr.slot0 = kr.slot_rest = kr.counter * p.S;
-        gemm_tile<BITS, CB, MB, false>(p, gt.problem, unit, kr, gt.which, smem, p.problems);
+        gemm_tile<BITS, CB, MB, false, CB != 2>(p, gt.problem, unit, kr, gt.which, smem, p.problems);
     }
 }
 
