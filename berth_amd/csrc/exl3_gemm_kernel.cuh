@@ -220,6 +220,38 @@ __device__ __forceinline__ const T* rows_uniform(const T* q)
 
 constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: conflict-free b128 reads)
 
+// The waves of a SIMD run nearly oldest first, so that the last ones end alone, with nobody to fill the cycles that they
+// wait.  A wave gives up its priority in three steps over its second half, which lets the ones behind it catch up.
+// Grouped launches of 32-row problems, layers of 2048 x 768: 64 tokens x 128 experts 104.8 -> 102.7 us, with popular
+// ones 80.2 -> 77.3, 20 tokens 96.0 -> 92.8, 100 tokens x 64 experts 77.2 -> 74.9; 512 experts at 64 tokens, whose
+// workgroups come in six rounds, 175 either way.  Not in mixed launches, whose long tiles have to end first (256
+// tokens x 512 experts 113.8 -> 115.8), nor dense, which have few waves a SIMD (76 rows of 1152x3584 14.7 -> 14.8).
+template <bool ON>
+struct PriorityRamp {
+    int k2, k1, k0, step;
+    __device__ __forceinline__ PriorityRamp(const int kb0, const int kb1, const int step_) : step(step_)
+    {
+        const int n = kb1 - kb0;
+        k2 = kb0 + (n >> 1);
+        k1 = kb0 + (n * 3 >> 2);
+        k0 = kb0 + (n * 7 >> 3);
+        if constexpr (ON) __builtin_amdgcn_s_setprio(3);
+    }
+    // ahead of the k-block kb of kb0, kb0 + step, ...
+    __device__ __forceinline__ void at(const int kb) const
+    {
+        if constexpr (ON) {
+            if ((unsigned)(kb - k2) < (unsigned)step) __builtin_amdgcn_s_setprio(2);
+            if ((unsigned)(kb - k1) < (unsigned)step) __builtin_amdgcn_s_setprio(1);
+            if ((unsigned)(kb - k0) < (unsigned)step) __builtin_amdgcn_s_setprio(0);
+        }
+    }
+    __device__ __forceinline__ void end() const
+    {
+        if constexpr (ON) __builtin_amdgcn_s_setprio(0);
+    }
+};
+
 // The k-loop of a 32-row tile, 64 columns from nw on: every wave is on its own.  The A operand of a lane (row
 // `slot`, 8 k values) is one 16-byte load straight from the rotated rows, so
 // there is no LDS tile and no barrier in the loop.  Trellis and A registers are
@@ -228,8 +260,8 @@ constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: 
 // them it lands in other registers and is moved, 16 of the 513 vector instructions of a k-block.  Layers of 64
 // and 20 tokens x 128 experts 120.7 -> 118.3 and 106.4 -> 104.3 us); on the last k-block the reload reads
 // the same addresses again and is ignored, which keeps the loop free of branches.
-// `requested` is called when the first loads are on their way.
-template <int BITS, int CB, typename F>
+// `requested` is called when the first loads are on their way; RAMP: PriorityRamp.
+template <int BITS, int CB, bool RAMP, typename F>
 __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
                                                    const int arow, const int K, const int kb0, const int kb1, const int step,
                                                    const int lane, float16_t (&acc)[2], F requested)
@@ -254,7 +286,9 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
         }
     }
     requested();
+    const PriorityRamp<RAMP> ramp(kb0, kb1, step);
     for (int kb = kb0; kb < kb1; kb += step) {
+        ramp.at(kb);
         const int nkb = kb + step < kb1 ? kb + step : kb;
         const global_ptr<const uint32_t> tnx = tb + (size_t)(nkb * 8) * row_dw;
         const global_ptr<const half8_t> anx = ab + nkb * 16;
@@ -283,6 +317,7 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
             av[st][1] = anx[4 * st + 1];
         }
     }
+    ramp.end();
 }
 
 // The same for an expert whose rows all fit into sixteen: v_mfma_f32_16x16x32_f16, half the matrix work of the
@@ -295,7 +330,7 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
 // products, whose partial sums they exchange.
 // Rows past the problem repeat its last row: zeros there, with the loads of their lanes switched off, cost the
 // loop more than the zeros save (that layer 104.2 -> 107.4, of 256 tokens x 512 experts 109.9 -> 112.9).
-template <int BITS, int CB, int CG, typename F>            // CG: column groups of 32 a wave
+template <int BITS, int CB, int CG, bool RAMP, typename F>            // CG: column groups of 32 a wave
 __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
                                                    const int arow, const int K, const int lane, float4_t (&acc)[CG][2], F requested)
 {
@@ -318,7 +353,9 @@ __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, cons
     }
     requested();
     const int KB = K >> 7;
+    const PriorityRamp<RAMP> ramp(0, KB, 1);
     for (int kb = 0; kb < KB; ++kb) {
+        ramp.at(kb);
         const int nkb = min(kb + 1, KB - 1);
         const global_ptr<const uint32_t> tnx = tb + (size_t)(nkb * 8) * row_dw;
         const global_ptr<const half8_t> anx = ab + nkb * 16;
@@ -350,6 +387,7 @@ __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, cons
             }
         }
     }
+    ramp.end();
 }
 // its sums to the fp32 tile, 32 * CG columns from z on
 template <int STRIDE, int CG>
@@ -365,8 +403,9 @@ __device__ __forceinline__ void stage_16_rows(float* z, const float4_t (&acc)[CG
 }
 
 // one output tile: rows of problem / row block `tile_y`, 256 columns
-// MB = 32-row blocks per workgroup; DENSE: never a problem list; SCALAR: the weights' pointer in scalar registers
-template <int BITS, int CB, int MB, bool DENSE, bool SCALAR = false>
+// MB = 32-row blocks per workgroup; DENSE: never a problem list; SCALAR: the weights' pointer in scalar registers;
+// RAMP: PriorityRamp in tiles of up to 32 rows
+template <int BITS, int CB, int MB, bool DENSE, bool SCALAR = false, bool RAMP = false>
 __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y, const int nblk, const KRange kr,
                                           const int which, unsigned char* smem, const GroupProblem* problems = nullptr)
 {
@@ -446,11 +485,11 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     float4_t acc16[2][2] = {};
     if (lone) {
         if (active)
-            accumulate_16_rows<BITS, CB>(trellis, row_dw, nw, a_had, a_row_at(min(lane & 15, rows_here - 1)), p.K, lane, acc16, keep_scale);
+            accumulate_16_rows<BITS, CB, 2, RAMP>(trellis, row_dw, nw, a_had, a_row_at(min(lane & 15, rows_here - 1)), p.K, lane, acc16, keep_scale);
         else keep_scale();
     } else if constexpr (MB == 1) {
         if (active && kr.kb0 < kr.kb1)
-            accumulate_32_rows<BITS, CB>(trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
+            accumulate_32_rows<BITS, CB, RAMP>(trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
                                          kr.step, lane, acc[0], keep_scale);      // (rows past the problem repeat its last row)
         else keep_scale();
     } else {
@@ -813,7 +852,7 @@ __global__ __launch_bounds__(256, MB > 1 || DENSE ? 2 : CB != 2 && BITS < 8 ? 4 
         // grouped: (linear, problem, column block)
         kr.counter = ((size_t)gt.which * p.tiles_y + gt.problem) * nblocks + unit;
         kr.slot0 = kr.slot_rest = kr.counter * p.S;
-        gemm_tile<BITS, CB, MB, false, CB != 2>(p, gt.problem, unit, kr, gt.which, smem, p.problems);
+        gemm_tile<BITS, CB, MB, false, CB != 2, true>(p, gt.problem, unit, kr, gt.which, smem, p.problems);
     }
 }
 
@@ -864,7 +903,7 @@ __global__ __launch_bounds__(256, CB != 2 ? 4 : 3) void exl3_gemm_pair_kernel(Ge
     const int at = n0 + 8 * chunk;
     if (gp.lone) {
         float4_t acc[2][2] = {};
-        accumulate_16_rows<BITS, CB>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, lane, acc, keep_scale);
+        accumulate_16_rows<BITS, CB, 2, true>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, lane, acc, keep_scale);
         stage_16_rows<kZStride>(z_tile + wave * 64, acc, lane);
     } else {
         float16_t acc[2];
@@ -872,7 +911,7 @@ __global__ __launch_bounds__(256, CB != 2 ? 4 : 3) void exl3_gemm_pair_kernel(Ge
         for (int f = 0; f < 2; ++f)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[f][r] = 0.0f;
-        accumulate_32_rows<BITS, CB>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, 0, p.K >> 7, 1, lane, acc, keep_scale);
+        accumulate_32_rows<BITS, CB, true>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, 0, p.K >> 7, 1, lane, acc, keep_scale);
         const int col = wave * 64 + (slot >> 3) * 16 + (slot & 7);
 #pragma unroll
         for (int f = 0; f < 2; ++f)
@@ -1100,7 +1139,7 @@ __device__ __forceinline__ void gemm_half_tile_16(const GemmParams& p, const Gro
     int arow = gp.row0 + min(lane & 15, gp.nrows - 1);  // rows past the problem repeat its last row
     if (p.a_rows && !shared) arow = as_global(p.a_rows)[arow];
     float4_t acc[1][2] = {};
-    accumulate_16_rows<BITS, CB>(lin.trellis, (size_t)(p.N >> 4) * (8 * BITS), n0 + 32 * wave, p.a_had[which], arow, p.K, lane, acc, [&]() {
+    accumulate_16_rows<BITS, CB, 1, false>(lin.trellis, (size_t)(p.N >> 4) * (8 * BITS), n0 + 32 * wave, p.a_had[which], arow, p.K, lane, acc, [&]() {
         if (threadIdx.x < 16) s_scale[threadIdx.x] = scale_mine;
     });
     stage_16_rows<kHalfZStride>(z_tile + 32 * wave, acc, lane);
