@@ -171,7 +171,7 @@ static void run_rows(const RowsPlan& pl, GemmParams& p, bool rotate, int k_bits,
 // ---- row blocks (exl3_gemm_block_kernel)
 struct BlockPlan {
     bool ok = false;
-    int rows_per_tile = 0, mt = 0, row_blocks = 0;     // mt: tiles of 16 rows a block has room for
+    int rows_per_tile = 0, mt = 0, row_blocks = 0;     // mt: tiles of 16 rows of a block
     long units = 0;             // steps of 256 x 128 weights
     unsigned grid = 0, q = 0, rem = 0, S = 0, spt = 0;
     size_t operand_at = 0;      // bytes into the partial-sum workspace
@@ -202,7 +202,7 @@ static BlockPlan plan_block(const Workspace& ws, int slices, int slabs, int size
     const int blocks_min = (size_m + 127) / 128;
     pl.rows_per_tile = ((size_m + blocks_min - 1) / blocks_min + 15) / 16 * 16;
     pl.row_blocks = (size_m + pl.rows_per_tile - 1) / pl.rows_per_tile;
-    pl.mt = std::max(4, (pl.rows_per_tile + 31) / 32 * 2);
+    pl.mt = pl.rows_per_tile / 16;
     const unsigned spt = (unsigned)(size_k / 64 + 3) / 4;
     const unsigned long long tiles = (unsigned long long)slices * (size_n / 128) * pl.row_blocks;
     const unsigned long long U = tiles * spt;

@@ -9,7 +9,8 @@
 // (1.66 GHz); both, interleaved in their proportion, 1.65 us; the kernel 1.9.  (Eight waves of
 // 32x32x16 MFMAs, decode interleaved by the instruction, loads three half steps ahead: 2.05.)
 //
-//   * Tile: rows_per_tile rows (a multiple of 16, at most 16 * MT) x 128 columns.  Tiles of one
+//   * Tile: rows_per_tile = 16 * MT rows x 128 columns, MT 3 to 8: a block of 112 rows as one of 128, with a
+//     row tile of nothing, cost a layer of 100 rows 4 % (one of 72 rows as 96: 5 %).  Tiles of one
 //     column block are neighbours, so their weights are in the caches for the next row block.
 //   * Sixteen waves: four column groups of 32 columns x four k groups.  A step is 256 rows of K,
 //     64 per k group (octet layout and operand assignment as in the few-row kernel).
@@ -23,14 +24,18 @@
 //     reads from LDS are lane-linear.
 //   * The steps of the launch, tile-major, are dealt out evenly to one workgroup per compute unit
 //     (or, with few tiles, each tile is cut into S parts).  At the end of a tile the k groups' sums
-//     meet in LDS.  A tile inside one workgroup's steps is finished there; of a shared one every
+//     meet in LDS, in two exchanges of which every wave takes its part: a step each of half of the row
+//     tiles and of a quarter, so that all sixteen waves add, and leave a quarter of the tile in rows.
+//     (Half of the waves adding, then a quarter, which left the rows: layers of 64 and 120 rows 141.8 ->
+//     139.3 and 194.3 -> 184.9 us, the latter also for nine registers that went to scratch memory.)  A tile inside one workgroup's steps is finished there; of a shared one every
 //     sharer leaves its sums in the workspace, and a second launch adds them in k order and
 //     finishes it (exl3_gemm_finish_kernel: inside the first launch the same work falls to the
 //     last sharer alone, which reads half a megabyte per tile through one compute unit: 28 us
 //     instead of 13 outside the steps).
 //
 // Measured (27B layer, 4 bits, whole layer on the host clock, against 32-row and 128-row tiles): 33
-// rows 181 -> 135 us, 64 rows 196 -> 151, 100 rows 245 -> 190, 256 rows 420 -> 311, 384 rows 548 -> 441.
+// rows 181 -> 135 us, 64 rows 196 -> 151, 100 rows 245 -> 190, 256 rows 420 -> 311, 384 rows 548 -> 441.  With
+// odd heights and the exchanges as they are now (another box) 40 rows 131.0 -> 125.4, 72 158 -> 149, 100 185 -> 171, 136 235 -> 222.
 #pragma once
 
 #include "exl3_gemm_rows_kernel.cuh"
@@ -39,9 +44,8 @@ namespace berth {
 
 __host__ __device__ constexpr size_t block_lds_bytes(int mt)
 {
-    // A buffers / the k groups' register dumps (16 KB per 16 rows), or half of that and the
-    // row-major tile behind it; then the output scales
-    return (size_t)mt * (8192 + 16 * kRowsStride * 4) + 256;
+    // A buffers / the k groups' sums on their way (16 KB per 16 rows); then the output scales
+    return (size_t)mt * 16384 + 256;
 }
 
 // Sixteen bytes a lane from base + offset to LDS at lds_at + 16 * lane.  m0 is an output, so that the
@@ -86,13 +90,13 @@ __device__ __forceinline__ void block_finish_row(const GemmParams& p, const Rows
     }
 }
 
-template <int BITS, int CB, int MT>         // MT (even): tiles of 16 rows a block can hold
+template <int BITS, int CB, int MT>         // MT: tiles of 16 rows of a block
 __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int tile_dw = 8 * BITS;
     constexpr int kBuf = MT * 8192;                     // bytes of one A buffer: [k group][row tile][k half][lane][16]
-    constexpr int kLoads = MT / 2;                      // A loads of a wave per step
+    constexpr int kLoads = (MT + 1) / 2;                // A loads of a wave per step
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cg = wave & 3, kg = wave >> 2;
@@ -100,7 +104,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
     const unsigned TR4 = (unsigned)p.K >> 6;
     const unsigned SPT = (TR4 + 3) >> 2;                // steps per tile
     const unsigned RT = (unsigned)p.tiles_y;            // row blocks
-    const int BM = p.rows_per_tile;
+    constexpr int BM = 16 * MT;
 
     // ---- this workgroup's steps [u0, u1)
     const unsigned w = blockIdx.x;
@@ -115,9 +119,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
     const unsigned t_first = div_exact(u0, p.m_tr), t_last = div_exact(u1 - 1, p.m_tr);
 
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
-    float* const dump = (float*)smem;                   // [2][4 column groups][8 * MT][64]
-    float* const z = (float*)(smem + MT * 8192);        // [16 * MT][kRowsStride]
-    uint32_t* const sv_lds = (uint32_t*)(z + 16 * MT * kRowsStride);
+    uint32_t* const sv_lds = (uint32_t*)(smem + MT * 16384);
 
     // ---- operands
     uint32_t own[2][BITS];
@@ -125,7 +127,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
     long t_step = 0;                                    // bytes per step
     uint32_t t_off = 0, t_kg = 0;                       // per lane; bytes from k group 0 to this one
     const char* a_base = nullptr;                       // rotated rows of the tile
-    const uint32_t a_unit = (uint32_t)BM * 128;         // bytes of 64 k of the block
+    constexpr uint32_t a_unit = (uint32_t)BM * 128;     // bytes of 64 k of the block
     auto seek = [&](unsigned tile) {
         const unsigned cb = div_exact(tile, p.m_rt);
         const RowsBlock b = rows_block(p, cb);
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
     auto a_source = [&](unsigned s) {
         return a_base + (size_t)(s * 4 + (s * 4 + (unsigned)kg < TR4 ? (unsigned)kg : 0u)) * a_unit;
     };
-    auto fetch_a = [&](const char* src, int buf, int j) {       // (a lower block than 16 * MT rows: the last piece again)
+    auto fetch_a = [&](const char* src, int buf, int j) {       // (MT odd: the last piece again)
         const uint32_t at = min((uint32_t)(cg * kLoads + j) * 1024u, a_unit - 1024u);
         load_to_lds(src + at, (uint32_t)lane * 16, lds0 + (uint32_t)(buf * kBuf + kg * 2048 * MT) + at);
     };
@@ -246,56 +248,90 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
             fetch_t(0, 0);
             fetch_t(1, min(1u, min(SPT, u1 - base - SPT) - 1));
         }
-        // ---- the k groups' sums: (0 + 2) + (1 + 3), through register dumps
-        float* const mine = dump + ((size_t)(kg & 1) * 4 + cg) * (8 * MT * 64) + lane;
+        // ---- the k groups' sums, (0 + 2) + (1 + 3): groups kg and kg ^ 2 exchange every other row tile, kg and
+        // kg ^ 1 every other one of those that they kept.  A row tile has a place for either parity of the
+        // group that reads it first; what a wave has read there is its own to write.
+        int at = lane;                                  // (what follows from it is worked out here, not kept over the steps)
+        asm volatile("" : "+v"(at));
+        const int par = kg & 1, hi = kg >> 1;
+        unsigned char* const mine = smem + par * 8192 + cg * 2048 + at * 16;
         __syncthreads();
-        if (kg >= 2) {
+        constexpr int kHalf = (MT + 1) / 2, kQuarter = (MT + 3) / 4;
+        float4_t half[kHalf][2], sum[kQuarter][2];
 #pragma unroll
-            for (int i = 0; i < 8 * MT; ++i) mine[i * 64] = acc[i >> 3][(i >> 2) & 1][i & 3];
-        }
-        __syncthreads();
-        if (kg < 2) {
+        for (int i = 0; i < kHalf; ++i) {
+            const bool both = 2 * i + 1 < MT;
 #pragma unroll
-            for (int i = 0; i < 8 * MT; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] += mine[i * 64];
-        }
-        if (kg == 1) {                                  // its own region has been read by nobody else
-#pragma unroll
-            for (int i = 0; i < 8 * MT; ++i) mine[i * 64] = acc[i >> 3][(i >> 2) & 1][i & 3];
-        }
-        __syncthreads();
-        if (kg == 0) {
-            const float* const other = dump + ((size_t)4 + cg) * (8 * MT * 64) + lane;
-#pragma unroll
-            for (int i = 0; i < 8 * MT; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] += other[i * 64];
-        }
-        if (wave == 0) sv_lds[lane] = sv_mine;
-        __syncthreads();                                // the row-major tile lies over the second dump
-        if (kg == 0) {
-            const int col = cg * 32 + (l16 >> 3) * 16 + (l16 & 7);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float* const row = z + (mt * 16 + 4 * lg + r) * kRowsStride + col;
-                    row[0] = acc[mt][0][r];
-                    row[8] = acc[mt][1][r];
+            for (int f = 0; f < 2; ++f) {
+                if (hi) {
+                    *(float4_t*)(mine + 2 * i * 16384 + f * 1024) = acc[2 * i][f];
+                    if (both) half[i][f] = acc[both ? 2 * i + 1 : 0][f];
+                } else {
+                    if (both) *(float4_t*)(mine + (2 * i + 1) * 16384 + f * 1024) = acc[both ? 2 * i + 1 : 0][f];
+                    half[i][f] = acc[2 * i][f];
                 }
+            }
+        }
+        if (wave == 0) sv_lds[at] = sv_mine;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kHalf; ++i) {
+            if (2 * i + 1 < MT || !hi) {
+#pragma unroll
+                for (int f = 0; f < 2; ++f) half[i][f] += *(const float4_t*)(mine + (2 * i + hi) * 16384 + f * 1024);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kQuarter; ++j) {
+            const bool both = 2 * j + 1 < kHalf;
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                if (par) {
+                    *(float4_t*)(mine + (4 * j + hi) * 16384 + f * 1024) = half[2 * j][f];
+                    if (both) sum[j][f] = half[both ? 2 * j + 1 : 0][f];
+                } else {
+                    if (both && (4 * j + 3 < MT || !hi)) *(float4_t*)(mine + (4 * j + 2 + hi) * 16384 + f * 1024) = half[both ? 2 * j + 1 : 0][f];
+                    sum[j][f] = half[2 * j][f];
+                }
+            }
+        }
+        __syncthreads();
+        // Row-major, 16 x 32 of a column group together; four columns at a time change places so that neither side
+        // meets more than two lanes of a bank.
+        const int l16e = at & 15, lge = at >> 4;
+        const uint32_t z_lane = (uint32_t)lge * 512 + (uint32_t)((((l16e >> 3) * 4 + ((l16e >> 2) & 1)) ^ (cg & 1) ^ (2 * (lge & 1))) * 16 + (l16e & 3) * 4);
+#pragma unroll
+        for (int j = 0; j < kQuarter; ++j) {
+            const int mt = 4 * j + 2 * par + hi;
+            if (mt < MT) {
+                const unsigned char* const other = smem + (2 * mt + 1 - par) * 8192 + cg * 2048 + at * 16;
+                unsigned char* const row = smem + (2 * mt + par) * 8192 + cg * 2048;
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    const float4_t v = sum[j][f] + *(const float4_t*)(other + f * 1024);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) *(float*)(row + (z_lane ^ (uint32_t)(f * 32)) + r * 128) = v[r];
+                }
+            }
         }
         __syncthreads();
         if (!b.empty) {
             // sixteen lanes a row, eight columns each: a wave takes four rows at a time
-            const int chunk = had_chunk(lane);
+            const int chunk = had_chunk(at);
             const bool whole = s0 == 0 && s1 == SPT;
             float* const part = p.partials + ((size_t)w * 2 + (tile == t_first ? 0 : 1)) * BM * 128;
+            const uint32_t z_read = (uint32_t)((wave >> 2) * 2 + (wave >> 3)) * 8192 + (uint32_t)(chunk >> 2) * 2048 +
+                                    (uint32_t)((wave & 3) * 4 + lge) * 128 +
+                                    (uint32_t)(((chunk & 3) * 2) ^ ((chunk >> 2) & 1) ^ (2 * (wave & 1))) * 16;
 #pragma unroll
-            for (int pass = 0; pass < MT / 4 + (MT % 4 != 0); ++pass) {
-                const int r = pass * 64 + wave * 4 + lg;
+            for (int pass = 0; pass < kQuarter; ++pass) {
+                const int r = pass * 64 + wave * 4 + lge;
                 if (pass * 64 + wave * 4 >= rows) break;
-                const float4_t* const zr = (const float4_t*)&z[min(r, 16 * MT - 1) * kRowsStride + 8 * chunk];
-                const float4_t v0 = zr[0], v1 = zr[1];
+                const float4_t v0 = *(const float4_t*)(smem + pass * 65536 + z_read);
+                const float4_t v1 = *(const float4_t*)(smem + pass * 65536 + (z_read ^ 16u));
                 if (whole) {
                     float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-                    block_finish_row(p, b, v, ((const half8_t*)sv_lds)[chunk], m0 + r, r < rows, lane);
+                    block_finish_row(p, b, v, ((const half8_t*)sv_lds)[chunk], m0 + r, r < rows, at);
                 } else if (r < rows) {
                     const global_ptr<float4_t> dst = (global_ptr<float4_t>)as_global(part + r * 128 + 8 * chunk);
                     dst[0] = v0;

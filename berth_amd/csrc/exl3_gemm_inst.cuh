@@ -95,7 +95,7 @@ static void gemm_launch_rows(const GemmParams& p, hipStream_t stream, std::strin
            (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
 }
 
-// row blocks of up to 16 * MT rows; mb = -8 - MT
+// row blocks of 16 * MT rows; mb = -8 - MT
 template <int BITS, int CB, int MT>
 static void gemm_launch_block(const GemmParams& p, hipStream_t stream, std::string& desc, dim3 grid)
 {
@@ -118,8 +118,11 @@ static void gemm_launch(const GemmParams& p, int mb, hipStream_t stream, std::st
     else if (mb == -5) gemm_launch_rows<BITS, CB, 1, false, true>(p, stream, desc, grid);
     else if (mb == -6) gemm_launch_rows<BITS, CB, 2, false, true>(p, stream, desc, grid);
     else if (mb == -4) gemm_launch_pair<BITS, CB>(p, stream, desc, grid);
+    else if (mb == -11) gemm_launch_block<BITS, CB, 3>(p, stream, desc, grid);
     else if (mb == -12) gemm_launch_block<BITS, CB, 4>(p, stream, desc, grid);
+    else if (mb == -13) gemm_launch_block<BITS, CB, 5>(p, stream, desc, grid);
     else if (mb == -14) gemm_launch_block<BITS, CB, 6>(p, stream, desc, grid);
+    else if (mb == -15) gemm_launch_block<BITS, CB, 7>(p, stream, desc, grid);
     else if (mb == -16) gemm_launch_block<BITS, CB, 8>(p, stream, desc, grid);
     else if (p.problems) {
         if (mb != 1) throw std::runtime_error("exl3 gemm: problem lists of 32-row tiles, alone or with 128-row ones");

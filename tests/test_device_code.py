@@ -14,7 +14,7 @@ from berth_amd import build as B
 
 # the row-block kernel at every height and over the bit rates' load shapes
 BLOCK_KERNELS = [f"exl3_gemm_block_kernel<{bits}, {cb}, {mt}>" for bits, cb, mt in
-                 ((4, 2, 4), (4, 2, 6), (4, 2, 8), (1, 2, 4), (3, 1, 8), (8, 0, 6))]
+                 ((4, 2, 4), (4, 2, 6), (4, 2, 8), (1, 2, 4), (3, 1, 8), (8, 0, 6), (4, 2, 3), (4, 2, 5), (3, 1, 7))]
 
 # every loop that multiplies freshly decoded weights, with the codebooks whose decode is inline assembly
 DECODING_KERNELS = (["exl3_gemm_kernel<3, 1, 4>", "exl3_gemm_balanced_kernel<3, 1, 4>", "exl3_gemm_kernel<4, 0, 1>",

@@ -46,6 +46,19 @@ def test_row_blocks_match_the_oracle_and_repeat(rows, Kk, N, bits, cb, fp32):
     assert np.array_equal(got.view(np.uint8), again.view(np.uint8)), launch
 
 
+@pytest.mark.parametrize("rows", [34, 48, 50, 66, 80, 81, 96, 99, 112, 113, 210])
+def test_every_height_with_whole_and_shared_tiles(rows):
+    """Blocks of 48 to 128 rows, full and not: the last row tiles of the exchange between the k groups, operand loads that do not
+    divide evenly.  136 tiles (or 272) of two steps for 256 workgroups: some inside one, some shared."""
+    Kk, N, bits = 512, 17408, 4
+    got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, bits, 2, True, 160 + rows, prefill=True)
+    height = (rows if rows <= 128 else rows // 2) + 15 & ~15
+    assert f"exl3_gemm_block_kernel<4,2,{height}x128>" in launch and "exl3_gemm_finish_kernel" in launch, launch
+    assert np.array_equal(ah, want_ah), launch
+    bad, worst = close(got, want)
+    assert bad == 0, (bad, worst, launch)
+
+
 @pytest.mark.parametrize("rows,unit", [(40, 128), (150, 128), (70, 0)])
 def test_bundle_with_narrower_slices(rows, unit):
     """Sliced lists whose widths differ: blocks past a slice's end are empty and touch nothing.  unit 0: four slices of one
