@@ -162,7 +162,7 @@ Knobs read_knobs()
     k.gemm_balanced = env_int("BERTH_GEMM_BALANCED", 1);
     k.gemm_rows256 = env_int("BERTH_GEMM_ROWS256", 1);
     k.gemm_block_steps = env_int("BERTH_GEMM_BLOCK_STEPS", -1);
-    k.gemm_block_rows = env_int("BERTH_GEMM_BLOCK_ROWS", 448);
+    k.gemm_block_rows = env_int("BERTH_GEMM_BLOCK_ROWS", 511);
     k.gemm_rows_units = env_int("BERTH_GEMM_ROWS_UNITS", -1);
     k.counter_stride = clamp(env_int("BERTH_COUNTER_STRIDE", 32), 1, 32);
     k.moe_big_min = env_int("BERTH_MOE_BIG_MIN", 33);

@@ -185,16 +185,41 @@ static bool fills_128_row_tiles(const Workspace& ws, long nblocks, int size_m)
 }
 
 // When row blocks are taken (more than 32 rows).  Measured against the tiles of exl3_gemm_kernel.cuh at 4 bits,
-// 40..448 rows (K x N, us, tiles -> row blocks):
+// 40..511 rows (K x N, us, tiles -> row blocks):
 //   * enough steps that the second launch and the hand-over pay: one per compute unit up to 64 rows (512x4096 14.0 ->
 //     14.7, 512x16384 20.4 -> 19.1, 4096x4096 23.5 -> 21.0), 2.25 of them above (4096x4096 at 100 rows 24.8 -> 27.0,
 //     7296x2688 33.8 -> 28.4);
 //   * narrow outputs, which would run as 32-row tiles and decode every weight once per 32 rows: always (17408x5120 at
 //     64, 128, 256 and 384 rows 59, 88, 162, 167 -> 32, 46, 72, 100), up to gemm_block_rows;
 //   * wide outputs: a launch of 128-row or 256-row tiles costs the same for any rows up to a multiple of those, row
-//     blocks go by the row.  One row block (5120x34816 at 64 rows 62 -> 51, at 128 rows even) and several of up to 96
-//     rows (160 rows 112 -> 104), not several of up to 128 (256 rows 123 -> 137).
-static BlockPlan plan_block(const Workspace& ws, int slices, int slabs, int size_m, int size_k, int size_n)
+//     blocks go by the row (blocks_beside_wide_tiles).
+static bool blocks_beside_wide_tiles(const Workspace& ws, int codebook, long nblocks, int size_m, const BlockPlan& pl, unsigned long long steps)
+{
+    // One row block (5120x34816 at 64 rows 62 -> 51, at 128 rows even) and several of up to 96 rows (160 rows 112 -> 104).
+    if (pl.row_blocks == 1 || pl.rows_per_tile <= 96 || !fills_128_row_tiles(ws, nblocks, size_m)) return true;
+    const long tiles = nblocks * ((size_m + 127) / 128), cus = ws.cu_count;
+    // (1024x6144 at 300 and 448 rows, 2.25 and 3 steps a compute unit: 26.2 -> 28.4, 27.2 -> 31.0)
+    if (steps < 4ull * (unsigned)cus) return false;
+    // 3INST and MCG decode a weight in 4.4 instead of 3.6 instructions, and row blocks decode it more often: where
+    // tiles are few (MCG, K 5120: 200, 256, 336 and 448 rows x 8192 50.6 -> 40.7, 49.5 -> 42.4, 58.2 -> 55.3, 68.8 -> 55.5,
+    // but 336 x 17408 94 -> 97, 200 x 34816 110 -> 119; 3INST 256 rows 2048x12288 39.0 -> 39.7)
+    if (codebook != 2) return tiles <= (pl.rows_per_tile > 112 ? cus / 4 : cus / 2);
+    // Blocks of 128 rows where whole 128-row tiles would fill half of the chip at most and the second launch pays
+    // (256 rows, K 5120 x 8192, 64 tiles: 47.4 -> 41.2; 2048x16384, 128 tiles and eight steps a compute unit: 39.1 -> 28.2;
+    // 2048x12288, 96 tiles and six steps: 36.5 -> 37.7; 384 rows of 5120x12288, 144 tiles: 74.8 -> 80).
+    // Four of them (449..511 rows) where a workgroup has one tile or a part of one: 8192x4096 61.5 -> 55.0, 3072x8192 48.3 ->
+    // 37.6, but 6144x5120, ranges across tiles, 58.2 -> 58.8.
+    if (pl.rows_per_tile > 112)
+        return tiles <= cus / 2 && steps >= 8ull * (unsigned)cus && steps <= 32ull * (unsigned)cus &&
+               (pl.row_blocks <= 3 || 4 * tiles <= cus || 2 * tiles % cus == 0);
+    // Of 112: two blocks (200 rows, K 5120 x 8192, 17408, 34816: 47.5 -> 37.3, 69.7 -> 63.1, 114 -> 113); three beside less than
+    // half a chip or more than a whole of tiles (336 rows x 8192, 17408, 25600, 34816: 57.3 -> 53.5, 91.3 -> 92.0, 134 ->
+    // 128, 175 -> 166); four, which leave little of the second 256 rows empty, beside up to a whole one and up to 32 steps a
+    // compute unit (448 rows x 8192, 12288, 25600: 67 -> 53.5, 86.4 -> 81.7, 155 -> 164; 17408x5120, 42.5 steps: 123 -> 133).
+    return pl.row_blocks == 2 || (pl.row_blocks == 3 ? tiles <= cus / 2 || tiles > cus : tiles <= cus && steps <= 32ull * (unsigned)cus);
+}
+
+static BlockPlan plan_block(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n)
 {
     BlockPlan pl;
     if (!knobs().gemm_balanced || size_m <= 32 || size_m > knobs().gemm_block_rows || size_n % 128 != 0) return pl;
@@ -209,8 +234,7 @@ static BlockPlan plan_block(const Workspace& ws, int slices, int slabs, int size
     if (U >= (1ull << 30)) return pl;
     const int least = knobs().gemm_block_steps;
     if (U < (unsigned long long)(least >= 0 ? least : size_m <= 64 ? 256 : 576)) return pl;
-    if (least < 0 && pl.row_blocks > 1 && pl.rows_per_tile > 96 && fills_128_row_tiles(ws, (long)slices * ((size_n + 255) / 256), size_m))
-        return pl;
+    if (least < 0 && !blocks_beside_wide_tiles(ws, codebook, (long)slices * ((size_n + 255) / 256), size_m, pl, U)) return pl;
     unsigned long long G = (unsigned long long)ws.cu_count;
     if (G > U) G = U;
     unsigned q = (unsigned)(U / G), rem = (unsigned)(U % G), S = 0;
@@ -275,9 +299,9 @@ static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebo
 struct OperandPlan {
     RowsPlan rows;
     BlockPlan block;
-    OperandPlan(const Workspace& ws, int slices, int slabs, int size_m, int size_k, int size_n)
+    OperandPlan(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n)
         : rows(plan_rows(ws, slices, slabs, size_m, size_k, size_n)),
-          block(rows.ok ? BlockPlan{} : plan_block(ws, slices, slabs, size_m, size_k, size_n))
+          block(rows.ok ? BlockPlan{} : plan_block(ws, codebook, slices, slabs, size_m, size_k, size_n))
     {
         stride = rows.ok ? rows_operand_elements(size_k, rows.mt) : block.operand_stride;
         at = (_Float16*)((char*)ws.partials + (rows.ok ? rows.operand_at : block.operand_at));
@@ -396,7 +420,7 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     if (!scratch) scope.emplace(a.stream);
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
-    const OperandPlan plan(ws, 1, 1, a.size_m, a.size_k, a.size_n);
+    const OperandPlan plan(ws, a.codebook, 1, 1, a.size_m, a.size_k, a.size_n);
     RotateArgs rot;
     rot.in = a.a;
     rot.up = a.a_up;
@@ -454,7 +478,7 @@ std::string launch_gemm_bundle(const MgemmArgs& m)
     Workspace& ws = scope.ws;
     throw_pending_device_fault(ws);
     const int slabs = sliced ? m.num_had_src : m.bszm_out;
-    const OperandPlan plan(ws, m.bszm_out, slabs, m.size_m, m.size_k, m.size_n);
+    const OperandPlan plan(ws, m.codebook, m.bszm_out, slabs, m.size_m, m.size_k, m.size_n);
     // what the kernel multiplies: the rotated rows, or their copy in operand order
     const size_t slab_stride = plan.ok() ? plan.stride : (size_t)m.size_m * m.size_k;
     const _Float16* const slab0 = (const _Float16*)(plan.ok() ? plan.at : m.a_had);
@@ -574,7 +598,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second, PairNext* ne
     if (!scratch) scope.emplace(a.stream);
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
-    const OperandPlan plan(ws, 2, 2, a.size_m, a.size_k, a.size_n);
+    const OperandPlan plan(ws, a.codebook, 2, 2, a.size_m, a.size_k, a.size_n);
     GemmParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
@@ -617,7 +641,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second, PairNext* ne
     std::string desc;
     // Row blocks finish their tiles in a second launch, which can go on to the next linear's input.  Its copy in
     // operand order lies behind the partial sums that the launch still reads.
-    const OperandPlan after(ws, 1, 1, a.size_m, a.size_n, next ? next->size_n : 128);
+    const OperandPlan after(ws, a.codebook, 1, 1, a.size_m, a.size_n, next ? next->size_n : 128);
     const size_t operand_at = std::max(plan.block.operand_at, after.block.operand_at);
     if (next && plan.block.ok && !after.rows.ok && operand_at + after.block.operand_stride * 2 <= ws.partial_bytes) {
         FinishActivation f{(const _Float16*)next->suh, (_Float16*)next->a_had, nullptr, 1};

@@ -270,7 +270,7 @@ typedef struct {
  * both; the up projection's rotated copy waits in act_had, so this form needs
  * intermediate >= hidden, else gate and up run one after the other), one launch that
  * forms silu(g) * u and rotates it, the down projection.  The row-block kernel
- * (33..448 rows) adds a launch that finishes its shared tiles; behind gate and up that
+ * (33..511 rows) adds a launch that finishes its shared tiles; behind gate and up that
  * launch also forms silu(g) * u and rotates it.
  * lins: HOST array {gate, up, down} of device pointers.  x fp16 [m][hidden];
  * gate_out, up_out fp16 [m][intermediate] (written; above 8 rows up_out ends up

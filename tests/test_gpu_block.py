@@ -59,6 +59,29 @@ def test_every_height_with_whole_and_shared_tiles(rows):
     assert bad == 0, (bad, worst, launch)
 
 
+@pytest.mark.parametrize("rows,Kk,N,cb,blocks", [
+    (200, 2048, 8192, 2, True),         # two blocks of 112 rows, four steps a compute unit
+    (300, 1024, 8192, 2, False),        # three steps a compute unit
+    (200, 2048, 8192, 1, True),         # MCG: beside up to half a chip of tiles
+    (300, 2048, 8192, 2, True),         # three blocks: up to half a chip
+    (300, 2048, 12288, 2, False),
+    (400, 2048, 8192, 2, True),         # four blocks: up to a whole chip, 32 steps a compute unit
+    (400, 8448, 8192, 2, False),
+    (450, 2048, 8192, 2, True),         # blocks of 128: one tile a workgroup
+    (450, 3072, 6144, 2, False),        # ranges across tiles
+    (513, 2048, 8192, 2, False),        # above the limit of rows
+])
+def test_the_rule_beside_wide_tiles(rows, Kk, N, cb, blocks):
+    """Both sides of the rule that sends several row blocks of wide outputs to this kernel, each against the oracle."""
+    with knobs(BERTH_GEMM_BLOCK_ROWS=511, BERTH_GEMM_BLOCK_STEPS=-1):        # the rule as it is, on a card of 256 compute units
+        got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, 3, cb, False, 260 + rows, prefill=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert ("exl3_gemm_block_kernel" in launch) == blocks, launch
+    assert np.array_equal(ah, want_ah), launch
+    bad, worst = close(got, want)
+    assert bad == 0, (bad, worst, launch)
+
+
 @pytest.mark.parametrize("rows,unit", [(40, 128), (150, 128), (70, 0)])
 def test_bundle_with_narrower_slices(rows, unit):
     """Sliced lists whose widths differ: blocks past a slice's end are empty and touch nothing.  unit 0: four slices of one
