@@ -578,13 +578,13 @@ extern "C" const char* berth_prefill_last_launch(void) { return g_prefill_launch
 // fills only afterwards), one dense launch runs both.
 static bool mlp_pair_on_matrix_units(int size_m, int hidden, int intermediate)
 {
-    return intermediate >= hidden && (size_m > 8 || gemv_rows_on_matrix_units(2, size_m, hidden, intermediate));
+    return intermediate >= hidden && size_m > 1 && (size_m > 8 || gemv_rows_on_matrix_units(2, size_m, hidden, intermediate));
 }
 
-// gate and up; `norm`: the input is that norm's rows instead of pair.a
-static std::string mlp_gate_up(const PairArgs& pair, void* act_had, PairNext* next, const Workspace* scratch)
+// gate and up where they are no bundle on the MFMA kernels, or one of few rows whose down projection takes the VALU kernel
+static std::string mlp_gate_up(const PairArgs& pair, void* act_had, bool on_matrix_units)
 {
-    if (mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n)) return launch_gemm_pair(pair, act_had, next, scratch);
+    if (on_matrix_units) return launch_gemm_pair(pair, act_had);
     if (pair.size_m <= 8) return launch_gemv_pair(pair);
     std::string desc;
     for (int i = 0; i < 2; ++i) {
@@ -595,31 +595,24 @@ static std::string mlp_gate_up(const PairArgs& pair, void* act_had, PairNext* ne
     return desc;
 }
 
-// down(silu(gate) * up), with out_add added to its output.  Above 8 rows up_out ends up holding the
-// activation, which is formed where it is rotated.
-static std::string mlp_down(LinearArgs down, void* gate_out, void* up_out, const float* out_add)
-{
-    down.a = gate_out;
-    down.a_up = up_out;
-    down.out_add = out_add;
-    if (down.size_m <= 8) return launch_gemv(down);
-    down.act_out = up_out;
-    return launch_gemm(down);
-}
-
-// gate, up and down: the finish of gate and up may leave down its input
+// gate, up and down(silu(gate) * up), with out_add added to its output; the finish of gate and up may leave
+// down its input.  Above 8 rows up_out ends up holding the activation, which is formed where it is rotated.
 static std::string mlp_linears(const PairArgs& pair, LinearArgs down, const float* out_add)
 {
     void* const act_had = down.a_had;
-    if (pair.size_m <= 32 || !mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n))
-        return mlp_gate_up(pair, act_had, nullptr, nullptr) + " ; " + mlp_down(down, pair.c[0], pair.c[1], out_add);
-    LaunchScope scope(pair.stream);
-    PairNext next{down.suh, act_had, down.size_n};
-    const std::string desc = mlp_gate_up(pair, act_had, &next, &scope.ws) + " ; ";
+    const bool few = pair.size_m <= 8;
     down.a = pair.c[0];
     down.a_up = pair.c[1];
-    down.act_out = pair.c[1];
+    down.act_out = few ? nullptr : pair.c[1];
     down.out_add = out_add;
+    const bool on_matrix_units = mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n);
+    if (!on_matrix_units || (few && !gemv_rows_on_matrix_units(1, down.size_m, down.size_k, down.size_n))) {
+        const std::string desc = mlp_gate_up(pair, act_had, on_matrix_units) + " ; ";
+        return desc + (few ? launch_gemv(down) : launch_gemm(down));
+    }
+    LaunchScope scope(pair.stream);
+    PairNext next{down.suh, act_had, down.size_n, few ? 1 : 0};
+    const std::string desc = launch_gemm_pair(pair, act_had, &next, &scope.ws) + " ; ";
     down.rotated = next.done;
     down.rotated_operand = next.operand;
     return desc + launch_gemm(down, &scope.ws);
@@ -661,9 +654,9 @@ extern "C" int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* g
 // it (ops.rs:522-552, add_f32), as crates/berth-engine/src/mlp.rs:118-150 is called from the
 // block.  One row whose linears take the streaming kernel: two launches, the norm formed while
 // the gate / up launch rotates its input, the sum added where the down launch writes its output.
-// Rows on the MFMA kernels: four launches, the norm formed where the input is rotated, the
-// activation likewise, the sum added where the down launch writes (row blocks: the activation where
-// gate's and up's tiles are finished, and a launch more where down shares tiles).
+// Rows on the MFMA kernels: three or four launches, the norm formed where the input is rotated, the
+// activation where gate and up are finished (2..32 rows: by their launch; row blocks: by one more, as
+// where down shares tiles) or where it is rotated, the sum added where the down launch writes.
 extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* residual_out, const berth_rms_norm* norm,
                                     const berth_exl3_lin* lins, void* h_norm, void* gate_out, void* up_out, void* a_had,
                                     void* act_had, void* y, int size_m, int hidden, int intermediate, int k_bits,

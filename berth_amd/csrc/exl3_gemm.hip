@@ -149,8 +149,9 @@ bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, 
     return plan_rows(ws, slices, slices, size_m, size_k, size_n).ok;
 }
 
-// rotate: p is a GemmRotateParams
-static void run_rows(const RowsPlan& pl, GemmParams& p, bool rotate, int k_bits, int codebook, hipStream_t stream, std::string& desc)
+// rotate: p is a GemmRotateParams; pair: a RowsPairParams
+static void run_rows(const RowsPlan& pl, GemmParams& p, bool rotate, int k_bits, int codebook, hipStream_t stream, std::string& desc,
+                     bool pair = false)
 {
     p.cstride = gemm_counter_stride((long)(p.num_slices > 0 ? p.num_slices : 1) * (p.N / 128));
     p.units = (int)pl.units;
@@ -164,7 +165,7 @@ static void run_rows(const RowsPlan& pl, GemmParams& p, bool rotate, int k_bits,
     p.m_q1 = magic(pl.q + 1);
     p.lds_bytes = (unsigned)(rotate ? pl.lds_rotate : pl.lds);
     if (rotate) static_cast<GemmRotateParams&>(p).m_rows = magic((unsigned)p.M);
-    gemm_bits(p, k_bits, codebook, (rotate ? -4 : 0) - pl.mt, stream, desc, dim3(pl.grid));
+    gemm_bits(p, k_bits, codebook, (pair ? -6 : rotate ? -4 : 0) - pl.mt, stream, desc, dim3(pl.grid));
     hip_ok(hipGetLastError(), "exl3_gemm_rows_kernel launch");
 }
 
@@ -599,7 +600,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second, PairNext* ne
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
     const OperandPlan plan(ws, a.codebook, 2, 2, a.size_m, a.size_k, a.size_n);
-    GemmParams p{};
+    RowsPairParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();
     p.a_had[0] = (const _Float16*)a.a_had;
@@ -621,6 +622,15 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second, PairNext* ne
         g.n_stride = a.size_n;
         g.a_had = (const _Float16*)slabs[i];
     }
+    // What the launch leaves for the next linear: few rows in the launch itself (its partial sums then take twice
+    // the room, and the copies of its input in operand order move up), row blocks in the one that finishes their
+    // tiles.  The next linear's copy lies behind its partial sums, and behind what of these is still read.
+    const OperandPlan after(ws, a.codebook, 1, 1, a.size_m, a.size_n, next ? next->size_n : 128);
+    // (Column blocks cut into more than two parts: a pair is handed over by all of them, and the next launch is short.)
+    const size_t in_at = plan.rows.operand_at * 2, next_at = std::max(in_at + 2 * plan.stride * 2, after.rows.operand_at);
+    const bool pair_rows = next && plan.rows.ok && plan.rows.S <= 2 && !after.block.ok &&
+                           next_at + (after.rows.ok ? after.stride * 2 : 0) <= ws.partial_bytes;
+    _Float16* const operand = pair_rows ? (_Float16*)((char*)ws.partials + in_at) : plan.at;
     RotateArgs rot;
     rot.in = a.a;
     rot.norm = a.norm;
@@ -631,19 +641,27 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second, PairNext* ne
     rot.cols = a.size_k;
     rot.stream = a.stream;
     if (plan.ok()) {
-        rot.operand = plan.at;
+        rot.operand = operand;
         rot.mt = plan.mt();
-        for (int i = 0; i < 2; ++i) p.slice[i].a_had = plan.at + i * plan.stride;
+        for (int i = 0; i < 2; ++i) p.slice[i].a_had = operand + i * plan.stride;
     }
     std::string d0 = launch_rotate(rot);
     const long nblocks = 2L * ((a.size_n + 255) / 256);
     if (nblocks * ((a.size_m + 31) / 32) > kCounters / 2) throw std::runtime_error("exl3 linear pair: too many output tiles");
     std::string desc;
-    // Row blocks finish their tiles in a second launch, which can go on to the next linear's input.  Its copy in
-    // operand order lies behind the partial sums that the launch still reads.
-    const OperandPlan after(ws, a.codebook, 1, 1, a.size_m, a.size_n, next ? next->size_n : 128);
     const size_t operand_at = std::max(plan.block.operand_at, after.block.operand_at);
-    if (next && plan.block.ok && !after.rows.ok && operand_at + after.block.operand_stride * 2 <= ws.partial_bytes) {
+    if (pair_rows) {
+        p.suh = (const _Float16*)next->suh;
+        p.act_had = (_Float16*)next->a_had;
+        p.keep_up = next->keep_up;
+        if (after.rows.ok) {
+            p.operand = (_Float16*)((char*)ws.partials + next_at);
+            p.operand_mt = after.mt();
+        }
+        run_rows(plan.rows, p, false, a.k_bits, a.codebook, a.stream, desc, true);
+        next->operand = p.operand;
+        next->done = true;
+    } else if (next && plan.block.ok && !after.rows.ok && operand_at + after.block.operand_stride * 2 <= ws.partial_bytes) {
         FinishActivation f{(const _Float16*)next->suh, (_Float16*)next->a_had, nullptr, 1};
         if (after.block.ok) {
             f.operand = (_Float16*)((char*)ws.partials + operand_at);

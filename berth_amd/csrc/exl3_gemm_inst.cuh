@@ -78,20 +78,24 @@ static void gemm_launch_pair(const GemmParams& p, hipStream_t stream, std::strin
 }
 
 // few rows (2..32), units dealt out evenly; mb = -1 / -2: one or two tiles of 16 rows (-5 / -6: which the launch
-// rotates itself, p a GemmRotateParams), -3: a list of problems of up to 16 rows
-template <int BITS, int CB, int MT, bool GROUPED = false, bool ROT = false>
+// rotates itself, p a GemmRotateParams), -3: a list of problems of up to 16 rows; -7 / -8: gate and up,
+// with the down projection's rotated input (p a RowsPairParams)
+template <int BITS, int CB, int MT, bool GROUPED = false, bool ROT = false, bool PAIR = false>
 static void gemm_launch_rows(const GemmParams& p, hipStream_t stream, std::string& desc, dim3 grid)
 {
     static bool raised[64] = {};
-    raise_dynamic_lds_limit((const void*)exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT>, 160 * 1024, raised,
+    raise_dynamic_lds_limit((const void*)exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT, PAIR>, 160 * 1024, raised,
                             "exl3_gemm_rows_kernel shared-memory attribute");
     if constexpr (ROT)
         hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT>), grid, dim3(1024), p.lds_bytes, stream,
                            static_cast<const GemmRotateParams&>(p));
+    else if constexpr (PAIR)
+        hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT, PAIR>), grid, dim3(1024), p.lds_bytes, stream,
+                           static_cast<const RowsPairParams&>(p));
     else
         hipLaunchKernelGGL((exl3_gemm_rows_kernel<BITS, CB, MT, GROUPED, ROT>), grid, dim3(1024), p.lds_bytes, stream, p);
     desc = "exl3_gemm_rows_kernel<" + std::to_string(BITS) + "," + std::to_string(CB) + "," + std::to_string(16 * MT) +
-           "x128" + (ROT ? ",rotate" : "") + "> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
+           "x128" + (ROT ? ",rotate" : PAIR ? ",silu,rotate" : "") + "> grid=" + std::to_string(grid.x) + " units=" + std::to_string(p.units) +
            (p.S ? " split_k=" + std::to_string(p.S) : "") + " smem=" + std::to_string(p.lds_bytes);
 }
 
@@ -117,6 +121,8 @@ static void gemm_launch(const GemmParams& p, int mb, hipStream_t stream, std::st
     else if (mb == -3) gemm_launch_rows<BITS, CB, 1, true>(p, stream, desc, grid);
     else if (mb == -5) gemm_launch_rows<BITS, CB, 1, false, true>(p, stream, desc, grid);
     else if (mb == -6) gemm_launch_rows<BITS, CB, 2, false, true>(p, stream, desc, grid);
+    else if (mb == -7) gemm_launch_rows<BITS, CB, 1, false, false, true>(p, stream, desc, grid);
+    else if (mb == -8) gemm_launch_rows<BITS, CB, 2, false, false, true>(p, stream, desc, grid);
     else if (mb == -4) gemm_launch_pair<BITS, CB>(p, stream, desc, grid);
     else if (mb == -11) gemm_launch_block<BITS, CB, 3>(p, stream, desc, grid);
     else if (mb == -12) gemm_launch_block<BITS, CB, 4>(p, stream, desc, grid);

@@ -34,6 +34,16 @@
 //     lanes past the last repeat it, so that a load touches as many lines as there are rows.
 //     Gate and up, 2048 x 768 at 4 bits, 2 / 8 / 16 tokens that choose 8 of 128 experts: 15 / 30 / 45 us.
 //
+//   * PAIR: gate and up of an MLP, their blocks of the same columns next to each other.  What is handed over is a
+//     pair of them, and its finisher goes on to silu(g) * u and the rotated input of the down projection, for which a
+//     launch of its own would read both back: decoder layers of 5120 x 17408 at 5 / 8 / 12 / 24 / 32 rows 89.1 -> 86.1,
+//     91.4 -> 87.9, 92.4 -> 89.4, 111.6 -> 108.4, 121.3 -> 118.5 us, of 2048 x 5632 at 5 and 32 rows 57.7 -> 54.5,
+//     72.2 -> 66.8.  The grouped form gained nothing (8 tokens 67.4 -> 66.7, 16 85.4 -> 85.3): its tail grew by what the
+//     launch took.  The tail of gate + up at 24 rows takes a quarter of the launch (the last wave ends its walk at 29 us, the
+//     finishers at 38): sums in LDS 2 us, stores until they are there 1, the counter 0.7, parts read and finished 2
+//     for each row of a wave, so that a wave asks for both of its rows together.  (The same at the end of the other
+//     launches, which have more sharers: 20 rows of 2048x8192 12.2 -> 12.8.)
+//
 // Measured (27B layer, traced): gate + up at 5 rows and 3 bits 62.6 -> 32.5 us against the VALU
 // kernel, at 24 rows and 4 bits 49.0 -> 40.6 against 32-row tiles (whose 544 workgroups also
 // ran in one and a bit rounds), down 47.4 -> 19.1 and 38 -> 23.0.  Of the 41 us at 24 rows the
@@ -85,6 +95,14 @@ __host__ __device__ constexpr size_t rows_group_lds_bytes(int rows, int ncb)
     return rows_lds_bytes(rows, ncb) + (size_t)ncb * sizeof(RowsGroupBlock);
 }
 
+// PAIR: what follows gate and up
+struct RowsPairParams : GemmParams {
+    const _Float16* suh;        // input scales of the down projection
+    _Float16* operand;          // a second copy of its rotated rows in operand order (may be null)
+    int operand_mt;
+    int keep_up;                // 1: up goes to its output; 0: the activation does
+};
+
 // x / d for the launch's exact divisors, m = floor(2^32 / d) + 1 (0 for d = 1)
 __device__ __forceinline__ unsigned div_exact(unsigned x, unsigned m) { return m ? __umulhi(x, m) : x; }
 
@@ -99,6 +117,7 @@ struct RowsBlock {
     bool empty;                 // past the end of a narrower slice: nothing to compute
     int rows;                   // of the block (GROUPED only)
 };
+template <bool PAIR = false>
 __device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsigned cb)
 {
     RowsBlock b;
@@ -110,7 +129,14 @@ __device__ __forceinline__ RowsBlock rows_block(const GemmParams& p, const unsig
     b.ldc = p.N;
     b.empty = false;
     b.rows = p.M;
-    if (p.num_slices > 0) {
+    if (PAIR) {
+        const GemmSlice& g = p.slice[cb & 1];
+        b.trellis = g.trellis;
+        b.svh = g.svh;
+        b.a_had = g.a_had;
+        b.c = g.c;
+        b.n0 = (int)(cb >> 1) * 128;
+    } else if (p.num_slices > 0) {
         const unsigned nb = (unsigned)p.N >> 7;
         const unsigned sl = div_exact(cb, p.m_nb);
         b.n0 = (int)(cb - sl * nb) * 128;
@@ -157,10 +183,11 @@ __device__ __forceinline__ GemmRotation rows_rotation(const GemmRotateParams& p,
             first ? p.rot_out + (size_t)sl * p.M * p.K : nullptr};
 }
 
-template <int BITS, int CB, int MT, bool GROUPED, bool ROT = false>     // MT: tiles of 16 rows
-__global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditional_t<ROT, GemmRotateParams, GemmParams> p)
+template <int BITS, int CB, int MT, bool GROUPED, bool ROT = false, bool PAIR = false>      // MT: tiles of 16 rows
+__global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(
+    std::conditional_t<ROT, GemmRotateParams, std::conditional_t<PAIR, RowsPairParams, GemmParams>> p)
 {
-    static_assert(!GROUPED || !ROT, "a problem list brings its rows rotated");
+    static_assert(GROUPED + ROT + PAIR <= 1, "a problem list and a pair bring their rows rotated");
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int tile_dw = 8 * BITS;
     const int lane = threadIdx.x & 63;
@@ -234,7 +261,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditiona
             b.rows = __builtin_amdgcn_readfirstlane(g.rows);
             return b;
         } else {
-            return rows_block(p, cb);
+            return rows_block<PAIR>(p, cb);
         }
     };
 
@@ -361,7 +388,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditiona
     }
     // the output scales, asked for now: the finish does not wait for them
     uint32_t sv_mine = 0;
-    if ((unsigned)wave < ncb) {
+    if (!PAIR && (unsigned)wave < ncb) {
         const RowsBlock b = block(cb_first + (unsigned)wave);
         if (!b.empty) sv_mine = as_global((const uint32_t*)(b.svh + b.n0))[lane];
     }
@@ -441,8 +468,151 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditiona
     if constexpr (!ROT) __builtin_amdgcn_s_setprio(0);
     if ((w1 - w0) & 1) stage(0);
     if (ROT || k != 0) flush();
-    if ((unsigned)wave < ncb) sv_lds[wave * 64 + lane] = sv_mine;
+    if (!PAIR && (unsigned)wave < ncb) sv_lds[wave * 64 + lane] = sv_mine;
     __syncthreads();
+
+    const unsigned qs1 = u0 + (L >> 2), qs2 = u0 + (L * 2 >> 2), qs3 = u0 + (L * 3 >> 2);
+    // this workgroup's sum of a row of column block cb_first + cbi, two columns a lane
+    auto own_sum = [&](const unsigned cbi, const int row, float& z0, float& z1) {
+        const unsigned c0 = (cb_first + cbi) * TR4, c1 = c0 + TR4;
+        const float* const base = red + (size_t)cbi * M * kRowsStride + row * kRowsStride + 2 * lane;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const unsigned a0 = g == 0 ? u0 : g == 1 ? qs1 : g == 2 ? qs2 : qs3;
+            const unsigned a1 = g == 0 ? qs1 : g == 1 ? qs2 : g == 2 ? qs3 : u1;
+            if (a0 < c1 && a1 > c0) {
+                const float2_t part = *(const float2_t*)(base + (size_t)g * M * kRowsStride);
+                z0 += part.x;
+                z1 += part.y;
+            }
+        }
+    };
+    // the workgroup that unit x of the launch belongs to
+    auto owner = [&](unsigned x) {
+        const unsigned big = rem * (q + 1);
+        if constexpr (GROUPED) return x < big ? x / (q + 1) : rem + (x - big) / q;
+        if (S) return div_exact(x, p.m_tr) * S + (x % TR4 ? S - 1 : 0u);     // asked for a block's first or last unit
+        return x < big ? div_exact(x, p.m_q1) : rem + div_exact(x - big, p.m_q);
+    };
+
+    if constexpr (PAIR) {
+        // ---- finish: a wave takes (pair, row) vectors, two columns a lane of gate, of up and of what follows them
+        const unsigned P0 = cb_first >> 1, P1 = cb_last >> 1, PU = 2 * TR4;
+        const bool first_shared = !(u0 == P0 * PU && u1 >= (P0 + 1) * PU), last_shared = P1 > P0 && u1 < (P1 + 1) * PU;
+        struct Scales {
+            half2_t sv[2], su;
+        };
+        auto scales = [&](const unsigned pair) -> Scales {
+            const int n0 = (int)pair * 128;
+            return {{((global_ptr<const half2_t>)as_global(p.slice[0].svh + n0))[lane], ((global_ptr<const half2_t>)as_global(p.slice[1].svh + n0))[lane]},
+                    ((global_ptr<const half2_t>)as_global(p.suh + n0))[lane]};
+        };
+        auto finish_row = [&](const unsigned pair, const int row, float (&z)[2][2], const Scales& sc) {
+            half2_t gu[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                had128_wave(z[h][0], z[h][1], lane);
+                gu[h].x = (_Float16)rounded((z[h][0] * kRsqrt128) * (float)sc.sv[h].x);
+                gu[h].y = (_Float16)rounded((z[h][1] * kRsqrt128) * (float)sc.sv[h].y);
+            }
+            half2_t x;
+            x.x = silu_mul_h(gu[0].x, gu[1].x);
+            x.y = silu_mul_h(gu[0].y, gu[1].y);
+            float v0 = __builtin_fmaf((float)x.x, (float)sc.su.x, 0.0f), v1 = __builtin_fmaf((float)x.y, (float)sc.su.y, 0.0f);
+            had128_wave(v0, v1, lane);
+            half2_t o;
+            o.x = (_Float16)had_scale(v0, kRsqrt128);
+            o.y = (_Float16)had_scale(v1, kRsqrt128);
+            const int col = (int)pair * 128 + 2 * lane;
+            const size_t at = (size_t)row * p.N + col;
+            *(global_ptr<half2_t>)(as_global((_Float16*)p.slice[0].c) + at) = gu[0];
+            *(global_ptr<half2_t>)(as_global((_Float16*)p.slice[1].c) + at) = p.keep_up ? gu[1] : x;
+            *(global_ptr<half2_t>)(as_global(p.act_had) + at) = o;
+            if (p.operand) *(global_ptr<half2_t>)(as_global(p.operand) + rows_operand_offset(row, col & ~7, p.operand_mt) + (col & 7)) = o;
+        };
+        // the partial sums: [workgroup][first or last pair][gate, up][M][128]
+        auto slot = [&](unsigned x, unsigned which) { return p.partials + ((size_t)x * 4 + which) * M * 128; };
+        for (unsigned pair = P0; pair <= P1; ++pair) {
+            const bool shared = (pair == P0 && first_shared) || (pair == P1 && last_shared);
+            for (int row = wave; row < M; row += kRowsWaves) {
+                float z[2][2] = {};
+#pragma unroll
+                for (unsigned h = 0; h < 2; ++h) {
+                    const unsigned cbx = 2 * pair + h;
+                    if (cbx < cb_first || cbx > cb_last) continue;
+                    own_sum(cbx - cb_first, row, z[h][0], z[h][1]);
+                    if (!shared) continue;
+                    unsigned long long* const dst = (unsigned long long*)(slot(w, (pair == P0 ? 0u : 2u) + h) + row * 128) + lane;
+                    __hip_atomic_store(dst, __builtin_bit_cast(unsigned long long, float2_t{z[h][0], z[h][1]}), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if (!shared) finish_row(pair, row, z, scales(pair));
+            }
+        }
+        if (!first_shared && !last_shared) return;
+        wait_own_stores();
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            unsigned done = 0;
+            if (threadIdx.x == 0 ? first_shared : last_shared) {
+                const unsigned pair = threadIdx.x == 0 ? P0 : P1;
+                const unsigned parts = owner(pair * PU + PU - 1) - owner(pair * PU) + 1;
+                unsigned* const counter = p.counters + (size_t)pair * p.cstride;
+                const unsigned old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (old == parts - 1) {
+                    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    done = 1;
+                }
+            }
+            flags[threadIdx.x] = done;
+        }
+        __syncthreads();
+        // The wave's one or two rows of a pair together, four parts of gate and of up at a time (there are seldom more).
+        constexpr int kRowsEach = MT;
+#pragma unroll 1
+        for (int t = 0; t < 2; ++t) {
+            if (!__builtin_amdgcn_readfirstlane((int)flags[t])) continue;
+            const unsigned pair = t == 0 ? P0 : P1;
+            const Scales sc = scales(pair);
+            const unsigned wp = owner(pair * PU);       // only the pair's first sharer may have begun ahead of it
+            const unsigned base_p = S || wp * q + min(wp, rem) >= pair * PU ? 0u : 2u;
+            unsigned wa[2], wb[2];
+#pragma unroll
+            for (unsigned h = 0; h < 2; ++h) {
+                wa[h] = owner((2 * pair + h) * TR4);
+                wb[h] = owner((2 * pair + h) * TR4 + TR4 - 1);
+            }
+            float z[kRowsEach][2][2] = {};
+            for (unsigned x = 0; x <= max(wb[0] - wa[0], wb[1] - wa[1]); x += 4) {
+                float2_t part[kRowsEach][2][4];
+#pragma unroll
+                for (int j = 0; j < kRowsEach; ++j)
+#pragma unroll
+                    for (unsigned h = 0; h < 2; ++h)
+#pragma unroll
+                        for (unsigned i = 0; i < 4; ++i) {
+                            const unsigned xi = min(wa[h] + x + i, wb[h]);
+                            const unsigned long long* const src =
+                                (const unsigned long long*)(slot(xi, (xi == wp ? base_p : 0u) + h) + min(wave + 16 * j, M - 1) * 128) + lane;
+                            part[j][h][i] = __builtin_bit_cast(float2_t, __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                        }
+#pragma unroll
+                for (int j = 0; j < kRowsEach; ++j)
+#pragma unroll
+                    for (unsigned h = 0; h < 2; ++h)
+#pragma unroll
+                        for (unsigned i = 0; i < 4; ++i)
+                            if (wa[h] + x + i <= wb[h]) {
+                                z[j][h][0] += part[j][h][i].x;
+                                z[j][h][1] += part[j][h][i].y;
+                            }
+            }
+#pragma unroll
+            for (int j = 0; j < kRowsEach; ++j)
+                if (wave + 16 * j < M) finish_row(pair, wave + 16 * j, z[j], sc);
+        }
+        return;
+    }
 
     // ---- finish: a wave takes (column block, row) vectors, two columns a lane
     auto store_row = [&](const RowsBlock& b, unsigned cbi, int row, float z0, float z1) {
@@ -469,7 +639,6 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditiona
     const bool last_shared = ncb > 1 && u1 < (cb_last + 1) * TR4;
     int row = wave;
     unsigned cbi = 0;
-    const unsigned qs1 = u0 + (L >> 2), qs2 = u0 + (L * 2 >> 2), qs3 = u0 + (L * 3 >> 2);
     while (true) {
         if constexpr (GROUPED) {
             for (int n; cbi < ncb && row >= (n = __builtin_amdgcn_readfirstlane(table[cbi].rows)); ++cbi) row -= n;
@@ -481,21 +650,10 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditiona
         }
         if (cbi >= ncb) break;
         const unsigned cbx = cb_first + cbi;
-        const unsigned c0 = cbx * TR4, c1 = c0 + TR4;
         const RowsBlock b = block(cbx);
         if (!b.empty) {
             float z0 = 0.0f, z1 = 0.0f;
-            const float* const base = red + (size_t)cbi * M * kRowsStride + row * kRowsStride + 2 * lane;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const unsigned a0 = g == 0 ? u0 : g == 1 ? qs1 : g == 2 ? qs2 : qs3;
-                const unsigned a1 = g == 0 ? qs1 : g == 1 ? qs2 : g == 2 ? qs3 : u1;
-                if (a0 < c1 && a1 > c0) {
-                    const float2_t part = *(const float2_t*)(base + (size_t)g * M * kRowsStride);
-                    z0 += part.x;
-                    z1 += part.y;
-                }
-            }
+            own_sum(cbi, row, z0, z1);
             if ((cbi == 0 && first_shared) || (cbi == ncb - 1 && last_shared)) {
                 unsigned long long* const slot =
                     (unsigned long long*)(p.partials + ((size_t)w * 2 + (cbi == 0 ? 0 : 1)) * M * 128 + row * 128) + lane;
@@ -511,12 +669,6 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_rows_kernel(std::conditiona
 
     // ---- shared column blocks (the first and the last of the range at most): count this
     // workgroup in; the last sharer to arrive adds the parts in k order and finishes the block
-    auto owner = [&](unsigned x) {
-        const unsigned big = rem * (q + 1);
-        if constexpr (GROUPED) return x < big ? x / (q + 1) : rem + (x - big) / q;
-        if (S) return div_exact(x, p.m_tr) * S + (x % TR4 ? S - 1 : 0u);     // asked for a block's first or last unit
-        return x < big ? div_exact(x, p.m_q1) : rem + div_exact(x - big, p.m_q);
-    };
     wait_own_stores();
     __syncthreads();
     if (threadIdx.x < 2) {

@@ -283,12 +283,13 @@ constexpr int kNormRotateMaxCols = 32768;
 // gate and up of an MLP above 8 rows as one bundle: two linears of one shape on one input, each
 // with its own output and its own buffer for the rotated input
 // next, optional: the linear behind silu(c[0]) * c[1].  Where the launch finishes its tiles in a launch of its own
-// that one leaves this activation in c[1] and its rotated rows as LinearArgs::rotated wants them, and sets `done`;
+// that one, and with few rows the launch itself, leaves this activation in c[1] and its rotated rows as LinearArgs::rotated wants them, and sets `done`;
 // the workspace may then serve no other launch in between (scratch: the scope that the caller holds over both).
 struct PairNext {
     const void* suh;
     void* a_had;
     int size_n;
+    int keep_up;                // 1: c[1] keeps up, not the activation (row blocks: 0 only)
     bool done = false;
     const void* operand = nullptr;
 };

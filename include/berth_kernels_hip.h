@@ -269,8 +269,9 @@ typedef struct {
  * one bundle (one launch rotates the input with either linear's scales, the next runs
  * both; the up projection's rotated copy waits in act_had, so this form needs
  * intermediate >= hidden, else gate and up run one after the other), one launch that
- * forms silu(g) * u and rotates it, the down projection.  The row-block kernel
- * (33..511 rows) adds a launch that finishes its shared tiles; behind gate and up that
+ * forms silu(g) * u and rotates it, the down projection.  The few-row kernel (2..32 rows)
+ * forms and rotates silu(g) * u itself where gate and up are wide enough; the row-block kernel
+ * (33..511 rows) adds a launch that finishes its shared tiles, and behind gate and up that
  * launch also forms silu(g) * u and rotates it.
  * lins: HOST array {gate, up, down} of device pointers.  x fp16 [m][hidden];
  * gate_out, up_out fp16 [m][intermediate] (written; above 8 rows up_out ends up
@@ -297,8 +298,8 @@ int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* gate_out, vo
  * differs), and where the down projection takes it the residual is added where it writes its
  * output: two launches when both do.  More rows where gate and up run on the MFMA kernels as one
  * bundle: the norm is formed where the input is rotated and the residual added where the down launch
- * writes (four launches; on the row-block kernel the third finishes gate's and up's tiles too, and a
- * fifth finishes those that down shares).  Anything else runs the same arithmetic as separate launches. */
+ * writes (four launches, three of few rows where gate and up are wide enough; on the row-block kernel
+ * the third finishes gate's and up's tiles too, and a fifth finishes those that down shares).  Anything else runs the same arithmetic as separate launches. */
 typedef struct {
     const void* weight;         /* fp16 or bf16 [hidden] */
     float epsilon, constant_bias, constant_scale;

@@ -210,7 +210,8 @@ def test_every_register_that_inline_assembly_writes_counts(write, regs, waits, c
 
 @pytest.mark.parametrize("kernels,params", [
     (["exl3_gemm_pair_kernel<3, 1>", "exl3_gemm_pair_kernel<4, 0>", "exl3_gemm_kernel<4, 0, 1, false>"], "GemmParams"),
-    (["exl3_gemm_rows_kernel<3, 1, 1, false, true>", "exl3_gemm_rows_kernel<4, 0, 2, false, true>"], "GemmRotateParams")])
+    (["exl3_gemm_rows_kernel<3, 1, 1, false, true>", "exl3_gemm_rows_kernel<4, 0, 2, false, true>"], "GemmRotateParams"),
+    (["exl3_gemm_rows_kernel<3, 1, 1, false, false, true>", "exl3_gemm_rows_kernel<4, 0, 2, false, false, true>"], "RowsPairParams")])
 def test_the_same_of_the_fused_launches(tmp_path, kernels, params):
     test_matrix_instructions_keep_their_distance_from_inline_assembly(tmp_path, kernels, ("exl3_gemm_rows_kernel.cuh",), params)
 

@@ -82,6 +82,37 @@ def test_mlp_of_few_rows_stage_by_stage(rows):
     assert launch.count("exl3_gemm_rows_kernel") == 2 and "silu_mul_had_r_128_kernel" in launch, launch
 
 
+@pytest.mark.parametrize("rows,H,I,bits", [
+    (2, 2048, 16384, 2),        # one column block a workgroup, each pair shared by two
+    (5, 2048, 5632, 4),         # column blocks in two parts
+    (8, 1152, 8448, 3),         # ranges across pairs; up stays in its buffer
+    (9, 1152, 8448, 5),         # the activation in its place
+    (16, 384, 8704, 4),         # pairs shared by four workgroups
+    (17, 640, 17408, 6),        # two rows a wave, the second of one wave only
+    (24, 128, 40960, 4),        # whole pairs inside a workgroup
+    (32, 640, 17408, 1),
+    (12, 256, 5120, 4),         # the down projection reads the row-major copy
+])
+def test_mlp_whose_gate_and_up_leave_the_next_input(rows, H, I, bits):
+    """Gate, up or activation, rotated activation and output, stage by stage; a second call gives the same bits."""
+    from berth_amd.device import Gpu
+    from tests.test_gpu_mlp import _layer, run_mlp_block
+    with knobs(BERTH_GEMM_ROWS_UNITS=192 if I == 5120 else 1):
+        launch = run_mlp_block(rows, H, I, bits)
+    assert ",silu,rotate>" in launch and "silu_mul_had_r_128_kernel" not in launch, launch
+    assert ("exl3_gemm_rows_kernel" in launch.split(" ; ")[1]) == (I != 5120), launch
+    gpu = Gpu(0)
+    _, mlp = _layer(gpu, H, I, bits, 9700 + rows, rows)
+    x = gpu.upload((synth.activations(9800 + rows, rows, H) / np.sqrt(H)).astype(np.float16).view(np.uint16))
+    got = []
+    for _ in range(2):
+        y = torch.zeros((rows, H), dtype=torch.float32, device=DEV)
+        mlp.forward(gpu, x, y, rows=rows)
+        got.append([y] + [getattr(mlp, n).clone() for n in ("g", "u", "act_had")])
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("rows,H,I,bits", [(2, 128, 256, 4),        # one block a row: a quarter of a wave
                                            (9, 1152, 1280, 3),      # a workgroup with a half-empty wave
                                            (33, 8320, 8320, 2),     # two chunks a thread, one row block with one row past its first 32
