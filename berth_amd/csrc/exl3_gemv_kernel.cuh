@@ -296,14 +296,16 @@ __global__ __launch_bounds__(256, 4) void exl3_gemv_kernel(GemvParams p)
         // One wave works the routing out and the others take its answer: a quarter of the reads
         // of the segment sums, which every workgroup of the launch wants at the same moment
         // (measured: 1.2 us off the layer against all four waves doing it side by side).
-        __shared__ int s_expert;
+        // The records of this launch's linear of all experts (at most 128: lane l holds experts l and l + 64) are asked
+        // for behind the segment sums, so that the weights are one dependent read away from the answer.
+        __shared__ __align__(8) unsigned s_lin[6];
         if (wave == 0) {
             // The first workgroup's first wave stores the routing results.  It also leaves, for
             // the launch that follows, the record of linear `resolved_lin` of the expert at
             // each sorted position (then of the always-on expert), so that that launch reaches
             // its weights with one dependent read instead of two.  It asks for the records of
-            // all experts (at most 128: lane l holds experts l and l + 64) ahead of the
-            // routing, so that its stores do not wait for a read that depends on the routing.
+            // all experts ahead of the
+            // routing too, so that its stores do not wait for a read that depends on the routing.
             const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
             const bool resolve = writer && p.resolved_out;
             unsigned rec[2][6];
@@ -316,9 +318,28 @@ __global__ __launch_bounds__(256, 4) void exl3_gemv_kernel(GemvParams p)
                     for (int q = 0; q < 6; ++q) rec[i][q] = src[q];
                 }
             }
-            const RouteOneToken r = route_one_token(p.route, lane, writer);
+            unsigned mine[2][6];
+            const RouteOneToken r = route_one_token(p.route, lane, writer, [&]() {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (i == 1 && p.route.E <= 64) break;
+                    const int e2 = min(lane + 64 * i, p.route.E - 1);
+                    const global_ptr<const unsigned> src = as_global((const unsigned*)(p.experts + e2 * p.lins_per_expert + p.lin_base + which));
+#pragma unroll
+                    for (int q = 0; q < 6; ++q) mine[i][q] = src[q];
+                }
+            });
             const int e = route_expert_at(p.route, r, lane, prob);
-            if (lane == 0) s_expert = e;
+            if (e == p.shared_expert) {
+                if (lane == 0) *(ExpertLin*)s_lin = p.shared[p.lin_base + which];
+            } else {
+#pragma unroll
+                for (int q = 0; q < 6; ++q) {
+                    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)mine[0][q], e & 63);
+                    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)mine[1][q], e & 63);
+                    s_lin[q] = e >= 64 ? hi : lo;
+                }
+            }
             if (resolve) {
                 unsigned got[6];
 #pragma unroll
@@ -336,8 +357,11 @@ __global__ __launch_bounds__(256, 4) void exl3_gemv_kernel(GemvParams p)
             }
         }
         __syncthreads();
-        const int expert = __builtin_amdgcn_readfirstlane(s_expert);
-        lin = expert_lin(expert);
+        unsigned rec[6];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) rec[q] = (unsigned)__builtin_amdgcn_readfirstlane((int)s_lin[q]);
+        static_assert(sizeof(ExpertLin) == 24, "three pointers");
+        __builtin_memcpy(&lin, rec, sizeof(lin));
         row0 = prob;
         rows = 1;
     } else if (p.resolved) {

@@ -226,38 +226,54 @@ __device__ __forceinline__ void route_sort_one_token(const PermuteParams& q, int
 // order, bias), top-k, and the sorted position of every selected expert (lane j < k: expert of
 // slot j and its sorted position).  Every wave that calls this gets the same bits; the wave
 // with `writer` set also stores the routing results (logits, idx, w, and what the sort of the
-// one token writes).
+// one token writes).  `requested` is called when the reads are on their way.
 struct RouteOneToken {
     int sel;
     int rank;
 };
 
-__device__ __forceinline__ RouteOneToken route_one_token(const RouteParams& p, int lane, bool writer)
+template <typename F>
+__device__ __forceinline__ RouteOneToken route_one_token(const RouteParams& p, int lane, bool writer, F requested)
 {
     float lg[kRoutePer];
 #pragma unroll
     for (int i = 0; i < kRoutePer; ++i) lg[i] = -INFINITY;
+    // Both of a lane's experts and their biases at once, 32 segments at a time (segments past the end re-read the last
+    // one, experts past the end the last one, and are ignored); the adds stay in segment order.  One after the other,
+    // the biases last, they were up to four round trips to memory instead of one.
+    const uint32_t at[2] = {(uint32_t)min(lane, p.E - 1), (uint32_t)min(lane + 64, p.E - 1)};
+    float v[2] = {0.0f, 0.0f}, bias[2] = {0.0f, 0.0f};
+    for (int s0 = 0; s0 < p.nseg; s0 += 32) {
+        float part[2][32];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (i == 1 && p.E <= 64) break;
+#pragma unroll
+            for (int j = 0; j < 32; ++j) part[i][j] = as_global(p.parts + (size_t)min(s0 + j, p.nseg - 1) * p.E)[at[i]];
+        }
+        if (s0 == 0) {
+            if (p.bias) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) bias[i] = as_global(p.bias)[at[i]];
+            }
+            requested();
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (i == 1 && p.E <= 64) break;
+#pragma unroll
+            for (int j = 0; j < 32; ++j) {
+                const float nv = v[i] + part[i][j];
+                v[i] = s0 + j < p.nseg ? nv : v[i];
+            }
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int e = lane + 64 * i;
         if (e < p.E) {
-            const float* src = p.parts + e;
-            float v = 0.0f;
-            // 32 loads in flight at a time (indices past the end re-read the last segment and
-            // are ignored); the adds stay in segment order
-            for (int s0 = 0; s0 < p.nseg; s0 += 32) {
-                float part[32];
-#pragma unroll
-                for (int j = 0; j < 32; ++j) part[j] = src[(size_t)min(s0 + j, p.nseg - 1) * p.E];
-#pragma unroll
-                for (int j = 0; j < 32; ++j) {
-                    const float nv = v + part[j];
-                    v = s0 + j < p.nseg ? nv : v;
-                }
-            }
-            if (p.bias) v += p.bias[e];
-            if (writer && p.logits) p.logits[e] = v;
-            lg[i] = v;
+            lg[i] = p.bias ? v[i] + bias[i] : v[i];
+            if (writer && p.logits) p.logits[e] = lg[i];
         }
     }
     RouteOneToken r;

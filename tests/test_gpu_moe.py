@@ -158,6 +158,29 @@ def _check_stages(layer, x, experts_np, shared_np, idx, w, out, T, H, E, k, I, b
     assert np.allclose(out, acc, rtol=1e-5, atol=1e-5 * max(1.0, float(np.abs(acc).max())))
 
 
+@pytest.mark.parametrize("H,E,shared_I,biased", [(128, 2, 0, True), (256, 64, 128, False), (256, 66, 0, True), (2176, 100, 128, True),
+                                                 (2304, 128, 0, False)])
+def test_one_token_and_the_experts_of_either_half(H, E, shared_I, biased):
+    """The one-token gate / up launch, whose routing wave holds experts l and l + 64 a lane: their sums over up to 32 segments and
+    more, biases, and the records of the chosen ones and of the always-on one."""
+    gpu = Gpu(0)
+    k, I, bits = min(E, 8), 128, 4
+    wr, experts_np, experts, shared_np, shared = _make_layer(gpu, 700 + E, H, E, I, bits, shared_I, 4.0)
+    bias = synth.zipf_bias(9, E) if biased else None
+    layer = MoeLayer(gpu, wr, experts, k, shared=shared, bias=bias)
+    for seed in range(3):
+        x = (synth.activations(950 + seed, 1, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
+        out = torch.zeros((1, H), dtype=torch.float32, device=DEV)
+        idx = torch.zeros((1, k), dtype=torch.int32, device=DEV)
+        w = torch.zeros((1, k), dtype=torch.float32, device=DEV)
+        layer.forward(gpu, dev(x.view(np.uint16)), out, 1, idx, w)
+        torch.cuda.synchronize()
+        _, oi, ow = O.moe_layer(x, wr, experts_np, k, I, bits, 2, bias=bias, shared=shared_np, shared_I=shared_I)
+        assert np.array_equal(idx.cpu().numpy(), oi), K.moe.last_launch()
+        assert np.allclose(w.cpu().numpy(), ow, rtol=1e-5, atol=1e-7)
+        _check_stages(layer, x, experts_np, shared_np, oi, w.cpu().numpy(), out.cpu().numpy(), 1, H, E, k, I, bits, shared_I)
+
+
 @pytest.mark.parametrize("T,H,E,k,I,bits,shared_I,scale", [
     (1, 256, 8, 2, 128, 4, 0, 1.0),
     (1, 256, 8, 2, 128, 4, 128, 1.0),       # one token, shared expert inside the grouped launches
