@@ -552,8 +552,7 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
 // w and w + 16 of every 32; their weights are requested at once, ahead of the token rows, which go
 // through LDS (lanes that read sixteen rows from memory cost an address cycle each).  Step i of a segment
 // multiplies its rows 4 i .. 4 i + 3: lane 16 q + j holds row 4 i + q, of token j and of expert j, or of
-// experts 2 j and 2 j + 1 with a tile each for the even and the odd ones.  (More than one slab: the launch
-// takes more than 128 experts.)
+// experts 2 j and 2 j + 1 with a tile each for the even and the odd ones.
 constexpr int kTileTokens = 16, kTileSegs = 32;
 constexpr int kTileXStride = kTileSegs * kRouteSeg + 8;             // halves; sixteen rows' same columns in different banks
 inline __host__ __device__ constexpr int route_tile_lds_bytes(int experts)
@@ -644,6 +643,18 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
     }
     if (p.bias) v += bias;
     if (mine && p.logits) p.logits[(size_t)(t0 + tt) * p.E + e0 + c] = v;
+    float lg[kRoutePer];
+    if (nslab == 1) {
+        __syncthreads();                                            // every sum is formed: the segment sums can go
+        if (mine) s_parts[threadIdx.x] = v;
+        __syncthreads();
+        if (t0 + wave >= p.T) return;
+#pragma unroll
+        for (int i = 0; i < kRoutePer; ++i) lg[i] = -INFINITY;
+        if (lane < p.E) lg[0] = s_parts[wave * EXPERTS + lane];
+        route_topk_n<2>(lg, lane, p, t0 + wave);
+        return;
+    }
 
     // ---- logits to memory ([T][E], the head of the segment-sum scratch); the last slab of the token
     // group to arrive selects, a wave per token
@@ -663,7 +674,6 @@ __global__ __launch_bounds__(1024) void moe_route_slab_kernel(RouteParams p)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     const int t = t0 + wave;
     if (t >= p.T) return;
-    float lg[kRoutePer];
 #pragma unroll
     for (int i = 0; i < kRoutePer; ++i) {
         const int e = lane + 64 * i;
@@ -1209,27 +1219,33 @@ std::string run_route(const void* x, const void* wr, const float* bias, int32_t*
             const long cost = ((long)nslab * groups_c + ws.cu_count - 1) / ws.cu_count * (4 + c);
             if (best < 0 || cost < best) { best = cost; tt = c; }
         }
-        // More than 128 experts and passes of 32 segments that are nearly full: tiles of sixteen tokens, with
-        // slabs of 16 experts where that is one round of the chip, where they are the quicker form.  The cost above is
-        // about half of the us beyond the first five, also here: 5 for a round of 16 experts and one more per sixteen slabs
-        // that hand over to one workgroup, 2 and 5 per round of 32.  Up to eight tokens the slabs of 128 are too few
+        // Passes of 32 segments that are nearly full: tiles of sixteen tokens, with slabs of 16 experts where that is one
+        // round of the chip, where they are the quicker form.  Up to eight tokens the slabs of 128 are too few
         // to pull the router weight in from memory.  us, slabs of 128 -> tiles, H = 2048, each call a weight of its own:
         //   512 experts at 2 / 8 / 16 / 64 / 128 tokens  18.6 17.3 16.6 15.9 16.9 -> 15.3 16.4 18.4 17.7 17.4,
         //               at 256 / 384 / 512 / 1500        19.4 25.6 33.0 81.8 -> 19.5 28.6 29.5 66.4
         //   256 experts at 8 / 64 / 256 / 384 / 1500     15.9 14.7 15.8 18.6 43.9 -> 15.1 16.1 15.9 17.7 37.2
         //   160 experts at 8 / 64 / 256 / 384 / 1500     16.2 14.7 15.6 18.1 44.7 -> 13.9 14.8 14.5 14.6 27.0
-        // (H = 1920, 30 segments, and H = 4096 the same way round).  With the weight in the caches, sparser passes: H = 1024, 512
-        // experts at 64 / 1500 tokens 11.5 / 48.9 -> 16.2 / 59.9; H = 2112 at 1500 101 -> 104.  Up to 128 experts need no
-        // hand-over without tiles: H = 2048 at 64 / 1500 tokens 10.6 / 22.4 -> 12.0 / 23.5 (but H = 4096 at 1500 50 -> 39).
+        // There the cost above is about half of the us beyond the first five, also for tiles: 5 for a round of 16 experts and
+        // one more per sixteen slabs that hand over to one workgroup, 2 and 5 per round of 32.
+        //   128 experts at 64 / 500 / 800 / 1000 / 1500  10.5 13.1 16.4 16.6 21.8 -> 12.4 12.0 14.4 14.7 23.5
+        //   64 experts at 128 / 300 / 700 / 1500         9.9 12.6 15.5 21.7 -> 11.4 12.5 12.1 14.4
+        //   32 experts at 600 / 1500                     15.1 21.4 -> 11.3 11.6
+        // Up to 128 experts slabs hand over to nobody: 2.2 us per unit of the cost, a round of tiles of 16 experts 12.6 (with
+        // what they differ by), rounds of 32 4.8 and 9.4 each.
+        // (H = 1920, 30 segments, and H = 4096 the same way round.)  With the weight in the caches, sparser passes: H = 1024, 512
+        // experts at 64 / 1500 tokens 11.5 / 48.9 -> 16.2 / 59.9, 128 at 1500 14.1 -> 22.3; H = 2112 at 1500 101 -> 104.
         // BERTH_MOE_ROUTE_SLAB=2: tiles wherever they can serve.
         const long tile_groups = (T + kTileTokens - 1) / kTileTokens;
         const int tile_experts = tile_groups * ((E + 15) / 16) <= ws.cu_count ? 16 : 32;
         const long tile_slabs = (E + tile_experts - 1) / tile_experts;
-        const long tile_cost = tile_experts == 16 ? 5 + tile_slabs / 16
-                                                  : 2 + 5 * ((tile_groups * tile_slabs + ws.cu_count - 1) / ws.cu_count);
+        const long tile_rounds = (tile_groups * tile_slabs + ws.cu_count - 1) / ws.cu_count;
+        const bool few = E <= kSlabExperts;
+        const bool tile_cheaper = few ? (tile_experts == 16 ? 126 : 48 + 94 * tile_rounds) <= 22 * best - 5
+                                      : (tile_experts == 16 ? 5 + tile_slabs / 16 : 2 + 5 * tile_rounds) <= best;
         const int tile_segs = (p.nseg + kTileSegs - 1) / kTileSegs * kTileSegs;
-        const bool tiles_serve = T > 1 && E > kSlabExperts && (uintptr_t)x % 16 == 0 && tile_groups * kRouteCounterStride <= kCounters;
-        const bool tiles_quicker = tile_segs * 8 <= p.nseg * 9 && (T <= kTileTokens / 2 || best < 0 || tile_cost <= best);
+        const bool tiles_serve = T > 1 && (uintptr_t)x % 16 == 0 && tile_groups * kRouteCounterStride <= kCounters;
+        const bool tiles_quicker = tile_segs * 8 <= p.nseg * 9 && (best < 0 || tile_cheaper || (!few && T <= kTileTokens / 2));
         if (tiles_serve && (tiles_quicker || knobs().moe_route_slab == 2)) {
             const dim3 grid((unsigned)tile_groups, (unsigned)tile_slabs);
             const int lds = route_tile_lds_bytes(tile_experts);

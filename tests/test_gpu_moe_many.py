@@ -201,6 +201,27 @@ def test_routing_tiles_of_sixteen_tokens(T, H, E, k, experts):
     assert np.allclose(w, ow, rtol=1e-5, atol=1e-7)
 
 
+@pytest.mark.parametrize("T,H,E,k,tiles", [
+    (17, 2048, 2, 2, False), (256, 2048, 128, 8, False), (257, 2048, 128, 8, True), (512, 2048, 100, 4, True), (600, 1920, 34, 6, True),
+    (1000, 2048, 128, 8, True), (1025, 2048, 128, 8, False), (1500, 2048, 64, 6, True), (1090, 4096, 16, 4, True), (1037, 2048, 62, 9, True),
+    (700, 1024, 64, 4, False)])
+def test_routing_tiles_of_up_to_128_experts(T, H, E, k, tiles):
+    """One slab, several, ragged ones, on either side of the rule's lines: the oracle's bits, from tiles and from slabs of 128."""
+    x, wr = synth.activations(T, T, H), synth.router_weight(E, H, E)
+    bias = synth.zipf_bias(6, E) if E % 4 == 0 else None
+    idx, w, logits = _route(x, wr, k, bias=bias)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert ("moe_route_slab_kernel<16," in K.moe.last_launch()) == tiles, K.moe.last_launch()
+    with knobs(BERTH_MOE_ROUTE_SLAB=2):
+        again = _route(x, wr, k, bias=bias)
+    assert "moe_route_slab_kernel<16," in K.moe.last_launch(), K.moe.last_launch()
+    assert all(np.array_equal(a, b) for a, b in zip((idx, w, logits), again))
+    oi, ow, ol = O.moe_route(x, wr, k, bias=bias, want_logits=True)
+    assert np.array_equal(logits.view(np.uint32), ol.view(np.uint32))
+    assert np.array_equal(idx, oi)
+    assert np.allclose(w, ow, rtol=1e-5, atol=1e-7)
+
+
 @pytest.mark.parametrize("T,H,E,tokens", [
     (8, 2048, 512, 16), (9, 2048, 512, 1), (64, 2048, 512, 1), (128, 2048, 512, 2), (256, 2048, 512, 16), (384, 2048, 512, 6),
     (512, 2048, 512, 16), (128, 2048, 256, 1), (129, 2048, 256, 16), (500, 1856, 160, 16), (500, 1792, 160, 4), (500, 2112, 160, 4)])
