@@ -258,7 +258,7 @@ extern "C" int berth_exl3_linear(const void* a, const void* trellis, void* c, co
 // The array has no initialiser, so it is zero when the code object is loaded, and every launch
 // leaves the counters and accumulators it used at zero again: nothing has to clear it, and a
 // first call inside a stream capture records only the linear's own launches (one kernel; two for
-// 2..8 rows of a weight large enough for the few-row MFMA kernel where that one does not rotate its input
+// 2..8 rows of a weight that takes the few-row MFMA kernel where that one does not rotate its input
 // itself: a launch ahead of it then leaves the rotated rows in the partial sums' scratch too).
 namespace {
 constexpr size_t kNoAllocPartialBytes = (size_t)8 << 20;
@@ -576,9 +576,9 @@ extern "C" const char* berth_prefill_last_launch(void) { return g_prefill_launch
 // Whether gate and up of an MLP run on the MFMA kernels as one bundle: one launch rotates the input
 // with either linear's scales (the up projection's copy waits in act_had, which the down projection
 // fills only afterwards), one dense launch runs both.
-static bool mlp_pair_on_matrix_units(int size_m, int hidden, int intermediate)
+static bool mlp_pair_on_matrix_units(int size_m, int hidden, int intermediate, RowsInput input)
 {
-    return intermediate >= hidden && size_m > 1 && (size_m > 8 || gemv_rows_on_matrix_units(2, size_m, hidden, intermediate));
+    return intermediate >= hidden && size_m > 1 && (size_m > 8 || gemv_rows_on_matrix_units(2, size_m, hidden, intermediate, input));
 }
 
 // gate and up where they are no bundle on the MFMA kernels, or one of few rows whose down projection takes the VALU kernel
@@ -605,8 +605,9 @@ static std::string mlp_linears(const PairArgs& pair, LinearArgs down, const floa
     down.a_up = pair.c[1];
     down.act_out = few ? nullptr : pair.c[1];
     down.out_add = out_add;
-    const bool on_matrix_units = mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n);
-    if (!on_matrix_units || (few && !gemv_rows_on_matrix_units(1, down.size_m, down.size_k, down.size_n))) {
+    const RowsInput input = pair.norm ? RowsInput::kNorm : RowsInput::kMlp;
+    const bool on_matrix_units = mlp_pair_on_matrix_units(pair.size_m, pair.size_k, pair.size_n, input);
+    if (!on_matrix_units || (few && !gemv_rows_on_matrix_units(1, down.size_m, down.size_k, down.size_n, input))) {
         const std::string desc = mlp_gate_up(pair, act_had, on_matrix_units) + " ; ";
         return desc + (few ? launch_gemv(down) : launch_gemm(down));
     }
@@ -690,10 +691,17 @@ extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* r
         // (the fused forms read and write 16 bytes at a time)
         const bool aligned = (((uintptr_t)x | (uintptr_t)residual | (uintptr_t)residual_out | (uintptr_t)norm->weight) & 15) == 0;
         const bool fuse_norm = size_m == 1 ? gemv_stream_applies(2, hidden, intermediate, false)
-                                           : aligned && mlp_pair_on_matrix_units(size_m, hidden, intermediate) &&
-                                                 hidden <= kNormRotateMaxCols;
+                                           : aligned && hidden <= kNormRotateMaxCols &&
+                                                 mlp_pair_on_matrix_units(size_m, hidden, intermediate, RowsInput::kNorm);
+        // (as mlp_linears asks for the down projection)
+        const auto down_on_matrix_units = [&] {
+            const RowsInput input = fuse_norm ? RowsInput::kNorm
+                                    : mlp_pair_on_matrix_units(size_m, hidden, intermediate, RowsInput::kMlp) ? RowsInput::kMlp
+                                                                                                             : RowsInput::kLaunch;
+            return gemv_rows_on_matrix_units(1, size_m, intermediate, hidden, input);
+        };
         const bool fuse_add = size_m == 1 ? gemv_stream_applies(1, intermediate, hidden, false)
-                                          : aligned && (size_m > 8 || gemv_rows_on_matrix_units(1, size_m, intermediate, hidden));
+                                          : aligned && (size_m > 8 || down_on_matrix_units());
         std::string desc;
         if (fuse_norm) {
             pair.a = nullptr;
@@ -925,7 +933,7 @@ extern "C" uint64_t berth_ops_mgemm_tune_key(int size_m, int size_k, int size_n,
 // Which of the reference's two QTIP GEMV configurations (0 narrow, 1 wide, -1 neither) its
 // rows-2..8 route would take (crates/berth-kernels/csrc/prefill_lin/gemv.cu:71-99: host
 // integer arithmetic; cc 2 = Ampere, 3 = Ada there).  On this device rows 2..8 take the few-row
-// MFMA kernel or the VALU kernel by the weight's size (rows_min_units) and nothing consumes the
+// MFMA kernel or the VALU kernel by the weight's size (gemm_rows_applies) and nothing consumes the
 // answer; the table is kept so that the crate links and its table test reads the same.
 extern "C" int berth_exl3_gemv_cfg(int cc, int size_m, int size_k, int size_n, int k_bits, int cb, int mode,
                                    int narrow_coresident)

@@ -72,18 +72,15 @@ struct RowsPlan {
 
 static unsigned magic(unsigned d) { return d == 1 ? 0u : (unsigned)((1ull << 32) / d) + 1u; }
 
-// Fewest units for which the few-row kernel is taken.  Up to 8 rows the alternative is the VALU
-// kernel of exl3_gemv.hip, which rotates the input itself (one launch instead of two) and pays half
-// an instruction per weight and row: 4096 x 2048 (1024 units) takes 9.8 / 13.4 / 16.8 us at 2 / 5
-// / 8 rows there and 10.3 / 10.9 / 11.3 here, 4096 x 8192 (4096 units) 13.4 against 12.8 at two.
-// Above 8 rows it is the 32-row MFMA kernel, whose hand-over and half-empty rounds cost more from
-// the start (2048 x 1024, 256 units: 14.1 -> 10.6 us at 12 rows, 16.0 -> 13.9 at 32).
-// BERTH_GEMM_ROWS_UNITS replaces the rule (0: never).
+// Fewest units for which a launch can take the few-row kernel.  Above 8 rows the alternative is the 32-row MFMA
+// kernel, whose hand-over and half-empty rounds cost more from the start (2048 x 1024, 256 units: 14.1 -> 10.6 us at
+// 12 rows, 16.0 -> 13.9 at 32).  Up to 8 rows it is the VALU kernel of exl3_gemv.hip, and gemm_rows_applies chooses.
+// BERTH_GEMM_ROWS_UNITS replaces both rules (0: never).
 static int rows_min_units(int size_m)
 {
     const int forced = knobs().gemm_rows_units;
     if (forced >= 0) return forced;
-    return size_m <= 3 ? 3072 : size_m <= 8 ? 1024 : 192;
+    return size_m <= 8 ? 32 : 192;
 }
 
 static RowsPlan plan_rows(const Workspace& ws, int slices, int slabs, int size_m, int size_k, int size_n)
@@ -144,9 +141,40 @@ static RowsPlan plan_rows(const Workspace& ws, int slices, int slabs, int size_m
     return pl;
 }
 
-bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, int size_n)
+// Up to 8 rows the VALU kernel of exl3_gemv.hip rotates the input itself, cuts size_k into parts of two k-blocks at
+// the least (four waves have a k-block of 512 each), and pays half an instruction per weight and row: 4 bits, K x N,
+// us, VALU -> here.
+bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, int size_n, RowsInput input)
 {
-    return plan_rows(ws, slices, slices, size_m, size_k, size_n).ok;
+    const RowsPlan pl = plan_rows(ws, slices, slices, size_m, size_k, size_n);
+    if (!pl.ok || size_m > 8 || knobs().gemm_rows_units >= 0) return pl.ok;
+    // large weights, whichever launches stand ahead (4096x8192, 4096 units, at two rows 13.4 -> 12.8; 4096x2048 with a
+    // rotation launch at 2 / 5 / 8 rows 9.8 / 13.4 / 16.8 -> 10.3 / 10.9 / 11.3)
+    if (pl.units >= (size_m <= 3 ? 3072 : 1024)) return true;
+    if (size_k < 512) return false;         // (256x512 at 2 / 4 / 8 rows 7.2 / 8.5 / 12.6 -> 8.2 / 10.4 / 10.4)
+    switch (input) {
+    case RowsInput::kSelf:
+        // The launch rotates its input itself: one launch either way.  1024x1024 at 2 / 3 / 5 / 8 rows 9.2 / 9.6 / 11.4 /
+        // 14.3 -> 8.4 / 8.3 / 8.5 / 8.5, 3072x2048 9.7 / 10.8 / 12.9 / 16.1 -> 8.8 / 9.0 / 9.2 / 9.7; four k-blocks, which
+        // the VALU kernel takes in one part without partial sums, 512x2048 at 2 / 3 / 4 / 8 rows 7.3 / 8.1 / 8.9 / 12.8 ->
+        // 7.8 / 8.2 / 8.5 / 8.5.
+        if (pl.rotate) return size_m >= (size_k < 768 ? 4 : 2);
+        break;
+    case RowsInput::kNorm:
+        // The launch that forms the norm rotates, gate and up leave down's input, the residual is added where down writes:
+        // three launches beside five.  Blocks of 512x1024 at 2 / 4 / 8 rows 23.4 / 26.6 / 36.4 -> 20.4 / 20.7 / 20.9,
+        // 1024x2048 25.1 / 28.6 / 38.5 -> 23.7 / 24.3 / 24.9, 2048x6144 at two 28.7 -> 25.2, 4096x4096 28.2 -> 28.0.
+        return true;
+    case RowsInput::kMlp:
+        // Three launches beside two: 512x1024 at 4 / 5 / 8 rows 20.2 / 22.5 / 30.4 -> 19.3 / 19.8 / 19.6, 1024x2048 at
+        // 2 / 3 / 4 / 5 rows 18.6 / 20.4 / 22.3 / 24.7 -> 22.7 / 22.6 / 22.8 / 22.9.
+        return size_m >= 5;
+    case RowsInput::kLaunch:
+        break;
+    }
+    // Two launches beside one: q / k / v of 1024 x (2048, 256, 256) at 4 / 5 / 8 rows 10.8 / 12.0 / 15.5 -> 11.9 / 11.8 /
+    // 11.8, of 512 x (512, 128, 128) at five 10.6 -> 11.9.
+    return size_m >= 5 && size_k >= 1024;
 }
 
 // rotate: p is a GemmRotateParams; pair: a RowsPairParams
@@ -467,7 +495,7 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     return d0 + desc + (a.out_fp32 ? " out=f32" : " out=f16");
 }
 
-// berth_ops_mgemm with more than 8 rows, or 2..8 of large weights: the bundle's linears on the MFMA kernels
+// berth_ops_mgemm with more than 8 rows, or 2..8 where gemm_rows_applies says so: the bundle's linears on the MFMA kernels
 // behind one launch that rotates every distinct input (slab s of a_had = Hh(input(s) * suh[s])).
 std::string launch_gemm_bundle(const MgemmArgs& m)
 {

@@ -202,13 +202,13 @@ static void pick_units(const Workspace& ws, GemvParams& p, long units, int mmax)
     p.S = pick_split(ws, units, p.KB, mmax);
 }
 
-// Two to eight rows of a weight large enough for the few-row MFMA kernel go there: it decodes as
+// Two to eight rows go to the few-row MFMA kernel where gemm_rows_applies finds it the quicker one: it decodes as
 // fast as the one-row kernel and its dot products cost nothing beside that, where the kernel of
 // this file pays half an instruction per weight and row.  A launch width chosen by hand
 // (BERTH_GEMV_WG_PER_CU) keeps the kernel that it tunes.
-static bool rows_on_matrix_units(const Workspace& ws, int problems, int size_m, int size_k, int size_n)
+static bool rows_on_matrix_units(const Workspace& ws, int problems, int size_m, int size_k, int size_n, RowsInput input)
 {
-    return size_m > 1 && knobs().gemv_wg_per_cu <= 0 && gemm_rows_applies(ws, problems, size_m, size_k, size_n);
+    return size_m > 1 && knobs().gemv_wg_per_cu <= 0 && gemm_rows_applies(ws, problems, size_m, size_k, size_n, input);
 }
 
 std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
@@ -220,7 +220,7 @@ std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
     const int mmax = a.size_m == 1 ? 1 : 8;
-    if (rows_on_matrix_units(ws, 1, a.size_m, a.size_k, a.size_n)) {
+    if (rows_on_matrix_units(ws, 1, a.size_m, a.size_k, a.size_n, a.a_up ? RowsInput::kLaunch : RowsInput::kSelf)) {
         scope.reset();          // the MFMA launcher holds its own
         return launch_gemm(a, scratch);
     }
@@ -272,9 +272,9 @@ std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
            std::to_string(p.S) + (p.half_units ? "/half" : "") + (a.out_fp32 ? " out=f32" : " out=f16");
 }
 
-bool gemv_rows_on_matrix_units(int problems, int size_m, int size_k, int size_n)
+bool gemv_rows_on_matrix_units(int problems, int size_m, int size_k, int size_n, RowsInput input)
 {
-    return rows_on_matrix_units(workspace_for_current_device(), problems, size_m, size_k, size_n);
+    return rows_on_matrix_units(workspace_for_current_device(), problems, size_m, size_k, size_n, input);
 }
 
 std::string launch_gemv_pair(const PairArgs& a)
@@ -347,7 +347,9 @@ std::string launch_mgemm(const MgemmArgs& m)
 {
     if (m.size_k % 128 != 0) throw std::runtime_error("exl3_mgemm: size_k must be a multiple of 128");
     if (m.size_m > 8) return launch_gemm_bundle(m);
-    if (!m.host_lists && rows_on_matrix_units(workspace_for_current_device(), m.bszm_out, m.size_m, m.size_k, m.size_n))
+    // (slices by lists in device memory get a rotation launch)
+    if (!m.host_lists && rows_on_matrix_units(workspace_for_current_device(), m.bszm_out, m.size_m, m.size_k, m.size_n,
+                                              m.had_src_list ? RowsInput::kLaunch : RowsInput::kSelf))
         return launch_gemm_bundle(m);
     LaunchScope scope(m.stream);
     Workspace& ws = scope.ws;

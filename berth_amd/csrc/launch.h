@@ -175,8 +175,11 @@ std::string launch_gemv_pair(const PairArgs& args);
 // with whole_rows, whether every workgroup of it then holds the whole input row)
 bool gemv_stream_applies(int problems, int size_k, int size_n, bool whole_rows);
 
+// What stands ahead of a launch of few rows: the launch rotates its input itself, a launch does so for it, gate and up
+// of an MLP whose down projection takes the kernel too, or the launch that forms an MLP block's norm.
+enum class RowsInput { kSelf, kLaunch, kMlp, kNorm };
 // whether 2..8 rows of `problems` linears of this shape run on the few-row MFMA kernel
-bool gemv_rows_on_matrix_units(int problems, int size_m, int size_k, int size_n);
+bool gemv_rows_on_matrix_units(int problems, int size_m, int size_k, int size_n, RowsInput input);
 
 // grouped (MoE) launches: problems, experts and num_problems are device memory
 struct GroupedArgs {
@@ -303,7 +306,7 @@ std::string launch_gemv(const LinearArgs& args, const Workspace* scratch = nullp
 // any row count, fp16 MFMA kernels: few rows, row blocks, or tiles of 32, 128 or 256 rows.
 std::string launch_gemm(const LinearArgs& args, const Workspace* scratch = nullptr);
 // whether a launch of this many linears of one shape takes the few-row kernel (2..32 rows)
-bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, int size_n);
+bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, int size_n, RowsInput input);
 // trellis -> fp16 [K][slice_n] (row stride slice_n), columns n_offset.. of a
 // [K][full_n] weight
 std::string launch_reconstruct(void* unpacked, const void* packed, int size_k, int slice_n,

@@ -251,8 +251,9 @@ class Exl3MultiLinear:
     `exl3_mgemm` (the qkv bundles of crates/berth-engine/src/attn.rs:1934-1973 and
     gdn.rs:1102-1130; list layout from crates/berth-kernels/src/ops.rs:264-293):
     every source is cut into slices of the greatest common width.  Any row count: one
-    row runs the streaming kernel, 2..8 of small weights the dot-product kernel, the rest the MFMA kernels
-    (the reference sends 9..32 rows through the same call, prefill.rs:81-85)."""
+    row runs the streaming kernel, 2..8 of small weights the dot-product kernel (2..4
+    from a size_k of 1024 on), the rest the MFMA kernels (the reference sends 9..32 rows through the
+    same call, prefill.rs:81-85)."""
 
     def __init__(self, gpu: Gpu, sources: list[Exl3Linear]):
         import math

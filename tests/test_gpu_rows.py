@@ -301,3 +301,65 @@ def test_rotated_rows_of_a_source_without_slices(rows):
         want, want_had = O.linear(x, *s["np"], Kk, widths[i], bits, 2, out_fp32=False)
         assert np.array_equal(host_u16(a_had)[i].reshape(-1), want_had.view(np.uint16).reshape(-1)), i
         assert i == 1 or close(host_f16(outs[i]), want)[0] == 0, i
+
+
+def _bundle(rows, Kk, widths, bits):
+    """Sources of different widths, lists in device memory."""
+    from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
+    gpu = Gpu(0)
+    lins = [synth.linear(640 + i, Kk, n, bits) for i, n in enumerate(widths)]
+    bundle = Exl3MultiLinear(gpu, [Exl3Linear(gpu, f"l{i}", *lin) for i, lin in enumerate(lins)])
+    x = synth.activations(650 + rows, rows, Kk)
+    outs = [torch.full((rows, n), 5.0, dtype=torch.float16, device=DEV) for n in widths]
+    bundle.forward(gpu, gpu.upload(x.view(np.uint16)), outs, OutDtype.F16, rows, by_value=False)
+    torch.cuda.synchronize()
+    for out, lin, n in zip(outs, lins, widths):
+        assert close(host_f16(out), O.linear(x, *lin, Kk, n, bits, 2, out_fp32=False)[0])[0] == 0, K.ops.last_launch()
+
+
+@pytest.mark.parametrize("kind,rows,Kk,N,bits,cb,matrix", [
+    ("linear", 2, 768, 768, 4, 2, True),        # six k-blocks
+    ("linear", 2, 512, 1024, 4, 2, False),
+    ("linear", 4, 512, 512, 3, 1, True),        # 32 units, four k-blocks
+    ("linear", 8, 512, 384, 4, 2, False),       # 24
+    ("linear", 8, 384, 4096, 2, 0, False),      # three k-blocks
+    ("linear", 3, 3072, 256, 5, 0, True),
+    ("bundle", 4, 1024, 512, 4, 2, False), ("bundle", 5, 1024, 512, 4, 2, True), ("bundle", 8, 896, 512, 4, 2, False),
+    ("mlp", 4, 512, 640, 4, 2, False), ("mlp", 5, 512, 640, 4, 2, True),
+])
+def test_small_weights_beside_the_dot_product_kernel(kind, rows, Kk, N, bits, cb, matrix):
+    """Which kernel two to eight rows of small weights take, on both sides of every line, and its results."""
+    with knobs(BERTH_GEMM_ROWS_UNITS=-1):
+        if kind == "linear":
+            got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, bits, cb, True, 70 + rows, prefill=True)
+            assert np.array_equal(ah, want_ah) and close(got, want)[0] == 0, launch
+        elif kind == "bundle":
+            _bundle(rows, Kk, (N, N // 4), bits)
+            launch = K.ops.last_launch()
+        else:
+            from tests.test_gpu_mlp import run_mlp_block
+            launch = run_mlp_block(rows, Kk, N, bits)
+    assert ("exl3_gemm_rows_kernel" in launch) == matrix and ("exl3_gemv_kernel" in launch) != matrix, launch
+
+
+@pytest.mark.parametrize("rows,H,I,bits", [(2, 512, 512, 4), (8, 640, 768, 3), (4, 384, 512, 4)])
+def test_small_block_with_fused_norm(rows, H, I, bits):
+    """Below five rows the block takes the kernel and the MLP by itself does not: one result within the summation-order
+    bound of the other; under 512 of `hidden` both keep the dot-product kernel."""
+    from berth_amd.device import Gpu, ptr
+    from tests.test_gpu_mlp import _block_inputs, _layer
+    gpu = Gpu(0)
+    _, mlp = _layer(gpu, H, I, bits, 9300 + rows, rows)
+    x, res, w = _block_inputs(gpu, H, rows, 9350 + rows)
+    res_ref, h = res.clone(), torch.zeros((rows, H), dtype=torch.float16, device=DEV)
+    res_out, y, y_ref = torch.zeros_like(res), torch.zeros_like(res), torch.zeros_like(res)
+    with knobs(BERTH_GEMM_ROWS_UNITS=-1):
+        K.ops.rms_norm_res_in(ptr(x), ptr(w), ptr(h), ptr(res_ref), rows, H, 1e-6, 1.0, 1.0, True, gpu.raw_stream())
+        mlp.forward(gpu, h, y_ref, rows=rows)
+        K.ops.add_f32(ptr(y_ref), ptr(res_ref), ptr(y_ref), rows * H, gpu.raw_stream())
+        mlp.forward_block(gpu, x, res, res_out, w, y, rows=rows)
+        launch = K.last_launch()
+    torch.cuda.synchronize()
+    assert ("add_rms_norm_had_r_128_kernel" in launch and "+add" in launch) == (H >= 512), launch
+    assert torch.equal(res_out, res_ref)
+    assert close(y.cpu().numpy(), y_ref.cpu().numpy())[0] == 0, launch
