@@ -693,15 +693,9 @@ extern "C" int berth_exl3_mlp_block(const void* x, const void* residual, void* r
         const bool fuse_norm = size_m == 1 ? gemv_stream_applies(2, hidden, intermediate, false)
                                            : aligned && hidden <= kNormRotateMaxCols &&
                                                  mlp_pair_on_matrix_units(size_m, hidden, intermediate, RowsInput::kNorm);
-        // (as mlp_linears asks for the down projection)
-        const auto down_on_matrix_units = [&] {
-            const RowsInput input = fuse_norm ? RowsInput::kNorm
-                                    : mlp_pair_on_matrix_units(size_m, hidden, intermediate, RowsInput::kMlp) ? RowsInput::kMlp
-                                                                                                             : RowsInput::kLaunch;
-            return gemv_rows_on_matrix_units(1, size_m, intermediate, hidden, input);
-        };
         const bool fuse_add = size_m == 1 ? gemv_stream_applies(1, intermediate, hidden, false)
-                                          : aligned && (size_m > 8 || down_on_matrix_units());
+                                          : aligned && (size_m > 8 || gemv_rows_on_matrix_units(1, size_m, intermediate, hidden,
+                                                                                            fuse_norm ? RowsInput::kNorm : RowsInput::kMlp));
         std::string desc;
         if (fuse_norm) {
             pair.a = nullptr;

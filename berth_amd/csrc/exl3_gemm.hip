@@ -166,9 +166,10 @@ bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, 
         // 1024x2048 25.1 / 28.6 / 38.5 -> 23.7 / 24.3 / 24.9, 2048x6144 at two 28.7 -> 25.2, 4096x4096 28.2 -> 28.0.
         return true;
     case RowsInput::kMlp:
-        // Three launches beside two: 512x1024 at 4 / 5 / 8 rows 20.2 / 22.5 / 30.4 -> 19.3 / 19.8 / 19.6, 1024x2048 at
-        // 2 / 3 / 4 / 5 rows 18.6 / 20.4 / 22.3 / 24.7 -> 22.7 / 22.6 / 22.8 / 22.9.
-        return size_m >= 5;
+        // Three launches beside two: MLPs of 2048x4096 at 2 / 3 rows 19.9 / 21.9 -> 24.1 / 24.4, of 1536x3072 at 4 / 5 / 8
+        // rows 23.6 / 25.1 / 29.8 -> 23.9 / 24.6 / 24.7; down alone, 1024 x 2048 at 4 / 5 / 8 rows, saves 0 / 3 / 7.  The
+        // smallest keep the two launches that the entry promises them.
+        return size_m >= 5 && size_k >= 1024 && (slices == 2 ? size_k : size_n) > 1024;
     case RowsInput::kLaunch:
         break;
     }

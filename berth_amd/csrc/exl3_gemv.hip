@@ -220,7 +220,7 @@ std::string launch_gemv(const LinearArgs& a, const Workspace* scratch)
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
     const int mmax = a.size_m == 1 ? 1 : 8;
-    if (rows_on_matrix_units(ws, 1, a.size_m, a.size_k, a.size_n, a.a_up ? RowsInput::kLaunch : RowsInput::kSelf)) {
+    if (rows_on_matrix_units(ws, 1, a.size_m, a.size_k, a.size_n, a.a_up ? RowsInput::kMlp : RowsInput::kSelf)) {
         scope.reset();          // the MFMA launcher holds its own
         return launch_gemm(a, scratch);
     }

@@ -175,8 +175,8 @@ std::string launch_gemv_pair(const PairArgs& args);
 // with whole_rows, whether every workgroup of it then holds the whole input row)
 bool gemv_stream_applies(int problems, int size_k, int size_n, bool whole_rows);
 
-// What stands ahead of a launch of few rows: the launch rotates its input itself, a launch does so for it, gate and up
-// of an MLP whose down projection takes the kernel too, or the launch that forms an MLP block's norm.
+// What stands ahead of a launch of few rows: the launch rotates its input itself, a launch does so for it, or it is one
+// of an MLP's (gate and up, down), by itself or in a block whose norm one launch forms and rotates.
 enum class RowsInput { kSelf, kLaunch, kMlp, kNorm };
 // whether 2..8 rows of `problems` linears of this shape run on the few-row MFMA kernel
 bool gemv_rows_on_matrix_units(int problems, int size_m, int size_k, int size_n, RowsInput input);

@@ -261,7 +261,7 @@ typedef struct {
  * y = down(silu(gate(x)) * up(x)), the four calls of MlpLayer::forward
  * (crates/berth-engine/src/mlp.rs:118-150: two berth_exl3_linear with fp16
  * output, berth_ops_silu_mul with act_limit 0, berth_exl3_linear with fp32
- * output) in one entry.  One row, and 2..8 rows of small weights (from five rows: of narrow ones), run as two
+ * output) in one entry.  One row, and 2..8 rows of small weights (hidden up to 1024 at least), run as two
  * launches: gate and up share one launch and the rotated input, and the down
  * projection evaluates silu(g) * u while it rotates its input (same fp16 steps as
  * berth_ops_silu_mul, so the activation is bit-identical to the unfused sequence).

@@ -325,7 +325,7 @@ def _bundle(rows, Kk, widths, bits):
     ("linear", 8, 384, 4096, 2, 0, False),      # three k-blocks
     ("linear", 3, 3072, 256, 5, 0, True),
     ("bundle", 4, 1024, 512, 4, 2, False), ("bundle", 5, 1024, 512, 4, 2, True), ("bundle", 8, 896, 512, 4, 2, False),
-    ("mlp", 4, 512, 640, 4, 2, False), ("mlp", 5, 512, 640, 4, 2, True),
+    ("mlp", 4, 1152, 1280, 4, 2, False), ("mlp", 5, 1152, 1280, 4, 2, True), ("mlp", 8, 1024, 1152, 3, 2, False),
 ])
 def test_small_weights_beside_the_dot_product_kernel(kind, rows, Kk, N, bits, cb, matrix):
     """Which kernel two to eight rows of small weights take, on both sides of every line, and its results."""
@@ -344,22 +344,30 @@ def test_small_weights_beside_the_dot_product_kernel(kind, rows, Kk, N, bits, cb
 
 @pytest.mark.parametrize("rows,H,I,bits", [(2, 512, 512, 4), (8, 640, 768, 3), (4, 384, 512, 4)])
 def test_small_block_with_fused_norm(rows, H, I, bits):
-    """Below five rows the block takes the kernel and the MLP by itself does not: one result within the summation-order
-    bound of the other; under 512 of `hidden` both keep the dot-product kernel."""
+    """From 512 of `hidden` on a block's MLP takes the kernel at any of these row counts: gate and up, the rotated
+    activation and the output, each from the device's own results of the stage before."""
     from berth_amd.device import Gpu, ptr
     from tests.test_gpu_mlp import _block_inputs, _layer
     gpu = Gpu(0)
-    _, mlp = _layer(gpu, H, I, bits, 9300 + rows, rows)
+    (gate, up, down), mlp = _layer(gpu, H, I, bits, 9300 + rows, rows)
     x, res, w = _block_inputs(gpu, H, rows, 9350 + rows)
     res_ref, h = res.clone(), torch.zeros((rows, H), dtype=torch.float16, device=DEV)
-    res_out, y, y_ref = torch.zeros_like(res), torch.zeros_like(res), torch.zeros_like(res)
+    res_out, y = torch.zeros_like(res), torch.zeros_like(res)
+    K.ops.rms_norm_res_in(ptr(x), ptr(w), ptr(h), ptr(res_ref), rows, H, 1e-6, 1.0, 1.0, True, gpu.raw_stream())
     with knobs(BERTH_GEMM_ROWS_UNITS=-1):
-        K.ops.rms_norm_res_in(ptr(x), ptr(w), ptr(h), ptr(res_ref), rows, H, 1e-6, 1.0, 1.0, True, gpu.raw_stream())
-        mlp.forward(gpu, h, y_ref, rows=rows)
-        K.ops.add_f32(ptr(y_ref), ptr(res_ref), ptr(y_ref), rows * H, gpu.raw_stream())
         mlp.forward_block(gpu, x, res, res_out, w, y, rows=rows)
         launch = K.last_launch()
     torch.cuda.synchronize()
     assert ("add_rms_norm_had_r_128_kernel" in launch and "+add" in launch) == (H >= 512), launch
     assert torch.equal(res_out, res_ref)
-    assert close(y.cpu().numpy(), y_ref.cpu().numpy())[0] == 0, launch
+    normed = host_f16(h)
+    g, u = (host_f16(t)[:rows * I].reshape(rows, I) for t in (mlp.g, mlp.u))
+    for got, lin in ((g, gate), (u, up)):
+        assert close(got, O.linear(normed, *lin, H, I, bits, 2)[0].reshape(rows, I))[0] == 0, launch
+    act = O.silu_mul(g, u).reshape(rows, I)
+    want, act_had = O.linear(act, *down, I, H, bits, 2, out_fp32=True)
+    assert np.array_equal(host_u16(mlp.act_had)[:rows * I], act_had.view(np.uint16).ravel())
+    # rows of a norm reach 5e4 here, and where they cancel what is left is the rounding of the sums: a wave adds eight
+    # products at a time, I / 8 roundings of half an ulp of partial sums as large as the largest output
+    atol = max(1e-3, I / 8 * 2.0 ** -24 * float(np.abs(want).max()))
+    assert close(y.cpu().numpy(), want.reshape(rows, H) + res_ref.cpu().numpy(), atol=atol)[0] == 0, launch
