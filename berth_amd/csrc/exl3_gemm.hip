@@ -102,12 +102,17 @@ static RowsPlan plan_rows(const Workspace& ws, int slices, int slabs, int size_m
         unsigned q = (unsigned)(U / G), rem = (unsigned)(U % G), S = 0;
         const unsigned most = q + (rem ? 1 : 0);
         unsigned ncb = (most + TR4 - 2) / TR4 + 1;                  // column blocks a range can touch
-        // At least two workgroups per column block: parts of its own for each block where the
-        // longest part is no more than an eighth above the even share.  A range across two blocks
-        // hands both over (2688 x 4096 at 8 / 32 rows: 12.8 / 22.1 -> 11.1 / 16.1 us with parts of its own).
+        // At least two workgroups per column block: parts of its own for each block where the longest part is no more than
+        // an eighth or six units above the even share.  A range across two blocks hands both over (2688 x 4096 at 8 / 32
+        // rows: 12.8 / 22.1 -> 11.1 / 16.1 us with parts of its own), and needs the whole input, which a launch ahead of it
+        // rotates then: 4096x3072, 7 units instead of 6, at 4 / 8 / 16 / 32 rows 13.2 / 14.5 / 17.7 / 23.5 -> 9.8 / 10.2 / 12.2 /
+        // 17.4; 2048x11264, 16 instead of 11, 14.1 / 14.5 / 16.1 / 20.8 -> 11.2 / 11.6 / 12.9 / 17.4; 17408x5632, 55 instead of
+        // 47, even (23.3 -> 23.8 at 8 rows, 31.1 -> 28.4 at 32); 5120x11520, 40 instead of 29, 19.2 -> 19.8; 8192x11264, 64
+        // instead of 44, 23.2 -> 26.1.  Gate and up whose input the norm's launch rotates, 16 units instead of 11: layers of
+        // hidden 2048 at 8 rows 51.0 -> 47.6.
         if (G >= 2 * (unsigned long long)blocks) {
-            const unsigned s = (unsigned)(G / blocks);
-            if (TR4 / s >= 4 && ((TR4 + s - 1) / s) * 8ull <= most * 9ull) {
+            const unsigned s = (unsigned)(G / blocks), longest = (TR4 + s - 1) / s;
+            if (TR4 / s >= 4 && (longest * 8ull <= most * 9ull || longest <= most + 6)) {
                 S = s;
                 G = (unsigned long long)blocks * s;
                 q = rem = 0;

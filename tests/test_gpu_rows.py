@@ -371,3 +371,17 @@ def test_small_block_with_fused_norm(rows, H, I, bits):
     # products at a time, I / 8 roundings of half an ulp of partial sums as large as the largest output
     atol = max(1e-3, I / 8 * 2.0 ** -24 * float(np.abs(want).max()))
     assert close(y.cpu().numpy(), want.reshape(rows, H) + res_ref.cpu().numpy(), atol=atol)[0] == 0, launch
+
+
+@pytest.mark.parametrize("rows,Kk,N,bits,own", [
+    (2, 2944, 256, 5, True),            # parts of four and five units beside an even share of four
+    (9, 1152, 512, 4, True),            # 18 units in four parts
+    (16, 4096, 3072, 3, True),          # ten parts of six and seven, in a grid of fewer than the compute units
+    (23, 2816, 11264, 2, True),         # two of 22 beside a share of 16
+    (16, 3072, 11264, 2, False),        # two of 24 beside 17
+])
+def test_parts_longer_than_the_even_share(rows, Kk, N, bits, own):
+    """Column blocks cut into parts of their own, whose launch rotates its input, up to six units above the even share."""
+    got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, bits, 2, True, 90 + rows, prefill=True)
+    assert "exl3_gemm_rows_kernel" in launch and ("had_r_128" not in launch) == own, launch
+    assert np.array_equal(ah, want_ah) and close(got, want)[0] == 0, launch
