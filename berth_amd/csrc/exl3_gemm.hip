@@ -224,6 +224,11 @@ static bool fills_128_row_tiles(const Workspace& ws, long nblocks, int size_m)
 //   * enough steps that the second launch and the hand-over pay: one per compute unit up to 64 rows (512x4096 14.0 ->
 //     14.7, 512x16384 20.4 -> 19.1, 4096x4096 23.5 -> 21.0), 2.25 of them above (4096x4096 at 100 rows 24.8 -> 27.0,
 //     7296x2688 33.8 -> 28.4);
+//     Fewer are enough of deep weights, whose 32-row tiles share a tile between many workgroups, for up to two blocks of
+//     96 rows (not for the last few rows of a third tile of sixteen): 48 steps at 36 / 64 / 96 rows of 3072x512 16.8 / 17.5 / 18.4 -> 14.4 / 15.1 / 16.5, 4096x1024 20.6 / 21.9 /
+//     22.9 -> 15.5 / 16.9 / 19.1, 8192x512 26.6 / 28.3 / 28.6 -> 18.8 / 20.4 / 23.6, at 160 rows 29.9 -> 26.6; but 3072x256
+//     at 80 rows 17.2 -> 18.1, 2048x2048 at 36 / 96 rows 17.3 / 19.6 -> 16.6 / 19.8, 1024x2048 13.0 / 14.8 -> 15.6 / 17.7,
+//     4864x1536 at 112 rows 24.3 -> 26.4.
 //   * narrow outputs, which would run as 32-row tiles and decode every weight once per 32 rows: always (17408x5120 at
 //     64, 128, 256 and 384 rows 59, 88, 162, 167 -> 32, 46, 72, 100), up to gemm_block_rows;
 //   * wide outputs: a launch of 128-row or 256-row tiles costs the same for any rows up to a multiple of those, row
@@ -268,7 +273,8 @@ static BlockPlan plan_block(const Workspace& ws, int codebook, int slices, int s
     const unsigned long long U = tiles * spt;
     if (U >= (1ull << 30)) return pl;
     const int least = knobs().gemm_block_steps;
-    if (U < (unsigned long long)(least >= 0 ? least : size_m <= 64 ? 256 : 576)) return pl;
+    const bool deep = size_m >= 36 && pl.rows_per_tile <= 96 && (pl.row_blocks == 1 ? size_k >= 3072 : pl.row_blocks == 2 && size_k >= 3584);
+    if (U < (unsigned long long)(least >= 0 ? least : deep ? 48 : size_m <= 64 ? 256 : 576)) return pl;
     if (least < 0 && !blocks_beside_wide_tiles(ws, codebook, (long)slices * ((size_n + 255) / 256), size_m, pl, U)) return pl;
     unsigned long long G = (unsigned long long)ws.cu_count;
     if (G > U) G = U;

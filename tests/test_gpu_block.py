@@ -82,6 +82,26 @@ def test_the_rule_beside_wide_tiles(rows, Kk, N, cb, blocks):
     assert bad == 0, (bad, worst, launch)
 
 
+@pytest.mark.parametrize("rows,Kk,N,cb,blocks", [
+    (36, 3072, 512, 2, True),           # 48 steps
+    (36, 3072, 384, 2, False),
+    (35, 4096, 1024, 2, False),
+    (96, 2944, 1024, 2, False),         # not deep enough
+    (97, 4096, 1024, 2, False),         # blocks of more than 96 rows
+    (160, 3584, 512, 1, True),          # two blocks of 80
+    (160, 3456, 512, 0, False),
+    (288, 4096, 512, 2, False),         # three
+])
+def test_the_rule_of_deep_weights(rows, Kk, N, cb, blocks):
+    """Both sides of the rule that sends deep and narrow weights to this kernel, each against the oracle."""
+    with knobs(BERTH_GEMM_BLOCK_ROWS=511, BERTH_GEMM_BLOCK_STEPS=-1):
+        got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, 4, cb, True, 280 + rows, prefill=True)
+    assert ("exl3_gemm_block_kernel" in launch) == blocks, launch
+    assert np.array_equal(ah, want_ah), launch
+    bad, worst = close(got, want)
+    assert bad == 0, (bad, worst, launch)
+
+
 @pytest.mark.parametrize("rows,unit", [(40, 128), (150, 128), (70, 0)])
 def test_bundle_with_narrower_slices(rows, unit):
     """Sliced lists whose widths differ: blocks past a slice's end are empty and touch nothing.  unit 0: four slices of one
