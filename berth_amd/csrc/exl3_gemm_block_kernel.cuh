@@ -287,7 +287,7 @@ __global__ __launch_bounds__(1024, 1) void exl3_gemm_block_kernel(GemmParams p)
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
                 if (par) {
-                    *(float4_t*)(mine + (4 * j + hi) * 16384 + f * 1024) = half[2 * j][f];
+                    if (4 * j + 1 < MT || !hi) *(float4_t*)(mine + (4 * j + hi) * 16384 + f * 1024) = half[2 * j][f];
                     if (both) sum[j][f] = half[both ? 2 * j + 1 : 0][f];
                 } else {
                     if (both && (4 * j + 3 < MT || !hi)) *(float4_t*)(mine + (4 * j + 2 + hi) * 16384 + f * 1024) = half[both ? 2 * j + 1 : 0][f];
