@@ -1032,7 +1032,8 @@ extern "C" int berth_ops_silu_mul(const void* gate, const void* up, void* out, i
 static int mgemm_entry(const void* a, const void* b_list, void* c, const void* suh_list, void* a_had,
                        const void* svh_list, int size_m, int size_k, int size_n, int k_bits, int codebook, int c_fp32,
                        int bszm_in, int bszm_out, const int* size_n_list, const void* c_ptrs, const int* n_stride_list,
-                       const int* had_src_list, int num_had_src, void* stream, bool host_lists)
+                       const int* had_src_list, int num_had_src, void* stream, bool host_lists,
+                       const berth_mgemm_lists* host = nullptr)
 {
     try {
         g_ops_err.clear();
@@ -1062,6 +1063,22 @@ static int mgemm_entry(const void* a, const void* b_list, void* c, const void* s
                     bszm_in, bszm_out, size_n_list, c_ptrs, n_stride_list, had_src_list, num_had_src,
                     (hipStream_t)stream};
         m.host_lists = host_lists;
+        MgemmArgs by_value = m;
+        if (host) {
+            if (!any_list) throw std::runtime_error("exl3_mgemm: host copies of the lists are for sliced mode");
+            if (!host->b_list || !host->suh_list || !host->svh_list || !host->size_n_list || !host->c_ptrs || !host->n_stride_list ||
+                !host->had_src_list)
+                throw std::runtime_error("exl3_mgemm: null host list");
+            by_value.b_list = host->b_list;
+            by_value.suh_list = host->suh_list;
+            by_value.svh_list = host->svh_list;
+            by_value.size_n_list = host->size_n_list;
+            by_value.c_ptrs = host->c_ptrs;
+            by_value.n_stride_list = host->n_stride_list;
+            by_value.had_src_list = host->had_src_list;
+            by_value.host_lists = true;
+            m.by_value = &by_value;
+        }
         g_ops_launch = launch_mgemm(m);
         return 1;
     } catch (const std::exception& err) {
@@ -1090,6 +1107,17 @@ extern "C" int berth_ops_mgemm_hostlists(const void* a, const void* b_list, void
 {
     return mgemm_entry(a, b_list, c, suh_list, a_had, svh_list, size_m, size_k, size_n, k_bits, codebook, c_fp32, bszm_in,
                        bszm_out, size_n_list, c_ptrs, n_stride_list, had_src_list, num_had_src, stream, true);
+}
+
+extern "C" int berth_ops_mgemm_both_lists(const void* a, const void* b_list, void* c, const void* suh_list,
+                                          void* a_had, const void* svh_list, int size_m, int size_k, int size_n,
+                                          int k_bits, int codebook, int c_fp32, int bszm_in, int bszm_out,
+                                          const int* size_n_list, const void* c_ptrs, const int* n_stride_list,
+                                          const int* had_src_list, int num_had_src, void* stream,
+                                          const berth_mgemm_lists* host)
+{
+    return mgemm_entry(a, b_list, c, suh_list, a_had, svh_list, size_m, size_k, size_n, k_bits, codebook, c_fp32, bszm_in,
+                       bszm_out, size_n_list, c_ptrs, n_stride_list, had_src_list, num_had_src, stream, false, host);
 }
 
 extern "C" const char* berth_ops_last_error(void) { return g_ops_err.c_str(); }

@@ -489,10 +489,12 @@ public:
             gpu.synchronize();
             c_host_ = c;
         }
-        if (berth_ops_mgemm(a.raw(), d_b_.raw(), (void*)(uintptr_t)outs[0], d_suh_.raw(), a_had_.raw(), d_svh_.raw(), rows,
-                            size_k_, width_, k_bits_, (int)codebook_, (int)out, 1, slices(), (const int*)d_size_n_.raw(),
-                            d_c_.raw(), (const int*)d_stride_.raw(), (const int*)d_src_.raw(), (int)sources_.size(),
-                            gpu.raw_stream()) <= 0)
+        // (2..8 rows go by value where the launch finds that of use)
+        const berth_mgemm_lists host{b_.data(), suh_.data(), svh_.data(), size_n_.data(), c.data(), stride_.data(), src_.data()};
+        if (berth_ops_mgemm_both_lists(a.raw(), d_b_.raw(), (void*)(uintptr_t)outs[0], d_suh_.raw(), a_had_.raw(), d_svh_.raw(),
+                                       rows, size_k_, width_, k_bits_, (int)codebook_, (int)out, 1, slices(),
+                                       (const int*)d_size_n_.raw(), d_c_.raw(), (const int*)d_stride_.raw(),
+                                       (const int*)d_src_.raw(), (int)sources_.size(), gpu.raw_stream(), &host) <= 0)
             throw KernelError(berth_ops_last_error());
     }
 

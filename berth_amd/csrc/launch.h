@@ -254,10 +254,11 @@ struct MgemmArgs {
     const int* had_src_list;
     int num_had_src;
     hipStream_t stream;
-    bool host_lists = false;    // the seven lists are host memory (one row, the streaming kernel only)
+    bool host_lists = false;    // the seven lists are host memory
+    const MgemmArgs* by_value = nullptr;        // the same call with the lists in host memory
 };
 std::string launch_mgemm(const MgemmArgs& args);
-// more than 8 rows: the bundle as one dense MFMA launch
+// the bundle as one dense MFMA launch
 std::string launch_gemm_bundle(const MgemmArgs& args);
 // Rotated inputs in one launch: out slab s = Hh(in(s) * suh(s)) for s < slabs, with in(s) = in +
 // s * in_stride and the slabs out_stride elements apart (or at out_host[s], by-value scales only);

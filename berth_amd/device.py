@@ -251,9 +251,8 @@ class Exl3MultiLinear:
     `exl3_mgemm` (the qkv bundles of crates/berth-engine/src/attn.rs:1934-1973 and
     gdn.rs:1102-1130; list layout from crates/berth-kernels/src/ops.rs:264-293):
     every source is cut into slices of the greatest common width.  Any row count: one
-    row runs the streaming kernel, 2..8 of small weights the dot-product kernel (2..4
-    from a size_k of 1024 on), the rest the MFMA kernels (the reference sends 9..32 rows through the
-    same call, prefill.rs:81-85)."""
+    row runs the streaming kernel, 2..8 of small weights the dot-product kernel, the rest the MFMA
+    kernels (the reference sends 9..32 rows through the same call, prefill.rs:81-85)."""
 
     def __init__(self, gpu: Gpu, sources: list[Exl3Linear]):
         import math
@@ -295,7 +294,7 @@ class Exl3MultiLinear:
                    "src": np.array(src, dtype=np.int32)}
         self._h_c = None
         self._h_at = {name: array.ctypes.data for name, array in self._h.items()}    # addresses, looked up once
-        self._h_c_at = 0
+        self._h_c_at, self._h_lists = 0, None
         self.host_lists = self.slices <= 16
 
     def forward(self, gpu: Gpu, a: torch.Tensor, outs: list[torch.Tensor], out: OutDtype, rows: int = 1,
@@ -313,9 +312,11 @@ class Exl3MultiLinear:
             self._c_ptrs = torch.tensor(ptrs, dtype=torch.int64, device=gpu.device)
             self._h_c = np.array(ptrs, dtype=np.uint64)
             self._h_c_at = self._h_c.ctypes.data
+            h = self._h_at
+            self._h_lists = K.MgemmLists(h["b"], h["suh"], h["svh"], h["size_n"], self._h_c_at, h["stride"], h["src"])
             self._c_key = key
-        # lists by value: one row through the streaming kernel, more than 8 rows through the MFMA
-        # kernels (2..8 rows read the device lists)
+        # lists by value: one row through the streaming kernel, more than 8 rows through the MFMA kernels, 2..8
+        # rows where the launch finds them of use
         if by_value and ((rows == 1 and self.host_lists) or (rows > 8 and self.slices <= 16)):
             h = self._h_at
             try:
@@ -328,6 +329,12 @@ class Exl3MultiLinear:
                 if rows > 1 or "host lists" not in str(err):
                     raise
                 self.host_lists = False         # too small for the streaming kernel: device lists from now on
+        if by_value and 1 < rows <= 8:
+            K.ops.exl3_mgemm_both_lists(self._h_lists, ptr(a), ptr(self.b_list), ptr(outs[0]), ptr(self.suh_list), ptr(self.a_had),
+                                        ptr(self.svh_list), rows, self.size_k, self.width, self.k_bits, self.codebook, out,
+                                        1, self.slices, ptr(self.size_n_list), ptr(self._c_ptrs), ptr(self.n_stride_list),
+                                        ptr(self.had_src_list), len(self.sources), gpu.raw_stream())
+            return
         K.ops.exl3_mgemm(ptr(a), ptr(self.b_list), ptr(outs[0]), ptr(self.suh_list), ptr(self.a_had),
                          ptr(self.svh_list), rows, self.size_k, self.width, self.k_bits, self.codebook, out,
                          1, self.slices, ptr(self.size_n_list), ptr(self._c_ptrs), ptr(self.n_stride_list),

@@ -74,6 +74,7 @@ def load() -> C.CDLL:
         L.berth_exl3_unpack_signs.restype = C.c_int
         L.berth_ops_mgemm.argtypes = [vp, vp, vp, vp, vp, vp, ci, ci, ci, ci, ci, ci, ci, ci, vp, vp, vp, vp, ci, vp]
         L.berth_ops_mgemm_hostlists.argtypes = L.berth_ops_mgemm.argtypes
+        L.berth_ops_mgemm_both_lists.argtypes = L.berth_ops_mgemm.argtypes + [vp]
         for name in ("berth_exl3_last_error", "berth_exl3_last_launch", "berth_prefill_last_error",
                      "berth_prefill_last_launch", "berth_ops_last_error", "berth_ops_last_launch"):
             getattr(L, name).restype = C.c_char_p
@@ -255,6 +256,12 @@ class prefill_lin:
         return _s(load().berth_prefill_last_error())
 
 
+class MgemmLists(C.Structure):
+    """`berth_mgemm_lists`: addresses of the seven lists of a sliced bundle in host memory."""
+    _fields_ = [(name, C.c_void_p) for name in ("b_list", "suh_list", "svh_list", "size_n_list", "c_ptrs", "n_stride_list",
+                                                "had_src_list")]
+
+
 class ops:
     """crates/berth-kernels/src/ops.rs (the EXL3-path subset)."""
 
@@ -282,6 +289,18 @@ class ops:
         if rc > 0:
             return rc
         raise LaunchError(ops.last_error() or f"exl3_mgemm (host lists) launch failed ({rc})")
+
+    @staticmethod
+    def exl3_mgemm_both_lists(host, a, b_list, c, suh_list, a_had, svh_list, size_m, size_k, size_n, k_bits,
+                              codebook: Codebook, out: OutDtype, bszm_in, bszm_out, size_n_list, c_ptrs,
+                              n_stride_list, had_src_list, num_had_src, stream=None) -> int:
+        """berth_ops_mgemm_both_lists: exl3_mgemm of slices with its lists on the host too (`host`: an MgemmLists)."""
+        rc = load().berth_ops_mgemm_both_lists(a, b_list, c, suh_list, a_had, svh_list, size_m, size_k, size_n, k_bits,
+                                               int(codebook), int(out), bszm_in, bszm_out, size_n_list, c_ptrs,
+                                               n_stride_list, had_src_list, num_had_src, stream, C.byref(host))
+        if rc > 0:
+            return rc
+        raise LaunchError(ops.last_error() or f"exl3_mgemm launch failed ({rc})")
 
     @staticmethod
     def rms_norm(x, weight, y, rows: int, dim: int, epsilon: float, constant_bias: float = 1.0,

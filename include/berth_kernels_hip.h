@@ -233,6 +233,25 @@ int berth_ops_mgemm_hostlists(const void* a, const void* b_list, void* c, const 
                               int codebook, int c_fp32, int bszm_in, int bszm_out, const int* size_n_list,
                               const void* c_ptrs, const int* n_stride_list, const int* had_src_list,
                               int num_had_src, void* stream);
+/* No counterpart in the reference: berth_ops_mgemm in sliced mode for a caller that holds its seven lists on
+ * the host too (`host`, arrays as for berth_ops_mgemm_hostlists, the same contents as the device lists).  Two
+ * to eight rows of at most 16 slices that run on the few-row MFMA kernel then travel by value, and the launch
+ * rotates the input itself where a workgroup needs a part of size_k only and no output lies over the input or
+ * a_had; any other call is berth_ops_mgemm with the device lists.  The host lists are read during the call only. */
+typedef struct {
+    const void* b_list;
+    const void* suh_list;
+    const void* svh_list;
+    const int* size_n_list;
+    const void* c_ptrs;
+    const int* n_stride_list;
+    const int* had_src_list;
+} berth_mgemm_lists;
+int berth_ops_mgemm_both_lists(const void* a, const void* b_list, void* c, const void* suh_list, void* a_had,
+                               const void* svh_list, int size_m, int size_k, int size_n, int k_bits,
+                               int codebook, int c_fp32, int bszm_in, int bszm_out, const int* size_n_list,
+                               const void* c_ptrs, const int* n_stride_list, const int* had_src_list,
+                               int num_had_src, void* stream, const berth_mgemm_lists* host);
 const char* berth_ops_last_error(void);    /* ops.rs:145 */
 const char* berth_ops_last_launch(void);   /* ops.rs:146 */
 

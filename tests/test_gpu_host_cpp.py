@@ -51,7 +51,7 @@ def test_cpp_linear(tmp_path, rows, fp32, use_rows):
 @pytest.mark.parametrize("rows,fp32", [(1, 0), (4, 1), (20, 0), (150, 1)])
 def test_cpp_bundle(tmp_path, rows, fp32):
     """MultiLinear: three linears on one input as one sliced berth_ops_mgemm, every row-count
-    route (one row, 2..8 rows from the device lists, more than 8 rows by value)."""
+    route (one row, 2..8 rows with the lists on both sides, more than 8 rows by value)."""
     Kk, Ns, bits = 256, (768, 256, 512), 4
     lins = [synth.linear(4500 + rows + i, Kk, n, bits) for i, n in enumerate(Ns)]
     x = synth.activations(4600 + rows, rows, Kk)

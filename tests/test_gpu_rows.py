@@ -317,6 +317,59 @@ def _bundle(rows, Kk, widths, bits):
         assert close(host_f16(out), O.linear(x, *lin, Kk, n, bits, 2, out_fp32=False)[0])[0] == 0, K.ops.last_launch()
 
 
+@pytest.mark.parametrize("rows,Kk,widths,bits,fp32,rotates", [
+    (2, 1024, (1024, 512, 512), 4, False, True),
+    (4, 512, (512, 256), 3, True, True),            # four k-blocks, the fewest rows
+    (3, 512, (512, 256), 3, False, False),          # the dot-product kernel, from the device lists
+    (8, 2304, (1024, 512, 512), 2, True, True),
+    (5, 384, (512, 256), 4, False, False),          # three k-blocks
+    (8, 1152, (128 * 17, 128), 4, False, False),    # eighteen slices stay in device memory
+    (7, 640, (256, 256, 128), 6, False, True),      # five k-blocks
+])
+def test_few_rows_of_a_bundle_by_value(rows, Kk, widths, bits, fp32, rotates):
+    """Lists on both sides: every source and its rotated rows, which the launch that rotates leaves once; twice the same bits."""
+    from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
+    gpu = Gpu(0)
+    lins = [synth.linear(760 + i, Kk, n, bits) for i, n in enumerate(widths)]
+    multi = Exl3MultiLinear(gpu, [Exl3Linear(gpu, f"l{i}", *l) for i, l in enumerate(lins)])
+    x = synth.activations(770 + rows, rows, Kk)
+    res = []
+    for _ in range(2):
+        outs = [torch.zeros((rows, n), dtype=torch.float32 if fp32 else torch.float16, device=DEV) for n in widths]
+        with knobs(BERTH_GEMM_ROWS_UNITS=-1):
+            multi.forward(gpu, dev(x.view(np.uint16)), outs, OutDtype.F32 if fp32 else OutDtype.F16, rows)
+            launch = K.ops.last_launch()
+        torch.cuda.synchronize()
+        assert (",rotate>" in launch) == rotates == ("by value" in launch), launch
+        res.append([o.cpu().numpy() for o in outs])
+    for i, lin in enumerate(lins):
+        want, want_had = O.linear(x, *lin, Kk, widths[i], bits, 2, out_fp32=fp32)
+        assert close(res[0][i], want)[0] == 0 and np.array_equal(res[0][i], res[1][i]), i
+        slab = host_u16(multi.a_had)[i * rows * Kk:(i + 1) * rows * Kk]
+        assert np.array_equal(slab, want_had.view(np.uint16).reshape(-1)), i
+
+
+def test_few_rows_by_value_with_outputs_over_the_input():
+    """The host sees that an output lies over the input: a launch of its own rotates, and the bits are those of other buffers."""
+    from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
+    gpu, rows, Kk, widths = Gpu(0), 6, 2304, (1024, 512)
+    multi = Exl3MultiLinear(gpu, [Exl3Linear(gpu, f"l{i}", *synth.linear(780 + i, Kk, n, 4)) for i, n in enumerate(widths)])
+    d_x = dev(synth.activations(785, rows, Kk).view(np.uint16))
+    res = []
+    for over in (False, True):
+        a, flat = d_x.clone(), torch.zeros(rows * Kk, dtype=torch.float16, device=DEV)
+        flat = a.view(torch.float16).reshape(-1) if over else flat
+        outs, at = [], 0
+        for n in widths:
+            outs.append(flat[at:at + rows * n].view(rows, n))
+            at += rows * n
+        multi.forward(gpu, a, outs, OutDtype.F16, rows)
+        torch.cuda.synchronize()
+        assert (",rotate>" in K.ops.last_launch()) == (not over), K.ops.last_launch()
+        res.append([host_u16(o).copy() for o in outs])
+    assert all(np.array_equal(u, v) for u, v in zip(*res))
+
+
 @pytest.mark.parametrize("kind,rows,Kk,N,bits,cb,matrix", [
     ("linear", 2, 768, 768, 4, 2, True),        # six k-blocks
     ("linear", 2, 512, 1024, 4, 2, False),
