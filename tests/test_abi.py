@@ -155,6 +155,17 @@ def test_mgemm_validation():
         K.ops.exl3_mgemm(P, P, P, P, P, P, 1, 128, 128, 4, Codebook.MUL1, OutDtype.F16, 1, 2, num_had_src=1)
 
 
+def test_mgemm_with_both_lists_validation():
+    whole = K.MgemmLists(*[P] * 7)
+    with pytest.raises(LaunchError, match="for sliced mode"):
+        K.ops.exl3_mgemm_both_lists(whole, P, P, P, P, P, P, 4, 128, 128, 4, Codebook.MUL1, OutDtype.F16, 1, 2, None, None, None, None, 0)
+    with pytest.raises(LaunchError, match="null host list"):
+        K.ops.exl3_mgemm_both_lists(K.MgemmLists(P, P, P, P, P, P, None), P, P, P, P, P, P, 4, 128, 128, 4, Codebook.MUL1,
+                                    OutDtype.F16, 1, 2, P, P, P, P, 1)
+    with pytest.raises(LaunchError, match="single-input"):
+        K.ops.exl3_mgemm_both_lists(whole, P, P, P, P, P, P, 4, 128, 128, 4, Codebook.MUL1, OutDtype.F16, 2, 2, P, P, P, P, 1)
+
+
 def test_fused_mlp_validation():
     P = 0x1000
     lins = [(P, P, P)] * 3
