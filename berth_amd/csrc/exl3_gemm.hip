@@ -219,47 +219,148 @@ static bool fills_128_row_tiles(const Workspace& ws, long nblocks, int size_m)
     return nblocks * ((size_m + 127) / 128) * 4 >= ws.cu_count;
 }
 
+// How a dense launch of 128-row tiles or larger is cut up.  Whole tiles: a workgroup of four waves per
+// 128 x 256 tile, two of them on a compute unit.  Dealt out: one workgroup per compute unit with an even
+// share of the (tile, k-block) units, the workgroups of a shared tile adding their parts in k order;
+// of 128-row tiles, or of 256-row tiles (eight waves, every weight decoded once per 256 rows).
+enum class DenseTiles { kWhole128, kDealt128, kDealt256 };
+
+// The cheapest by what a compute unit spends, in 10 ns: k-blocks, the epilogue of every tile, and the
+// hand-over of shared ones, which takes longer the more workgroups share a tile.
+//   * Whole tiles hide part of an epilogue behind the other workgroup's k-loop, but come in rounds; a
+//     round with r of its tiles takes about (1 + r) / 2 of a full one, the first a whole one.
+//   * Dealt-out tiles have no partial round; their epilogue and hand-over are in nobody's shadow.  So a
+//     short K, where those weigh against few k-blocks, takes whole tiles, and a long one is dealt out.
+//   * The decode of 128-row tiles does not quite fit behind their MFMAs, so a k-block costs more with the
+//     codebooks of longer decode; with 256-row tiles it does fit (6144 columns of 4096 at 1500 rows, dealt 128 /
+//     dealt 256 us: MUL1 108/105, MCG 112/103, 3INST 123/105; the bit rate matters less).
+// Fitted to 499 launches at 4 bits (K 128 .. 10240, 2048 .. 32768 columns, 460 .. 1500 rows): the choice costs
+// 0.7 % over the fastest of the three on average, 14 % at most.  Examples, K x N at rows: whole / dealt
+// 128 / dealt 256 us: 256x8192 at 512 16/26/31, 512x16384 at 1500 46/59/59, 1024x4096 at 512 27/31/50,
+// 1024x16384 at 1500 72/88/81, 2048x4096 at 512 43/36/54, 2048x16384 at 1024 87/96/83, 5120x12288 at 600
+// 99/106/121, 4096x16384 at 600 128/111/122 and at 1500 231/254/225.
+struct TilesCost {
+    DenseTiles tiles;
+    long cost;          // in 10 ns, without what every form has in common
+};
+static TilesCost cheapest_tiles(long cus, int codebook, long KB, long tiles128, long tiles256, bool whole_allowed, bool wide_allowed)
+{
+    const long whole_kb = codebook == 0 ? 250 : codebook == 1 ? 236 : 230;
+    const long dealt_kb = codebook == 0 ? 260 : codebook == 1 ? 243 : 235;
+    const long n = tiles128 / cus, r = tiles128 % cus;          // full rounds, tiles of the last one
+    const long m = tiles256 / cus, s = tiles256 % cus;
+    // (one workgroup on a compute unit has no other to hide its epilogue behind)
+    const long whole = n == 0 || tiles128 == cus ? KB * whole_kb + 500 + 400 * tiles128 / cus
+                                                 : (2 * n * cus + (r ? cus + r : 0)) * (KB * whole_kb + 500) / (2 * cus);
+    const long dealt128 = tiles128 * KB * dealt_kb / cus + 800 * n + (r == 0 ? 0 : n ? 800 : 2500 - 1600 * r / cus);
+    const long dealt256 = tiles256 * KB * 415 / cus + 900 * m + (s == 0 ? 0 : m ? 1900 : 3700 - 2200 * s / cus);
+    if (whole_allowed && whole < dealt128 && (!wide_allowed || whole <= dealt256)) return {DenseTiles::kWhole128, whole};
+    return wide_allowed && dealt256 < dealt128 ? TilesCost{DenseTiles::kDealt256, dealt256} : TilesCost{DenseTiles::kDealt128, dealt128};
+}
+
 // When row blocks are taken (more than 32 rows).  Measured against the tiles of exl3_gemm_kernel.cuh at 4 bits,
 // 40..511 rows (K x N, us, tiles -> row blocks):
 //   * enough steps that the second launch and the hand-over pay: one per compute unit up to 64 rows (512x4096 14.0 ->
 //     14.7, 512x16384 20.4 -> 19.1, 4096x4096 23.5 -> 21.0), 2.25 of them above (4096x4096 at 100 rows 24.8 -> 27.0,
 //     7296x2688 33.8 -> 28.4);
 //     Fewer are enough of deep weights, whose 32-row tiles share a tile between many workgroups, for up to two blocks of
-//     96 rows (not for the last few rows of a third tile of sixteen): 48 steps at 36 / 64 / 96 rows of 3072x512 16.8 / 17.5 / 18.4 -> 14.4 / 15.1 / 16.5, 4096x1024 20.6 / 21.9 /
-//     22.9 -> 15.5 / 16.9 / 19.1, 8192x512 26.6 / 28.3 / 28.6 -> 18.8 / 20.4 / 23.6, at 160 rows 29.9 -> 26.6; but 3072x256
-//     at 80 rows 17.2 -> 18.1, 2048x2048 at 36 / 96 rows 17.3 / 19.6 -> 16.6 / 19.8, 1024x2048 13.0 / 14.8 -> 15.6 / 17.7,
-//     4864x1536 at 112 rows 24.3 -> 26.4.
+//     96 rows (not for the last few rows of a third tile of sixteen): 48 steps at 36 / 64 / 96 rows of 3072x512 16.8 / 17.5 /
+//     18.4 -> 14.4 / 15.1 / 16.5, 4096x1024 20.6 / 21.9 / 22.9 -> 15.5 / 16.9 / 19.1, 8192x512 26.6 / 28.3 / 28.6 -> 18.8 / 20.4 /
+//     23.6, at 160 rows 29.9 -> 26.6; but 3072x256 at 80 rows 17.2 -> 18.1, 2048x2048 at 36 / 96 rows 17.3 / 19.6 -> 16.6 /
+//     19.8, 1024x2048 13.0 / 14.8 -> 15.6 / 17.7, 4864x1536 at 112 rows 24.3 -> 26.4.  Bundles of several inputs, whose
+//     copies in operand order are several as well, want 300 of two blocks (174 rows of 5120 x (384, 128, 128), 200 steps:
+//     23.4 -> 26.5; 155 rows of 4096 x (1536, 256, 256), 512: 28.9 -> 25.9).
 //   * narrow outputs, which would run as 32-row tiles and decode every weight once per 32 rows: always (17408x5120 at
-//     64, 128, 256 and 384 rows 59, 88, 162, 167 -> 32, 46, 72, 100), up to gemm_block_rows;
-//   * wide outputs: a launch of 128-row or 256-row tiles costs the same for any rows up to a multiple of those, row
-//     blocks go by the row (blocks_beside_wide_tiles).
-static bool blocks_beside_wide_tiles(const Workspace& ws, int codebook, long nblocks, int size_m, const BlockPlan& pl, unsigned long long steps)
+//     64, 128, 256 and 384 rows 59, 88, 162, 167 -> 32, 46, 72, 100), of 449 rows and more where they cost less
+//     (narrow_blocks_cost), up to gemm_block_rows;
+//   * wide outputs: one row block (5120x34816 at 64 rows 62 -> 51, at 128 rows even) and several of up to 96 rows (160
+//     rows 112 -> 104); several of more where they cost less than 128-row or 256-row tiles, a launch of which costs the
+//     same for any rows up to a multiple of those (blocks_beside_wide_tiles, wide_blocks_cost).
+
+// what a step costs beyond MUL1's, whose decode is the shortest
+static long block_decode(int codebook, long mcg, long inst3) { return codebook == 1 ? mcg : codebook == 0 ? inst3 : 0; }
+// whether some tile is shared by ranges of steps that are no parts of it
+static bool uneven_ranges(const BlockPlan& pl) { return !pl.S && (pl.rem || pl.q % pl.spt); }
+static long longest_range(const BlockPlan& pl) { return pl.S ? (pl.spt + pl.S - 1) / pl.S : pl.q + (pl.rem ? 1 : 0); }
+
+// Several row blocks of more than 96 rows, in cheapest_tiles' unit: a step goes by the block's rows, the copies of the
+// input by their elements (in millions), a finished tile 3.4 us; the launch that finishes shared tiles, with the stores and
+// the uneven end that come with it, 13 us.  Fitted to 1700 linears and bundles (129..511 rows, 2..6 bits, K 256 .. 17408, up
+// to 32768 columns) for the choice beside cheapest_tiles.
+static long wide_blocks_cost(const Workspace& ws, int codebook, int slabs, int size_m, int size_k, const BlockPlan& pl, long tiles)
 {
-    // One row block (5120x34816 at 64 rows 62 -> 51, at 128 rows even) and several of up to 96 rows (160 rows 112 -> 104).
-    if (pl.row_blocks == 1 || pl.rows_per_tile <= 96 || !fills_128_row_tiles(ws, nblocks, size_m)) return true;
-    const long tiles = nblocks * ((size_m + 127) / 128), cus = ws.cu_count;
+    return 240 + 110 * slabs * ((long)size_m * size_k >> 10) / 1024 + longest_range(pl) * (28 * pl.mt - 16 + block_decode(codebook, 24, 35)) +
+           (pl.S || uneven_ranges(pl) ? 1340 : 0) + 338 * tiles / ws.cu_count;
+}
+
+// Four row blocks beside 32-row tiles, likewise: 650 launches of 449..511 rows.  32-row tiles cost by the k-blocks of a
+// workgroup, nearly twice as much where more than one of them comes to a compute unit, and by the rows of the output;
+// row blocks also by the partial tiles that they leave.  511 rows of 3072x2048, 256 tiles on 256 compute units, 29.2 -> 31.0,
+// 450 rows, 360 tiles, 33.0 -> 29.6; 505 rows of 2304 x (1536, 256, 256) 28.2 -> 35.8; 468 rows of 8192x1024 51.9 -> 37.0.
+// Of 187 launches 14 were slower as row blocks; from 3 % below none of the 146 that are left.
+static long narrow_blocks_cost(int codebook, int slabs, int size_m, int size_k, const BlockPlan& pl, long tiles)
+{
+    const long parts = pl.S ? tiles * pl.S : uneven_ranges(pl) ? std::min<long>(pl.grid + tiles, 2l * pl.grid) : 0;
+    return 430 + 144 * slabs * ((long)size_m * size_k >> 10) / 1024 + longest_range(pl) * (16 * pl.mt + block_decode(codebook, 25, 32)) +
+           parts * pl.mt * 537 / 1000;
+}
+static long tiles_of_32_rows_cost(const Workspace& ws, int codebook, long nblocks, int size_m, int size_k, long columns)
+{
+    const long KB = size_k / 128, tiles = nblocks * ((size_m + 31) / 32), S = gemm_split(ws, tiles, (int)KB, 1);
+    return (KB + S - 1) / S * (126 + (tiles * S > ws.cu_count ? 110 : 0) + block_decode(codebook, 12, 43)) + 62 * S +
+           247 * (size_m * columns >> 10) / 1024;
+}
+
+static bool blocks_beside_wide_tiles(const Workspace& ws, int codebook, long nblocks, int size_m, const BlockPlan& pl)
+{
+    const long tiles128 = nblocks * ((size_m + 127) / 128), cus = ws.cu_count, steps = pl.units;
     // (1024x6144 at 300 and 448 rows, 2.25 and 3 steps a compute unit: 26.2 -> 28.4, 27.2 -> 31.0)
-    if (steps < 4ull * (unsigned)cus) return false;
+    if (steps < 4 * cus) return false;
     // 3INST and MCG decode a weight in 4.4 instead of 3.6 instructions, and row blocks decode it more often: where
     // tiles are few (MCG, K 5120: 200, 256, 336 and 448 rows x 8192 50.6 -> 40.7, 49.5 -> 42.4, 58.2 -> 55.3, 68.8 -> 55.5,
     // but 336 x 17408 94 -> 97, 200 x 34816 110 -> 119; 3INST 256 rows 2048x12288 39.0 -> 39.7)
-    if (codebook != 2) return tiles <= (pl.rows_per_tile > 112 ? cus / 4 : cus / 2);
+    if (codebook != 2) return tiles128 <= (pl.rows_per_tile > 112 ? cus / 4 : cus / 2);
     // Blocks of 128 rows where whole 128-row tiles would fill half of the chip at most and the second launch pays
     // (256 rows, K 5120 x 8192, 64 tiles: 47.4 -> 41.2; 2048x16384, 128 tiles and eight steps a compute unit: 39.1 -> 28.2;
     // 2048x12288, 96 tiles and six steps: 36.5 -> 37.7; 384 rows of 5120x12288, 144 tiles: 74.8 -> 80).
     // Four of them (449..511 rows) where a workgroup has one tile or a part of one: 8192x4096 61.5 -> 55.0, 3072x8192 48.3 ->
     // 37.6, but 6144x5120, ranges across tiles, 58.2 -> 58.8.
     if (pl.rows_per_tile > 112)
-        return tiles <= cus / 2 && steps >= 8ull * (unsigned)cus && steps <= 32ull * (unsigned)cus &&
-               (pl.row_blocks <= 3 || 4 * tiles <= cus || 2 * tiles % cus == 0);
+        return tiles128 <= cus / 2 && steps >= 8 * cus && steps <= 32 * cus &&
+               (pl.row_blocks <= 3 || !uneven_ranges(pl));
     // Of 112: two blocks (200 rows, K 5120 x 8192, 17408, 34816: 47.5 -> 37.3, 69.7 -> 63.1, 114 -> 113); three beside less than
     // half a chip or more than a whole of tiles (336 rows x 8192, 17408, 25600, 34816: 57.3 -> 53.5, 91.3 -> 92.0, 134 ->
     // 128, 175 -> 166); four, which leave little of the second 256 rows empty, beside up to a whole one and up to 32 steps a
     // compute unit (448 rows x 8192, 12288, 25600: 67 -> 53.5, 86.4 -> 81.7, 155 -> 164; 17408x5120, 42.5 steps: 123 -> 133).
-    return pl.row_blocks == 2 || (pl.row_blocks == 3 ? tiles <= cus / 2 || tiles > cus : tiles <= cus && steps <= 32ull * (unsigned)cus);
+    return pl.row_blocks == 2 || (pl.row_blocks == 3 ? tiles128 <= cus / 2 || tiles128 > cus : tiles128 <= cus && steps <= 32 * cus);
 }
 
-static BlockPlan plan_block(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n)
+// activation: the launch that finishes gate's and up's tiles forms an MLP's activation too, which tiles leave to one more
+static bool blocks_beside_tiles(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n,
+                                const BlockPlan& pl, bool activation)
+{
+    const long nblocks = (long)slices * ((size_n + 255) / 256), tiles = (long)slices * (size_n / 128) * pl.row_blocks;
+    if (!fills_128_row_tiles(ws, nblocks, size_m))
+        return activation || pl.row_blocks < 4 || pl.mt < 8 ||
+               narrow_blocks_cost(codebook, slabs, size_m, size_k, pl, tiles) * 33 <=
+                   tiles_of_32_rows_cost(ws, codebook, nblocks, size_m, size_k, (long)slices * size_n) * 32;
+    // One row block (5120x34816 at 64 rows 62 -> 51, at 128 rows even) and several of up to 96 rows (160 rows 112 -> 104).
+    if (pl.row_blocks == 1 || pl.rows_per_tile <= 96) return true;
+    if (!blocks_beside_wide_tiles(ws, codebook, nblocks, size_m, pl)) return false;
+    if (activation) return true;
+    // Of these the ones whose ranges across tiles are no longer than 32 steps, where the row blocks of a column block come at
+    // different times and each brings its weights in again (13568x6016 at 410 rows, MCG, 128 -> 134; 17408x8064 at 450, 172 ->
+    // 227), and that cost 2 % less than tiles: of 470 launches 56 were slower than tiles, 4 of the 320 that are left, by 6 % at most:
+    // 640x12288 at 385 rows 21.9 -> 35.8, 1024x29312 at 224 29.9 -> 41.4, 1152x15872 at 435 33.9 -> 42.7, 2304 x ten slices of
+    // 1024 at 418 47.2 -> 52.1.
+    if (uneven_ranges(pl) && longest_range(pl) > 32) return false;
+    const Knobs& kn = knobs();
+    const long best = cheapest_tiles(ws.cu_count, codebook, size_k / 128, nblocks * ((size_m + 127) / 128), nblocks * ((size_m + 255) / 256),
+                                     kn.gemm_balanced == 1, kn.gemm_rows256 > 0).cost;
+    return wide_blocks_cost(ws, codebook, slabs, size_m, size_k, pl, tiles) * 50 <= best * 49;
+}
+
+static BlockPlan plan_block(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n, bool activation)
 {
     BlockPlan pl;
     if (!knobs().gemm_balanced || size_m <= 32 || size_m > knobs().gemm_block_rows || size_n % 128 != 0) return pl;
@@ -274,8 +375,8 @@ static BlockPlan plan_block(const Workspace& ws, int codebook, int slices, int s
     if (U >= (1ull << 30)) return pl;
     const int least = knobs().gemm_block_steps;
     const bool deep = size_m >= 36 && pl.rows_per_tile <= 96 && (pl.row_blocks == 1 ? size_k >= 3072 : pl.row_blocks == 2 && size_k >= 3584);
-    if (U < (unsigned long long)(least >= 0 ? least : deep ? 48 : size_m <= 64 ? 256 : 576)) return pl;
-    if (least < 0 && !blocks_beside_wide_tiles(ws, codebook, (long)slices * ((size_n + 255) / 256), size_m, pl, U)) return pl;
+    const int deep_least = slabs > 1 && pl.row_blocks > 1 && !activation ? 300 : 48;
+    if (U < (unsigned long long)(least >= 0 ? least : deep ? deep_least : size_m <= 64 ? 256 : 576)) return pl;
     unsigned long long G = (unsigned long long)ws.cu_count;
     if (G > U) G = U;
     unsigned q = (unsigned)(U / G), rem = (unsigned)(U % G), S = 0;
@@ -293,13 +394,14 @@ static BlockPlan plan_block(const Workspace& ws, int codebook, int slices, int s
     pl.operand_at = (size_t)G * 2 * pl.rows_per_tile * 512;
     pl.operand_stride = (size_t)pl.row_blocks * rows_operand_elements(size_k, pl.rows_per_tile / 16);
     if (pl.operand_at + slabs * pl.operand_stride * 2 > ws.partial_bytes) return pl;
-    pl.ok = true;
     pl.units = (long)U;
     pl.grid = (unsigned)G;
     pl.q = q;
     pl.rem = rem;
     pl.S = S;
     pl.spt = spt;
+    if (least < 0 && !blocks_beside_tiles(ws, codebook, slices, slabs, size_m, size_k, size_n, pl, activation)) return BlockPlan{};
+    pl.ok = true;
     return pl;
 }
 
@@ -340,9 +442,9 @@ static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebo
 struct OperandPlan {
     RowsPlan rows;
     BlockPlan block;
-    OperandPlan(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n)
+    OperandPlan(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n, bool activation = false)
         : rows(plan_rows(ws, slices, slabs, size_m, size_k, size_n)),
-          block(rows.ok ? BlockPlan{} : plan_block(ws, codebook, slices, slabs, size_m, size_k, size_n))
+          block(rows.ok ? BlockPlan{} : plan_block(ws, codebook, slices, slabs, size_m, size_k, size_n, activation))
     {
         stride = rows.ok ? rows_operand_elements(size_k, rows.mt) : block.operand_stride;
         at = (_Float16*)((char*)ws.partials + (rows.ok ? rows.operand_at : block.operand_at));
@@ -357,41 +459,6 @@ struct OperandPlan {
     _Float16* at = nullptr;     // the first slab's copy
     size_t stride = 0;          // elements between slabs
 };
-
-// How a dense launch of 128-row tiles or larger is cut up.  Whole tiles: a workgroup of four waves per
-// 128 x 256 tile, two of them on a compute unit.  Dealt out: one workgroup per compute unit with an even
-// share of the (tile, k-block) units, the workgroups of a shared tile adding their parts in k order;
-// of 128-row tiles, or of 256-row tiles (eight waves, every weight decoded once per 256 rows).
-enum class DenseTiles { kWhole128, kDealt128, kDealt256 };
-
-// The cheapest by what a compute unit spends, in 10 ns: k-blocks, the epilogue of every tile, and the
-// hand-over of shared ones, which takes longer the more workgroups share a tile.
-//   * Whole tiles hide part of an epilogue behind the other workgroup's k-loop, but come in rounds; a
-//     round with r of its tiles takes about (1 + r) / 2 of a full one, the first a whole one.
-//   * Dealt-out tiles have no partial round; their epilogue and hand-over are in nobody's shadow.  So a
-//     short K, where those weigh against few k-blocks, takes whole tiles, and a long one is dealt out.
-//   * The decode of 128-row tiles does not quite fit behind their MFMAs, so a k-block costs more with the
-//     codebooks of longer decode; with 256-row tiles it does fit (6144 columns of 4096 at 1500 rows, dealt 128 /
-//     dealt 256 us: MUL1 108/105, MCG 112/103, 3INST 123/105; the bit rate matters less).
-// Fitted to 499 launches at 4 bits (K 128 .. 10240, 2048 .. 32768 columns, 460 .. 1500 rows): the choice costs
-// 0.7 % over the fastest of the three on average, 14 % at most.  Examples, K x N at rows: whole / dealt
-// 128 / dealt 256 us: 256x8192 at 512 16/26/31, 512x16384 at 1500 46/59/59, 1024x4096 at 512 27/31/50,
-// 1024x16384 at 1500 72/88/81, 2048x4096 at 512 43/36/54, 2048x16384 at 1024 87/96/83, 5120x12288 at 600
-// 99/106/121, 4096x16384 at 600 128/111/122 and at 1500 231/254/225.
-static DenseTiles cheapest_tiles(long cus, int codebook, long KB, long tiles128, long tiles256, bool whole_allowed, bool wide_allowed)
-{
-    const long whole_kb = codebook == 0 ? 250 : codebook == 1 ? 236 : 230;
-    const long dealt_kb = codebook == 0 ? 260 : codebook == 1 ? 243 : 235;
-    const long n = tiles128 / cus, r = tiles128 % cus;          // full rounds, tiles of the last one
-    const long m = tiles256 / cus, s = tiles256 % cus;
-    // (one workgroup on a compute unit has no other to hide its epilogue behind)
-    const long whole = n == 0 || tiles128 == cus ? KB * whole_kb + 500 + 400 * tiles128 / cus
-                                                 : (2 * n * cus + (r ? cus + r : 0)) * (KB * whole_kb + 500) / (2 * cus);
-    const long dealt128 = tiles128 * KB * dealt_kb / cus + 800 * n + (r == 0 ? 0 : n ? 800 : 2500 - 1600 * r / cus);
-    const long dealt256 = tiles256 * KB * 415 / cus + 900 * m + (s == 0 ? 0 : m ? 1900 : 3700 - 2200 * s / cus);
-    if (whole_allowed && whole < dealt128 && (!wide_allowed || whole <= dealt256)) return DenseTiles::kWhole128;
-    return wide_allowed && dealt256 < dealt128 ? DenseTiles::kDealt256 : DenseTiles::kDealt128;
-}
 
 // Tile shape and work split of a dense launch: `nblocks` column blocks of 256 (all slices of
 // a bundle together), size_m rows.  Fills the split fields of p and launches.
@@ -433,7 +500,7 @@ static void dispatch_dense(const Workspace& ws, GemmParams& p, int k_bits, int c
     bool whole = false;
     if (mb_plain == 4 && balance) {
         const long tiles128 = (long)nblocks * ((size_m + 127) / 128), tiles256 = (long)nblocks * ((size_m + 255) / 256);
-        const DenseTiles cheapest = cheapest_tiles(ws.cu_count, codebook, KB, tiles128, tiles256, balance == 1, rows256 > 0 && size_m > 128);
+        const DenseTiles cheapest = cheapest_tiles(ws.cu_count, codebook, KB, tiles128, tiles256, balance == 1, rows256 > 0 && size_m > 128).tiles;
         const bool wide = size_m > 128 && (rows256 >= 2 || cheapest == DenseTiles::kDealt256);
         if (wide && balanced(8)) return;
         whole = cheapest == DenseTiles::kWhole128;
@@ -639,7 +706,7 @@ std::string launch_gemm_pair(const PairArgs& a, void* a_had_second, PairNext* ne
     if (!scratch) scope.emplace(a.stream);
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
-    const OperandPlan plan(ws, a.codebook, 2, 2, a.size_m, a.size_k, a.size_n);
+    const OperandPlan plan(ws, a.codebook, 2, 2, a.size_m, a.size_k, a.size_n, next != nullptr);
     RowsPairParams p{};
     p.fault = ws.fault_dev;
     p.spin_limit = spin_limit();

@@ -102,6 +102,36 @@ def test_the_rule_of_deep_weights(rows, Kk, N, cb, blocks):
     assert bad == 0, (bad, worst, launch)
 
 
+@pytest.mark.parametrize("rows,Kk,N,blocks", [
+    (385, 640, 12288, False),           # three steps a tile, in ranges across tiles
+    (450, 2304, 8064, False),           # ranges across tiles, in as many row blocks as 8192 columns in whole tiles have
+    (511, 3072, 2048, False),           # beside one round of 32-row tiles
+    (450, 3072, 2048, True),            # beside one and a half
+    (505, 2304, (1536, 256, 256), False),
+    (174, 5120, (384, 128, 128), False),        # 200 steps of deep weights, three inputs
+    (155, 4096, (1536, 256, 256), True),        # 512
+])
+def test_several_row_blocks_only_where_they_cost_less(rows, Kk, N, blocks):
+    """Launches of several row blocks that tiles are quicker for, and their neighbours, each against the oracle."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rule goes by the compute units")
+    with knobs(BERTH_GEMM_BLOCK_ROWS=511, BERTH_GEMM_BLOCK_STEPS=-1):
+        if isinstance(N, int):
+            got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, 2, 2, True, 270 + rows, prefill=True)
+            assert np.array_equal(ah, want_ah) and close(got, want)[0] == 0, launch
+        else:
+            from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
+            gpu, lins = Gpu(0), [synth.linear(660 + i, Kk, n, 2) for i, n in enumerate(N)]
+            x, outs = synth.activations(670 + rows, rows, Kk), [torch.zeros((rows, n), dtype=torch.float16, device=DEV) for n in N]
+            Exl3MultiLinear(gpu, [Exl3Linear(gpu, f"l{i}", *lin) for i, lin in enumerate(lins)]).forward(
+                gpu, dev(x.view(np.uint16)), outs, OutDtype.F16, rows)
+            torch.cuda.synchronize()
+            launch = K.ops.last_launch()
+            for out, lin, n in zip(outs, lins, N):
+                assert close(host_f16(out), O.linear(x, *lin, Kk, n, 2, 2, out_fp32=False)[0])[0] == 0, launch
+    assert ("exl3_gemm_block_kernel" in launch) == blocks, launch
+
+
 @pytest.mark.parametrize("rows,unit", [(40, 128), (150, 128), (70, 0)])
 def test_bundle_with_narrower_slices(rows, unit):
     """Sliced lists whose widths differ: blocks past a slice's end are empty and touch nothing.  unit 0: four slices of one
