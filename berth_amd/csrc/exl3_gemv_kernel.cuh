@@ -297,36 +297,35 @@ __global__ __launch_bounds__(256, 4) void exl3_gemv_kernel(GemvParams p)
         // of the segment sums, which every workgroup of the launch wants at the same moment
         // (measured: 1.2 us off the layer against all four waves doing it side by side).
         // The records of this launch's linear of all experts (at most 128: lane l holds experts l and l + 64) are asked
-        // for behind the segment sums, so that the weights are one dependent read away from the answer.
+        // for behind the segment sums, ahead of the selection, so that the weights are one dependent read away from the
+        // answer.  Not with the segment sums, and not the next launch's records by the same wave: 92 registers leave room for
+        // five workgroups on a compute unit, 120 for four, and launches of four to five a compute unit then come in two
+        // rounds.  gate + up, us, records behind the answer / with the sums / as it is: 1260 workgroups of 3584x1280 20.5 /
+        // 24.9 / 21.0, 1210 of 2304x1408 20.4 / 24.1 / 21.0, 1600 of 4096x2048 39.1 / 39.7 / 39.0, 1536 of 4096x1536 31.8 / 30.3 /
+        // 30.4, 768 of 2048x768 13.6 / 12.6 / 12.8, 256 of 1024x512 11.3 / 10.7 / 10.8.
         __shared__ __align__(8) unsigned s_lin[6];
+        __shared__ int s_sel[64], s_rank[64];
+        auto ask_record = [&](const int i, const int which_lin, unsigned (&to)[6]) {
+            const int e2 = min(lane + 64 * i, p.route.E - 1);
+            const global_ptr<const unsigned> src = as_global((const unsigned*)(p.experts + e2 * p.lins_per_expert + which_lin));
+#pragma unroll
+            for (int q = 0; q < 6; ++q) to[q] = src[q];
+        };
+        // The first workgroup's first wave stores the routing results.  Its second leaves, for
+        // the launch that follows, the record of linear `resolved_lin` of the expert at
+        // each sorted position (then of the always-on expert), so that that launch reaches
+        // its weights with one dependent read instead of two.  It asks for the records of
+        // all experts while the first works the routing out.
+        const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
+        const bool resolve = writer && p.resolved_out && wave == 1;
+        unsigned next[2][6];
         if (wave == 0) {
-            // The first workgroup's first wave stores the routing results.  It also leaves, for
-            // the launch that follows, the record of linear `resolved_lin` of the expert at
-            // each sorted position (then of the always-on expert), so that that launch reaches
-            // its weights with one dependent read instead of two.  It asks for the records of
-            // all experts ahead of the
-            // routing too, so that its stores do not wait for a read that depends on the routing.
-            const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
-            const bool resolve = writer && p.resolved_out;
-            unsigned rec[2][6];
-            if (resolve) {
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int e2 = min(lane + 64 * i, p.route.E - 1);
-                    const unsigned* src = (const unsigned*)(p.experts + e2 * p.lins_per_expert + p.resolved_lin);
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) rec[i][q] = src[q];
-                }
-            }
             unsigned mine[2][6];
             const RouteOneToken r = route_one_token(p.route, lane, writer, [&]() {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     if (i == 1 && p.route.E <= 64) break;
-                    const int e2 = min(lane + 64 * i, p.route.E - 1);
-                    const global_ptr<const unsigned> src = as_global((const unsigned*)(p.experts + e2 * p.lins_per_expert + p.lin_base + which));
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) mine[i][q] = src[q];
+                    ask_record(i, p.lin_base + which, mine[i]);
                 }
             });
             const int e = route_expert_at(p.route, r, lane, prob);
@@ -340,23 +339,29 @@ __global__ __launch_bounds__(256, 4) void exl3_gemv_kernel(GemvParams p)
                     s_lin[q] = e >= 64 ? hi : lo;
                 }
             }
-            if (resolve) {
-                unsigned got[6];
+            s_sel[lane] = r.sel;
+            s_rank[lane] = r.rank;
+        } else if (resolve) {
 #pragma unroll
-                for (int q = 0; q < 6; ++q) {
-                    const unsigned lo = (unsigned)__shfl((int)rec[0][q], r.sel & 63, 64);
-                    const unsigned hi = (unsigned)__shfl((int)rec[1][q], r.sel & 63, 64);
-                    got[q] = r.sel >= 64 ? hi : lo;
-                }
-                if (lane < p.route.k) {
-                    unsigned* dst = (unsigned*)(p.resolved_out + r.rank);
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) dst[q] = got[q];
-                }
-                if (lane == 0 && p.shared_expert >= 0) p.resolved_out[p.route.k] = p.shared[p.resolved_lin];
-            }
+            for (int i = 0; i < 2; ++i) ask_record(i, p.resolved_lin, next[i]);
         }
         __syncthreads();
+        if (resolve) {
+            const int sel = s_sel[lane];
+            unsigned got[6];
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                const unsigned lo = (unsigned)__shfl((int)next[0][q], sel & 63, 64);
+                const unsigned hi = (unsigned)__shfl((int)next[1][q], sel & 63, 64);
+                got[q] = sel >= 64 ? hi : lo;
+            }
+            if (lane < p.route.k) {
+                unsigned* dst = (unsigned*)(p.resolved_out + s_rank[lane]);
+#pragma unroll
+                for (int q = 0; q < 6; ++q) dst[q] = got[q];
+            }
+            if (lane == 0 && p.shared_expert >= 0) p.resolved_out[p.route.k] = p.shared[p.resolved_lin];
+        }
         unsigned rec[6];
 #pragma unroll
         for (int q = 0; q < 6; ++q) rec[q] = (unsigned)__builtin_amdgcn_readfirstlane((int)s_lin[q]);

@@ -226,14 +226,14 @@ __device__ __forceinline__ void route_sort_one_token(const PermuteParams& q, int
 // order, bias), top-k, and the sorted position of every selected expert (lane j < k: expert of
 // slot j and its sorted position).  Every wave that calls this gets the same bits; the wave
 // with `writer` set also stores the routing results (logits, idx, w, and what the sort of the
-// one token writes).  `requested` is called when the reads are on their way.
+// one token writes).  `summed` is called ahead of the selection.
 struct RouteOneToken {
     int sel;
     int rank;
 };
 
 template <typename F>
-__device__ __forceinline__ RouteOneToken route_one_token(const RouteParams& p, int lane, bool writer, F requested)
+__device__ __forceinline__ RouteOneToken route_one_token(const RouteParams& p, int lane, bool writer, F summed)
 {
     float lg[kRoutePer];
 #pragma unroll
@@ -251,12 +251,9 @@ __device__ __forceinline__ RouteOneToken route_one_token(const RouteParams& p, i
 #pragma unroll
             for (int j = 0; j < 32; ++j) part[i][j] = as_global(p.parts + (size_t)min(s0 + j, p.nseg - 1) * p.E)[at[i]];
         }
-        if (s0 == 0) {
-            if (p.bias) {
+        if (s0 == 0 && p.bias) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) bias[i] = as_global(p.bias)[at[i]];
-            }
-            requested();
+            for (int i = 0; i < 2; ++i) bias[i] = as_global(p.bias)[at[i]];
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -268,6 +265,7 @@ __device__ __forceinline__ RouteOneToken route_one_token(const RouteParams& p, i
             }
         }
     }
+    summed();
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int e = lane + 64 * i;

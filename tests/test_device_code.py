@@ -216,17 +216,30 @@ def test_the_same_of_the_fused_launches(tmp_path, kernels, params):
     test_matrix_instructions_keep_their_distance_from_inline_assembly(tmp_path, kernels, ("exl3_gemm_rows_kernel.cuh",), params)
 
 
+def _registers(tmp_path, kernels, headers, params="GemmParams"):
+    """(vector registers, scratch bytes a lane) of each kernel"""
+    found = {}
+    for entry in _assembly(tmp_path, kernels, headers, params).split("  - .agpr_count:")[1:]:
+        found[re.search(r"\.name:\s+(\S+)", entry)[1]] = tuple(int(re.search(rf"\.{key}:\s+(\d+)", entry)[1])
+                                                                for key in ("vgpr_count", "private_segment_fixed_size"))
+    assert len(found) == len(kernels)
+    return found
+
+
 def test_grouped_tiles_of_one_block_leave_room_for_four_workgroups(tmp_path):
     """Four workgroups of four waves on a compute unit: at most 128 of a SIMD's 512 registers a lane, and no scratch.
     (8 bits outside the pair kernel and MUL1 above 6 take three.)"""
     kernels = ([f"exl3_gemm_pair_kernel<{bits}, {cb}>" for bits, cb in ((3, 0), (4, 0), (4, 1), (4, 2), (8, 0))] +
                [f"exl3_gemm_kernel<{bits}, {cb}, 1, false>" for bits, cb in ((3, 0), (3, 1), (3, 2), (4, 0), (7, 1))])
-    found = {}
-    for entry in _assembly(tmp_path, kernels, ("exl3_gemm_kernel.cuh",)).split("  - .agpr_count:")[1:]:
-        found[re.search(r"\.name:\s+(\S+)", entry)[1]] = tuple(int(re.search(rf"\.{key}:\s+(\d+)", entry)[1])
-                                                                for key in ("vgpr_count", "private_segment_fixed_size"))
-    assert len(found) == len(kernels)
+    found = _registers(tmp_path, kernels, ("exl3_gemm_kernel.cuh",))
     assert {name: at for name, at in found.items() if at[0] > 128 or at[1]} == {}
+
+
+def test_one_token_gate_and_up_leave_room_for_five_workgroups(tmp_path):
+    """The one-token launch that works the routing out: at most 96 registers up to 5 bits, and no scratch."""
+    kernels = [f"exl3_gemv_kernel<{bits}, {cb}, 1, false, {trs}, true>" for bits, cb, trs in ((2, 2, 8), (4, 0, 8), (4, 2, 4), (5, 1, 8))]
+    found = _registers(tmp_path, kernels, ("exl3_gemv_kernel.cuh",), "GemvParams")
+    assert {name: at for name, at in found.items() if at[0] > 96 or at[1]} == {}
 
 
 def test_every_tile_of_a_mixed_launch_is_taken_once(tmp_path):
