@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256, 4) void exl3_gemv_kernel(GemvParams p)
             });
             const int e = route_expert_at(p.route, r, lane, prob);
             if (e == p.shared_expert) {
-                if (lane == 0) *(ExpertLin*)s_lin = p.shared[p.lin_base + which];
+                if (lane == 0) __builtin_memcpy(s_lin, &p.shared[p.lin_base + which], sizeof(ExpertLin));
             } else {
 #pragma unroll
                 for (int q = 0; q < 6; ++q) {
