@@ -868,6 +868,7 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         if (g.max_problems > 65535) throw std::runtime_error("moe grouped linear: too many problems");
         p.act_had = (_Float16*)g.act_had;
         p.group_lins = 1;
+        p.ramp_problems = 6 * ws.cu_count / (g.size_n / 128);
         std::string desc;
         gemm_bits(p, g.k_bits, g.codebook, -4, g.stream, desc, group_grid(g.size_n / 128, 1, g.max_problems));
         hip_ok(hipGetLastError(), "exl3_gemm_pair_kernel launch");
@@ -894,6 +895,7 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         hip_ok(hipGetLastError(), "exl3_gemm_mixed_kernel launch");
         return desc + " grouped";
     }
+    p.ramp_problems = 4 * ws.cu_count / (nblocks * p.S * g.num_lins);
     gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, group_grid(nblocks * p.S, g.num_lins, g.max_problems));
     hip_ok(hipGetLastError(), "exl3_gemm_kernel grouped launch");
     return desc + " grouped";

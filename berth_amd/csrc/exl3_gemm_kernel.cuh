@@ -110,6 +110,7 @@ struct GemmParams {
     const int32_t* a_rows;
     int group_lins;             // linears of a problem that are units of their own (1 or 2)
     int places;                 // exl3_gemm_mixed_kernel: workgroups that run at a time; tiles run as halves of 128 columns up to this many
+    int ramp_problems;          // grouped 32-row tiles: PriorityRamp up to this many problems
     _Float16* act_had;          // exl3_gemm_pair_kernel: the down projection's rotated input, in sorted order
 };
 
@@ -223,19 +224,25 @@ constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: 
 // The waves of a SIMD run nearly oldest first, so that the last ones end alone, with nobody to fill the cycles that they
 // wait.  A wave gives up its priority in three steps over its second half, which lets the ones behind it catch up.
 // Grouped launches of 32-row problems, layers of 2048 x 768: 64 tokens x 128 experts 104.8 -> 102.7 us, with popular
-// ones 80.2 -> 77.3, 20 tokens 96.0 -> 92.8, 100 tokens x 64 experts 77.2 -> 74.9; 512 experts at 64 tokens, whose
-// workgroups come in six rounds, 175 either way.  Not in mixed launches, whose long tiles have to end first (256
+// ones 80.2 -> 77.3, 20 tokens 96.0 -> 92.8, 100 tokens x 64 experts 77.2 -> 74.9.  Only where the workgroups there are come
+// in one round of four a compute unit, of gate and up together in one and a half: those of a later round start ahead
+// of the ones that give way, which end the later (down, traced: 128 tokens x 512 experts of 768x2048, 3760 workgroups, 122 ->
+// 133 us, 64 tokens x 160 of 1664x4096, 2500, 195 -> 207, 40 tokens x 64 of 2048x7168, 1790, 148 -> 155; gate and up of
+// 128 tokens x 512 experts, 2820, 245 -> 257, but 64 tokens x 512 experts x 512, 1470, 130 -> 122, 40 tokens x 64 of 7168x2048,
+// 1020, 295 -> 281).  Not in mixed launches, whose long tiles have to end first (256
 // tokens x 512 experts 113.8 -> 115.8), nor dense, which have few waves a SIMD (76 rows of 1152x3584 14.7 -> 14.8).
 template <bool ON>
 struct PriorityRamp {
     int k2, k1, k0, step;
-    __device__ __forceinline__ PriorityRamp(const int kb0, const int kb1, const int step_) : step(step_)
+    __device__ __forceinline__ PriorityRamp(const int kb0, const int kb1, const int step_, const bool on) : step(step_)
     {
         const int n = kb1 - kb0;
-        k2 = kb0 + (n >> 1);
-        k1 = kb0 + (n * 3 >> 2);
-        k0 = kb0 + (n * 7 >> 3);
-        if constexpr (ON) __builtin_amdgcn_s_setprio(3);
+        k2 = on ? kb0 + (n >> 1) : kb1;                 // (never reached)
+        k1 = on ? kb0 + (n * 3 >> 2) : kb1;
+        k0 = on ? kb0 + (n * 7 >> 3) : kb1;
+        if constexpr (ON) {
+            if (on) __builtin_amdgcn_s_setprio(3);
+        }
     }
     // ahead of the k-block kb of kb0, kb0 + step, ...
     __device__ __forceinline__ void at(const int kb) const
@@ -260,11 +267,11 @@ struct PriorityRamp {
 // them it lands in other registers and is moved, 16 of the 513 vector instructions of a k-block.  Layers of 64
 // and 20 tokens x 128 experts 120.7 -> 118.3 and 106.4 -> 104.3 us); on the last k-block the reload reads
 // the same addresses again and is ignored, which keeps the loop free of branches.
-// `requested` is called when the first loads are on their way; RAMP: PriorityRamp.
+// `requested` is called when the first loads are on their way; RAMP: PriorityRamp, where `ramp_on`.
 template <int BITS, int CB, bool RAMP, typename F>
 __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
                                                    const int arow, const int K, const int kb0, const int kb1, const int step,
-                                                   const int lane, float16_t (&acc)[2], F requested)
+                                                   const int lane, float16_t (&acc)[2], F requested, const bool ramp_on = false)
 {
     constexpr int tile_dw = 8 * BITS;
     const int half_id = lane >> 5, slot = lane & 31;
@@ -286,7 +293,7 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
         }
     }
     requested();
-    const PriorityRamp<RAMP> ramp(kb0, kb1, step);
+    const PriorityRamp<RAMP> ramp(kb0, kb1, step, ramp_on);
     for (int kb = kb0; kb < kb1; kb += step) {
         ramp.at(kb);
         const int nkb = kb + step < kb1 ? kb + step : kb;
@@ -332,7 +339,8 @@ __device__ __forceinline__ void accumulate_32_rows(const uint32_t* trellis, cons
 // loop more than the zeros save (that layer 104.2 -> 107.4, of 256 tokens x 512 experts 109.9 -> 112.9).
 template <int BITS, int CB, int CG, bool RAMP, typename F>            // CG: column groups of 32 a wave
 __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, const size_t row_dw, const int nw, const _Float16* a_had,
-                                                   const int arow, const int K, const int lane, float4_t (&acc)[CG][2], F requested)
+                                                   const int arow, const int K, const int lane, float4_t (&acc)[CG][2], F requested,
+                                                   const bool ramp_on = false)
 {
     constexpr int tile_dw = 8 * BITS;
     const int l16 = lane & 15, lg = lane >> 4;
@@ -353,7 +361,7 @@ __device__ __forceinline__ void accumulate_16_rows(const uint32_t* trellis, cons
     }
     requested();
     const int KB = K >> 7;
-    const PriorityRamp<RAMP> ramp(0, KB, 1);
+    const PriorityRamp<RAMP> ramp(0, KB, 1, ramp_on);
     for (int kb = 0; kb < KB; ++kb) {
         ramp.at(kb);
         const int nkb = min(kb + 1, KB - 1);
@@ -407,7 +415,8 @@ __device__ __forceinline__ void stage_16_rows(float* z, const float4_t (&acc)[CG
 // RAMP: PriorityRamp in tiles of up to 32 rows
 template <int BITS, int CB, int MB, bool DENSE, bool SCALAR = false, bool RAMP = false>
 __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y, const int nblk, const KRange kr,
-                                          const int which, unsigned char* smem, const GroupProblem* problems = nullptr)
+                                          const int which, unsigned char* smem, const GroupProblem* problems = nullptr,
+                                          const bool ramp_on = false)
 {
     constexpr int BM = MB * 32;
     _Float16* a_tile = (_Float16*)smem;                 // [2][BM][kAStride]
@@ -485,12 +494,12 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int tile_y,
     float4_t acc16[2][2] = {};
     if (lone) {
         if (active)
-            accumulate_16_rows<BITS, CB, 2, RAMP>(trellis, row_dw, nw, a_had, a_row_at(min(lane & 15, rows_here - 1)), p.K, lane, acc16, keep_scale);
+            accumulate_16_rows<BITS, CB, 2, RAMP>(trellis, row_dw, nw, a_had, a_row_at(min(lane & 15, rows_here - 1)), p.K, lane, acc16, keep_scale, ramp_on);
         else keep_scale();
     } else if constexpr (MB == 1) {
         if (active && kr.kb0 < kr.kb1)
             accumulate_32_rows<BITS, CB, RAMP>(trellis, row_dw, nw, a_had, a_row_at(min(slot, rows_here - 1)), p.K, kr.kb0, kr.kb1,
-                                         kr.step, lane, acc[0], keep_scale);      // (rows past the problem repeat its last row)
+                                         kr.step, lane, acc[0], keep_scale, ramp_on);      // (rows past the problem repeat its last row)
         else keep_scale();
     } else {
         // lane's trellis position inside a k-block: tile row 2*step + half_id, tile (nw/16 + slot/8)
@@ -848,11 +857,12 @@ __global__ __launch_bounds__(256, MB > 1 || DENSE ? 2 : CB != 2 && BITS < 8 ? 4 
         kr.slot0 = kr.slot_rest = kr.counter * p.S;
         gemm_tile<BITS, CB, MB, true>(p, tile / nblocks, tile % nblocks, kr, 0, smem);
     } else {
-        if (gt.problem >= *p.num_problems) return;
+        const int problems = *p.num_problems;
+        if (gt.problem >= problems) return;
         // grouped: (linear, problem, column block)
         kr.counter = ((size_t)gt.which * p.tiles_y + gt.problem) * nblocks + unit;
         kr.slot0 = kr.slot_rest = kr.counter * p.S;
-        gemm_tile<BITS, CB, MB, false, CB != 2, true>(p, gt.problem, unit, kr, gt.which, smem, p.problems);
+        gemm_tile<BITS, CB, MB, false, CB != 2, true>(p, gt.problem, unit, kr, gt.which, smem, p.problems, problems <= p.ramp_problems);
     }
 }
 
@@ -871,7 +881,9 @@ __global__ __launch_bounds__(256, CB != 2 ? 4 : 3) void exl3_gemm_pair_kernel(Ge
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const GroupTile gt = group_tile(p);
-    if (gt.problem >= *p.num_problems) return;
+    const int problems = *p.num_problems;
+    if (gt.problem >= problems) return;
+    const bool ramp_on = problems <= p.ramp_problems;
     constexpr int kZStride = 256 + 4;
     float* const z_tile = (float*)smem;                 // [32][kZStride]: gate's 128 columns, up's
     const int lane = threadIdx.x & 63, slot = lane & 31, half_id = lane >> 5;
@@ -903,7 +915,7 @@ __global__ __launch_bounds__(256, CB != 2 ? 4 : 3) void exl3_gemm_pair_kernel(Ge
     const int at = n0 + 8 * chunk;
     if (gp.lone) {
         float4_t acc[2][2] = {};
-        accumulate_16_rows<BITS, CB, 2, true>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, lane, acc, keep_scale);
+        accumulate_16_rows<BITS, CB, 2, true>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, lane, acc, keep_scale, ramp_on);
         stage_16_rows<kZStride>(z_tile + wave * 64, acc, lane);
     } else {
         float16_t acc[2];
@@ -911,7 +923,7 @@ __global__ __launch_bounds__(256, CB != 2 ? 4 : 3) void exl3_gemm_pair_kernel(Ge
         for (int f = 0; f < 2; ++f)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[f][r] = 0.0f;
-        accumulate_32_rows<BITS, CB, true>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, 0, p.K >> 7, 1, lane, acc, keep_scale);
+        accumulate_32_rows<BITS, CB, true>(lin.trellis, row_dw, nw, p.a_had[which], arow, p.K, 0, p.K >> 7, 1, lane, acc, keep_scale, ramp_on);
         const int col = wave * 64 + (slot >> 3) * 16 + (slot & 7);
 #pragma unroll
         for (int f = 0; f < 2; ++f)
