@@ -212,13 +212,13 @@ void check_shape(const char* who, const LinearArgs& a)
         throw std::runtime_error(w + ": size_k must be a multiple of 128 (one Hadamard block)");
 }
 
-// rows up to this count go through launch_gemv (one row: the streaming or the VALU kernel; more: the few-row
-// MFMA kernel, the VALU kernel for small weights), more rows through launch_gemm
-int gemv_max_rows() { return knobs().gemv_max_rows; }
-
-std::string dispatch_linear(const LinearArgs& a)
+// Rows up to BERTH_GEMV_MAX_ROWS go through launch_gemv (one row: the streaming or the VALU kernel; more: the few-row
+// MFMA kernel or the VALU kernel, whichever is the quicker), more rows through launch_gemm, up to eight of them
+// on the few-row kernel for large weights only.
+std::string dispatch_linear(LinearArgs a)
 {
-    if (a.size_m <= gemv_max_rows()) return launch_gemv(a);
+    if (a.size_m <= knobs().gemv_max_rows) return launch_gemv(a);
+    a.few_rows_if_large = a.size_m <= 8;
     return launch_gemm(a);
 }
 

@@ -146,6 +146,10 @@ static RowsPlan plan_rows(const Workspace& ws, int slices, int slabs, int size_m
     return pl;
 }
 
+// Up to 8 rows: units from which the few-row kernel is the quicker one whichever launches stand ahead (4096x8192, 4096
+// units, at two rows 13.4 -> 12.8; 4096x2048 with a rotation launch at 2 / 5 / 8 rows 9.8 / 13.4 / 16.8 -> 10.3 / 10.9 / 11.3).
+static long rows_large_units(int size_m) { return size_m <= 3 ? 3072 : 1024; }
+
 // Up to 8 rows the VALU kernel of exl3_gemv.hip rotates the input itself, cuts size_k into parts of two k-blocks at
 // the least (four waves have a k-block of 512 each), and pays half an instruction per weight and row: 4 bits, K x N,
 // us, VALU -> here.
@@ -153,9 +157,7 @@ bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, 
 {
     const RowsPlan pl = plan_rows(ws, slices, slices, size_m, size_k, size_n);
     if (!pl.ok || size_m > 8 || knobs().gemm_rows_units >= 0) return pl.ok;
-    // large weights, whichever launches stand ahead (4096x8192, 4096 units, at two rows 13.4 -> 12.8; 4096x2048 with a
-    // rotation launch at 2 / 5 / 8 rows 9.8 / 13.4 / 16.8 -> 10.3 / 10.9 / 11.3)
-    if (pl.units >= (size_m <= 3 ? 3072 : 1024)) return true;
+    if (pl.units >= rows_large_units(size_m)) return true;
     if (size_k < 512) return false;         // (256x512 at 2 / 4 / 8 rows 7.2 / 8.5 / 12.6 -> 8.2 / 10.4 / 10.4)
     switch (input) {
     case RowsInput::kSelf:
@@ -442,10 +444,12 @@ static void run_block(const BlockPlan& pl, GemmParams& p, int k_bits, int codebo
 struct OperandPlan {
     RowsPlan rows;
     BlockPlan block;
-    OperandPlan(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n, bool activation = false)
+    OperandPlan(const Workspace& ws, int codebook, int slices, int slabs, int size_m, int size_k, int size_n, bool activation = false,
+                bool few_rows_if_large = false)
         : rows(plan_rows(ws, slices, slabs, size_m, size_k, size_n)),
           block(rows.ok ? BlockPlan{} : plan_block(ws, codebook, slices, slabs, size_m, size_k, size_n, activation))
     {
+        if (few_rows_if_large && rows.ok && knobs().gemm_rows_units < 0 && rows.units < rows_large_units(size_m)) rows = RowsPlan{};
         stride = rows.ok ? rows_operand_elements(size_k, rows.mt) : block.operand_stride;
         at = (_Float16*)((char*)ws.partials + (rows.ok ? rows.operand_at : block.operand_at));
     }
@@ -528,7 +532,7 @@ std::string launch_gemm(const LinearArgs& a, const Workspace* scratch)
     if (!scratch) scope.emplace(a.stream);
     const Workspace& ws = scratch ? *scratch : scope->ws;
     throw_pending_device_fault(ws);
-    const OperandPlan plan(ws, a.codebook, 1, 1, a.size_m, a.size_k, a.size_n);
+    const OperandPlan plan(ws, a.codebook, 1, 1, a.size_m, a.size_k, a.size_n, false, a.few_rows_if_large);
     RotateArgs rot;
     rot.in = a.a;
     rot.up = a.a_up;

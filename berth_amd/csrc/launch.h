@@ -145,6 +145,7 @@ struct LinearArgs {
     // (launch_gemm_pair's PairNext::operand), so does that place in the workspace
     bool rotated = false;
     const void* rotated_operand = nullptr;
+    bool few_rows_if_large = false;     // MFMA kernels: 2..8 rows of small weights as 32-row tiles, not on the few-row kernel
 };
 
 // RMS norm with the residual added first, as the input of a launch of the streaming kernel or of a

@@ -395,6 +395,19 @@ def test_small_weights_beside_the_dot_product_kernel(kind, rows, Kk, N, bits, cb
     assert ("exl3_gemm_rows_kernel" in launch) == matrix and ("exl3_gemv_kernel" in launch) != matrix, launch
 
 
+@pytest.mark.parametrize("rows,Kk,N,kernel", [
+    (2, 1024, 1024, "exl3_gemm_rows_kernel"),       # up to the knob's rows: whichever is the quicker
+    (3, 3072, 2048, "exl3_gemm_kernel"),            # above: 768 units of three rows want 3072
+    (8, 1024, 1024, "exl3_gemm_kernel"),            # 128 of eight 1024
+    (8, 2048, 4096, "exl3_gemm_rows_kernel"),
+])
+def test_rows_above_the_knob_of_the_dot_product_kernel(rows, Kk, N, kernel):
+    """BERTH_GEMV_MAX_ROWS: above it small weights take the MFMA tiles of 32 rows, large ones the few-row kernel."""
+    with knobs(BERTH_GEMM_ROWS_UNITS=-1, BERTH_GEMV_MAX_ROWS=2):
+        got, want, ah, want_ah, launch = _run_linear(rows, Kk, N, 3, 2, True, 75 + rows, prefill=True)
+    assert kernel + "<" in launch and np.array_equal(ah, want_ah) and close(got, want)[0] == 0, launch
+
+
 @pytest.mark.parametrize("rows,H,I,bits", [(2, 512, 512, 4), (8, 640, 768, 3), (4, 384, 512, 4)])
 def test_small_block_with_fused_norm(rows, H, I, bits):
     """From 512 of `hidden` on a block's MLP takes the kernel at any of these row counts: gate and up, the rotated
