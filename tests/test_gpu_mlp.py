@@ -21,9 +21,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 EXE = os.path.join(ROOT, "berth_amd", "lib", "berth_host_check")
 
 
-def _layer(gpu, H, I, bits, seed, rows):
+def _layer(gpu, H, I, bits, seed, rows, cb=2):
     lins = [synth.linear(seed, H, I, bits), synth.linear(seed + 3, H, I, bits), synth.linear(seed + 6, I, H, bits)]
-    mlp = MlpLayer(gpu, *(Exl3Linear(gpu, n, *l) for n, l in zip(("gate", "up", "down"), lins)), max_rows=rows)
+    mlp = MlpLayer(gpu, *(Exl3Linear(gpu, n, *l, K.Codebook(cb)) for n, l in zip(("gate", "up", "down"), lins)), max_rows=rows)
     return lins, mlp
 
 
@@ -42,18 +42,18 @@ def test_fused_mlp_stage_by_stage(rows, H, I, bits):
         assert len(dense) == 3 and "silu_mul" in launch
 
 
-def run_mlp_block(rows, H, I, bits):
+def run_mlp_block(rows, H, I, bits, cb=2):
     """One berth_exl3_mlp call checked stage by stage against the oracle; returns the launch text."""
     gpu = Gpu(0)
-    (gate, up, down), mlp = _layer(gpu, H, I, bits, 9000 + rows, rows)
+    (gate, up, down), mlp = _layer(gpu, H, I, bits, 9000 + rows, rows, cb)
     x = (synth.activations(9100 + rows, rows, H).astype(np.float32) / np.sqrt(H)).astype(np.float16)
     y = torch.zeros((rows, H), dtype=torch.float32, device=gpu.device)
     mlp.forward(gpu, gpu.upload(x.view(np.uint16)), y, rows=rows)
     gpu.synchronize()
     launch = K.last_launch()
 
-    g_want, xh_want = O.linear(x, *gate, H, I, bits, 2)
-    u_want, _ = O.linear(x, *up, H, I, bits, 2)
+    g_want, xh_want = O.linear(x, *gate, H, I, bits, cb)
+    u_want, _ = O.linear(x, *up, H, I, bits, cb)
     g_got = host_f16(mlp.g)[:rows * I].reshape(rows, I)
     assert close(g_got, g_want.reshape(rows, I))[0] == 0
     if rows <= 8 or I >= H:
@@ -70,7 +70,7 @@ def run_mlp_block(rows, H, I, bits):
     else:
         act = host_f16(mlp.u)[:rows * I].reshape(rows, I)          # up_out holds the activation
         assert close(act, O.silu_mul(g_want, u_want).reshape(rows, I), rtol=4e-3, atol=2e-3)[0] == 0
-    y_want, _ = O.linear(act, *down, I, H, bits, 2, out_fp32=True)
+    y_want, _ = O.linear(act, *down, I, H, bits, cb, out_fp32=True)
     assert close(y.cpu().numpy(), y_want.reshape(rows, H))[0] == 0
     return launch
 

@@ -14,6 +14,7 @@ from berth_amd.kernels import Codebook, OutDtype
 from oracle import oracle as O
 from tests.gpu_util import DEV, close, dev, host_f16, host_u16, knobs
 from tests.test_gpu_linear import _run_linear
+from tests.test_gpu_mlp import run_mlp_block
 
 pytestmark = pytest.mark.gpu
 
@@ -77,7 +78,6 @@ def test_bundle_with_narrower_slices(rows, unit):
 
 @pytest.mark.parametrize("rows", [4, 12])
 def test_mlp_of_few_rows_stage_by_stage(rows):
-    from tests.test_gpu_mlp import run_mlp_block
     launch = run_mlp_block(rows, 1536, 4096, 4)
     assert launch.count("exl3_gemm_rows_kernel") == 2 and "silu_mul_had_r_128_kernel" in launch, launch
 
@@ -96,7 +96,7 @@ def test_mlp_of_few_rows_stage_by_stage(rows):
 def test_mlp_whose_gate_and_up_leave_the_next_input(rows, H, I, bits):
     """Gate, up or activation, rotated activation and output, stage by stage; a second call gives the same bits."""
     from berth_amd.device import Gpu
-    from tests.test_gpu_mlp import _layer, run_mlp_block
+    from tests.test_gpu_mlp import _layer
     with knobs(BERTH_GEMM_ROWS_UNITS=192 if I == 5120 else 1):
         launch = run_mlp_block(rows, H, I, bits)
     assert ",silu,rotate>" in launch and "silu_mul_had_r_128_kernel" not in launch, launch
@@ -111,6 +111,13 @@ def test_mlp_whose_gate_and_up_leave_the_next_input(rows, H, I, bits):
         got.append([y] + [getattr(mlp, n).clone() for n in ("g", "u", "act_had")])
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("rows,H,I,bits,cb", [(5, 2048, 5632, 3, 1), (24, 640, 17408, 4, 1),       # one tile of sixteen rows and two
+                                              (8, 1152, 8448, 2, 0), (17, 1152, 8448, 5, 0)])
+def test_gate_and_up_leave_the_next_input_with_the_other_codebooks(rows, H, I, bits, cb):
+    launch = run_mlp_block(rows, H, I, bits, cb)
+    assert f"exl3_gemm_rows_kernel<{bits},{cb},{16 if rows <= 16 else 32}x128,silu,rotate>" in launch, launch
 
 
 @pytest.mark.parametrize("rows,H,I,bits", [(2, 128, 256, 4),        # one block a row: a quarter of a wave
@@ -349,6 +356,22 @@ def test_few_rows_of_a_bundle_by_value(rows, Kk, widths, bits, fp32, rotates):
         assert np.array_equal(slab, want_had.view(np.uint16).reshape(-1)), i
 
 
+@pytest.mark.parametrize("rows,bits,cb", [(2, 4, 0), (5, 3, 1), (8, 6, 1)])
+def test_few_rows_of_a_bundle_by_value_with_the_other_codebooks(rows, bits, cb):
+    from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
+    gpu, Kk, widths = Gpu(0), 2304, (1024, 512, 512)
+    lins = [synth.linear(790 + i, Kk, n, bits) for i, n in enumerate(widths)]
+    multi = Exl3MultiLinear(gpu, [Exl3Linear(gpu, f"l{i}", *lin, Codebook(cb)) for i, lin in enumerate(lins)])
+    x, outs = synth.activations(795 + rows, rows, Kk), [torch.zeros((rows, n), dtype=torch.float16, device=DEV) for n in widths]
+    with knobs(BERTH_GEMM_ROWS_UNITS=-1):
+        multi.forward(gpu, dev(x.view(np.uint16)), outs, OutDtype.F16, rows)
+    torch.cuda.synchronize()
+    launch = K.ops.last_launch()
+    assert "by value" in launch and f"exl3_gemm_rows_kernel<{bits},{cb},16x128,rotate>" in launch, launch
+    for out, lin, n in zip(outs, lins, widths):
+        assert close(host_f16(out), O.linear(x, *lin, Kk, n, bits, cb, out_fp32=False)[0])[0] == 0, launch
+
+
 def test_few_rows_by_value_with_outputs_over_the_input():
     """The host sees that an output lies over the input: a launch of its own rotates, and the bits are those of other buffers."""
     from berth_amd.device import Exl3Linear, Exl3MultiLinear, Gpu
@@ -390,7 +413,6 @@ def test_small_weights_beside_the_dot_product_kernel(kind, rows, Kk, N, bits, cb
             _bundle(rows, Kk, (N, N // 4), bits)
             launch = K.ops.last_launch()
         else:
-            from tests.test_gpu_mlp import run_mlp_block
             launch = run_mlp_block(rows, Kk, N, bits)
     assert ("exl3_gemm_rows_kernel" in launch) == matrix and ("exl3_gemv_kernel" in launch) != matrix, launch
 
