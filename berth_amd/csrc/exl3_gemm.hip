@@ -174,8 +174,10 @@ bool gemm_rows_applies(const Workspace& ws, int slices, int size_m, int size_k, 
         return true;
     case RowsInput::kMlp:
         // Three launches beside two: MLPs of 2048x4096 at 2 / 3 rows 19.9 / 21.9 -> 24.1 / 24.4, of 1536x3072 at 4 / 5 / 8
-        // rows 23.6 / 25.1 / 29.8 -> 23.9 / 24.6 / 24.7; down alone, 1024 x 2048 at 4 / 5 / 8 rows, saves 0 / 3 / 7.  The
-        // smallest keep the two launches that the entry promises them.
+        // rows 23.6 / 25.1 / 29.8 -> 23.9 / 24.6 / 24.7; down alone, 1024 x 2048 at 4 / 5 / 8 rows, saves 0 / 3 / 7.  Up to
+        // 1024 of hidden the two launches stay, which the entry states for small weights, although three would be quicker
+        // (512x1024 at 2 / 4 / 5 / 8 rows 15.9 / 19.3 / 21.7 / 29.3 beside 15.9 / 16.1 / 16.5 / 16.7, 1024x2048 18.3 / 21.7 / 24.3 /
+        // 32.1 beside 19.6 / 19.3 / 19.1 / 20.4).
         return size_m >= 5 && size_k >= 1024 && (slices == 2 ? size_k : size_n) > 1024;
     case RowsInput::kLaunch:
         break;

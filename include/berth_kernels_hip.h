@@ -205,9 +205,9 @@ int berth_ops_cat_f16_last(const void* embedding, const void* hidden, void* out,
  * size_n_list[s] <= size_n = slice width; had_src_list[s] = source index;
  * a_had holds num_had_src slabs of size_m*size_k.  Uniform mode (lists NULL):
  * bszm_out linears of one shape, inputs a[i] (bszm_in == bszm_out) or a[0]
- * (bszm_in == 1), outputs c[i] contiguous.  Any row count: one row and 2..8 rows of
- * small weights rotate the input inside the one launch (so neither the input nor a_had may
- * overlap an output there); up to 32 rows where a workgroup needs a part of size_k only do so
+ * (bszm_in == 1), outputs c[i] contiguous.  Any row count: one row, and 2..8 rows of
+ * weights for which the few-row MFMA kernel is not the quicker one, rotate the input inside the one
+ * launch (so up to 8 rows neither the input nor a_had may overlap an output); up to 32 rows where a workgroup needs a part of size_k only do so
  * in uniform mode, or with lists in host memory, where no output overlaps either; the others take
  * one launch that rotates the input once per source / linear, whether a slice uses it or
  * not, and MFMA launches over all slices (the reference sends
@@ -280,13 +280,14 @@ typedef struct {
  * y = down(silu(gate(x)) * up(x)), the four calls of MlpLayer::forward
  * (crates/berth-engine/src/mlp.rs:118-150: two berth_exl3_linear with fp16
  * output, berth_ops_silu_mul with act_limit 0, berth_exl3_linear with fp32
- * output) in one entry.  One row, and 2..8 rows of small weights (hidden up to 1024 at least), run as two
- * launches: gate and up share one launch and the rotated input, and the down
- * projection evaluates silu(g) * u while it rotates its input (same fp16 steps as
- * berth_ops_silu_mul, so the activation is bit-identical to the unfused sequence).
- * More rows, and 2..8 rows of larger weights, run on the MFMA kernels: gate and up as
- * one bundle (one launch rotates the input with either linear's scales, the next runs
- * both; the up projection's rotated copy waits in act_had, so this form needs
+ * output) in one entry.  One row, and 2..8 rows of small weights, run as two launches
+ * (small: gate and up together below 1024 units of 64 x 128 weights, 3072 at two and three
+ * rows, and hidden up to 1024 or fewer than five rows): gate and up share one launch and the
+ * rotated input, and the down projection evaluates silu(g) * u while it rotates its input (same
+ * fp16 steps as berth_ops_silu_mul, so the activation is bit-identical to the unfused sequence).
+ * More rows, and 2..8 rows of larger weights (the down projection by its own size), run on the
+ * MFMA kernels: gate and up as one bundle (one launch rotates the input with either linear's
+ * scales, the next runs both; the up projection's rotated copy waits in act_had, so this form needs
  * intermediate >= hidden, else gate and up run one after the other), one launch that
  * forms silu(g) * u and rotates it, the down projection.  The few-row kernel (2..32 rows)
  * forms and rotates silu(g) * u itself where gate and up are wide enough; the row-block kernel
@@ -318,7 +319,10 @@ int berth_exl3_mlp(const void* x, const berth_exl3_lin* lins, void* gate_out, vo
  * output: two launches when both do.  More rows where gate and up run on the MFMA kernels as one
  * bundle: the norm is formed where the input is rotated and the residual added where the down launch
  * writes (four launches, three of few rows where gate and up are wide enough; on the row-block kernel
- * the third finishes gate's and up's tiles too, and a fifth finishes those that down shares).  Anything else runs the same arithmetic as separate launches. */
+ * the third finishes gate's and up's tiles too, and a fifth finishes those that down shares).  Anything else
+ * runs the same arithmetic as separate launches.  2..8 rows of hidden 512 and more take the few-row MFMA kernel in
+ * the block, with which three launches stand beside five, also where berth_exl3_mlp by itself stays on two launches of
+ * the VALU kernel: the fp32 sums of gate, up and down are then added in another order than by the separate calls. */
 typedef struct {
     const void* weight;         /* fp16 or bf16 [hidden] */
     float epsilon, constant_bias, constant_scale;

@@ -456,9 +456,59 @@ def test_small_block_with_fused_norm(rows, H, I, bits):
     want, act_had = O.linear(act, *down, I, H, bits, 2, out_fp32=True)
     assert np.array_equal(host_u16(mlp.act_had)[:rows * I], act_had.view(np.uint16).ravel())
     # rows of a norm reach 5e4 here, and where they cancel what is left is the rounding of the sums: a wave adds eight
-    # products at a time, I / 8 roundings of half an ulp of partial sums as large as the largest output
-    atol = max(1e-3, I / 8 * 2.0 ** -24 * float(np.abs(want).max()))
-    assert close(y.cpu().numpy(), want.reshape(rows, H) + res_ref.cpu().numpy(), atol=atol)[0] == 0, launch
+    # products at a time, I / 8 roundings of half an ulp of partial sums as large as the row's largest output
+    want = want.reshape(rows, H)
+    atol = np.maximum(1e-3, I / 8 * 2.0 ** -24 * np.abs(want).max(axis=1, keepdims=True))
+    assert close(y.cpu().numpy(), want + res_ref.cpu().numpy(), atol=atol)[0] == 0, launch
+
+
+@pytest.mark.parametrize("rows,H,I,bits,same", [
+    (2, 512, 512, 4, False), (8, 640, 768, 3, False),   # the block takes the few-row kernel, the call the dot-product kernel
+    (4, 384, 512, 4, True),                             # both the dot-product kernel
+    (5, 1280, 3072, 2, True), (9, 1152, 1280, 3, True), # both the few-row kernel
+])
+def test_block_beside_the_separate_calls_at_default_knobs(rows, H, I, bits, same):
+    """berth_exl3_mlp_block against norm -> berth_exl3_mlp -> add: the same bits where both take the same kernels.  Elsewhere
+    gate, up and the output are fp32 sums of the same products in another order: four fp16 roundings (gate, up, activation,
+    rotated activation) of half a unit, 2^-11, may fall either way, and rotations and random weights keep a row's
+    relative 2-norm."""
+    from berth_amd.device import Gpu, ptr
+    from tests.test_gpu_mlp import _block_inputs, _layer
+    gpu = Gpu(0)
+    _, mlp = _layer(gpu, H, I, bits, 9400 + rows, rows)
+    x, res, w = _block_inputs(gpu, H, rows, 9450 + rows)
+    stream, h, add = res.clone(), torch.zeros((rows, H), dtype=torch.float16, device=DEV), torch.zeros_like(res)
+    res_out, y = torch.zeros_like(res), torch.zeros_like(res)
+    with knobs(BERTH_GEMM_ROWS_UNITS=-1):
+        K.ops.rms_norm_res_in(ptr(x), ptr(w), ptr(h), ptr(stream), rows, H, 1e-6, 1.0, 1.0, True, gpu.raw_stream())
+        mlp.forward(gpu, h, add, rows=rows)
+        separate = K.last_launch()
+        sums, x_had = add.clone(), mlp.x_had.clone()
+        K.ops.add_f32(ptr(add), ptr(stream), ptr(add), rows * H, gpu.raw_stream())
+        mlp.forward_block(gpu, x, res, res_out, w, y, rows=rows)
+        launch = K.last_launch()
+    torch.cuda.synchronize()
+    assert torch.equal(res_out, stream) and torch.equal(x_had, mlp.x_had), launch
+    assert (("exl3_gemv_kernel" in separate) == ("exl3_gemv_kernel" in launch)) == same, (separate, launch)
+    if same:
+        assert torch.equal(y, add), launch
+    else:
+        off = (y.double() - add.double()).norm(dim=1) / sums.double().norm(dim=1)
+        assert float(off.max()) <= 4 * 2 * 2.0 ** -11, (off, launch)
+
+
+@pytest.mark.parametrize("rows,H,I,matrix,dots", [
+    (4, 1024, 3072, 0, 2),      # 768 units of gate and up: two launches of the dot-product kernel
+    (4, 1024, 4096, 1, 1),      # 1024, from which gate and up take the few-row kernel whatever hidden is
+    (4, 512, 8192, 1, 1),
+    (3, 1024, 4096, 0, 2),      # 3072 at two and three rows
+    (8, 1024, 2048, 0, 2), (4, 1152, 2048, 0, 2),
+    (5, 1152, 2048, 2, 0),      # above 1024 of hidden five rows and more
+])
+def test_launches_of_small_mlps(rows, H, I, matrix, dots):
+    with knobs(BERTH_GEMM_ROWS_UNITS=-1):
+        launch = run_mlp_block(rows, H, I, 2)
+    assert (launch.count("exl3_gemm_rows_kernel"), launch.count("exl3_gemv_kernel")) == (matrix, dots), launch
 
 
 @pytest.mark.parametrize("rows,Kk,N,bits,own", [
