@@ -820,6 +820,20 @@ static GroupRowsPlan plan_group_rows(const Workspace& ws, const GroupedArgs& g)
     return pl;
 }
 
+// Workgroups a compute unit up to which the waves of a grouped launch give way (PriorityRamp): one round of four, of gate
+// and up together (`pair`) one and a half.  The more bits, the more of the launch waits for the weights instead of for the
+// vector pipes, and waves that give way then ask later.  560 random layers of 4..160 tokens at sums of 100 to 2600
+// workgroups, the whole layer with and without in turn: gate and up at 2..5 bits 1 to 5 % quicker up to four, 0 to 2 up
+// to six, 2 to 5 slower from seven; 6 bits 1 to 3 quicker up to four, then up to 7 slower (112 tokens x 128 experts of
+// 3584x1280, 1280 workgroups, 296 -> 308 us; 5 bits as the others, 3INST up to six at 6 and 7 bits too: 1 to 3 quicker); 7 bits 1 to 3
+// quicker up to three, then 2 to 5 slower; 8 bits 1 to 3 quicker up to two, 0 to 2 slower up to three, 2 to 6 at four (3INST 1 to 3
+// quicker up to three).  Down likewise, with half of each: at 6 bits 1 to 2 % up to four, 7 bits up to 3.9 slower from three, 8 from two.
+static int ramp_workgroups(int bits, int codebook, bool pair)
+{
+    if (codebook == 0) return bits < 8 ? (pair ? 6 : 4) : 3;
+    return bits == 8 ? 2 : bits == 7 ? 3 : pair && bits < 6 ? 6 : 4;
+}
+
 // grouped: problems of at most 32 rows each (and, in a list of their own, of up to 128); a_had rows are in problem
 // order, or found through a_rows
 std::string launch_gemm_grouped(const GroupedArgs& g)
@@ -874,7 +888,7 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         if (g.max_problems > 65535) throw std::runtime_error("moe grouped linear: too many problems");
         p.act_had = (_Float16*)g.act_had;
         p.group_lins = 1;
-        p.ramp_problems = 6 * ws.cu_count / (g.size_n / 128);
+        p.ramp_problems = ramp_workgroups(g.k_bits, g.codebook, true) * ws.cu_count / (g.size_n / 128);
         std::string desc;
         gemm_bits(p, g.k_bits, g.codebook, -4, g.stream, desc, group_grid(g.size_n / 128, 1, g.max_problems));
         hip_ok(hipGetLastError(), "exl3_gemm_pair_kernel launch");
@@ -901,7 +915,7 @@ std::string launch_gemm_grouped(const GroupedArgs& g)
         hip_ok(hipGetLastError(), "exl3_gemm_mixed_kernel launch");
         return desc + " grouped";
     }
-    p.ramp_problems = 4 * ws.cu_count / (nblocks * p.S * g.num_lins);
+    p.ramp_problems = ramp_workgroups(g.k_bits, g.codebook, false) * ws.cu_count / (nblocks * p.S * g.num_lins);
     gemm_bits(p, g.k_bits, g.codebook, mb, g.stream, desc, group_grid(nblocks * p.S, g.num_lins, g.max_problems));
     hip_ok(hipGetLastError(), "exl3_gemm_kernel grouped launch");
     return desc + " grouped";

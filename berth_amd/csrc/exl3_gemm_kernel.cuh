@@ -225,7 +225,8 @@ constexpr int kAStride = 128 + 8;   // halves per LDS row of the A tile (272 B: 
 // wait.  A wave gives up its priority in three steps over its second half, which lets the ones behind it catch up.
 // Grouped launches of 32-row problems, layers of 2048 x 768: 64 tokens x 128 experts 104.8 -> 102.7 us, with popular
 // ones 80.2 -> 77.3, 20 tokens 96.0 -> 92.8, 100 tokens x 64 experts 77.2 -> 74.9.  Only where the workgroups there are come
-// in one round of four a compute unit, of gate and up together in one and a half: those of a later round start ahead
+// in one round of four a compute unit, of gate and up together in one and a half, and in fewer with many bits
+// (ramp_workgroups): those of a later round start ahead
 // of the ones that give way, which end the later (down, traced: 128 tokens x 512 experts of 768x2048, 3760 workgroups, 122 ->
 // 133 us, 64 tokens x 160 of 1664x4096, 2500, 195 -> 207, 40 tokens x 64 of 2048x7168, 1790, 148 -> 155; gate and up of
 // 128 tokens x 512 experts, 2820, 245 -> 257, but 64 tokens x 512 experts x 512, 1470, 130 -> 122, 40 tokens x 64 of 7168x2048,
