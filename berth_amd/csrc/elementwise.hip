@@ -131,6 +131,10 @@ __global__ __launch_bounds__(256) void silu_mul_had_r_128_kernel(RotateParams p)
 // element against 42 of the four launches (residual add, norm, two rotations).
 // With few rows a launch is a chain of waits: row, norm weights and both scales asked for together, and the wave's sum by
 // DPP moves, 5 rows of 5120 5.6 -> 5.1 us, 100 rows 7.9 -> 7.4 (traced).
+// So with two and four chunks a thread too, for all that these hold 70 and 127 registers (and four of the latter in
+// scratch) instead of 46 and 62: 2 / 100 / 600 rows of 9216 8.1 / 10.2 / 21.9 -> 7.3 / 9.6 / 17.7, of 16384 11.2 / 14.5 / 42.6 ->
+// 9.2 / 14.0 / 38.9, of 17408 12.4 / 15.8 / 45.5 -> 11.1 / 16.1 / 45.7, of 24576 15.7 / 24.5 / 61.0 -> 13.5 / 21.7 / 58.6, of
+// 32768 28.2 / 38.7 / 81.3 -> 22.0 / 27.2 / 76.3 (scales and weight of four chunks behind the sum, no scratch: 25.1 / 33.0 / 76.2).
 struct NormParams {
     const float* x;
     const float* res;
@@ -142,7 +146,8 @@ struct NormParams {
 };
 constexpr int kNormSlabs = 2;           // gate and up
 // the sum over a wave by butterflies over lane distances 32 .. 1, the partner's two dwords by DPP moves and the row swaps
-// instead of LDS permutes
+// instead of LDS permutes: one row of 2048 / 5120 / 17408 1.91 / 2.18 / 3.48 -> 1.76 / 2.08 / 3.40 us, with the residual 2.10 /
+// 2.82 / 5.88 -> 1.90 / 2.64 / 5.73, 48000 fp16 rows of 128 30.0 -> 26.6, 32 of them 2.8 -> 2.6; 1500 rows of 5120 9.1 either way
 __device__ __forceinline__ double wave_sum(double v)
 {
     auto partner = [](double x, auto move) {
